@@ -7,6 +7,7 @@ or the device is not an MI355X the operators raise.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 from typing import Optional
@@ -15,6 +16,7 @@ import torch
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_PKG_DIR), "lib", "libsba.so")
+EXT_PATH = os.path.join(os.path.dirname(_PKG_DIR), "lib", "_sba_torch.so")
 
 SBA_BF16 = 1
 SBA_F16 = 2
@@ -115,6 +117,28 @@ def load():
         lib.sba_last_kernel_ms.argtypes = [ctypes.c_int]
         _lib = lib
     return _lib
+
+
+_ext = None
+
+
+def load_ext():
+    """Import _sba_torch.so (csrc/sba_torch.cpp), the PyTorch binding the eager operators go through."""
+    global _ext
+    if _ext is not None:
+        return _ext
+    load()
+    with _lock:
+        if _ext is None:
+            if not os.path.exists(EXT_PATH):
+                raise RuntimeError(
+                    f"_sba_torch.so not found at {EXT_PATH}: build it with "
+                    "`make -C stickbreaking-attention_amd/csrc` (g++ against the installed PyTorch)")
+            spec = importlib.util.spec_from_file_location("_sba_torch", EXT_PATH)
+            ext = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(ext)
+            _ext = ext
+    return _ext
 
 
 def check(code: int, what: str) -> None:

@@ -384,8 +384,13 @@ def _schedule_workspace(cu: Optional[torch.Tensor], sched_bytes: int, batch: int
     must not depend on a tensor this cache may drop), every call gets a workspace of its own."""
     if torch.compiler.is_compiling() or torch.cuda.is_current_stream_capturing():
         return torch.empty(sched_bytes, dtype=torch.uint8, device=device), True
+    return _cached_schedule(cu, sched_bytes, batch, tokens, device)
+
+
+def _cached_schedule(cu: Optional[torch.Tensor], sched_bytes: int, batch: int, tokens: int, device):
     version = None if cu is None else _version_of(cu)
-    key = (device, torch.cuda.current_stream(device).cuda_stream, batch, tokens, sched_bytes)
+    # (the raw stream handle: torch.cuda.current_stream() builds two Python objects to hold it, 2 us per call)
+    key = (device, torch._C._cuda_getCurrentRawStream(device.index), batch, tokens, sched_bytes)
     with _cache_lock:
         if cu is None or version is not None:
             for i in range(len(_sched_cache) - 1, -1, -1):
@@ -455,6 +460,44 @@ def run_forward(q, k, v, fixed: bool, cu_seqlens, max_seqlens, inv_temp: float, 
         rem = rem.to(q.dtype)
     state = (table, sched, cu, max_len, product)
     return (o, rem, state, weights) if return_attention else (o, rem, state)
+
+
+@functools.lru_cache(maxsize=64)
+def _sizes(fixed: bool, batch: int, heads: int, tokens: int, n_docs: int, max_doc_len: int, entries: Optional[int]) -> Tuple[int, int]:
+    return workspace_sizes(fixed, batch, heads, tokens, n_docs, max_doc_len, entries)
+
+
+def runs_natively(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether a call goes to the C++ operator (``eager``): everything in eager mode except the switches that change
+    what the backward does and calls recorded into a graph, which take the launchers above."""
+    return (q.is_cuda and not torch.compiler.is_compiling() and not torch._C._cuda_isCurrentStreamCapturing()
+            and k.shape == q.shape and v.shape == q.shape and not RECOMPUTE_TABLE and not VALIDATE
+            and not (F32_AS_F16 and q.dtype == torch.float32))
+
+
+def eager(q, k, v, fixed: bool, cu_seqlens, max_seqlens, inv_temp: float, attend_current: bool, fused: bool = False):
+    """The differentiable operator for eager calls: finds the schedule and the table size of the documents (both
+    remembered) and hands everything to csrc/sba_torch.cpp, whose autograd node runs the backward without Python.
+    Returns [o, rem], or [o + rem * v] with ``fused``."""
+    if fixed:
+        B, H, T, _ = q.shape
+        n_docs, max_len, cu, entries = 0, T, None, None
+    else:
+        H, T, _ = q.shape
+        B, entries = 1, None
+        cu = _check_cu(cu_seqlens, q)
+        n_docs = cu.numel()
+        max_len = T if max_seqlens is None else max(1, min(int(max_seqlens), T))
+        cu_vals = host_cu_seqlens(cu)
+        if cu_vals is not None:      # (see run_forward)
+            _, max_len, entries = _lengths_info(cu_vals, T)
+    sched_bytes, table_floats = _sizes(fixed, B, H, T, n_docs, max_len, entries)
+    if q.dtype not in (torch.bfloat16, torch.float16):
+        _warn_reduced_precision(q.dtype)
+    sched, build = _cached_schedule(cu, sched_bytes, B, T, q.device)
+    flags = ((nat.FLAG_ATTEND_CURRENT if attend_current else 0) | (nat.FLAG_PRODUCT_SPACE if PRODUCT_SPACE else 0) |
+             (nat.FLAG_FUSE_REMAINDER if fused else 0))
+    return nat.load_ext().attention(q, k, v, cu, sched, build, table_floats, max_len, inv_temp, flags)
 
 
 def check_status(sched: torch.Tensor, table: Optional[torch.Tensor] = None, heads: int = 1,
@@ -535,6 +578,8 @@ def _rebuild_table(qp, kp, vp, fixed: bool, sched, cu, max_len: int, inv_temp: f
 
 def release_workspaces() -> None:
     """Drop the cached gradient tables, schedules and host copies of cu_seqlens."""
+    if nat._ext is not None:
+        nat._ext.release()
     with _cache_lock:
         _gtab_cache.clear()
         del _host_cu_cache[:]

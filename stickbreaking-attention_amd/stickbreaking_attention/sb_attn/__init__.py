@@ -62,6 +62,9 @@ def sb_attn(q, k, v, inv_temp=None, zero_start=True, attend_current=False):
 
 
 def sb_attn_(q, k, v, inv_temp, attend_current):
+    if _ops.runs_natively(q, k, v):
+        o, rem = _ops.eager(q, k, v, True, None, None, inv_temp, attend_current)
+        return o, rem
     return StickBreakingAttention.apply(q, k, v, inv_temp, attend_current)
 
 
@@ -94,4 +97,6 @@ def sb_attn_fused(q, k, v, inv_temp=None, zero_start=True, attend_current=False)
     tests/test_attn.py:64) as one tensor."""
     if inv_temp is None:
         inv_temp = 1 / math.sqrt(q.size(-1))
+    if _ops.runs_natively(q, k, v):
+        return _ops.eager(q, k, v, True, None, None, inv_temp, attend_current, fused=True)[0]
     return StickBreakingAttentionFused.apply(q, k, v, inv_temp, attend_current)

@@ -119,6 +119,9 @@ def sb_attn_varlen(q, k, v, cu_seqlens, max_seqlens=None, inv_temp=None, zero_st
 
 
 def sb_attn_varlen_(q, k, v, inv_temp, cu_seqlens, max_seqlens, attend_current):
+    if _ops.runs_natively(q, k, v):
+        o, rem = _ops.eager(q, k, v, False, cu_seqlens, max_seqlens, inv_temp, attend_current)
+        return o, rem
     return StickBreakingAttention.apply(q, k, v, cu_seqlens, max_seqlens, inv_temp, attend_current)
 
 
@@ -156,4 +159,6 @@ def sb_attn_varlen_fused(q, k, v, cu_seqlens, max_seqlens=None, inv_temp=None, z
         cu_seqlens = _strip_leading_zero(cu_seqlens)
     if inv_temp is None:
         inv_temp = 1 / math.sqrt(q.size(-1))
+    if _ops.runs_natively(q, k, v):
+        return _ops.eager(q, k, v, False, cu_seqlens, max_seqlens, inv_temp, attend_current, fused=True)[0]
     return StickBreakingAttentionFused.apply(q, k, v, cu_seqlens, max_seqlens, inv_temp, attend_current)
