@@ -104,9 +104,9 @@ __device__ __forceinline__ void grad_dz(const float (&p)[16], const float (&r)[1
 // dq pass
 // -------------------------------------------------------------------------------------------
 // (head_dim 256: the tiles take 128 KiB, one workgroup per CU, one wave per SIMD with 512 registers)
-template <int D, bool AC, bool PROD>
+template <int D, bool AC, bool PROD, int U = D>
 __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dq_kernel(const KArgs a) {
-  constexpr int KS = D / 16, DB = D / 32;
+  constexpr int KS = U / 16, DB = U / 32;
   constexpr int TILE = BN * D;   // elements of one K or V tile (unpadded, swizzled)
   // K (row reads for the scores, transpose reads for dq) and V (row reads) tiles,
   // double-buffered, filled by asynchronous global -> LDS copies.
@@ -130,9 +130,9 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dq_kernel(const KArgs
       int row0, row1;
       unsigned pair;
       spare_rows(refused, slot, hdr.y, sched[SCHED_TOTAL], a.tokens, a.nan_pair, row0, row1, pair);
-      fill_rows16(a.dq, head, row0, row1, D, pair, threadIdx.x, NT);
-      fill_rows16(a.dk, head, row0, row1, D, pair, threadIdx.x, NT);
-      fill_rows16(a.dv, head, row0, row1, D, pair, threadIdx.x, NT);
+      fill_rows16(a.dq, head, row0, row1, a.head_dim, pair, threadIdx.x, NT);
+      fill_rows16(a.dk, head, row0, row1, a.head_dim, pair, threadIdx.x, NT);
+      fill_rows16(a.dv, head, row0, row1, a.head_dim, pair, threadIdx.x, NT);
     }
     return;
   }
@@ -151,14 +151,14 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dq_kernel(const KArgs
   const elem_t* vb = reinterpret_cast<const elem_t*>(a.v.ptr) + t.batch * a.v.sb + head * a.v.sh + tok0 * a.v.st;
   const elem_t* gob = reinterpret_cast<const elem_t*>(a.go.ptr) + t.batch * a.go.sb + head * a.go.sh + tok0 * a.go.st;
   elem_t* dqb = reinterpret_cast<elem_t*>(a.dq.ptr) + t.batch * a.dq.sb + head * a.dq.sh + tok0 * a.dq.st;
-  const Rows qrows = make_rows(qb, a.q.st, t.doc_len);
-  const Rows grows = make_rows(gob, a.go.st, t.doc_len);
-  const Rows krows = make_rows(kb, a.k.st, t.doc_len);
-  const Rows vrows = make_rows(vb, a.v.st, t.doc_len);
+  const Rows qrows = make_rows(qb, a.q.st, t.doc_len, a.head_dim);
+  const Rows grows = make_rows(gob, a.go.st, t.doc_len, a.head_dim);
+  const Rows krows = make_rows(kb, a.k.st, t.doc_len, a.head_dim);
+  const Rows vrows = make_rows(vb, a.v.st, t.doc_len, a.head_dim);
 
   TileCopy<D, BN, NT, true> kcopy, vcopy;
-  kcopy.init(tid, krows.row_bytes);
-  vcopy.init(tid, vrows.row_bytes);
+  kcopy.init(tid, krows.row_bytes, krows.used_bytes);
+  vcopy.init(tid, vrows.row_bytes, vrows.used_bytes);
   kcopy.issue(krows, 0, Ks);
   vcopy.issue(vrows, 0, Vs);
 
@@ -320,7 +320,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dq_kernel(const KArgs
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   if (pend_ix >= 0 && qvalid && h == 0) gtab[(unsigned)(pend_ix + qrow)] = Cst[w][n];
   lds_barrier();   // every wave is done with the K/V tiles: their memory becomes the dq staging area
-  store_block32<D>(Ks + w * 32 * D, dqacc, a.inv_temp, dqb, a.dq.st, qw0, t.doc_len, lane);
+  store_block32<D, U>(Ks + w * 32 * D, dqacc, a.inv_temp, dqb, a.dq.st, qw0, t.doc_len, a.head_dim, lane);
 }
 
 // -------------------------------------------------------------------------------------------
@@ -347,9 +347,9 @@ constexpr int BQ = 32;     // queries per step of the dk/dv pass
 constexpr int RING = 6;    // Q/dO tile slots: tiles i-1 (products) .. i+4 (in flight) of step i
 constexpr int AHEAD = 4;   // a tile is requested this many steps before the products use it + 1
 
-template <int D, bool AC, bool PROD>
+template <int D, bool AC, bool PROD, int U = D>
 __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
-  constexpr int KS = D / 16, DB = D / 32;
+  constexpr int KS = U / 16, DB = U / 32;
   constexpr int NPT = NT2 / 2;                 // threads of one role
   constexpr int QTILE = BQ * D;     // elements of one Q or dO tile (swizzled, unpadded)
   constexpr int PTILE = BQ * BKV;   // elements of one staged p or dz block [query][key]
@@ -403,9 +403,10 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
     it.head = item - slot * a.heads;
     return it;
   };
-  auto rows_of = [](const View& v, const Item& it) {
+  const int head_dim = a.head_dim;
+  auto rows_of = [head_dim](const View& v, const Item& it) {
     return make_rows(reinterpret_cast<const elem_t*>(v.ptr) + it.batch * v.sb + it.head * v.sh + (int64_t)it.tok_start * v.st,
-                     v.st, it.doc_len);
+                     v.st, it.doc_len, head_dim);
   };
   Item cur = describe(blockIdx.x, t_first);
   // The item after the current one and its tile descriptor, as the first score wave left them in `mbox` (every wave,
@@ -516,8 +517,8 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
       request(2, r2);
       const Rows qrows = rows_of(a.q, it), grows = rows_of(a.go, it);
       Copy qcopy, gcopy;      // (formed here, once per item: a score wave has no register to keep them in)
-      qcopy.init(64 * rw + 32 * h + n, qrows.row_bytes);
-      gcopy.init(64 * rw + 32 * h + n, grows.row_bytes);
+      qcopy.init(64 * rw + 32 * h + n, qrows.row_bytes, qrows.used_bytes);
+      gcopy.init(64 * rw + 32 * h + n, grows.row_bytes, grows.used_bytes);
       auto tiles = [&](int from, int to) {
         if (!(copier && with_tiles)) return;
 #pragma unroll
@@ -633,7 +634,7 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
     auto bulk = [&](auto band_tag, auto slot_tag, int i, f32x16& xc, f32x16& dc, f32x16& xn, f32x16& dn, Raw& set) {
       constexpr bool BAND = decltype(band_tag)::value;
       constexpr int SLOT = decltype(slot_tag)::value;
-      constexpr int NCHUNK = 8, PER = 2 * KS / NCHUNK;
+      constexpr int NCHUNK = 8, PER = 2 * (D / 16) / NCHUNK;   // (U < D: the last chunks have no MFMAs left)
       settle(i, set, carry_e, carry_c, dr);   // requested three steps ago
       request(i + 3, set);
       const int slot8 = SLOT >= 0 ? SLOT : ((i + 1) % RING);
@@ -651,6 +652,7 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
 #pragma unroll
         for (int m = 0; m < PER; ++m) {
           const int k = c * PER + m;   // even: q.k chain step k/2, odd: do.v chain step k/2
+          if (k >= 2 * KS) continue;
           fr[c % (LEAD + 1)][m] = lds_row8(((k & 1) ? Gt : Qt) + roff[k >> 1]);
         }
       };
@@ -658,6 +660,7 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
 #pragma unroll
         for (int m = 0; m < PER; ++m) {
           const int k = c * PER + m;
+          if (k >= 2 * KS) continue;
           if (k & 1) dn = mfma32(vf[k >> 1], fr[c % (LEAD + 1)][m], dn);
           else xn = mfma32(kf[k >> 1], fr[c % (LEAD + 1)][m], xn);
         }
@@ -872,8 +875,8 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
       }
     }
     Copy qcopy, gcopy;
-    qcopy.init(ptid, (unsigned)a.q.st * 2u);
-    gcopy.init(ptid, (unsigned)a.go.st * 2u);
+    qcopy.init(ptid, (unsigned)a.q.st * 2u, 2 * a.head_dim);
+    gcopy.init(ptid, (unsigned)a.go.st * 2u, 2 * a.head_dim);
     // of the current item
     Rows qrows = rows_of(a.q, cur), grows = rows_of(a.go, cur);
     int q_first = cur.kt * BKV;
@@ -962,8 +965,8 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
       unsigned short* scratch = (rw & 2 ? Gs : Qs) + (AHEAD + (rw & 1)) * QTILE;
 #pragma unroll
       for (int kb2 = 0; kb2 < 2; ++kb2) {
-        store_block32<D>(scratch, acc[kb2], mat ? a.inv_temp : 1.0f, outb, ov.st, cur.kt * BKV + 64 * half + 32 * kb2,
-                         cur.doc_len, lane_e);
+        store_block32<D, U>(scratch, acc[kb2], mat ? a.inv_temp : 1.0f, outb, ov.st, cur.kt * BKV + 64 * half + 32 * kb2,
+                         cur.doc_len, a.head_dim, lane_e);
 #pragma unroll
         for (int j = 0; j < DB; ++j)
 #pragma unroll
@@ -1000,9 +1003,9 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
 // -------------------------------------------------------------------------------------------
 template <int D> struct StreamKernel { static constexpr bool value = D > 128; };
 
-template <int D, bool AC, bool PROD, bool STREAM>
+template <int D, bool AC, bool PROD, bool STREAM, int U = D>
 __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(const KArgs a) {
-  constexpr int KS = D / 16, DB = D / 32;
+  constexpr int KS = U / 16, DB = U / 32;
   constexpr int SEG = 64;                             // STREAM: query rows per buffer
   constexpr int QROWS = STREAM ? 2 * SEG : TAIL_TILES * BKV;   // rows the buffers hold (not STREAM: every query that can follow the tile's first key)
   __shared__ __attribute__((aligned(16))) unsigned short Qs[QROWS * D];   // Q rows from the tile's first key on (swizzled like every tile)
@@ -1031,17 +1034,17 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
   const elem_t* kb = reinterpret_cast<const elem_t*>(a.k.ptr) + t.batch * a.k.sb + head * a.k.sh + tok0 * a.k.st;
   const elem_t* vb = reinterpret_cast<const elem_t*>(a.v.ptr) + t.batch * a.v.sb + head * a.v.sh + tok0 * a.v.st;
   const elem_t* gob = reinterpret_cast<const elem_t*>(a.go.ptr) + t.batch * a.go.sb + head * a.go.sh + tok0 * a.go.st;
-  const Rows qrows = make_rows(qb, a.q.st, L);
-  const Rows grows = make_rows(gob, a.go.st, L);
-  const Rows krows = make_rows(kb, a.k.st, L);
-  const Rows vrows = make_rows(vb, a.v.st, L);
+  const Rows qrows = make_rows(qb, a.q.st, L, a.head_dim);
+  const Rows grows = make_rows(gob, a.go.st, L, a.head_dim);
+  const Rows krows = make_rows(kb, a.k.st, L, a.head_dim);
+  const Rows vrows = make_rows(vb, a.v.st, L, a.head_dim);
 
   const int q_first = kt * BKV;                      // first query that can see the tile
   const int nblk = (L - q_first + 31) / 32;          // query blocks behind the tile's first key (not STREAM: 1 .. QROWS / 32)
   // all of those Q and dO rows at once, or the first block of them (rows past the document arrive as zeros)
   TileCopy<D, STREAM ? SEG : QROWS, NT, false> qcopy, gcopy;
-  qcopy.init(tid, qrows.row_bytes);
-  gcopy.init(tid, grows.row_bytes);
+  qcopy.init(tid, qrows.row_bytes, qrows.used_bytes);
+  gcopy.init(tid, grows.row_bytes, grows.used_bytes);
   qcopy.issue(qrows, q_first, Qs, STREAM ? SEG : 32 * nblk);      // (32 or 64 rows per instruction of all waves: whole query blocks)
   gcopy.issue(grows, q_first, Gs, STREAM ? SEG : 32 * nblk);
   // Wave w of workgroup b takes key block (w + b) mod 4: the block with the most queries behind it
@@ -1174,7 +1177,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
         if constexpr (DV) acc[j] = mfma32(ap, lds_tr8(Gr + yoff[0][j], Gr + yoff[1][j]), acc[j]);
         if constexpr (WHAT == 1) acc[j] = mfma32(az, lds_tr8(Qr + yoff[0][j], Qr + yoff[1][j]), acc[j]);
         if constexpr (WHAT == 2) acc2[j] = mfma32(az, lds_tr8(Qr + yoff[0][j], Qr + yoff[1][j]), acc2[j]);
-        if constexpr (D > 128) { if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0); }
+        if constexpr (D > 128) { if (j % 4 == 3 || j == DB - 1) __builtin_amdgcn_sched_barrier(0); }
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads are done before the next block overwrites the piece
@@ -1197,9 +1200,9 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
     for (int qblk = kblk; qblk < nblk; ++qblk) block(std::integral_constant<int, 2>{}, acc_v, acc_k, qblk, 32 * qblk);
     // the private piece becomes the output scratch (at most its size)
     static_assert(STREAM || 2 * 32 * 32 >= 32 * D, "the staging piece of a wave doubles as its output scratch");
-    store_block32<D>(Pt, acc_v, 1.0f, dvb, a.dv.st, k0, L, lane);
+    store_block32<D, U>(Pt, acc_v, 1.0f, dvb, a.dv.st, k0, L, a.head_dim, lane);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    store_block32<D>(Pt, acc_k, a.inv_temp, dkb, a.dk.st, k0, L, lane);
+    store_block32<D, U>(Pt, acc_k, a.inv_temp, dkb, a.dk.st, k0, L, a.head_dim, lane);
   } else {
     // Two passes over the queries, dv first and dk second; the scores are formed in each.
     // Segment s (SEG query rows) sits in buffer s & 1.  At its top every wave is done with segment s - 1,
@@ -1227,8 +1230,8 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
       }
       lds_barrier();            // every wave is done with the buffers: they become the output staging
       if (active) {
-        if constexpr (decltype(what_tag)::value == 0) store_block32<D>(scratch, acc, 1.0f, dvb, a.dv.st, k0, L, lane);
-        else store_block32<D>(scratch, acc, a.inv_temp, dkb, a.dk.st, k0, L, lane);
+        if constexpr (decltype(what_tag)::value == 0) store_block32<D, U>(scratch, acc, 1.0f, dvb, a.dv.st, k0, L, a.head_dim, lane);
+        else store_block32<D, U>(scratch, acc, a.inv_temp, dkb, a.dk.st, k0, L, a.head_dim, lane);
       }
     };
     pass(std::integral_constant<int, 0>{});
@@ -1282,9 +1285,27 @@ template __global__ void bwd_dkdv_kernel<128, false, true>(const KArgs);
 template __global__ void bwd_dkdv_kernel<128, true, false>(const KArgs);
 template __global__ void bwd_dkdv_kernel<128, true, true>(const KArgs);
 
+template __global__ void bwd_dq_kernel<128, false, true, 96>(const KArgs);
+template __global__ void bwd_dq_kernel<128, true, true, 96>(const KArgs);
+template __global__ void bwd_dq_kernel<256, false, true, 192>(const KArgs);
+template __global__ void bwd_dq_kernel<256, true, true, 192>(const KArgs);
+template __global__ void bwd_dkdv_kernel<128, false, true, 96>(const KArgs);
+template __global__ void bwd_dkdv_kernel<128, true, true, 96>(const KArgs);
+template __global__ void bwd_dkdv_tail_kernel<256, false, true, true, 192>(const KArgs);
+template __global__ void bwd_dkdv_tail_kernel<256, true, true, true, 192>(const KArgs);
+
+// Width of the narrower instantiation a kernel width has (see used_width), or the width itself.
+template <int D> constexpr int narrow_width() { return D == 128 ? 96 : D == 256 ? 192 : D; }
+
 template <int D>
 static hipError_t launch_dq_d(const KArgs& a, bool ac, bool prod, int n_q_max, hipStream_t s) {
   const dim3 grid((unsigned)n_q_max * (unsigned)a.heads), block(NT);
+  constexpr int W = narrow_width<D>();
+  if (W < D && prod && used_width(a.head_dim) == W) {
+    if (ac) hipLaunchKernelGGL((bwd_dq_kernel<D, true, true, W>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((bwd_dq_kernel<D, false, true, W>), grid, block, 0, s, a);
+    return hipGetLastError();
+  }
   if (ac) {
     if (prod) hipLaunchKernelGGL((bwd_dq_kernel<D, true, true>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((bwd_dq_kernel<D, true, false>), grid, block, 0, s, a);
@@ -1299,7 +1320,11 @@ static hipError_t launch_dq_d(const KArgs& a, bool ac, bool prod, int n_q_max, h
 template <int D, bool STREAM>
 static void launch_dkdv_four_waves(const KArgs& a, bool ac, bool prod, unsigned tiles, hipStream_t s) {
   const dim3 grid(tiles * (unsigned)a.heads), block(NT);
-  if (ac) {
+  constexpr int W = STREAM ? narrow_width<D>() : D;
+  if (W < D && prod && used_width(a.head_dim) == W) {
+    if (ac) hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, true, true, STREAM, W>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, false, true, STREAM, W>), grid, block, 0, s, a);
+  } else if (ac) {
     if (prod) hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, true, true, STREAM>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, true, false, STREAM>), grid, block, 0, s, a);
   } else {
@@ -1322,7 +1347,11 @@ static hipError_t launch_dkdv_d(const KArgs& a_in, bool ac, bool prod, int n_lon
     if (n_main > 0) {
       a.n_items = (int)(n_main * (unsigned)a.heads);
       const dim3 grid(launch_grid(a, a.n_items)), block(NT2);
-      if (ac) {
+      constexpr int W = narrow_width<D>();
+      if (W < D && prod && used_width(a.head_dim) == W) {
+        if (ac) hipLaunchKernelGGL((bwd_dkdv_kernel<D, true, true, W>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((bwd_dkdv_kernel<D, false, true, W>), grid, block, 0, s, a);
+      } else if (ac) {
         if (prod) hipLaunchKernelGGL((bwd_dkdv_kernel<D, true, true>), grid, block, 0, s, a);
         else hipLaunchKernelGGL((bwd_dkdv_kernel<D, true, false>), grid, block, 0, s, a);
       } else {
@@ -1338,6 +1367,7 @@ static hipError_t launch_dkdv_d(const KArgs& a_in, bool ac, bool prod, int n_lon
 }
 
 hipError_t launch_bwd_dq(const KArgs& a, int head_dim, bool ac, bool prod, int n_q_max, hipStream_t s) {
+  head_dim = kernel_width(head_dim);
   if (head_dim == 256) return launch_dq_d<256>(a, ac, prod, n_q_max, s);
   if (head_dim == 128) return launch_dq_d<128>(a, ac, prod, n_q_max, s);
   if (head_dim == 64) return launch_dq_d<64>(a, ac, prod, n_q_max, s);
@@ -1346,6 +1376,7 @@ hipError_t launch_bwd_dq(const KArgs& a, int head_dim, bool ac, bool prod, int n
 
 hipError_t launch_bwd_dkdv(const KArgs& a, int head_dim, bool ac, bool prod, int n_long_max, int n_last_max,
                            hipStream_t s) {
+  head_dim = kernel_width(head_dim);
   if (head_dim == 256) return launch_dkdv_d<256>(a, ac, prod, n_long_max, n_last_max, s);
   if (head_dim == 128) return launch_dkdv_d<128>(a, ac, prod, n_long_max, n_last_max, s);
   if (head_dim == 64) return launch_dkdv_d<64>(a, ac, prod, n_long_max, n_last_max, s);

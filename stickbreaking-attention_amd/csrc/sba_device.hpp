@@ -423,13 +423,14 @@ __device__ __forceinline__ void stick_weights_fwd(const f32x16& x, float c, int 
 // D/16 fully coalesced 16-byte stores per lane.  Wave-private: no workgroup barrier inside,
 // but the caller must make sure nobody else still uses the scratch memory.
 // ---------------------------------------------------------------------------------------------
-template <int D>
-__device__ __forceinline__ void store_block32(unsigned short* scratch, const f32x16 (&acc)[D / 32], float scale,
-                                              elem_t* out, int64_t stride_t, int row0, int limit, int lane) {
+// (U: columns the accumulators cover, a multiple of 32 up to the row width D of the scratch; head_dim <= U)
+template <int D, int U = D>
+__device__ __forceinline__ void store_block32(unsigned short* scratch, const f32x16 (&acc)[U / 32], float scale,
+                                              elem_t* out, int64_t stride_t, int row0, int limit, int head_dim, int lane) {
   const int n = lane & 31, h = lane >> 5;
   elem_t* sc = reinterpret_cast<elem_t*>(scratch);
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db) {
+  for (int db = 0; db < U / 32; ++db) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int row = 8 * (i >> 2) + 4 * h + (i & 3);
@@ -443,7 +444,7 @@ __device__ __forceinline__ void store_block32(unsigned short* scratch, const f32
     const int cidx = lane + 64 * j;
     const int row = cidx / C8, c8 = cidx % C8;
     const uint4 v = *reinterpret_cast<const uint4*>(scratch + row * D + c8 * 8);
-    if (row0 + row < limit) *reinterpret_cast<uint4*>(out + (int64_t)(row0 + row) * stride_t + c8 * 8) = v;
+    if (row0 + row < limit && 8 * c8 < head_dim) *reinterpret_cast<uint4*>(out + (int64_t)(row0 + row) * stride_t + c8 * 8) = v;
   }
 }
 
@@ -452,14 +453,14 @@ __device__ __forceinline__ void store_block32(unsigned short* scratch, const f32
 // (`rowscale(r)` = the fp32 factor of block row r, 0 <= r < 32, called once per 16-byte chunk).
 // The accumulators are rounded to bf16 once in the scratch, the sum is formed in fp32 and
 // rounded again: one rounding fewer than a caller adding the two bf16 tensors afterwards.
-template <int D, class RowScale>
-__device__ __forceinline__ void store_block32_axpy(unsigned short* scratch, const f32x16 (&acc)[D / 32], float scale,
-                                                   elem_t* out, int64_t stride_t, int row0, int limit, int lane,
+template <int D, int U, class RowScale>
+__device__ __forceinline__ void store_block32_axpy(unsigned short* scratch, const f32x16 (&acc)[U / 32], float scale,
+                                                   elem_t* out, int64_t stride_t, int row0, int limit, int head_dim, int lane,
                                                    const elem_t* addend, int64_t addend_stride_t, RowScale rowscale) {
   const int n = lane & 31, h = lane >> 5;
   elem_t* sc = reinterpret_cast<elem_t*>(scratch);
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db) {
+  for (int db = 0; db < U / 32; ++db) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int row = 8 * (i >> 2) + 4 * h + (i & 3);
@@ -472,7 +473,7 @@ __device__ __forceinline__ void store_block32_axpy(unsigned short* scratch, cons
   for (int j = 0; j < 32 * C8 / 64; ++j) {
     const int cidx = lane + 64 * j;
     const int row = cidx / C8, c8 = cidx % C8;
-    const bool ok = row0 + row < limit;
+    const bool ok = row0 + row < limit && 8 * c8 < head_dim;
     const float f = rowscale(row);
     const el8 mine = *reinterpret_cast<const el8*>(scratch + row * D + c8 * 8);
     el8 other;
@@ -501,16 +502,25 @@ __device__ __forceinline__ bool sub_full(int k0, int qw0) {
 // Global -> register tile loads through a buffer resource that covers exactly the rows of one
 // (document, head) slice: rows at or past the end of the document fall outside the resource
 // and the hardware returns zeros for them, so no branch and no 64-bit address arithmetic.
+//
+// A kernel of width D also serves every head_dim below it that is a multiple of 8 (one 16-byte chunk):
+// a lane whose chunk lies at or past the head_dim asks for an offset outside the resource and gets zeros
+// the same way, and the output stores leave those chunks out.  Padded copies of q, k, v, dO and slices of
+// the outputs, made by the caller, were seven extra passes with two launches each (175 of 445 us for a
+// training step of 16 heads x 7001 tokens x 96).
 // ---------------------------------------------------------------------------------------------
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 
 struct Rows {
   __amdgpu_buffer_rsrc_t rsrc;
   unsigned row_bytes;   // stride between consecutive tokens, in bytes
+  int used_bytes;       // bytes of a row that belong to this head (2 * head_dim)
 };
+constexpr int OUTSIDE = (int)0x80000000u;   // a byte offset beyond every resource (slices span less than 2 GiB)
 
-__device__ __forceinline__ Rows make_rows(const elem_t* base, int64_t stride_t, int n_rows) {
+__device__ __forceinline__ Rows make_rows(const elem_t* base, int64_t stride_t, int n_rows, int head_dim) {
   Rows r;
+  r.used_bytes = 2 * head_dim;
   const uint64_t bytes = (uint64_t)n_rows * (uint64_t)stride_t * 2u;
   r.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<elem_t*>(base), 0,
                                              bytes > 0xffffffffull ? 0xffffffffu : (unsigned)bytes, 0x00020000);
@@ -519,7 +529,8 @@ __device__ __forceinline__ Rows make_rows(const elem_t* base, int64_t stride_t, 
 }
 
 __device__ __forceinline__ uint4 load16(const Rows& r, int row, int col_bytes) {
-  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r.rsrc, row * (int)r.row_bytes + col_bytes, 0, 0);
+  const int off = col_bytes < r.used_bytes ? row * (int)r.row_bytes + col_bytes : OUTSIDE;
+  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r.rsrc, off, 0, 0);
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
@@ -599,14 +610,15 @@ struct TileCopy {
   }
 
   // gtid = index of the thread inside the group of THREADS loading threads
-  __device__ __forceinline__ void init(int gtid, unsigned row_bytes) {
+  __device__ __forceinline__ void init(int gtid, unsigned row_bytes, int used_bytes) {
     wave = __builtin_amdgcn_readfirstlane(gtid >> 6);
     const int lane = gtid & 63;
     const int m = wave * RPI + lane / C8, phys = lane % C8;
     const int logical = phys ^ swz<D>(m);
     const int src = KEYS ? ((m & ~31) | kperm(m & 31)) : m;
-    voff = src * (int)row_bytes + logical * 16;
-    voff_odd = src * (int)row_bytes + (phys ^ swz<D>(m + 8)) * 16;
+    const int odd = phys ^ swz<D>(m + 8);
+    voff = 16 * logical < used_bytes ? src * (int)row_bytes + logical * 16 : OUTSIDE;
+    voff_odd = 16 * odd < used_bytes ? src * (int)row_bytes + odd * 16 : OUTSIDE;
   }
 
   // `rows_needed` (uniform): instructions whose rows all lie at or beyond it are skipped; the tile

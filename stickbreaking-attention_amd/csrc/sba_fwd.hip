@@ -18,11 +18,12 @@ inline namespace SBA_ELEM_NS {
 // instantiations, so the production kernel (MODE 0) carries none of it.
 // head_dim 256: the ring takes 96 KiB, so one workgroup per CU and one wave per SIMD, with the whole register
 // file (512 registers per lane) for its 64 registers of Q fragments and 128 of accumulators.
-template <int D, bool AC, bool PROD, int MODE>
+// U: columns that are multiplied (see used_width); tile rows in LDS keep the width D.
+template <int D, bool AC, bool PROD, int MODE, int U = D>
 __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a) {
   constexpr bool WOUT = MODE == 1, TAB = MODE == 2;
-  constexpr int KS = D / 16;     // contraction steps of K.Q^T
-  constexpr int DB = D / 32;     // 32-wide output column blocks of P.V
+  constexpr int KS = U / 16;     // contraction steps of K.Q^T
+  constexpr int DB = U / 32;     // 32-wide output column blocks of P.V
   constexpr int BF = 32;         // keys per staged tile: one MFMA sub-block
   constexpr int TILE = BF * D;   // elements of one K or V tile (unpadded, swizzled)
   // K and V tiles of 32 keys in a three-slot ring filled by asynchronous global -> LDS copies:
@@ -45,7 +46,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
       int row0, row1;
       unsigned pair;
       spare_rows(refused, slot, hdr.y, sched[SCHED_TOTAL], a.tokens, a.nan_pair, row0, row1, pair);
-      fill_rows16(a.o, head, row0, row1, D, pair, threadIdx.x, NT);
+      fill_rows16(a.o, head, row0, row1, a.head_dim, pair, threadIdx.x, NT);
       fill_rows16(a.rem, head, row0, row1, 1, pair, threadIdx.x, NT);
     }
     return;
@@ -65,9 +66,9 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
   const elem_t* vb = reinterpret_cast<const elem_t*>(a.v.ptr) + t.batch * a.v.sb + head * a.v.sh + tok0 * a.v.st;
   elem_t* ob = reinterpret_cast<elem_t*>(a.o.ptr) + t.batch * a.o.sb + head * a.o.sh + tok0 * a.o.st;
   elem_t* rb = reinterpret_cast<elem_t*>(a.rem.ptr) + t.batch * a.rem.sb + head * a.rem.sh + tok0 * a.rem.st;
-  const Rows qrows = make_rows(qb, a.q.st, t.doc_len);
-  const Rows krows = make_rows(kb, a.k.st, t.doc_len);
-  const Rows vrows = make_rows(vb, a.v.st, t.doc_len);
+  const Rows qrows = make_rows(qb, a.q.st, t.doc_len, a.head_dim);
+  const Rows krows = make_rows(kb, a.k.st, t.doc_len, a.head_dim);
+  const Rows vrows = make_rows(vb, a.v.st, t.doc_len, a.head_dim);
 
   const int last_key = min(m0 + BM - 1, t.doc_len - 1);
   const int kt_last = last_key / BF;
@@ -83,8 +84,8 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
   constexpr int CT = D == 32 ? NT / 2 : NT;   // threads that copy tiles
   const bool copier = tid < CT;               // (uniform per wave)
   TileCopy<D, BF, CT, true> kcopy, vcopy;
-  kcopy.init(tid, krows.row_bytes);
-  vcopy.init(tid, vrows.row_bytes);
+  kcopy.init(tid, krows.row_bytes, krows.used_bytes);
+  vcopy.init(tid, vrows.row_bytes, vrows.used_bytes);
   constexpr int LOADS_PER_TILE = (TAB ? 1 : 2) * TileCopy<D, BF, CT, true>::NCH;
   if (copier) {
     kcopy.issue(krows, kt_last * BF, Ks);
@@ -211,10 +212,10 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
   lds_barrier();   // every wave is done with the K/V tiles: their memory becomes the o staging area
   if (a.fuse) {
     // what every caller computes next (upstream tests/test_varlen.py:101): o + rem * v
-    store_block32_axpy<D>(smem + w * 32 * D, oacc, 1.0f, ob, a.o.st, qw0, t.doc_len, lane, vb, a.v.st,
+    store_block32_axpy<D, U>(smem + w * 32 * D, oacc, 1.0f, ob, a.o.st, qw0, t.doc_len, a.head_dim, lane, vb, a.v.st,
                           [&](int row) { return __shfl(r, row, 64); });
   } else {
-    store_block32<D>(smem + w * 32 * D, oacc, 1.0f, ob, a.o.st, qw0, t.doc_len, lane);
+    store_block32<D, U>(smem + w * 32 * D, oacc, 1.0f, ob, a.o.st, qw0, t.doc_len, a.head_dim, lane);
   }
 }
 
@@ -269,6 +270,19 @@ template __global__ void fwd_kernel<256, false, true, 2>(const KArgs);
 template __global__ void fwd_kernel<256, true, false, 2>(const KArgs);
 template __global__ void fwd_kernel<256, true, true, 2>(const KArgs);
 
+template __global__ void fwd_kernel<128, false, true, 0, 96>(const KArgs);
+template __global__ void fwd_kernel<128, true, true, 0, 96>(const KArgs);
+template __global__ void fwd_kernel<256, false, true, 0, 192>(const KArgs);
+template __global__ void fwd_kernel<256, true, true, 0, 192>(const KArgs);
+
+template <int D, int U>
+static hipError_t launch_fwd_narrow(const KArgs& a, bool ac, int n_q_max, hipStream_t s) {
+  const dim3 grid((unsigned)n_q_max * (unsigned)a.heads), block(NT);
+  if (ac) hipLaunchKernelGGL((fwd_kernel<D, true, true, 0, U>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((fwd_kernel<D, false, true, 0, U>), grid, block, 0, s, a);
+  return hipGetLastError();
+}
+
 template <int D, int MODE>
 static hipError_t launch_fwd_d(const KArgs& a, bool ac, bool prod, int n_q_max, hipStream_t s) {
   const dim3 grid((unsigned)n_q_max * (unsigned)a.heads), block(NT);
@@ -284,6 +298,12 @@ static hipError_t launch_fwd_d(const KArgs& a, bool ac, bool prod, int n_q_max, 
 
 // mode: 0 = o and rem (and the table when one is given), 1 = the attention weights as well, 2 = the table alone
 hipError_t launch_fwd(const KArgs& a, int head_dim, bool ac, bool prod, int mode, int n_q_max, hipStream_t s) {
+  if (mode == 0 && prod) {
+    const int u = used_width(head_dim);
+    if (u == 96) return launch_fwd_narrow<128, 96>(a, ac, n_q_max, s);
+    if (u == 192) return launch_fwd_narrow<256, 192>(a, ac, n_q_max, s);
+  }
+  head_dim = kernel_width(head_dim);
   if (mode == 1) {
     if (head_dim == 256) return launch_fwd_d<256, 1>(a, ac, prod, n_q_max, s);
     if (head_dim == 128) return launch_fwd_d<128, 1>(a, ac, prod, n_q_max, s);

@@ -21,6 +21,7 @@ struct KArgs {
   float* weights;              // forward, debug variant only: dense attention weights
                                // [batch][heads][tokens][tokens] (row = query token, column = key token)
   int heads;
+  int head_dim;                // a multiple of 8, at most the width D of the kernel (see make_rows)
   int tokens;                  // tokens per batch entry
   int fuse;                    // the output is o + rem * v (and grad_o is the gradient of that)
   int clear_spare;             // packed input: spare workgroups clear the rows that belong to no document (or fill
@@ -97,6 +98,16 @@ inline DkdvGrid dkdv_grid(bool has_tail_kernel, int n_long_max, int n_last_max, 
                                  : (n_long_max + n_last_max < n_kv_alloc ? n_long_max + n_last_max : n_kv_alloc);
   g.tail_tiles = has_tail_kernel ? n_last_max : 0;
   return g;
+}
+// Width of the kernels a head_dim runs on.
+inline int kernel_width(int head_dim) { return head_dim <= 32 ? 32 : head_dim <= 64 ? 64 : head_dim <= 128 ? 128 : 256; }
+// Columns the product-space kernels multiply.  A head_dim in the lower half of a width's range would leave up to half of
+// the matrix instructions multiplying zeros, so the two wide kernels exist with three quarters of theirs as
+// well (same tiles in LDS, fewer contraction steps and output columns); below 64 a call is not bound by them.
+inline int used_width(int head_dim) {
+  if (head_dim > 64 && head_dim <= 96) return 96;
+  if (head_dim > 128 && head_dim <= 192) return 192;
+  return kernel_width(head_dim);
 }
 inline bool has_dkdv_tail_kernel(int head_dim) { return head_dim <= 64; }
 

@@ -88,7 +88,7 @@ sba_problem problem(const Tensor& q, const Call& c) {
   return p;
 }
 
-// Element type `dt`, head_dim padded with zeros to `dpad`, unit inner stride, other strides multiples of
+// Element type `dt`, head_dim padded with zeros to `dpad` (the next multiple of 8), unit inner stride, other strides multiples of
 // 8 elements, 16-byte aligned rows.
 Tensor prepared(Tensor t, int64_t dpad, at::ScalarType dt) {
   if (t.scalar_type() != dt) t = t.to(dt);
@@ -102,9 +102,8 @@ Tensor prepared(Tensor t, int64_t dpad, at::ScalarType dt) {
 }
 
 int64_t padded_dim(int64_t d) {
-  for (int64_t s : {32, 64, 128, 256})
-    if (d <= s) return s;
-  TORCH_CHECK_VALUE(false, "head_dim ", d, " is not supported (maximum 256)");
+  TORCH_CHECK_VALUE(d <= 256, "head_dim ", d, " is not supported (maximum 256)");
+  return (d + 7) & ~int64_t(7);   // (rows of 16-byte chunks; the kernels take every multiple of 8)
 }
 
 at::ScalarType compute_type(at::ScalarType t) { return t == at::kHalf ? at::kHalf : at::kBFloat16; }

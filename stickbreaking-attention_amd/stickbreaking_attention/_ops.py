@@ -56,7 +56,7 @@ RECOMPUTE_TABLE = os.environ.get("SBA_RECOMPUTE_TABLE", "0") == "1"
 # to a maximum between 4 and 8 by a power of two before it is rounded and the gradients are scaled back (exact).
 F32_AS_F16 = os.environ.get("SBA_F32_AS_F16", "0") == "1"
 
-SUPPORTED_HEAD_DIMS = (32, 64, 128, 256)
+MAX_HEAD_DIM = 256
 
 # Tile sizes the library's workspace formulas are built on (query tile, dk/dv key tile, table block).
 _BM, _BKV, _BT, _SCHED_HDR, _TILE_WORDS = 128, 128, 32, 16, 8
@@ -64,10 +64,10 @@ _WORK_WORDS = 64      # words at the end of every carry table: the work counters
 
 
 def _padded_dim(d: int) -> int:
-    for s in SUPPORTED_HEAD_DIMS:
-        if d <= s:
-            return s
-    raise ValueError(f"head_dim {d} is not supported (maximum {SUPPORTED_HEAD_DIMS[-1]})")
+    """The library takes every multiple of 8 (rows of 16-byte chunks)."""
+    if d > MAX_HEAD_DIM:
+        raise ValueError(f"head_dim {d} is not supported (maximum {MAX_HEAD_DIM})")
+    return -(-d // 8) * 8
 
 
 def table_entries(length: int) -> int:
