@@ -230,6 +230,25 @@ int sba_attn_bwd(const sba_problem* p, const void* schedule, size_t schedule_siz
                  const sba_view* dq, const sba_view* dk, const sba_view* dv,
                  void* stream);
 
+/* The backward in one pass: every score is formed once, dq is handed from key tile to key tile through scratch
+ * memory (csrc/sba_chain.hip).  For the problems it is the faster form of, sba_chain_scratch_bytes
+ * returns the scratch it needs (16-byte aligned, contents irrelevant, one per concurrent call) and 0 for every other;
+ * a caller then takes sba_varlen_bwd / sba_attn_bwd.  Same inputs, outputs, table and refusals; it
+ * needs no gradient table, and the results differ from the two-pass form's by rounding.  Problems it
+ * cannot take (log-space carry, head_dim <= 32 or > 128, a device that is not eight XCDs of 32 compute units)
+ * return SBA_E_SHAPE.  The stream's CU mask, if it has one, must leave every XCD at least one CU. */
+size_t sba_chain_scratch_bytes(const sba_problem* p);
+int sba_varlen_bwd_chained(const sba_problem* p, const void* schedule, size_t schedule_size,
+                           const sba_view* q, const sba_view* k, const sba_view* v,
+                           const sba_view* grad_o, const sba_view* grad_rem,
+                           const float* stick_table, size_t table_size, void* scratch, size_t scratch_size,
+                           const sba_view* dq, const sba_view* dk, const sba_view* dv, void* stream);
+int sba_attn_bwd_chained(const sba_problem* p, const void* schedule, size_t schedule_size,
+                         const sba_view* q, const sba_view* k, const sba_view* v,
+                         const sba_view* grad_o, const sba_view* grad_rem,
+                         const float* stick_table, size_t table_size, void* scratch, size_t scratch_size,
+                         const sba_view* dq, const sba_view* dk, const sba_view* dv, void* stream);
+
 /* ---- misc ------------------------------------------------------------------------------- */
 
 /* Launch geometry of a problem: host arithmetic only, nothing is launched and no device is
@@ -275,6 +294,10 @@ float sba_last_kernel_ms(int which);
  * tile.  The results do not depend on it (every tile is computed by the same instructions in the
  * same order whichever workgroup takes it). */
 void  sba_set_dkdv_workgroups(int n);
+
+/* Test and tuning switch (process-wide): which form of the backward sba_chain_scratch_bytes asks for.  0: by size,
+ * 1: never the one-pass form, 2: wherever it is possible. */
+void  sba_set_backward_form(int form);
 
 #ifdef __cplusplus
 }

@@ -17,6 +17,7 @@ using namespace sba;
 // Process-wide on purpose: PyTorch runs the backward on its own autograd thread.
 std::atomic<int> g_timing{0};
 std::atomic<int> g_dkdv_workgroups{0};   // sba_set_dkdv_workgroups
+std::atomic<int> g_backward_form{0};     // sba_set_backward_form
 std::atomic<float> g_ms[3];
 
 inline int cdiv_i(long long a, long long b) { return (int)((a + b - 1) / b); }
@@ -281,6 +282,105 @@ int backward(const sba_problem* p, bool fixed, const void* schedule, size_t sche
   return (int)he;
 }
 
+// ---- the one-pass backward (sba_chain.hip) ------------------------------------------------------------
+struct ChainScratch { size_t partial, carry, flags, queues, total; };   // byte offsets
+ChainScratch chain_scratch(const sba_problem* p, const Sizes& sz) {
+  const size_t tiles = (size_t)p->heads * (size_t)sz.n_kv_max;
+  auto line = [](size_t n) { return (n + 255) & ~(size_t)255; };
+  ChainScratch c;
+  c.partial = 0;
+  c.carry = line(tiles * BM * kernel_width(p->head_dim) * sizeof(float));
+  c.flags = c.carry + line(2 * tiles * BM * sizeof(float));
+  c.queues = c.flags + line(tiles * sizeof(int));
+  c.total = c.queues + line(CHAIN_QUEUES * CHAIN_QUEUE_STRIDE * sizeof(unsigned));
+  return c;
+}
+
+// Whether the kernels can take the problem at all: eight XCDs whose queues are all served (a grid of one workgroup
+// per compute unit reaches every XCD), ranked documents, room for the queue's groups in LDS and 32-bit
+// offsets into a document's partial dq.
+bool chain_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
+  const long long chains = (long long)sz.n_docs * p->heads;
+  return (p->flags & SBA_PRODUCT_SPACE) && (kernel_width(p->head_dim) == 128 || kernel_width(p->head_dim) == 64) && sz.n_docs > 0 && sz.n_docs <= RANK_LIMIT &&
+         chains <= (long long)CHAIN_QUEUES * CHAIN_GROUP * CHAIN_MAX_GROUPS &&
+         ((long long)declared_max_doc_len(p, fixed) + BM) * kernel_width(p->head_dim) * 4 < (1ll << 31) && device_cus() == 256;
+}
+// Where the one-pass form is the faster one (gain over the two passes, measured on 270 problems of 1 to 32 heads and
+// 512 to 16 K tokens in 1 to 128 documents, declared lengths exact).
+bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
+  const int form = g_backward_form.load();
+  if (form == 1 || g_dkdv_workgroups.load() != 0 || !chain_possible(p, fixed, sz)) return false;
+  if (form == 2) return true;
+  const long long chains = (long long)sz.n_docs * p->heads, items = (long long)sz.n_kv_max * p->heads;
+  const long long mean = sz.rows / sz.n_docs, longest = declared_max_doc_len(p, fixed);
+  // a document of one or two steps: nothing to hand on, and one launch more (0.85 .. 1.01)
+  if (longest <= 64) return false;
+  // Every chain stays on one XCD.  While an XCD holds all its tiles at once (32 CUs, 4096 keys) how the chains fall on the
+  // XCDs does not matter (1.1 .. 1.4, one chain alone included); beyond, the XCDs have to come out even: no more than a tenth idle
+  // in the last round (12 chains of 4096 and more: 0.87 .. 0.95), and no chain longer than its share of the whole (one
+  // of 8192 next to seven short ones: 0.89).
+  const long long per_xcd = (chains + CHAIN_QUEUES - 1) / CHAIN_QUEUES;
+  if (per_xcd * longest > 32 * BKV) {
+    if (10 * chains < 9 * CHAIN_QUEUES * per_xcd) return false;
+    if (longest > 32 * BKV && chains * mean * mean < (CHAIN_QUEUES + 4) * longest * longest) return false;
+  }
+  // Width 128 gains from there on (1.03 .. 1.38; 0.96 where every document ends in a nearly empty tile).  At width 64 what
+  // an item costs before its first step weighs twice as much: with several items per CU only documents of
+  // some length gain (512 long: 0.90 .. 1.16, 768: 1.03 .. 1.42).
+  if (kernel_width(p->head_dim) == 128) return true;
+  return mean >= 5 * BKV || (longest >= BKV && items <= 512) || (mean >= 3 * BKV && items <= 1024);
+}
+
+int backward_chained(const sba_problem* p, bool fixed, const void* schedule, size_t sched_bytes, const sba_view* q,
+                     const sba_view* k, const sba_view* v, const sba_view* go, const sba_view* grem, const float* stick,
+                     size_t table_bytes, void* scratch, size_t scratch_bytes, const sba_view* dq, const sba_view* dk,
+                     const sba_view* dv, void* stream) {
+  Sizes sz;
+  int e = check_problem(p, fixed, &sz);
+  if (e) return e;
+  if ((e = check_mat(q, p)) || (e = check_mat(k, p)) || (e = check_mat(v, p)) || (e = check_mat(go, p)) ||
+      (e = check_mat(dq, p)) || (e = check_mat(dk, p)) || (e = check_mat(dv, p)))
+    return e;
+  if (stick == nullptr || scratch == nullptr) return SBA_E_NULL;
+  KArgs c;
+  std::memset(&c, 0, sizeof(c));
+  if ((e = fill_common(p, fixed, sz, schedule, sched_bytes, true, table_bytes, &c))) return e;
+  const ChainScratch at = chain_scratch(p, sz);
+  if (scratch_bytes < at.total || (reinterpret_cast<uintptr_t>(scratch) & 15)) return SBA_E_WORKSPACE;
+  if ((e = check_arch())) return e;
+  if (sz.rows == 0) return 0;
+  if (!chain_possible(p, fixed, sz)) return SBA_E_SHAPE;
+  ChainArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.q = to_view(q); a.k = to_view(k); a.v = to_view(v); a.go = to_view(go); a.grem = to_view(grem);
+  a.dq = to_view(dq); a.dk = to_view(dk); a.dv = to_view(dv);
+  a.sched = c.sched;
+  a.stick = stick;
+  char* const base = static_cast<char*>(scratch);
+  a.partial = reinterpret_cast<float*>(base + at.partial);
+  a.carry = reinterpret_cast<float*>(base + at.carry);
+  a.flags = reinterpret_cast<int*>(base + at.flags);
+  a.queues = reinterpret_cast<unsigned*>(base + at.queues);
+  a.tab_stride = c.tab_stride;
+  a.docs_off = SCHED_HDR + TILE_WORDS * (sz.n_q_max + sz.n_kv_max) + chain_docs_offset(sz.n_docs);
+  a.n_docs = sz.n_docs;
+  a.heads = p->heads;
+  a.head_dim = p->head_dim;
+  a.tokens = p->tokens;
+  a.tiles = sz.n_kv_max;
+  a.fixed = fixed ? 1 : 0;
+  a.fuse = c.fuse;
+  a.clear_spare = fixed ? 0 : 1;
+  a.nan_pair = p->dtype == SBA_F16 ? 0x7e007e00u : 0x7fc07fc0u;
+  a.max_doc_len = declared_max_doc_len(p, fixed);
+  a.c = c.c;
+  a.inv_temp = c.inv_temp;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  Timer tm(2, s);
+  return (int)(p->dtype == SBA_F16 ? f16::launch_bwd_chain : bf16::launch_bwd_chain)(a, (p->flags & SBA_ATTEND_CURRENT) != 0, sz.n_q_max,
+                                                                                    device_cus(), s);
+}
+
 // Schedule workspace of sba_varlen_fwd_static: one array per GPU, inside the code object, so the
 // entry point needs no allocation.  In host code the name `scratch` is only a handle for
 // hipGetSymbolAddress; kernels get the device address looked up once per device.
@@ -420,6 +520,29 @@ int sba_attn_bwd(const sba_problem* p, const void* schedule, size_t schedule_siz
                   dq, dk, dv, stream);
 }
 
+size_t sba_chain_scratch_bytes(const sba_problem* p) {
+  Sizes sz;
+  const bool fixed = p != nullptr && (p->flags & SBA_FIXED_LENGTH) != 0;
+  if (check_problem(p, fixed, &sz) || !chain_wanted(p, fixed, sz)) return 0;
+  return chain_scratch(p, sz).total;
+}
+
+int sba_varlen_bwd_chained(const sba_problem* p, const void* schedule, size_t schedule_size, const sba_view* q,
+                           const sba_view* k, const sba_view* v, const sba_view* grad_o, const sba_view* grad_rem,
+                           const float* stick_table, size_t table_size, void* scratch, size_t scratch_size,
+                           const sba_view* dq, const sba_view* dk, const sba_view* dv, void* stream) {
+  return backward_chained(p, false, schedule, schedule_size, q, k, v, grad_o, grad_rem, stick_table, table_size, scratch, scratch_size,
+                          dq, dk, dv, stream);
+}
+
+int sba_attn_bwd_chained(const sba_problem* p, const void* schedule, size_t schedule_size, const sba_view* q,
+                         const sba_view* k, const sba_view* v, const sba_view* grad_o, const sba_view* grad_rem,
+                         const float* stick_table, size_t table_size, void* scratch, size_t scratch_size,
+                         const sba_view* dq, const sba_view* dk, const sba_view* dv, void* stream) {
+  return backward_chained(p, true, schedule, schedule_size, q, k, v, grad_o, grad_rem, stick_table, table_size, scratch, scratch_size,
+                          dq, dk, dv, stream);
+}
+
 int sba_varlen_fwd_static(const sba_problem* p, const sba_view* q, const sba_view* k, const sba_view* v,
                           const sba_view* o, const sba_view* rem, void* stream) {
   Sizes sz;
@@ -461,6 +584,7 @@ int sba_launch_geometry(const sba_problem* p, sba_geometry* out) {
 
 void sba_set_timing(int on) { g_timing.store(on); }
 void sba_set_dkdv_workgroups(int n) { g_dkdv_workgroups.store(n); }
+void sba_set_backward_form(int form) { g_backward_form.store(form); }
 float sba_last_kernel_ms(int which) {
   if (which < 0 || which >= 3) return 0.f;
   std::lock_guard<std::mutex> lock(g_ev_mutex);

@@ -1,0 +1,746 @@
+// Backward in one pass: dq, dk and dv of long documents by workgroups that hand their queries' partial
+// results from key tile to key tile.
+//
+// The two-pass backward (sba_bwd.hip) forms every score twice, once for dq and once for dk / dv, because
+// dq is summed over keys and dk, dv over queries: 56 matrix instructions per 32 x 32 block at head_dim 128
+// and the vector work of the weights and of dz twice.  One pass needs 40 and does the vector work once, but
+// one of the two sums then crosses workgroups.  fp32 atomics are out (1.36 TB/s of payload on
+// this part, see sba_bwd.hip).  Here a workgroup owns 128 keys of one (document, head) -- dk and dv stay in
+// registers -- and dq of 32 queries at a time is handed on: the workgroup of key tile c takes the partial
+// sum that tile c - 1 left in scratch memory, adds its own keys on the matrix cores and leaves it for tile
+// c + 1; the tile that holds the queries' own keys writes dq.  The running sum along the keys that
+// dz needs travels the same way, so the gradient table of the two-pass form and the pass that fills it are gone.
+//
+// What makes this affordable is the XCD's L2: 16 KiB in and out per 32 queries is 8 TB/s over the chip, which the
+// L2s deliver (11 TB/s each way measured with plain stores and one chain per XCD; 1.9 TB/s with
+// stores that write through to memory, as a hand-over between XCDs would need).  So all key tiles of a
+// (document, head) -- a chain -- run on one XCD: a workgroup reads which XCD it is on (XCC_ID) and draws its
+// items from that XCD's queue.  Every CU of an XCD shares that XCD's L2 and L1 is write-through, so a
+// store is visible to the XCD's other CUs when vmcnt says it has been acknowledged; consumers read with sc1,
+// which L1 does not answer.
+//
+// Order and progress.  Queries are walked from the document's end down to the tile's own keys, so that the
+// tiles of a chain start together and end one after the other; the items of a queue are ordered by key tile, so
+// the item an item waits for was drawn before it by a workgroup that is running: waits end.  A tile is
+// published three steps after it was formed (`flags`: steps done per item).
+//
+// Measured (kernel time of the backward, two passes -> prep and chain; MI355X): 32 heads x 16 K tokens in eight documents,
+// head_dim 128, 1606 -> 1388 us; 12 x 4 x 4096 fused 837 -> 750; 16 x 7001 in six documents, head_dim 96, 225 -> 174; 4 x 16 x
+// 2048, head_dim 64, 234 -> 222; 1 x 4 x 512, head_dim 64, 42 -> 31.  At head_dim 128 what bounds it is the partial dq
+// that does not stay in L2 (5.1 GB fetched and 3.3 GB written of 8.6 GB each way in the first of these) and the
+// steps' barriers: 2860 cycles per step where the score waves and the product waves issue for 2350 each.
+//
+// Carried sum: with C[j] the sum of G over the keys up to j and ex the stick on entering a key, D = C + drem ex
+// obeys D[j] = D[j-1] + p_j (do.v_j) and dz_j = r_j D[j] - D[j-1] (see grad_dz in sba_bwd.hip); the gradient of
+// rem enters only through the value in front of the row's oldest key, D = drem * rem (chain_prep_kernel).
+#include <type_traits>
+
+#include "sba_kernels.hpp"
+
+namespace sba {
+inline namespace SBA_ELEM_NS {
+
+// Rows of one 32-row fp32 block of partial dq: four dwordx4 per lane.
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+// Ahead of the main kernel: clears the flags and the queues, forms D in front of the oldest key of every row, and
+// writes the rows that belong to no document (or NaN everywhere when the launch is refused).  One
+// workgroup per query tile and head.
+template <int D>
+__global__ void __launch_bounds__(NT) chain_prep_kernel(const ChainArgs a) {
+  const int* sched = a.sched;
+  const int slot = blockIdx.x / a.heads;
+  const int head = blockIdx.x - slot * a.heads;
+  const int4 hdr = *reinterpret_cast<const int4*>(sched);   // status, query tiles, key tiles, table entries needed
+  const Tile t = reinterpret_cast<const Tile*>(sched + SCHED_HDR)[slot];
+  asm volatile("" ::"s"(t.tok_start), "s"(t.doc_len), "s"(t.idx), "s"(t.batch), "s"(t.tab_base));
+  const bool refused = hdr.x != 0 || hdr.w > a.tab_stride || sched[SCHED_MAXLEN] > a.max_doc_len;
+  const int tid = threadIdx.x;
+  if (blockIdx.x == 0 && tid < CHAIN_QUEUES * CHAIN_QUEUE_STRIDE) a.queues[tid] = 0u;
+  if (tid == 0) a.flags[head * a.tiles + slot] = 0;
+  if (refused || slot >= hdr.y) {
+    if (a.clear_spare) {
+      int row0, row1;
+      unsigned pair;
+      spare_rows(refused, slot, hdr.y, sched[SCHED_TOTAL], a.tokens, a.nan_pair, row0, row1, pair);
+      fill_rows16(a.dq, head, row0, row1, a.head_dim, pair, tid, NT);
+      fill_rows16(a.dk, head, row0, row1, a.head_dim, pair, tid, NT);
+      fill_rows16(a.dv, head, row0, row1, a.head_dim, pair, tid, NT);
+    }
+    return;
+  }
+  __shared__ float dots[BM];
+  const int row0 = t.idx * BM;
+  const int n_rows = min(BM, t.doc_len - row0);
+  const int64_t tok0 = t.tok_start + row0;
+  if (a.fuse) {   // d(rem) = do . v_row as well (see bwd_dq_kernel): 16-byte chunks, the lanes of a row next to one another
+    constexpr int LPR = D / 8 < 16 ? D / 8 : 16;    // lanes per row
+    const elem_t* gb = reinterpret_cast<const elem_t*>(a.go.ptr) + t.batch * a.go.sb + head * a.go.sh + tok0 * a.go.st;
+    const elem_t* vb = reinterpret_cast<const elem_t*>(a.v.ptr) + t.batch * a.v.sb + head * a.v.sh + tok0 * a.v.st;
+    const int sub = tid % LPR;
+    for (int r = tid / LPR; r < BM; r += NT / LPR) {
+      float dot = 0.0f;
+      if (r < n_rows && 8 * sub < a.head_dim) {
+        const el8 g = *reinterpret_cast<const el8*>(gb + r * a.go.st + 8 * sub);
+        const el8 v = *reinterpret_cast<const el8*>(vb + r * a.v.st + 8 * sub);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dot = fmaf((float)g[e], (float)v[e], dot);
+      }
+#pragma unroll
+      for (int m = LPR / 2; m > 0; m >>= 1) dot += __shfl_xor(dot, m, 64);
+      if (sub == 0) dots[r] = dot;
+    }
+    __syncthreads();
+  }
+  if (tid < n_rows) {
+    float dr = a.fuse ? dots[tid] : 0.0f;
+    if (a.grem.ptr != nullptr)
+      dr += (float)(reinterpret_cast<const elem_t*>(a.grem.ptr) + t.batch * a.grem.sb + head * a.grem.sh + tok0 * a.grem.st)[(int64_t)tid * a.grem.st];
+    const float rem = a.stick[(int64_t)head * a.tab_stride + t.tab_base + tab_rowplane32(t.doc_len) + row0 + tid];
+    a.carry[((int64_t)head * a.tiles + t.tile_base) * BM + row0 + tid] = dr * rem;
+  }
+}
+
+// NSQ: 32-query blocks per step.  4 * NSQ score waves (one per 32-key block and query block) and 4 product waves.
+template <int D, int U, bool AC, int NSQ>
+__global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const ChainArgs a) {
+  constexpr int KS = U / 16, DB = U / 32;
+  constexpr int TQ = 32 * NSQ;      // queries per step
+  constexpr int RING = 6;           // Q / dO slots: tiles w-1 (dk) .. w+2 (scores) of step w and two in flight
+  constexpr int AHEAD = 4;
+  constexpr int QTILE = TQ * D, PTILE = TQ * BKV;
+  constexpr int DIAG = BKV / TQ;    // steps of an item whose queries may not see all of its keys: its last ones
+  __shared__ __attribute__((aligned(16))) unsigned short Qs[RING * QTILE];
+  __shared__ __attribute__((aligned(16))) unsigned short Gs[RING * QTILE];
+  __shared__ __attribute__((aligned(16))) unsigned short PZ[5 * PTILE];   // p: three buffers, dz: two buffers, [query][key]
+  __shared__ float tot[2][NSQ][4][32];       // by step parity: every key block's sum of p (do.v) per query
+  __shared__ int prefix[CHAIN_MAX_GROUPS];   // items of this XCD's queue up to and including each group
+  __shared__ int mbox[2][8];
+  __shared__ __attribute__((aligned(16))) unsigned short spare[4][512];   // where a product wave's copies of nothing go
+  unsigned short* const Ps = PZ;
+  unsigned short* const Zs = PZ + 3 * PTILE;
+  static_assert(5 * PTILE >= BKV * D, "the key tile is staged in the p / dz buffers between items");
+
+  const int* sched = a.sched;
+  const int4 hdr = *reinterpret_cast<const int4*>(sched);
+  if (hdr.x != 0 || hdr.w > a.tab_stride || sched[SCHED_MAXLEN] > a.max_doc_len) return;
+
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, n = lane & 31, h = lane >> 5;
+  const int i16 = lane & 15, blk = (lane >> 4) & 1;
+  const bool scorer = w < 4 * NSQ;
+
+  struct Item { int kt, head, tok_start, doc_len, tab_base, tile_base, batch; };
+  const int2* const docs = reinterpret_cast<const int2*>(sched + a.docs_off);   // per rank: {token start, length}, {table base, tile base}
+  const int n_chains = a.n_docs * a.heads;
+  const int head_dim = a.head_dim;
+  auto rows_of = [head_dim](const View& v, const Item& it) {
+    return make_rows(reinterpret_cast<const elem_t*>(v.ptr) + it.batch * v.sb + it.head * v.sh + (int64_t)it.tok_start * v.st,
+                     v.st, it.doc_len, head_dim);
+  };
+  auto read_box = [&](int parity, Item& it) {
+    it.kt = __builtin_amdgcn_readfirstlane(mbox[parity][0]);
+    it.head = __builtin_amdgcn_readfirstlane(mbox[parity][1]);
+    it.tok_start = __builtin_amdgcn_readfirstlane(mbox[parity][2]);
+    it.doc_len = __builtin_amdgcn_readfirstlane(mbox[parity][3]);
+    it.tab_base = __builtin_amdgcn_readfirstlane(mbox[parity][4]);
+    it.tile_base = __builtin_amdgcn_readfirstlane(mbox[parity][5]);
+    it.batch = __builtin_amdgcn_readfirstlane(mbox[parity][6]);
+    return it.kt >= 0;
+  };
+  // Q and dO rows, which every key tile of the chain reads again, stream past L2's partial sums of dq: those are written
+  // back and fetched again where they do not stay (1.50 -> 1.41 ms on 32 heads x 16 K tokens in 8 documents)
+  using Copy = TileCopy<D, TQ, 256, false, true>;
+  constexpr int LOADS_PER_TILE = 2 * Copy::NCH;
+
+  // ---- the queue of this XCD ---------------------------------------------------------------------
+  // Chains (document rank, head), longest documents first, are dealt to the XCDs in turn.  An XCD's chains are taken in
+  // groups of CHAIN_GROUP whose key tiles are interleaved (tile 0 of each, tile 1 of each, ...), so that the
+  // tiles that start together at the beginning of a launch have few predecessors to wait for.  Ticket
+  // numbers run over the groups' items; a group has room for its longest chain, the tickets behind a
+  // shorter one's end name no item and are drawn past.
+  const int xcd = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & (CHAIN_QUEUES - 1);   // HW_REG_XCC_ID, bits 3:0
+  unsigned* const ctr = a.queues + xcd * CHAIN_QUEUE_STRIDE;
+  const int n_groups = (n_chains + CHAIN_QUEUES * CHAIN_GROUP - 1) / (CHAIN_QUEUES * CHAIN_GROUP);
+  auto group_items = [&](int g) {   // room of group g: its first chain belongs to its longest document
+    if (g >= n_groups) return 0;
+    const int len = docs[2 * (CHAIN_QUEUES * CHAIN_GROUP * g / a.heads)].y;
+    return CHAIN_GROUP * ((len + BKV - 1) / BKV);
+  };
+  // first score wave: the item of a ticket, or the items of further tickets, as `mbox` words of the lanes 0 .. 7
+  auto resolve = [&](unsigned ticket) -> int {
+    for (;;) {
+      const int tk = __builtin_amdgcn_readfirstlane((int)ticket);
+      int group = -1, before = 0;
+      for (int g0 = 0; g0 < n_groups; g0 += 64) {
+        const int upto = g0 + lane < n_groups ? prefix[g0 + lane] : 0x7fffffff;
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(tk < upto && g0 + lane < n_groups);
+        if (m != 0) {
+          group = g0 + __builtin_ctzll(m);
+          break;
+        }
+      }
+      if (group < 0) return -1;
+      before = group > 0 ? __builtin_amdgcn_readfirstlane(prefix[group - 1]) : 0;
+      const int rel = tk - before;
+      const int kt = rel / CHAIN_GROUP;
+      const int chain = CHAIN_QUEUES * (CHAIN_GROUP * group + rel % CHAIN_GROUP) + xcd;
+      if (chain < n_chains) {
+        const int rank = chain / a.heads;
+        const int2 d0 = docs[2 * rank], d1 = docs[2 * rank + 1];
+        if (kt * BKV < d0.y) {
+          int v = kt;
+          v = lane == 1 ? chain - rank * a.heads : v;
+          v = lane == 2 ? d0.x : v;
+          v = lane == 3 ? d0.y : v;
+          v = lane == 4 ? d1.x : v;
+          v = lane == 5 ? d1.y : v;
+          v = lane == 6 ? (a.fixed ? rank : 0) : v;
+          return v;
+        }
+      }
+      unsigned next = 0;
+      if (lane == 0) next = atomicAdd(ctr, 1u);
+      ticket = next;
+    }
+  };
+  if (w == 0) {
+    unsigned ticket = 0;
+    if (lane == 0) ticket = atomicAdd(ctr, 1u);
+    int base = 0;
+    for (int g0 = 0; g0 < n_groups; g0 += 64) {
+      int v = group_items(g0 + lane);
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(v, o, 64);
+        if (lane >= o) v += u;
+      }
+      if (g0 + lane < n_groups) prefix[g0 + lane] = base + v;
+      base += __shfl(v, 63, 64);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const int word = resolve(ticket);
+    if (lane < 8) mbox[1][lane] = word;
+  }
+  lds_barrier();
+  Item cur;
+  if (!read_box(1, cur)) return;
+
+  if (scorer) {
+    __builtin_amdgcn_s_setprio(3);
+    const int kb = w & 3, sq = w >> 2;            // 32-key block and 32-query block of this wave
+    el8 kf[KS], vf[KS];                           // MFMA row n holds key k0 + kperm(n)
+    int k0, nsteps, doc_len, t_last, n_wait;
+    float rem_own, poison = 0.0f;
+    int row4, last4;
+    __amdgpu_buffer_rsrc_t stick_rs, in_rs, out_rs;
+    float se0, se1, se2;                          // stick on entering the block, requested ahead, three steps in turn
+    float d_next;                                 // carried sum of the next step's query, requested one step ahead
+    const int* pred = nullptr;                    // steps the chain's tile before this one has published
+    int* mine = nullptr;
+    int seen = 0;
+    int roff[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) roff[ks] = swz_off<D>(32 * sq + n, 2 * ks + h);
+
+    auto row_off = [&](int step) { return min(row4 - step * (4 * TQ), last4); };   // (below zero: outside the resource)
+    auto request_e = [&](int step, float& e) { e = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(stick_rs, row_off(step), 0, 0)); };
+    auto request_d = [&](int step) { d_next = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(in_rs, row_off(step), 0, 16 /* sc1 */)); };
+    auto open_item = [&](const ChainArgs& a, const Item& it) {
+      int n = lane & 31, h = lane >> 5;           // (opaque here: nothing per-lane of an item's prologue is to live through its steps)
+      asm volatile("" : "+v"(n), "+v"(h));
+      doc_len = it.doc_len;
+      k0 = it.kt * BKV + 32 * kb;
+      t_last = (doc_len - 1) / TQ;
+      nsteps = t_last - it.kt * DIAG + 1;
+      const int tblock = min((BKV / 32) * it.kt + kb, (doc_len - 1) / 32);   // (a block behind the document's end reads the last one's rows, unused)
+      const int64_t tab = (int64_t)it.head * a.tab_stride + it.tab_base;
+      rem_own = 0.0f;
+      if (a.fuse && k0 + n < doc_len) rem_own = a.stick[tab + tab_rowplane32(doc_len) + k0 + n];
+      const unsigned run_bytes = (unsigned)doc_len * 4u;
+      stick_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.stick) + tab + tab_seg32(doc_len, tblock), 0, run_bytes, 0x00020000);
+      const int64_t plane = (int64_t)a.heads * a.tiles * BM, at = ((int64_t)it.head * a.tiles + it.tile_base) * BM;
+      in_rs = __builtin_amdgcn_make_buffer_rsrc(a.carry + (it.kt & 1) * plane + at, 0, run_bytes, 0x00020000);
+      out_rs = __builtin_amdgcn_make_buffer_rsrc(a.carry + ((it.kt + 1) & 1) * plane + at, 0, run_bytes, 0x00020000);
+      row4 = 4 * (t_last * TQ + 32 * sq + n);
+      last4 = 4 * (doc_len - 1);
+      int* fl = a.flags + (int64_t)it.head * a.tiles + it.tile_base + it.kt;
+      pred = fl - 1;
+      mine = fl;
+      n_wait = it.kt > 0 ? nsteps : 0;
+      seen = 0;
+      request_e(0, se0);
+      request_e(1, se1);
+      request_e(2, se2);
+    };
+    // the first AHEAD tiles of an item (first query block's score waves copy)
+    auto open_tiles = [&](const ChainArgs& a, const Item& it) {
+      if (sq != 0) return;
+      int l = lane;
+      asm volatile("" : "+v"(l));
+      const Rows qrows = rows_of(a.q, it), grows = rows_of(a.go, it);
+      Copy qcopy, gcopy;
+      qcopy.init(64 * kb + l, qrows.row_bytes, qrows.used_bytes);
+      gcopy.init(64 * kb + l, grows.row_bytes, grows.used_bytes);
+#pragma unroll
+      for (int s = 0; s < AHEAD; ++s)
+        if (s < nsteps) {
+          qcopy.issue(qrows, (t_last - s) * TQ, Qs + s * QTILE);
+          gcopy.issue(grows, (t_last - s) * TQ, Gs + s * QTILE);
+        }
+    };
+    // K and V fragments of this wave's keys from the tiles the product waves have staged
+    auto take_fragments = [&]() {
+      int n = lane & 31, h = lane >> 5;
+      asm volatile("" : "+v"(n), "+v"(h));
+      const int r = 32 * kb + kperm(n);
+      const unsigned short* Vt = (kb < 2 ? Qs : Gs) + AHEAD * QTILE;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        kf[ks] = lds_row8(PZ + swz_off<D>(r, 2 * ks + h));
+        vf[ks] = lds_row8(Vt + swz_off<D>(r & 63, 2 * ks + h));
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+    // first score wave: the tile before this one has published `steps` steps (all of them: nothing to wait for any more)
+    auto await = [&](int steps) {
+      const int need = min(steps, n_wait);
+      if (seen >= need) return;
+      for (int tries = 0; tries < CHAIN_SPIN_LIMIT; ++tries) {
+        seen = __builtin_amdgcn_readfirstlane(__hip_atomic_load(pred, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        if (seen >= need) return;
+        __builtin_amdgcn_s_sleep(2);
+      }
+      poison = __builtin_nanf("");      // (cannot happen while workgroups make progress: never a plausible result, never a hang)
+      n_wait = 0;
+    };
+    auto chains = [&](int slot, f32x16& x, f32x16& da) {
+      const unsigned short* Qt = Qs + slot * QTILE;
+      const unsigned short* Gt = Gs + slot * QTILE;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) { x[j] = 0.0f; da[j] = 0.0f; }
+      el8 qfr[KS], gfr[KS];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) { qfr[ks] = lds_row8(Qt + roff[ks]); gfr[ks] = lds_row8(Gt + roff[ks]); }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        x = mfma32(kf[ks], qfr[ks], x);
+        da = mfma32(vf[ks], gfr[ks], da);
+      }
+    };
+
+    // What a step keeps of a block between forming its weights and forming its dz, one step later.
+    struct Weights { float p[16], r[16], lo; };
+    // Step w: dz of block w (weights and do.v in `wc`, `dc`, formed a step ago), weights of block w + 1 (scores `xn`,
+    // do.v `dn`) into `wn`, and the two MFMA chains of block w + 2 into `xf`, `df`, interleaved with the vector work in
+    // eight chunks (see bulk in sba_bwd.hip).  The sum over the key blocks before this wave's goes through `tot`: written
+    // with the weights, read a step later.  FIRST: there is no block w yet.  BAND: block w + 1 may hold keys its
+    // queries must not see.  SLOT >= 0: ring slot of tile w + 2, else taken from w.
+    auto step = [&](auto first_tag, auto band_tag, auto slot_tag, const int w, Weights& wc, f32x16& dc, f32x16& xn, f32x16& dn,
+                    Weights& wn, f32x16& xf, f32x16& df, float& se) __attribute__((always_inline)) {
+      constexpr bool FIRST = decltype(first_tag)::value, BAND = decltype(band_tag)::value;
+      constexpr int SLOT = decltype(slot_tag)::value;
+      constexpr int NCHUNK = 8, PER = 2 * (D / 16) / NCHUNK, LEAD = 2;
+      const int slot = SLOT >= 0 ? SLOT : (w + 2) % RING;
+      const int par = SLOT >= 0 ? (SLOT & 1) : (w & 1);
+      const int p_buf = SLOT >= 0 ? (SLOT + 2) % 3 : (w + 1) % 3;    // of block w + 1
+      float d_in = 0.0f, t0 = 0.0f, t1 = 0.0f, t2 = 0.0f;
+      if constexpr (!FIRST) {
+        d_in = d_next + poison;
+        if (kb > 0) t0 = tot[par][sq][0][n];
+        if (kb > 1) t1 = tot[par][sq][1][n];
+        if (kb > 2) t2 = tot[par][sq][2][n];
+      }
+      request_d(w + 1);
+      float e_in = se;
+      request_e(w + 4, se);
+      const unsigned short* Qt = Qs + slot * QTILE;
+      const unsigned short* Gt = Gs + slot * QTILE;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) { xf[j] = 0.0f; df[j] = 0.0f; }
+      el8 fr[LEAD + 1][PER];
+      auto pre = [&](int c) {
+        if (c >= NCHUNK) return;
+#pragma unroll
+        for (int m = 0; m < PER; ++m) {
+          const int k = c * PER + m;
+          if (k >= 2 * KS) continue;
+          fr[c % (LEAD + 1)][m] = lds_row8(((k & 1) ? Gt : Qt) + roff[k >> 1]);
+        }
+      };
+      auto post = [&](int c) {
+#pragma unroll
+        for (int m = 0; m < PER; ++m) {
+          const int k = c * PER + m;
+          if (k >= 2 * KS) continue;
+          if (k & 1) df = mfma32(vf[k >> 1], fr[c % (LEAD + 1)][m], df);
+          else xf = mfma32(kf[k >> 1], fr[c % (LEAD + 1)][m], xf);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      const int qw0 = (t_last - (w + 1)) * TQ + 32 * sq;
+      const int lim = qw0 + n - k0 - 16 * h + (AC ? 1 : 0);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        wn.r[j] = fast_rcp(1.0f + fast_exp2(a.c * xn[j]));
+        if (BAND && !(j < lim)) wn.r[j] = 1.0f;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      pre(0);
+      pre(1);
+#pragma unroll
+      for (int j = 8; j < 16; ++j) {
+        wn.r[j] = fast_rcp(1.0f + fast_exp2(a.c * xn[j]));
+        if (BAND && !(j < lim)) wn.r[j] = 1.0f;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      pre(2);
+      const int row = n;
+      if constexpr (!FIRST) {
+        const float before = d_in + ((t0 + t1) + t2);
+        float dprev = h == 1 ? before + wc.lo : before;
+        float dz[16];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) { const float dj = fmaf(wc.p[j], dc[j], dprev); dz[j] = fmaf(wc.r[j], dj, -dprev); dprev = dj; }
+        post(0);
+        pre(3);
+#pragma unroll
+        for (int j = 8; j < 16; ++j) { const float dj = fmaf(wc.p[j], dc[j], dprev); dz[j] = fmaf(wc.r[j], dj, -dprev); dprev = dj; }
+        unsigned short* Zt = Zs + par * PTILE;
+        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h)) = pack8(dz);
+        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h + 1)) = pack8(dz + 8);
+        // what the next key tile starts from (the half-wave with the newer keys ends with the sum over all)
+        if (kb == 3 && h == 1) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dprev), out_rs, row4 - w * (4 * TQ), 0, 0);
+        post(1);
+      } else {
+        post(0);
+        pre(3);
+        post(1);
+      }
+      pre(4);
+      post(2);
+      // block w + 1: stick left after the newer keys, weights
+      pre(5);
+      float ex[16];
+      // (a block none of whose keys the queries may see: the table holds no value for it)
+      if (BAND) e_in = sub_skip<AC>(k0, qw0) ? 0.0f : e_in;
+      (void)suffix_prod32_excl(wn.r, ex, h, e_in);
+      post(3);
+      pre(6);
+      wn.p[0] = ex[0] - ex[0] * wn.r[0];
+#pragma unroll
+      for (int j = 1; j < 16; ++j) wn.p[j] = ex[j] - ex[j - 1];
+      unsigned short* Pt = Ps + p_buf * PTILE;
+      if (BAND && a.fuse && qw0 == k0) {      // o + rem v: rem_j do_j reaches dv_j through the diagonal of p (see sba_bwd.hip)
+        float pd[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) pd[j] = wn.p[j] + (16 * h + j == n ? rem_own : 0.0f);
+        *reinterpret_cast<el8*>(Pt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h)) = pack8(pd);
+        *reinterpret_cast<el8*>(Pt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h + 1)) = pack8(pd + 8);
+      } else {
+        *reinterpret_cast<el8*>(Pt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h)) = pack8(wn.p);
+        *reinterpret_cast<el8*>(Pt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h + 1)) = pack8(wn.p + 8);
+      }
+      post(4);
+      pre(7);
+      float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 16; j += 2) { s0 = fmaf(wn.p[j], dn[j], s0); s1 = fmaf(wn.p[j + 1], dn[j + 1], s1); }
+      float lo, hi;
+      both_halves(s0 + s1, lo, hi);
+      wn.lo = lo;
+      if (h == 0) tot[par ^ 1][sq][kb][n] = lo + hi;
+      post(5);
+      post(6);
+      post(7);
+    };
+    // ends a step: the first score wave makes sure that what the others request behind the barrier is there, the second
+    // publishes what this tile has finished (formed two steps ago and acknowledged since)
+    auto finish = [&](int w) {
+      if (sq == 0 && kb == 0 && n_wait > 0) await(w + 3);
+      lds_barrier();
+    };
+    auto publish = [&](int w) {
+      if (sq == 0 && kb == 1 && w >= 3 && lane == 0) __hip_atomic_store(mine, w - 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    const bool keeper = w == 0;
+    unsigned ticket = 0;
+    int word = -1;
+    auto queue = [&](int w, int parity) {
+      if (!keeper) return;
+      if (w == max(nsteps - 6, 0) && lane == 0) ticket = atomicAdd(ctr, 1u);
+      if (w == max(nsteps - 2, 0)) word = resolve(ticket);
+      if (w == nsteps - 1 && lane < 8) mbox[parity][lane] = word;
+    };
+
+    using std::integral_constant;
+    using Yes = std::true_type;
+    using No = std::false_type;
+    using RT = integral_constant<int, -1>;
+    open_item(a, cur);
+    open_tiles(a, cur);
+#pragma unroll 1
+    for (int m = 0;; ++m) {
+      if (keeper) await(1);
+      wait_loads<0>();
+      lds_barrier();                 // tiles 0 .. AHEAD-1 and the K and V tiles have landed
+      take_fragments();
+      lds_barrier();                 // every wave has its share of K and V in registers: their places are free
+      f32x16 x0, x1, da0, da1, da2;
+      Weights wa, wb;
+      chains(0, x0, da0);
+      // weights of block 0 (as step -1), chains of block 1
+      step(Yes{}, Yes{}, RT{}, -1, wb, da2, x0, da0, wa, x1, da1, se0);
+      if (keeper) await(2);
+      lds_barrier();
+      int i = 0;
+      // Everything repeats with period six (ring slots, staging buffers, weights, scores, do.v sums, carries): step i = 6 m has
+      // block i's weights in wa, its do.v in da0, block i+1's scores in x1 and do.v in da1.
+#pragma unroll 1
+      for (; i + 6 < nsteps - DIAG - 2; i += 6) {
+        publish(i);     step(No{}, No{}, integral_constant<int, 2>{}, i, wa, da0, x1, da1, wb, x0, da2, se1);     finish(i);
+        publish(i + 1); step(No{}, No{}, integral_constant<int, 3>{}, i + 1, wb, da1, x0, da2, wa, x1, da0, se2); finish(i + 1);
+        publish(i + 2); step(No{}, No{}, integral_constant<int, 4>{}, i + 2, wa, da2, x1, da0, wb, x0, da1, se0); finish(i + 2);
+        publish(i + 3); step(No{}, No{}, integral_constant<int, 5>{}, i + 3, wb, da0, x0, da1, wa, x1, da2, se1); finish(i + 3);
+        publish(i + 4); step(No{}, No{}, integral_constant<int, 0>{}, i + 4, wa, da1, x1, da2, wb, x0, da0, se2); finish(i + 4);
+        publish(i + 5); step(No{}, No{}, integral_constant<int, 1>{}, i + 5, wb, da2, x0, da0, wa, x1, da1, se0); finish(i + 5);
+      }
+#pragma unroll 1
+      for (;; i += 6) {
+        if (i >= nsteps) break;
+        queue(i, m & 1);     publish(i);     step(No{}, Yes{}, RT{}, i, wa, da0, x1, da1, wb, x0, da2, se1);     finish(i);
+        if (i + 1 >= nsteps) break;
+        queue(i + 1, m & 1); publish(i + 1); step(No{}, Yes{}, RT{}, i + 1, wb, da1, x0, da2, wa, x1, da0, se2); finish(i + 1);
+        if (i + 2 >= nsteps) break;
+        queue(i + 2, m & 1); publish(i + 2); step(No{}, Yes{}, RT{}, i + 2, wa, da2, x1, da0, wb, x0, da1, se0); finish(i + 2);
+        if (i + 3 >= nsteps) break;
+        queue(i + 3, m & 1); publish(i + 3); step(No{}, Yes{}, RT{}, i + 3, wb, da0, x0, da1, wa, x1, da2, se1); finish(i + 3);
+        if (i + 4 >= nsteps) break;
+        queue(i + 4, m & 1); publish(i + 4); step(No{}, Yes{}, RT{}, i + 4, wa, da1, x1, da2, wb, x0, da0, se2); finish(i + 4);
+        if (i + 5 >= nsteps) break;
+        queue(i + 5, m & 1); publish(i + 5); step(No{}, Yes{}, RT{}, i + 5, wb, da2, x0, da0, wa, x1, da1, se0); finish(i + 5);
+      }
+      publish(nsteps);
+      const bool more = read_box(m & 1, cur);
+      if (more) open_item(fresh_args<ChainArgs>(), cur);
+      lds_barrier();                 // the product waves are done with the last Q tile
+      if (!more) break;
+      open_tiles(fresh_args<ChainArgs>(), cur);
+    }
+  } else {
+    __builtin_amdgcn_s_setprio(0);
+    const int pw = w - 4 * NSQ;
+    const int ptid = pw * 64 + lane;
+    const int mat = pw >> 1, half = pw & 1;       // (dv | dk) x 64 keys; all columns
+    const bool has_dq = pw < NSQ * DB;            // 32 x 32 block of dq: query block pw / DB, columns 32 (pw % DB)
+    const int dsq = pw / DB, dcol = pw % DB;
+    f32x16 acc[2][DB];
+#pragma unroll
+    for (int kb2 = 0; kb2 < 2; ++kb2)
+#pragma unroll
+      for (int j = 0; j < DB; ++j)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[kb2][j][i] = 0.0f;
+    // Offsets (elements) of this lane's reads.  The swizzle is an XOR of the chunk number, so the offset of a further chunk
+    // is the first one's with a constant XORed in: one register per row instead of one per read -- there is none to
+    // spare, and a spilled one would be reloaded through the counter that the waits below count on.
+    int xb[2], yb[2];      // transpose reads of rows 8 h + 4 u + i16 / 4: staged block (chunk of key 64 half), tile (chunk of column 0)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int r = 8 * h + 4 * u + (i16 >> 2), c = 16 * blk + 4 * (i16 & 3);
+      xb[u] = swz_off<BKV>(r, (64 * half + c) >> 3) + (c & 7);
+      yb[u] = swz_off<D>(r, c >> 3) + (c & 7);
+    }
+    int zb = swz_off<BKV>(32 * dsq + n, h);      // row reads of staged dz: chunk 2 ks + h of row n
+    Copy qcopy, gcopy;
+    qcopy.init(ptid, (unsigned)a.q.st * 2u, 2 * a.head_dim);
+    gcopy.init(ptid, (unsigned)a.go.st * 2u, 2 * a.head_dim);
+    el8 kt_f[BKV / 16];                            // this wave's 32 columns of the key tile, as the B operand of dq = dz K
+    Rows qrows, grows;
+    __amdgpu_buffer_rsrc_t part_rs;
+    int t_last, nsteps, doc_len, kt;
+    auto open_item = [&](const ChainArgs& a, const Item& it) {
+      qrows = rows_of(a.q, it);
+      grows = rows_of(a.go, it);
+      doc_len = it.doc_len;
+      kt = it.kt;
+      t_last = (doc_len - 1) / TQ;
+      nsteps = t_last - kt * DIAG + 1;
+      // partial dq: per 32 rows and 32 columns 1024 floats as the accumulators lie
+      float* part = a.partial + ((int64_t)it.head * a.tiles + it.tile_base) * (BM * D) + dcol * 1024;
+      part_rs = __builtin_amdgcn_make_buffer_rsrc(part, 0, (unsigned)((doc_len + BM - 1) / BM) * (BM * D * 4u) - (unsigned)dcol * 4096u, 0x00020000);
+      // The K tile into the staging buffers and the V tile into the two ring slots the item's first tiles leave free, in
+      // natural order.  (Fragments straight from global memory -- 32 rows of 32 bytes per instruction -- took
+      // 6400 cycles of an item's beginning to issue, these copies 1000.)
+      static_assert(AHEAD + 2 <= RING && 2 * QTILE >= 64 * D, "half of the V tile per ring");
+      int l = ptid;
+      asm volatile("" : "+v"(l));
+      const Rows krows = rows_of(a.k, it), vrows = rows_of(a.v, it);
+      TileCopy<D, BKV, 256, false, true> kcopy;
+      kcopy.init(l, krows.row_bytes, krows.used_bytes);
+      kcopy.issue(krows, kt * BKV, PZ);
+      TileCopy<D, 64, 256, false, true> vcopy;
+      vcopy.init(l, vrows.row_bytes, vrows.used_bytes);
+      vcopy.issue(vrows, kt * BKV, Qs + AHEAD * QTILE);
+      vcopy.issue(vrows, kt * BKV + 64, Gs + AHEAD * QTILE);
+    };
+    auto take_key_tile = [&]() {
+      if (has_dq) {
+#pragma unroll
+        for (int ks = 0; ks < BKV / 16; ++ks)
+          kt_f[ks] = lds_tr8(PZ + (yb[0] ^ (dcol << 5)) + 16 * ks * D, PZ + (yb[1] ^ (dcol << 5)) + 16 * ks * D);
+      } else {
+#pragma unroll
+        for (int ks = 0; ks < BKV / 16; ++ks) kt_f[ks] = zero8();
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+    const int lane16 = lane * 16;
+    Item nxt;
+    open_item(a, cur);
+#pragma unroll 1
+    for (int m = 0;; ++m) {
+      // the K and V tiles have landed (the stores of the item before may still be on their way)
+      if (m == 0) wait_loads<0>();
+      else wait_loads<4 * DB>();
+      lds_barrier();
+      take_key_tile();
+      lds_barrier();
+      lds_barrier();                 // weights of block 0 are staged
+      // Iteration w: dq, and dv or dk, of block w - 1; a tile is copied and the next partial dq requested.
+      // A product wave is bound by what it can issue next to a score wave: the eight dependent products of dq are
+      // spread between those of dk / dv, and the memory instructions -- the partial dq stored, the next one requested, a
+      // tile copied -- go out one behind each further product (in one go, 4 + 4 + 4 of every wave queue up in front of the
+      // CU's address unit: 500 cycles of an iteration of 2800).  Every iteration issues the same ones in the
+      // same order, with an offset outside the resource where there is nothing to store, request or copy, so that
+      // the waits count constants and no value on its way has to be moved where two paths join.
+      f32x4 l0, l1, l2, l3;           // partial dq on its way in
+      const unsigned short* const Ys = mat ? Qs : Gs;
+      constexpr int KQ = TQ / 16, KZ = BKV / 16, ZH = KZ / 2;
+      auto store_part = [&](const int w, const int i, const f32x16& dq, const bool store) __attribute__((always_inline)) {
+        const f32x4 part = {dq[4 * i], dq[4 * i + 1], dq[4 * i + 2], dq[4 * i + 3]};
+        const int soff = ((t_last - w + 1) * NSQ + dsq) * (D * 128);    // bytes of partial dq ahead of this query tile's 32 rows
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, part), part_rs, (store ? lane16 : OUTSIDE) + 1024 * i, soff, 0);
+      };
+      constexpr int FETCH_OPS = 4 + 2 * Copy::NCH;
+      auto fetch = [&](const int w, const int i) __attribute__((always_inline)) {
+        const int soff = (max(t_last - w, 0) * NSQ + dsq) * (D * 128);
+        const int l_off = has_dq && kt > 0 && w < nsteps ? lane16 : OUTSIDE;
+        if (i == 0) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen sc1" : "=&v"(l0) : "v"(l_off), "s"(part_rs), "s"(soff) : "memory");
+        if (i == 1) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:1024 sc1" : "=&v"(l1) : "v"(l_off), "s"(part_rs), "s"(soff) : "memory");
+        if (i == 2) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:2048 sc1" : "=&v"(l2) : "v"(l_off), "s"(part_rs), "s"(soff) : "memory");
+        if (i == 3) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:3072 sc1" : "=&v"(l3) : "v"(l_off), "s"(part_rs), "s"(soff) : "memory");
+        const bool fetched = w + AHEAD < nsteps;
+        const int row0 = (t_last - (w + AHEAD)) * TQ, slot = (w + AHEAD) % RING;
+        if (i >= 4 && i < 4 + Copy::NCH) qcopy.issue_one(qrows, row0, Qs + slot * QTILE, i - 4, fetched, spare[pw]);
+        if (i >= 4 + Copy::NCH && i < FETCH_OPS) gcopy.issue_one(grows, row0, Gs + slot * QTILE, i - 4 - Copy::NCH, fetched, spare[pw]);
+      };
+      auto read_y = [&](const unsigned short* Yt, const int j) { return lds_tr8(Yt + (yb[0] ^ (j << 5)), Yt + (yb[1] ^ (j << 5))); };
+      // iteration 0 has no block yet
+#pragma unroll
+      for (int i = 0; i < FETCH_OPS; ++i) fetch(0, i);
+      lds_barrier();
+      constexpr int N_PRODUCTS = KQ * 2 * DB, REST = N_PRODUCTS - KZ / 2, OPS = 4 + FETCH_OPS;
+#pragma unroll 1
+      for (int w = 1; w <= nsteps; ++w) {
+        asm volatile("" : "+v"(xb[0]), "+v"(xb[1]), "+v"(yb[0]), "+v"(yb[1]), "+v"(zb));   // (the XORs stay in the loop)
+        const int b = w - 1;
+        const unsigned short* Zt = Zs + (b & 1) * PTILE;
+        const unsigned short* Xt = mat ? Zt : Ps + (b % 3) * PTILE;
+        const unsigned short* Yt = Ys + (b % RING) * QTILE;
+        const bool finished = b >= nsteps - DIAG;               // the queries of this tile's own keys: nothing is missing any more
+        el8 zf[ZH], af[2], bf[DB];
+        auto read_x = [&](int ks, int kb2) { return lds_tr8(Xt + (xb[0] ^ (kb2 << 5)) + 16 * ks * BKV, Xt + (xb[1] ^ (kb2 << 5)) + 16 * ks * BKV); };
+#pragma unroll
+        for (int ks = 0; ks < ZH; ++ks) zf[ks] = lds_row8(Zt + (zb ^ (ks << 4)));
+        af[0] = read_x(0, 0);
+        bf[0] = read_y(Yt, 0);
+        af[1] = read_x(0, 1);
+#pragma unroll
+        for (int j = 1; j < DB; ++j) bf[j] = read_y(Yt, j);
+        // product number i of dk / dv: contraction step i / (2 DB), column block, 32-key block; the fragment a column block
+        // is done with gives way to the next step's
+        auto product = [&](const int i) __attribute__((always_inline)) {
+          const int ks = i / (2 * DB), j = (i / 2) % DB, kb2 = i & 1;
+          acc[kb2][j] = mfma32(bf[j], af[kb2], acc[kb2][j]);
+          if (kb2 == 1 && ks + 1 < KQ) bf[j] = read_y(Yt + 16 * (ks + 1) * D, j);
+          if (j == DB - 1 && ks + 1 < KQ) af[kb2] = read_x(ks + 1, kb2);
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        // the partial dq requested an iteration ago has arrived (and everything requested or stored before it is done)
+        asm volatile("s_waitcnt vmcnt(%4)" : "+v"(l0), "+v"(l1), "+v"(l2), "+v"(l3) : "n"(LOADS_PER_TILE) : "memory");
+        f32x16 dq = {l0[0], l0[1], l0[2], l0[3], l1[0], l1[1], l1[2], l1[3], l2[0], l2[1], l2[2], l2[3], l3[0], l3[1], l3[2], l3[3]};
+#pragma unroll
+        for (int ks = 0; ks < KZ; ++ks) {
+          dq = mfma32(kt_f[ks], zf[ks % ZH], dq);
+          if (ks + ZH < KZ) zf[ks % ZH] = lds_row8(Zt + (zb ^ ((ks + ZH) << 4)));
+          if (ks & 1) product(ks >> 1);
+        }
+        if (finished) {
+          const int row = (t_last - b) * TQ + 32 * dsq + n;
+          const Rows out = rows_of(a.dq, cur);
+          store_block32_rows(dq, a.inv_temp, out, row < doc_len && has_dq ? row * (int)out.row_bytes : OUTSIDE, 32 * dcol, h);
+        }
+#pragma unroll
+        for (int i = 0; i < (REST > OPS ? REST : OPS); ++i) {
+          if (i < 4) store_part(w, i, dq, has_dq && !finished);
+          else if (i < OPS) fetch(w, i - 4);
+          if (i < REST) product(KZ / 2 + i);
+        }
+        // The tile copied an iteration ago (read behind this barrier) has landed, what came after it may be in flight.  An item's
+        // last request, of nothing, has to come back all the same before its registers are used for something else.
+        if (w < nsteps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + LOADS_PER_TILE) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS_PER_TILE) : "memory");
+        lds_barrier();
+      }
+      // (behind the barrier of the last iteration every product wave is done with the staged blocks and the last tiles)
+      const bool more = read_box(m & 1, nxt);
+      const Item done = cur;
+      const ChainArgs a = fresh_args<ChainArgs>();
+      if (more) {
+        cur = nxt;
+        open_item(a, cur);
+      }
+      const Rows out = rows_of(mat ? a.dk : a.dv, done);
+#pragma unroll
+      for (int kb2 = 0; kb2 < 2; ++kb2) {
+        const int row = done.kt * BKV + 64 * half + 32 * kb2 + n;
+        const int off = row < done.doc_len ? row * (int)out.row_bytes : OUTSIDE;
+#pragma unroll
+        for (int j = 0; j < DB; ++j) {
+          store_block32_rows(acc[kb2][j], mat ? a.inv_temp : 1.0f, out, off, 32 * j, h);
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[kb2][j][e] = 0.0f;
+        }
+      }
+      if (!more) break;
+    }
+  }
+}
+
+template __global__ void bwd_chain_kernel<128, 128, false, 1>(const ChainArgs);
+template __global__ void bwd_chain_kernel<128, 128, true, 1>(const ChainArgs);
+template __global__ void bwd_chain_kernel<128, 96, false, 1>(const ChainArgs);
+template __global__ void bwd_chain_kernel<128, 96, true, 1>(const ChainArgs);
+
+template __global__ void bwd_chain_kernel<64, 64, false, 1>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 64, true, 1>(const ChainArgs);
+
+template <int D, int U, int NSQ>
+static hipError_t launch_chain_d(const ChainArgs& a, bool ac, int n_q_max, int workgroups, hipStream_t s) {
+  hipLaunchKernelGGL((chain_prep_kernel<D>), dim3((unsigned)n_q_max * (unsigned)a.heads), dim3(NT), 0, s, a);
+  const dim3 grid(workgroups), block((4 * NSQ + 4) * 64);
+  if (ac) hipLaunchKernelGGL((bwd_chain_kernel<D, U, true, NSQ>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((bwd_chain_kernel<D, U, false, NSQ>), grid, block, 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_bwd_chain(const ChainArgs& a, bool ac, int n_q_max, int workgroups, hipStream_t s) {
+  if (a.head_dim <= 64) return launch_chain_d<64, 64, 1>(a, ac, n_q_max, workgroups, s);
+  if (used_width(a.head_dim) == 96) return launch_chain_d<128, 96, 1>(a, ac, n_q_max, workgroups, s);
+  return launch_chain_d<128, 128, 1>(a, ac, n_q_max, workgroups, s);
+}
+
+}  // inline namespace SBA_ELEM_NS
+}  // namespace sba

@@ -52,6 +52,10 @@ constexpr int SCHED_MAXLEN = 6;  // longest document found (read together with t
 constexpr int SCHED_NKV_LONG = 7; // key tiles of the first group of the key-tile list (see kv_tail_tiles)
 constexpr int SCHED_HDR = 16;    // tile lists start here
 constexpr int TILE_WORDS = 8;    // int32 words of one Tile
+constexpr int RANK_LIMIT = 4096; // beyond this many documents the input order is kept
+// Behind the two tile lists: 6 n_docs + 2 words of the scheduler's, of which the ranked documents take the last
+// 4 n_docs once it is done (8-byte aligned: the lists are whole 32-byte tiles).
+__host__ __device__ inline int chain_docs_offset(int n_docs) { return (2 * n_docs + 3) & ~3; }
 
 struct Tile {
   int tok_start;  // first token of the document inside the packed token axis (0 for fixed-length)
@@ -59,7 +63,8 @@ struct Tile {
   int idx;        // tile index inside the document
   int batch;      // batch entry (0 for varlen)
   int tab_base;   // first carry-table entry of the document inside a head's share of the tables
-  int rsv[3];
+  int tile_base;  // 128-row tiles of the documents ranked before this one
+  int rsv[2];
 };
 
 // Carry tables (fp32).  Inside a head's share every document owns a triangular area: for each
@@ -538,6 +543,27 @@ __device__ __forceinline__ el8 load_frag(const Rows& r, int row, int col_bytes) 
   return __builtin_bit_cast(el8, load16(r, row, col_bytes));
 }
 
+// The same without the detour through LDS, for accumulators formed the other way round (lane = row n of the output, register i
+// = column 8*(i/4) + 4*h + i%4 of a 32-wide block): the half-waves exchange packed quads so that every
+// lane holds 8 consecutive columns of its row, two 16-byte stores per block.  `off`: byte offset of the lane's row in
+// the buffer, or OUTSIDE for a row that is not to be stored (the stores are issued either way: their number is known).
+__device__ __forceinline__ void store_block32_rows(const f32x16& acc, float scale, const Rows& out, int off, int col0, int h) {
+#pragma unroll
+  for (int g = 0; g < 4; g += 2) {
+    u32x4 v;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const unsigned a = __builtin_bit_cast(unsigned, cvt2(acc[4 * g + 2 * e] * scale, acc[4 * g + 2 * e + 1] * scale));
+      const unsigned b = __builtin_bit_cast(unsigned, cvt2(acc[4 * g + 4 + 2 * e] * scale, acc[4 * g + 5 + 2 * e] * scale));
+      const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+      v[e] = (unsigned)r[0];
+      v[2 + e] = (unsigned)r[1];
+    }
+    const int bytes = 2 * (col0 + 8 * g + 8 * h);
+    __builtin_amdgcn_raw_buffer_store_b128(v, out.rsrc, bytes < out.used_bytes ? off + bytes : OUTSIDE, 0, 0);
+  }
+}
+
 // XOR swizzle of the 16-byte chunks of an UNPADDED row-major tile (row = D*2 bytes) that makes
 // both access patterns of a dual-use tile bank-conflict free: row reads (16 consecutive rows,
 // one chunk each) and transpose reads (4 consecutive rows, 64 contiguous bytes each).
@@ -577,14 +603,21 @@ __device__ __forceinline__ int swz_off(int row, int chunk) {   // element offset
 // that pass, and the counted waits the kernels place themselves (wait_loads<N>, then a barrier,
 // before any wave reads a slot) are the only ones left.  Those are REQUIRED for correctness:
 // nothing else orders an LDS read after the copy that fills its slot.
+// STREAM: the lines are not to displace others from L2 (nt).
+template <bool STREAM = false>
 __device__ __forceinline__ void async_copy16(__amdgpu_buffer_rsrc_t rsrc, const unsigned short* dst, int voff, int soff) {
   const unsigned lds_addr = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               ::"s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
-               : "memory", "m0");
+  if constexpr (STREAM)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                 ::"s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
+                 : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 ::"s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
+                 : "memory", "m0");
 }
 
-template <int D, int ROWS, int THREADS, bool KEYS>
+template <int D, int ROWS, int THREADS, bool KEYS, bool STREAM = false>
 struct TileCopy {
   static constexpr int C8 = D / 8;
   static constexpr int NCH = ROWS * C8 / THREADS;
@@ -621,6 +654,13 @@ struct TileCopy {
     voff_odd = 16 * odd < used_bytes ? src * (int)row_bytes + odd * 16 : OUTSIDE;
   }
 
+  // Instruction j alone; with `wanted` false (uniform) it writes 1 KiB of zeros to `spare` instead.
+  __device__ __forceinline__ void issue_one(const Rows& r, int row0, unsigned short* lds_tile, int j, bool wanted, unsigned short* spare) const {
+    static_assert(!TWO_PHASE, "one offset per lane");
+    const int soff = wanted ? (row0 + row_delta(j)) * (int)r.row_bytes : 0;
+    async_copy16<STREAM>(r.rsrc, wanted ? lds_tile + (j * STEP + wave * RPI) * D : spare, wanted ? voff : OUTSIDE, __builtin_amdgcn_readfirstlane(soff));
+  }
+
   // `rows_needed` (uniform): instructions whose rows all lie at or beyond it are skipped; the tile
   // rows they would have filled keep whatever they held.
   __device__ __forceinline__ void issue(const Rows& r, int row0, unsigned short* lds_tile, int rows_needed = ROWS) const {
@@ -633,7 +673,7 @@ struct TileCopy {
           r.rsrc, (__attribute__((address_space(3))) void*)(lds_tile + (j * STEP + wave * RPI) * D), 16,
           TWO_PHASE && (j & 1) ? voff_odd : voff, soff, 0, 0);
 #else
-      async_copy16(r.rsrc, lds_tile + (j * STEP + wave * RPI) * D, TWO_PHASE && (j & 1) ? voff_odd : voff, soff);
+      async_copy16<STREAM>(r.rsrc, lds_tile + (j * STEP + wave * RPI) * D, TWO_PHASE && (j & 1) ? voff_odd : voff, soff);
 #endif
     }
   }

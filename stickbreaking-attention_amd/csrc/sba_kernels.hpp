@@ -39,30 +39,64 @@ struct KArgs {
   int min_items_each;          // host side: a launch is persistent when it has this many items per workgroup
 };
 
+// Arguments of the one-pass backward (sba_chain.hip).
+constexpr int CHAIN_QUEUES = 8;            // one per XCD
+constexpr int CHAIN_QUEUE_STRIDE = 32;     // words between the queues' counters: a 128-byte line each
+constexpr int CHAIN_GROUP = 8;             // chains of a queue whose items are interleaved
+constexpr int CHAIN_MAX_GROUPS = 256;
+constexpr int CHAIN_SPIN_LIMIT = 1 << 20;  // polls of a wait (about a second) before it gives up and the results turn to NaN
+struct ChainArgs {
+  View q, k, v, go, grem, dq, dk, dv;
+  const int* sched;
+  const float* stick;          // carry table written by the forward
+  float* partial;              // [heads][tiles][BM x D] fp32: dq of a query over the key tiles so far
+  float* carry;                // [2][heads][tiles][BM] fp32: the running sum along the keys, by parity of the key tile that reads it
+  int* flags;                  // [heads][tiles]: steps a key tile has published
+  unsigned* queues;            // CHAIN_QUEUES counters
+  int64_t tab_stride;
+  int docs_off;                // int32 offset of the ranked documents inside `sched`
+  int n_docs, heads, head_dim, tokens, tiles;
+  int fixed, fuse, clear_spare;
+  unsigned nan_pair;
+  int max_doc_len;
+  float c, inv_temp;
+  int pad;
+};
+
+// Pointers rebuilt from integer words are generic pointers to the compiler (64-bit flat addresses in
+// vector registers for every access); say again what it knows of pointers in a kernel's argument
+// list: they point into global memory.
+template <class T>
+__device__ __forceinline__ void as_global(T*& p) {
+  typedef __attribute__((address_space(1))) char* GlobalBytes;
+  p = reinterpret_cast<T*>((char*)(GlobalBytes)(unsigned long long)p);
+}
+__device__ __forceinline__ void globals_of(KArgs& a) {
+  as_global(a.q.ptr); as_global(a.k.ptr); as_global(a.v.ptr); as_global(a.o.ptr); as_global(a.rem.ptr);
+  as_global(a.go.ptr); as_global(a.grem.ptr); as_global(a.dq.ptr); as_global(a.dk.ptr); as_global(a.dv.ptr);
+  as_global(a.sched); as_global(a.stick); as_global(a.gtab); as_global(a.weights); as_global(a.work);
+}
+__device__ __forceinline__ void globals_of(ChainArgs& a) {
+  as_global(a.q.ptr); as_global(a.k.ptr); as_global(a.v.ptr); as_global(a.go.ptr); as_global(a.grem.ptr);
+  as_global(a.dq.ptr); as_global(a.dk.ptr); as_global(a.dv.ptr);
+  as_global(a.sched); as_global(a.stick); as_global(a.partial); as_global(a.carry); as_global(a.flags); as_global(a.queues);
+}
+
 // The argument block read afresh from the kernel-argument segment.  A persistent kernel calls this at
 // the top of every work item with a pointer the compiler cannot see through: argument words it
 // needs would otherwise be loaded once, ahead of the item loop, and stay in scalar registers across
 // the whole loop (the block is 380 bytes; the loop bodies have no such room, and spilled scalar
 // registers end up as vector registers spilled to scratch memory).
-__device__ __forceinline__ KArgs fresh_args() {
+template <class Args = KArgs>
+__device__ __forceinline__ Args fresh_args() {
   typedef const __attribute__((address_space(4))) unsigned long long* Words;
   Words w = (Words)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(w));
-  static_assert(sizeof(KArgs) % 8 == 0, "copied in 8-byte words");
-  union { KArgs a; unsigned long long u[sizeof(KArgs) / 8]; } out;
+  static_assert(sizeof(Args) % 8 == 0, "copied in 8-byte words");
+  union { Args a; unsigned long long u[sizeof(Args) / 8]; } out;
 #pragma unroll
-  for (unsigned i = 0; i < sizeof(KArgs) / 8; ++i) out.u[i] = w[i];
-  // Pointers rebuilt from integer words are generic pointers to the compiler (64-bit flat addresses in
-  // vector registers for every access); say again what it knows of pointers in a kernel's argument
-  // list: they point into global memory.
-  auto global = [](auto*& p) {
-    typedef __attribute__((address_space(1))) char* GlobalBytes;
-    p = reinterpret_cast<std::remove_reference_t<decltype(p)>>((char*)(GlobalBytes)(unsigned long long)p);
-  };
-  KArgs& a = out.a;
-  global(a.q.ptr); global(a.k.ptr); global(a.v.ptr); global(a.o.ptr); global(a.rem.ptr);
-  global(a.go.ptr); global(a.grem.ptr); global(a.dq.ptr); global(a.dk.ptr); global(a.dv.ptr);
-  global(a.sched); global(a.stick); global(a.gtab); global(a.weights); global(a.work);
+  for (unsigned i = 0; i < sizeof(Args) / 8; ++i) out.u[i] = w[i];
+  globals_of(out.a);
   return out.a;
 }
 
@@ -128,6 +162,8 @@ inline bool has_dkdv_tail_kernel(int head_dim) { return head_dim <= 64; }
                            hipStream_t s);                                                                       \
   hipError_t launch_bwd_dkdv(const KArgs& a, int head_dim, bool attend_current, bool product, int n_long_max,    \
                              int n_last_max, hipStream_t s);                                                     \
+  hipError_t launch_bwd_chain(const ChainArgs& a, bool attend_current, int n_q_max, int workgroups,              \
+                              hipStream_t s);                                                                    \
   }
 SBA_DECLARE_LAUNCHERS(bf16)
 SBA_DECLARE_LAUNCHERS(f16)

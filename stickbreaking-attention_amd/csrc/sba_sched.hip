@@ -10,8 +10,6 @@
 
 namespace sba {
 
-constexpr int RANK_LIMIT = 4096;   // beyond this many documents the input order is kept
-
 __device__ __forceinline__ int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 // Scratch (int32) behind the two tile lists, per document: start, len, order, qoff, kvoff, table base.
@@ -151,7 +149,8 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
           t.idx = nkv - ntail + j2;
           t.batch = fixed ? d : 0;
           t.tab_base = tab_ok ? (int)btab : 0;
-          t.rsv[0] = t.rsv[1] = t.rsv[2] = 0;
+          t.tile_base = bq;
+          t.rsv[0] = t.rsv[1] = 0;
           kvtiles[total_long + bne + j2] = t;
         }
       }
@@ -173,13 +172,14 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
   // the same CU.)  Packed documents of different lengths stay document-major, which keeps the
   // K/V rows a workgroup's neighbours read in the caches.
   for (int s = tid; s < total_q && ok; s += SCHED_THREADS) {
-    int d, within;   // document, position among its tiles in cost order
+    int d, within, rank = 0;   // document, position among its tiles in cost order
     if (fixed) {
       d = s % nd;
       within = s / nd;
     } else {
       int lo = 0, hi = nd;   // largest i with qoff[i] <= s
       while (hi - lo > 1) { const int mid = (lo + hi) >> 1; if (q_before[mid] <= s) lo = mid; else hi = mid; }
+      rank = lo;
       d = ranked[lo];
       within = s - q_before[lo];
     }
@@ -190,7 +190,8 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
     t.idx = nq - 1 - within;             // newest (most expensive) query tile first
     t.batch = fixed ? d : 0;
     t.tab_base = tab_of[d];
-    t.rsv[0] = t.rsv[1] = t.rsv[2] = 0;
+    t.tile_base = q_before[fixed ? d : rank];
+    t.rsv[0] = t.rsv[1] = 0;
     qtiles[s] = t;
   }
   // Key tiles stay document-major for every input: one workgroup per CU runs at a time, so the
@@ -206,8 +207,19 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
     t.idx = s - kv_before[lo];               // oldest keys are seen by the most queries: first
     t.batch = fixed ? d : 0;
     t.tab_base = tab_of[d];
-    t.rsv[0] = t.rsv[1] = t.rsv[2] = 0;
+    t.tile_base = q_before[lo];
+    t.rsv[0] = t.rsv[1] = 0;
     kvtiles[s] = t;
+  }
+  // E. the documents in ranked order, {first token, length, first table entry, 128-row tiles before}: what the one-pass
+  // backward names its chains by.  With the working arrays in LDS their places in the workspace are free.
+  if (in_lds && ok) {
+    int2* const docs = reinterpret_cast<int2*>(dstart + chain_docs_offset(nd));
+    for (int i = tid; i < nd; i += SCHED_THREADS) {
+      const int d = ranked[i];
+      docs[2 * i] = make_int2(fixed ? 0 : start_of[d], len_of[d]);
+      docs[2 * i + 1] = make_int2(tab_of[d], q_before[i]);
+    }
   }
   if (tid == 0) {
     hdr[SCHED_STATUS] = s_status;

@@ -113,7 +113,7 @@ Tensor as_caller(const Tensor& t, int64_t d, at::ScalarType dt) {
   return r.scalar_type() == dt ? r : r.to(dt);
 }
 
-// The gradient table of a backward: one grow-only buffer per (device, stream), shared by every layer (the dk/dv pass
+// The scratch of a backward (gradient table, or the one-pass form's): one grow-only buffer per (device, stream), shared by every layer (the dk/dv pass
 // of one backward has read it before the next backward on that stream writes it).  Packed documents change
 // the size with every batch; growth goes to the next eighth of a power of two, and by at least a quarter.
 // The lock is held while a backward's kernels are enqueued: two threads on one stream must not interleave theirs.
@@ -196,18 +196,27 @@ struct Attention : public torch::autograd::Function<Attention> {
     void* const stream = current_stream(qp);
     const sba_view vq = view(qp, c.fixed), vk = view(kp, c.fixed), vv = view(vp, c.fixed), vg = view(go, c.fixed), vr = view(gr, c.fixed);
     const sba_view wq = view(dq, c.fixed), wk = view(dk, c.fixed), wv = view(dv, c.fixed);
-    auto launch = [&](const Tensor& gtab) {
+    const size_t chain_bytes = sba_chain_scratch_bytes(&p);   // 0: the two-pass form
+    const int64_t scratch_floats = chain_bytes ? (int64_t)(chain_bytes / 4) : table.numel();
+    auto launch = [&](const Tensor& scratch) {
+      if (chain_bytes) {
+        check((c.fixed ? sba_attn_bwd_chained : sba_varlen_bwd_chained)(&p, c.sched.data_ptr(), (size_t)c.sched.numel(), &vq, &vk, &vv, &vg, &vr,
+                                                                        table.data_ptr<float>(), (size_t)table.numel() * 4,
+                                                                        scratch.data_ptr(), chain_bytes, &wq, &wk, &wv, stream),
+              c.fixed ? "sba_attn_bwd_chained" : "sba_varlen_bwd_chained");
+        return;
+      }
       check((c.fixed ? sba_attn_bwd : sba_varlen_bwd)(&p, c.sched.data_ptr(), (size_t)c.sched.numel(), &vq, &vk, &vv, &vg, &vr,
-                                                      table.data_ptr<float>(), gtab.data_ptr<float>(), (size_t)table.numel() * 4,
+                                                      table.data_ptr<float>(), scratch.data_ptr<float>(), (size_t)table.numel() * 4,
                                                       &wq, &wk, &wv, stream),
             c.fixed ? "sba_attn_bwd" : "sba_varlen_bwd");
     };
     if (capturing(stream)) {   // a graph's replays must not depend on a buffer that may be replaced
-      launch(at::empty({table.numel()}, table.options()));
+      launch(at::empty({scratch_floats}, table.options()));
     } else {
       GradTables& g = grad_tables();
       const std::lock_guard<std::mutex> lock(g.mutex);
-      launch(g.get(table.numel(), table, stream));
+      launch(g.get(scratch_floats, table, stream));
     }
     return {as_caller(dq, d, (at::ScalarType)(types >> 16)), as_caller(dk, d, (at::ScalarType)((types >> 8) & 255)),
             as_caller(dv, d, (at::ScalarType)(types & 255)), Tensor()};

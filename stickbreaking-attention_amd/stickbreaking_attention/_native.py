@@ -60,7 +60,7 @@ EXPORTS = (
     "sba_build_schedule",
     "sba_varlen_fwd", "sba_varlen_bwd", "sba_attn_fwd", "sba_attn_bwd", "sba_set_timing", "sba_set_dkdv_workgroups",
     "sba_last_kernel_ms", "sba_varlen_fwd_weights", "sba_attn_fwd_weights", "sba_varlen_fwd_static",
-    "sba_launch_geometry",
+    "sba_launch_geometry", "sba_chain_scratch_bytes", "sba_varlen_bwd_chained", "sba_attn_bwd_chained", "sba_set_backward_form",
 )
 
 _lib = None
@@ -107,6 +107,14 @@ def load():
             f = getattr(lib, name)
             f.restype = ctypes.c_int
             f.argtypes = [P, vp, sz, V, V, V, V, V, vp, vp, sz, V, V, V, vp]
+        for name in ("sba_varlen_bwd_chained", "sba_attn_bwd_chained"):
+            f = getattr(lib, name)
+            f.restype = ctypes.c_int
+            f.argtypes = [P, vp, sz, V, V, V, V, V, vp, sz, vp, sz, V, V, V, vp]
+        lib.sba_chain_scratch_bytes.restype = sz
+        lib.sba_chain_scratch_bytes.argtypes = [P]
+        lib.sba_set_backward_form.restype = None
+        lib.sba_set_backward_form.argtypes = [ctypes.c_int]
         lib.sba_varlen_fwd_static.restype = ctypes.c_int
         lib.sba_varlen_fwd_static.argtypes = [P, V, V, V, V, V, vp]
         lib.sba_set_timing.restype = None

@@ -304,19 +304,32 @@ def _launch_bwd(fixed: bool, do, dr, q, k, v, cu_seqlens, max_doc_len: int, logi
     lib = nat.load()
     q, k, v, do = _aligned(q), _aligned(k), _aligned(v), _aligned(do)
     prob, _keep = _problem(q, fixed, cu_seqlens, max_doc_len, logit_scale, attend_current, product, fused)
-    fn = lib.sba_attn_bwd if fixed else lib.sba_varlen_bwd
     drv = dr if dr is not None and dr.numel() else None
     if table.numel() == 0:
         raise ValueError("the backward needs the carry table of a forward that ran with gradients enabled")
+    name = "sba_attn_bwd" if fixed else "sba_varlen_bwd"
     with torch.cuda.device(q.device):
-        code = fn(ctypes.byref(prob), sched.data_ptr(), _nbytes(sched),
-                  ctypes.byref(nat.view4(q, fixed)), ctypes.byref(nat.view4(k, fixed)),
-                  ctypes.byref(nat.view4(v, fixed)), ctypes.byref(nat.view4(do, fixed)),
-                  ctypes.byref(nat.view4(drv, fixed, per_row=True)),
-                  table.data_ptr(), gtab.data_ptr(), min(_nbytes(table), _nbytes(gtab)),
-                  ctypes.byref(nat.view4(dq, fixed)), ctypes.byref(nat.view4(dk, fixed)),
-                  ctypes.byref(nat.view4(dv, fixed)), nat.stream_ptr(q.device))
-    nat.check(code, "sba_attn_bwd" if fixed else "sba_varlen_bwd")
+        chain = lib.sba_chain_scratch_bytes(ctypes.byref(prob))   # 0: the two-pass form
+        if chain:
+            name += "_chained"
+            if _nbytes(gtab) < chain:
+                gtab = _scratch_table((chain + 3) // 4, q.device, "grad")
+            work = (_nbytes(table), gtab.data_ptr(), _nbytes(gtab))
+        else:
+            work = (gtab.data_ptr(), min(_nbytes(table), _nbytes(gtab)))
+        code = getattr(lib, name)(ctypes.byref(prob), sched.data_ptr(), _nbytes(sched),
+                                  ctypes.byref(nat.view4(q, fixed)), ctypes.byref(nat.view4(k, fixed)),
+                                  ctypes.byref(nat.view4(v, fixed)), ctypes.byref(nat.view4(do, fixed)),
+                                  ctypes.byref(nat.view4(drv, fixed, per_row=True)), table.data_ptr(), *work,
+                                  ctypes.byref(nat.view4(dq, fixed)), ctypes.byref(nat.view4(dk, fixed)),
+                                  ctypes.byref(nat.view4(dv, fixed)), nat.stream_ptr(q.device))
+    nat.check(code, name)
+
+
+def _runs_chained(q: torch.Tensor, fixed: bool, cu_seqlens, max_doc_len: int, product: bool) -> bool:
+    prob, _keep = _problem(q, fixed, cu_seqlens, max_doc_len, 1.0, False, product, False)
+    with torch.cuda.device(q.device):
+        return nat.load().sba_chain_scratch_bytes(ctypes.byref(prob)) > 0
 
 
 # The four operators under upstream's names.  Outputs and workspaces are arguments that are
@@ -619,7 +632,9 @@ def run_backward(q, k, v, do, drem, fixed: bool, state, inv_temp: float, attend_
     if table.numel() == 0 and RECOMPUTE_TABLE:
         table = _rebuild_table(qp, kp, vp, fixed, sched, cu, max_len, float(inv_temp), bool(attend_current), product,
                                bool(fused))
-    gtab = _grad_table(table)
+    # (the one-pass form needs no gradient table and finds its own scratch memory; a compiled graph cannot know yet)
+    chained = not torch.compiler.is_compiling() and _runs_chained(qp, fixed, cu, max_len, product)
+    gtab = torch.empty(0, dtype=torch.float32, device=q.device) if chained else _grad_table(table)
     if fixed:
         _compileable_bwd(dop, dremp, qp, kp, vp, float(inv_temp), bool(attend_current), product, bool(fused),
                          table, sched, gtab, dq, dk, dv)

@@ -1,0 +1,66 @@
+"""The one-pass backward (csrc/sba_chain.hip), forced wherever it is possible: documents at the edges of its 32-query steps
+and 128-key tiles and of the three steps a tile lags behind its predecessor, both kernel widths and heads narrower
+than them, against the oracle; and queues of many items per workgroup and many groups, against the two-pass form."""
+import pytest
+import torch
+
+from oracle import sb_oracle as orc
+from tests.helpers import assert_close, cu_from_lengths, oracle_varlen
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture
+def form():
+    from stickbreaking_attention import _native
+    lib = _native.load()
+    yield lib.sba_set_backward_form
+    lib.sba_set_backward_form(0)
+
+
+def gradients(op, tensors, cu, longest, ac, grads):
+    x = [t.to(DEV).requires_grad_() for t in tensors]
+    out = op(*x, cu, longest, zero_start=False, attend_current=ac)
+    out = out if isinstance(out, tuple) else (out,)
+    return torch.autograd.grad(out, x, [g.to(DEV) for g in grads[:len(out)]])
+
+
+@pytest.mark.parametrize("ac", [False, True])
+@pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (96, torch.float16), (104, torch.bfloat16), (64, torch.bfloat16),
+                                     (40, torch.float16)])
+def test_tile_edges(form, d, dtype, ac):
+    from stickbreaking_attention import sb_attn_varlen, sb_attn_varlen_fused
+    lengths = [1, 32, 33, 127, 128, 129, 224, 256, 257, 550]
+    H, used = 3, sum(lengths)
+    T = used + 9
+    q, k, v, do = (t.to(dtype) for t in orc.make_inputs((H, T, d), 40 + d))
+    drem = torch.randn((H, T), generator=torch.Generator().manual_seed(d)).to(dtype)
+    cu = cu_from_lengths(lengths, device=DEV)
+    form(2)
+    got = gradients(sb_attn_varlen, (q, k, v), cu, max(lengths), ac, (do, drem))
+    fused = gradients(sb_attn_varlen_fused, (q, k, v), cu, max(lengths), ac, (do,))
+    form(1)
+    fused_two = gradients(sb_attn_varlen_fused, (q, k, v), cu, max(lengths), ac, (do,))
+    ref = oracle_varlen(q[:, :used], k[:, :used], v[:, :used], do[:, :used], lengths, ac, drem=drem[:, :used])[2:]
+    for name, g, r, f, f2 in zip(("dq", "dk", "dv"), got, ref, fused, fused_two):
+        assert not g[:, used:].any() and not f[:, used:].any()
+        assert_close(name, g[:, :used], r)
+        assert_close(name + " of o + rem v", f[:, :used], f2[:, :used].float())
+
+
+@pytest.mark.parametrize("H,lengths", [(5, [37 + 61 * i % 400 for i in range(90)]), (12, [2000, 1, 900, 4000]), (3, [4600, 700])])
+def test_queues(form, H, lengths):
+    from stickbreaking_attention import sb_attn_varlen
+    T = sum(lengths)
+    tensors = orc.make_inputs((H, T, 64), T)
+    drem = torch.randn((H, T), generator=torch.Generator().manual_seed(T)).to(torch.bfloat16)
+    cu = cu_from_lengths(lengths, device=DEV)
+    form(1)
+    two = gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem))
+    form(2)
+    first = gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem))
+    again = gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem))
+    for name, a, b, c in zip(("dq", "dk", "dv"), two, first, again):
+        assert_close(name, b, a.float())
+        assert torch.equal(b, c)
