@@ -235,7 +235,7 @@ int sba_attn_bwd(const sba_problem* p, const void* schedule, size_t schedule_siz
  * returns the scratch it needs (16-byte aligned, contents irrelevant, one per concurrent call) and 0 for every other;
  * a caller then takes sba_varlen_bwd / sba_attn_bwd.  Same inputs, outputs, table and refusals; it
  * needs no gradient table, and the results differ from the two-pass form's by rounding.  Problems it
- * cannot take (log-space carry, head_dim <= 32 or > 128, a device that is not eight XCDs of 32 compute units)
+ * cannot take (log-space carry, head_dim > 128, a device that is not eight XCDs of 32 compute units)
  * return SBA_E_SHAPE.  The stream's CU mask, if it has one, must leave every XCD at least one CU. */
 size_t sba_chain_scratch_bytes(const sba_problem* p);
 int sba_varlen_bwd_chained(const sba_problem* p, const void* schedule, size_t schedule_size,
@@ -296,7 +296,7 @@ float sba_last_kernel_ms(int which);
 void  sba_set_dkdv_workgroups(int n);
 
 /* Test and tuning switch (process-wide): which form of the backward sba_chain_scratch_bytes asks for.  0: by size,
- * 1: never the one-pass form, 2: wherever it is possible. */
+ * 1: never the one-pass form, 2: wherever it is possible, 3: the same in steps of 64 queries (head_dim <= 64). */
 void  sba_set_backward_form(int form);
 
 #ifdef __cplusplus

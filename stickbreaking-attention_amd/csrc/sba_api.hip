@@ -283,13 +283,14 @@ int backward(const sba_problem* p, bool fixed, const void* schedule, size_t sche
 }
 
 // ---- the one-pass backward (sba_chain.hip) ------------------------------------------------------------
+int chain_width(int head_dim) { return head_dim <= 64 ? 64 : 128; }   // columns of its rows
 struct ChainScratch { size_t partial, carry, flags, queues, total; };   // byte offsets
 ChainScratch chain_scratch(const sba_problem* p, const Sizes& sz) {
   const size_t tiles = (size_t)p->heads * (size_t)sz.n_kv_max;
   auto line = [](size_t n) { return (n + 255) & ~(size_t)255; };
   ChainScratch c;
   c.partial = 0;
-  c.carry = line(tiles * BM * kernel_width(p->head_dim) * sizeof(float));
+  c.carry = line(tiles * BM * chain_width(p->head_dim) * sizeof(float));
   c.flags = c.carry + line(2 * tiles * BM * sizeof(float));
   c.queues = c.flags + line(tiles * sizeof(int));
   c.total = c.queues + line(CHAIN_QUEUES * CHAIN_QUEUE_STRIDE * sizeof(unsigned));
@@ -301,16 +302,27 @@ ChainScratch chain_scratch(const sba_problem* p, const Sizes& sz) {
 // offsets into a document's partial dq.
 bool chain_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
   const long long chains = (long long)sz.n_docs * p->heads;
-  return (p->flags & SBA_PRODUCT_SPACE) && (kernel_width(p->head_dim) == 128 || kernel_width(p->head_dim) == 64) && sz.n_docs > 0 && sz.n_docs <= RANK_LIMIT &&
+  return (p->flags & SBA_PRODUCT_SPACE) && p->head_dim <= 128 && sz.n_docs > 0 && sz.n_docs <= RANK_LIMIT &&
          chains <= (long long)CHAIN_QUEUES * CHAIN_GROUP * CHAIN_MAX_GROUPS &&
-         ((long long)declared_max_doc_len(p, fixed) + BM) * kernel_width(p->head_dim) * 4 < (1ll << 31) && device_cus() == 256;
+         ((long long)declared_max_doc_len(p, fixed) + BM) * chain_width(p->head_dim) * 4 < (1ll << 31) && device_cus() == 256;
+}
+// Steps of 64 queries instead of 32 (head_dim <= 64).  They do more per step and CU (4 x 16 x 2048 at head_dim 64: 166 us
+// for 199) but a key tile lags its predecessor by four steps of either size, so as long as that lag is what a problem takes
+// (one head of 1024 keys: 58 us for 49) the small ones are the better ones.  The line: the work of a CU in steps, chains mean^2
+// / (2 x 64 x 128 x 256 CUs), against the steps of the longest document, where beyond 2048 keys more of a chain's tiles
+// start behind one another than side by side (16 x 4096: 250 us for 224, 16 x 8192: 589 for 653).
+bool chain_wide(const sba_problem* p, bool fixed, const Sizes& sz) {
+  const int form = g_backward_form.load();
+  if (form == 2 || form == 3) return form == 3;
+  const long long mean = sz.rows / sz.n_docs, longest = declared_max_doc_len(p, fixed);
+  return 2 * (long long)sz.n_docs * p->heads * mean * mean >= longest * (longest > 2048 ? 3 : 2) * 65536;
 }
 // Where the one-pass form is the faster one (gain over the two passes, measured on 270 problems of 1 to 32 heads and
 // 512 to 16 K tokens in 1 to 128 documents, declared lengths exact).
 bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
   const int form = g_backward_form.load();
   if (form == 1 || g_dkdv_workgroups.load() != 0 || !chain_possible(p, fixed, sz)) return false;
-  if (form == 2) return true;
+  if (form == 2 || form == 3) return true;
   const long long chains = (long long)sz.n_docs * p->heads, items = (long long)sz.n_kv_max * p->heads;
   const long long mean = sz.rows / sz.n_docs, longest = declared_max_doc_len(p, fixed);
   // a document of one or two steps: nothing to hand on, and one launch more (0.85 .. 1.01)
@@ -324,11 +336,14 @@ bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
     if (10 * chains < 9 * CHAIN_QUEUES * per_xcd) return false;
     if (longest > 32 * BKV && chains * mean * mean < (CHAIN_QUEUES + 4) * longest * longest) return false;
   }
-  // Width 128 gains from there on (1.03 .. 1.38; 0.96 where every document ends in a nearly empty tile).  At width 64 what
-  // an item costs before its first step weighs twice as much: with several items per CU only documents of
-  // some length gain (512 long: 0.90 .. 1.16, 768: 1.03 .. 1.42).
-  if (kernel_width(p->head_dim) == 128) return true;
-  return mean >= 5 * BKV || (longest >= BKV && items <= 512) || (mean >= 3 * BKV && items <= 1024);
+  // Wide heads gain from there on (1.03 .. 1.38; 0.96 where every document ends in a nearly empty tile).  For narrow ones what
+  // an item costs before its first step weighs more: with several items per CU only documents of some length gain
+  // (head_dim 64: 320 long 0.94 .. 1.02, 512 1.04 .. 1.25, 2048 1.3; head_dim 32: 512 long 0.92 .. 1.06, 768 1.01 .. 1.07,
+  // 2048 1.3 .. 1.5), with about one per CU also shorter ones (head_dim 64: 1.03 .. 1.5; head_dim 32: 200 long 1.0, 384 1.2).
+  if (chain_width(p->head_dim) == 128) return true;
+  const bool narrow = p->head_dim <= 32;
+  return mean >= (narrow ? 5 * BKV : 7 * BKV / 2) || (items <= 512 && longest >= (narrow ? 3 * BKV : BKV)) ||
+         (items <= 1024 && mean >= (narrow ? 3 * BKV : 15 * BKV / 8));
 }
 
 int backward_chained(const sba_problem* p, bool fixed, const void* schedule, size_t sched_bytes, const sba_view* q,
@@ -377,7 +392,7 @@ int backward_chained(const sba_problem* p, bool fixed, const void* schedule, siz
   a.inv_temp = c.inv_temp;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   Timer tm(2, s);
-  return (int)(p->dtype == SBA_F16 ? f16::launch_bwd_chain : bf16::launch_bwd_chain)(a, (p->flags & SBA_ATTEND_CURRENT) != 0, sz.n_q_max,
+  return (int)(p->dtype == SBA_F16 ? f16::launch_bwd_chain : bf16::launch_bwd_chain)(a, (p->flags & SBA_ATTEND_CURRENT) != 0, chain_wide(p, fixed, sz), sz.n_q_max,
                                                                                     device_cus(), s);
 }
 

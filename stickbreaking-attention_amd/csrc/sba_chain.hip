@@ -101,25 +101,30 @@ __global__ void __launch_bounds__(NT) chain_prep_kernel(const ChainArgs a) {
   }
 }
 
-// NSQ: 32-query blocks per step.  4 * NSQ score waves (one per 32-key block and query block) and 4 product waves.
+// NSQ: 32-query blocks per step.  4 * NSQ score waves (one per 32-key block and query block) and 4 product waves.  At head_dim
+// 128 registers leave room for one score wave per SIMD, whose vector work (180 instructions, 32 of them transcendental,
+// per block) is the step; at 64 and below two fit (168 registers), and a step of 64 queries takes 3750 cycles where two of 32
+// take 5800: 16 heads x 4 documents of 2048 at head_dim 64 166 us for 199, at head_dim 32 139 for 167 (two passes: 233, 216).
 template <int D, int U, bool AC, int NSQ>
 __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const ChainArgs a) {
   constexpr int KS = U / 16, DB = U / 32;
   constexpr int TQ = 32 * NSQ;      // queries per step
-  constexpr int RING = 6;           // Q / dO slots: tiles w-1 (dk) .. w+2 (scores) of step w and two in flight
-  constexpr int AHEAD = 4;
+  constexpr bool DEEP = NSQ == 1;   // score waves form block w + 2's products in step w, else block w + 1's
+  constexpr int RING = DEEP ? 6 : 5;     // Q / dO slots: tiles w-1 (dk) .. w+2 or w+1 (scores) of step w and two in flight
+  constexpr int AHEAD = RING - 2;
+  constexpr int PBUF = DEEP ? 3 : 2;     // staged p: with the weights, one step ahead of dz, or with dz
   constexpr int QTILE = TQ * D, PTILE = TQ * BKV;
   constexpr int DIAG = BKV / TQ;    // steps of an item whose queries may not see all of its keys: its last ones
   __shared__ __attribute__((aligned(16))) unsigned short Qs[RING * QTILE];
   __shared__ __attribute__((aligned(16))) unsigned short Gs[RING * QTILE];
-  __shared__ __attribute__((aligned(16))) unsigned short PZ[5 * PTILE];   // p: three buffers, dz: two buffers, [query][key]
+  __shared__ __attribute__((aligned(16))) unsigned short PZ[(PBUF + 2) * PTILE];   // p: PBUF buffers, dz: two buffers, [query][key]
   __shared__ float tot[2][NSQ][4][32];       // by step parity: every key block's sum of p (do.v) per query
   __shared__ int prefix[CHAIN_MAX_GROUPS];   // items of this XCD's queue up to and including each group
   __shared__ int mbox[2][8];
   __shared__ __attribute__((aligned(16))) unsigned short spare[4][512];   // where a product wave's copies of nothing go
   unsigned short* const Ps = PZ;
-  unsigned short* const Zs = PZ + 3 * PTILE;
-  static_assert(5 * PTILE >= BKV * D, "the key tile is staged in the p / dz buffers between items");
+  unsigned short* const Zs = PZ + PBUF * PTILE;
+  static_assert((PBUF + 2) * PTILE >= (DEEP ? 1 : 2) * BKV * D, "the key tile (and the value tile) is staged in the p / dz buffers between items");
 
   const int* sched = a.sched;
   const int4 hdr = *reinterpret_cast<const int4*>(sched);
@@ -272,7 +277,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       seen = 0;
       request_e(0, se0);
       request_e(1, se1);
-      request_e(2, se2);
+      if constexpr (DEEP) request_e(2, se2);
     };
     // the first AHEAD tiles of an item (first query block's score waves copy)
     auto open_tiles = [&](const ChainArgs& a, const Item& it) {
@@ -295,11 +300,11 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       int n = lane & 31, h = lane >> 5;
       asm volatile("" : "+v"(n), "+v"(h));
       const int r = 32 * kb + kperm(n);
-      const unsigned short* Vt = (kb < 2 ? Qs : Gs) + AHEAD * QTILE;
+      const unsigned short* Vt = DEEP ? (kb < 2 ? Qs : Gs) + AHEAD * QTILE : PZ + BKV * D;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         kf[ks] = lds_row8(PZ + swz_off<D>(r, 2 * ks + h));
-        vf[ks] = lds_row8(Vt + swz_off<D>(r & 63, 2 * ks + h));
+        vf[ks] = lds_row8(Vt + swz_off<D>(DEEP ? r & 63 : r, 2 * ks + h));
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
@@ -455,6 +460,91 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       post(6);
       post(7);
     };
+    // The same with one step less between a block's products and its weights, for three waves per SIMD (168 registers), which
+    // hide what the pipeline above hides: step w forms the products of block w + 1 next to dz of block w, stages p and
+    // dz of block w and then forms the weights of block w + 1 in their place.  `dc`, `dn`: do.v of the two blocks.
+    auto shallow = [&](auto first_tag, auto band_tag, const int w, const int slot, Weights& wc, f32x16& dc, f32x16& dn, float& se) __attribute__((always_inline)) {
+      constexpr bool FIRST = decltype(first_tag)::value, BAND = decltype(band_tag)::value;
+      const int par = w & 1;
+      float d_in = 0.0f, t0 = 0.0f, t1 = 0.0f, t2 = 0.0f;
+      if constexpr (!FIRST) {
+        d_in = d_next + poison;
+        if (kb > 0) t0 = tot[par][sq][0][n];
+        if (kb > 1) t1 = tot[par][sq][1][n];
+        if (kb > 2) t2 = tot[par][sq][2][n];
+      }
+      request_d(w + 1);
+      float e_in = se;
+      request_e(w + 3, se);
+      const unsigned short* Qt = Qs + slot * QTILE;
+      const unsigned short* Gt = Gs + slot * QTILE;
+      f32x16 x;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) { x[j] = 0.0f; dn[j] = 0.0f; }
+      el8 fq[2], fg[2];
+      auto pre = [&](int c) {
+        if (c >= KS) return;
+        fq[c & 1] = lds_row8(Qt + roff[c]);
+        fg[c & 1] = lds_row8(Gt + roff[c]);
+      };
+      auto post = [&](int c) {
+        if (c >= KS) return;
+        x = mfma32(kf[c], fq[c & 1], x);
+        dn = mfma32(vf[c], fg[c & 1], dn);
+        pre(c + 2);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      const int qw1 = (t_last - (w + 1)) * TQ + 32 * sq, qw0 = qw1 + TQ;
+      pre(0);
+      pre(1);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!FIRST) {
+        const float before = d_in + ((t0 + t1) + t2);
+        float dprev = h == 1 ? before + wc.lo : before;
+        float dz[16];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) { const float dj = fmaf(wc.p[j], dc[j], dprev); dz[j] = fmaf(wc.r[j], dj, -dprev); dprev = dj; }
+        post(0);
+        unsigned short* Zt = Zs + par * PTILE;
+        unsigned short* Pt = Ps + par * PTILE;
+        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h)) = pack8(dz);
+#pragma unroll
+        for (int j = 8; j < 16; ++j) { const float dj = fmaf(wc.p[j], dc[j], dprev); dz[j] = fmaf(wc.r[j], dj, -dprev); dprev = dj; }
+        post(1);
+        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h + 1)) = pack8(dz + 8);
+        if (kb == 3 && h == 1) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dprev), out_rs, row4 - w * (4 * TQ), 0, 0);
+        if (BAND && a.fuse && qw0 == k0) {
+#pragma unroll
+          for (int j = 0; j < 16; ++j) wc.p[j] += 16 * h + j == n ? rem_own : 0.0f;
+        }
+        *reinterpret_cast<el8*>(Pt + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h)) = pack8(wc.p);
+        *reinterpret_cast<el8*>(Pt + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h + 1)) = pack8(wc.p + 8);
+        post(2);
+        post(3);
+      } else {
+#pragma unroll
+        for (int c = 0; c < KS; ++c) post(c);
+      }
+      const int lim = qw1 + n - k0 - 16 * h + (AC ? 1 : 0);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        wc.r[j] = fast_rcp(1.0f + fast_exp2(a.c * x[j]));
+        if (BAND && !(j < lim)) wc.r[j] = 1.0f;
+      }
+      float ex[16];
+      if (BAND) e_in = sub_skip<AC>(k0, qw1) ? 0.0f : e_in;
+      (void)suffix_prod32_excl(wc.r, ex, h, e_in);
+      wc.p[0] = ex[0] - ex[0] * wc.r[0];
+#pragma unroll
+      for (int j = 1; j < 16; ++j) wc.p[j] = ex[j] - ex[j - 1];
+      float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 16; j += 2) { s0 = fmaf(wc.p[j], dn[j], s0); s1 = fmaf(wc.p[j + 1], dn[j + 1], s1); }
+      float lo, hi;
+      both_halves(s0 + s1, lo, hi);
+      wc.lo = lo;
+      if (h == 0) tot[par ^ 1][sq][kb][n] = lo + hi;
+    };
     // ends a step: the first score wave makes sure that what the others request behind the barrier is there, the second
     // publishes what this tile has finished (formed two steps ago and acknowledged since)
     auto finish = [&](int w) {
@@ -487,39 +577,60 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       lds_barrier();                 // tiles 0 .. AHEAD-1 and the K and V tiles have landed
       take_fragments();
       lds_barrier();                 // every wave has its share of K and V in registers: their places are free
-      f32x16 x0, x1, da0, da1, da2;
-      Weights wa, wb;
-      chains(0, x0, da0);
-      // weights of block 0 (as step -1), chains of block 1
-      step(Yes{}, Yes{}, RT{}, -1, wb, da2, x0, da0, wa, x1, da1, se0);
-      if (keeper) await(2);
-      lds_barrier();
-      int i = 0;
-      // Everything repeats with period six (ring slots, staging buffers, weights, scores, do.v sums, carries): step i = 6 m has
-      // block i's weights in wa, its do.v in da0, block i+1's scores in x1 and do.v in da1.
+      if constexpr (DEEP) {
+        f32x16 x0, x1, da0, da1, da2;
+        Weights wa, wb;
+        chains(0, x0, da0);
+        // weights of block 0 (as step -1), chains of block 1
+        step(Yes{}, Yes{}, RT{}, -1, wb, da2, x0, da0, wa, x1, da1, se0);
+        if (keeper) await(2);
+        lds_barrier();
+        int i = 0;
+        // Everything repeats with period six (ring slots, staging buffers, weights, scores, do.v sums, carries): step i = 6 m has
+        // block i's weights in wa, its do.v in da0, block i+1's scores in x1 and do.v in da1.
 #pragma unroll 1
-      for (; i + 6 < nsteps - DIAG - 2; i += 6) {
-        publish(i);     step(No{}, No{}, integral_constant<int, 2>{}, i, wa, da0, x1, da1, wb, x0, da2, se1);     finish(i);
-        publish(i + 1); step(No{}, No{}, integral_constant<int, 3>{}, i + 1, wb, da1, x0, da2, wa, x1, da0, se2); finish(i + 1);
-        publish(i + 2); step(No{}, No{}, integral_constant<int, 4>{}, i + 2, wa, da2, x1, da0, wb, x0, da1, se0); finish(i + 2);
-        publish(i + 3); step(No{}, No{}, integral_constant<int, 5>{}, i + 3, wb, da0, x0, da1, wa, x1, da2, se1); finish(i + 3);
-        publish(i + 4); step(No{}, No{}, integral_constant<int, 0>{}, i + 4, wa, da1, x1, da2, wb, x0, da0, se2); finish(i + 4);
-        publish(i + 5); step(No{}, No{}, integral_constant<int, 1>{}, i + 5, wb, da2, x0, da0, wa, x1, da1, se0); finish(i + 5);
-      }
+        for (; i + 6 < nsteps - DIAG - 2; i += 6) {
+          publish(i);     step(No{}, No{}, integral_constant<int, 2>{}, i, wa, da0, x1, da1, wb, x0, da2, se1);     finish(i);
+          publish(i + 1); step(No{}, No{}, integral_constant<int, 3>{}, i + 1, wb, da1, x0, da2, wa, x1, da0, se2); finish(i + 1);
+          publish(i + 2); step(No{}, No{}, integral_constant<int, 4>{}, i + 2, wa, da2, x1, da0, wb, x0, da1, se0); finish(i + 2);
+          publish(i + 3); step(No{}, No{}, integral_constant<int, 5>{}, i + 3, wb, da0, x0, da1, wa, x1, da2, se1); finish(i + 3);
+          publish(i + 4); step(No{}, No{}, integral_constant<int, 0>{}, i + 4, wa, da1, x1, da2, wb, x0, da0, se2); finish(i + 4);
+          publish(i + 5); step(No{}, No{}, integral_constant<int, 1>{}, i + 5, wb, da2, x0, da0, wa, x1, da1, se0); finish(i + 5);
+        }
 #pragma unroll 1
-      for (;; i += 6) {
-        if (i >= nsteps) break;
-        queue(i, m & 1);     publish(i);     step(No{}, Yes{}, RT{}, i, wa, da0, x1, da1, wb, x0, da2, se1);     finish(i);
-        if (i + 1 >= nsteps) break;
-        queue(i + 1, m & 1); publish(i + 1); step(No{}, Yes{}, RT{}, i + 1, wb, da1, x0, da2, wa, x1, da0, se2); finish(i + 1);
-        if (i + 2 >= nsteps) break;
-        queue(i + 2, m & 1); publish(i + 2); step(No{}, Yes{}, RT{}, i + 2, wa, da2, x1, da0, wb, x0, da1, se0); finish(i + 2);
-        if (i + 3 >= nsteps) break;
-        queue(i + 3, m & 1); publish(i + 3); step(No{}, Yes{}, RT{}, i + 3, wb, da0, x0, da1, wa, x1, da2, se1); finish(i + 3);
-        if (i + 4 >= nsteps) break;
-        queue(i + 4, m & 1); publish(i + 4); step(No{}, Yes{}, RT{}, i + 4, wa, da1, x1, da2, wb, x0, da0, se2); finish(i + 4);
-        if (i + 5 >= nsteps) break;
-        queue(i + 5, m & 1); publish(i + 5); step(No{}, Yes{}, RT{}, i + 5, wb, da2, x0, da0, wa, x1, da1, se0); finish(i + 5);
+        for (;; i += 6) {
+          if (i >= nsteps) break;
+          queue(i, m & 1);     publish(i);     step(No{}, Yes{}, RT{}, i, wa, da0, x1, da1, wb, x0, da2, se1);     finish(i);
+          if (i + 1 >= nsteps) break;
+          queue(i + 1, m & 1); publish(i + 1); step(No{}, Yes{}, RT{}, i + 1, wb, da1, x0, da2, wa, x1, da0, se2); finish(i + 1);
+          if (i + 2 >= nsteps) break;
+          queue(i + 2, m & 1); publish(i + 2); step(No{}, Yes{}, RT{}, i + 2, wa, da2, x1, da0, wb, x0, da1, se0); finish(i + 2);
+          if (i + 3 >= nsteps) break;
+          queue(i + 3, m & 1); publish(i + 3); step(No{}, Yes{}, RT{}, i + 3, wb, da0, x0, da1, wa, x1, da2, se1); finish(i + 3);
+          if (i + 4 >= nsteps) break;
+          queue(i + 4, m & 1); publish(i + 4); step(No{}, Yes{}, RT{}, i + 4, wa, da1, x1, da2, wb, x0, da0, se2); finish(i + 4);
+          if (i + 5 >= nsteps) break;
+          queue(i + 5, m & 1); publish(i + 5); step(No{}, Yes{}, RT{}, i + 5, wb, da2, x0, da0, wa, x1, da1, se0); finish(i + 5);
+        }
+      } else {
+        f32x16 da0, da1;
+        Weights wa;
+        shallow(Yes{}, Yes{}, -1, 0, wa, da1, da0, se0);
+        if (keeper) await(2);
+        lds_barrier();
+        int i = 0, slot = 1;
+        auto advance = [&]() { slot = slot + 1 == RING ? 0 : slot + 1; };
+#pragma unroll 1
+        for (; i + 1 < nsteps - 6; i += 2) {
+          publish(i);     shallow(No{}, No{}, i, slot, wa, da0, da1, se1);     advance(); finish(i);
+          publish(i + 1); shallow(No{}, No{}, i + 1, slot, wa, da1, da0, se0); advance(); finish(i + 1);
+        }
+#pragma unroll 1
+        for (; i < nsteps; i += 2) {
+          queue(i, m & 1);     publish(i);     shallow(No{}, Yes{}, i, slot, wa, da0, da1, se1);     advance(); finish(i);
+          if (i + 1 >= nsteps) break;
+          queue(i + 1, m & 1); publish(i + 1); shallow(No{}, Yes{}, i + 1, slot, wa, da1, da0, se0); advance(); finish(i + 1);
+        }
       }
       publish(nsteps);
       const bool more = read_box(m & 1, cur);
@@ -532,9 +643,10 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
     __builtin_amdgcn_s_setprio(0);
     const int pw = w - 4 * NSQ;
     const int ptid = pw * 64 + lane;
+    const int lane16 = lane * 16;
     const int mat = pw >> 1, half = pw & 1;       // (dv | dk) x 64 keys; all columns
     const bool has_dq = pw < NSQ * DB;            // 32 x 32 block of dq: query block pw / DB, columns 32 (pw % DB)
-    const int dsq = pw / DB, dcol = pw % DB;
+    const int dsq = has_dq ? pw / DB : 0, dcol = pw % DB;
     f32x16 acc[2][DB];
 #pragma unroll
     for (int kb2 = 0; kb2 < 2; ++kb2)
@@ -573,17 +685,24 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       // The K tile into the staging buffers and the V tile into the two ring slots the item's first tiles leave free, in
       // natural order.  (Fragments straight from global memory -- 32 rows of 32 bytes per instruction -- took
       // 6400 cycles of an item's beginning to issue, these copies 1000.)
-      static_assert(AHEAD + 2 <= RING && 2 * QTILE >= 64 * D, "half of the V tile per ring");
-      int l = ptid;
+      static_assert(!DEEP || (AHEAD + 2 <= RING && 2 * QTILE >= 64 * D), "half of the V tile per ring");
+      int l = lane16;
       asm volatile("" : "+v"(l));
+      l = pw * 64 + (l >> 4);
       const Rows krows = rows_of(a.k, it), vrows = rows_of(a.v, it);
       TileCopy<D, BKV, 256, false, true> kcopy;
       kcopy.init(l, krows.row_bytes, krows.used_bytes);
       kcopy.issue(krows, kt * BKV, PZ);
-      TileCopy<D, 64, 256, false, true> vcopy;
-      vcopy.init(l, vrows.row_bytes, vrows.used_bytes);
-      vcopy.issue(vrows, kt * BKV, Qs + AHEAD * QTILE);
-      vcopy.issue(vrows, kt * BKV + 64, Gs + AHEAD * QTILE);
+      if constexpr (DEEP) {
+        TileCopy<D, 64, 256, false, true> vcopy;
+        vcopy.init(l, vrows.row_bytes, vrows.used_bytes);
+        vcopy.issue(vrows, kt * BKV, Qs + AHEAD * QTILE);
+        vcopy.issue(vrows, kt * BKV + 64, Gs + AHEAD * QTILE);
+      } else {
+        TileCopy<D, BKV, 256, false, true> vcopy;
+        vcopy.init(l, vrows.row_bytes, vrows.used_bytes);
+        vcopy.issue(vrows, kt * BKV, PZ + BKV * D);
+      }
     };
     auto take_key_tile = [&]() {
       if (has_dq) {
@@ -596,7 +715,6 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
-    const int lane16 = lane * 16;
     Item nxt;
     open_item(a, cur);
 #pragma unroll 1
@@ -617,7 +735,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       // the waits count constants and no value on its way has to be moved where two paths join.
       f32x4 l0, l1, l2, l3;           // partial dq on its way in
       const unsigned short* const Ys = mat ? Qs : Gs;
-      constexpr int KQ = TQ / 16, KZ = BKV / 16, ZH = KZ / 2;
+      constexpr int KQ = TQ / 16, KZ = BKV / 16, ZH = DEEP ? KZ / 2 : 2;
       auto store_part = [&](const int w, const int i, const f32x16& dq, const bool store) __attribute__((always_inline)) {
         const f32x4 part = {dq[4 * i], dq[4 * i + 1], dq[4 * i + 2], dq[4 * i + 3]};
         const int soff = ((t_last - w + 1) * NSQ + dsq) * (D * 128);    // bytes of partial dq ahead of this query tile's 32 rows
@@ -647,7 +765,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         asm volatile("" : "+v"(xb[0]), "+v"(xb[1]), "+v"(yb[0]), "+v"(yb[1]), "+v"(zb));   // (the XORs stay in the loop)
         const int b = w - 1;
         const unsigned short* Zt = Zs + (b & 1) * PTILE;
-        const unsigned short* Xt = mat ? Zt : Ps + (b % 3) * PTILE;
+        const unsigned short* Xt = mat ? Zt : Ps + (b % PBUF) * PTILE;
         const unsigned short* Yt = Ys + (b % RING) * QTILE;
         const bool finished = b >= nsteps - DIAG;               // the queries of this tile's own keys: nothing is missing any more
         el8 zf[ZH], af[2], bf[DB];
@@ -678,6 +796,9 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
           if (ks & 1) product(ks >> 1);
         }
         if (finished) {
+          int at = lane16;      // (opaque: its offsets are not to be kept through the steps before)
+          asm volatile("" : "+v"(at));
+          const int n = (at >> 4) & 31, h = at >> 9;
           const int row = (t_last - b) * TQ + 32 * dsq + n;
           const Rows out = rows_of(a.dq, cur);
           store_block32_rows(dq, a.inv_temp, out, row < doc_len && has_dq ? row * (int)out.row_bytes : OUTSIDE, 32 * dcol, h);
@@ -703,6 +824,9 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         open_item(a, cur);
       }
       const Rows out = rows_of(mat ? a.dk : a.dv, done);
+      int at = lane16;
+      asm volatile("" : "+v"(at));
+      const int n = (at >> 4) & 31, h = at >> 9;
 #pragma unroll
       for (int kb2 = 0; kb2 < 2; ++kb2) {
         const int row = done.kt * BKV + 64 * half + 32 * kb2 + n;
@@ -726,6 +850,12 @@ template __global__ void bwd_chain_kernel<128, 96, true, 1>(const ChainArgs);
 
 template __global__ void bwd_chain_kernel<64, 64, false, 1>(const ChainArgs);
 template __global__ void bwd_chain_kernel<64, 64, true, 1>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 64, false, 2>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 64, true, 2>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 32, false, 1>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 32, true, 1>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 32, false, 2>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 32, true, 2>(const ChainArgs);
 
 template <int D, int U, int NSQ>
 static hipError_t launch_chain_d(const ChainArgs& a, bool ac, int n_q_max, int workgroups, hipStream_t s) {
@@ -736,8 +866,9 @@ static hipError_t launch_chain_d(const ChainArgs& a, bool ac, int n_q_max, int w
   return hipGetLastError();
 }
 
-hipError_t launch_bwd_chain(const ChainArgs& a, bool ac, int n_q_max, int workgroups, hipStream_t s) {
-  if (a.head_dim <= 64) return launch_chain_d<64, 64, 1>(a, ac, n_q_max, workgroups, s);
+hipError_t launch_bwd_chain(const ChainArgs& a, bool ac, bool wide, int n_q_max, int workgroups, hipStream_t s) {
+  if (a.head_dim <= 32) return wide ? launch_chain_d<64, 32, 2>(a, ac, n_q_max, workgroups, s) : launch_chain_d<64, 32, 1>(a, ac, n_q_max, workgroups, s);
+  if (a.head_dim <= 64) return wide ? launch_chain_d<64, 64, 2>(a, ac, n_q_max, workgroups, s) : launch_chain_d<64, 64, 1>(a, ac, n_q_max, workgroups, s);
   if (used_width(a.head_dim) == 96) return launch_chain_d<128, 96, 1>(a, ac, n_q_max, workgroups, s);
   return launch_chain_d<128, 128, 1>(a, ac, n_q_max, workgroups, s);
 }

@@ -1,6 +1,6 @@
-"""The one-pass backward (csrc/sba_chain.hip), forced wherever it is possible: documents at the edges of its 32-query steps
-and 128-key tiles and of the three steps a tile lags behind its predecessor, both kernel widths and heads narrower
-than them, against the oracle; and queues of many items per workgroup and many groups, against the two-pass form."""
+"""The one-pass backward (csrc/sba_chain.hip), forced wherever it is possible: documents at the edges of its steps of 32 and
+64 queries and 128-key tiles and of the three steps a tile lags behind its predecessor, both kernel widths and heads
+narrower than them, against the oracle; and queues of many items per workgroup and many groups, against the two-pass form."""
 import pytest
 import torch
 
@@ -27,9 +27,10 @@ def gradients(op, tensors, cu, longest, ac, grads):
 
 
 @pytest.mark.parametrize("ac", [False, True])
-@pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (96, torch.float16), (104, torch.bfloat16), (64, torch.bfloat16),
-                                     (40, torch.float16)])
-def test_tile_edges(form, d, dtype, ac):
+@pytest.mark.parametrize("steps,d,dtype", [(2, 128, torch.bfloat16), (2, 96, torch.float16), (2, 104, torch.bfloat16),
+                                           (2, 64, torch.bfloat16), (2, 32, torch.float16), (3, 64, torch.bfloat16),
+                                           (3, 40, torch.float16), (3, 24, torch.bfloat16)])
+def test_tile_edges(form, steps, d, dtype, ac):
     from stickbreaking_attention import sb_attn_varlen, sb_attn_varlen_fused
     lengths = [1, 32, 33, 127, 128, 129, 224, 256, 257, 550]
     H, used = 3, sum(lengths)
@@ -37,7 +38,7 @@ def test_tile_edges(form, d, dtype, ac):
     q, k, v, do = (t.to(dtype) for t in orc.make_inputs((H, T, d), 40 + d))
     drem = torch.randn((H, T), generator=torch.Generator().manual_seed(d)).to(dtype)
     cu = cu_from_lengths(lengths, device=DEV)
-    form(2)
+    form(steps)
     got = gradients(sb_attn_varlen, (q, k, v), cu, max(lengths), ac, (do, drem))
     fused = gradients(sb_attn_varlen_fused, (q, k, v), cu, max(lengths), ac, (do,))
     form(1)
@@ -49,8 +50,9 @@ def test_tile_edges(form, d, dtype, ac):
         assert_close(name + " of o + rem v", f[:, :used], f2[:, :used].float())
 
 
+@pytest.mark.parametrize("steps", [2, 3])
 @pytest.mark.parametrize("H,lengths", [(5, [37 + 61 * i % 400 for i in range(90)]), (12, [2000, 1, 900, 4000]), (3, [4600, 700])])
-def test_queues(form, H, lengths):
+def test_queues(form, steps, H, lengths):
     from stickbreaking_attention import sb_attn_varlen
     T = sum(lengths)
     tensors = orc.make_inputs((H, T, 64), T)
@@ -58,7 +60,7 @@ def test_queues(form, H, lengths):
     cu = cu_from_lengths(lengths, device=DEV)
     form(1)
     two = gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem))
-    form(2)
+    form(steps)
     first = gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem))
     again = gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem))
     for name, a, b, c in zip(("dq", "dk", "dv"), two, first, again):
