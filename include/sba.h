@@ -82,6 +82,10 @@ extern "C" {
                                    front of sba_*_bwd: same kernel, same bits, about 60 % of
                                    a forward's time.  No upstream counterpart             */
 
+#define SBA_F32_OUT        64u  /* o, rem, dq, dk and dv are float32 tensors and take the 16-bit
+                                   results converted, so that a float32 caller needs no pass
+                                   of its own for that (grad_o and grad_rem stay 16-bit)   */
+
 /* A strided view over [batch, heads, tokens, head_dim]; the last dimension is contiguous.
  * Strides are in ELEMENTS.  For packed variable-length input batch == 1 and stride_b is
  * ignored.  For per-row tensors (rem, grad_rem) the head_dim axis is absent. */
@@ -250,6 +254,10 @@ int sba_attn_bwd_chained(const sba_problem* p, const void* schedule, size_t sche
                          const sba_view* dq, const sba_view* dk, const sba_view* dv, void* stream);
 
 /* ---- misc ------------------------------------------------------------------------------- */
+
+/* The operands of a float32 caller: rounds n (at most 3) dense float32 arrays of counts[i] elements, multiples
+ * of 8 at 16-byte aligned addresses, to `dtype` (nearest even), all in one launch. */
+int sba_round_floats(int dtype, int n, const void* const* src, void* const* dst, const int64_t* counts, void* stream);
 
 /* Launch geometry of a problem: host arithmetic only, nothing is launched and no device is
  * looked at.  It has no counterpart upstream (Triton computes its grids inside the launchers,

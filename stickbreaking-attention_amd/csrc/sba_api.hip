@@ -93,12 +93,12 @@ int check_view(const sba_view* v, bool need_ptr) {
 // 16-byte vector loads/stores need every row start aligned: strides multiple of 8 elements.
 // Tile loads address a (document, head) slice with 32-bit byte offsets: the token stride must
 // keep every row of the slice (plus one tile of slack) below 2 GiB.
-int check_mat(const sba_view* v, const sba_problem* p) {
+int check_mat(const sba_view* v, const sba_problem* p, bool out = false) {
   int e = check_view(v, true);
   if (e) return e;
   if ((v->stride_b % 8) || (v->stride_h % 8) || (v->stride_t % 8) || ((uintptr_t)v->ptr % 16)) return SBA_E_STRIDE;
   if (v->stride_t < p->head_dim) return SBA_E_STRIDE;
-  if (((long long)p->tokens + 8 * BM) * v->stride_t * 2 >= (1ll << 31)) return SBA_E_SHAPE;
+  if (((long long)p->tokens + 8 * BM) * v->stride_t * (out && (p->flags & SBA_F32_OUT) ? 4 : 2) >= (1ll << 31)) return SBA_E_SHAPE;
   return 0;
 }
 
@@ -108,6 +108,12 @@ View to_view(const sba_view* v) {
   r.sb = v ? v->stride_b : 0;
   r.sh = v ? v->stride_h : 0;
   r.st = v ? v->stride_t : 0;
+  return r;
+}
+// An output's view.  The kernels address every tensor in 16-bit words, so float32 strides count double.
+View to_view_out(const sba_view* v, const sba_problem* p) {
+  View r = to_view(v);
+  if (p->flags & SBA_F32_OUT) { r.sb *= 2; r.sh *= 2; r.st *= 2; }
   return r;
 }
 
@@ -194,6 +200,7 @@ int fill_common(const sba_problem* p, bool fixed, const Sizes& sz, const void* s
   a->head_dim = p->head_dim;
   a->tokens = p->tokens;
   a->fuse = (p->flags & SBA_FUSE_REMAINDER) ? 1 : 0;
+  a->out_f32 = (p->flags & SBA_F32_OUT) ? 1 : 0;
   a->inv_temp = p->inv_temp;
   a->c = p->inv_temp * 1.4426950408889634f;
   return 0;
@@ -208,7 +215,7 @@ int forward(const sba_problem* p, bool fixed, const void* schedule, size_t sched
   const bool table_only = (p->flags & SBA_TABLE_ONLY) != 0;   // nothing but the carry table is written; v, o, rem are not looked at
   if (table_only && (stick == nullptr || weights != nullptr)) return SBA_E_NULL;
   if ((e = check_mat(q, p)) || (e = check_mat(k, p))) return e;
-  if (!table_only && ((e = check_mat(v, p)) || (e = check_mat(o, p)) || (e = check_view(rem, true)))) return e;
+  if (!table_only && ((e = check_mat(v, p)) || (e = check_mat(o, p, true)) || (e = check_view(rem, true)))) return e;
   if (weights != nullptr &&
       weights_bytes / sizeof(float) < (size_t)p->batch * p->heads * (size_t)p->tokens * (size_t)p->tokens)
     return SBA_E_WORKSPACE;
@@ -219,11 +226,11 @@ int forward(const sba_problem* p, bool fixed, const void* schedule, size_t sched
   if (sz.rows == 0) return 0;
   a.q = to_view(q); a.k = to_view(k);
   if (table_only) a.v = a.o = a.rem = to_view(k);   // (placeholders: the kernel touches none of them)
-  else { a.v = to_view(v); a.o = to_view(o); a.rem = to_view(rem); }
+  else { a.v = to_view(v); a.o = to_view_out(o, p); a.rem = to_view_out(rem, p); }
   a.stick = stick;
   a.weights = weights;
   a.clear_spare = fixed ? 0 : 1;
-  a.nan_pair = p->dtype == SBA_F16 ? 0x7e007e00u : 0x7fc07fc0u;
+  a.nan_pair = p->dtype == SBA_F16 && !a.out_f32 ? 0x7e007e00u : 0x7fc07fc0u;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   hipError_t he = hipSuccess;
   {   // (packed input without a single document still launches: the spare workgroups clear the outputs)
@@ -242,7 +249,7 @@ int backward(const sba_problem* p, bool fixed, const void* schedule, size_t sche
   int e = check_problem(p, fixed, &sz);
   if (e) return e;
   if ((e = check_mat(q, p)) || (e = check_mat(k, p)) || (e = check_mat(v, p)) || (e = check_mat(go, p)) ||
-      (e = check_mat(dq, p)) || (e = check_mat(dk, p)) || (e = check_mat(dv, p)))
+      (e = check_mat(dq, p, true)) || (e = check_mat(dk, p, true)) || (e = check_mat(dv, p, true)))
     return e;
   if (stick == nullptr || gtab == nullptr) return SBA_E_NULL;
   KArgs a;
@@ -252,7 +259,7 @@ int backward(const sba_problem* p, bool fixed, const void* schedule, size_t sche
   if (sz.rows == 0) return 0;
   a.q = to_view(q); a.k = to_view(k); a.v = to_view(v); a.go = to_view(go);
   a.grem = to_view(grem);
-  a.dq = to_view(dq); a.dk = to_view(dk); a.dv = to_view(dv);
+  a.dq = to_view_out(dq, p); a.dk = to_view_out(dk, p); a.dv = to_view_out(dv, p);
   a.stick = const_cast<float*>(stick);
   a.gtab = gtab;
   // The main kernel of the dk/dv pass fills a compute unit with one workgroup.  With many more key tiles than
@@ -269,7 +276,7 @@ int backward(const sba_problem* p, bool fixed, const void* schedule, size_t sche
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const bool ac = (p->flags & SBA_ATTEND_CURRENT) != 0, prod = (p->flags & SBA_PRODUCT_SPACE) != 0;
   a.clear_spare = fixed ? 0 : 1;
-  a.nan_pair = p->dtype == SBA_F16 ? 0x7e007e00u : 0x7fc07fc0u;
+  a.nan_pair = p->dtype == SBA_F16 && !a.out_f32 ? 0x7e007e00u : 0x7fc07fc0u;
   hipError_t he = hipSuccess;
   {
     Timer tm(1, s);
@@ -354,7 +361,7 @@ int backward_chained(const sba_problem* p, bool fixed, const void* schedule, siz
   int e = check_problem(p, fixed, &sz);
   if (e) return e;
   if ((e = check_mat(q, p)) || (e = check_mat(k, p)) || (e = check_mat(v, p)) || (e = check_mat(go, p)) ||
-      (e = check_mat(dq, p)) || (e = check_mat(dk, p)) || (e = check_mat(dv, p)))
+      (e = check_mat(dq, p, true)) || (e = check_mat(dk, p, true)) || (e = check_mat(dv, p, true)))
     return e;
   if (stick == nullptr || scratch == nullptr) return SBA_E_NULL;
   KArgs c;
@@ -368,7 +375,7 @@ int backward_chained(const sba_problem* p, bool fixed, const void* schedule, siz
   ChainArgs a;
   std::memset(&a, 0, sizeof(a));
   a.q = to_view(q); a.k = to_view(k); a.v = to_view(v); a.go = to_view(go); a.grem = to_view(grem);
-  a.dq = to_view(dq); a.dk = to_view(dk); a.dv = to_view(dv);
+  a.dq = to_view_out(dq, p); a.dk = to_view_out(dk, p); a.dv = to_view_out(dv, p);
   a.sched = c.sched;
   a.stick = stick;
   char* const base = static_cast<char*>(scratch);
@@ -385,8 +392,9 @@ int backward_chained(const sba_problem* p, bool fixed, const void* schedule, siz
   a.tiles = sz.n_kv_max;
   a.fixed = fixed ? 1 : 0;
   a.fuse = c.fuse;
+  a.out_f32 = c.out_f32;
   a.clear_spare = fixed ? 0 : 1;
-  a.nan_pair = p->dtype == SBA_F16 ? 0x7e007e00u : 0x7fc07fc0u;
+  a.nan_pair = p->dtype == SBA_F16 && !a.out_f32 ? 0x7e007e00u : 0x7fc07fc0u;
   a.max_doc_len = declared_max_doc_len(p, fixed);
   a.c = c.c;
   a.inv_temp = c.inv_temp;
@@ -572,6 +580,29 @@ int sba_varlen_fwd_static(const sba_problem* p, const sba_view* q, const sba_vie
   if ((e = sba_build_schedule(p, sched, SBA_STATIC_SCRATCH_BYTES, stream))) return e;
   return forward(p, false, sched, SBA_STATIC_SCRATCH_BYTES, q, k, v, o, rem, nullptr, 0, nullptr, 0, stream,
                  /*timed=*/false);   // (timing creates events)
+}
+
+int sba_round_floats(int dtype, int n, const void* const* src, void* const* dst, const int64_t* counts, void* stream) {
+  if (dtype != SBA_BF16 && dtype != SBA_F16) return SBA_E_DTYPE;
+  if (n < 1 || n > 3) return SBA_E_SHAPE;
+  if (src == nullptr || dst == nullptr || counts == nullptr) return SBA_E_NULL;
+  RoundArgs a;
+  std::memset(&a, 0, sizeof(a));
+  int64_t groups = 0;
+  for (int i = 0; i < 3; ++i) {
+    if (i < n) {
+      if (counts[i] < 0 || counts[i] % 8) return SBA_E_SHAPE;
+      if (counts[i] > 0 && (src[i] == nullptr || dst[i] == nullptr)) return SBA_E_NULL;
+      if ((reinterpret_cast<uintptr_t>(src[i]) | reinterpret_cast<uintptr_t>(dst[i])) & 15) return SBA_E_STRIDE;
+      a.src[i] = static_cast<const float*>(src[i]);
+      a.dst[i] = static_cast<unsigned short*>(dst[i]);
+      groups += counts[i] / 8;
+    }
+    a.upto[i] = groups;
+  }
+  int e;
+  if ((e = check_arch())) return e;
+  return groups == 0 ? 0 : (int)launch_round_f32(a, dtype == SBA_F16, reinterpret_cast<hipStream_t>(stream));
 }
 
 int sba_launch_geometry(const sba_problem* p, sba_geometry* out) {

@@ -130,9 +130,9 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dq_kernel(const KArgs
       int row0, row1;
       unsigned pair;
       spare_rows(refused, slot, hdr.y, sched[SCHED_TOTAL], a.tokens, a.nan_pair, row0, row1, pair);
-      fill_rows16(a.dq, head, row0, row1, a.head_dim, pair, threadIdx.x, NT);
-      fill_rows16(a.dk, head, row0, row1, a.head_dim, pair, threadIdx.x, NT);
-      fill_rows16(a.dv, head, row0, row1, a.head_dim, pair, threadIdx.x, NT);
+      fill_rows16(a.dq, head, row0, row1, a.head_dim << a.out_f32, pair, threadIdx.x, NT);
+      fill_rows16(a.dk, head, row0, row1, a.head_dim << a.out_f32, pair, threadIdx.x, NT);
+      fill_rows16(a.dv, head, row0, row1, a.head_dim << a.out_f32, pair, threadIdx.x, NT);
     }
     return;
   }
@@ -320,7 +320,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dq_kernel(const KArgs
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   if (pend_ix >= 0 && qvalid && h == 0) gtab[(unsigned)(pend_ix + qrow)] = Cst[w][n];
   lds_barrier();   // every wave is done with the K/V tiles: their memory becomes the dq staging area
-  store_block32<D, U>(Ks + w * 32 * D, dqacc, a.inv_temp, dqb, a.dq.st, qw0, t.doc_len, a.head_dim, lane);
+  store_block32<D, U>(Ks + w * 32 * D, dqacc, a.inv_temp, dqb, a.dq.st, qw0, t.doc_len, a.head_dim, lane, a.out_f32);
 }
 
 // -------------------------------------------------------------------------------------------
@@ -966,7 +966,7 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
 #pragma unroll
       for (int kb2 = 0; kb2 < 2; ++kb2) {
         store_block32<D, U>(scratch, acc[kb2], mat ? a.inv_temp : 1.0f, outb, ov.st, cur.kt * BKV + 64 * half + 32 * kb2,
-                         cur.doc_len, a.head_dim, lane_e);
+                         cur.doc_len, a.head_dim, lane_e, a.out_f32);
 #pragma unroll
         for (int j = 0; j < DB; ++j)
 #pragma unroll
@@ -1200,9 +1200,9 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
     for (int qblk = kblk; qblk < nblk; ++qblk) block(std::integral_constant<int, 2>{}, acc_v, acc_k, qblk, 32 * qblk);
     // the private piece becomes the output scratch (at most its size)
     static_assert(STREAM || 2 * 32 * 32 >= 32 * D, "the staging piece of a wave doubles as its output scratch");
-    store_block32<D, U>(Pt, acc_v, 1.0f, dvb, a.dv.st, k0, L, a.head_dim, lane);
+    store_block32<D, U>(Pt, acc_v, 1.0f, dvb, a.dv.st, k0, L, a.head_dim, lane, a.out_f32);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    store_block32<D, U>(Pt, acc_k, a.inv_temp, dkb, a.dk.st, k0, L, a.head_dim, lane);
+    store_block32<D, U>(Pt, acc_k, a.inv_temp, dkb, a.dk.st, k0, L, a.head_dim, lane, a.out_f32);
   } else {
     // Two passes over the queries, dv first and dk second; the scores are formed in each.
     // Segment s (SEG query rows) sits in buffer s & 1.  At its top every wave is done with segment s - 1,
@@ -1230,8 +1230,8 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
       }
       lds_barrier();            // every wave is done with the buffers: they become the output staging
       if (active) {
-        if constexpr (decltype(what_tag)::value == 0) store_block32<D, U>(scratch, acc, 1.0f, dvb, a.dv.st, k0, L, a.head_dim, lane);
-        else store_block32<D, U>(scratch, acc, a.inv_temp, dkb, a.dk.st, k0, L, a.head_dim, lane);
+        if constexpr (decltype(what_tag)::value == 0) store_block32<D, U>(scratch, acc, 1.0f, dvb, a.dv.st, k0, L, a.head_dim, lane, a.out_f32);
+        else store_block32<D, U>(scratch, acc, a.inv_temp, dkb, a.dk.st, k0, L, a.head_dim, lane, a.out_f32);
       }
     };
     pass(std::integral_constant<int, 0>{});

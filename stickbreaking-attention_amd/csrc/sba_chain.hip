@@ -63,9 +63,9 @@ __global__ void __launch_bounds__(NT) chain_prep_kernel(const ChainArgs a) {
       int row0, row1;
       unsigned pair;
       spare_rows(refused, slot, hdr.y, sched[SCHED_TOTAL], a.tokens, a.nan_pair, row0, row1, pair);
-      fill_rows16(a.dq, head, row0, row1, a.head_dim, pair, tid, NT);
-      fill_rows16(a.dk, head, row0, row1, a.head_dim, pair, tid, NT);
-      fill_rows16(a.dv, head, row0, row1, a.head_dim, pair, tid, NT);
+      fill_rows16(a.dq, head, row0, row1, a.head_dim << a.out_f32, pair, tid, NT);
+      fill_rows16(a.dk, head, row0, row1, a.head_dim << a.out_f32, pair, tid, NT);
+      fill_rows16(a.dv, head, row0, row1, a.head_dim << a.out_f32, pair, tid, NT);
     }
     return;
   }
@@ -801,7 +801,9 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
           const int n = (at >> 4) & 31, h = at >> 9;
           const int row = (t_last - b) * TQ + 32 * dsq + n;
           const Rows out = rows_of(a.dq, cur);
-          store_block32_rows(dq, a.inv_temp, out, row < doc_len && has_dq ? row * (int)out.row_bytes : OUTSIDE, 32 * dcol, h);
+#pragma unroll
+          for (int j = 0; j < 16; ++j) dq[j] *= a.inv_temp;      // (in place: it is not needed unscaled, and there is no register to spare)
+          store_block32_rows(dq, 1.0f, out, row < doc_len && has_dq ? row * (int)out.row_bytes : OUTSIDE, 32 * dcol, h, a.out_f32);
         }
 #pragma unroll
         for (int i = 0; i < (REST > OPS ? REST : OPS); ++i) {
@@ -833,7 +835,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         const int off = row < done.doc_len ? row * (int)out.row_bytes : OUTSIDE;
 #pragma unroll
         for (int j = 0; j < DB; ++j) {
-          store_block32_rows(acc[kb2][j], mat ? a.inv_temp : 1.0f, out, off, 32 * j, h);
+          store_block32_rows(acc[kb2][j], mat ? a.inv_temp : 1.0f, out, off, 32 * j, h, a.out_f32);
 #pragma unroll
           for (int e = 0; e < 16; ++e) acc[kb2][j][e] = 0.0f;
         }

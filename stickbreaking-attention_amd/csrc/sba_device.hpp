@@ -93,8 +93,8 @@ __device__ inline void fill_rows16(const View& v, int head, int row0, int row1, 
                                    int tid, int nthreads) {
   if (v.ptr == nullptr || row1 <= row0) return;
   unsigned short* base = reinterpret_cast<unsigned short*>(v.ptr) + head * v.sh;
-  if (width == 1) {
-    for (int r = row0 + tid; r < row1; r += nthreads) base[(int64_t)r * v.st] = (unsigned short)pair;
+  if (width <= 2) {           // per-row values (float32: two words)
+    for (int i = width * row0 + tid; i < width * row1; i += nthreads) base[(int64_t)(i / width) * v.st + i % width] = (unsigned short)(i % width ? pair >> 16 : pair);
     return;
   }
   const int c8 = width / 8;
@@ -428,11 +428,25 @@ __device__ __forceinline__ void stick_weights_fwd(const f32x16& x, float c, int 
 // D/16 fully coalesced 16-byte stores per lane.  Wave-private: no workgroup barrier inside,
 // but the caller must make sure nobody else still uses the scratch memory.
 // ---------------------------------------------------------------------------------------------
+// f32: the output is a float32 tensor (its stride still counts 16-bit words) of the same values; then a register of
+// the wave is two 128-byte pieces of rows and needs no detour.
 // (U: columns the accumulators cover, a multiple of 32 up to the row width D of the scratch; head_dim <= U)
 template <int D, int U = D>
 __device__ __forceinline__ void store_block32(unsigned short* scratch, const f32x16 (&acc)[U / 32], float scale,
-                                              elem_t* out, int64_t stride_t, int row0, int limit, int head_dim, int lane) {
+                                              elem_t* out, int64_t stride_t, int row0, int limit, int head_dim, int lane, bool f32) {
   const int n = lane & 31, h = lane >> 5;
+  if (f32) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = row0 + 8 * (i >> 2) + 4 * h + (i & 3);
+      float* const to = reinterpret_cast<float*>(out + (int64_t)row * stride_t) + n;
+#pragma unroll
+      for (int db = 0; db < U / 32; ++db)
+        if (row < limit && 32 * db + n < head_dim) to[32 * db] = (float)(elem_t)(acc[db][i] * scale);
+      __builtin_amdgcn_sched_barrier(0);   // (one row's address at a time)
+    }
+    return;
+  }
   elem_t* sc = reinterpret_cast<elem_t*>(scratch);
 #pragma unroll
   for (int db = 0; db < U / 32; ++db) {
@@ -461,8 +475,21 @@ __device__ __forceinline__ void store_block32(unsigned short* scratch, const f32
 template <int D, int U, class RowScale>
 __device__ __forceinline__ void store_block32_axpy(unsigned short* scratch, const f32x16 (&acc)[U / 32], float scale,
                                                    elem_t* out, int64_t stride_t, int row0, int limit, int head_dim, int lane,
-                                                   const elem_t* addend, int64_t addend_stride_t, RowScale rowscale) {
+                                                   const elem_t* addend, int64_t addend_stride_t, bool f32, RowScale rowscale) {
   const int n = lane & 31, h = lane >> 5;
+  if (f32) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = 8 * (i >> 2) + 4 * h + (i & 3);
+      const float f = rowscale(r);
+#pragma unroll
+      for (int db = 0; db < U / 32; ++db)
+        if (row0 + r < limit && 32 * db + n < head_dim)
+          reinterpret_cast<float*>(out + (int64_t)(row0 + r) * stride_t)[32 * db + n] =
+              (float)(elem_t)fmaf(f, (float)addend[(int64_t)(row0 + r) * addend_stride_t + 32 * db + n], (float)(elem_t)(acc[db][i] * scale));
+    }
+    return;
+  }
   elem_t* sc = reinterpret_cast<elem_t*>(scratch);
 #pragma unroll
   for (int db = 0; db < U / 32; ++db) {
@@ -547,7 +574,19 @@ __device__ __forceinline__ el8 load_frag(const Rows& r, int row, int col_bytes) 
 // = column 8*(i/4) + 4*h + i%4 of a 32-wide block): the half-waves exchange packed quads so that every
 // lane holds 8 consecutive columns of its row, two 16-byte stores per block.  `off`: byte offset of the lane's row in
 // the buffer, or OUTSIDE for a row that is not to be stored (the stores are issued either way: their number is known).
-__device__ __forceinline__ void store_block32_rows(const f32x16& acc, float scale, const Rows& out, int off, int col0, int h) {
+// f32: a float32 tensor of the same values, a quad of the lane's columns at a time.
+__device__ __forceinline__ void store_block32_rows(const f32x16& acc, float scale, const Rows& out, int off, int col0, int h, bool f32) {
+  if (f32) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      u32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = __builtin_bit_cast(unsigned, (float)(elem_t)(acc[4 * g + e] * scale));
+      const int bytes = 4 * (col0 + 8 * g + 4 * h);
+      __builtin_amdgcn_raw_buffer_store_b128(v, out.rsrc, bytes < 2 * out.used_bytes ? off + bytes : OUTSIDE, 0, 0);
+    }
+    return;
+  }
 #pragma unroll
   for (int g = 0; g < 4; g += 2) {
     u32x4 v;

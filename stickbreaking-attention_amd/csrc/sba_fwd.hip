@@ -46,8 +46,8 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
       int row0, row1;
       unsigned pair;
       spare_rows(refused, slot, hdr.y, sched[SCHED_TOTAL], a.tokens, a.nan_pair, row0, row1, pair);
-      fill_rows16(a.o, head, row0, row1, a.head_dim, pair, threadIdx.x, NT);
-      fill_rows16(a.rem, head, row0, row1, 1, pair, threadIdx.x, NT);
+      fill_rows16(a.o, head, row0, row1, a.head_dim << a.out_f32, pair, threadIdx.x, NT);
+      fill_rows16(a.rem, head, row0, row1, 1 << a.out_f32, pair, threadIdx.x, NT);
     }
     return;
   }
@@ -204,7 +204,11 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
   // epilogue: rem = what is left of the stick; o rows in the accumulator layout
   const float r = PROD ? carry : fast_exp2(carry);
   if (h == 0 && qvalid) {
-    if (!TAB) rb[(int64_t)qrow * a.rem.st] = (elem_t)r;
+    if (!TAB) {
+      elem_t* const at = rb + (int64_t)qrow * a.rem.st;
+      if (a.out_f32) *reinterpret_cast<float*>(at) = (float)(elem_t)r;
+      else *at = (elem_t)r;
+    }
     // rem in full precision for the backward of the fused output (last plane of the table)
     if (stick != nullptr) stick[(unsigned)(tab_rowplane32(t.doc_len) + qrow)] = r;
   }
@@ -212,10 +216,10 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
   lds_barrier();   // every wave is done with the K/V tiles: their memory becomes the o staging area
   if (a.fuse) {
     // what every caller computes next (upstream tests/test_varlen.py:101): o + rem * v
-    store_block32_axpy<D, U>(smem + w * 32 * D, oacc, 1.0f, ob, a.o.st, qw0, t.doc_len, a.head_dim, lane, vb, a.v.st,
+    store_block32_axpy<D, U>(smem + w * 32 * D, oacc, 1.0f, ob, a.o.st, qw0, t.doc_len, a.head_dim, lane, vb, a.v.st, a.out_f32,
                           [&](int row) { return __shfl(r, row, 64); });
   } else {
-    store_block32<D, U>(smem + w * 32 * D, oacc, 1.0f, ob, a.o.st, qw0, t.doc_len, a.head_dim, lane);
+    store_block32<D, U>(smem + w * 32 * D, oacc, 1.0f, ob, a.o.st, qw0, t.doc_len, a.head_dim, lane, a.out_f32);
   }
 }
 

@@ -26,7 +26,8 @@ struct KArgs {
   int fuse;                    // the output is o + rem * v (and grad_o is the gradient of that)
   int clear_spare;             // packed input: spare workgroups clear the rows that belong to no document (or fill
                                // everything with NaN when the launch is refused)
-  unsigned nan_pair;           // two NaNs of the 16-bit element type
+  unsigned nan_pair;           // two NaNs of the 16-bit element type (one of float32 outputs)
+  int out_f32;                 // outputs are float32; their strides still count 16-bit words (see to_view_out)
   int64_t tab_stride;          // carry-table entries per head the caller's tables hold
   int max_doc_len;             // backward: the longest document the caller declared (its grids are sized with it;
                                // the kernels refuse to run when the scheduler found a longer one)
@@ -56,11 +57,10 @@ struct ChainArgs {
   int64_t tab_stride;
   int docs_off;                // int32 offset of the ranked documents inside `sched`
   int n_docs, heads, head_dim, tokens, tiles;
-  int fixed, fuse, clear_spare;
+  int fixed, fuse, clear_spare, out_f32;
   unsigned nan_pair;
   int max_doc_len;
   float c, inv_temp;
-  int pad;
 };
 
 // Pointers rebuilt from integer words are generic pointers to the compiler (64-bit flat addresses in
@@ -109,6 +109,13 @@ inline unsigned launch_grid(const KArgs& a, long long n_items) {
   return (unsigned)(persistent ? resident : n_items);
 }
 
+// Arrays of sba_round_floats: 8-element groups, `upto` counted over the arrays so far.
+struct RoundArgs {
+  const float* src[3];
+  unsigned short* dst[3];
+  int64_t upto[3];
+};
+
 struct SchedArgs {
   const void* cu;   // null for fixed-length
   int cu_is64;
@@ -119,6 +126,7 @@ struct SchedArgs {
 };
 
 hipError_t launch_schedule(const SchedArgs& a, hipStream_t s);
+hipError_t launch_round_f32(const RoundArgs& a, bool f16, hipStream_t s);
 
 // Key-tile slots the two kernels of the dk/dv pass are launched over (one workgroup per slot and
 // head).  Every workgroup of the main kernel reads the tile descriptor of its slot BEFORE it knows

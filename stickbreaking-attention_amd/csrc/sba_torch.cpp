@@ -113,6 +113,36 @@ Tensor as_caller(const Tensor& t, int64_t d, at::ScalarType dt) {
   return r.scalar_type() == dt ? r : r.to(dt);
 }
 
+// Tensors of a float32 caller that need nothing but rounding (dense, head_dim and addresses fit the kernels): all of them
+// in one launch of sba_round_floats.  False: nothing was done, every tensor goes its own way.
+bool rounded(std::initializer_list<const Tensor*> from, std::initializer_list<Tensor*> to, int64_t d, at::ScalarType ct, void* stream) {
+  if (d % 8) return false;
+  for (const Tensor* t : from) {
+    bool ok = t->scalar_type() == at::kFloat && t->is_non_overlapping_and_dense() && reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0 && t->stride(-1) == 1;
+    for (int64_t i = 0; i + 1 < t->dim(); ++i) ok = ok && t->stride(i) % 8 == 0;
+    if (!ok) return false;
+  }
+  const void* src[3];
+  void* dst[3];
+  int64_t counts[3];
+  int n = 0;
+  auto out = to.begin();
+  for (const Tensor* t : from) {
+    **out = at::empty_like(*t, t->options().dtype(ct));
+    src[n] = t->data_ptr();
+    dst[n] = (*out)->data_ptr();
+    counts[n++] = t->numel();
+    ++out;
+  }
+  check(sba_round_floats(ct == at::kHalf ? SBA_F16 : SBA_BF16, n, src, dst, counts, stream), "sba_round_floats");
+  return true;
+}
+
+// float32 outputs straight from the kernels: where no column has to be cut off and 32-bit offsets reach every row.
+bool writes_f32(const Tensor& like, int64_t d, bool fixed) {
+  return like.size(-1) == d && (like.size(fixed ? 2 : 1) + 1024) * like.stride(fixed ? 2 : 1) * 4 < (int64_t(1) << 31);
+}
+
 // The scratch of a backward (gradient table, or the one-pass form's): one grow-only buffer per (device, stream), shared by every layer (the dk/dv pass
 // of one backward has read it before the next backward on that stream writes it).  Packed documents change
 // the size with every batch; growth goes to the next eighth of a power of two, and by at least a quarter.
@@ -147,11 +177,19 @@ struct Attention : public torch::autograd::Function<Attention> {
     const c10::DeviceGuard guard(q.device());
     const int64_t d = q.size(-1), dpad = padded_dim(d);
     const at::ScalarType dt = q.scalar_type(), ct = compute_type(dt);
-    const Tensor qp = prepared(q, dpad, ct), kp = prepared(k, dpad, ct), vp = prepared(v, dpad, ct);
-    Tensor o = at::empty_like(qp), rem = at::empty_like(qp.select(-1, 0));
+    void* const stream = current_stream(q);
+    Tensor qp, kp, vp;
+    if (dt != at::kFloat || !rounded({&q, &k, &v}, {&qp, &kp, &vp}, d, ct, stream)) {
+      qp = prepared(q, dpad, ct);
+      kp = prepared(k, dpad, ct);
+      vp = prepared(v, dpad, ct);
+    }
+    const bool f32 = dt == at::kFloat && writes_f32(qp, d, c.fixed);
+    const auto out = qp.options().dtype(f32 ? at::kFloat : ct);
+    Tensor o = at::empty_like(qp, out), rem = at::empty_like(qp.select(-1, 0), out);
     const Tensor table = c.need_table ? at::empty({c.table_floats}, qp.options().dtype(at::kFloat)) : Tensor();
-    const sba_problem p = problem(qp, c);
-    void* const stream = current_stream(qp);
+    sba_problem p = problem(qp, c);
+    if (f32) p.flags |= SBA_F32_OUT;
     void* const sched = c.sched.data_ptr();
     const size_t sched_bytes = (size_t)c.sched.numel();
     if (c.build) check(sba_build_schedule(&p, sched, sched_bytes, stream), "sba_build_schedule");
@@ -188,12 +226,18 @@ struct Attention : public torch::autograd::Function<Attention> {
     c.fixed = ctx->saved_data["fixed"].toBool();
     const int64_t d = ctx->saved_data["d"].toInt(), types = ctx->saved_data["types"].toInt(), dpad = qp.size(-1);
     const at::ScalarType ct = qp.scalar_type();
-    const Tensor go = grads[0].defined() ? prepared(grads[0], dpad, ct) : at::zeros_like(qp);   // (undefined: only rem was used)
+    void* const stream = current_stream(qp);
+    Tensor go;
+    if (!grads[0].defined()) go = at::zeros_like(qp);   // (only rem was used)
+    else if (!rounded({&grads[0]}, {&go}, dpad, ct, stream)) go = prepared(grads[0], dpad, ct);
     Tensor gr = grads.size() > 1 ? grads[1] : Tensor();
     if (gr.defined() && gr.scalar_type() != ct) gr = gr.to(ct);
-    Tensor dq = at::empty_like(qp), dk = at::empty_like(kp), dv = at::empty_like(vp);
-    const sba_problem p = problem(qp, c);
-    void* const stream = current_stream(qp);
+    constexpr int64_t kAllFloat = ((int64_t)at::kFloat << 16) | ((int64_t)at::kFloat << 8) | (int64_t)at::kFloat;
+    const bool f32 = types == kAllFloat && writes_f32(qp, d, c.fixed) && writes_f32(kp, d, c.fixed) && writes_f32(vp, d, c.fixed);
+    const auto out = qp.options().dtype(f32 ? at::kFloat : ct);
+    Tensor dq = at::empty_like(qp, out), dk = at::empty_like(kp, out), dv = at::empty_like(vp, out);
+    sba_problem p = problem(qp, c);
+    if (f32) p.flags |= SBA_F32_OUT;
     const sba_view vq = view(qp, c.fixed), vk = view(kp, c.fixed), vv = view(vp, c.fixed), vg = view(go, c.fixed), vr = view(gr, c.fixed);
     const sba_view wq = view(dq, c.fixed), wk = view(dk, c.fixed), wv = view(dv, c.fixed);
     const size_t chain_bytes = sba_chain_scratch_bytes(&p);   // 0: the two-pass form
