@@ -305,7 +305,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dq_kernel(const KArgs
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-        for (int db = 0; db < DB; ++db) dqacc[db] = mfma32(zf[tt], ktr[tt][db], dqacc[db]);
+        for (int db = 0; db < DB; ++db) dqacc[db] = mfma32(ktr[tt][db], zf[tt], dqacc[db]);   // (dq^T: see store_block32_rows)
     }
     ce[0] = ce_next[0];
     ce[1] = ce_next[1];
@@ -319,8 +319,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dq_kernel(const KArgs
 
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   if (pend_ix >= 0 && qvalid && h == 0) gtab[(unsigned)(pend_ix + qrow)] = Cst[w][n];
-  lds_barrier();   // every wave is done with the K/V tiles: their memory becomes the dq staging area
-  store_block32<D, U>(Ks + w * 32 * D, dqacc, a.inv_temp, dqb, a.dq.st, qw0, t.doc_len, a.head_dim, lane, a.out_f32);
+  store_rows(dqacc, a.inv_temp, make_rows(dqb, a.dq.st, t.doc_len, a.head_dim), qrow, t.doc_len, h, a.out_f32);
 }
 
 // -------------------------------------------------------------------------------------------
@@ -927,7 +926,7 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
 #pragma unroll
         for (int kb2 = 0; kb2 < 2; ++kb2)
 #pragma unroll
-          for (int j = 0; j < DB; ++j) acc[kb2][j] = mfma32(af[ks][kb2], cur[ks][j], acc[kb2][j]);
+          for (int j = 0; j < DB; ++j) acc[kb2][j] = mfma32(cur[ks][j], af[ks][kb2], acc[kb2][j]);
         read_y(i, nxt, ks);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -950,11 +949,7 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
         iter(i, ya, yb);
         if (i + 1 <= nsteps) iter(i + 1, yb, ya);
       }
-      // dk / dv leave through ring slots 4 and 5, which nothing uses between the barrier of the item's last
-      // score step and the next item's first barrier (the score waves are filling slots 0 .. AHEAD-1 with the
-      // next item's first tiles by now; the staging buffers may still be feeding another product wave's last
-      // products).  This wave reaches that barrier only after the stores below.
-      static_assert(AHEAD + 2 <= RING, "two ring slots free for the output staging");
+      // (the score waves are filling slots 0 .. AHEAD-1 with the next item's first tiles by now)
       Item nxt = cur;
       const int next = next_item(m & 1, nxt);
       const KArgs a = fresh_args();          // (see open_item)
@@ -962,11 +957,10 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
       asm volatile("" : "+v"(lane_e));
       const View& ov = mat ? a.dk : a.dv;
       elem_t* outb = reinterpret_cast<elem_t*>(ov.ptr) + cur.batch * ov.sb + cur.head * ov.sh + (int64_t)cur.tok_start * ov.st;
-      unsigned short* scratch = (rw & 2 ? Gs : Qs) + (AHEAD + (rw & 1)) * QTILE;
+      const Rows out = make_rows(outb, ov.st, cur.doc_len, a.head_dim);
 #pragma unroll
       for (int kb2 = 0; kb2 < 2; ++kb2) {
-        store_block32<D, U>(scratch, acc[kb2], mat ? a.inv_temp : 1.0f, outb, ov.st, cur.kt * BKV + 64 * half + 32 * kb2,
-                         cur.doc_len, a.head_dim, lane_e, a.out_f32);
+        store_rows(acc[kb2], mat ? a.inv_temp : 1.0f, out, cur.kt * BKV + 64 * half + 32 * kb2 + (lane_e & 31), cur.doc_len, lane_e >> 5, a.out_f32);
 #pragma unroll
         for (int j = 0; j < DB; ++j)
 #pragma unroll
@@ -1174,9 +1168,9 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
       const unsigned short* Qr = Qs + (lrow0 + 16 * ks) * D;
 #pragma unroll
       for (int j = 0; j < DB; ++j) {
-        if constexpr (DV) acc[j] = mfma32(ap, lds_tr8(Gr + yoff[0][j], Gr + yoff[1][j]), acc[j]);
-        if constexpr (WHAT == 1) acc[j] = mfma32(az, lds_tr8(Qr + yoff[0][j], Qr + yoff[1][j]), acc[j]);
-        if constexpr (WHAT == 2) acc2[j] = mfma32(az, lds_tr8(Qr + yoff[0][j], Qr + yoff[1][j]), acc2[j]);
+        if constexpr (DV) acc[j] = mfma32(lds_tr8(Gr + yoff[0][j], Gr + yoff[1][j]), ap, acc[j]);
+        if constexpr (WHAT == 1) acc[j] = mfma32(lds_tr8(Qr + yoff[0][j], Qr + yoff[1][j]), az, acc[j]);
+        if constexpr (WHAT == 2) acc2[j] = mfma32(lds_tr8(Qr + yoff[0][j], Qr + yoff[1][j]), az, acc2[j]);
         if constexpr (D > 128) { if (j % 4 == 3 || j == DB - 1) __builtin_amdgcn_sched_barrier(0); }
       }
     }
@@ -1191,6 +1185,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
   };
   elem_t* dvb = reinterpret_cast<elem_t*>(a.dv.ptr) + t.batch * a.dv.sb + head * a.dv.sh + tok0 * a.dv.st;
   elem_t* dkb = reinterpret_cast<elem_t*>(a.dk.ptr) + t.batch * a.dk.sb + head * a.dk.sh + tok0 * a.dk.st;
+  const Rows dvrows = make_rows(dvb, a.dv.st, L, a.head_dim), dkrows = make_rows(dkb, a.dk.st, L, a.head_dim);
   if constexpr (!STREAM) {
     f32x16 acc_v[DB], acc_k[DB];
     clear(acc_v);
@@ -1198,17 +1193,12 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
     // query blocks at or after the key block (those before it see none of these keys)
 #pragma unroll 1
     for (int qblk = kblk; qblk < nblk; ++qblk) block(std::integral_constant<int, 2>{}, acc_v, acc_k, qblk, 32 * qblk);
-    // the private piece becomes the output scratch (at most its size)
-    static_assert(STREAM || 2 * 32 * 32 >= 32 * D, "the staging piece of a wave doubles as its output scratch");
-    store_block32<D, U>(Pt, acc_v, 1.0f, dvb, a.dv.st, k0, L, a.head_dim, lane, a.out_f32);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    store_block32<D, U>(Pt, acc_k, a.inv_temp, dkb, a.dk.st, k0, L, a.head_dim, lane, a.out_f32);
+    store_rows(acc_v, 1.0f, dvrows, k0 + n, L, h, a.out_f32);
+    store_rows(acc_k, a.inv_temp, dkrows, k0 + n, L, h, a.out_f32);
   } else {
     // Two passes over the queries, dv first and dk second; the scores are formed in each.
     // Segment s (SEG query rows) sits in buffer s & 1.  At its top every wave is done with segment s - 1,
     // whose buffer takes the rows of segment s + 1 while this one is worked on.
-    static_assert(!STREAM || (QROWS >= 64 && NT / 64 == 4), "a quarter of the first 64 rows of the two buffers per wave for its output");
-    unsigned short* const scratch = (w & 2 ? Gs : Qs) + (w & 1) * 32 * D;
     constexpr int BPS = SEG / 32;                     // query blocks per segment
     const int nseg = (nblk + BPS - 1) / BPS;
     auto pass = [&](auto what_tag) {
@@ -1228,14 +1218,13 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
           if (active && qblk >= kblk && qblk < nblk) block(what_tag, acc, acc, qblk, (sgm & 1) * SEG + 32 * b);
         }
       }
-      lds_barrier();            // every wave is done with the buffers: they become the output staging
       if (active) {
-        if constexpr (decltype(what_tag)::value == 0) store_block32<D, U>(scratch, acc, 1.0f, dvb, a.dv.st, k0, L, a.head_dim, lane, a.out_f32);
-        else store_block32<D, U>(scratch, acc, a.inv_temp, dkb, a.dk.st, k0, L, a.head_dim, lane, a.out_f32);
+        if constexpr (decltype(what_tag)::value == 0) store_rows(acc, 1.0f, dvrows, k0 + n, L, h, a.out_f32);
+        else store_rows(acc, a.inv_temp, dkrows, k0 + n, L, h, a.out_f32);
       }
     };
     pass(std::integral_constant<int, 0>{});
-    lds_barrier();              // and buffers again: the first block's rows once more
+    lds_barrier();              // every wave is done with the buffers: the first block's rows once more
     qcopy.issue(qrows, q_first, Qs, SEG);
     gcopy.issue(grows, q_first, Gs, SEG);
     request(kblk, cur);

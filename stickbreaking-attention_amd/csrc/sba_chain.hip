@@ -803,7 +803,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
           const Rows out = rows_of(a.dq, cur);
 #pragma unroll
           for (int j = 0; j < 16; ++j) dq[j] *= a.inv_temp;      // (in place: it is not needed unscaled, and there is no register to spare)
-          store_block32_rows(dq, 1.0f, out, row < doc_len && has_dq ? row * (int)out.row_bytes : OUTSIDE, 32 * dcol, h, a.out_f32);
+          store_block32_rows(dq, 1.0f, out, row * (int)out.row_bytes, row < doc_len && has_dq, 32 * dcol, h, a.out_f32);
         }
 #pragma unroll
         for (int i = 0; i < (REST > OPS ? REST : OPS); ++i) {
@@ -832,10 +832,9 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
 #pragma unroll
       for (int kb2 = 0; kb2 < 2; ++kb2) {
         const int row = done.kt * BKV + 64 * half + 32 * kb2 + n;
-        const int off = row < done.doc_len ? row * (int)out.row_bytes : OUTSIDE;
 #pragma unroll
         for (int j = 0; j < DB; ++j) {
-          store_block32_rows(acc[kb2][j], mat ? a.inv_temp : 1.0f, out, off, 32 * j, h, a.out_f32);
+          store_block32_rows(acc[kb2][j], mat ? a.inv_temp : 1.0f, out, row * (int)out.row_bytes, row < done.doc_len, 32 * j, h, a.out_f32);
 #pragma unroll
           for (int e = 0; e < 16; ++e) acc[kb2][j][e] = 0.0f;
         }

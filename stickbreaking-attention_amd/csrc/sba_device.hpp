@@ -420,105 +420,6 @@ __device__ __forceinline__ void stick_weights_fwd(const f32x16& x, float c, int 
   carry *= lo * hi;
 }
 
-// ---------------------------------------------------------------------------------------------
-// Epilogue: one wave writes its 32 x D block of fp32 accumulators (lane = column n of a 32-wide
-// block, register i = row 8*(i/4) + 4*h + i%4) to global memory as bf16.  Storing straight from
-// that layout would take 16*D/32 two-byte stores per lane; instead the block goes through a
-// wave-private LDS scratch of 32*D elements (2-byte LDS writes, 16-byte reads) and leaves as
-// D/16 fully coalesced 16-byte stores per lane.  Wave-private: no workgroup barrier inside,
-// but the caller must make sure nobody else still uses the scratch memory.
-// ---------------------------------------------------------------------------------------------
-// f32: the output is a float32 tensor (its stride still counts 16-bit words) of the same values; then a register of
-// the wave is two 128-byte pieces of rows and needs no detour.
-// (U: columns the accumulators cover, a multiple of 32 up to the row width D of the scratch; head_dim <= U)
-template <int D, int U = D>
-__device__ __forceinline__ void store_block32(unsigned short* scratch, const f32x16 (&acc)[U / 32], float scale,
-                                              elem_t* out, int64_t stride_t, int row0, int limit, int head_dim, int lane, bool f32) {
-  const int n = lane & 31, h = lane >> 5;
-  if (f32) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = row0 + 8 * (i >> 2) + 4 * h + (i & 3);
-      float* const to = reinterpret_cast<float*>(out + (int64_t)row * stride_t) + n;
-#pragma unroll
-      for (int db = 0; db < U / 32; ++db)
-        if (row < limit && 32 * db + n < head_dim) to[32 * db] = (float)(elem_t)(acc[db][i] * scale);
-      __builtin_amdgcn_sched_barrier(0);   // (one row's address at a time)
-    }
-    return;
-  }
-  elem_t* sc = reinterpret_cast<elem_t*>(scratch);
-#pragma unroll
-  for (int db = 0; db < U / 32; ++db) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = 8 * (i >> 2) + 4 * h + (i & 3);
-      sc[row * D + 32 * db + n] = (elem_t)(acc[db][i] * scale);
-    }
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's own LDS writes have landed
-  constexpr int C8 = D / 8;
-#pragma unroll
-  for (int j = 0; j < 32 * C8 / 64; ++j) {
-    const int cidx = lane + 64 * j;
-    const int row = cidx / C8, c8 = cidx % C8;
-    const uint4 v = *reinterpret_cast<const uint4*>(scratch + row * D + c8 * 8);
-    if (row0 + row < limit && 8 * c8 < head_dim) *reinterpret_cast<uint4*>(out + (int64_t)(row0 + row) * stride_t + c8 * 8) = v;
-  }
-}
-
-// Same, with a per-row multiple of another bf16 matrix added on the way out:
-//   out[row] = acc[row] * scale + rowscale(row) * addend[row]
-// (`rowscale(r)` = the fp32 factor of block row r, 0 <= r < 32, called once per 16-byte chunk).
-// The accumulators are rounded to bf16 once in the scratch, the sum is formed in fp32 and
-// rounded again: one rounding fewer than a caller adding the two bf16 tensors afterwards.
-template <int D, int U, class RowScale>
-__device__ __forceinline__ void store_block32_axpy(unsigned short* scratch, const f32x16 (&acc)[U / 32], float scale,
-                                                   elem_t* out, int64_t stride_t, int row0, int limit, int head_dim, int lane,
-                                                   const elem_t* addend, int64_t addend_stride_t, bool f32, RowScale rowscale) {
-  const int n = lane & 31, h = lane >> 5;
-  if (f32) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int r = 8 * (i >> 2) + 4 * h + (i & 3);
-      const float f = rowscale(r);
-#pragma unroll
-      for (int db = 0; db < U / 32; ++db)
-        if (row0 + r < limit && 32 * db + n < head_dim)
-          reinterpret_cast<float*>(out + (int64_t)(row0 + r) * stride_t)[32 * db + n] =
-              (float)(elem_t)fmaf(f, (float)addend[(int64_t)(row0 + r) * addend_stride_t + 32 * db + n], (float)(elem_t)(acc[db][i] * scale));
-    }
-    return;
-  }
-  elem_t* sc = reinterpret_cast<elem_t*>(scratch);
-#pragma unroll
-  for (int db = 0; db < U / 32; ++db) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = 8 * (i >> 2) + 4 * h + (i & 3);
-      sc[row * D + 32 * db + n] = (elem_t)(acc[db][i] * scale);
-    }
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's own LDS writes have landed
-  constexpr int C8 = D / 8;
-#pragma unroll
-  for (int j = 0; j < 32 * C8 / 64; ++j) {
-    const int cidx = lane + 64 * j;
-    const int row = cidx / C8, c8 = cidx % C8;
-    const bool ok = row0 + row < limit && 8 * c8 < head_dim;
-    const float f = rowscale(row);
-    const el8 mine = *reinterpret_cast<const el8*>(scratch + row * D + c8 * 8);
-    el8 other;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) other[e] = (elem_t)0.0f;
-    if (ok) other = *reinterpret_cast<const el8*>(addend + (int64_t)(row0 + row) * addend_stride_t + c8 * 8);
-    float sum[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) sum[e] = fmaf(f, (float)other[e], (float)mine[e]);
-    if (ok) *reinterpret_cast<el8*>(out + (int64_t)(row0 + row) * stride_t + c8 * 8) = pack8(sum);
-  }
-}
-
 // Is the 32-key sub-block starting at k0 entirely invisible / entirely visible to the 32
 // queries starting at qw0?
 template <bool AC>
@@ -570,12 +471,15 @@ __device__ __forceinline__ el8 load_frag(const Rows& r, int row, int col_bytes) 
   return __builtin_bit_cast(el8, load16(r, row, col_bytes));
 }
 
-// The same without the detour through LDS, for accumulators formed the other way round (lane = row n of the output, register i
-// = column 8*(i/4) + 4*h + i%4 of a 32-wide block): the half-waves exchange packed quads so that every
-// lane holds 8 consecutive columns of its row, two 16-byte stores per block.  `off`: byte offset of the lane's row in
-// the buffer, or OUTSIDE for a row that is not to be stored (the stores are issued either way: their number is known).
+// ---------------------------------------------------------------------------------------------
+// Epilogue: one wave writes a 32 x 32 block of fp32 accumulators formed with the output's rows as the second
+// operand (lane = row n of the output, register i = column 8*(i/4) + 4*h + i%4): the half-waves exchange packed quads so
+// that every lane holds 8 consecutive columns of its row, two 16-byte stores per block.  With the operands the other way
+// round (lane = column) a block had to be turned around through LDS -- a barrier, 16 two-byte writes and 2 reads per lane and
+// block.  `off`: byte offset of the lane's row in the buffer; `ok`: the row is to be stored (the
+// stores are issued either way: their number is known).
 // f32: a float32 tensor of the same values, a quad of the lane's columns at a time.
-__device__ __forceinline__ void store_block32_rows(const f32x16& acc, float scale, const Rows& out, int off, int col0, int h, bool f32) {
+__device__ __forceinline__ void store_block32_rows(const f32x16& acc, float scale, const Rows& out, int off, bool ok, int col0, int h, bool f32) {
   if (f32) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
@@ -583,7 +487,7 @@ __device__ __forceinline__ void store_block32_rows(const f32x16& acc, float scal
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = __builtin_bit_cast(unsigned, (float)(elem_t)(acc[4 * g + e] * scale));
       const int bytes = 4 * (col0 + 8 * g + 4 * h);
-      __builtin_amdgcn_raw_buffer_store_b128(v, out.rsrc, bytes < 2 * out.used_bytes ? off + bytes : OUTSIDE, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(v, out.rsrc, ok && bytes < 2 * out.used_bytes ? off + bytes : OUTSIDE, 0, 0);
     }
     return;
   }
@@ -599,7 +503,38 @@ __device__ __forceinline__ void store_block32_rows(const f32x16& acc, float scal
       v[2 + e] = (unsigned)r[1];
     }
     const int bytes = 2 * (col0 + 8 * g + 8 * h);
-    __builtin_amdgcn_raw_buffer_store_b128(v, out.rsrc, bytes < out.used_bytes ? off + bytes : OUTSIDE, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(v, out.rsrc, ok && bytes < out.used_bytes ? off + bytes : OUTSIDE, 0, 0);
+  }
+}
+
+// All of a wave's column blocks, optionally with a multiple of another matrix added on the way out:
+//   out[row] = acc[row] * scale + factor * addend[row]      (factor: the lane's row's)
+// The accumulators are rounded to the element type once, the sum is formed in fp32 and rounded again: one rounding fewer
+// than a caller adding the two 16-bit tensors afterwards.
+template <int DB>
+__device__ __forceinline__ void store_rows(const f32x16 (&acc)[DB], float scale, const Rows& out, int row, int limit, int h, bool f32) {
+  asm volatile("" : "+v"(row), "+v"(h));      // (nothing of the addresses is to be kept in registers through the loops before)
+#pragma unroll
+  for (int j = 0; j < DB; ++j) store_block32_rows(acc[j], scale, out, row * (int)out.row_bytes, row < limit, 32 * j, h, f32);
+}
+template <int DB>
+__device__ __forceinline__ void store_rows_axpy(const f32x16 (&acc)[DB], const Rows& out, int row, int limit, int h, bool f32,
+                                                const Rows& addend, float factor) {
+  typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
+  typedef __attribute__((ext_vector_type(4))) elem_t el4;
+  asm volatile("" : "+v"(row), "+v"(h));
+#pragma unroll
+  for (int j = 0; j < DB; ++j) {
+    f32x16 sum;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int bytes = 2 * (32 * j + 8 * g + 4 * h);
+      const u32x2 raw = __builtin_amdgcn_raw_buffer_load_b64(addend.rsrc, bytes < addend.used_bytes ? row * (int)addend.row_bytes + bytes : OUTSIDE, 0, 0);
+      const el4 other = __builtin_bit_cast(el4, raw);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[4 * g + e] = fmaf(factor, (float)other[e], (float)(elem_t)acc[j][4 * g + e]);
+    }
+    store_block32_rows(sum, 1.0f, out, row * (int)out.row_bytes, row < limit, 32 * j, h, f32);
   }
 }
 

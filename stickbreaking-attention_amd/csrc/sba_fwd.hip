@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
       }
     }
     if constexpr (TAB) return;
-    // P as the A operand of O = P.V: slot s of step tt is key 16*h + 8*tt + s, which the
+    // P as the B operand of O^T = V^T.P^T: slot s of step tt is key 16*h + 8*tt + s, which the
     // permuted tile keeps in LDS row 16*tt + 8*(s/4) + 4*h + s%4.
     el8 vfr[2][DB];
 #pragma unroll
@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
     for (int tt = 0; tt < 2; ++tt) {
       const el8 pf = pack8(p + 8 * tt);
 #pragma unroll
-      for (int db = 0; db < DB; ++db) oacc[db] = mfma32(pf, vfr[tt][db], oacc[db]);
+      for (int db = 0; db < DB; ++db) oacc[db] = mfma32(vfr[tt][db], pf, oacc[db]);   // (o^T: see store_block32_rows)
     }
   };
 
@@ -213,14 +213,10 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
     if (stick != nullptr) stick[(unsigned)(tab_rowplane32(t.doc_len) + qrow)] = r;
   }
   if constexpr (TAB) return;
-  lds_barrier();   // every wave is done with the K/V tiles: their memory becomes the o staging area
-  if (a.fuse) {
-    // what every caller computes next (upstream tests/test_varlen.py:101): o + rem * v
-    store_block32_axpy<D, U>(smem + w * 32 * D, oacc, 1.0f, ob, a.o.st, qw0, t.doc_len, a.head_dim, lane, vb, a.v.st, a.out_f32,
-                          [&](int row) { return __shfl(r, row, 64); });
-  } else {
-    store_block32<D, U>(smem + w * 32 * D, oacc, 1.0f, ob, a.o.st, qw0, t.doc_len, a.head_dim, lane, a.out_f32);
-  }
+  const Rows orows = make_rows(ob, a.o.st, t.doc_len, a.head_dim);
+  // what every caller computes next (upstream tests/test_varlen.py:101): o + rem * v
+  if (a.fuse) store_rows_axpy(oacc, orows, qrow, t.doc_len, h, a.out_f32, vrows, r);
+  else store_rows(oacc, 1.0f, orows, qrow, t.doc_len, h, a.out_f32);
 }
 
 // Explicit instantiations: every (head_dim, attend_current, carry space) variant the launchers use.
