@@ -1035,22 +1035,37 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
 
   const int q_first = kt * BKV;                      // first query that can see the tile
   const int nblk = (L - q_first + 31) / 32;          // query blocks behind the tile's first key (not STREAM: 1 .. QROWS / 32)
-  // all of those Q and dO rows at once, or the first block of them (rows past the document arrive as zeros)
-  TileCopy<D, STREAM ? SEG : QROWS, NT, false> qcopy, gcopy;
+  // The first of those Q and dO rows (rows past the document arrive as zeros).  Not STREAM: as many as there are keys, and
+  // into the place of the others first this tile's K and V rows, which every wave takes its fragments from.
+  constexpr int FIRST = STREAM ? SEG : BKV;
+  static_assert(STREAM || QROWS == 2 * BKV, "the second half of the query buffers holds the key tile first");
+  TileCopy<D, FIRST, NT, false> qcopy, gcopy;
   qcopy.init(tid, qrows.row_bytes, qrows.used_bytes);
   gcopy.init(tid, grows.row_bytes, grows.used_bytes);
   qcopy.issue(qrows, q_first, Qs, STREAM ? SEG : 32 * nblk);      // (32 or 64 rows per instruction of all waves: whole query blocks)
   gcopy.issue(grows, q_first, Gs, STREAM ? SEG : 32 * nblk);
+  if constexpr (!STREAM) {
+    // (through LDS: a fragment load straight from memory is 32 rows of 32 bytes, which keeps the CU's address unit busy; 16 K
+    // tokens in documents of 16 to 256, 32 heads, head_dim 64: forward + backward 281 -> 276 us.  A kernel small enough
+    // for three workgroups per CU was no faster, 287: what is left is the traffic, 4 TB/s.)
+    TileCopy<D, BKV, NT, true> kcopy, vcopy;
+    kcopy.init(tid, krows.row_bytes, krows.used_bytes);
+    vcopy.init(tid, vrows.row_bytes, vrows.used_bytes);
+    kcopy.issue(krows, q_first, Qs + BKV * D);
+    vcopy.issue(vrows, q_first, Gs + BKV * D);
+  }
   // Wave w of workgroup b takes key block (w + b) mod 4: the block with the most queries behind it
   // is the first one, and two workgroups that share a CU should not both put it on the same SIMD.
   const int kblk = (w + blockIdx.x) & (BKV / 32 - 1);
   const int k0 = q_first + 32 * kblk;                // this wave's keys
   const bool active = k0 < L;
   el8 kf[KS], vf[KS];                                // MFMA row n holds key k0 + kperm(n)
+  if constexpr (STREAM) {
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    kf[ks] = load_frag(krows, k0 + kperm(n), 32 * ks + 16 * h);
-    vf[ks] = load_frag(vrows, k0 + kperm(n), 32 * ks + 16 * h);
+    for (int ks = 0; ks < KS; ++ks) {
+      kf[ks] = load_frag(krows, k0 + kperm(n), 32 * ks + 16 * h);
+      vf[ks] = load_frag(vrows, k0 + kperm(n), 32 * ks + 16 * h);
+    }
   }
   // A block that starts past the end of the document is never visible; its table reads are
   // redirected into the document's area and never used.
@@ -1091,8 +1106,18 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
   }
   if constexpr (!STREAM) {
     wait_loads<0>();
-    lds_barrier();            // the only barrier: every wave's part of the Q / dO rows has landed
-    if (!active) return;
+    lds_barrier();            // every wave's part of the rows has landed
+    if (!active) return;      // (a document that ends ahead of this wave's keys has no second half of queries: no barrier follows)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      kf[ks] = lds_row8(Qs + BKV * D + 32 * kblk * D + roff[ks]);
+      vf[ks] = lds_row8(Gs + BKV * D + 32 * kblk * D + roff[ks]);
+    }
+    if (nblk > BKV / 32) {
+      lds_barrier();          // every wave has its keys in registers
+      qcopy.issue(qrows, q_first + BKV, Qs + BKV * D, 32 * nblk - BKV);
+      gcopy.issue(grows, q_first + BKV, Gs + BKV * D, 32 * nblk - BKV);
+    }
   }
 
   unsigned short* Pt = St[w][0];
@@ -1192,7 +1217,13 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
     clear(acc_k);
     // query blocks at or after the key block (those before it see none of these keys)
 #pragma unroll 1
-    for (int qblk = kblk; qblk < nblk; ++qblk) block(std::integral_constant<int, 2>{}, acc_v, acc_k, qblk, 32 * qblk);
+    for (int qblk = kblk; qblk < nblk; ++qblk) {
+      if (qblk == BKV / 32) {
+        wait_loads<0>();
+        lds_barrier();        // the second half has landed (every wave of a tile that has one comes here)
+      }
+      block(std::integral_constant<int, 2>{}, acc_v, acc_k, qblk, 32 * qblk);
+    }
     store_rows(acc_v, 1.0f, dvrows, k0 + n, L, h, a.out_f32);
     store_rows(acc_k, a.inv_temp, dkrows, k0 + n, L, h, a.out_f32);
   } else {
