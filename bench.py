@@ -38,6 +38,17 @@ MEASURED = {"sba_version": 213,
                    "bwd_dkdv_kernel": {"traffic": 1.228e9, "mfma_busy": 0.421, "valu_busy": 0.503, "coexec": 0.181}}}
 
 KERNELS = ["fwd_kernel", "bwd_dq_kernel", "bwd_dkdv_kernel"]
+# algorithmic and executed FLOPs per causal pair and head_dim of each, and of the one-pass backward, which takes the
+# last one's place (and its event pair) where the library chooses it: no dq pass is recorded then
+ALGORITHMIC, EXECUTED = [4.0, 6.0, 4.0], [4.0, 6.0, 8.0]
+CHAINED = "bwd_chain_kernel"
+
+
+def kernel_figures(m):
+    """[(name, ms, algorithmic, executed, tensors moved)] of a measured workload's kernels."""
+    if m["backward"] and m["kern_ms"][1] == 0.0:
+        return [(KERNELS[0], m["kern_ms"][0], 4.0, 4.0, 4.0), (CHAINED, m["kern_ms"][2], 10.0, 10.0, 7.0)]
+    return [(n, m["kern_ms"][i], ALGORITHMIC[i], EXECUTED[i], [4.0, 5.0, 6.0][i]) for i, n in enumerate(KERNELS)]
 
 
 def workload(name):
@@ -221,25 +232,24 @@ def roofline(m, lib):
     """Roofline object of the dominant kernel of a measured workload.
     MFMA bound: algorithmic FLOPs per launch -- forward 4*d per causal pair (QK^T, AV); the
     backward's 10*d (recompute QK^T, dO V^T, dQ, dK, dV) split as 6*d for the dq pass and 4*d for
-    the dk/dv pass, whose own recomputation of QK^T and dO V^T is executed, not algorithmic, work.
+    the dk/dv pass, whose own recomputation of QK^T and dO V^T is executed, not algorithmic, work; all 10*d
+    for the one-pass backward.
     HBM bound: the tensors a kernel must read and write once -- forward q,k,v in and o out (4 N,
     N = heads*tokens*head_dim*2 bytes), dq pass q,k,v,dO in and dq out (5 N), dk/dv pass
-    q,k,v,dO in and dk,dv out (6 N)."""
-    d, pairs, kern_ms = m["d"], m["pairs"], m["kern_ms"]
-    dom = max(range(3), key=lambda i: kern_ms[i])
+    q,k,v,dO in and dk,dv out (6 N), one-pass backward q,k,v,dO in and dq,dk,dv out (7 N)."""
+    d, pairs = m["d"], m["pairs"]
+    name, ms, alg, _, tensors = max(kernel_figures(m), key=lambda f: f[1])
     seen = {"traffic": None, "mfma_busy": None, "valu_busy": None, "coexec": None}
     if lib.sba_version() == MEASURED["sba_version"]:
-        seen.update(MEASURED.get(m["name"], {}).get(KERNELS[dom], {}))
+        seen.update(MEASURED.get(m["name"], {}).get(name, {}))
     traffic = seen["traffic"]
     counters = {k: seen[k] for k in ("mfma_busy", "valu_busy", "coexec")}
     if m["cfg"]["bound"] == "hbm":
-        alg = [4.0, 5.0, 6.0][dom] * m["tensor_bytes"]
-        achieved = alg / (kern_ms[dom] * 1e-3) / 1e9
-        return {"bound": "hbm", "kernel": KERNELS[dom], "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
+        achieved = tensors * m["tensor_bytes"] / (ms * 1e-3) / 1e9
+        return {"bound": "hbm", "kernel": name, "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                 "frac": achieved / PEAK_HBM_GBS, "traffic": traffic, **counters}
-    alg = [4.0, 6.0, 4.0][dom] * d * pairs
-    achieved = alg / (kern_ms[dom] * 1e-3) / 1e12
-    return {"bound": "mfma", "kernel": KERNELS[dom], "achieved": achieved, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
+    achieved = alg * d * pairs / (ms * 1e-3) / 1e12
+    return {"bound": "mfma", "kernel": name, "achieved": achieved, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
             "frac": achieved / PEAK_BF16_TFLOPS, "traffic": traffic, **counters}
 
 
@@ -294,7 +304,6 @@ def main():
     m = measure(args.workload, args.steps, args.warmup, args, torch, lib, override)
     label = args.workload + ("/custom" if override else "")
     d, pairs, backward = m["d"], m["pairs"], m["backward"]
-    executed = [4.0 * d * pairs, 6.0 * d * pairs, 8.0 * d * pairs]
     total_flops = (14.0 if backward else 4.0) * d * pairs
     step_bytes = (11.0 if backward else 4.0) * m["tensor_bytes"]
     out = {
@@ -312,9 +321,9 @@ def main():
         "fwd_ms": m["ms_fwd"], "fwd_tflops": 4.0 * d * pairs / (m["ms_fwd"] * 1e-3) / 1e12,
         "frac_of_bf16_peak": total_flops / (m["ms_step"] * 1e-3) / 1e12 / PEAK_BF16_TFLOPS,
         "step_gbs_mandatory": step_bytes / (m["ms_step"] * 1e-3) / 1e9,
-        "kernel_ms": dict(zip(KERNELS, m["kern_ms"])),
-        "kernel_executed_tflops": {n: (executed[i] / (m["kern_ms"][i] * 1e-3) / 1e12 if m["kern_ms"][i] > 0 else 0.0)
-                                   for i, n in enumerate(KERNELS)},
+        "kernel_ms": {n: ms for n, ms, *_ in kernel_figures(m)},
+        "kernel_executed_tflops": {n: (ex * d * pairs / (ms * 1e-3) / 1e12 if ms > 0 else 0.0)
+                                   for n, ms, _, ex, _ in kernel_figures(m)},
         "roofline": roofline(m, lib) if _ops.PRODUCT_SPACE else dict(roofline(m, lib), traffic=None, mfma_busy=None, valu_busy=None, coexec=None),
         "device": {"name": props.name, "cus": props.multi_processor_count, "clock_mhz": device_clock_mhz(torch),
                    "sba_version": lib.sba_version()},
@@ -332,7 +341,7 @@ def main():
                       "frac_of_bf16_peak": fl / (s["ms_step"] * 1e-3) / 1e12 / PEAK_BF16_TFLOPS,
                       "step_gbs_mandatory": by / (s["ms_step"] * 1e-3) / 1e9,
                       "frac_of_hbm_peak": by / (s["ms_step"] * 1e-3) / 1e9 / PEAK_HBM_GBS,
-                      "kernel_ms": dict(zip(KERNELS, s["kern_ms"])), "roofline": roofline(s, lib)}
+                      "kernel_ms": {n: ms for n, ms, *_ in kernel_figures(s)}, "roofline": roofline(s, lib)}
         out["secondary"] = sec
     if not args.no_cpu_baseline:
         lengths3, cfg3 = workload("c3")
