@@ -387,16 +387,20 @@ def _check_cu(cu_seqlens: torch.Tensor, like: torch.Tensor) -> torch.Tensor:
 # cu_seqlens tensor to every layer, so the scheduler kernel runs once per tensor instead of once per
 # layer.  Entries: (weak reference to cu_seqlens or None, its version, key, schedule tensor), newest
 # last; the key holds the stream, so a schedule is only ever reused behind the launch that wrote it.
+# An entry is made once that launch is on its stream (`_schedule_built`) and not before: a call can
+# fail on its way there (an output that does not fit, a head_dim that is refused), and what it
+# leaves behind is an uninitialised workspace.
 _sched_cache = []
 _SCHED_CACHE_SIZE = 8
 
 
 def _schedule_workspace(cu: Optional[torch.Tensor], sched_bytes: int, batch: int, tokens: int, device):
-    """(schedule tensor, whether its contents still have to be built).  Eager mode only remembers;
-    while torch.compile traces, and while the stream is being captured into a graph (whose replays
-    must not depend on a tensor this cache may drop), every call gets a workspace of its own."""
+    """(schedule tensor, whether its contents still have to be built, what `_schedule_built` is to be
+    told then).  Eager mode only remembers; while torch.compile traces, and while the stream is being
+    captured into a graph (whose replays must not depend on a tensor this cache may drop), every call
+    gets a workspace of its own."""
     if torch.compiler.is_compiling() or torch.cuda.is_current_stream_capturing():
-        return torch.empty(sched_bytes, dtype=torch.uint8, device=device), True
+        return torch.empty(sched_bytes, dtype=torch.uint8, device=device), True, None
     return _cached_schedule(cu, sched_bytes, batch, tokens, device)
 
 
@@ -404,20 +408,29 @@ def _cached_schedule(cu: Optional[torch.Tensor], sched_bytes: int, batch: int, t
     version = None if cu is None else _version_of(cu)
     # (the raw stream handle: torch.cuda.current_stream() builds two Python objects to hold it, 2 us per call)
     key = (device, torch._C._cuda_getCurrentRawStream(device.index), batch, tokens, sched_bytes)
+    if cu is not None and version is None:
+        return torch.empty(sched_bytes, dtype=torch.uint8, device=device), True, None
     with _cache_lock:
-        if cu is None or version is not None:
-            for i in range(len(_sched_cache) - 1, -1, -1):
-                ref, ver, k, sched = _sched_cache[i]
-                if k == key and (ref is None if cu is None else (ref is not None and ref() is cu)):
-                    if ver == version:
-                        return sched, False
-                    del _sched_cache[i]
-                    break
-        sched = torch.empty(sched_bytes, dtype=torch.uint8, device=device)
-        if cu is None or version is not None:
-            _sched_cache[:] = [e for e in _sched_cache if e[0] is None or e[0]() is not None][-(_SCHED_CACHE_SIZE - 1):]
-            _sched_cache.append((None if cu is None else weakref.ref(cu), version, key, sched))
-        return sched, True
+        for i in range(len(_sched_cache) - 1, -1, -1):
+            ref, ver, k, sched = _sched_cache[i]
+            if k == key and (ref is None if cu is None else (ref is not None and ref() is cu)):
+                if ver == version:
+                    return sched, False, None
+                del _sched_cache[i]
+                break
+    sched = torch.empty(sched_bytes, dtype=torch.uint8, device=device)
+    return sched, True, (None if cu is None else weakref.ref(cu), version, key, sched)
+
+
+def _schedule_built(entry) -> None:
+    """The launch that builds a schedule `_schedule_workspace` handed out has been enqueued."""
+    if entry is None:
+        return
+    with _cache_lock:
+        # (two threads on one stream may both have built it: the newer takes the older's place)
+        _sched_cache[:] = [e for e in _sched_cache if (e[0] is None or e[0]() is not None)
+                           and (e[0] is not entry[0] or e[2] != entry[2])][-(_SCHED_CACHE_SIZE - 1):]
+        _sched_cache.append(entry)
 
 
 def run_forward(q, k, v, fixed: bool, cu_seqlens, max_seqlens, inv_temp: float, attend_current: bool,
@@ -455,7 +468,7 @@ def run_forward(q, k, v, fixed: bool, cu_seqlens, max_seqlens, inv_temp: float, 
     rem = torch.empty_like(qp[..., 0])
     keep_table = need_table and not RECOMPUTE_TABLE
     table = torch.empty(table_floats if keep_table else 0, dtype=torch.float32, device=q.device)
-    sched, build = _schedule_workspace(cu, sched_bytes, B, T, q.device)
+    sched, build, entry = _schedule_workspace(cu, sched_bytes, B, T, q.device)
     if return_attention:
         weights = torch.zeros(qp.shape[:-1] + (T,), dtype=torch.float32, device=q.device)
         _launch_fwd(fixed, qp, kp, vp, cu, max_len, float(inv_temp), bool(attend_current), product, bool(fused),
@@ -466,8 +479,9 @@ def run_forward(q, k, v, fixed: bool, cu_seqlens, max_seqlens, inv_temp: float, 
     else:
         _compileable_forward(qp, kp, vp, cu, max_len, float(inv_temp), bool(attend_current), product,
                              bool(fused), o, rem, table, sched, build)
-        if VALIDATE and not torch.compiler.is_compiling():
-            check_status(sched, table, H, max_len)
+    _schedule_built(entry)
+    if VALIDATE and not fixed and not return_attention and not torch.compiler.is_compiling():
+        check_status(sched, table, H, max_len)
     if dpad != d or q.dtype != cdt:
         o = o[..., :d].to(q.dtype)
         rem = rem.to(q.dtype)
@@ -507,10 +521,12 @@ def eager(q, k, v, fixed: bool, cu_seqlens, max_seqlens, inv_temp: float, attend
     sched_bytes, table_floats = _sizes(fixed, B, H, T, n_docs, max_len, entries)
     if q.dtype not in (torch.bfloat16, torch.float16):
         _warn_reduced_precision(q.dtype)
-    sched, build = _cached_schedule(cu, sched_bytes, B, T, q.device)
+    sched, build, entry = _cached_schedule(cu, sched_bytes, B, T, q.device)
     flags = ((nat.FLAG_ATTEND_CURRENT if attend_current else 0) | (nat.FLAG_PRODUCT_SPACE if PRODUCT_SPACE else 0) |
              (nat.FLAG_FUSE_REMAINDER if fused else 0))
-    return nat.load_ext().attention(q, k, v, cu, sched, build, table_floats, max_len, inv_temp, flags)
+    out = nat.load_ext().attention(q, k, v, cu, sched, build, table_floats, max_len, inv_temp, flags)
+    _schedule_built(entry)
+    return out
 
 
 def check_status(sched: torch.Tensor, table: Optional[torch.Tensor] = None, heads: int = 1,

@@ -379,3 +379,49 @@ def test_scratch_tables_grow_instead_of_multiplying(monkeypatch):
     assert held <= int(4 * base * 1.13) + (1 << 17)
     _ops.release_workspaces()
     assert not _ops._gtab_cache
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("fixed", [True, False])
+def test_a_failed_call_leaves_no_schedule_behind(monkeypatch, native, fixed):
+    """A call that fails before its launches (an output that does not fit, a head_dim that is refused) leaves an
+    uninitialised schedule workspace: the next call on the same documents has to build its own, and the one
+    after that finds it."""
+    from stickbreaking_attention import _ops
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(nat, "require_gpu", lambda t: None)
+    calls, fail = [], [True]
+
+    def launch(sched, build):
+        calls.append((build, sched.data_ptr()))
+        if fail[0]:
+            raise RuntimeError("out of memory")
+
+    class Ext:
+        def attention(self, q, k, v, cu, sched, build, *rest):
+            launch(sched, build)
+            return [q, q[..., 0]]
+
+        def release(self):
+            pass
+    monkeypatch.setattr(nat, "load_ext", lambda: Ext())
+    monkeypatch.setattr(_ops, "_launch_fwd", lambda *a, build_schedule, **kw: launch(a[-1], build_schedule))
+    _ops.release_workspaces()
+    q = torch.zeros((2, 3, 40, 16) if fixed else (3, 80, 16), dtype=torch.bfloat16)
+    cu = None if fixed else torch.tensor([30, 80], dtype=torch.int32)
+
+    def call():
+        if native:
+            return _ops.eager(q, q, q, fixed, cu, 50, 1.0, False)
+        return _ops.run_forward(q, q, q, fixed, cu, 50, 1.0, False, need_table=False)
+
+    for _ in range(2):
+        with pytest.raises(RuntimeError):
+            call()
+    assert not _ops._sched_cache
+    fail[0] = False
+    call()
+    call()
+    assert [b for b, _ in calls] == [True, True, True, False] and calls[2][1] == calls[3][1]
+    _ops.release_workspaces()

@@ -61,3 +61,23 @@ def test_fixed_length_schedule_is_reused_per_shape():
     assert _ops._sched_cache[-1][3] is not sched1
     o3, _ = sb_attn(q, k, v)          # the first shape again: still right
     assert torch.equal(o1, o3)
+
+
+def test_a_refused_call_leaves_no_schedule_behind():
+    """A head_dim that is refused has been given a schedule workspace nobody builds: the next call on the same
+    documents builds its own."""
+    from stickbreaking_attention import _ops, sb_attn, sb_attn_varlen
+    dev = torch.device("cuda:0")
+    torch.manual_seed(5)
+    cu = torch.tensor([0, 150, 150, 384], device=dev, dtype=torch.int32)
+    for op, shape in ((lambda *x: sb_attn_varlen(*x, cu, 234), (2, 384)), (sb_attn, (3, 2, 200))):
+        _ops.release_workspaces()
+        wide = torch.randn(*shape, 300, device=dev, dtype=torch.bfloat16)
+        with pytest.raises(ValueError):
+            op(wide, wide, wide)
+        assert not _ops._sched_cache
+        q, k, v = (torch.randn(*shape, 64, device=dev, dtype=torch.bfloat16) for _ in range(3))
+        first = op(q, k, v)
+        _ops.release_workspaces()
+        for a, b in zip(first, op(q, k, v)):
+            assert torch.equal(a, b)
