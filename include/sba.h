@@ -304,7 +304,10 @@ float sba_last_kernel_ms(int which);
 void  sba_set_dkdv_workgroups(int n);
 
 /* Test and tuning switch (process-wide): which form of the backward sba_chain_scratch_bytes asks for.  0: by size,
- * 1: never the one-pass form, 2: wherever it is possible, 3: the same in steps of 64 queries (head_dim <= 64). */
+ * 1: never the one-pass form, 2: wherever it is possible, 3: the same in steps of 64 queries (head_dim <= 64).
+ * With SBA_FORM_SHORT_WAITS added, a wait of the one-pass form for the key tile before gives up after its
+ * first look, as it otherwise does after about a second: what the missing partial sums belong to is NaN. */
+#define SBA_FORM_SHORT_WAITS 0x100
 void  sba_set_backward_form(int form);
 
 #ifdef __cplusplus

@@ -18,6 +18,7 @@ using namespace sba;
 std::atomic<int> g_timing{0};
 std::atomic<int> g_dkdv_workgroups{0};   // sba_set_dkdv_workgroups
 std::atomic<int> g_backward_form{0};     // sba_set_backward_form
+int backward_form() { return g_backward_form.load() & 0xff; }
 std::atomic<float> g_ms[3];
 
 inline int cdiv_i(long long a, long long b) { return (int)((a + b - 1) / b); }
@@ -319,7 +320,7 @@ bool chain_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
 // / (2 x 64 x 128 x 256 CUs), against the steps of the longest document, where beyond 2048 keys more of a chain's tiles
 // start behind one another than side by side (16 x 4096: 250 us for 224, 16 x 8192: 589 for 653).
 bool chain_wide(const sba_problem* p, bool fixed, const Sizes& sz) {
-  const int form = g_backward_form.load();
+  const int form = backward_form();
   if (form == 2 || form == 3) return form == 3;
   const long long mean = sz.rows / sz.n_docs, longest = declared_max_doc_len(p, fixed);
   return 2 * (long long)sz.n_docs * p->heads * mean * mean >= longest * (longest > 2048 ? 3 : 2) * 65536;
@@ -327,7 +328,7 @@ bool chain_wide(const sba_problem* p, bool fixed, const Sizes& sz) {
 // Where the one-pass form is the faster one (gain over the two passes, measured on 270 problems of 1 to 32 heads and
 // 512 to 16 K tokens in 1 to 128 documents, declared lengths exact).
 bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
-  const int form = g_backward_form.load();
+  const int form = backward_form();
   if (form == 1 || g_dkdv_workgroups.load() != 0 || !chain_possible(p, fixed, sz)) return false;
   if (form == 2 || form == 3) return true;
   const long long chains = (long long)sz.n_docs * p->heads, items = (long long)sz.n_kv_max * p->heads;
@@ -396,6 +397,7 @@ int backward_chained(const sba_problem* p, bool fixed, const void* schedule, siz
   a.clear_spare = fixed ? 0 : 1;
   a.nan_pair = p->dtype == SBA_F16 && !a.out_f32 ? 0x7e007e00u : 0x7fc07fc0u;
   a.max_doc_len = declared_max_doc_len(p, fixed);
+  a.spin_limit = g_backward_form.load() & SBA_FORM_SHORT_WAITS ? 0 : CHAIN_SPIN_LIMIT;
   a.c = c.c;
   a.inv_temp = c.inv_temp;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);

@@ -119,6 +119,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
   __shared__ __attribute__((aligned(16))) unsigned short Gs[RING * QTILE];
   __shared__ __attribute__((aligned(16))) unsigned short PZ[(PBUF + 2) * PTILE];   // p: PBUF buffers, dz: two buffers, [query][key]
   __shared__ float tot[2][NSQ][4][32];       // by step parity: every key block's sum of p (do.v) per query
+  __shared__ float given_up;                 // 0, or NaN once a wait of this workgroup has run out (see await)
   __shared__ int prefix[CHAIN_MAX_GROUPS];   // items of this XCD's queue up to and including each group
   __shared__ int mbox[2][8];
   __shared__ __attribute__((aligned(16))) unsigned short spare[4][512];   // where a product wave's copies of nothing go
@@ -212,7 +213,10 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
   };
   if (w == 0) {
     unsigned ticket = 0;
-    if (lane == 0) ticket = atomicAdd(ctr, 1u);
+    if (lane == 0) {
+      ticket = atomicAdd(ctr, 1u);
+      given_up = 0.0f;
+    }
     int base = 0;
     for (int g0 = 0; g0 < n_groups; g0 += 64) {
       int v = group_items(g0 + lane);
@@ -237,7 +241,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
     const int kb = w & 3, sq = w >> 2;            // 32-key block and 32-query block of this wave
     el8 kf[KS], vf[KS];                           // MFMA row n holds key k0 + kperm(n)
     int k0, nsteps, doc_len, t_last, n_wait;
-    float rem_own, poison = 0.0f;
+    float rem_own;
     int row4, last4;
     __amdgpu_buffer_rsrc_t stick_rs, in_rs, out_rs;
     float se0, se1, se2;                          // stick on entering the block, requested ahead, three steps in turn
@@ -308,16 +312,25 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
-    // first score wave: the tile before this one has published `steps` steps (all of them: nothing to wait for any more)
+    // First score wave: the tile before this one has published `steps` steps (all of them: nothing to wait for any more).
+    // A wait that runs out -- it cannot while workgroups make progress -- must end in NaN and not in plausible numbers, in
+    // every wave: what it stood for is requested by all of them behind the barrier that follows.  The waves of the oldest
+    // key block add `given_up` to the stick of the block whose weights they form next, the first that is in doubt: its p
+    // and dz are NaN, so is the sum every newer key block takes from `tot` for its D, and with dz of all of the tile's
+    // keys dk, dq and what is handed on.
     auto await = [&](int steps) {
       const int need = min(steps, n_wait);
-      if (seen >= need) return;
-      for (int tries = 0; tries < CHAIN_SPIN_LIMIT; ++tries) {
+      auto published = [&]() {
         seen = __builtin_amdgcn_readfirstlane(__hip_atomic_load(pred, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        if (seen >= need) return;
+        return seen >= need;
+      };
+      if (seen >= need || published()) return;
+      const int limit = fresh_args<ChainArgs>().spin_limit;
+      for (int tries = 0; tries < limit; ++tries) {
         __builtin_amdgcn_s_sleep(2);
+        if (published()) return;
       }
-      poison = __builtin_nanf("");      // (cannot happen while workgroups make progress: never a plausible result, never a hang)
+      if (lane == 0) given_up = __builtin_nanf("");
       n_wait = 0;
     };
     auto chains = [&](int slot, f32x16& x, f32x16& da) {
@@ -352,13 +365,14 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       const int p_buf = SLOT >= 0 ? (SLOT + 2) % 3 : (w + 1) % 3;    // of block w + 1
       float d_in = 0.0f, t0 = 0.0f, t1 = 0.0f, t2 = 0.0f;
       if constexpr (!FIRST) {
-        d_in = d_next + poison;
+        d_in = d_next;
         if (kb > 0) t0 = tot[par][sq][0][n];
         if (kb > 1) t1 = tot[par][sq][1][n];
         if (kb > 2) t2 = tot[par][sq][2][n];
       }
       request_d(w + 1);
       float e_in = se;
+      if (kb == 0) e_in += given_up;
       request_e(w + 4, se);
       const unsigned short* Qt = Qs + slot * QTILE;
       const unsigned short* Gt = Gs + slot * QTILE;
@@ -468,13 +482,14 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       const int par = w & 1;
       float d_in = 0.0f, t0 = 0.0f, t1 = 0.0f, t2 = 0.0f;
       if constexpr (!FIRST) {
-        d_in = d_next + poison;
+        d_in = d_next;
         if (kb > 0) t0 = tot[par][sq][0][n];
         if (kb > 1) t1 = tot[par][sq][1][n];
         if (kb > 2) t2 = tot[par][sq][2][n];
       }
       request_d(w + 1);
       float e_in = se;
+      if (kb == 0) e_in += given_up;
       request_e(w + 3, se);
       const unsigned short* Qt = Qs + slot * QTILE;
       const unsigned short* Gt = Gs + slot * QTILE;

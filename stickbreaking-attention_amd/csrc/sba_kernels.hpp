@@ -60,6 +60,7 @@ struct ChainArgs {
   int fixed, fuse, clear_spare, out_f32;
   unsigned nan_pair;
   int max_doc_len;
+  int spin_limit;              // CHAIN_SPIN_LIMIT, or what a test asks for
   float c, inv_temp;
 };
 

@@ -66,3 +66,27 @@ def test_queues(form, steps, H, lengths):
     for name, a, b, c in zip(("dq", "dk", "dv"), two, first, again):
         assert_close(name, b, a.float())
         assert torch.equal(b, c)
+
+
+@pytest.mark.parametrize("steps,d", [(2, 128), (2, 64), (3, 64), (2, 32), (3, 32)])
+def test_a_wait_that_runs_out_gives_nan_and_nothing_else(form, steps, d):
+    """Every wait for the key tile before ends after one look, so that tiles go on without the partial sums they
+    waited for, at whatever step they have got to.  An element that depends on a missing one has to be NaN: what is
+    not NaN has to be the same bits as ever."""
+    from stickbreaking_attention import sb_attn_varlen
+    lengths = [2000, 128, 700, 1400, 257, 1000]
+    H, T = 24, sum(lengths)
+    tensors = orc.make_inputs((H, T, d), 9 + d)
+    drem = torch.randn((H, T), generator=torch.Generator().manual_seed(d)).to(torch.bfloat16)
+    cu = cu_from_lengths(lengths, device=DEV)
+    form(steps)
+    whole = gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem))
+    form(steps | 0x100)
+    cut = gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem))
+    lost = [torch.isnan(b) for b in cut]
+    for name, a, b, nan in zip(("dq", "dk", "dv"), whole, cut, lost):
+        assert torch.isfinite(a).all()
+        assert torch.equal(torch.where(nan, a, b), a), name
+    assert lost[0].any() and lost[1].any() and not all(nan.all() for nan in lost)
+    for nan in lost:      # (a row is lost as a whole)
+        assert torch.equal(nan.any(-1), nan.all(-1))
