@@ -348,13 +348,20 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       }
     };
 
+    // ~0, or 0 for a block none of whose keys the queries from qw0 on may see (a mask and no select: the compiler makes a
+    // branch of one, and the values alive across it do not fit the registers any more)
+    auto seen_mask = [&](int qw0) {
+      return (unsigned)__builtin_amdgcn_readfirstlane(sub_skip<AC>(k0, qw0) ? 0 : -1);
+    };
+    auto and8 = [](el8 v, unsigned m) { return __builtin_bit_cast(el8, __builtin_bit_cast(u32x4, v) & u32x4{m, m, m, m}); };
     // What a step keeps of a block between forming its weights and forming its dz, one step later.
     struct Weights { float p[16], r[16], lo; };
     // Step w: dz of block w (weights and do.v in `wc`, `dc`, formed a step ago), weights of block w + 1 (scores `xn`,
     // do.v `dn`) into `wn`, and the two MFMA chains of block w + 2 into `xf`, `df`, interleaved with the vector work in
     // eight chunks (see bulk in sba_bwd.hip).  The sum over the key blocks before this wave's goes through `tot`: written
-    // with the weights, read a step later.  FIRST: there is no block w yet.  BAND: block w + 1 may hold keys its
-    // queries must not see.  SLOT >= 0: ring slot of tile w + 2, else taken from w.
+    // with the weights, read a step later.  FIRST: there is no block w yet.  BAND: block w or w + 1 may hold keys its
+    // queries must not see.  A block that hides all of them stages zeros and nothing computed: where a key has a value that is
+    // not finite, or a query a running sum that is not, 0 times it is not zero.  SLOT >= 0: ring slot of tile w + 2, else taken from w.
     auto step = [&](auto first_tag, auto band_tag, auto slot_tag, const int w, Weights& wc, f32x16& dc, f32x16& xn, f32x16& dn,
                     Weights& wn, f32x16& xf, f32x16& df, float& se) __attribute__((always_inline)) {
       constexpr bool FIRST = decltype(first_tag)::value, BAND = decltype(band_tag)::value;
@@ -427,8 +434,9 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
 #pragma unroll
         for (int j = 8; j < 16; ++j) { const float dj = fmaf(wc.p[j], dc[j], dprev); dz[j] = fmaf(wc.r[j], dj, -dprev); dprev = dj; }
         unsigned short* Zt = Zs + par * PTILE;
-        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h)) = pack8(dz);
-        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h + 1)) = pack8(dz + 8);
+        const unsigned keep = BAND ? seen_mask(qw0 + TQ) : ~0u;
+        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h)) = and8(pack8(dz), keep);
+        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h + 1)) = and8(pack8(dz + 8), keep);
         // what the next key tile starts from (the half-wave with the newer keys ends with the sum over all)
         if (kb == 3 && h == 1) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dprev), out_rs, row4 - w * (4 * TQ), 0, 0);
         post(1);
@@ -522,11 +530,12 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         post(0);
         unsigned short* Zt = Zs + par * PTILE;
         unsigned short* Pt = Ps + par * PTILE;
-        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h)) = pack8(dz);
+        const unsigned keep = BAND ? seen_mask(qw0) : ~0u;
+        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h)) = and8(pack8(dz), keep);
 #pragma unroll
         for (int j = 8; j < 16; ++j) { const float dj = fmaf(wc.p[j], dc[j], dprev); dz[j] = fmaf(wc.r[j], dj, -dprev); dprev = dj; }
         post(1);
-        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h + 1)) = pack8(dz + 8);
+        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h + 1)) = and8(pack8(dz + 8), keep);
         if (kb == 3 && h == 1) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dprev), out_rs, row4 - w * (4 * TQ), 0, 0);
         if (BAND && a.fuse && qw0 == k0) {
 #pragma unroll
@@ -783,6 +792,12 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         const unsigned short* Xt = mat ? Zt : Ps + (b % PBUF) * PTILE;
         const unsigned short* Yt = Ys + (b % RING) * QTILE;
         const bool finished = b >= nsteps - DIAG;               // the queries of this tile's own keys: nothing is missing any more
+        if (finished) {    // key blocks behind these queries stay out of their dq, finite or not (later steps have older queries)
+          const int visible = 2 * ((t_last - b) * NSQ + dsq - (BKV / 32) * kt + 1);
+#pragma unroll
+          for (int ks = 2; ks < KZ; ++ks)
+            if (ks >= visible) kt_f[ks] = zero8();
+        }
         el8 zf[ZH], af[2], bf[DB];
         auto read_x = [&](int ks, int kb2) { return lds_tr8(Xt + (xb[0] ^ (kb2 << 5)) + 16 * ks * BKV, Xt + (xb[1] ^ (kb2 << 5)) + 16 * ks * BKV); };
 #pragma unroll

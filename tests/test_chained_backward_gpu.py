@@ -90,3 +90,38 @@ def test_a_wait_that_runs_out_gives_nan_and_nothing_else(form, steps, d):
     assert lost[0].any() and lost[1].any() and not all(nan.all() for nan in lost)
     for nan in lost:      # (a row is lost as a whole)
         assert torch.equal(nan.any(-1), nan.all(-1))
+
+
+@pytest.mark.parametrize("ac", [False, True])
+@pytest.mark.parametrize("steps,d", [(1, 128), (2, 128), (2, 96), (1, 64), (2, 64), (3, 64), (2, 32), (3, 32)])
+def test_rows_that_are_not_finite_stay_behind_the_blocks_that_hide_them(form, steps, d, ac):
+    """A key that is not finite must not reach the gradients of queries that cannot see it, nor a query the gradients of
+    keys it cannot see, beyond the 32-row block of its own: there, the matrix products multiply it by zero."""
+    from stickbreaking_attention import sb_attn_varlen
+    lengths = [300, 128, 77]
+    H, T = 2, sum(lengths)
+    tensors = orc.make_inputs((H, T, d), 77 + d)
+    drem = torch.randn((H, T), generator=torch.Generator().manual_seed(d)).to(torch.bfloat16)
+    cu = cu_from_lengths(lengths, device=DEV)
+    form(steps)
+    def run(x):
+        return [g.cpu() for g in gradients(sb_attn_varlen, x[:3], cu, max(lengths), ac, (x[3], drem))]
+    clean = run(tensors)
+    for start, row in ((0, 3), (0, 40), (0, 100), (0, 127), (0, 200), (0, 299), (300, 90), (428, 33)):
+        at, length = start + row, lengths[[0, 300, 428].index(start)]
+        block = start + row // 32 * 32
+        older, newer = range(0, block), [i for i in range(T) if i < start or i >= min(block + 32, start + length)]
+        other = [i for i in range(T) if i != at]
+        for which, value in ((0, float("nan")), (1, float("nan")), (1, float("-inf")), (2, float("inf")), (2, float("nan")), (3, float("inf"))):
+            x = [t.clone() for t in tensors]
+            x[which][:, at] = value
+            dq, dk, dv = run(x)
+            same = lambda a, b, rows: torch.equal(a[:, list(rows)], b[:, list(rows)])
+            name = f"{'q k v do'.split()[which]}[{at}] = {value}"
+            if which in (1, 2):       # a key: queries before its block
+                assert same(dq, clean[0], older), name
+            if which == 2:            # and its value: keys before its block, and no dv
+                assert same(dk, clean[1], older) and torch.equal(dv, clean[2]), name
+            if which in (0, 3):       # a query: all other queries, keys behind its block
+                assert same(dq, clean[0], other), name
+                assert same((dv, dk)[which // 3], clean[2 - which // 3], newer), name
