@@ -240,7 +240,7 @@ int sba_attn_bwd(const sba_problem* p, const void* schedule, size_t schedule_siz
  * a caller then takes sba_varlen_bwd / sba_attn_bwd.  Same inputs, outputs, table and refusals; it
  * needs no gradient table, and the results differ from the two-pass form's by rounding.  Problems it
  * cannot take (log-space carry, head_dim > 128, a device that is not eight XCDs of 32 compute units)
- * return SBA_E_SHAPE.  The stream's CU mask, if it has one, must leave every XCD at least one CU. */
+ * return SBA_E_SHAPE. */
 size_t sba_chain_scratch_bytes(const sba_problem* p);
 int sba_varlen_bwd_chained(const sba_problem* p, const void* schedule, size_t schedule_size,
                            const sba_view* q, const sba_view* k, const sba_view* v,
@@ -306,8 +306,11 @@ void  sba_set_dkdv_workgroups(int n);
 /* Test and tuning switch (process-wide): which form of the backward sba_chain_scratch_bytes asks for.  0: by size,
  * 1: never the one-pass form, 2: wherever it is possible, 3: the same in steps of 64 queries (head_dim <= 64).
  * With SBA_FORM_SHORT_WAITS added, a wait of the one-pass form for the key tile before gives up after its
- * first look, as it otherwise does after about a second: what the missing partial sums belong to is NaN. */
+ * first look, as it otherwise does after about a second: what the missing partial sums belong to is NaN.
+ * With SBA_FORM_IDLE_XCDS(mask), the XCDs in `mask` (of bits 0 .. 7, not all) count as without a compute unit for
+ * the one-pass form, as a CU mask may leave them. */
 #define SBA_FORM_SHORT_WAITS 0x100
+#define SBA_FORM_IDLE_XCDS(mask) ((mask) << 16)
 void  sba_set_backward_form(int form);
 
 #ifdef __cplusplus

@@ -292,7 +292,7 @@ int backward(const sba_problem* p, bool fixed, const void* schedule, size_t sche
 
 // ---- the one-pass backward (sba_chain.hip) ------------------------------------------------------------
 int chain_width(int head_dim) { return head_dim <= 64 ? 64 : 128; }   // columns of its rows
-struct ChainScratch { size_t partial, carry, flags, queues, total; };   // byte offsets
+struct ChainScratch { size_t partial, carry, flags, queues, homes, total; };   // byte offsets
 ChainScratch chain_scratch(const sba_problem* p, const Sizes& sz) {
   const size_t tiles = (size_t)p->heads * (size_t)sz.n_kv_max;
   auto line = [](size_t n) { return (n + 255) & ~(size_t)255; };
@@ -301,12 +301,12 @@ ChainScratch chain_scratch(const sba_problem* p, const Sizes& sz) {
   c.carry = line(tiles * BM * chain_width(p->head_dim) * sizeof(float));
   c.flags = c.carry + line(2 * tiles * BM * sizeof(float));
   c.queues = c.flags + line(tiles * sizeof(int));
-  c.total = c.queues + line(CHAIN_QUEUES * CHAIN_QUEUE_STRIDE * sizeof(unsigned));
+  c.homes = c.queues + line(CHAIN_QUEUES * CHAIN_QUEUE_STRIDE * sizeof(unsigned));
+  c.total = c.homes + line(CHAIN_HOMES * sizeof(int));
   return c;
 }
 
-// Whether the kernels can take the problem at all: eight XCDs whose queues are all served (a grid of one workgroup
-// per compute unit reaches every XCD), ranked documents, room for the queue's groups in LDS and 32-bit
+// Whether the kernels can take the problem at all: a device of eight XCDs with 32 compute units each, ranked documents, room for the queue's groups in LDS and 32-bit
 // offsets into a document's partial dq.
 bool chain_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
   const long long chains = (long long)sz.n_docs * p->heads;
@@ -384,6 +384,7 @@ int backward_chained(const sba_problem* p, bool fixed, const void* schedule, siz
   a.carry = reinterpret_cast<float*>(base + at.carry);
   a.flags = reinterpret_cast<int*>(base + at.flags);
   a.queues = reinterpret_cast<unsigned*>(base + at.queues);
+  a.homes = reinterpret_cast<int*>(base + at.homes);
   a.tab_stride = c.tab_stride;
   a.docs_off = SCHED_HDR + TILE_WORDS * (sz.n_q_max + sz.n_kv_max) + chain_docs_offset(sz.n_docs);
   a.n_docs = sz.n_docs;
@@ -397,7 +398,10 @@ int backward_chained(const sba_problem* p, bool fixed, const void* schedule, siz
   a.clear_spare = fixed ? 0 : 1;
   a.nan_pair = p->dtype == SBA_F16 && !a.out_f32 ? 0x7e007e00u : 0x7fc07fc0u;
   a.max_doc_len = declared_max_doc_len(p, fixed);
-  a.spin_limit = g_backward_form.load() & SBA_FORM_SHORT_WAITS ? 0 : CHAIN_SPIN_LIMIT;
+  const int form = g_backward_form.load();
+  a.spin_limit = form & SBA_FORM_SHORT_WAITS ? 0 : CHAIN_SPIN_LIMIT;
+  a.idle_xcds = ((form >> 16) & 0xff) == 0xff ? 0 : (form >> 16) & 0xff;
+  a.n_homes = (int)std::min<long long>(CHAIN_HOMES, (long long)sz.n_q_max * p->heads);
   a.c = c.c;
   a.inv_temp = c.inv_temp;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);

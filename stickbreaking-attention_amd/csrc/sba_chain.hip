@@ -43,9 +43,11 @@ inline namespace SBA_ELEM_NS {
 // Rows of one 32-row fp32 block of partial dq: four dwordx4 per lane.
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-// Ahead of the main kernel: clears the flags and the queues, forms D in front of the oldest key of every row, and
-// writes the rows that belong to no document (or NaN everywhere when the launch is refused).  One
-// workgroup per query tile and head.
+__device__ __forceinline__ int this_xcd() { return __builtin_amdgcn_s_getreg(20 | (3 << 11)) & (CHAIN_QUEUES - 1); }   // HW_REG_XCC_ID, bits 3:0
+
+// Ahead of the main kernel: clears the flags and the queues, notes which XCDs its workgroups run on (the main kernel's
+// will run on the same), forms D in front of the oldest key of every row, and writes the rows that belong to no
+// document (or NaN everywhere when the launch is refused).  One workgroup per query tile and head.
 template <int D>
 __global__ void __launch_bounds__(NT) chain_prep_kernel(const ChainArgs a) {
   const int* sched = a.sched;
@@ -57,6 +59,10 @@ __global__ void __launch_bounds__(NT) chain_prep_kernel(const ChainArgs a) {
   const bool refused = hdr.x != 0 || hdr.w > a.tab_stride || sched[SCHED_MAXLEN] > a.max_doc_len;
   const int tid = threadIdx.x;
   if (blockIdx.x == 0 && tid < CHAIN_QUEUES * CHAIN_QUEUE_STRIDE) a.queues[tid] = 0u;
+  if (blockIdx.x < CHAIN_HOMES && tid == 0) {
+    const int xcd = this_xcd();
+    a.homes[blockIdx.x] = (a.idle_xcds >> xcd) & 1 ? -1 : xcd;
+  }
   if (tid == 0) a.flags[head * a.tiles + slot] = 0;
   if (refused || slot >= hdr.y) {
     if (a.clear_spare) {
@@ -120,7 +126,8 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
   __shared__ __attribute__((aligned(16))) unsigned short PZ[(PBUF + 2) * PTILE];   // p: PBUF buffers, dz: two buffers, [query][key]
   __shared__ float tot[2][NSQ][4][32];       // by step parity: every key block's sum of p (do.v) per query
   __shared__ float given_up;                 // 0, or NaN once a wait of this workgroup has run out (see await)
-  __shared__ int prefix[CHAIN_MAX_GROUPS];   // items of this XCD's queue up to and including each group
+  __shared__ int prefix[CHAIN_MAX_GROUPS];   // key tiles of the longest chains, up to and including each group's
+  __shared__ int place;                      // this XCD's number among those that serve a queue, their count (bits 8 ..)
   __shared__ int mbox[2][8];
   __shared__ __attribute__((aligned(16))) unsigned short spare[4][512];   // where a product wave's copies of nothing go
   unsigned short* const Ps = PZ;
@@ -161,27 +168,32 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
   constexpr int LOADS_PER_TILE = 2 * Copy::NCH;
 
   // ---- the queue of this XCD ---------------------------------------------------------------------
-  // Chains (document rank, head), longest documents first, are dealt to the XCDs in turn.  An XCD's chains are taken in
-  // groups of CHAIN_GROUP whose key tiles are interleaved (tile 0 of each, tile 1 of each, ...), so that the
-  // tiles that start together at the beginning of a launch have few predecessors to wait for.  Ticket
-  // numbers run over the groups' items; a group has room for its longest chain, the tickets behind a
+  // Chains (document rank, head), longest documents first, are dealt to the XCDs in turn, CHAIN_GROUP to each from every
+  // group of eight times as many.  The key tiles of an XCD's chains of a group are interleaved (tile 0 of each, tile 1 of
+  // each, ...), so that the tiles that start together at the beginning of a launch have few predecessors to wait for.
+  // Ticket numbers run over the groups' items; a group has room for its longest chain, the tickets behind a
   // shorter one's end name no item and are drawn past.
-  const int xcd = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & (CHAIN_QUEUES - 1);   // HW_REG_XCC_ID, bits 3:0
+  // An XCD that the launch cannot run on (a CU mask) is dealt none: the XCDs counted are those that the prep kernel met.
+  // With n of them each takes every n-th chain of a group, in room for the next power of two.
+  const int xcd = this_xcd();
   unsigned* const ctr = a.queues + xcd * CHAIN_QUEUE_STRIDE;
   const int n_groups = (n_chains + CHAIN_QUEUES * CHAIN_GROUP - 1) / (CHAIN_QUEUES * CHAIN_GROUP);
-  auto group_items = [&](int g) {   // room of group g: its first chain belongs to its longest document
+  auto group_tiles = [&](int g) {   // of group g's longest chain: the first one belongs to its longest document
     if (g >= n_groups) return 0;
     const int len = docs[2 * (CHAIN_QUEUES * CHAIN_GROUP * g / a.heads)].y;
-    return CHAIN_GROUP * ((len + BKV - 1) / BKV);
+    return (len + BKV - 1) / BKV;
   };
   // first score wave: the item of a ticket, or the items of further tickets, as `mbox` words of the lanes 0 .. 7
   auto resolve = [&](unsigned ticket) -> int {
+    const int here = __builtin_amdgcn_readfirstlane(place), n_xcds = here >> 8;
+    const int lg = 3 + __builtin_clz(n_xcds) - __builtin_clz(CHAIN_QUEUES);    // room for 2^lg chains per group
+    static_assert(CHAIN_GROUP == 8, "lg");
     for (;;) {
       const int tk = __builtin_amdgcn_readfirstlane((int)ticket);
       int group = -1, before = 0;
       for (int g0 = 0; g0 < n_groups; g0 += 64) {
         const int upto = g0 + lane < n_groups ? prefix[g0 + lane] : 0x7fffffff;
-        const unsigned long long m = __builtin_amdgcn_ballot_w64(tk < upto && g0 + lane < n_groups);
+        const unsigned long long m = __builtin_amdgcn_ballot_w64((tk >> lg) < upto && g0 + lane < n_groups);
         if (m != 0) {
           group = g0 + __builtin_ctzll(m);
           break;
@@ -189,10 +201,9 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       }
       if (group < 0) return -1;
       before = group > 0 ? __builtin_amdgcn_readfirstlane(prefix[group - 1]) : 0;
-      const int rel = tk - before;
-      const int kt = rel / CHAIN_GROUP;
-      const int chain = CHAIN_QUEUES * (CHAIN_GROUP * group + rel % CHAIN_GROUP) + xcd;
-      if (chain < n_chains) {
+      const int kt = (tk >> lg) - before, in_group = (tk & ((1 << lg) - 1)) * n_xcds + (here & 0xff);
+      const int chain = CHAIN_QUEUES * CHAIN_GROUP * group + in_group;
+      if (in_group < CHAIN_QUEUES * CHAIN_GROUP && chain < n_chains) {
         const int rank = chain / a.heads;
         const int2 d0 = docs[2 * rank], d1 = docs[2 * rank + 1];
         if (kt * BKV < d0.y) {
@@ -217,9 +228,10 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       ticket = atomicAdd(ctr, 1u);
       given_up = 0.0f;
     }
+    const int home = lane < a.n_homes ? a.homes[lane] : -1;
     int base = 0;
     for (int g0 = 0; g0 < n_groups; g0 += 64) {
-      int v = group_items(g0 + lane);
+      int v = group_tiles(g0 + lane);
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
         const int u = __shfl_up(v, o, 64);
@@ -228,8 +240,12 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       if (g0 + lane < n_groups) prefix[g0 + lane] = base + v;
       base += __shfl(v, 63, 64);
     }
+    int met = 0;
+#pragma unroll
+    for (int x = 0; x < CHAIN_QUEUES; ++x) met |= __builtin_amdgcn_ballot_w64(home == x) != 0 ? 1 << x : 0;
+    if (lane == 0) place = __builtin_popcount(met) << 8 | __builtin_popcount(met & ((1 << xcd) - 1));
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    const int word = resolve(ticket);
+    const int word = (met >> xcd) & 1 ? resolve(ticket) : -1;
     if (lane < 8) mbox[1][lane] = word;
   }
   lds_barrier();

@@ -43,6 +43,7 @@ struct KArgs {
 // Arguments of the one-pass backward (sba_chain.hip).
 constexpr int CHAIN_QUEUES = 8;            // one per XCD
 constexpr int CHAIN_QUEUE_STRIDE = 32;     // words between the queues' counters: a 128-byte line each
+constexpr int CHAIN_HOMES = 64;            // workgroups of the prep kernel that note their XCD: dealt out in turn, 8 of them meet all
 constexpr int CHAIN_GROUP = 8;             // chains of a queue whose items are interleaved
 constexpr int CHAIN_MAX_GROUPS = 256;
 constexpr int CHAIN_SPIN_LIMIT = 1 << 20;  // polls of a wait (about a second) before it gives up and the results turn to NaN
@@ -54,6 +55,7 @@ struct ChainArgs {
   float* carry;                // [2][heads][tiles][BM] fp32: the running sum along the keys, by parity of the key tile that reads it
   int* flags;                  // [heads][tiles]: steps a key tile has published
   unsigned* queues;            // CHAIN_QUEUES counters
+  int* homes;                  // [n_homes] XCD of the prep kernel's first workgroups
   int64_t tab_stride;
   int docs_off;                // int32 offset of the ranked documents inside `sched`
   int n_docs, heads, head_dim, tokens, tiles;
@@ -61,6 +63,8 @@ struct ChainArgs {
   unsigned nan_pair;
   int max_doc_len;
   int spin_limit;              // CHAIN_SPIN_LIMIT, or what a test asks for
+  int n_homes;
+  int idle_xcds;               // test: XCDs (a bit each) taken for ones this launch cannot run on
   float c, inv_temp;
 };
 
@@ -80,7 +84,7 @@ __device__ __forceinline__ void globals_of(KArgs& a) {
 __device__ __forceinline__ void globals_of(ChainArgs& a) {
   as_global(a.q.ptr); as_global(a.k.ptr); as_global(a.v.ptr); as_global(a.go.ptr); as_global(a.grem.ptr);
   as_global(a.dq.ptr); as_global(a.dk.ptr); as_global(a.dv.ptr);
-  as_global(a.sched); as_global(a.stick); as_global(a.partial); as_global(a.carry); as_global(a.flags); as_global(a.queues);
+  as_global(a.sched); as_global(a.stick); as_global(a.partial); as_global(a.carry); as_global(a.flags); as_global(a.queues); as_global(a.homes);
 }
 
 // The argument block read afresh from the kernel-argument segment.  A persistent kernel calls this at

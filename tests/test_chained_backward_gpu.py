@@ -125,3 +125,20 @@ def test_rows_that_are_not_finite_stay_behind_the_blocks_that_hide_them(form, st
             if which in (0, 3):       # a query: all other queries, keys behind its block
                 assert same(dq, clean[0], other), name
                 assert same((dv, dk)[which // 3], clean[2 - which // 3], newer), name
+
+
+@pytest.mark.parametrize("idle", [0x01, 0x20, 0xaa, 0xf7, 0xfe])
+@pytest.mark.parametrize("steps,d,H,lengths", [(2, 128, 1, [500]), (2, 96, 12, [900, 31, 2000, 128]), (3, 64, 40, [1500, 700, 129])])
+def test_queues_of_xcds_that_cannot_run_the_launch(form, idle, steps, d, H, lengths):
+    """What a CU mask can do: some XCDs get no workgroup.  Their queues are served by the others, with the same bits."""
+    from stickbreaking_attention import sb_attn_varlen
+    T = sum(lengths)
+    tensors = orc.make_inputs((H, T, d), 5 + d)
+    drem = torch.randn((H, T), generator=torch.Generator().manual_seed(d)).to(torch.bfloat16)
+    cu = cu_from_lengths(lengths, device=DEV)
+    form(steps)
+    whole = gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem))
+    form(steps | idle << 16)
+    some = gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem))
+    for name, a, b in zip(("dq", "dk", "dv"), whole, some):
+        assert torch.isfinite(a).all() and torch.equal(a, b), name
