@@ -287,7 +287,8 @@ const char* sba_error_string(int code);
  * compute launch is bracketed by HIP events on the caller's stream (event creation, no waiting:
  * timed kernels follow one another on the device as untimed ones do); sba_last_kernel_ms WAITS
  * for the most recent launch of the kernel asked for and returns its duration in milliseconds
- * (which: 0 = forward, 1 = backward dq pass, 2 = backward dk/dv pass).  One process-wide switch
+ * (which: 0 = forward, 1 = backward dq pass, 2 = backward dk/dv pass, or the whole of the one-pass
+ * backward), 0 if it has not been launched since the switch was turned on.  One process-wide switch
  * and one process-wide set of results (the backward may run on PyTorch's autograd thread): do
  * not use with concurrent callers, under graph capture, or in production.  Off by default;
  * sba_varlen_fwd_static ignores it. */

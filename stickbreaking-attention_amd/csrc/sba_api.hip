@@ -634,7 +634,18 @@ int sba_launch_geometry(const sba_problem* p, sba_geometry* out) {
   return 0;
 }
 
-void sba_set_timing(int on) { g_timing.store(on); }
+void sba_set_timing(int on) {
+  if (on) {   // what was timed before is forgotten: a kernel that is not launched from here on reads 0
+    std::lock_guard<std::mutex> lock(g_ev_mutex);
+    for (int i = 0; i < 3; ++i) {
+      if (g_ev[i].e0) (void)hipEventDestroy(g_ev[i].e0);
+      if (g_ev[i].e1) (void)hipEventDestroy(g_ev[i].e1);
+      g_ev[i] = EventPair();
+      g_ms[i].store(0.0f);
+    }
+  }
+  g_timing.store(on);
+}
 void sba_set_dkdv_workgroups(int n) { g_dkdv_workgroups.store(n); }
 void sba_set_backward_form(int form) { g_backward_form.store(form); }
 float sba_last_kernel_ms(int which) {

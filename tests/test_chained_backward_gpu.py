@@ -142,3 +142,22 @@ def test_queues_of_xcds_that_cannot_run_the_launch(form, idle, steps, d, H, leng
     some = gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem))
     for name, a, b in zip(("dq", "dk", "dv"), whole, some):
         assert torch.isfinite(a).all() and torch.equal(a, b), name
+
+
+def test_timing_forgets_the_launches_of_another_run(form):
+    """bench.py takes a dq pass without a duration for a sign of the one-pass form: what an earlier run left there must
+    not be seen."""
+    from stickbreaking_attention import _native, sb_attn_varlen
+    lib = _native.load()
+    tensors = orc.make_inputs((2, 300, 64), 1)
+    cu = cu_from_lengths([300], device=DEV)
+    ms = {}
+    try:
+        for steps in (1, 2):
+            form(steps)
+            lib.sba_set_timing(1)
+            gradients(sb_attn_varlen, tensors[:3], cu, 300, False, (tensors[3], torch.zeros((2, 300), dtype=torch.bfloat16)))
+            ms[steps] = [lib.sba_last_kernel_ms(i) for i in range(3)]
+    finally:
+        lib.sba_set_timing(0)
+    assert min(ms[1]) > 0 and ms[2][0] > 0 and ms[2][1] == 0 and ms[2][2] > 0
