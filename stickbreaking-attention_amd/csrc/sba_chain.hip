@@ -185,22 +185,23 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
   };
   // first score wave: the item of a ticket, or the items of further tickets, as `mbox` words of the lanes 0 .. 7
   auto resolve = [&](unsigned ticket) -> int {
-    const int here = __builtin_amdgcn_readfirstlane(place), n_xcds = here >> 8;
+    const int first = prefix[min(lane, n_groups - 1)], here = __builtin_amdgcn_readfirstlane(place), n_xcds = here >> 8;
     const int lg = 3 + __builtin_clz(n_xcds) - __builtin_clz(CHAIN_QUEUES);    // room for 2^lg chains per group
     static_assert(CHAIN_GROUP == 8, "lg");
     for (;;) {
       const int tk = __builtin_amdgcn_readfirstlane((int)ticket);
       int group = -1, before = 0;
       for (int g0 = 0; g0 < n_groups; g0 += 64) {
-        const int upto = g0 + lane < n_groups ? prefix[g0 + lane] : 0x7fffffff;
-        const unsigned long long m = __builtin_amdgcn_ballot_w64((tk >> lg) < upto && g0 + lane < n_groups);
+        const int upto = g0 == 0 ? first : prefix[min(g0 + lane, n_groups - 1)];
+        const unsigned long long m = __builtin_amdgcn_ballot_w64((tk >> lg) < upto);    // (lanes past the last group repeat it)
         if (m != 0) {
-          group = g0 + __builtin_ctzll(m);
+          const int at = __builtin_ctzll(m);
+          group = g0 + at;
+          before = at > 0 ? __builtin_amdgcn_readlane(upto, at - 1) : g0 > 0 ? __builtin_amdgcn_readfirstlane(prefix[g0 - 1]) : 0;
           break;
         }
       }
       if (group < 0) return -1;
-      before = group > 0 ? __builtin_amdgcn_readfirstlane(prefix[group - 1]) : 0;
       const int kt = (tk >> lg) - before, in_group = (tk & ((1 << lg) - 1)) * n_xcds + (here & 0xff);
       const int chain = CHAIN_QUEUES * CHAIN_GROUP * group + in_group;
       if (in_group < CHAIN_QUEUES * CHAIN_GROUP && chain < n_chains) {
@@ -364,12 +365,14 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       }
     };
 
-    // ~0, or 0 for a block none of whose keys the queries from qw0 on may see (a mask and no select: the compiler makes a
-    // branch of one, and the values alive across it do not fit the registers any more)
-    auto seen_mask = [&](int qw0) {
-      return (unsigned)__builtin_amdgcn_readfirstlane(sub_skip<AC>(k0, qw0) ? 0 : -1);
+    // A block none of whose keys the queries from qw0 on may see: zeros in the place of its dz, staged before.  (By a second
+    // store: with a choice between the two values in the step itself the values alive across it do not fit the registers, and a
+    // mask costs every step.)
+    auto hide = [&](int qw0, int par) {
+      if (!sub_skip<AC>(k0, qw0)) return;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) *reinterpret_cast<el8*>(Zs + par * PTILE + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h + c)) = zero8();
     };
-    auto and8 = [](el8 v, unsigned m) { return __builtin_bit_cast(el8, __builtin_bit_cast(u32x4, v) & u32x4{m, m, m, m}); };
     // What a step keeps of a block between forming its weights and forming its dz, one step later.
     struct Weights { float p[16], r[16], lo; };
     // Step w: dz of block w (weights and do.v in `wc`, `dc`, formed a step ago), weights of block w + 1 (scores `xn`,
@@ -450,9 +453,8 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
 #pragma unroll
         for (int j = 8; j < 16; ++j) { const float dj = fmaf(wc.p[j], dc[j], dprev); dz[j] = fmaf(wc.r[j], dj, -dprev); dprev = dj; }
         unsigned short* Zt = Zs + par * PTILE;
-        const unsigned keep = BAND ? seen_mask(qw0 + TQ) : ~0u;
-        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h)) = and8(pack8(dz), keep);
-        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h + 1)) = and8(pack8(dz + 8), keep);
+        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h)) = pack8(dz);
+        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + row, 4 * kb + 2 * h + 1)) = pack8(dz + 8);
         // what the next key tile starts from (the half-wave with the newer keys ends with the sum over all)
         if (kb == 3 && h == 1) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dprev), out_rs, row4 - w * (4 * TQ), 0, 0);
         post(1);
@@ -497,6 +499,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       post(5);
       post(6);
       post(7);
+      if constexpr (BAND && !FIRST) hide(qw0 + TQ, par);
     };
     // The same with one step less between a block's products and its weights, for three waves per SIMD (168 registers), which
     // hide what the pipeline above hides: step w forms the products of block w + 1 next to dz of block w, stages p and
@@ -546,12 +549,11 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         post(0);
         unsigned short* Zt = Zs + par * PTILE;
         unsigned short* Pt = Ps + par * PTILE;
-        const unsigned keep = BAND ? seen_mask(qw0) : ~0u;
-        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h)) = and8(pack8(dz), keep);
+        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h)) = pack8(dz);
 #pragma unroll
         for (int j = 8; j < 16; ++j) { const float dj = fmaf(wc.p[j], dc[j], dprev); dz[j] = fmaf(wc.r[j], dj, -dprev); dprev = dj; }
         post(1);
-        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h + 1)) = and8(pack8(dz + 8), keep);
+        *reinterpret_cast<el8*>(Zt + swz_off<BKV>(32 * sq + n, 4 * kb + 2 * h + 1)) = pack8(dz + 8);
         if (kb == 3 && h == 1) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, dprev), out_rs, row4 - w * (4 * TQ), 0, 0);
         if (BAND && a.fuse && qw0 == k0) {
 #pragma unroll
@@ -584,6 +586,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       both_halves(s0 + s1, lo, hi);
       wc.lo = lo;
       if (h == 0) tot[par ^ 1][sq][kb][n] = lo + hi;
+      if constexpr (BAND && !FIRST) hide(qw0, par);
     };
     // ends a step: the first score wave makes sure that what the others request behind the barrier is there, the second
     // publishes what this tile has finished (formed two steps ago and acknowledged since)
@@ -809,10 +812,10 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         const unsigned short* Yt = Ys + (b % RING) * QTILE;
         const bool finished = b >= nsteps - DIAG;               // the queries of this tile's own keys: nothing is missing any more
         if (finished) {    // key blocks behind these queries stay out of their dq, finite or not (later steps have older queries)
-          const int visible = 2 * ((t_last - b) * NSQ + dsq - (BKV / 32) * kt + 1);
+          const int newest = (t_last - b) * NSQ + dsq - (BKV / 32) * kt;
 #pragma unroll
-          for (int ks = 2; ks < KZ; ++ks)
-            if (ks >= visible) kt_f[ks] = zero8();
+          for (int kb = 1; kb < BKV / 32; ++kb)
+            if (kb > newest) kt_f[2 * kb] = kt_f[2 * kb + 1] = zero8();
         }
         el8 zf[ZH], af[2], bf[DB];
         auto read_x = [&](int ks, int kb2) { return lds_tr8(Xt + (xb[0] ^ (kb2 << 5)) + 16 * ks * BKV, Xt + (xb[1] ^ (kb2 << 5)) + 16 * ks * BKV); };
