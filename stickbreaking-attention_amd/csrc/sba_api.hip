@@ -314,8 +314,8 @@ bool chain_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
          chains <= (long long)CHAIN_QUEUES * CHAIN_GROUP * CHAIN_MAX_GROUPS &&
          ((long long)declared_max_doc_len(p, fixed) + BM) * chain_width(p->head_dim) * 4 < (1ll << 31) && device_cus() == 256;
 }
-// Steps of 64 queries instead of 32 (head_dim <= 64).  They do more per step and CU (4 x 16 x 2048 at head_dim 64: 166 us
-// for 199) but a key tile lags its predecessor by four steps of either size, so as long as that lag is what a problem takes
+// Steps of 64 queries instead of 32 (head_dim <= 64).  They do more per step and CU (4 x 16 x 2048 at head_dim 64: 167 us
+// for 198) but a key tile lags its predecessor by four steps of either size, so as long as that lag is what a problem takes
 // (one head of 1024 keys: 58 us for 49) the small ones are the better ones.  The line: the work of a CU in steps, chains mean^2
 // / (2 x 64 x 128 x 256 CUs), against the steps of the longest document, where beyond 2048 keys more of a chain's tiles
 // start behind one another than side by side (16 x 4096: 250 us for 224, 16 x 8192: 589 for 653).

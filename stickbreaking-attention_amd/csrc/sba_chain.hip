@@ -24,11 +24,13 @@
 // the item an item waits for was drawn before it by a workgroup that is running: waits end.  A tile is
 // published three steps after it was formed (`flags`: steps done per item).
 //
-// Measured (kernel time of the backward, two passes -> prep and chain; MI355X): 32 heads x 16 K tokens in eight documents,
-// head_dim 128, 1606 -> 1388 us; 12 x 4 x 4096 fused 837 -> 750; 16 x 7001 in six documents, head_dim 96, 225 -> 174; 4 x 16 x
-// 2048, head_dim 64, 234 -> 222; 1 x 4 x 512, head_dim 64, 42 -> 31.  At head_dim 128 what bounds it is the partial dq
-// that does not stay in L2 (5.1 GB fetched and 3.3 GB written of 8.6 GB each way in the first of these) and the
-// steps' barriers: 2860 cycles per step where the score waves and the product waves issue for 2350 each.
+// Measured (kernel time of the backward, two passes -> prep and chain, alternating on one MI355X): 32 heads x 16 K tokens in
+// eight documents, head_dim 128, 1560 -> 1411 us (forward and backward as a program calls them: 1979 -> 1856); 12 x 4 x 4096
+// fused 819 -> 716; 16 x 7001 in six documents, head_dim 96, 187 -> 177; 4 x 16 x 2048, head_dim 64, 213 -> 167; 1 x 4 x 512,
+// head_dim 64, 45 -> 36.  At head_dim 128 it waits: 41 % of the wave cycles on 32 heads x 16 K tokens (22 .. 25 % in the two
+// passes; profiles/c3_sq_counters_pmc.txt), with the matrix pipe busy for 34 %.  Such a launch fetches 4.7 GB from behind
+// the L2s and writes 3.1 GB there, 6.0 TB/s where a plain copy reaches 4.9: of the 2.8 GB of partial dq each way, all
+// that is written leaves L2 (eight chains of 2 MiB share 4 MiB).
 //
 // Carried sum: with C[j] the sum of G over the keys up to j and ex the stick on entering a key, D = C + drem ex
 // obeys D[j] = D[j-1] + p_j (do.v_j) and dz_j = r_j D[j] - D[j-1] (see grad_dz in sba_bwd.hip); the gradient of
@@ -109,8 +111,8 @@ __global__ void __launch_bounds__(NT) chain_prep_kernel(const ChainArgs a) {
 
 // NSQ: 32-query blocks per step.  4 * NSQ score waves (one per 32-key block and query block) and 4 product waves.  At head_dim
 // 128 registers leave room for one score wave per SIMD, whose vector work (180 instructions, 32 of them transcendental,
-// per block) is the step; at 64 and below two fit (168 registers), and a step of 64 queries takes 3750 cycles where two of 32
-// take 5800: 16 heads x 4 documents of 2048 at head_dim 64 166 us for 199, at head_dim 32 139 for 167 (two passes: 233, 216).
+// per block) is the step; at 64 and below two fit (168 registers): 16 heads x 4 documents of 2048 at head_dim 64 in steps of 64
+// queries 167 us for 198 in steps of 32, at head_dim 32 139 for 169 (two passes: 213, 174).
 template <int D, int U, bool AC, int NSQ>
 __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const ChainArgs a) {
   constexpr int KS = U / 16, DB = U / 32;
@@ -185,15 +187,15 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
   };
   // first score wave: the item of a ticket, or the items of further tickets, as `mbox` words of the lanes 0 .. 7
   auto resolve = [&](unsigned ticket) -> int {
-    const int first = prefix[min(lane, n_groups - 1)], here = __builtin_amdgcn_readfirstlane(place), n_xcds = here >> 8;
+    const int first = prefix[lane], here = __builtin_amdgcn_readfirstlane(place), n_xcds = here >> 8;
     const int lg = 3 + __builtin_clz(n_xcds) - __builtin_clz(CHAIN_QUEUES);    // room for 2^lg chains per group
-    static_assert(CHAIN_GROUP == 8, "lg");
+    static_assert(CHAIN_GROUP == 8 && CHAIN_MAX_GROUPS % 64 == 0, "lg; 64 prefixes at a time");
     for (;;) {
       const int tk = __builtin_amdgcn_readfirstlane((int)ticket);
       int group = -1, before = 0;
       for (int g0 = 0; g0 < n_groups; g0 += 64) {
-        const int upto = g0 == 0 ? first : prefix[min(g0 + lane, n_groups - 1)];
-        const unsigned long long m = __builtin_amdgcn_ballot_w64((tk >> lg) < upto);    // (lanes past the last group repeat it)
+        const int upto = g0 == 0 ? first : prefix[g0 + lane];       // (past the last group: anything)
+        const unsigned long long m = __builtin_amdgcn_ballot_w64((tk >> lg) < upto && g0 + lane < n_groups);
         if (m != 0) {
           const int at = __builtin_ctzll(m);
           group = g0 + at;
