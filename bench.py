@@ -24,18 +24,20 @@ for p in (ROOT, os.path.join(ROOT, "stickbreaking-attention_amd")):
 PEAK_BF16_TFLOPS = 2500.0   # MI355X published dense bf16 MFMA peak
 PEAK_HBM_GBS = 8000.0       # MI355X published HBM3E bandwidth
 
-# Figures that only rocprofv3 can see, on workload c3, recorded from the runs whose summaries are under profiles/
+# Figures that only rocprofv3 can see, on workloads c3 and c2, recorded from the runs whose summaries are under profiles/
 # and valid for the library version they were measured with (any other version of libsba.so reports null).
-#   traffic: HBM bytes per launch from two `--pmc` runs of this script (FETCH_SIZE, then WRITE_SIZE, KiB per
-#     dispatch, summed over XCDs), each scaled by what the same counter reads for the 256 MiB device copy of
-#     --calibrate-copy (FETCH_SIZE x2.0, WRITE_SIZE x1.0): profiles/c3_hbm_traffic_pmc.txt
+#   traffic: bytes per launch between the L2s and the fabric from two `--pmc` runs of this script (FETCH_SIZE, then
+#     WRITE_SIZE, KiB per dispatch, summed over XCDs), each scaled by what the same counter reads for the 256 MiB device
+#     copy of --calibrate-copy (FETCH_SIZE x2.0, WRITE_SIZE x1.0): profiles/c3_hbm_traffic_pmc.txt
 #   mfma_busy, valu_busy, coexec: fractions of the launch's SIMD-cycles in which the matrix pipe is busy
 #     (SQ_VALU_MFMA_BUSY_CYCLES), a vector instruction is active (4 x SQ_ACTIVE_INST_VALU) and both at once
 #     (SQ_VALU_MFMA_COEXEC_CYCLES), over 1024 SIMDs x GRBM_GUI_ACTIVE / 8: profiles/c3_sq_counters_pmc.txt
-MEASURED = {"sba_version": 213,
-            "c3": {"fwd_kernel": {"traffic": 1.097e9, "mfma_busy": 0.462, "valu_busy": 0.554, "coexec": 0.193},
-                   "bwd_dq_kernel": {"traffic": 1.108e9, "mfma_busy": 0.428, "valu_busy": 0.578, "coexec": 0.166},
-                   "bwd_dkdv_kernel": {"traffic": 1.228e9, "mfma_busy": 0.421, "valu_busy": 0.503, "coexec": 0.181}}}
+#   (c2: profiles/c2_one_pass_backward.txt)
+MEASURED = {"sba_version": 214,
+            "c3": {"fwd_kernel": {"traffic": 1.041e9, "mfma_busy": 0.463, "valu_busy": 0.552, "coexec": 0.191},
+                   "bwd_chain_kernel": {"traffic": 7.872e9, "mfma_busy": 0.344, "valu_busy": 0.376, "coexec": 0.104}},
+            "c2": {"fwd_kernel": {"traffic": 1.135e8, "mfma_busy": 0.245, "valu_busy": 0.541, "coexec": 0.150},
+                   "bwd_chain_kernel": {"traffic": 6.485e8, "mfma_busy": 0.229, "valu_busy": 0.466, "coexec": 0.115}}}
 
 KERNELS = ["fwd_kernel", "bwd_dq_kernel", "bwd_dkdv_kernel"]
 # algorithmic and executed FLOPs per causal pair and head_dim of each, and of the one-pass backward, which takes the
