@@ -230,6 +230,7 @@ int forward(const sba_problem* p, bool fixed, const void* schedule, size_t sched
   else { a.v = to_view(v); a.o = to_view_out(o, p); a.rem = to_view_out(rem, p); }
   a.stick = stick;
   a.weights = weights;
+  a.resident = device_cus();
   a.clear_spare = fixed ? 0 : 1;
   a.nan_pair = p->dtype == SBA_F16 && !a.out_f32 ? 0x7e007e00u : 0x7fc07fc0u;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);

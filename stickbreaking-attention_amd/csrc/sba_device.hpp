@@ -40,6 +40,7 @@ __host__ __device__ inline int kv_tail_tiles(int len) {   // key tiles of a docu
   const int nkv = (len + BKV - 1) / BKV;
   return len <= TAIL_TILES * BKV ? nkv : 1;
 }
+constexpr int CLASS_TILES = 4;   // query tiles a document has at least for its tiles to be listed among those of others (sched_kernel)
 constexpr int NT = 256;  // threads per workgroup
 
 // Schedule workspace layout (int32 words).

@@ -166,33 +166,51 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
   // D. emit tiles: slot -> ranked document by binary search over the prefix
   // The hardware deals workgroups to the CUs round-robin in launch order (workgroups i and
   // i + number of CUs start on the same CU and run side by side), and hands out the rest as
-  // slots free up.  Equal-length documents are therefore listed tile-major, the most expensive
-  // tile of every document first: all expensive tiles start at once and the cheap ones fill
-  // in behind them.  (Document-major order would put the same tile of every batch entry on
-  // the same CU.)  Packed documents of different lengths stay document-major, which keeps the
-  // K/V rows a workgroup's neighbours read in the caches.
+  // slots free up.  Documents of like length -- a class: more than half as many tiles as its longest -- are therefore
+  // listed tile-major, the most expensive tile of every document first: the expensive tiles start together and the cheap
+  // ones fill in behind them.  Document-major, the last document's most expensive tile starts when most of the launch is
+  // over, and documents of one length put the same tile on the same CU.  Classes follow one another,
+  // so that a workgroup's neighbours still share K/V rows in the caches.  Forward, document-major / one class for all / as
+  // built: 12 heads x 4 x 4096 at head_dim 128 264 / 206 / 206 us, 32 heads x 16 K tokens in 8 documents 422 / 426 / 410, 8 heads
+  // x 32 K tokens in documents of 1024 .. 8192 426 / 384 / 393, 32 heads x 64 K tokens, one document of 32 K among shorter
+  // ones, 10.11 / 10.43 / 10.15 ms.  Documents of less than CLASS_TILES tiles stay document-major: their tiles cost about the
+  // same and share most of their rows (32 heads x 16 K tokens in 207 documents of 16 .. 256: 66.2 / 67.4 us).
   for (int s = tid; s < total_q && ok; s += SCHED_THREADS) {
-    int d, within, rank = 0;   // document, position among its tiles in cost order
+    int d, idx, rank = 0, slot = s;
     if (fixed) {
       d = s % nd;
-      within = s / nd;
+      idx = cdiv(len_of[d], BM) - 1 - s / nd;
     } else {
+      auto tiles_of = [&](int r) { return q_before[r + 1] - q_before[r]; };
+      // the first rank from r0 on with at most n tiles (ranks are in descending order)
+      auto first_with_at_most = [&](int r0, int n) {
+        int lo = r0, hi = nd;
+        while (lo < hi) { const int mid = (lo + hi) >> 1; if (tiles_of(mid) <= n) hi = mid; else lo = mid + 1; }
+        return lo;
+      };
       int lo = 0, hi = nd;   // largest i with qoff[i] <= s
       while (hi - lo > 1) { const int mid = (lo + hi) >> 1; if (q_before[mid] <= s) lo = mid; else hi = mid; }
       rank = lo;
       d = ranked[lo];
-      within = s - q_before[lo];
+      idx = tiles_of(rank) - 1 - (s - q_before[rank]);             // newest (most expensive) query tile first
+      if (in_lds && tiles_of(rank) >= CLASS_TILES) {
+        int r0 = 0;          // of this document's class: its first rank
+        for (int n = tiles_of(0); 2 * tiles_of(rank) <= n; n = tiles_of(r0)) r0 = first_with_at_most(r0, n / 2);
+        // ahead of tile idx of this document: every tile of the class above idx, then the same tile of longer documents
+        const int longer = first_with_at_most(r0, idx + 1) - r0;   // documents of the class that have a tile idx + 1 ...
+        const int r1 = min(r0 + longer, first_with_at_most(r0, max(tiles_of(r0) / 2, CLASS_TILES - 1)));   // ... and are in it
+        slot = q_before[r0] + (q_before[r1] - q_before[r0] - (r1 - r0) * (idx + 1)) + (rank - r0);
+      }
     }
-    const int nq = cdiv(len_of[d], BM);
     Tile t;
     t.tok_start = fixed ? 0 : start_of[d];
     t.doc_len = len_of[d];
-    t.idx = nq - 1 - within;             // newest (most expensive) query tile first
+    t.idx = idx;
     t.batch = fixed ? d : 0;
     t.tab_base = tab_of[d];
     t.tile_base = q_before[fixed ? d : rank];
     t.rsv[0] = t.rsv[1] = 0;
-    qtiles[s] = t;
+    qtiles[slot] = t;
   }
   // Key tiles stay document-major for every input: one workgroup per CU runs at a time, so the
   // hardware hands them out one by one as CUs free up, and neighbours that share a document

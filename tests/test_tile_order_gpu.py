@@ -1,0 +1,52 @@
+"""In which order the query tiles of packed documents are listed, and which of them a workgroup of the forward takes."""
+import random
+
+import pytest
+import torch
+
+from stickbreaking_attention import sb_attn_varlen
+from tests import helpers
+from tests.test_schedule_gpu import DEV, _schedule
+
+pytestmark = pytest.mark.gpu
+CLASS_TILES = 4
+
+
+def _listed(lengths):
+    """(length, tile) in the order of the list: classes of documents of more than half as many tiles as their longest, a class tile-major;
+    documents of less than CLASS_TILES tiles one by one."""
+    lengths = sorted(lengths, reverse=True)
+    tiles = [-(-n // 128) for n in lengths]
+    out, r = [], 0
+    while r < len(tiles):
+        end = r + 1
+        while tiles[r] >= CLASS_TILES and end < len(tiles) and 2 * tiles[end] > tiles[r] and tiles[end] >= CLASS_TILES:
+            end += 1
+        for i in range(tiles[r] - 1, -1, -1):
+            out += [(lengths[x], i) for x in range(r, end) if tiles[x] > i]
+        r = end
+    return out
+
+
+@pytest.mark.parametrize("lengths", [[512], [385, 384, 383, 1], [4096] * 4, [100] * 30, [0, 1024, 513, 512, 511, 0, 128, 129],
+                                     [2048, 1025, 1024, 897, 896, 600, 512, 385, 384, 300, 7],
+                                     [random.Random(5).randint(1, 3000) for _ in range(40)],
+                                     [random.Random(6).choice([200, 400, 500, 900]) for _ in range(600)]])
+def test_order_of_the_list(lengths):
+    _, q_tiles, _, _ = _schedule(lengths, sum(lengths))
+    assert [(t[1], t[2]) for t in q_tiles] == _listed(lengths)
+
+
+@pytest.mark.parametrize("heads,head_dim,lengths", [(12, 64, [1500, 700, 129, 2100]), (20, 32, [3000, 1, 1111]), (7, 128, [4096, 900]),
+                                                    (3, 64, [97] * 100)])
+def test_a_launch_dealt_in_turns_covers_every_tile(heads, head_dim, lengths):
+    """More items than compute units, all on the chip at once: the same bits as head by head, which is dealt straight."""
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    q, k, v = (torch.randn(heads, sum(lengths), head_dim, generator=gen, device=DEV).to(torch.bfloat16) for _ in range(3))
+    cu = helpers.cu_from_lengths(lengths, device=DEV)
+    items = heads * sum(-(-n // 128) for n in lengths)
+    assert 256 < items <= 768
+    o, rem = sb_attn_varlen(q, k, v, cu, max(lengths), zero_start=False)
+    for h in range(heads):
+        o1, rem1 = sb_attn_varlen(q[h:h + 1], k[h:h + 1], v[h:h + 1], cu, max(lengths), zero_start=False)
+        assert torch.equal(o[h], o1[0]) and torch.equal(rem[h], rem1[0])
