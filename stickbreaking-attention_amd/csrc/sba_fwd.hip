@@ -18,7 +18,7 @@ inline namespace SBA_ELEM_NS {
 // 4 x 16 x 2048: 53.0 -> 49.9 us at head_dim 64, 40.3 -> 38.2 at 32.
 template <int D>
 __device__ __forceinline__ int deal_item(int n_cus) {
-  constexpr int PER_CU = D <= 32 ? 6 : D <= 64 ? 4 : D <= 128 ? 3 : 1;    // workgroups a CU holds
+  constexpr int PER_CU = D <= 32 ? 6 : D <= 64 ? 4 : D <= 128 ? 3 : 2;    // workgroups a CU holds
   const int b = blockIdx.x, n = gridDim.x;
   if (n <= n_cus || n > PER_CU * n_cus) return b;
   const int round = b / n_cus, first = round * n_cus, eights = min(n_cus, n - first) >> 3, at = (b - first) >> 3;
@@ -30,21 +30,23 @@ __device__ __forceinline__ int deal_item(int n_cus) {
 // (sb_varlen_fwd.py:195-202).  MODE 2 (TAB): write the carry table and nothing else -- no V tiles,
 // no P.V products, no o, no rem -- for a backward whose forward kept no table.  Separate
 // instantiations, so the production kernel (MODE 0) carries none of it.
-// head_dim 256: the ring takes 96 KiB, so one workgroup per CU and one wave per SIMD, with the whole register
-// file (512 registers per lane) for its 64 registers of Q fragments and 128 of accumulators.
+// head_dim 256: two workgroups per CU, so that a wave's waits are another's time: a ring of two slots (64 KiB) and 256 registers, 64 of them
+// Q fragments and 128 accumulators, the tile offsets of columns 128 .. 255 as immediates.  (One workgroup per CU, one wave per SIMD with
+// 512 registers and three slots: 554 us on 16 heads x 16 K tokens in eight documents, this 415.)
 // U: columns that are multiplied (see used_width); tile rows in LDS keep the width D.
 template <int D, bool AC, bool PROD, int MODE, int U = D>
-__global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a) {
+__global__ void __launch_bounds__(NT, D > 128 ? 2 : 3) fwd_kernel(const KArgs a) {
   constexpr bool WOUT = MODE == 1, TAB = MODE == 2;
   constexpr int KS = U / 16;     // contraction steps of K.Q^T
   constexpr int DB = U / 32;     // 32-wide output column blocks of P.V
   constexpr int BF = 32;         // keys per staged tile: one MFMA sub-block
   constexpr int TILE = BF * D;   // elements of one K or V tile (unpadded, swizzled)
-  // K and V tiles of 32 keys in a three-slot ring filled by asynchronous global -> LDS copies:
+  // K and V tiles of 32 keys in a ring of three slots (two at head_dim 256) filled by asynchronous global -> LDS copies:
   // 48 KiB per workgroup at head_dim 128, so three workgroups share a CU.
-  __shared__ __attribute__((aligned(16))) unsigned short smem[6 * TILE];
-  unsigned short* const Ks = smem;              // three K tiles
-  unsigned short* const Vs = smem + 3 * TILE;   // three V tiles
+  constexpr int RING = D > 128 ? 2 : 3;
+  __shared__ __attribute__((aligned(16))) unsigned short smem[2 * RING * TILE];
+  unsigned short* const Ks = smem;
+  unsigned short* const Vs = smem + RING * TILE;
 
   // Header words and this workgroup's tile are fetched together (the grid never exceeds the
   // allocated list, so the tile read is safe before the count is known): one round trip.
@@ -93,7 +95,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) qf[ks] = load_frag(qrows, qrow, 32 * ks + 16 * h);
 
-  // Three-stage ring of K/V tiles: two tiles are in flight while one is consumed.
+  // RING - 1 tiles are in flight while one is consumed.
   // (a 32 x 32 tile is one instruction each for two waves: the other two request nothing, wait for
   // nothing and meet the copies at the barrier)
   constexpr int CT = D == 32 ? NT / 2 : NT;   // threads that copy tiles
@@ -105,7 +107,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
   if (copier) {
     kcopy.issue(krows, kt_last * BF, Ks);
     if (!TAB) vcopy.issue(vrows, kt_last * BF, Vs);
-    if (kt_last >= 1) {
+    if (RING == 3 && kt_last >= 1) {
       kcopy.issue(krows, (kt_last - 1) * BF, Ks + TILE);
       if (!TAB) vcopy.issue(vrows, (kt_last - 1) * BF, Vs + TILE);
     }
@@ -120,15 +122,17 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
 
   // Offsets (elements) inside a tile.  K: row read of chunk 2*ks + h of LDS row n (= MFMA row n).
   // V: transpose reads of rows 8*u + 4*h + i/4 (+ 16*tt), columns 32*db + 16*blk + 4*(i%4).
+  // (Rows of 512 bytes: the swizzle leaves the upper half of the columns where it is, 256 bytes on.)
   const int i16 = lane & 15, blk = (lane >> 4) & 1;
-  int koff[KS], voff[2][DB];
+  constexpr int KO = KS < 8 ? KS : 8, DO = DB < 4 ? DB : 4;
+  int koff[KO], voff[2][DO];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) koff[ks] = swz_off<D>(n, 2 * ks + h);
+  for (int ks = 0; ks < KO; ++ks) koff[ks] = swz_off<D>(n, 2 * ks + h);
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int r = 8 * u + 4 * h + (i16 >> 2);
 #pragma unroll
-    for (int db = 0; db < DB; ++db) {
+    for (int db = 0; db < DO; ++db) {
       const int col = 32 * db + 16 * blk + 4 * (i16 & 3);
       voff[u][db] = swz_off<D>(r, col >> 3) + (col & 7);
     }
@@ -140,14 +144,14 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
   // register plus an immediate.
   auto tile = [&](auto slot_c, const int kt) {
     constexpr int SLOT = decltype(slot_c)::value;
-    constexpr int REFILL = (SLOT + 2) % 3;   // slot of tile kt + 1, free once every wave is past it
-    // Tile kt has landed when only the loads of tile kt - 1 (issued after it, returning in
+    constexpr int REFILL = (SLOT + RING - 1) % RING;   // slot of tile kt + 1, free once every wave is past it
+    // Tile kt has landed when only the loads of tile kt - 1 (with three slots issued after it, returning in
     // order) can still be in flight; stores in between only make the wait stricter.
-    if (kt >= 1) wait_loads<LOADS_PER_TILE>(); else wait_loads<0>();
+    if (RING == 3 && kt >= 1) wait_loads<LOADS_PER_TILE>(); else wait_loads<0>();
     lds_barrier();
-    if (kt >= 2 && copier) {
-      kcopy.issue(krows, (kt - 2) * BF, Ks + REFILL * TILE);
-      if (!TAB) vcopy.issue(vrows, (kt - 2) * BF, Vs + REFILL * TILE);
+    if (kt >= RING - 1 && copier) {
+      kcopy.issue(krows, (kt - RING + 1) * BF, Ks + REFILL * TILE);
+      if (!TAB) vcopy.issue(vrows, (kt - RING + 1) * BF, Vs + REFILL * TILE);
     }
     const unsigned short* Kt = Ks + SLOT * TILE;
     const unsigned short* Vt = Vs + SLOT * TILE;
@@ -161,7 +165,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
     {
       el8 kfr[KS];
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) kfr[ks] = lds_row8(Kt + koff[ks]);
+      for (int ks = 0; ks < KS; ++ks) kfr[ks] = lds_row8(Kt + koff[ks % KO] + 128 * (ks / KO));
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) x = mfma32(kfr[ks], qf[ks], x);
     }
@@ -193,7 +197,8 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
     for (int tt = 0; tt < 2; ++tt) {
       const unsigned short* vrow = Vt + 16 * tt * D;
 #pragma unroll
-      for (int db = 0; db < DB; ++db) vfr[tt][db] = lds_tr8(vrow + voff[0][db], vrow + voff[1][db]);
+      for (int db = 0; db < DB; ++db)
+        vfr[tt][db] = lds_tr8(vrow + voff[0][db % DO] + 128 * (db / DO), vrow + voff[1][db % DO] + 128 * (db / DO));
     }
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt) {
@@ -212,8 +217,10 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 3) fwd_kernel(const KArgs a)
     if (--kt < 0) break;
     tile(std::integral_constant<int, 1>{}, kt);
     if (--kt < 0) break;
-    tile(std::integral_constant<int, 2>{}, kt);
-    if (--kt < 0) break;
+    if constexpr (RING == 3) {
+      tile(std::integral_constant<int, 2>{}, kt);
+      if (--kt < 0) break;
+    }
   }
 
   // epilogue: rem = what is left of the stick; o rows in the accumulator layout
