@@ -15,11 +15,8 @@
 //                    the stick carry (table written by the forward) and the G prefix (table
 //                    written by bwd_dq_kernel) of each sub-block, recomputes p and dz and
 //                    accumulates dk and dv in registers; every output element is written once.
-//                    (bwd_dkdv_tail_kernel: the same for the key tiles that few queries follow.)
-//
-// Per-score math (upstream sb_varlen_bwd.py:439-453):
-//   G = A * (do.v - drem),  C = inclusive running sum of G over keys,  dz = G - beta * C,
-//   dq = s * dz K,  dk = s * dz^T Q,  dv = A^T do.
+//                    (bwd_dkdv_tail_kernel: the same for the key tiles that few queries follow;
+//                    sba_wide.hip: the same for head_dim 129 .. 256.)
 #include <algorithm>
 #include <type_traits>
 
@@ -27,78 +24,6 @@
 
 namespace sba {
 inline namespace SBA_ELEM_NS {
-
-// One 32-key sub-block for the 32 queries of a wave, in two phases so that the do.v^T
-// accumulators need not be live while the weights are formed:
-//   grad_weights  p and r = 1 - beta from the raw scores and the stick carry at the sub-block's newer edge
-//   grad_dz       dz = G - beta C with G = p (do.v - drem) and the running prefix C of G
-//                 (carry_c: in = prefix before the sub-block, out = after it)
-// p and dz leave as bf16 A-operand fragments: slot s of fragment [tt] is key 16*h + 8*tt + s.
-template <bool AC, bool PROD>
-__device__ __forceinline__ void grad_weights(const f32x16& x, float c, int k0, int qw0, int qrow, int h,
-                                             float carry_e, float (&p)[16], float (&bt)[16], float (&ends)[2]) {
-  if (sub_full<AC>(k0, qw0)) {
-    stick_weights<AC, PROD, false, true>(x, c, k0, qrow, h, carry_e, p, bt, ends);
-  } else {
-    stick_weights<AC, PROD, true, true>(x, c, k0, qrow, h, carry_e, p, bt, ends);
-  }
-}
-
-// With G = p (do.v - drem), C the inclusive running sum of G along the keys and r = 1 - beta:
-//   dz = G - beta C = r C - (C - G) = r * C[i] - C[i-1],
-// so neither G nor beta is formed: the running sum is an fma chain and dz one more fma.  A
-// masked key has p = 0 and r = 1, which gives dz = 0 exactly.
-//
-// In product space the subtraction of drem disappears as well.  With ex[i] the stick left on
-// entering key i (so that p[i] = ex[i] - ex[i-1] and r[i] * ex[i] = ex[i-1]) define
-// D[i] = C[i] + drem * ex[i].  Then
-//   D[i] - D[i-1] = p[i] (do.v - drem) + drem p[i] = p[i] do.v          (one fma, no subtraction)
-//   r[i] D[i] - D[i-1] = r[i] C[i] - C[i-1] + drem (r[i] ex[i] - ex[i-1]) = dz[i],
-// so the chain runs on do.v directly and starts from C + drem * (stick after the lane's oldest
-// key); the lane's total of G is sum(p do.v) - drem * sum(p) with sum(p) = ends[0] - ends[1].
-template <bool PROD>
-__device__ __forceinline__ void grad_dz(const float (&p)[16], const float (&r)[16], const f32x16& da,
-                                        const float (&ends)[2], int h, float& carry_c, float dr,
-                                        el8 (&zf)[2]) {
-  float dz[16];
-  if constexpr (PROD) {
-    float t0 = 0.0f, t1 = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; i += 2) { t0 = fmaf(p[i], da[i], t0); t1 = fmaf(p[i + 1], da[i + 1], t1); }
-    const float total = fmaf(-dr, ends[0] - ends[1], t0 + t1);   // this lane's sum of G
-    float lo, hi;
-    both_halves(total, lo, hi);
-    const float cstart = h == 1 ? carry_c + lo : carry_c;        // keys of the h=0 lane come first
-    float dprev = fmaf(dr, ends[1], cstart);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float d = fmaf(p[i], da[i], dprev);
-      dz[i] = fmaf(r[i], d, -dprev);
-      dprev = d;
-    }
-    carry_c += lo + hi;
-  } else {
-    float dA[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) dA[i] = da[i] - dr;
-    // this lane's total of G (two partial chains), then both half-waves' totals
-    float t0 = 0.0f, t1 = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; i += 2) { t0 = fmaf(p[i], dA[i], t0); t1 = fmaf(p[i + 1], dA[i + 1], t1); }
-    float lo, hi;
-    both_halves(t0 + t1, lo, hi);
-    float cprev = h == 1 ? carry_c + lo : carry_c;   // keys of the h=0 lane come first
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float c = fmaf(p[i], dA[i], cprev);
-      dz[i] = fmaf(r[i], c, -cprev);
-      cprev = c;
-    }
-    carry_c += lo + hi;
-  }
-  zf[0] = pack8(dz);
-  zf[1] = pack8(dz + 8);
-}
 
 // -------------------------------------------------------------------------------------------
 // dq pass
@@ -984,24 +909,11 @@ __global__ void __launch_bounds__(NT2, 1) bwd_dkdv_kernel(const KArgs a) {
 // w, recomputes p and dz of the query blocks at or after it exactly as a score wave does, turns
 // its own 32x32 blocks around through a private piece of LDS and accumulates its own rows of dk
 // and dv.  One barrier (after the Q / dO rows have landed), two workgroups per CU.
-//
-// STREAM: the same four independent waves on EVERY key tile, whatever number of queries follows
-// it: the Q / dO rows then come 64 at a time through two LDS buffers, with one barrier per 64
-// rows (one per 32 rows costs a quarter more time: the waves wait for one another at each).
-// This is the whole dk/dv pass of head_dim 256, where a wave's K and V fragments (128 registers)
-// and the accumulators of ONE of dk and dv (128) with the chains' own temporaries need the
-// register file of a SIMD to themselves: one workgroup per CU, one wave per SIMD, nothing to
-// split into roles, and two passes over the queries, dv first and dk second (both outputs'
-// accumulators at once leave the chains no accumulation registers: 150 to 210 spilled values,
-// whether or not the V fragments wait in LDS instead).
 // -------------------------------------------------------------------------------------------
-template <int D> struct StreamKernel { static constexpr bool value = D > 128; };
-
-template <int D, bool AC, bool PROD, bool STREAM, int U = D>
-__global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(const KArgs a) {
-  constexpr int KS = U / 16, DB = U / 32;
-  constexpr int SEG = 64;                             // STREAM: query rows per buffer
-  constexpr int QROWS = STREAM ? 2 * SEG : TAIL_TILES * BKV;   // rows the buffers hold (not STREAM: every query that can follow the tile's first key)
+template <int D, bool AC, bool PROD>
+__global__ void __launch_bounds__(NT, 2) bwd_dkdv_tail_kernel(const KArgs a) {
+  constexpr int KS = D / 16, DB = D / 32;
+  constexpr int QROWS = TAIL_TILES * BKV;   // rows the buffers hold: every query that can follow the tile's first key
   __shared__ __attribute__((aligned(16))) unsigned short Qs[QROWS * D];   // Q rows from the tile's first key on (swizzled like every tile)
   __shared__ __attribute__((aligned(16))) unsigned short Gs[QROWS * D];   // dO rows
   __shared__ __attribute__((aligned(16))) unsigned short St[NT / 64][2][32 * 32];   // per wave: p and dz of one block, [query][key]
@@ -1012,7 +924,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
   if (hdr.x != 0 || hdr.w > a.tab_stride || hdr2.x > a.max_doc_len) return;
   const int which = blockIdx.x / a.heads;
   const int head = blockIdx.x - which * a.heads;
-  const int slot = STREAM ? which : hdr2.y + which;   // STREAM: both groups of the list
+  const int slot = hdr2.y + which;
   if (slot >= hdr.z) return;
   const Tile t = reinterpret_cast<const Tile*>(sched + a.kv_list_off)[slot];
   const int kt = t.idx;
@@ -1034,17 +946,16 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
   const Rows vrows = make_rows(vb, a.v.st, L, a.head_dim);
 
   const int q_first = kt * BKV;                      // first query that can see the tile
-  const int nblk = (L - q_first + 31) / 32;          // query blocks behind the tile's first key (not STREAM: 1 .. QROWS / 32)
-  // The first of those Q and dO rows (rows past the document arrive as zeros).  Not STREAM: as many as there are keys, and
+  const int nblk = (L - q_first + 31) / 32;          // query blocks behind the tile's first key: 1 .. QROWS / 32
+  // The first of those Q and dO rows (rows past the document arrive as zeros), as many as there are keys, and
   // into the place of the others first this tile's K and V rows, which every wave takes its fragments from.
-  constexpr int FIRST = STREAM ? SEG : BKV;
-  static_assert(STREAM || QROWS == 2 * BKV, "the second half of the query buffers holds the key tile first");
-  TileCopy<D, FIRST, NT, false> qcopy, gcopy;
+  static_assert(QROWS == 2 * BKV, "the second half of the query buffers holds the key tile first");
+  TileCopy<D, BKV, NT, false> qcopy, gcopy;
   qcopy.init(tid, qrows.row_bytes, qrows.used_bytes);
   gcopy.init(tid, grows.row_bytes, grows.used_bytes);
-  qcopy.issue(qrows, q_first, Qs, STREAM ? SEG : 32 * nblk);      // (32 or 64 rows per instruction of all waves: whole query blocks)
-  gcopy.issue(grows, q_first, Gs, STREAM ? SEG : 32 * nblk);
-  if constexpr (!STREAM) {
+  qcopy.issue(qrows, q_first, Qs, 32 * nblk);      // (32 or 64 rows per instruction of all waves: whole query blocks)
+  gcopy.issue(grows, q_first, Gs, 32 * nblk);
+  {
     // (through LDS: a fragment load straight from memory is 32 rows of 32 bytes, which keeps the CU's address unit busy; 16 K
     // tokens in documents of 16 to 256, 32 heads, head_dim 64: forward + backward 281 -> 276 us.  A kernel small enough
     // for three workgroups per CU was no faster, 287: what is left is the traffic, 4 TB/s.)
@@ -1060,13 +971,6 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
   const int k0 = q_first + 32 * kblk;                // this wave's keys
   const bool active = k0 < L;
   el8 kf[KS], vf[KS];                                // MFMA row n holds key k0 + kperm(n)
-  if constexpr (STREAM) {
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      kf[ks] = load_frag(krows, k0 + kperm(n), 32 * ks + 16 * h);
-      vf[ks] = load_frag(vrows, k0 + kperm(n), 32 * ks + 16 * h);
-    }
-  }
   // A block that starts past the end of the document is never visible; its table reads are
   // redirected into the document's area and never used.
   const int tblock = min((BKV / 32) * kt + kblk, (L - 1) / 32);
@@ -1104,29 +1008,28 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
       yoff[u][j] = swz_off<D>(r, yc >> 3) + (yc & 7);
     }
   }
-  if constexpr (!STREAM) {
-    wait_loads<0>();
-    lds_barrier();            // every wave's part of the rows has landed
-    if (!active) return;      // (a document that ends ahead of this wave's keys has no second half of queries: no barrier follows)
+  wait_loads<0>();
+  lds_barrier();            // every wave's part of the rows has landed
+  if (!active) return;      // (a document that ends ahead of this wave's keys has no second half of queries: no barrier follows)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      kf[ks] = lds_row8(Qs + BKV * D + 32 * kblk * D + roff[ks]);
-      vf[ks] = lds_row8(Gs + BKV * D + 32 * kblk * D + roff[ks]);
-    }
-    if (nblk > BKV / 32) {
-      lds_barrier();          // every wave has its keys in registers
-      qcopy.issue(qrows, q_first + BKV, Qs + BKV * D, 32 * nblk - BKV);
-      gcopy.issue(grows, q_first + BKV, Gs + BKV * D, 32 * nblk - BKV);
-    }
+  for (int ks = 0; ks < KS; ++ks) {
+    kf[ks] = lds_row8(Qs + BKV * D + 32 * kblk * D + roff[ks]);
+    vf[ks] = lds_row8(Gs + BKV * D + 32 * kblk * D + roff[ks]);
+  }
+  if (nblk > BKV / 32) {
+    lds_barrier();          // every wave has its keys in registers
+    qcopy.issue(qrows, q_first + BKV, Qs + BKV * D, 32 * nblk - BKV);
+    gcopy.issue(grows, q_first + BKV, Gs + BKV * D, 32 * nblk - BKV);
   }
 
   unsigned short* Pt = St[w][0];
   unsigned short* Zt = St[w][1];
-  // Query block qblk, whose Q / dO rows begin at buffer row lrow0.  WHAT: 0 = p alone and its
-  // products into `acc` (dv), 1 = dz alone and its products into `acc` (dk), 2 = both, dk into `acc2`.
-  auto block = [&](auto what_tag, f32x16 (&acc)[DB], f32x16 (&acc2)[DB], const int qblk, const int lrow0) {
-    constexpr int WHAT = decltype(what_tag)::value;
-    constexpr bool DV = WHAT != 1, DK = WHAT != 0;
+  f32x16 acc_v[DB], acc_k[DB];
+#pragma unroll
+  for (int j = 0; j < DB; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc_v[j][i] = acc_k[j][i] = 0.0f;
+  auto block = [&](const int qblk) {
     request(qblk + 1, nxt);                           // (clamped; unused past the last block)
     const int qw0 = q_first + 32 * qblk;
     const int qrow = qw0 + n;
@@ -1138,129 +1041,71 @@ __global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dkdv_tail_kernel(cons
 #pragma unroll
     for (int j = 0; j < 16; ++j) { x[j] = 0.0f; da[j] = 0.0f; }
     {
-      const unsigned short* Qt = Qs + lrow0 * D;
-      const unsigned short* Gt = Gs + lrow0 * D;
-      // (head_dim 256: four contraction steps at a time, so that the operand fragments of a whole
-      // chain are never in registers at once)
-      constexpr int CH = D > 128 ? 4 : KS;
+      const unsigned short* Qt = Qs + 32 * qblk * D;
+      const unsigned short* Gt = Gs + 32 * qblk * D;
+      el8 qfr[KS], gfr[KS];
 #pragma unroll
-      for (int c0 = 0; c0 < KS; c0 += CH) {
-        el8 qfr[CH], gfr[CH];
+      for (int ks = 0; ks < KS; ++ks) {
+        qfr[ks] = lds_row8(Qt + roff[ks]);
+        gfr[ks] = lds_row8(Gt + roff[ks]);
+      }
 #pragma unroll
-        for (int ks = 0; ks < CH; ++ks) {
-          qfr[ks] = lds_row8(Qt + roff[c0 + ks]);
-          if constexpr (DK) gfr[ks] = lds_row8(Gt + roff[c0 + ks]);
-        }
-#pragma unroll
-        for (int ks = 0; ks < CH; ++ks) {
-          x = mfma32(kf[c0 + ks], qfr[ks], x);
-          if constexpr (DK) da = mfma32(vf[c0 + ks], gfr[ks], da);
-        }
-        if constexpr (D > 128) __builtin_amdgcn_sched_barrier(0);
+      for (int ks = 0; ks < KS; ++ks) {
+        x = mfma32(kf[ks], qfr[ks], x);
+        da = mfma32(vf[ks], gfr[ks], da);
       }
     }
     el8 pf[2], zf[2];
     {
       float p[16], bt[16], ends[2] = {0.0f, 0.0f};
       grad_weights<AC, PROD>(x, a.c, k0, qw0, qrow, h, carry_e, p, bt, ends);
-      if constexpr (DV) {
-        if (a.fuse && qblk == kblk) {
-          float pd[16];
+      if (a.fuse && qblk == kblk) {
+        float pd[16];
 #pragma unroll
-          for (int j = 0; j < 16; ++j) pd[j] = p[j] + (16 * h + j == n ? rem_own : 0.0f);
-          pf[0] = pack8(pd);
-          pf[1] = pack8(pd + 8);
-        } else {
-          pf[0] = pack8(p);
-          pf[1] = pack8(p + 8);
-        }
+        for (int j = 0; j < 16; ++j) pd[j] = p[j] + (16 * h + j == n ? rem_own : 0.0f);
+        pf[0] = pack8(pd);
+        pf[1] = pack8(pd + 8);
+      } else {
+        pf[0] = pack8(p);
+        pf[1] = pack8(p + 8);
       }
-      if constexpr (DK) grad_dz<PROD>(p, bt, da, ends, h, carry_c, dr, zf);
+      grad_dz<PROD>(p, bt, da, ends, h, carry_c, dr, zf);
     }
     // turn the block around: [query][key] rows in, key-major MFMA operands out
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt) {
-      if constexpr (DV) *reinterpret_cast<el8*>(Pt + blk_off(n, 2 * h + tt)) = pf[tt];
-      if constexpr (DK) *reinterpret_cast<el8*>(Zt + blk_off(n, 2 * h + tt)) = zf[tt];
+      *reinterpret_cast<el8*>(Pt + blk_off(n, 2 * h + tt)) = pf[tt];
+      *reinterpret_cast<el8*>(Zt + blk_off(n, 2 * h + tt)) = zf[tt];
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's own writes have landed
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      el8 ap, az;
-      if constexpr (DV) ap = lds_tr8(Pt + xoff[0] + 16 * ks * 32, Pt + xoff[1] + 16 * ks * 32);
-      if constexpr (DK) az = lds_tr8(Zt + xoff[0] + 16 * ks * 32, Zt + xoff[1] + 16 * ks * 32);
-      const unsigned short* Gr = Gs + (lrow0 + 16 * ks) * D;
-      const unsigned short* Qr = Qs + (lrow0 + 16 * ks) * D;
+      const el8 ap = lds_tr8(Pt + xoff[0] + 16 * ks * 32, Pt + xoff[1] + 16 * ks * 32);
+      const el8 az = lds_tr8(Zt + xoff[0] + 16 * ks * 32, Zt + xoff[1] + 16 * ks * 32);
+      const unsigned short* Gr = Gs + (32 * qblk + 16 * ks) * D;
+      const unsigned short* Qr = Qs + (32 * qblk + 16 * ks) * D;
 #pragma unroll
       for (int j = 0; j < DB; ++j) {
-        if constexpr (DV) acc[j] = mfma32(lds_tr8(Gr + yoff[0][j], Gr + yoff[1][j]), ap, acc[j]);
-        if constexpr (WHAT == 1) acc[j] = mfma32(lds_tr8(Qr + yoff[0][j], Qr + yoff[1][j]), az, acc[j]);
-        if constexpr (WHAT == 2) acc2[j] = mfma32(lds_tr8(Qr + yoff[0][j], Qr + yoff[1][j]), az, acc2[j]);
-        if constexpr (D > 128) { if (j % 4 == 3 || j == DB - 1) __builtin_amdgcn_sched_barrier(0); }
+        acc_v[j] = mfma32(lds_tr8(Gr + yoff[0][j], Gr + yoff[1][j]), ap, acc_v[j]);
+        acc_k[j] = mfma32(lds_tr8(Qr + yoff[0][j], Qr + yoff[1][j]), az, acc_k[j]);
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads are done before the next block overwrites the piece
     cur = nxt;
   };
-  auto clear = [&](f32x16 (&acc)[DB]) {
-#pragma unroll
-    for (int j = 0; j < DB; ++j)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[j][i] = 0.0f;
-  };
+  // query blocks at or after the key block (those before it see none of these keys)
+#pragma unroll 1
+  for (int qblk = kblk; qblk < nblk; ++qblk) {
+    if (qblk == BKV / 32) {
+      wait_loads<0>();
+      lds_barrier();        // the second half has landed (every wave of a tile that has one comes here)
+    }
+    block(qblk);
+  }
   elem_t* dvb = reinterpret_cast<elem_t*>(a.dv.ptr) + t.batch * a.dv.sb + head * a.dv.sh + tok0 * a.dv.st;
   elem_t* dkb = reinterpret_cast<elem_t*>(a.dk.ptr) + t.batch * a.dk.sb + head * a.dk.sh + tok0 * a.dk.st;
-  const Rows dvrows = make_rows(dvb, a.dv.st, L, a.head_dim), dkrows = make_rows(dkb, a.dk.st, L, a.head_dim);
-  if constexpr (!STREAM) {
-    f32x16 acc_v[DB], acc_k[DB];
-    clear(acc_v);
-    clear(acc_k);
-    // query blocks at or after the key block (those before it see none of these keys)
-#pragma unroll 1
-    for (int qblk = kblk; qblk < nblk; ++qblk) {
-      if (qblk == BKV / 32) {
-        wait_loads<0>();
-        lds_barrier();        // the second half has landed (every wave of a tile that has one comes here)
-      }
-      block(std::integral_constant<int, 2>{}, acc_v, acc_k, qblk, 32 * qblk);
-    }
-    store_rows(acc_v, 1.0f, dvrows, k0 + n, L, h, a.out_f32);
-    store_rows(acc_k, a.inv_temp, dkrows, k0 + n, L, h, a.out_f32);
-  } else {
-    // Two passes over the queries, dv first and dk second; the scores are formed in each.
-    // Segment s (SEG query rows) sits in buffer s & 1.  At its top every wave is done with segment s - 1,
-    // whose buffer takes the rows of segment s + 1 while this one is worked on.
-    constexpr int BPS = SEG / 32;                     // query blocks per segment
-    const int nseg = (nblk + BPS - 1) / BPS;
-    auto pass = [&](auto what_tag) {
-      f32x16 acc[DB];
-      clear(acc);
-#pragma unroll 1
-      for (int sgm = 0; sgm < nseg; ++sgm) {
-        wait_loads<0>();
-        lds_barrier();
-        if (sgm + 1 < nseg) {
-          qcopy.issue(qrows, q_first + (sgm + 1) * SEG, Qs + ((sgm + 1) & 1) * SEG * D);
-          gcopy.issue(grows, q_first + (sgm + 1) * SEG, Gs + ((sgm + 1) & 1) * SEG * D);
-        }
-#pragma unroll
-        for (int b = 0; b < BPS; ++b) {
-          const int qblk = BPS * sgm + b;
-          if (active && qblk >= kblk && qblk < nblk) block(what_tag, acc, acc, qblk, (sgm & 1) * SEG + 32 * b);
-        }
-      }
-      if (active) {
-        if constexpr (decltype(what_tag)::value == 0) store_rows(acc, 1.0f, dvrows, k0 + n, L, h, a.out_f32);
-        else store_rows(acc, a.inv_temp, dkrows, k0 + n, L, h, a.out_f32);
-      }
-    };
-    pass(std::integral_constant<int, 0>{});
-    lds_barrier();              // every wave is done with the buffers: the first block's rows once more
-    qcopy.issue(qrows, q_first, Qs, SEG);
-    gcopy.issue(grows, q_first, Gs, SEG);
-    request(kblk, cur);
-    pass(std::integral_constant<int, 1>{});
-  }
+  store_rows(acc_v, 1.0f, make_rows(dvb, a.dv.st, L, a.head_dim), k0 + n, L, h, a.out_f32);
+  store_rows(acc_k, a.inv_temp, make_rows(dkb, a.dk.st, L, a.head_dim), k0 + n, L, h, a.out_f32);
 }
 
 // Explicit instantiations: every (head_dim, attend_current, carry space) variant the launchers use.
@@ -1280,18 +1125,14 @@ template __global__ void bwd_dq_kernel<256, false, false>(const KArgs);
 template __global__ void bwd_dq_kernel<256, false, true>(const KArgs);
 template __global__ void bwd_dq_kernel<256, true, false>(const KArgs);
 template __global__ void bwd_dq_kernel<256, true, true>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<256, false, false, true>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<256, false, true, true>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<256, true, false, true>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<256, true, true, true>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<32, false, false, false>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<32, false, true, false>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<32, true, false, false>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<32, true, true, false>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<64, false, false, false>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<64, false, true, false>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<64, true, false, false>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<64, true, true, false>(const KArgs);
+template __global__ void bwd_dkdv_tail_kernel<32, false, false>(const KArgs);
+template __global__ void bwd_dkdv_tail_kernel<32, false, true>(const KArgs);
+template __global__ void bwd_dkdv_tail_kernel<32, true, false>(const KArgs);
+template __global__ void bwd_dkdv_tail_kernel<32, true, true>(const KArgs);
+template __global__ void bwd_dkdv_tail_kernel<64, false, false>(const KArgs);
+template __global__ void bwd_dkdv_tail_kernel<64, false, true>(const KArgs);
+template __global__ void bwd_dkdv_tail_kernel<64, true, false>(const KArgs);
+template __global__ void bwd_dkdv_tail_kernel<64, true, true>(const KArgs);
 template __global__ void bwd_dkdv_kernel<32, false, false>(const KArgs);
 template __global__ void bwd_dkdv_kernel<32, false, true>(const KArgs);
 template __global__ void bwd_dkdv_kernel<32, true, false>(const KArgs);
@@ -1311,8 +1152,6 @@ template __global__ void bwd_dq_kernel<256, false, true, 192>(const KArgs);
 template __global__ void bwd_dq_kernel<256, true, true, 192>(const KArgs);
 template __global__ void bwd_dkdv_kernel<128, false, true, 96>(const KArgs);
 template __global__ void bwd_dkdv_kernel<128, true, true, 96>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<256, false, true, true, 192>(const KArgs);
-template __global__ void bwd_dkdv_tail_kernel<256, true, true, true, 192>(const KArgs);
 
 // Width of the narrower instantiation a kernel width has (see used_width), or the width itself.
 template <int D> constexpr int narrow_width() { return D == 128 ? 96 : D == 256 ? 192 : D; }
@@ -1336,20 +1175,15 @@ static hipError_t launch_dq_d(const KArgs& a, bool ac, bool prod, int n_q_max, h
   return hipGetLastError();
 }
 
-// n_long_max / n_last_max: upper bounds on the key tiles of the first / second group of the list.
-template <int D, bool STREAM>
-static void launch_dkdv_four_waves(const KArgs& a, bool ac, bool prod, unsigned tiles, hipStream_t s) {
+template <int D>
+static void launch_dkdv_tail(const KArgs& a, bool ac, bool prod, unsigned tiles, hipStream_t s) {
   const dim3 grid(tiles * (unsigned)a.heads), block(NT);
-  constexpr int W = STREAM ? narrow_width<D>() : D;
-  if (W < D && prod && used_width(a.head_dim) == W) {
-    if (ac) hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, true, true, STREAM, W>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, false, true, STREAM, W>), grid, block, 0, s, a);
-  } else if (ac) {
-    if (prod) hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, true, true, STREAM>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, true, false, STREAM>), grid, block, 0, s, a);
+  if (ac) {
+    if (prod) hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, true, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, true, false>), grid, block, 0, s, a);
   } else {
-    if (prod) hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, false, true, STREAM>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, false, false, STREAM>), grid, block, 0, s, a);
+    if (prod) hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, false, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((bwd_dkdv_tail_kernel<D, false, false>), grid, block, 0, s, a);
   }
 }
 
@@ -1360,9 +1194,9 @@ static hipError_t launch_dkdv_d(const KArgs& a_in, bool ac, bool prod, int n_lon
   KArgs a = a_in;
   const DkdvGrid g = dkdv_grid(TailKernel<D>::value, n_long_max, n_last_max, a.n_kv_alloc);
   const unsigned n_main = (unsigned)g.main_tiles;
-  if constexpr (StreamKernel<D>::value) {
-    // every key tile of both groups to the four independent waves, queries streamed
-    if (n_main > 0) launch_dkdv_four_waves<D, true>(a, ac, prod, n_main, s);
+  if constexpr (D > 128) {
+    // every key tile of both groups
+    return n_main > 0 ? launch_bwd_dkdv_wide(a, ac, prod, (int)n_main, s) : hipSuccess;
   } else {
     if (n_main > 0) {
       a.n_items = (int)(n_main * (unsigned)a.heads);
@@ -1380,7 +1214,7 @@ static hipError_t launch_dkdv_d(const KArgs& a_in, bool ac, bool prod, int n_lon
       }
     }
     if constexpr (TailKernel<D>::value) {
-      if (g.tail_tiles > 0) launch_dkdv_four_waves<D, false>(a, ac, prod, (unsigned)g.tail_tiles, s);
+      if (g.tail_tiles > 0) launch_dkdv_tail<D>(a, ac, prod, (unsigned)g.tail_tiles, s);
     }
   }
   return hipGetLastError();

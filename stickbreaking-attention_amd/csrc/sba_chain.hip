@@ -42,9 +42,6 @@
 namespace sba {
 inline namespace SBA_ELEM_NS {
 
-// Rows of one 32-row fp32 block of partial dq: four dwordx4 per lane.
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
 __device__ __forceinline__ int this_xcd() { return __builtin_amdgcn_s_getreg(20 | (3 << 11)) & (CHAIN_QUEUES - 1); }   // HW_REG_XCC_ID, bits 3:0
 
 // Ahead of the main kernel: clears the flags and the queues, notes which XCDs its workgroups run on (the main kernel's

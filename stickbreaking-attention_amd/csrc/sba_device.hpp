@@ -24,6 +24,7 @@
 namespace sba {
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(4))) short s16x4;
 typedef __attribute__((ext_vector_type(8))) short s16x8;
@@ -430,6 +431,85 @@ __device__ __forceinline__ bool sub_skip(int k0, int qw0) {
 template <bool AC>
 __device__ __forceinline__ bool sub_full(int k0, int qw0) {
   return AC ? (k0 + 31 <= qw0) : (k0 + 31 < qw0);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Backward.
+//
+// Per-score math (upstream sb_varlen_bwd.py:439-453):
+//   G = A * (do.v - drem),  C = inclusive running sum of G over keys,  dz = G - beta * C,
+//   dq = s * dz K,  dk = s * dz^T Q,  dv = A^T do.
+//
+// One 32-key sub-block for the 32 queries of a wave, in two phases so that the do.v^T
+// accumulators need not be live while the weights are formed:
+//   grad_weights  p and r = 1 - beta from the raw scores and the stick carry at the sub-block's newer edge
+//   grad_dz       dz = G - beta C with G = p (do.v - drem) and the running prefix C of G
+//                 (carry_c: in = prefix before the sub-block, out = after it)
+// p and dz leave as bf16 A-operand fragments: slot s of fragment [tt] is key 16*h + 8*tt + s.
+template <bool AC, bool PROD>
+__device__ __forceinline__ void grad_weights(const f32x16& x, float c, int k0, int qw0, int qrow, int h,
+                                             float carry_e, float (&p)[16], float (&bt)[16], float (&ends)[2]) {
+  if (sub_full<AC>(k0, qw0)) {
+    stick_weights<AC, PROD, false, true>(x, c, k0, qrow, h, carry_e, p, bt, ends);
+  } else {
+    stick_weights<AC, PROD, true, true>(x, c, k0, qrow, h, carry_e, p, bt, ends);
+  }
+}
+
+// With G = p (do.v - drem), C the inclusive running sum of G along the keys and r = 1 - beta:
+//   dz = G - beta C = r C - (C - G) = r * C[i] - C[i-1],
+// so neither G nor beta is formed: the running sum is an fma chain and dz one more fma.  A
+// masked key has p = 0 and r = 1, which gives dz = 0 exactly.
+//
+// In product space the subtraction of drem disappears as well.  With ex[i] the stick left on
+// entering key i (so that p[i] = ex[i] - ex[i-1] and r[i] * ex[i] = ex[i-1]) define
+// D[i] = C[i] + drem * ex[i].  Then
+//   D[i] - D[i-1] = p[i] (do.v - drem) + drem p[i] = p[i] do.v          (one fma, no subtraction)
+//   r[i] D[i] - D[i-1] = r[i] C[i] - C[i-1] + drem (r[i] ex[i] - ex[i-1]) = dz[i],
+// so the chain runs on do.v directly and starts from C + drem * (stick after the lane's oldest
+// key); the lane's total of G is sum(p do.v) - drem * sum(p) with sum(p) = ends[0] - ends[1].
+template <bool PROD>
+__device__ __forceinline__ void grad_dz(const float (&p)[16], const float (&r)[16], const f32x16& da,
+                                        const float (&ends)[2], int h, float& carry_c, float dr,
+                                        el8 (&zf)[2]) {
+  float dz[16];
+  if constexpr (PROD) {
+    float t0 = 0.0f, t1 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i += 2) { t0 = fmaf(p[i], da[i], t0); t1 = fmaf(p[i + 1], da[i + 1], t1); }
+    const float total = fmaf(-dr, ends[0] - ends[1], t0 + t1);   // this lane's sum of G
+    float lo, hi;
+    both_halves(total, lo, hi);
+    const float cstart = h == 1 ? carry_c + lo : carry_c;        // keys of the h=0 lane come first
+    float dprev = fmaf(dr, ends[1], cstart);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float d = fmaf(p[i], da[i], dprev);
+      dz[i] = fmaf(r[i], d, -dprev);
+      dprev = d;
+    }
+    carry_c += lo + hi;
+  } else {
+    float dA[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) dA[i] = da[i] - dr;
+    // this lane's total of G (two partial chains), then both half-waves' totals
+    float t0 = 0.0f, t1 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i += 2) { t0 = fmaf(p[i], dA[i], t0); t1 = fmaf(p[i + 1], dA[i + 1], t1); }
+    float lo, hi;
+    both_halves(t0 + t1, lo, hi);
+    float cprev = h == 1 ? carry_c + lo : carry_c;   // keys of the h=0 lane come first
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float c = fmaf(p[i], dA[i], cprev);
+      dz[i] = fmaf(r[i], c, -cprev);
+      cprev = c;
+    }
+    carry_c += lo + hi;
+  }
+  zf[0] = pack8(dz);
+  zf[1] = pack8(dz + 8);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -1,0 +1,383 @@
+// dk / dv pass of head_dim 129 .. 256 (see sba_bwd.hip for the two-pass backward and its other kernels).
+//
+// At twice the width of the eight-wave kernel of sba_bwd.hip a wave's K and V fragments are 128 registers and the accumulators of 64
+// keys of one output 256: neither role fits two waves per SIMD.  So the work is cut smaller.  A workgroup owns 64 keys of
+// one (document, head) and walks the queries that can see them, 32 per step:
+//
+//   waves 0, 1   "weights", one 32-key block each, K fragments in registers: scores, p, dz
+//   waves 2, 3   "do.v" of the same blocks, V fragments in registers; handed to the weights wave through LDS in fp32
+//   waves 4 .. 7 "products": dv = p^T dO and dk = dz^T Q, 64 keys x half of the columns of one output each (128 registers);
+//                they also copy the Q / dO tiles
+//
+// A step has two phases with a barrier behind each.  In the first the weights waves have vector work only (p of block i) and
+// the product waves, which share SIMDs 0 and 1 with them, multiply block i - 1; in the second the weights waves form the
+// scores of block i + 1 between the vector instructions of dz, the do.v waves theirs, and the product waves read the Q / dO
+// fragments of block i.  A tile is requested two steps before it is read (four slots of 32 KiB).
+//
+// Bound by the vector work of the two weights waves, alone with it on their SIMDs (of 2400 cycles of a step, stamped, they wait 350,
+// the product waves 650, the do.v waves 1300), and by what a work item costs beside its steps (8000 cycles, 45 steps on average);
+// the matrix pipes are busy for a third of the time.  16 heads x 16 K tokens in eight documents, head_dim 256: 1525 -> 890 us against
+// four independent waves of 32 keys each, which formed the scores twice, once for dv and once for dk, because both outputs'
+// accumulators (256 registers) left the chains nowhere to go.  Tried: a quarter or half of a block's products in the second phase (942,
+// 970 for 922), the next tile requested ahead of the products (950).
+#include <type_traits>
+
+#include "sba_kernels.hpp"
+
+namespace sba {
+inline namespace SBA_ELEM_NS {
+
+constexpr int WIDE_KEYS = 64;     // keys of a workgroup: half a tile of the key-tile list
+
+template <bool AC, bool PROD, int U>
+__global__ void __launch_bounds__(512, 1) bwd_dkdv_wide_kernel(const KArgs a) {
+  constexpr int D = 256, KS = U / 16, DBH = U / 64;     // U: columns multiplied; DBH: 32-wide column blocks of a product wave
+  constexpr int TQ = 32, SLOTS = 4, QTILE = TQ * D, PTILE = TQ * WIDE_KEYS;
+  __shared__ __attribute__((aligned(16))) unsigned short Qs[SLOTS * QTILE];
+  __shared__ __attribute__((aligned(16))) unsigned short Gs[SLOTS * QTILE];
+  __shared__ __attribute__((aligned(16))) unsigned short Ps[2 * PTILE];   // p and dz, [query][key]
+  __shared__ __attribute__((aligned(16))) unsigned short Zs[2 * PTILE];
+  __shared__ __attribute__((aligned(16))) float hand[WIDE_KEYS / 32][16 * 64];   // do.v of a block as the accumulators lie, a quad of every lane at a time
+
+  // (the grid never exceeds the room of the list: its tile is read along with the header)
+  const int* sched = a.sched;
+  const int which = blockIdx.x / a.heads;
+  const int head = blockIdx.x - which * a.heads;
+  const int4 hdr = *reinterpret_cast<const int4*>(sched);   // status, query tiles, key tiles, table entries needed
+  const int longest = sched[SCHED_MAXLEN];
+  const Tile t = reinterpret_cast<const Tile*>(sched + a.kv_list_off)[which >> 1];
+  asm volatile("" ::"s"(t.tok_start), "s"(t.doc_len), "s"(t.idx), "s"(t.batch), "s"(t.tab_base));   // keep the tile read above the branch
+  if (hdr.x != 0 || hdr.w > a.tab_stride || longest > a.max_doc_len || (which >> 1) >= hdr.z) return;
+  const int L = t.doc_len;
+  const int q_first = t.idx * BKV + (which & 1) * WIDE_KEYS;       // first key, and first query that can see one
+  if (q_first >= L) return;
+  const int nsteps = (L - q_first + TQ - 1) / TQ;
+
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, n = lane & 31, h = lane >> 5;
+  const int i16 = lane & 15, blk = (lane >> 4) & 1;
+  const int64_t tok0 = t.tok_start;
+  auto rows_of = [&](const View& v) {
+    return make_rows(reinterpret_cast<const elem_t*>(v.ptr) + t.batch * v.sb + head * v.sh + tok0 * v.st, v.st, L, a.head_dim);
+  };
+
+  if (w < 4) {
+    __builtin_amdgcn_s_setprio(3);
+    const int kb = w & 1;
+    const bool weights = w < 2;
+    const int k0 = q_first + 32 * kb;
+    float* const mine = &hand[kb][4 * lane];
+    int roff[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) roff[ks] = swz_off<D>(n, 2 * ks + h);
+    el8 fr[KS];                               // K or V; MFMA row n holds key k0 + kperm(n)
+    auto take_fragments = [&]() {
+      const unsigned short* const T = (weights ? Qs : Gs) + 2 * QTILE;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) fr[ks] = lds_row8(T + swz_off<D>(32 * kb + kperm(n), 2 * ks + h));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+    // one chain of a 32 x 32 block: rows of the tile in slot `T` against this wave's keys, operand reads LEAD ahead
+    constexpr int LEAD = 4;
+    el8 op[LEAD];
+    auto chain_begin = [&](const unsigned short* T) {
+#pragma unroll
+      for (int k = 0; k < LEAD; ++k) op[k] = lds_row8(T + roff[k]);
+    };
+    auto chain_step = [&](const unsigned short* T, f32x16& x, int k) {
+      x = mfma32(fr[k], op[k % LEAD], x);
+      if (k + LEAD < KS) op[k % LEAD] = lds_row8(T + roff[k + LEAD]);
+    };
+    auto clear = [](f32x16& x) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) x[j] = 0.0f;
+    };
+    lds_barrier();                            // the K and V rows and tiles 0 and 1 have landed
+    take_fragments();
+    lds_barrier();                            // their places are free
+    using std::integral_constant;
+    if (weights) {
+      // a block that starts past the document's end is never visible; its table reads stay inside the document's area
+      const int tblock = min(k0, L - 1) / 32;
+      const int64_t tab_row0 = (int64_t)head * a.tab_stride + t.tab_base;
+      const int64_t tab = tab_row0 + tab_seg32(L, tblock), tab_rowval = tab_row0 + tab_rowplane32(L);
+      // fused output: rem_j * do_j reaches dv_j through the diagonal of p (see bwd_dkdv_kernel)
+      float rem_own = 0.0f;
+      if (a.fuse && k0 + n < L) rem_own = a.stick[tab_rowval + k0 + n];
+      // carries of a step, requested three steps ahead; rows past the document's end take its last row's (see bwd_dkdv_kernel)
+      const unsigned run_bytes = (unsigned)L * 4u;
+      const __amdgpu_buffer_rsrc_t stick_rs = __builtin_amdgcn_make_buffer_rsrc(a.stick + tab, 0, run_bytes, 0x00020000);
+      const __amdgpu_buffer_rsrc_t gtab_rs = __builtin_amdgcn_make_buffer_rsrc(a.gtab + tab, 0, run_bytes, 0x00020000);
+      const __amdgpu_buffer_rsrc_t drem_rs = __builtin_amdgcn_make_buffer_rsrc(a.gtab + tab_rowval, 0, run_bytes, 0x00020000);
+      const int row4 = 4 * (q_first + n), last4 = 4 * (L - 1);
+      struct Raw { float e, g, d; };
+      Raw r0, r1, r2, r3;
+      auto request = [&](int step, Raw& r) {
+        const int off = min(row4 + step * (4 * TQ), last4);
+        r.e = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(stick_rs, off, 0, 0));
+        r.g = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(gtab_rs, off, 0, 0));
+        r.d = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(drem_rs, off, 0, 0));
+      };
+      request(0, r0);
+      request(1, r1);
+      request(2, r2);
+      f32x16 x;
+      clear(x);
+      chain_begin(Qs);
+#pragma unroll
+      for (int k = 0; k < KS; ++k) chain_step(Qs, x, k);
+      // Step i.  SLOT: i mod 4, the tile's slot.  BAND: one of the first two steps, whose queries may not see all keys.
+      auto step = [&](auto band_tag, auto slot_tag, const int i, Raw& set, Raw& ahead) __attribute__((always_inline)) {
+        constexpr bool BAND = decltype(band_tag)::value;
+        constexpr int SLOT = decltype(slot_tag)::value;
+        unsigned short* const Pt = Ps + (SLOT & 1) * PTILE;
+        unsigned short* const Zt = Zs + (SLOT & 1) * PTILE;
+        const unsigned short* const Tn = Qs + ((SLOT + 1) % SLOTS) * QTILE;
+        const float carry_e = set.e, carry_c = set.g, dr = set.d;
+        request(i + 3, ahead);
+        const int qw0 = q_first + i * TQ, qrow = qw0 + n;
+        const bool hidden = BAND && sub_skip<AC>(k0, qw0);     // (the table holds nothing for such a block)
+        float p[16], r[16], ends[2] = {0.0f, 0.0f};
+        {
+          float e = carry_e;
+          stick_weights<AC, PROD, BAND, true>(x, a.c, k0, qrow, h, e, p, r, ends);
+        }
+        auto put = [&](unsigned short* T, const float* v, int c) {
+          *reinterpret_cast<el8*>(T + swz_off<WIDE_KEYS>(n, 4 * kb + 2 * h + c)) = hidden ? zero8() : pack8(v + 8 * c);
+        };
+        if (BAND && a.fuse && qw0 == k0) {
+          float pd[16];
+#pragma unroll
+          for (int j = 0; j < 16; ++j) pd[j] = p[j] + (16 * h + j == n ? rem_own : 0.0f);
+          put(Pt, pd, 0);
+          put(Pt, pd, 1);
+        } else {
+          put(Pt, p, 0);
+          put(Pt, p, 1);
+        }
+        lds_barrier();
+        f32x16 da;
+        {
+          f32x4 q4[4];
+#pragma unroll
+          for (int g = 0; g < 4; ++g) q4[g] = *reinterpret_cast<const f32x4*>(mine + 256 * g);
+#pragma unroll
+          for (int j = 0; j < 16; ++j) da[j] = q4[j >> 2][j & 3];
+        }
+        chain_begin(Tn);
+        __builtin_amdgcn_sched_barrier(0);
+        clear(x);
+        float dz[16];
+        if constexpr (PROD) {                 // grad_dz with the next block's chain between its instructions
+          constexpr int A0 = KS / 4;
+#pragma unroll
+          for (int k = 0; k < A0; ++k) chain_step(Tn, x, k);
+          __builtin_amdgcn_sched_barrier(0);
+          float t0 = 0.0f, t1 = 0.0f;
+#pragma unroll
+          for (int j = 0; j < 16; j += 2) { t0 = fmaf(p[j], da[j], t0); t1 = fmaf(p[j + 1], da[j + 1], t1); }
+          float lo, hi;
+          both_halves(fmaf(-dr, ends[0] - ends[1], t0 + t1), lo, hi);
+          float dprev = fmaf(dr, ends[1], h == 1 ? carry_c + lo : carry_c);
+          __builtin_amdgcn_sched_barrier(0);
+          constexpr int REST = KS - A0;
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            const float dj = fmaf(p[j], da[j], dprev);
+            dz[j] = fmaf(r[j], dj, -dprev);
+            dprev = dj;
+#pragma unroll
+            for (int k = j * REST / 16; k < (j + 1) * REST / 16; ++k) chain_step(Tn, x, A0 + k);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          put(Zt, dz, 0);
+          put(Zt, dz, 1);
+        } else {
+#pragma unroll
+          for (int k = 0; k < KS; ++k) chain_step(Tn, x, k);
+          el8 zf[2];
+          float c = carry_c;
+          grad_dz<PROD>(p, r, da, ends, h, c, dr, zf);
+#pragma unroll
+          for (int c2 = 0; c2 < 2; ++c2)
+            *reinterpret_cast<el8*>(Zt + swz_off<WIDE_KEYS>(n, 4 * kb + 2 * h + c2)) = hidden ? zero8() : zf[c2];
+        }
+        lds_barrier();
+      };
+      using Yes = std::true_type;
+      using No = std::false_type;
+      step(Yes{}, integral_constant<int, 0>{}, 0, r0, r3);
+      if (nsteps > 1) step(Yes{}, integral_constant<int, 1>{}, 1, r1, r0);
+#pragma unroll 1
+      for (int i = 2;; i += 4) {
+        if (i >= nsteps) break;
+        step(No{}, integral_constant<int, 2>{}, i, r2, r1);
+        if (i + 1 >= nsteps) break;
+        step(No{}, integral_constant<int, 3>{}, i + 1, r3, r2);
+        if (i + 2 >= nsteps) break;
+        step(No{}, integral_constant<int, 0>{}, i + 2, r0, r3);
+        if (i + 3 >= nsteps) break;
+        step(No{}, integral_constant<int, 1>{}, i + 3, r1, r0);
+      }
+    } else {
+      f32x16 da;
+      clear(da);
+      chain_begin(Gs);
+#pragma unroll
+      for (int k = 0; k < KS; ++k) chain_step(Gs, da, k);
+      auto step = [&](auto slot_tag) __attribute__((always_inline)) {
+        const unsigned short* const Tn = Gs + ((decltype(slot_tag)::value + 1) % SLOTS) * QTILE;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 q4 = {da[4 * g], da[4 * g + 1], da[4 * g + 2], da[4 * g + 3]};
+          *reinterpret_cast<f32x4*>(mine + 256 * g) = q4;
+        }
+        lds_barrier();
+        clear(da);
+        chain_begin(Tn);
+#pragma unroll
+        for (int k = 0; k < KS; ++k) chain_step(Tn, da, k);
+        lds_barrier();
+      };
+#pragma unroll 1
+      for (int i = 0;; i += 4) {
+        step(integral_constant<int, 0>{});
+        if (i + 1 >= nsteps) break;
+        step(integral_constant<int, 1>{});
+        if (i + 2 >= nsteps) break;
+        step(integral_constant<int, 2>{});
+        if (i + 3 >= nsteps) break;
+        step(integral_constant<int, 3>{});
+        if (i + 4 >= nsteps) break;
+      }
+    }
+  } else {
+    __builtin_amdgcn_s_setprio(0);
+    const int pw = w - 4, ptid = pw * 64 + lane;
+    const int mat = pw >> 1, half = pw & 1;       // (dv | dk), half of the columns
+    const Rows qrows = rows_of(a.q), grows = rows_of(a.go);
+    using Copy = TileCopy<D, TQ, 256, false>;
+    constexpr int LOADS_PER_TILE = 2 * Copy::NCH;
+    Copy qcopy, gcopy;
+    qcopy.init(ptid, qrows.row_bytes, qrows.used_bytes);
+    gcopy.init(ptid, grows.row_bytes, grows.used_bytes);
+    auto fetch = [&](int step) {
+      qcopy.issue(qrows, q_first + step * TQ, Qs + (step % SLOTS) * QTILE);
+      gcopy.issue(grows, q_first + step * TQ, Gs + (step % SLOTS) * QTILE);
+    };
+    fetch(0);
+    {   // the 64 K and V rows wait in the places of tiles 2 and 3
+      const Rows krows = rows_of(a.k), vrows = rows_of(a.v);
+      TileCopy<D, WIDE_KEYS, 256, false> kcopy, vcopy;
+      kcopy.init(ptid, krows.row_bytes, krows.used_bytes);
+      vcopy.init(ptid, vrows.row_bytes, vrows.used_bytes);
+      kcopy.issue(krows, q_first, Qs + 2 * QTILE);
+      vcopy.issue(vrows, q_first, Gs + 2 * QTILE);
+    }
+    if (nsteps > 1) fetch(1);
+    f32x16 acc[2][DBH];
+#pragma unroll
+    for (int kb2 = 0; kb2 < 2; ++kb2)
+#pragma unroll
+      for (int j = 0; j < DBH; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[kb2][j][e] = 0.0f;
+    // transpose reads of rows 8 h + 4 u + i16 / 4 (+ 16 ks): staged block, tile
+    int xoff[2][2], yoff[2][DBH];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int r = 8 * h + 4 * u + (i16 >> 2);
+#pragma unroll
+      for (int kb2 = 0; kb2 < 2; ++kb2) {
+        const int xc = 32 * kb2 + 16 * blk + 4 * (i16 & 3);
+        xoff[u][kb2] = swz_off<WIDE_KEYS>(r, xc >> 3) + (xc & 7);
+      }
+#pragma unroll
+      for (int j = 0; j < DBH; ++j) {
+        const int yc = 32 * (half * DBH + j) + 16 * blk + 4 * (i16 & 3);
+        yoff[u][j] = swz_off<D>(r, yc >> 3) + (yc & 7);
+      }
+    }
+    el8 bf[2][DBH];
+    auto read_y = [&](int b) {
+      const unsigned short* Yt = (mat ? Qs : Gs) + (b % SLOTS) * QTILE;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int j = 0; j < DBH; ++j) bf[ks][j] = lds_tr8(Yt + yoff[0][j] + 16 * ks * D, Yt + yoff[1][j] + 16 * ks * D);
+    };
+    // (the queries of block 0 see none of the newer 32 keys: those rows stay out of its products, finite or not)
+    auto products = [&](int b) __attribute__((always_inline)) {
+      const unsigned short* Xt = (mat ? Zs : Ps) + (b & 1) * PTILE;
+      el8 af[2][2];
+#pragma unroll
+      for (int kb2 = 0; kb2 < 2; ++kb2)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) af[kb2][ks] = lds_tr8(Xt + xoff[0][kb2] + 16 * ks * WIDE_KEYS, Xt + xoff[1][kb2] + 16 * ks * WIDE_KEYS);
+      auto half_of = [&](int kb2) __attribute__((always_inline)) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (int j = 0; j < DBH; ++j) acc[kb2][j] = mfma32(bf[ks][j], af[kb2][ks], acc[kb2][j]);
+      };
+      half_of(0);
+      if (b > 0) half_of(1);
+    };
+    // Behind the products of step i - 1: tile i + 1, which the others read behind the barrier, has landed; the fragments of
+    // tile i; tile i + 3 is requested (into the slot of tile i - 1; here and not ahead of the products, which the weights waves wait for).
+    auto turn = [&](int i) __attribute__((always_inline)) {
+      if (i + 2 < nsteps) wait_loads<LOADS_PER_TILE>();
+      else wait_loads<0>();
+      lds_barrier();
+      read_y(i);
+      if (i + 3 < nsteps) fetch(i + 3);
+      lds_barrier();
+    };
+    wait_loads<0>();
+    lds_barrier();
+    lds_barrier();
+    if (2 < nsteps) fetch(2);
+    turn(0);
+#pragma unroll 1
+    for (int i = 1; i < nsteps; ++i) {
+      products(i - 1);
+      turn(i);
+    }
+    products(nsteps - 1);
+    const Rows out = rows_of(mat ? a.dk : a.dv);
+#pragma unroll
+    for (int kb2 = 0; kb2 < 2; ++kb2) {
+      const int row = q_first + 32 * kb2 + n;
+#pragma unroll
+      for (int j = 0; j < DBH; ++j)
+        store_block32_rows(acc[kb2][j], mat ? a.inv_temp : 1.0f, out, row * (int)out.row_bytes, row < L, 32 * (half * DBH + j), h, a.out_f32);
+    }
+  }
+}
+
+template __global__ void bwd_dkdv_wide_kernel<false, false, 256>(const KArgs);
+template __global__ void bwd_dkdv_wide_kernel<true, false, 256>(const KArgs);
+template __global__ void bwd_dkdv_wide_kernel<false, true, 256>(const KArgs);
+template __global__ void bwd_dkdv_wide_kernel<true, true, 256>(const KArgs);
+template __global__ void bwd_dkdv_wide_kernel<false, true, 192>(const KArgs);
+template __global__ void bwd_dkdv_wide_kernel<true, true, 192>(const KArgs);
+
+// tiles: upper bound on the tiles of the key-tile list, no more than it has room for
+hipError_t launch_bwd_dkdv_wide(const KArgs& a, bool ac, bool prod, int tiles, hipStream_t s) {
+  const dim3 grid((unsigned)tiles * (BKV / WIDE_KEYS) * (unsigned)a.heads), block(512);
+  if (prod && used_width(a.head_dim) == 192) {
+    if (ac) hipLaunchKernelGGL((bwd_dkdv_wide_kernel<true, true, 192>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((bwd_dkdv_wide_kernel<false, true, 192>), grid, block, 0, s, a);
+  } else if (ac) {
+    if (prod) hipLaunchKernelGGL((bwd_dkdv_wide_kernel<true, true, 256>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((bwd_dkdv_wide_kernel<true, false, 256>), grid, block, 0, s, a);
+  } else {
+    if (prod) hipLaunchKernelGGL((bwd_dkdv_wide_kernel<false, true, 256>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((bwd_dkdv_wide_kernel<false, false, 256>), grid, block, 0, s, a);
+  }
+  return hipGetLastError();
+}
+
+}  // inline namespace SBA_ELEM_NS
+}  // namespace sba

@@ -1,7 +1,6 @@
 """head_dim 256 (upstream takes any head_dim through BLOCK_D = next_power_of_2(d), sb_varlen_fwd.py:479).
-The forward and the dq pass are the kernels of the smaller head dims instantiated with one wave per
-SIMD; the dk/dv pass is a kernel of its own kind (four independent waves per key tile, the queries
-streamed through LDS, two passes: dv, then dk).  Everything here goes against the fp32 CPU oracle
+The forward and the dq pass are the kernels of the smaller head dims instantiated with two workgroups and one per compute unit; the
+dk/dv pass is a kernel of its own kind (64 keys per workgroup, three kinds of waves).  Everything here goes against the fp32 CPU oracle
 with the gate of the other head dims: max-abs 2e-2 before the output's own bf16 rounding."""
 import os
 
@@ -43,8 +42,8 @@ def _run(q, k, v, do, lengths, ac=False, drem=None, fused=False):
 @pytest.mark.parametrize("product_space", [False, True])
 @pytest.mark.parametrize("ac", [False, True])
 def test_long_documents(ac, product_space, monkeypatch):
-    """Documents of 23 and 5 key tiles and a short one: the streamed query blocks wrap the two LDS buffers many
-    times in both passes of the dk/dv kernel; a gradient for rem as well."""
+    """Documents of 23 and 5 key tiles and a short one: the queries wrap the ring of the dk/dv kernel many
+    times; a gradient for rem as well."""
     from stickbreaking_attention import _ops
     monkeypatch.setattr(_ops, "PRODUCT_SPACE", product_space)
     lengths = [2900, 611, 77]
