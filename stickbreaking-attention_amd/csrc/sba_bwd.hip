@@ -28,9 +28,8 @@ inline namespace SBA_ELEM_NS {
 // -------------------------------------------------------------------------------------------
 // dq pass
 // -------------------------------------------------------------------------------------------
-// (head_dim 256: the tiles take 128 KiB, one workgroup per CU, one wave per SIMD with 512 registers)
 template <int D, bool AC, bool PROD, int U = D>
-__global__ void __launch_bounds__(NT, D > 128 ? 1 : 2) bwd_dq_kernel(const KArgs a) {
+__global__ void __launch_bounds__(NT, 2) bwd_dq_kernel(const KArgs a) {
   constexpr int KS = U / 16, DB = U / 32;
   constexpr int TILE = BN * D;   // elements of one K or V tile (unpadded, swizzled)
   // K (row reads for the scores, transpose reads for dq) and V (row reads) tiles,
@@ -1121,10 +1120,6 @@ template __global__ void bwd_dq_kernel<128, false, false>(const KArgs);
 template __global__ void bwd_dq_kernel<128, false, true>(const KArgs);
 template __global__ void bwd_dq_kernel<128, true, false>(const KArgs);
 template __global__ void bwd_dq_kernel<128, true, true>(const KArgs);
-template __global__ void bwd_dq_kernel<256, false, false>(const KArgs);
-template __global__ void bwd_dq_kernel<256, false, true>(const KArgs);
-template __global__ void bwd_dq_kernel<256, true, false>(const KArgs);
-template __global__ void bwd_dq_kernel<256, true, true>(const KArgs);
 template __global__ void bwd_dkdv_tail_kernel<32, false, false>(const KArgs);
 template __global__ void bwd_dkdv_tail_kernel<32, false, true>(const KArgs);
 template __global__ void bwd_dkdv_tail_kernel<32, true, false>(const KArgs);
@@ -1148,13 +1143,11 @@ template __global__ void bwd_dkdv_kernel<128, true, true>(const KArgs);
 
 template __global__ void bwd_dq_kernel<128, false, true, 96>(const KArgs);
 template __global__ void bwd_dq_kernel<128, true, true, 96>(const KArgs);
-template __global__ void bwd_dq_kernel<256, false, true, 192>(const KArgs);
-template __global__ void bwd_dq_kernel<256, true, true, 192>(const KArgs);
 template __global__ void bwd_dkdv_kernel<128, false, true, 96>(const KArgs);
 template __global__ void bwd_dkdv_kernel<128, true, true, 96>(const KArgs);
 
 // Width of the narrower instantiation a kernel width has (see used_width), or the width itself.
-template <int D> constexpr int narrow_width() { return D == 128 ? 96 : D == 256 ? 192 : D; }
+template <int D> constexpr int narrow_width() { return D == 128 ? 96 : D; }
 
 template <int D>
 static hipError_t launch_dq_d(const KArgs& a, bool ac, bool prod, int n_q_max, hipStream_t s) {
@@ -1222,7 +1215,7 @@ static hipError_t launch_dkdv_d(const KArgs& a_in, bool ac, bool prod, int n_lon
 
 hipError_t launch_bwd_dq(const KArgs& a, int head_dim, bool ac, bool prod, int n_q_max, hipStream_t s) {
   head_dim = kernel_width(head_dim);
-  if (head_dim == 256) return launch_dq_d<256>(a, ac, prod, n_q_max, s);
+  if (head_dim == 256) return launch_bwd_dq_wide(a, ac, prod, n_q_max, s);
   if (head_dim == 128) return launch_dq_d<128>(a, ac, prod, n_q_max, s);
   if (head_dim == 64) return launch_dq_d<64>(a, ac, prod, n_q_max, s);
   return launch_dq_d<32>(a, ac, prod, n_q_max, s);

@@ -176,6 +176,7 @@ inline bool has_dkdv_tail_kernel(int head_dim) { return head_dim <= 64; }
                            hipStream_t s);                                                                       \
   hipError_t launch_bwd_dkdv(const KArgs& a, int head_dim, bool attend_current, bool product, int n_long_max,    \
                              int n_last_max, hipStream_t s);                                                     \
+  hipError_t launch_bwd_dq_wide(const KArgs& a, bool attend_current, bool product, int n_q_max, hipStream_t s);   \
   hipError_t launch_bwd_dkdv_wide(const KArgs& a, bool attend_current, bool product, int tiles, hipStream_t s);   \
   hipError_t launch_bwd_chain(const ChainArgs& a, bool attend_current, bool wide, int n_q_max, int workgroups,              \
                               hipStream_t s);                                                                    \

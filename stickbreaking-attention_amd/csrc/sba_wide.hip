@@ -356,12 +356,337 @@ __global__ void __launch_bounds__(512, 1) bwd_dkdv_wide_kernel(const KArgs a) {
   }
 }
 
+// -------------------------------------------------------------------------------------------
+// dq pass of the same head dims: 128 queries of one (document, head) per workgroup, the keys walked from the oldest to the diagonal, 32
+// per step.  Q and dO fragments of 32 queries and their dq are 256 registers, so two waves of a SIMD share a block of 32 queries:
+//
+//   waves 0 .. 3  "scores": Q fragments; p, dz, the running sum and the gradient table
+//   waves 4 .. 7  "sums": dO fragments and dq; do.v of a block, handed to the scores wave through LDS in fp32, and dq += dz K of the
+//                 block before, whose dz comes back the same way; they also copy the K / V tiles
+//
+// A step has two phases with a barrier behind each: weights of block i next to the products of block i - 1, then dz of block i
+// between the scores of block i + 1 next to its do.v.  A tile is requested two steps before it is read (four slots of 32 KiB).
+// Bound by the two phases, 3300 cycles of a step: vector work of one wave, then 32 matrix instructions of two.  16 heads x 16 K tokens in
+// eight documents, head_dim 256: 795 -> 620 us against one wave per SIMD with 512 registers for everything.  Reading
+// operands six or eight instead of four products ahead changes nothing.
+// -------------------------------------------------------------------------------------------
+template <bool AC, bool PROD, int U>
+__global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
+  constexpr int D = 256, KS = U / 16, DB = U / 32;
+  constexpr int BF = 32, SLOTS = 4, TILE = BF * D;
+  static_assert(SLOTS * BF == BM, "the query rows wait in the ring first");
+  __shared__ __attribute__((aligned(16))) unsigned short Ks[SLOTS * TILE];
+  __shared__ __attribute__((aligned(16))) unsigned short Vs[SLOTS * TILE];
+  // per block of queries: do.v of a key block as the accumulators lie, a quad of every lane at a time, and dz as operand fragments
+  constexpr int HAND_Z = 16 * 64, HAND = HAND_Z + 2 * 64 * 4;
+  __shared__ __attribute__((aligned(16))) float hand[4 * HAND];
+  __shared__ float drs[4][32];                                               // do . v_row of the fused output
+
+  const int* sched = a.sched;
+  const int slot = blockIdx.x / a.heads;
+  const int head = blockIdx.x - slot * a.heads;
+  const int4 hdr = *reinterpret_cast<const int4*>(sched);   // status, query tiles, key tiles, table entries needed
+  const int longest = sched[SCHED_MAXLEN];
+  const Tile t = reinterpret_cast<const Tile*>(sched + SCHED_HDR)[slot];
+  asm volatile("" ::"s"(t.tok_start), "s"(t.doc_len), "s"(t.idx), "s"(t.batch), "s"(t.tab_base));   // keep the tile read above the branch
+  const int tid = threadIdx.x;
+  const bool refused = hdr.x != 0 || hdr.w > a.tab_stride || longest > a.max_doc_len;
+  if (refused || slot >= hdr.y) {
+    if (a.clear_spare) {     // for the dk/dv pass as well, which has no slots to spare
+      int row0, row1;
+      unsigned pair;
+      spare_rows(refused, slot, hdr.y, sched[SCHED_TOTAL], a.tokens, a.nan_pair, row0, row1, pair);
+      fill_rows16(a.dq, head, row0, row1, a.head_dim << a.out_f32, pair, tid, 512);
+      fill_rows16(a.dk, head, row0, row1, a.head_dim << a.out_f32, pair, tid, 512);
+      fill_rows16(a.dv, head, row0, row1, a.head_dim << a.out_f32, pair, tid, 512);
+    }
+    return;
+  }
+  const int L = t.doc_len;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, n = lane & 31, h = lane >> 5;
+  const int rb = w & 3;                                  // 32-query block of this wave
+  const int m0 = t.idx * BM, qw0 = m0 + 32 * rb, qrow = qw0 + n;
+  const bool qvalid = qrow < L;
+  const int nblk = min(m0 + BM - 1, L - 1) / BF + 1;     // key blocks any query of the tile sees
+  const int own = qw0 / BF;                              // the block's own keys: the last one it sees
+  const int64_t tok0 = t.tok_start;
+  auto rows_of = [&](const View& v) {
+    return make_rows(reinterpret_cast<const elem_t*>(v.ptr) + t.batch * v.sb + head * v.sh + tok0 * v.st, v.st, L, a.head_dim);
+  };
+  // Row reads of chunk 2 ks + h: the swizzle is an XOR of the chunk number's low four bits, so the offset of a further chunk is
+  // the first one's with a constant XORed in, and of the upper half's 256 bytes on: one register instead of sixteen.
+  int rbase = swz_off<D>(n, h);
+  el8 fr[KS];                                            // Q or dO: operand column n is query qw0 + n
+  constexpr int LEAD = 4;
+  el8 op[LEAD];
+  auto read_op = [&](const unsigned short* T, int k) { return lds_row8(T + (rbase ^ ((k % 8) << 4)) + 128 * (k / 8)); };
+  auto chain_begin = [&](const unsigned short* T) {
+#pragma unroll
+    for (int k = 0; k < LEAD; ++k) op[k] = read_op(T, k);
+  };
+  auto chain_step = [&](const unsigned short* T, f32x16& x, int k) {
+    x = mfma32(op[k % LEAD], fr[k], x);
+    if (k + LEAD < KS) op[k % LEAD] = read_op(T, k + LEAD);
+  };
+  auto clear = [](f32x16& x) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) x[j] = 0.0f;
+  };
+  // the tile's Q and dO rows by way of LDS (Q by the scores waves, dO by the others)
+  {
+    const Rows rows = rows_of(w < 4 ? a.q : a.go);
+    TileCopy<D, BM, 256, false> copy;
+    copy.init(tid & 255, rows.row_bytes, rows.used_bytes);
+    copy.issue(rows, m0, w < 4 ? Ks : Vs);
+  }
+  wait_loads<0>();
+  lds_barrier();
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) fr[ks] = read_op((w < 4 ? Ks : Vs) + 32 * rb * D, ks);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  lds_barrier();                              // the places are free
+  float* const mine = hand + HAND * rb + 4 * lane;
+
+  using std::integral_constant;
+  if (w < 4) {
+    __builtin_amdgcn_s_setprio(3);
+    float dr = 0.0f;                          // d(rem) of this lane's row (see bwd_dq_kernel)
+    if (a.grem.ptr != nullptr && qvalid) {
+      const elem_t* grb = reinterpret_cast<const elem_t*>(a.grem.ptr) + t.batch * a.grem.sb + head * a.grem.sh + tok0 * a.grem.st;
+      dr = (float)grb[(int64_t)qrow * a.grem.st];
+    }
+    // the document's area of the two tables (uniform); a lane adds its row and a block's 32-bit offset
+    const int64_t tab0 = (int64_t)head * a.tab_stride + t.tab_base;
+    const float* stick = a.stick + tab0;
+    float* gtab = a.gtab + tab0;
+    auto carry_of = [&](int i) {
+      float e = PROD ? 1.0f : 0.0f;
+      if (qvalid && i <= own) e = stick[(unsigned)(tab_seg32(L, i) + qrow)];
+      return e;
+    };
+    float e0 = carry_of(0), e1 = carry_of(1), e2 = carry_of(2), e3;     // requested three steps ahead
+    float carry_c = 0.0f;
+    lds_barrier();                            // tile 0 has landed, do . v_row is there
+    if (a.fuse) dr += drs[rb][n];
+    if (qvalid && h == 0) gtab[(unsigned)(tab_rowplane32(L) + qrow)] = dr;
+    f32x16 x;
+    clear(x);
+    chain_begin(Ks);
+#pragma unroll
+    for (int k = 0; k < KS; ++k) chain_step(Ks, x, k);
+    auto step = [&](auto slot_tag, const int i, const float e, float& ahead) __attribute__((always_inline)) {
+      constexpr int SLOT = decltype(slot_tag)::value;
+      const unsigned short* const Tn = Ks + ((SLOT + 1) % SLOTS) * TILE;
+      ahead = carry_of(i + 3);
+      const bool visible = i <= own;
+      float p[16], r[16], ends[2] = {0.0f, 0.0f};
+      if (visible) {
+        if (qvalid && h == 0) gtab[(unsigned)(tab_seg32(L, i) + qrow)] = carry_c;
+        float c = e;
+        if (i < own) stick_weights<AC, PROD, false, true>(x, a.c, i * BF, qrow, h, c, p, r, ends);
+        else stick_weights<AC, PROD, true, true>(x, a.c, i * BF, qrow, h, c, p, r, ends);
+      }
+      lds_barrier();
+      if (visible) {
+        f32x16 da;
+        {
+          f32x4 q4[4];
+#pragma unroll
+          for (int g = 0; g < 4; ++g) q4[g] = *reinterpret_cast<const f32x4*>(mine + 256 * g);
+#pragma unroll
+          for (int j = 0; j < 16; ++j) da[j] = q4[j >> 2][j & 3];
+        }
+        chain_begin(Tn);                      // (behind the last visible block: a tile that may not be there, unused)
+        __builtin_amdgcn_sched_barrier(0);
+        clear(x);
+        el8 zf[2];
+        if constexpr (PROD) {                 // grad_dz with the next block's chain between its instructions
+          constexpr int A0 = KS / 4, REST = KS - A0;
+#pragma unroll
+          for (int k = 0; k < A0; ++k) chain_step(Tn, x, k);
+          __builtin_amdgcn_sched_barrier(0);
+          float t0 = 0.0f, t1 = 0.0f;
+#pragma unroll
+          for (int j = 0; j < 16; j += 2) { t0 = fmaf(p[j], da[j], t0); t1 = fmaf(p[j + 1], da[j + 1], t1); }
+          float lo, hi;
+          both_halves(fmaf(-dr, ends[0] - ends[1], t0 + t1), lo, hi);
+          float dprev = fmaf(dr, ends[1], h == 1 ? carry_c + lo : carry_c);
+          carry_c += lo + hi;
+          __builtin_amdgcn_sched_barrier(0);
+          float dz[16];
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            const float dj = fmaf(p[j], da[j], dprev);
+            dz[j] = fmaf(r[j], dj, -dprev);
+            dprev = dj;
+#pragma unroll
+            for (int k = j * REST / 16; k < (j + 1) * REST / 16; ++k) chain_step(Tn, x, A0 + k);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          zf[0] = pack8(dz);
+          zf[1] = pack8(dz + 8);
+        } else {
+#pragma unroll
+          for (int k = 0; k < KS; ++k) chain_step(Tn, x, k);
+          grad_dz<PROD>(p, r, da, ends, h, carry_c, dr, zf);
+        }
+        *reinterpret_cast<el8*>(mine + HAND_Z) = zf[0];
+        *reinterpret_cast<el8*>(mine + HAND_Z + 256) = zf[1];
+      }
+      lds_barrier();
+    };
+#pragma unroll 1
+    for (int i = 0;; i += 4) {
+      step(integral_constant<int, 0>{}, i, e0, e3);
+      if (i + 1 >= nblk) break;
+      step(integral_constant<int, 1>{}, i + 1, e1, e0);
+      if (i + 2 >= nblk) break;
+      step(integral_constant<int, 2>{}, i + 2, e2, e1);
+      if (i + 3 >= nblk) break;
+      step(integral_constant<int, 3>{}, i + 3, e3, e2);
+      if (i + 4 >= nblk) break;
+    }
+  } else {
+    __builtin_amdgcn_s_setprio(0);
+    const int i16 = lane & 15, blk = (lane >> 4) & 1;
+    const Rows krows = rows_of(a.k), vrows = rows_of(a.v);
+    using Copy = TileCopy<D, BF, 256, true>;
+    constexpr int LOADS_PER_TILE = 2 * Copy::NCH;
+    Copy kcopy, vcopy;
+    kcopy.init(tid & 255, krows.row_bytes, krows.used_bytes);
+    vcopy.init(tid & 255, vrows.row_bytes, vrows.used_bytes);
+    auto fetch = [&](int i) {
+      kcopy.issue(krows, i * BF, Ks + (i % SLOTS) * TILE);
+      vcopy.issue(vrows, i * BF, Vs + (i % SLOTS) * TILE);
+    };
+    if (a.fuse) {
+      float dot = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const el8 vown = load_frag(vrows, qrow, 32 * ks + 16 * h);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dot = fmaf((float)fr[ks][e], (float)vown[e], dot);
+      }
+      float lo, hi;
+      both_halves(dot, lo, hi);
+      if (h == 0) drs[rb][n] = lo + hi;
+    }
+    wait_loads<0>();
+    fetch(0);
+    if (1 < nblk) fetch(1);
+    if (2 < nblk) fetch(2);
+    f32x16 dq[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) dq[db][j] = 0.0f;
+    int tbase[2];                             // transpose reads of rows 8 u + 4 h + i16 / 4 (+ 16 tt), columns of block 0
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int col = 16 * blk + 4 * (i16 & 3);
+      tbase[u] = swz_off<D>(8 * u + 4 * h + (i16 >> 2), col >> 3) + (col & 7);
+    }
+    if (nblk > 2) wait_loads<2 * LOADS_PER_TILE>();
+    else if (nblk > 1) wait_loads<LOADS_PER_TILE>();
+    else wait_loads<0>();
+    lds_barrier();
+    f32x16 da;
+    clear(da);
+    chain_begin(Vs);
+#pragma unroll
+    for (int k = 0; k < KS; ++k) chain_step(Vs, da, k);
+    // dq += dz K of a block, whose tile is at Kt
+    auto product = [&](const unsigned short* Kt) __attribute__((always_inline)) {
+      const el8 zf[2] = {*reinterpret_cast<const el8*>(mine + HAND_Z), *reinterpret_cast<const el8*>(mine + HAND_Z + 256)};
+      constexpr int N = 2 * DB, AHEAD = 4;    // operand reads run AHEAD products ahead
+      el8 kt[AHEAD];
+      auto read_k = [&](int m) {
+        const int tt = m / DB, db = m % DB;
+        const unsigned short* const krow = Kt + 16 * tt * D + 128 * (db / 4);
+        return lds_tr8(krow + (tbase[0] ^ ((db % 4) << 5)), krow + (tbase[1] ^ ((db % 4) << 5)));
+      };
+#pragma unroll
+      for (int m = 0; m < AHEAD; ++m) kt[m] = read_k(m);
+#pragma unroll
+      for (int m = 0; m < N; ++m) {
+        dq[m % DB] = mfma32(kt[m % AHEAD], zf[m / DB], dq[m % DB]);   // (dq^T: see store_block32_rows)
+        if (m + AHEAD < N) kt[m % AHEAD] = read_k(m + AHEAD);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    auto step = [&](auto slot_tag, const int i) __attribute__((always_inline)) {
+      constexpr int SLOT = decltype(slot_tag)::value;
+      const unsigned short* const Tn = Vs + ((SLOT + 1) % SLOTS) * TILE;
+      asm volatile("" : "+v"(rbase), "+v"(tbase[0]), "+v"(tbase[1]));     // (the XORs stay here: there are no registers for their results)
+      if (i <= own) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 q4 = {da[4 * g], da[4 * g + 1], da[4 * g + 2], da[4 * g + 3]};
+          *reinterpret_cast<f32x4*>(mine + 256 * g) = q4;
+        }
+      }
+      if (i > 0 && i - 1 <= own) product(Ks + ((SLOT + SLOTS - 1) % SLOTS) * TILE);
+      // tile i + 1, which everyone reads behind this barrier, has landed
+      if (i + 2 < nblk) wait_loads<LOADS_PER_TILE>();
+      else wait_loads<0>();
+      lds_barrier();
+      if (i + 3 < nblk) fetch(i + 3);
+      clear(da);        // (always: it must not live through the products)
+      if (i + 1 <= own) {
+        chain_begin(Tn);
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+          chain_step(Tn, da, k);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      lds_barrier();
+    };
+#pragma unroll 1
+    for (int i = 0;; i += 4) {
+      step(integral_constant<int, 0>{}, i);
+      if (i + 1 >= nblk) break;
+      step(integral_constant<int, 1>{}, i + 1);
+      if (i + 2 >= nblk) break;
+      step(integral_constant<int, 2>{}, i + 2);
+      if (i + 3 >= nblk) break;
+      step(integral_constant<int, 3>{}, i + 3);
+      if (i + 4 >= nblk) break;
+    }
+    if (nblk - 1 <= own) product(Ks + ((nblk - 1) % SLOTS) * TILE);
+    store_rows(dq, a.inv_temp, rows_of(a.dq), qrow, L, h, a.out_f32);
+  }
+}
+
 template __global__ void bwd_dkdv_wide_kernel<false, false, 256>(const KArgs);
 template __global__ void bwd_dkdv_wide_kernel<true, false, 256>(const KArgs);
 template __global__ void bwd_dkdv_wide_kernel<false, true, 256>(const KArgs);
 template __global__ void bwd_dkdv_wide_kernel<true, true, 256>(const KArgs);
 template __global__ void bwd_dkdv_wide_kernel<false, true, 192>(const KArgs);
 template __global__ void bwd_dkdv_wide_kernel<true, true, 192>(const KArgs);
+
+template __global__ void bwd_dq_wide_kernel<false, false, 256>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<true, false, 256>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<false, true, 256>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<true, true, 256>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<false, true, 192>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<true, true, 192>(const KArgs);
+
+hipError_t launch_bwd_dq_wide(const KArgs& a, bool ac, bool prod, int n_q_max, hipStream_t s) {
+  const dim3 grid((unsigned)n_q_max * (unsigned)a.heads), block(512);
+  if (prod && used_width(a.head_dim) == 192) {
+    if (ac) hipLaunchKernelGGL((bwd_dq_wide_kernel<true, true, 192>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((bwd_dq_wide_kernel<false, true, 192>), grid, block, 0, s, a);
+  } else if (ac) {
+    if (prod) hipLaunchKernelGGL((bwd_dq_wide_kernel<true, true, 256>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((bwd_dq_wide_kernel<true, false, 256>), grid, block, 0, s, a);
+  } else {
+    if (prod) hipLaunchKernelGGL((bwd_dq_wide_kernel<false, true, 256>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((bwd_dq_wide_kernel<false, false, 256>), grid, block, 0, s, a);
+  }
+  return hipGetLastError();
+}
 
 // tiles: upper bound on the tiles of the key-tile list, no more than it has room for
 hipError_t launch_bwd_dkdv_wide(const KArgs& a, bool ac, bool prod, int tiles, hipStream_t s) {

@@ -1,4 +1,4 @@
-"""The dk / dv pass of head_dim 129 .. 256 where its step structure can go wrong: documents that end on either side of its 64-key tiles,
+"""The two passes of the backward at head_dim 129 .. 256 where its step structure can go wrong: documents that end on either side of their 64-key and 128-query tiles,
 32-query steps and four ring slots, columns that end inside a product wave's half; and rows that are not finite."""
 import pytest
 import torch
@@ -26,11 +26,11 @@ def test_edges(d, lengths, ac, product_space, monkeypatch):
 
 
 @pytest.mark.parametrize("ac", [False, True])
-def test_a_query_that_is_not_finite_stays_out_of_the_blocks_it_cannot_see(ac):
+def test_rows_that_are_not_finite_stay_behind_the_blocks_that_hide_them(ac):
     lengths = [300, 77]
     T = sum(lengths)
     tensors = orc.make_inputs((2, T, 256), 9)
-    clean = _run(*tensors, lengths, ac)[3:]
+    _, _, clean_dq, *clean = _run(*tensors, lengths, ac)
     for at in (3, 40, 64, 100, 200, 299, 333):
         start, length = (0, 300) if at < 300 else (300, 77)
         block = start + (at - start) // 32 * 32
@@ -40,3 +40,8 @@ def test_a_query_that_is_not_finite_stays_out_of_the_blocks_it_cannot_see(ac):
             x[which][:, at] = float("inf")
             for got, want in zip(_run(*x, lengths, ac)[3:], clean):
                 assert torch.equal(got[:, newer], want[:, newer]), (at, which)
+        for which in (1, 2):          # a key: queries ahead of its block
+            x = [t.clone() for t in tensors]
+            x[which][:, at] = float("inf")
+            dq = _run(*x, lengths, ac)[2]
+            assert torch.equal(dq[:, :block], clean_dq[:, :block]), (at, which)
