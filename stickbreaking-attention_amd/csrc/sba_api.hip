@@ -231,6 +231,7 @@ int forward(const sba_problem* p, bool fixed, const void* schedule, size_t sched
   a.stick = stick;
   a.weights = weights;
   a.resident = device_cus();
+  a.n_items = (int)std::min<long long>(0x7fffffff, (fixed ? (long long)p->batch * ((p->tokens + BM - 1) / BM) : sz.rows / BM) * p->heads);
   a.clear_spare = fixed ? 0 : 1;
   a.nan_pair = p->dtype == SBA_F16 && !a.out_f32 ? 0x7e007e00u : 0x7fc07fc0u;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);

@@ -35,7 +35,8 @@ struct KArgs {
   float inv_temp;
   unsigned* work;              // work counters of the backward's persistent launch (WORK_WORDS words at the end of the
                                // gradient table; the dq pass clears them), or null: one workgroup per work item
-  int n_items;                 // work items of this launch (what the grid would be with one workgroup per item)
+  int n_items;                 // work items of this launch (what the grid would be with one workgroup per item; forward: without spare
+                               // slots and, for packed documents, without their last, partial tiles)
   int resident;                // backward, host side: workgroups of a persistent launch (0: never persistent); forward: the
                                // device's compute units
   int min_items_each;          // host side: a launch is persistent when it has this many items per workgroup
