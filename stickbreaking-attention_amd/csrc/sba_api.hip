@@ -207,6 +207,26 @@ int fill_common(const sba_problem* p, bool fixed, const Sizes& sz, const void* s
   return 0;
 }
 
+// Where the forward's kernel for problems that leave most of the chip idle (sba_small.hip) is the faster one: both times
+// estimated, in us, from what 90 problems of 4 to 32 heads, 128 to 4096 tokens and 1 to 16 documents took at head_dim 32, 64 and 128.
+//   fwd_kernel takes at least `base` and `step` for every 32 keys of the longest document (more, once several workgroups share a compute unit);
+//   the other one its own `small_base` and the longer of what the longest document's rounds of 128 keys take one after the other (`round` each)
+//   and of what 1024 (above head_dim 64: 512) workgroups at a time need: `group` each and `per_round` for every round, of which a workgroup has half
+//   its document's and half a one for the remainder.  (By tokens, documents are about halfway between the mean and the longest.)
+// A tenth must be gained, and 2 us, with which four times as many workgroups pay at the dispatcher (13 prompts of up to 172 tokens 9.9 us alone
+// with either, 10.6 for 11.3 in a row).  Of the problems taken all gain (head_dim 64: 4 heads x 512 14.4 / 9.7, 16 x 4096 78 / 68, 32 x 1024 24 / 17.5), and
+// of those left to fwd_kernel none would gain more than a tenth (head_dim 64: 16 heads of 4 x 1024 25.6 / 28, 32 x 2048 43 / 40; head_dim 128: 32 x 2048 58 / 74).
+bool forward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
+  if (!(p->flags & SBA_PRODUCT_SPACE) || p->head_dim > 128 || sz.n_docs <= 0) return false;
+  struct Cost { double base, step, small_base, round, group, per_round; int at_once; };
+  static constexpr Cost COSTS[3] = {{5.2, 0.46, 5.5, 0.75, 2.7, 1.33, 1024}, {5.8, 0.55, 6.2, 0.90, 3.4, 1.66, 1024}, {6.5, 0.73, 7.0, 1.19, 4.0, 1.60, 512}};
+  const Cost& c = COSTS[p->head_dim <= 32 ? 0 : (p->head_dim <= 64 ? 1 : 2)];
+  const double longest = declared_max_doc_len(p, fixed), typical = 0.5 * (longest + std::min(longest, (double)sz.rows / sz.n_docs));
+  const double round = 32 * SMALL_WAVES, groups = (double)(sz.rows / 32 + sz.n_docs) * p->heads / c.at_once;
+  const double small = c.small_base + std::max(c.round * longest / round, groups * (c.group + c.per_round * (0.5 * typical / round + 0.5)));
+  return std::max(1.1 * small, small + 2.0) < c.base + c.step * longest / 32;
+}
+
 int forward(const sba_problem* p, bool fixed, const void* schedule, size_t sched_bytes, const sba_view* q,
             const sba_view* k, const sba_view* v, const sba_view* o, const sba_view* rem, float* stick,
             size_t table_bytes, float* weights, size_t weights_bytes, void* stream, bool timed = true) {
@@ -238,7 +258,9 @@ int forward(const sba_problem* p, bool fixed, const void* schedule, size_t sched
   hipError_t he = hipSuccess;
   {   // (packed input without a single document still launches: the spare workgroups clear the outputs)
     Timer tm(0, s, timed);
-    he = (p->dtype == SBA_F16 ? f16::launch_fwd : bf16::launch_fwd)(a, p->head_dim, (p->flags & SBA_ATTEND_CURRENT) != 0,
+    if (weights == nullptr && !table_only && forward_small(p, fixed, sz))
+      he = (p->dtype == SBA_F16 ? f16::launch_fwd_small : bf16::launch_fwd_small)(a, (p->flags & SBA_ATTEND_CURRENT) != 0, sz.n_q_max, s);
+    else he = (p->dtype == SBA_F16 ? f16::launch_fwd : bf16::launch_fwd)(a, p->head_dim, (p->flags & SBA_ATTEND_CURRENT) != 0,
                     (p->flags & SBA_PRODUCT_SPACE) != 0, weights != nullptr ? 1 : (table_only ? 2 : 0), sz.n_q_max, s);
   }
   return (int)he;

@@ -30,6 +30,7 @@ typedef __attribute__((ext_vector_type(4))) short s16x4;
 typedef __attribute__((ext_vector_type(8))) short s16x8;
 
 constexpr int BM = 128;  // query rows per workgroup tile (4 waves x 32 rows)
+constexpr int SMALL_WAVES = 4;   // waves of a workgroup of sba_small.hip
 constexpr int BN = 64;   // keys per KV tile staged in LDS by the dq pass
 constexpr int BKV = 128;  // keys owned by one workgroup of the dk/dv pass
 constexpr int BT = 32;   // keys per carry-table entry (one MFMA sub-block)

@@ -1,0 +1,247 @@
+// Kernels for problems that leave most of the chip idle.
+//
+// With few tiles a launch takes as long as one workgroup's walk along the other axis, a block of 32 at a time: 47 steps of 0.65 us
+// for the forward of 1500 tokens, whatever the chip could do beside them.  Here a workgroup owns 32 rows instead of 128, and
+// its four waves take four consecutive blocks of the other axis at a time.  (Eight waves: a single head of 4096 keys 30 us for 35, but
+// a full chip is served worse, since the last round of every walk is the emptier: 16 x 2048 29 us for 26, 16 x 4 x 1024 38 for 28.)
+#include <type_traits>
+
+#include "sba_kernels.hpp"
+
+namespace sba {
+inline namespace SBA_ELEM_NS {
+
+// One wave's copy of a 32 x D block into its own unpadded, swizzled tile, keys permuted as by TileCopy<.., KEYS = true>.
+template <int D>
+struct WaveCopy {
+  static constexpr int C8 = D / 8, RPI = 64 / C8, NCH = 32 / RPI;
+  static constexpr int KINDS = D == 128 ? 4 : 2;      // instructions apart by this many have their rows' swizzle in common
+  int voff[KINDS];
+  __device__ __forceinline__ void init(int lane, unsigned row_bytes, int used_bytes) {
+#pragma unroll
+    for (int k = 0; k < KINDS; ++k) {
+      const int m = k * RPI + lane / C8, logical = (lane % C8) ^ swz<D>(m);
+      voff[k] = 16 * logical < used_bytes ? (kperm(m) - row_delta(k)) * (int)row_bytes + 16 * logical : OUTSIDE;
+    }
+  }
+  // source row of instruction j's first row
+  static constexpr int row_delta(int j) { return D == 128 ? 16 * (j & 1) + 4 * (j >> 1) : 4 * j; }
+  __device__ __forceinline__ void issue(const Rows& r, int row0, unsigned short* tile) const {
+#pragma unroll
+    for (int j = 0; j < NCH; ++j)
+      async_copy16(r.rsrc, tile + j * RPI * D, voff[j % KINDS], __builtin_amdgcn_readfirstlane((row0 + row_delta(j)) * (int)r.row_bytes));
+  }
+};
+
+// Four consecutive columns of a lane's output row, from `col` on (see store_rows_axpy for the sum).
+__device__ __forceinline__ void store_quad(f32x4 v, const Rows& out, const Rows& addend, int row, bool ok, int col, bool fuse, float factor, bool f32) {
+  typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
+  typedef __attribute__((ext_vector_type(4))) elem_t el4;
+  if (fuse) {
+    const u32x2 raw = __builtin_amdgcn_raw_buffer_load_b64(addend.rsrc, 2 * col < addend.used_bytes ? row * (int)addend.row_bytes + 2 * col : OUTSIDE, 0, 0);
+    const el4 other = __builtin_bit_cast(el4, raw);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = fmaf(factor, (float)other[e], (float)(elem_t)v[e]);
+  }
+  ok = ok && 2 * col < out.used_bytes;
+  const el2 a = cvt2(v[0], v[1]), b = cvt2(v[2], v[3]);
+  if (f32) {
+    const f32x4 r = {(float)a[0], (float)a[1], (float)b[0], (float)b[1]};
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, r), out.rsrc, ok ? row * (int)out.row_bytes + 4 * col : OUTSIDE, 0, 0);
+  } else {
+    const u32x2 r = {__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b)};
+    __builtin_amdgcn_raw_buffer_store_b64(r, out.rsrc, ok ? row * (int)out.row_bytes + 2 * col : OUTSIDE, 0, 0);
+  }
+}
+
+// The waves' accumulators of one output, a quad of every lane at a time, into LDS; behind a barrier wave w adds up and stores quads w, w + W ..
+template <int DB, int W>
+__device__ __forceinline__ void add_waves(float* sums, const f32x16 (&acc)[DB], int w, int lane) {
+#pragma unroll
+  for (int q = 0; q < 4 * DB; ++q) {
+    const f32x4 v = {acc[q >> 2][4 * (q & 3)], acc[q >> 2][4 * (q & 3) + 1], acc[q >> 2][4 * (q & 3) + 2], acc[q >> 2][4 * (q & 3) + 3]};
+    *reinterpret_cast<f32x4*>(sums + ((q * W + w) * 64 + lane) * 4) = v;
+  }
+}
+template <int W>
+__device__ __forceinline__ f32x4 sum_quad(const float* sums, int q, int lane) {
+  f32x4 v = *reinterpret_cast<const f32x4*>(sums + (q * W * 64 + lane) * 4);
+#pragma unroll
+  for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4*>(sums + ((q * W + k) * 64 + lane) * 4);
+  return v;
+}
+
+// Forward.  32 query rows of one (document, head); in a round wave w has the w-th newest key block that is left.  What a block leaves of
+// the stick (its product of 1 - beta) is known before its weights are, so the waves form odds and products side by side,
+// exchange the products through LDS (one barrier a round) and go on to weights and p V each on its own.  The output is the sum
+// over the waves.  K and V rows come to every wave's own piece of LDS, the next round's as soon as this one's are read.
+// What bounds it: the round's serial chain (products, odds, barrier, weights) while the chip is empty, 0.9 us a round of 128 keys against
+// 0.54 us a step of 32 in fwd_kernel; then the additive time of matrix and vector instructions, with
+// 16 waves per compute unit at head_dim 64 and 8 at 128.  Measured (us, fwd_kernel first): head_dim 64, 4 heads of 512 tokens 14.4 / 9.7,
+// of 2048 40 / 20; 16 heads of 1024 23.7 / 15.2; head_dim 128, 4 heads of 512 18.0 / 11.7, 16 heads of 2048 54 / 43.
+template <int D, bool AC, int U>
+__global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 4 : 2) fwd_small_kernel(const KArgs a) {
+  constexpr int W = SMALL_WAVES, KS = U / 16, DB = U / 32, TILE = 32 * D;
+  __shared__ __attribute__((aligned(16))) unsigned short smem[2 * W * TILE];   // per wave: K block, V block; then the waves' outputs
+  __shared__ float left[2][W][32];              // by round parity: what a wave's block leaves of a query's stick
+  static_assert(2 * W * TILE * 2 >= W * 64 * DB * 16 * 4, "the waves' accumulators fit the tiles' place");
+
+  const int* sched = a.sched;
+  const int part = blockIdx.x / a.heads;
+  const int head = blockIdx.x - part * a.heads;
+  const int slot = part / (BM / 32), sub = part % (BM / 32);
+  const int4 hdr = *reinterpret_cast<const int4*>(sched);   // status, query tiles, key tiles, table entries needed
+  const Tile t = reinterpret_cast<const Tile*>(sched + SCHED_HDR)[slot];
+  asm volatile("" ::"s"(t.tok_start), "s"(t.doc_len), "s"(t.idx), "s"(t.batch));   // keep the tile read above the branch
+  const int tid = threadIdx.x;
+  const bool refused = hdr.x != 0 || (a.stick != nullptr && hdr.w > a.tab_stride);
+  if (refused || slot >= hdr.y) {
+    if (a.clear_spare && sub == 0) {
+      int row0, row1;
+      unsigned pair;
+      spare_rows(refused, slot, hdr.y, sched[SCHED_TOTAL], a.tokens, a.nan_pair, row0, row1, pair);
+      fill_rows16(a.o, head, row0, row1, a.head_dim << a.out_f32, pair, tid, W * 64);
+      fill_rows16(a.rem, head, row0, row1, 1 << a.out_f32, pair, tid, W * 64);
+    }
+    return;
+  }
+  const int L = t.doc_len, qw0 = t.idx * BM + 32 * sub;
+  if (qw0 >= L) return;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, n = lane & 31, h = lane >> 5;
+  const int i16 = lane & 15, blk = (lane >> 4) & 1;
+  const int qrow = qw0 + n;
+  const bool qvalid = qrow < L;
+  const int64_t tok0 = t.tok_start;
+  auto rows_of = [&](const View& v) {
+    return make_rows(reinterpret_cast<const elem_t*>(v.ptr) + t.batch * v.sb + head * v.sh + tok0 * v.st, v.st, L, a.head_dim);
+  };
+  const Rows qrows = rows_of(a.q), krows = rows_of(a.k), vrows = rows_of(a.v);
+  unsigned short* const Kt = smem + 2 * w * TILE;
+  unsigned short* const Vt = Kt + TILE;
+  WaveCopy<D> kcopy, vcopy;
+  kcopy.init(lane, krows.row_bytes, krows.used_bytes);
+  vcopy.init(lane, vrows.row_bytes, vrows.used_bytes);
+  constexpr int LOADS = WaveCopy<D>::NCH;
+  const int n_blocks = qw0 / 32 + 1, n_rounds = (n_blocks + W - 1) / W;
+  auto block_of = [&](int r) { return n_blocks - 1 - (r * W + w); };   // (below zero: none left for this wave)
+  // (a wave without a block copies rows outside the document: zeros, nothing is fetched)
+  auto row_of = [&](int r) { const int b = block_of(r); return b >= 0 ? 32 * b : L; };
+  kcopy.issue(krows, row_of(0), Kt);
+  vcopy.issue(vrows, row_of(0), Vt);
+  el8 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) qf[ks] = load_frag(qrows, qrow, 32 * ks + 16 * h);
+  f32x16 o[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[db][i] = 0.0f;
+  const int kbase = swz_off<D>(n, h);
+  int vbase[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int c = 16 * blk + 4 * (i16 & 3);
+    vbase[u] = swz_off<D>(8 * u + 4 * h + (i16 >> 2), c >> 3) + (c & 7);
+  }
+  // the document's table area: every round's store is issued, outside the area where there is nothing to write
+  const bool table = a.stick != nullptr;
+  float* const stick = table ? a.stick + (int64_t)head * a.tab_stride + t.tab_base : nullptr;
+  const __amdgpu_buffer_rsrc_t stick_rs = __builtin_amdgcn_make_buffer_rsrc(stick, 0, table ? (unsigned)min((int64_t)0x7fffffff, 4 * (int64_t)tab_doc_entries(L)) : 0u, 0x00020000);
+  float run = 1.0f;                             // stick left in front of this round's newest block
+  wait_loads<0>();
+#pragma unroll 1
+  for (int r = 0; r < n_rounds; ++r) {
+    const int b = block_of(r), k0 = 32 * b;
+    // K of this round has landed; behind it only the table's store and V may be on their way
+    wait_loads<LOADS + 1>();
+    f32x16 x;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = 0.0f;
+    {
+      el8 kfr[KS];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kfr[ks] = lds_row8(Kt + (kbase ^ (ks << 4)));
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) x = mfma32(kfr[ks], qf[ks], x);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    kcopy.issue(krows, r + 1 < n_rounds ? row_of(r + 1) : L, Kt);
+    const int lim = b >= 0 ? qrow - k0 - 16 * h + (AC ? 1 : 0) : 0;     // visible keys of this lane: i < lim (all of them but in the newest block)
+    float e[16], inv[4];
+    float total = stick_odds<true, false>(x, a.c, lim, e, inv);
+    if (__builtin_amdgcn_ballot_w64(!(total > 0.0f)) != 0) total = stick_odds<true, true>(x, a.c, lim, e, inv);   // (see stick_weights_fwd)
+    float lo, hi;
+    both_halves(total, lo, hi);
+    if (h == 0) left[r & 1][w][n] = lo * hi;
+    lds_barrier();
+    float carry = run;
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      if (k == w) carry = run;
+      run *= left[r & 1][k][n];
+    }
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, carry), stick_rs, b >= 0 && qvalid && h == 0 ? 4 * (tab_seg32(L, b) + qrow) : OUTSIDE, 0, 0);
+    float s = h == 0 ? carry * hi : carry, p[16];      // (keys of the h = 1 lane are the newer ones)
+#pragma unroll
+    for (int g = 3; g >= 0; --g) {
+      s *= inv[g];
+      float left_of = s;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        p[4 * g + j] = left_of * e[4 * g + j];
+        if (j < 3) left_of += p[4 * g + j];
+      }
+    }
+    wait_loads<LOADS + 1>();                    // V of this round
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      const el8 pf = pack8(p + 8 * tt);
+      const unsigned short* const vrow = Vt + 16 * tt * D;
+#pragma unroll
+      for (int db = 0; db < DB; ++db) o[db] = mfma32(lds_tr8(vrow + (vbase[0] ^ (db << 5)), vrow + (vbase[1] ^ (db << 5))), pf, o[db]);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    vcopy.issue(vrows, r + 1 < n_rounds ? row_of(r + 1) : L, Vt);
+  }
+  if (w == 0 && h == 0 && qvalid) {
+    elem_t* const at = reinterpret_cast<elem_t*>(a.rem.ptr) + t.batch * a.rem.sb + head * a.rem.sh + (tok0 + qrow) * a.rem.st;
+    if (a.out_f32) *reinterpret_cast<float*>(at) = (float)(elem_t)run;
+    else *at = (elem_t)run;
+    if (table) stick[(unsigned)(tab_rowplane32(L) + qrow)] = run;
+  }
+  wait_loads<0>();                              // (copies of nothing into the place that is written now)
+  lds_barrier();
+  float* const sums = reinterpret_cast<float*>(smem);
+  add_waves<DB, W>(sums, o, w, lane);
+  lds_barrier();
+  const Rows orows = rows_of(a.o);
+  for (int q = w; q < 4 * DB; q += W)
+    store_quad(sum_quad<W>(sums, q, lane), orows, vrows, qrow, qvalid, 32 * (q >> 2) + 8 * (q & 3) + 4 * h, a.fuse, run, a.out_f32);
+}
+
+#define SBA_SMALL(D, U)                                                   \
+  template __global__ void fwd_small_kernel<D, false, U>(const KArgs);    \
+  template __global__ void fwd_small_kernel<D, true, U>(const KArgs);
+SBA_SMALL(64, 32)
+SBA_SMALL(64, 64)
+SBA_SMALL(128, 96)
+SBA_SMALL(128, 128)
+#undef SBA_SMALL
+
+template <int D, int U>
+static hipError_t launch_fwd_small_d(const KArgs& a, bool ac, int n_q_max, hipStream_t s) {
+  const dim3 grid((unsigned)n_q_max * (BM / 32) * (unsigned)a.heads), block(SMALL_WAVES * 64);
+  if (ac) hipLaunchKernelGGL((fwd_small_kernel<D, true, U>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((fwd_small_kernel<D, false, U>), grid, block, 0, s, a);
+  return hipGetLastError();
+}
+hipError_t launch_fwd_small(const KArgs& a, bool ac, int n_q_max, hipStream_t s) {
+  if (a.head_dim <= 32) return launch_fwd_small_d<64, 32>(a, ac, n_q_max, s);
+  if (a.head_dim <= 64) return launch_fwd_small_d<64, 64>(a, ac, n_q_max, s);
+  if (used_width(a.head_dim) == 96) return launch_fwd_small_d<128, 96>(a, ac, n_q_max, s);
+  return launch_fwd_small_d<128, 128>(a, ac, n_q_max, s);
+}
+
+}  // inline namespace SBA_ELEM_NS
+}  // namespace sba

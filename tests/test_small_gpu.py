@@ -1,0 +1,49 @@
+"""Problems of few tiles take kernels of their own (sba_small.hip): on either side of their blocks of 32 and rounds of 128, in every form
+that the rule lets in, against the oracle and against the general kernels, which the same heads take when there are enough of them."""
+import pytest
+import torch
+
+from oracle import sb_oracle as orc
+from stickbreaking_attention import sb_attn
+from tests.helpers import assert_close, oracle_varlen
+from tests.test_fused_gpu import check, fused_reference
+from tests.test_head_dim_256_gpu import DEV, _need_gpu, _run  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d,lengths", [(64, [193, 128, 1]), (64, [129, 31, 32, 33]), (64, [255, 257, 300]), (64, [1, 1025]), (32, [500, 129]),
+                                       (8, [385, 384]), (40, [640]), (72, [161, 260]), (96, [513]), (104, [290, 100]), (128, [511, 2]),
+                                       (128, [256, 255, 257])])
+@pytest.mark.parametrize("ac,fused", [(False, False), (True, False), (False, True), (True, True)])
+def test_packed_edges(d, lengths, ac, fused):
+    T = sum(lengths)
+    q, k, v, do = orc.make_inputs((3, T, d), d + T)
+    if fused:
+        check(_run(q, k, v, do, lengths, ac, fused=True), fused_reference(q, k, v, do, lengths, ac))
+        return
+    drem = torch.randn((3, T), generator=torch.Generator().manual_seed(d)).to(torch.bfloat16)
+    ref = oracle_varlen(q, k, v, do, lengths, ac, drem=drem)
+    for name, g, r in zip(("o", "rem", "dq", "dk", "dv"), _run(q, k, v, do, lengths, ac, drem=drem), ref):
+        assert_close(name, g, r)
+
+
+_ROUND = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 2.0 ** -7}   # one step of the output (float32 inputs round to bfloat16)
+
+
+@pytest.mark.parametrize("dtype", list(_ROUND))
+@pytest.mark.parametrize("d,batch,T,layout", [(64, 1, 600, "heads"), (64, 2, 257, "tokens"), (32, 3, 130, "heads"), (96, 1, 400, "tokens"), (128, 2, 321, "heads")])
+@pytest.mark.parametrize("ac", [False, True])
+def test_the_same_as_the_general_kernels(d, batch, T, layout, dtype, ac):
+    """Remainders to the bit (the table goes to the backward of either form), outputs up to the order of a float32 sum."""
+    gen = torch.Generator(device=DEV).manual_seed(T)
+    shape = (batch, 2, T, d) if layout == "heads" else (batch, T, 2, d)
+    q, k, v = (torch.randn(shape, generator=gen, device=DEV).to(dtype) for _ in range(3))
+    if layout == "tokens":
+        q, k, v = (t.transpose(1, 2) for t in (q, k, v))
+    times = 64 * 1024 // T                    # (fills the chip several times over)
+    o, rem = sb_attn(q, k, v, attend_current=ac)
+    o_many, rem_many = sb_attn(*(t.repeat(1, times, 1, 1) for t in (q, k, v)), attend_current=ac)
+    assert torch.equal(rem, rem_many[:, :2])
+    # a float32 sum of T weighted values below 6 in another order, which may round to the neighbour
+    torch.testing.assert_close(o, o_many[:, :2], rtol=_ROUND[dtype], atol=T * 6 * 2.0 ** -24)

@@ -40,7 +40,8 @@ def test_order_of_the_list(lengths):
 @pytest.mark.parametrize("heads,head_dim,lengths", [(12, 64, [1500, 700, 129, 2100]), (20, 32, [3000, 1, 1111]), (7, 128, [4096, 900]),
                                                     (3, 64, [97] * 100)])
 def test_a_launch_dealt_in_turns_covers_every_tile(heads, head_dim, lengths):
-    """More items than compute units, all on the chip at once: the same bits as head by head, which is dealt straight."""
+    """More items than compute units, all on the chip at once: the same as head by head, which is dealt straight or small enough for the kernel
+    of few tiles.  The two add a row up in another order: float32 sums of at most 3000 weighted values below 6, which may round to a neighbour."""
     gen = torch.Generator(device=DEV).manual_seed(3)
     q, k, v = (torch.randn(heads, sum(lengths), head_dim, generator=gen, device=DEV).to(torch.bfloat16) for _ in range(3))
     cu = helpers.cu_from_lengths(lengths, device=DEV)
@@ -49,4 +50,5 @@ def test_a_launch_dealt_in_turns_covers_every_tile(heads, head_dim, lengths):
     o, rem = sb_attn_varlen(q, k, v, cu, max(lengths), zero_start=False)
     for h in range(heads):
         o1, rem1 = sb_attn_varlen(q[h:h + 1], k[h:h + 1], v[h:h + 1], cu, max(lengths), zero_start=False)
-        assert torch.equal(o[h], o1[0]) and torch.equal(rem[h], rem1[0])
+        torch.testing.assert_close(o[h], o1[0], rtol=2.0 ** -7, atol=3000 * 6 * 2.0 ** -24)
+        assert torch.equal(rem[h], rem1[0])
