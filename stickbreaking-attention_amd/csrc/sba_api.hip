@@ -207,24 +207,36 @@ int fill_common(const sba_problem* p, bool fixed, const Sizes& sz, const void* s
   return 0;
 }
 
-// Where the forward's kernel for problems that leave most of the chip idle (sba_small.hip) is the faster one: both times
+// Where the kernels for problems that leave most of the chip idle (sba_small.hip) are the faster ones: both times
 // estimated, in us, from what 90 problems of 4 to 32 heads, 128 to 4096 tokens and 1 to 16 documents took at head_dim 32, 64 and 128.
-//   fwd_kernel takes at least `base` and `step` for every 32 keys of the longest document (more, once several workgroups share a compute unit);
-//   the other one its own `small_base` and the longer of what the longest document's rounds of 128 keys take one after the other (`round` each)
-//   and of what 1024 (above head_dim 64: 512) workgroups at a time need: `group` each and `per_round` for every round, of which a workgroup has half
+//   The general kernels take at least `base` and `step` for every 32 tokens of the longest document (more, once workgroups share a compute unit);
+//   the small ones their own `small_base` and the longer of what the longest document's rounds of 128 take one after the other (`round` each)
+//   and of what `at_once` workgroups at a time need: `group` each and `per_round` for every round, of which a workgroup has half
 //   its document's and half a one for the remainder.  (By tokens, documents are about halfway between the mean and the longest.)
-// A tenth must be gained, and 2 us, with which four times as many workgroups pay at the dispatcher (13 prompts of up to 172 tokens 9.9 us alone
-// with either, 10.6 for 11.3 in a row).  Of the problems taken all gain (head_dim 64: 4 heads x 512 14.4 / 9.7, 16 x 4096 78 / 68, 32 x 1024 24 / 17.5), and
-// of those left to fwd_kernel none would gain more than a tenth (head_dim 64: 16 heads of 4 x 1024 25.6 / 28, 32 x 2048 43 / 40; head_dim 128: 32 x 2048 58 / 74).
-bool forward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
+// `gain` must be gained, and 2 us, with which four times as many workgroups pay at the dispatcher (the forward of 13 prompts of up to 172 tokens: 9.9 us
+// alone with either, 10.6 for 11.3 in a row).
+struct SmallCost { double base, step, small_base, round, group, per_round; int at_once; };
+bool small_wins(const SmallCost (&costs)[3], double gain, const sba_problem* p, bool fixed, const Sizes& sz) {
   if (!(p->flags & SBA_PRODUCT_SPACE) || p->head_dim > 128 || sz.n_docs <= 0) return false;
-  struct Cost { double base, step, small_base, round, group, per_round; int at_once; };
-  static constexpr Cost COSTS[3] = {{5.2, 0.46, 5.5, 0.75, 2.7, 1.33, 1024}, {5.8, 0.55, 6.2, 0.90, 3.4, 1.66, 1024}, {6.5, 0.73, 7.0, 1.19, 4.0, 1.60, 512}};
-  const Cost& c = COSTS[p->head_dim <= 32 ? 0 : (p->head_dim <= 64 ? 1 : 2)];
+  const SmallCost& c = costs[p->head_dim <= 32 ? 0 : (p->head_dim <= 64 ? 1 : 2)];
   const double longest = declared_max_doc_len(p, fixed), typical = 0.5 * (longest + std::min(longest, (double)sz.rows / sz.n_docs));
   const double round = 32 * SMALL_WAVES, groups = (double)(sz.rows / 32 + sz.n_docs) * p->heads / c.at_once;
   const double small = c.small_base + std::max(c.round * longest / round, groups * (c.group + c.per_round * (0.5 * typical / round + 0.5)));
-  return std::max(1.1 * small, small + 2.0) < c.base + c.step * longest / 32;
+  return std::max(gain * small, small + 2.0) < c.base + c.step * longest / 32;
+}
+// Of the problems taken all gain (head_dim 64: 4 heads x 512 14.4 / 9.7, 16 x 4096 78 / 68, 32 x 1024 24 / 17.5), and of those left to fwd_kernel none
+// would gain more than a tenth (head_dim 64: 16 heads of 4 x 1024 25.6 / 28, 32 x 2048 43 / 40; head_dim 128: 32 x 2048 58 / 74).
+bool forward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
+  static constexpr SmallCost COSTS[3] = {{5.2, 0.46, 5.5, 0.75, 2.7, 1.33, 1024}, {5.8, 0.55, 6.2, 0.90, 3.4, 1.66, 1024}, {6.5, 0.73, 7.0, 1.19, 4.0, 1.60, 512}};
+  return small_wins(COSTS, 1.1, p, fixed, sz);
+}
+// The backward, both passes, against the one-pass form (head_dim 64: 4 heads x 512 36.2 / 23.5, 16 x 1024 55 / 38, 16 x 2048 91 / 80, left out
+// 16 x 4096 229 / 219, 32 x 4 x 256 28 / 34; head_dim 128: 4 heads x 512 42 / 32, 16 x 512 43 / 33.5, left out 16 x 1024 66 / 66).  Documents of one or two
+// blocks are with the general two passes (head_dim 64: 64 tokens 16.0 / 16.8).
+bool backward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
+  if (backward_form() != 0 || g_dkdv_workgroups.load() != 0 || declared_max_doc_len(p, fixed) <= 64) return false;
+  static constexpr SmallCost COSTS[3] = {{16.0, 1.04, 12.5, 1.9, 3.7, 2.35, 512}, {17.0, 1.15, 14.0, 2.34, 6.0, 2.75, 512}, {19.0, 1.42, 18.5, 3.6, 9.5, 3.6, 256}};
+  return small_wins(COSTS, 1.05, p, fixed, sz);
 }
 
 int forward(const sba_problem* p, bool fixed, const void* schedule, size_t sched_bytes, const sba_view* q,
@@ -303,6 +315,17 @@ int backward(const sba_problem* p, bool fixed, const void* schedule, size_t sche
   a.clear_spare = fixed ? 0 : 1;
   a.nan_pair = p->dtype == SBA_F16 && !a.out_f32 ? 0x7e007e00u : 0x7fc07fc0u;
   hipError_t he = hipSuccess;
+  if (backward_small(p, fixed, sz)) {
+    {
+      Timer tm(1, s);
+      he = (p->dtype == SBA_F16 ? f16::launch_bwd_dq_small : bf16::launch_bwd_dq_small)(a, ac, sz.n_q_max, s);
+    }
+    if (he == hipSuccess) {
+      Timer tm(2, s);
+      he = (p->dtype == SBA_F16 ? f16::launch_bwd_dkdv_small : bf16::launch_bwd_dkdv_small)(a, ac, sz.n_q_max, s);
+    }
+    return (int)he;
+  }
   {
     Timer tm(1, s);
     he = (p->dtype == SBA_F16 ? f16::launch_bwd_dq : bf16::launch_bwd_dq)(a, p->head_dim, ac, prod, sz.n_q_max, s);
@@ -355,6 +378,7 @@ bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
   const int form = backward_form();
   if (form == 1 || g_dkdv_workgroups.load() != 0 || !chain_possible(p, fixed, sz)) return false;
   if (form == 2 || form == 3) return true;
+  if (backward_small(p, fixed, sz)) return false;
   const long long chains = (long long)sz.n_docs * p->heads, items = (long long)sz.n_kv_max * p->heads;
   const long long mean = sz.rows / sz.n_docs, longest = declared_max_doc_len(p, fixed);
   // a document of one or two steps: nothing to hand on, and one launch more (0.85 .. 1.01)

@@ -180,6 +180,8 @@ inline bool has_dkdv_tail_kernel(int head_dim) { return head_dim <= 64; }
   hipError_t launch_bwd_dq_wide(const KArgs& a, bool attend_current, bool product, int n_q_max, hipStream_t s);   \
   hipError_t launch_bwd_dkdv_wide(const KArgs& a, bool attend_current, bool product, int tiles, hipStream_t s);   \
   hipError_t launch_fwd_small(const KArgs& a, bool attend_current, int n_q_max, hipStream_t s);                  \
+  hipError_t launch_bwd_dq_small(const KArgs& a, bool attend_current, int n_q_max, hipStream_t s);                  \
+  hipError_t launch_bwd_dkdv_small(const KArgs& a, bool attend_current, int n_q_max, hipStream_t s);                  \
   hipError_t launch_bwd_chain(const ChainArgs& a, bool attend_current, bool wide, int n_q_max, int workgroups,              \
                               hipStream_t s);                                                                    \
   }

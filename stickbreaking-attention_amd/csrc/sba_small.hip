@@ -11,8 +11,8 @@
 namespace sba {
 inline namespace SBA_ELEM_NS {
 
-// One wave's copy of a 32 x D block into its own unpadded, swizzled tile, keys permuted as by TileCopy<.., KEYS = true>.
-template <int D>
+// One wave's copy of a 32 x D block into its own unpadded, swizzled tile; KEYS: rows permuted as by TileCopy<.., KEYS = true>.
+template <int D, bool KEYS>
 struct WaveCopy {
   static constexpr int C8 = D / 8, RPI = 64 / C8, NCH = 32 / RPI;
   static constexpr int KINDS = D == 128 ? 4 : 2;      // instructions apart by this many have their rows' swizzle in common
@@ -21,11 +21,11 @@ struct WaveCopy {
 #pragma unroll
     for (int k = 0; k < KINDS; ++k) {
       const int m = k * RPI + lane / C8, logical = (lane % C8) ^ swz<D>(m);
-      voff[k] = 16 * logical < used_bytes ? (kperm(m) - row_delta(k)) * (int)row_bytes + 16 * logical : OUTSIDE;
+      voff[k] = 16 * logical < used_bytes ? ((KEYS ? kperm(m) : m) - row_delta(k)) * (int)row_bytes + 16 * logical : OUTSIDE;
     }
   }
   // source row of instruction j's first row
-  static constexpr int row_delta(int j) { return D == 128 ? 16 * (j & 1) + 4 * (j >> 1) : 4 * j; }
+  static constexpr int row_delta(int j) { return !KEYS ? j * RPI : D == 128 ? 16 * (j & 1) + 4 * (j >> 1) : 4 * j; }
   __device__ __forceinline__ void issue(const Rows& r, int row0, unsigned short* tile) const {
 #pragma unroll
     for (int j = 0; j < NCH; ++j)
@@ -69,6 +69,11 @@ __device__ __forceinline__ f32x4 sum_quad(const float* sums, int q, int lane) {
 #pragma unroll
   for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4*>(sums + ((q * W + k) * 64 + lane) * 4);
   return v;
+}
+
+template <int DB, int W>
+__device__ __forceinline__ void store_sum(const float* sums, int w, int lane, float scale, const Rows& out, int row, bool ok, int h, bool f32) {
+  for (int q = w; q < 4 * DB; q += W) store_quad(sum_quad<W>(sums, q, lane) * scale, out, out, row, ok, 32 * (q >> 2) + 8 * (q & 3) + 4 * h, false, 0.0f, f32);
 }
 
 // Forward.  32 query rows of one (document, head); in a round wave w has the w-th newest key block that is left.  What a block leaves of
@@ -119,10 +124,10 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 4 : 2) fwd_small_k
   const Rows qrows = rows_of(a.q), krows = rows_of(a.k), vrows = rows_of(a.v);
   unsigned short* const Kt = smem + 2 * w * TILE;
   unsigned short* const Vt = Kt + TILE;
-  WaveCopy<D> kcopy, vcopy;
+  WaveCopy<D, true> kcopy, vcopy;
   kcopy.init(lane, krows.row_bytes, krows.used_bytes);
   vcopy.init(lane, vrows.row_bytes, vrows.used_bytes);
-  constexpr int LOADS = WaveCopy<D>::NCH;
+  constexpr int LOADS = WaveCopy<D, true>::NCH;
   const int n_blocks = qw0 / 32 + 1, n_rounds = (n_blocks + W - 1) / W;
   auto block_of = [&](int r) { return n_blocks - 1 - (r * W + w); };   // (below zero: none left for this wave)
   // (a wave without a block copies rows outside the document: zeros, nothing is fetched)
@@ -220,28 +225,341 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 4 : 2) fwd_small_k
     store_quad(sum_quad<W>(sums, q, lane), orows, vrows, qrow, qvalid, 32 * (q >> 2) + 8 * (q & 3) + 4 * h, a.fuse, run, a.out_f32);
 }
 
+// -------------------------------------------------------------------------------------------
+// Backward, in two passes of the same kind.  The first owns 32 queries, four waves walk the keys from the oldest
+// on, a block each at a time; they exchange every block's sum of p (do.v) and with it each knows the running sum D in front of its block (see
+// sba_chain.hip), which goes into the gradient table.  With the table the second, which owns 32 keys, needs no order at all: its
+// waves take the query blocks that can see them in turn.  Sums over the waves at the end.
+// What bounds them: up to 8 waves per compute unit (head_dim 64; 4 at 128) each a round's chain of its own: two products, odds and weights, the
+// barrier, the gradient of the logits, one or two products more: 1.1 us a round.  That is no shorter than a step of bwd_chain_kernel, but
+// a round is 128 keys, and nothing is handed from one workgroup to the next.  Measured (us, one-pass form first): head_dim 64, 4 heads of 512 tokens
+// 36.2 / 11.3 + 12.2, of 2048 89 / 25 + 26; 16 heads of 1024 55 / 17 + 21; 2 x 8 of 1500 78 / 23 + 33; head_dim 128, 4 heads of 512 42 / 15 + 16.
+// Eight waves a workgroup gain where 4 heads are all there is (2048 tokens: 51 to 43) and lose from 16 heads on (1024 tokens: 37 to 45); two lose everywhere
+// else (2 x 8 of 1500: 57 to 75).
+// -------------------------------------------------------------------------------------------
+template <int D, bool AC, int U>
+__global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_dq_small_kernel(const KArgs a) {
+  constexpr int W = SMALL_WAVES, KS = U / 16, DB = U / 32, TILE = 32 * D;
+  __shared__ __attribute__((aligned(16))) unsigned short smem[3 * W * TILE];   // per wave: two K blocks, a V block; then the waves' dq
+  __shared__ float tot[2][W][32];               // by round parity: a block's sum of p (do.v) per query
+  static_assert(3 * W * TILE * 2 >= W * 64 * DB * 16 * 4, "the waves' accumulators fit the tiles' place");
+
+  const int* sched = a.sched;
+  const int part = blockIdx.x / a.heads;
+  const int head = blockIdx.x - part * a.heads;
+  const int slot = part / (BM / 32), sub = part % (BM / 32);
+  const int4 hdr = *reinterpret_cast<const int4*>(sched);   // status, query tiles, key tiles, table entries needed
+  const int longest = sched[SCHED_MAXLEN];
+  const Tile t = reinterpret_cast<const Tile*>(sched + SCHED_HDR)[slot];
+  asm volatile("" ::"s"(t.tok_start), "s"(t.doc_len), "s"(t.idx), "s"(t.batch), "s"(t.tab_base));   // keep the tile read above the branch
+  const int tid = threadIdx.x;
+  const bool refused = hdr.x != 0 || hdr.w > a.tab_stride || longest > a.max_doc_len;
+  if (refused || slot >= hdr.y) {
+    if (a.clear_spare && sub == 0) {            // for the second pass as well, which has no slots to spare
+      int row0, row1;
+      unsigned pair;
+      spare_rows(refused, slot, hdr.y, sched[SCHED_TOTAL], a.tokens, a.nan_pair, row0, row1, pair);
+      fill_rows16(a.dq, head, row0, row1, a.head_dim << a.out_f32, pair, tid, W * 64);
+      fill_rows16(a.dk, head, row0, row1, a.head_dim << a.out_f32, pair, tid, W * 64);
+      fill_rows16(a.dv, head, row0, row1, a.head_dim << a.out_f32, pair, tid, W * 64);
+    }
+    return;
+  }
+  const int L = t.doc_len, qw0 = t.idx * BM + 32 * sub;
+  if (qw0 >= L) return;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, n = lane & 31, h = lane >> 5;
+  const int i16 = lane & 15, blk = (lane >> 4) & 1;
+  const int qrow = qw0 + n;
+  const bool qvalid = qrow < L;
+  const int64_t tok0 = t.tok_start;
+  auto rows_of = [&](const View& v) {
+    return make_rows(reinterpret_cast<const elem_t*>(v.ptr) + t.batch * v.sb + head * v.sh + tok0 * v.st, v.st, L, a.head_dim);
+  };
+  const Rows qrows = rows_of(a.q), grows = rows_of(a.go), krows = rows_of(a.k), vrows = rows_of(a.v);
+  unsigned short* const Kt = smem + 3 * w * TILE;       // (two of them)
+  unsigned short* const Vt = Kt + 2 * TILE;
+  WaveCopy<D, true> kcopy, vcopy;
+  kcopy.init(lane, krows.row_bytes, krows.used_bytes);
+  vcopy.init(lane, vrows.row_bytes, vrows.used_bytes);
+  const int n_blocks = qw0 / 32 + 1, n_rounds = (n_blocks + W - 1) / W;
+  auto block_of = [&](int r) { return r * W + w; };
+  auto row_of = [&](int r) { return block_of(r) < n_blocks ? 32 * block_of(r) : L; };   // (outside the document: zeros, nothing is fetched)
+  kcopy.issue(krows, row_of(0), Kt);
+  vcopy.issue(vrows, row_of(0), Vt);
+  el8 qf[KS], gf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    qf[ks] = load_frag(qrows, qrow, 32 * ks + 16 * h);
+    gf[ks] = load_frag(grows, qrow, 32 * ks + 16 * h);
+  }
+  float* const stick = a.stick + (int64_t)head * a.tab_stride + t.tab_base;
+  float* const gtab = a.gtab + (int64_t)head * a.tab_stride + t.tab_base;
+  const unsigned area = 4u * (unsigned)tab_doc_entries(L);
+  const __amdgpu_buffer_rsrc_t stick_rs = __builtin_amdgcn_make_buffer_rsrc(stick, 0, area, 0x00020000);
+  const __amdgpu_buffer_rsrc_t gtab_rs = __builtin_amdgcn_make_buffer_rsrc(gtab, 0, area, 0x00020000);
+  auto entry = [&](int r) { const int b = block_of(r); return b < n_blocks && qvalid ? 4 * (tab_seg32(L, b) + qrow) : OUTSIDE; };
+  float e_next = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(stick_rs, entry(0), 0, 0));
+  // D in front of the oldest key: the complete gradient of rem, times rem
+  float run;
+  {
+    float dr = 0.0f;
+    if (a.grem.ptr != nullptr && qvalid)
+      dr = (float)(reinterpret_cast<const elem_t*>(a.grem.ptr) + t.batch * a.grem.sb + head * a.grem.sh + tok0 * a.grem.st)[(int64_t)qrow * a.grem.st];
+    if (a.fuse) {                               // d(rem) = do . v_row as well (see bwd_dq_kernel)
+      float dot = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const el8 vown = load_frag(vrows, qrow, 32 * ks + 16 * h);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dot = fmaf((float)gf[ks][e], (float)vown[e], dot);
+      }
+      float lo, hi;
+      both_halves(dot, lo, hi);
+      dr += lo + hi;
+    }
+    run = qvalid ? dr * stick[(unsigned)(tab_rowplane32(L) + qrow)] : 0.0f;
+  }
+  f32x16 dq[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) dq[db][i] = 0.0f;
+  const int kbase = swz_off<D>(n, h);
+  int tbase[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int c = 16 * blk + 4 * (i16 & 3);
+    tbase[u] = swz_off<D>(8 * u + 4 * h + (i16 >> 2), c >> 3) + (c & 7);
+  }
+  wait_loads<0>();
+#pragma unroll 1
+  for (int r = 0; r < n_rounds; ++r) {
+    const int b = block_of(r), k0 = 32 * b;
+    wait_loads<1>();                            // K, V and the stick of this round; the table's store may be on its way
+    const float e_in = b < n_blocks && qvalid ? e_next : 1.0f;
+    const unsigned short* const Kr = Kt + (r & 1) * TILE;
+    e_next = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(stick_rs, r + 1 < n_rounds ? entry(r + 1) : OUTSIDE, 0, 0));
+    kcopy.issue(krows, r + 1 < n_rounds ? row_of(r + 1) : L, Kt + ((r + 1) & 1) * TILE);
+    f32x16 x, da;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = da[i] = 0.0f;
+    {
+      el8 kfr[KS], vfr[KS];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) { kfr[ks] = lds_row8(Kr + (kbase ^ (ks << 4))); vfr[ks] = lds_row8(Vt + (kbase ^ (ks << 4))); }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) { x = mfma32(kfr[ks], qf[ks], x); da = mfma32(vfr[ks], gf[ks], da); }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    vcopy.issue(vrows, r + 1 < n_rounds ? row_of(r + 1) : L, Vt);
+    float p[16], m[16], ends[2], c = e_in;      // m: 1 - beta
+    stick_weights<AC, true, true, true>(x, a.c, b < n_blocks ? k0 : L + 32, qrow, h, c, p, m, ends);   // (no block: all keys masked)
+    float t0 = 0.0f, t1 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 16; j += 2) { t0 = fmaf(p[j], da[j], t0); t1 = fmaf(p[j + 1], da[j + 1], t1); }
+    float lo, hi;
+    both_halves(t0 + t1, lo, hi);
+    if (h == 0) tot[r & 1][w][n] = lo + hi;
+    lds_barrier();
+    float before = run;
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      if (k == w) before = run;
+      run += tot[r & 1][k][n];
+    }
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, before), gtab_rs, h == 0 ? entry(r) : OUTSIDE, 0, 0);
+    float dprev = h == 1 ? before + lo : before, dz[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) { const float dj = fmaf(p[j], da[j], dprev); dz[j] = fmaf(m[j], dj, -dprev); dprev = dj; }
+    if (b < n_blocks) {
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) {
+        const el8 zf = pack8(dz + 8 * tt);
+        const unsigned short* const krow = Kr + 16 * tt * D;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) dq[db] = mfma32(lds_tr8(krow + (tbase[0] ^ (db << 5)), krow + (tbase[1] ^ (db << 5))), zf, dq[db]);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+  wait_loads<0>();                              // (copies of nothing into the place that is written now)
+  lds_barrier();
+  add_waves<DB, W>(reinterpret_cast<float*>(smem), dq, w, lane);
+  lds_barrier();
+  store_sum<DB, W>(reinterpret_cast<const float*>(smem), w, lane, a.inv_temp, rows_of(a.dq), qrow, qvalid, h, a.out_f32);
+}
+
+template <int D, bool AC, int U>
+__global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_dkdv_small_kernel(const KArgs a) {
+  constexpr int W = SMALL_WAVES, KS = U / 16, DB = U / 32, TILE = 32 * D, OWN = 4 * TILE + 32 * 32;
+  __shared__ __attribute__((aligned(16))) unsigned short smem[W * OWN];   // per wave: two Q and two dO blocks, p or dz; then the waves' dk and dv
+  static_assert(W * OWN * 2 >= 2 * W * 64 * DB * 16 * 4, "the waves' accumulators fit the tiles' place");
+
+  const int* sched = a.sched;
+  const int part = blockIdx.x / a.heads;
+  const int head = blockIdx.x - part * a.heads;
+  const int slot = part / (BM / 32), sub = part % (BM / 32);
+  const int4 hdr = *reinterpret_cast<const int4*>(sched);   // status, query tiles, key tiles, table entries needed
+  const int longest = sched[SCHED_MAXLEN];
+  const Tile t = reinterpret_cast<const Tile*>(sched + SCHED_HDR)[slot];     // (the key blocks of a query tile's own rows)
+  asm volatile("" ::"s"(t.tok_start), "s"(t.doc_len), "s"(t.idx), "s"(t.batch), "s"(t.tab_base));   // keep the tile read above the branch
+  if (hdr.x != 0 || hdr.w > a.tab_stride || longest > a.max_doc_len || slot >= hdr.y) return;
+  const int L = t.doc_len, k0 = t.idx * BM + 32 * sub, kb = k0 / 32;
+  if (k0 >= L) return;
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, n = lane & 31, h = lane >> 5;
+  const int i16 = lane & 15, blk = (lane >> 4) & 1;
+  const int64_t tok0 = t.tok_start;
+  auto rows_of = [&](const View& v) {
+    return make_rows(reinterpret_cast<const elem_t*>(v.ptr) + t.batch * v.sb + head * v.sh + tok0 * v.st, v.st, L, a.head_dim);
+  };
+  const Rows qrows = rows_of(a.q), grows = rows_of(a.go), krows = rows_of(a.k), vrows = rows_of(a.v);
+  unsigned short* const Qt = smem + w * OWN;            // (two of them)
+  unsigned short* const Gt = Qt + 2 * TILE;
+  unsigned short* const Bt = Gt + 2 * TILE;
+  WaveCopy<D, false> qcopy, gcopy;
+  qcopy.init(lane, qrows.row_bytes, qrows.used_bytes);
+  gcopy.init(lane, grows.row_bytes, grows.used_bytes);
+  const int n_blocks = (L + 31) / 32 - kb;              // query blocks that see these keys
+  auto row_of = [&](int i) { return i < n_blocks ? k0 + 32 * i : L; };   // (outside the document: zeros, nothing is fetched)
+  const unsigned area = 4u * (unsigned)tab_doc_entries(L);
+  float* const stick = a.stick + (int64_t)head * a.tab_stride + t.tab_base;
+  const __amdgpu_buffer_rsrc_t stick_rs = __builtin_amdgcn_make_buffer_rsrc(stick, 0, area, 0x00020000);
+  const __amdgpu_buffer_rsrc_t gtab_rs = __builtin_amdgcn_make_buffer_rsrc(a.gtab + (int64_t)head * a.tab_stride + t.tab_base, 0, area, 0x00020000);
+  auto entry = [&](int i) { const int row = k0 + 32 * i + n; return i < n_blocks && row < L ? 4 * (tab_seg32(L, kb) + row) : OUTSIDE; };
+  float e_next = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(stick_rs, entry(w), 0, 0));
+  float d_next = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(gtab_rs, entry(w), 0, 0));
+  qcopy.issue(qrows, row_of(w), Qt);
+  gcopy.issue(grows, row_of(w), Gt);
+  el8 kf[KS], vf[KS];                           // MFMA row n holds key k0 + kperm(n)
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    kf[ks] = load_frag(krows, k0 + kperm(n), 32 * ks + 16 * h);
+    vf[ks] = load_frag(vrows, k0 + kperm(n), 32 * ks + 16 * h);
+  }
+  float rem_own = 0.0f;                         // fused output: rem_j * do_j reaches dv_j through the diagonal of p (see bwd_dkdv_kernel)
+  if (a.fuse && k0 + n < L) rem_own = stick[(unsigned)(tab_rowplane32(L) + k0 + n)];
+  f32x16 dk[DB], dv[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) dk[db][i] = dv[db][i] = 0.0f;
+  const int qbase = swz_off<D>(n, h);
+  // the private block has rows of 64 bytes, its chunks rotated with row / 4 (see bwd_dkdv_tail_kernel)
+  auto blk_off = [](int row, int chunk) { return row * 32 + ((chunk ^ ((row >> 2) & 3)) << 3); };
+  int xoff[2], ybase[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int row = 8 * h + 4 * u + (i16 >> 2), c = 16 * blk + 4 * (i16 & 3);
+    xoff[u] = blk_off(row, c >> 3) + (c & 7);
+    ybase[u] = swz_off<D>(row, c >> 3) + (c & 7);
+  }
+  wait_loads<0>();
+#pragma unroll 1
+  for (int i = w, buf = 0; i < n_blocks; i += W, buf ^= 1) {
+    wait_loads<0>();
+    const int qw0 = k0 + 32 * i, qrow = qw0 + n;
+    const bool ok = qrow < L;
+    float e_in = ok ? e_next : 1.0f;
+    const float before = ok ? d_next : 0.0f;
+    e_next = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(stick_rs, entry(i + W), 0, 0));
+    d_next = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(gtab_rs, entry(i + W), 0, 0));
+    qcopy.issue(qrows, row_of(i + W), Qt + (buf ^ 1) * TILE);
+    gcopy.issue(grows, row_of(i + W), Gt + (buf ^ 1) * TILE);
+    const unsigned short* const Qr = Qt + buf * TILE;
+    const unsigned short* const Gr = Gt + buf * TILE;
+    f32x16 x, da;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) x[j] = da[j] = 0.0f;
+    {
+      el8 qfr[KS], gfr[KS];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) { qfr[ks] = lds_row8(Qr + (qbase ^ (ks << 4))); gfr[ks] = lds_row8(Gr + (qbase ^ (ks << 4))); }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) { x = mfma32(kf[ks], qfr[ks], x); da = mfma32(vf[ks], gfr[ks], da); }
+    }
+    float p[16], m[16], ends[2];
+    if (i > 0) stick_weights<AC, true, false, true>(x, a.c, k0, qrow, h, e_in, p, m, ends);
+    else stick_weights<AC, true, true, true>(x, a.c, k0, qrow, h, e_in, p, m, ends);
+    float t0 = 0.0f, t1 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 16; j += 2) { t0 = fmaf(p[j], da[j], t0); t1 = fmaf(p[j + 1], da[j + 1], t1); }
+    float lo, hi;
+    both_halves(t0 + t1, lo, hi);
+    float dprev = h == 1 ? before + lo : before, dz[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) { const float dj = fmaf(p[j], da[j], dprev); dz[j] = fmaf(m[j], dj, -dprev); dprev = dj; }
+    if (a.fuse && i == 0) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) p[j] += 16 * h + j == n ? rem_own : 0.0f;
+    }
+    // turn the blocks around, p first: [query][key] rows in, key-major operands out
+    auto turn = [&](const float (&v)[16], el8 (&f)[2]) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c) *reinterpret_cast<el8*>(Bt + blk_off(n, 2 * h + c)) = pack8(v + 8 * c);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) f[ks] = lds_tr8(Bt + xoff[0] + 16 * ks * 32, Bt + xoff[1] + 16 * ks * 32);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+    el8 pf[2], zf[2];
+    turn(p, pf);
+    turn(dz, zf);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        dv[db] = mfma32(lds_tr8(Gr + (ybase[0] ^ (db << 5)) + 16 * ks * D, Gr + (ybase[1] ^ (db << 5)) + 16 * ks * D), pf[ks], dv[db]);
+        dk[db] = mfma32(lds_tr8(Qr + (ybase[0] ^ (db << 5)) + 16 * ks * D, Qr + (ybase[1] ^ (db << 5)) + 16 * ks * D), zf[ks], dk[db]);
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+  wait_loads<0>();                              // (copies of nothing into the place that is written now)
+  lds_barrier();
+  float* const sums = reinterpret_cast<float*>(smem);
+  constexpr int HALF = W * 64 * DB * 16;
+  add_waves<DB, W>(sums, dk, w, lane);
+  add_waves<DB, W>(sums + HALF, dv, w, lane);
+  lds_barrier();
+  store_sum<DB, W>(sums, w, lane, a.inv_temp, rows_of(a.dk), k0 + n, k0 + n < L, h, a.out_f32);
+  store_sum<DB, W>(sums + HALF, w, lane, 1.0f, rows_of(a.dv), k0 + n, k0 + n < L, h, a.out_f32);
+}
+
 #define SBA_SMALL(D, U)                                                   \
   template __global__ void fwd_small_kernel<D, false, U>(const KArgs);    \
-  template __global__ void fwd_small_kernel<D, true, U>(const KArgs);
+  template __global__ void fwd_small_kernel<D, true, U>(const KArgs);     \
+  template __global__ void bwd_dq_small_kernel<D, false, U>(const KArgs);    \
+  template __global__ void bwd_dq_small_kernel<D, true, U>(const KArgs);     \
+  template __global__ void bwd_dkdv_small_kernel<D, false, U>(const KArgs);  \
+  template __global__ void bwd_dkdv_small_kernel<D, true, U>(const KArgs);
 SBA_SMALL(64, 32)
 SBA_SMALL(64, 64)
 SBA_SMALL(128, 96)
 SBA_SMALL(128, 128)
 #undef SBA_SMALL
 
-template <int D, int U>
-static hipError_t launch_fwd_small_d(const KArgs& a, bool ac, int n_q_max, hipStream_t s) {
+enum class SmallPass { FWD, DQ, DKDV };
+template <SmallPass PASS, int D, int U>
+static void launch_small_d(const KArgs& a, bool ac, int n_q_max, hipStream_t s) {
   const dim3 grid((unsigned)n_q_max * (BM / 32) * (unsigned)a.heads), block(SMALL_WAVES * 64);
-  if (ac) hipLaunchKernelGGL((fwd_small_kernel<D, true, U>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((fwd_small_kernel<D, false, U>), grid, block, 0, s, a);
+  auto launch = [&](void (*plain)(KArgs), void (*current)(KArgs)) { hipLaunchKernelGGL(ac ? current : plain, grid, block, 0, s, a); };
+  if constexpr (PASS == SmallPass::FWD) launch(fwd_small_kernel<D, false, U>, fwd_small_kernel<D, true, U>);
+  else if constexpr (PASS == SmallPass::DQ) launch(bwd_dq_small_kernel<D, false, U>, bwd_dq_small_kernel<D, true, U>);
+  else launch(bwd_dkdv_small_kernel<D, false, U>, bwd_dkdv_small_kernel<D, true, U>);
+}
+template <SmallPass PASS>
+static hipError_t launch_small(const KArgs& a, bool ac, int n_q_max, hipStream_t s) {
+  if (a.head_dim <= 32) launch_small_d<PASS, 64, 32>(a, ac, n_q_max, s);
+  else if (a.head_dim <= 64) launch_small_d<PASS, 64, 64>(a, ac, n_q_max, s);
+  else if (used_width(a.head_dim) == 96) launch_small_d<PASS, 128, 96>(a, ac, n_q_max, s);
+  else launch_small_d<PASS, 128, 128>(a, ac, n_q_max, s);
   return hipGetLastError();
 }
-hipError_t launch_fwd_small(const KArgs& a, bool ac, int n_q_max, hipStream_t s) {
-  if (a.head_dim <= 32) return launch_fwd_small_d<64, 32>(a, ac, n_q_max, s);
-  if (a.head_dim <= 64) return launch_fwd_small_d<64, 64>(a, ac, n_q_max, s);
-  if (used_width(a.head_dim) == 96) return launch_fwd_small_d<128, 96>(a, ac, n_q_max, s);
-  return launch_fwd_small_d<128, 128>(a, ac, n_q_max, s);
-}
+hipError_t launch_fwd_small(const KArgs& a, bool ac, int n_q_max, hipStream_t s) { return launch_small<SmallPass::FWD>(a, ac, n_q_max, s); }
+hipError_t launch_bwd_dq_small(const KArgs& a, bool ac, int n_q_max, hipStream_t s) { return launch_small<SmallPass::DQ>(a, ac, n_q_max, s); }
+hipError_t launch_bwd_dkdv_small(const KArgs& a, bool ac, int n_q_max, hipStream_t s) { return launch_small<SmallPass::DKDV>(a, ac, n_q_max, s); }
 
 }  // inline namespace SBA_ELEM_NS
 }  // namespace sba

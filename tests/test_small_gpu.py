@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from oracle import sb_oracle as orc
-from stickbreaking_attention import sb_attn
+from stickbreaking_attention import sb_attn, sb_attn_fused
 from tests.helpers import assert_close, oracle_varlen
 from tests.test_fused_gpu import check, fused_reference
 from tests.test_head_dim_256_gpu import DEV, _need_gpu, _run  # noqa: F401
@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("d,lengths", [(64, [193, 128, 1]), (64, [129, 31, 32, 33]), (64, [255, 257, 300]), (64, [1, 1025]), (32, [500, 129]),
-                                       (8, [385, 384]), (40, [640]), (72, [161, 260]), (96, [513]), (104, [290, 100]), (128, [511, 2]),
+                                       (8, [385, 384]), (40, [640]), (72, [161, 260]), (96, [513]), (104, [290, 100]), (128, [401, 2]),
                                        (128, [256, 255, 257])])
 @pytest.mark.parametrize("ac,fused", [(False, False), (True, False), (False, True), (True, True)])
 def test_packed_edges(d, lengths, ac, fused):
@@ -29,6 +29,41 @@ def test_packed_edges(d, lengths, ac, fused):
 
 
 _ROUND = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 2.0 ** -7}   # one step of the output (float32 inputs round to bfloat16)
+
+
+def _both(shape, dtype, times, layout, ac, fused, with_rem):
+    """Outputs and gradients of a small call, and those of the same heads `times` over."""
+    gen = torch.Generator(device=DEV).manual_seed(shape[-2])
+    B, H, T, d = shape
+    t = [torch.randn((B, T, H, d) if layout == "tokens" else shape, generator=gen, device=DEV).to(dtype) for _ in range(4)]
+    if layout == "tokens":
+        t = [x.transpose(1, 2) for x in t]
+    drem = torch.randn((B, H, T), generator=gen, device=DEV).to(dtype)
+    results = []
+    for n in (1, times):
+        q, k, v, do = (x.repeat(1, n, 1, 1) if n > 1 else x for x in t)
+        q, k, v = (x.detach().requires_grad_() for x in (q, k, v))
+        if fused:
+            out = (sb_attn_fused(q, k, v, attend_current=ac),)
+            grads = torch.autograd.grad(out, (q, k, v), do)
+        else:
+            out = sb_attn(q, k, v, attend_current=ac)
+            grads = torch.autograd.grad(out if with_rem else out[:1], (q, k, v), (do, drem.repeat(1, n, 1)) if with_rem else (do,))
+        results.append([x.detach()[:, :H] for x in out + tuple(grads)])
+    return results
+
+
+@pytest.mark.parametrize("dtype", list(_ROUND))
+@pytest.mark.parametrize("d,batch,T,layout", [(64, 1, 600, "heads"), (64, 2, 257, "tokens"), (32, 3, 130, "heads"), (96, 1, 400, "tokens"), (128, 2, 321, "heads")])
+@pytest.mark.parametrize("ac,fused,with_rem", [(False, False, True), (True, False, False), (False, True, False), (True, True, False)])
+def test_gradients_like_the_general_kernels(d, batch, T, layout, dtype, ac, fused, with_rem):
+    """Both round weights and logit gradients to 16 bits before the same products, from float32 values that differ in the last bits: of the at most T terms
+    of an element some land on the neighbour (one step, independently), and the output may."""
+    small, many = _both((batch, 2, T, d), dtype, 64 * 1024 // T, layout, ac, fused, with_rem)
+    for g, r in zip(small, many):
+        scale = float(r.float().abs().max())
+        torch.testing.assert_close(g, r, rtol=_ROUND[dtype], atol=_ROUND[dtype] / 4 * scale)
+        assert float((g.float() - r.float()).norm()) <= _ROUND[dtype] / 4 * float(r.float().norm())
 
 
 @pytest.mark.parametrize("dtype", list(_ROUND))
