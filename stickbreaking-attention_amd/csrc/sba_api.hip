@@ -197,6 +197,8 @@ int fill_common(const sba_problem* p, bool fixed, const Sizes& sz, const void* s
   a->sched = reinterpret_cast<const int*>(schedule);
   a->kv_list_off = SCHED_HDR + TILE_WORDS * sz.n_q_max;
   a->n_kv_alloc = sz.n_kv_max;
+  a->docs_off = a->kv_list_off + TILE_WORDS * sz.n_kv_max + chain_docs_offset(sz.n_docs);
+  a->n_docs = sz.n_docs;
   a->heads = p->heads;
   a->head_dim = p->head_dim;
   a->tokens = p->tokens;
@@ -237,6 +239,23 @@ bool backward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
   if (backward_form() != 0 || g_dkdv_workgroups.load() != 0 || declared_max_doc_len(p, fixed) <= 64) return false;
   static constexpr SmallCost COSTS[3] = {{16.0, 1.04, 12.5, 1.9, 3.7, 2.35, 512}, {17.0, 1.15, 14.0, 2.34, 6.0, 2.75, 512}, {19.0, 1.42, 18.5, 3.6, 9.5, 3.6, 256}};
   return small_wins(COSTS, 1.05, p, fixed, sz);
+}
+
+// Where bwd_short_kernel (sba_small.hip) is the faster one: short documents, and enough of them for a wave on two of three SIMDs (a wave has 64
+// tokens; dq and dk/dv passes / one-pass form before, us, at head_dim 64: 32 heads of 8 x 256 tokens 44.5 / 31.6, of 32 x 128 49.6 / 35.3, of
+// 128 x 33 75 / 45.5, of 128 x 256 390 / 322, 8 heads of 5000 tokens in documents of 1 .. 256 33.6 / 30.3; left out: 4 heads of 128 x 64 20.1 / 19.9, of
+// 32 x 64 16.6 / 19.0).
+bool backward_short(const sba_problem* p, bool fixed, const Sizes& sz) {
+  if (backward_form() != 0 || g_dkdv_workgroups.load() != 0) return false;
+  return (p->flags & SBA_PRODUCT_SPACE) && p->head_dim <= 64 && sz.n_docs > 0 && sz.n_docs <= RANK_LIMIT && declared_max_doc_len(p, fixed) <= 32 * SHORT_BLOCKS &&
+         sz.rows * p->heads >= 40000;
+}
+// Workgroups per head: documents of more than 128 tokens one each, the others two or four (each class rounded up).
+int short_parts(const sba_problem* p, bool fixed, const Sizes& sz) {
+  const int longest = declared_max_doc_len(p, fixed);
+  if (longest <= 64) return (sz.n_docs + 3) / 4;
+  const long long alone = longest <= 128 ? 0 : std::min<long long>(sz.n_docs, sz.rows / 129);
+  return (int)(alone + (sz.n_docs - alone + 1) / 2 + 1);
 }
 
 int forward(const sba_problem* p, bool fixed, const void* schedule, size_t sched_bytes, const sba_view* q,
@@ -315,6 +334,10 @@ int backward(const sba_problem* p, bool fixed, const void* schedule, size_t sche
   a.clear_spare = fixed ? 0 : 1;
   a.nan_pair = p->dtype == SBA_F16 && !a.out_f32 ? 0x7e007e00u : 0x7fc07fc0u;
   hipError_t he = hipSuccess;
+  if (backward_short(p, fixed, sz)) {
+    Timer tm(2, s);
+    return (int)(p->dtype == SBA_F16 ? f16::launch_bwd_short : bf16::launch_bwd_short)(a, ac, short_parts(p, fixed, sz), s);
+  }
   if (backward_small(p, fixed, sz)) {
     {
       Timer tm(1, s);
@@ -378,7 +401,7 @@ bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
   const int form = backward_form();
   if (form == 1 || g_dkdv_workgroups.load() != 0 || !chain_possible(p, fixed, sz)) return false;
   if (form == 2 || form == 3) return true;
-  if (backward_small(p, fixed, sz)) return false;
+  if (backward_short(p, fixed, sz) || backward_small(p, fixed, sz)) return false;
   const long long chains = (long long)sz.n_docs * p->heads, items = (long long)sz.n_kv_max * p->heads;
   const long long mean = sz.rows / sz.n_docs, longest = declared_max_doc_len(p, fixed);
   // a document of one or two steps: nothing to hand on, and one launch more (0.85 .. 1.01)
@@ -434,7 +457,7 @@ int backward_chained(const sba_problem* p, bool fixed, const void* schedule, siz
   a.queues = reinterpret_cast<unsigned*>(base + at.queues);
   a.homes = reinterpret_cast<int*>(base + at.homes);
   a.tab_stride = c.tab_stride;
-  a.docs_off = SCHED_HDR + TILE_WORDS * (sz.n_q_max + sz.n_kv_max) + chain_docs_offset(sz.n_docs);
+  a.docs_off = c.docs_off;
   a.n_docs = sz.n_docs;
   a.heads = p->heads;
   a.head_dim = p->head_dim;

@@ -31,6 +31,7 @@ typedef __attribute__((ext_vector_type(8))) short s16x8;
 
 constexpr int BM = 128;  // query rows per workgroup tile (4 waves x 32 rows)
 constexpr int SMALL_WAVES = 4;   // waves of a workgroup of sba_small.hip
+constexpr int SHORT_BLOCKS = 8;  // bwd_short_kernel: most blocks of 32 tokens of a document
 constexpr int BN = 64;   // keys per KV tile staged in LDS by the dq pass
 constexpr int BKV = 128;  // keys owned by one workgroup of the dk/dv pass
 constexpr int BT = 32;   // keys per carry-table entry (one MFMA sub-block)
@@ -53,11 +54,13 @@ constexpr int SCHED_TABLE = 3;   // carry-table entries per head the documents n
 constexpr int SCHED_TOTAL = 4;   // tokens covered by the documents (0 when the input is rejected)
 constexpr int SCHED_MAXLEN = 6;  // longest document found (read together with the next word: keep the pair 8-byte aligned)
 constexpr int SCHED_NKV_LONG = 7; // key tiles of the first group of the key-tile list (see kv_tail_tiles)
+constexpr int SCHED_OVER_64 = 8;   // documents of more than 64 tokens
+constexpr int SCHED_OVER_128 = 9;  // documents of more than 128 tokens
 constexpr int SCHED_HDR = 16;    // tile lists start here
 constexpr int TILE_WORDS = 8;    // int32 words of one Tile
 constexpr int RANK_LIMIT = 4096; // beyond this many documents the input order is kept
 // Behind the two tile lists: 6 n_docs + 2 words of the scheduler's, of which the ranked documents take the last
-// 4 n_docs once it is done (8-byte aligned: the lists are whole 32-byte tiles).
+// 4 n_docs once it is done (16-byte aligned: the lists are whole 32-byte tiles).
 __host__ __device__ inline int chain_docs_offset(int n_docs) { return (2 * n_docs + 3) & ~3; }
 
 struct Tile {

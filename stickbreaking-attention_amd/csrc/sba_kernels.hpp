@@ -15,6 +15,7 @@ struct KArgs {
   const int* sched;            // schedule workspace
   int kv_list_off;             // int32 offset of the KV tile list inside `sched`
   int n_kv_alloc;              // tiles that list has room for (no launch may index it beyond)
+  int docs_off, n_docs;        // the ranked documents in the schedule, if there are at most RANK_LIMIT
   float* stick;                // carry table written by the forward (may be null in fwd): per (row, 32-key block) the
                                // stick left on entering the block; per-row plane: rem in fp32
   float* gtab;                 // gradient prefix table (backward scratch); per-row plane: the full d(rem)
@@ -180,6 +181,7 @@ inline bool has_dkdv_tail_kernel(int head_dim) { return head_dim <= 64; }
   hipError_t launch_bwd_dq_wide(const KArgs& a, bool attend_current, bool product, int n_q_max, hipStream_t s);   \
   hipError_t launch_bwd_dkdv_wide(const KArgs& a, bool attend_current, bool product, int tiles, hipStream_t s);   \
   hipError_t launch_fwd_small(const KArgs& a, bool attend_current, int n_q_max, hipStream_t s);                  \
+  hipError_t launch_bwd_short(const KArgs& a, bool attend_current, int parts, hipStream_t s);                  \
   hipError_t launch_bwd_dq_small(const KArgs& a, bool attend_current, int n_q_max, hipStream_t s);                  \
   hipError_t launch_bwd_dkdv_small(const KArgs& a, bool attend_current, int n_q_max, hipStream_t s);                  \
   hipError_t launch_bwd_chain(const ChainArgs& a, bool attend_current, bool wide, int n_q_max, int workgroups,              \

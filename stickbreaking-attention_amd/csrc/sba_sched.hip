@@ -17,7 +17,7 @@ __device__ __forceinline__ int cdiv(int a, int b) { return (a + b - 1) / b; }
 // and every phase boundary is a workgroup barrier, which costs by the wave).
 template <int SCHED_THREADS>
 __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a) {
-  __shared__ int s_status, s_maxlen;
+  __shared__ int s_status, s_maxlen, s_over_64, s_over_128;
   __shared__ int s_scan_q[SCHED_THREADS], s_scan_kv[SCHED_THREADS], s_scan_ne[SCHED_THREADS];
   __shared__ long long s_scan_tab[SCHED_THREADS];
   // Lengths, ranking and tile-count prefixes of up to RANK_LIMIT documents are kept in LDS: the
@@ -47,7 +47,7 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
   int* const start_of = in_lds ? s_start : dstart;    // by document index: first token
   int* const tab_of = in_lds ? s_tab : dtab;          // by document index: first carry-table entry
 
-  if (tid == 0) { s_status = 0; s_maxlen = 0; }
+  if (tid == 0) s_status = s_maxlen = s_over_64 = s_over_128 = 0;
   __syncthreads();
 
   // A. document bounds + validation
@@ -74,6 +74,8 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
     dlen[d] = len;
     if (in_lds) s_len[d] = len;
     atomicMax(&s_maxlen, len);
+    if (len > 64) atomicAdd(&s_over_64, 1);
+    if (len > 128) atomicAdd(&s_over_128, 1);
   }
   __syncthreads();
 
@@ -230,7 +232,7 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
     kvtiles[s] = t;
   }
   // E. the documents in ranked order, {first token, length, first table entry, 128-row tiles before}: what the one-pass
-  // backward names its chains by.  With the working arrays in LDS their places in the workspace are free.
+  // backward names its chains by and bwd_short_kernel goes by.  With the working arrays in LDS their places in the workspace are free.
   if (in_lds && ok) {
     int2* const docs = reinterpret_cast<int2*>(dstart + chain_docs_offset(nd));
     for (int i = tid; i < nd; i += SCHED_THREADS) {
@@ -245,6 +247,8 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
     hdr[SCHED_NKV] = ok ? total_kv : 0;
     hdr[SCHED_NKV_LONG] = ok ? total_long : 0;
     hdr[SCHED_MAXLEN] = s_maxlen;
+    hdr[SCHED_OVER_64] = s_over_64;
+    hdr[SCHED_OVER_128] = s_over_128;
     hdr[SCHED_TABLE] = tab_ok ? (int)total_tab : 0x7fffffff;
     hdr[SCHED_TOTAL] = (ok && nd > 0) ? dstart[nd - 1] + dlen[nd - 1] : 0;
   }

@@ -527,6 +527,263 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_dkdv_sm
   store_sum<DB, W>(sums + HALF, w, lane, 1.0f, rows_of(a.dv), k0 + n, k0 + n < L, h, a.out_f32);
 }
 
+// -------------------------------------------------------------------------------------------
+// Backward of documents of at most 32 x SHORT_BLOCKS tokens, head_dim <= 64, both passes in one: a team of waves takes one (document, head),
+// half as many waves as it has blocks of 32 tokens, and a workgroup has one team of four, two of two or four of one.  K and V
+// go to LDS; every wave walks the keys of its own queries, oldest first, for dq, and leaves the running sum D of every block of
+// 32 x 32 in LDS.  Then Q and dO, which the waves hold as their own operands, take the place of K and V, and the waves own keys.
+// Query block i takes i + 1 steps, key block i of n takes n - i: with blocks w and n - 1 - w a wave has n + 1 in either half.
+// What bounds it: the two passes it stands in for ran at the rate of a copy, four operands read by each and the sums D written and read
+// between them; here operands come in once (32 heads x 16 K tokens in documents of 16 .. 256: 228 us for 161, of which 94 are its traffic).  What is
+// left is that a workgroup loads, computes and stores one after the other, two of them (8 waves of 220 registers, 77 KB of LDS) per compute unit.  One document
+// to a workgroup whatever its length: 204 us, most waves idle; four slots of the tile list to a workgroup, long documents one after the other: 166 us,
+// and 104 for 31 us where there are few of them.
+// -------------------------------------------------------------------------------------------
+template <bool AC, int U>
+__global__ void __launch_bounds__(SMALL_WAVES * 64, 2) bwd_short_kernel(const KArgs a) {
+  constexpr int D = 64, W = SMALL_WAVES, KS = U / 16, DB = U / 32, TILE = 32 * D, NB = SHORT_BLOCKS;
+  static_assert(NB == 2 * W && W == 4, "two blocks for each wave");
+  __shared__ __attribute__((aligned(16))) unsigned short smem[2 * NB * TILE + W * 32 * 32];   // K, V blocks, Q, dO blocks in their place; p or dz of a wave
+  __shared__ float sums[NB * (NB + 1) / 2 * 32];                  // D in front of key block b, from its own queries on
+
+  const int* sched = a.sched;
+  const int part = blockIdx.x / a.heads;
+  const int head = blockIdx.x - part * a.heads;
+  const int4 hdr = *reinterpret_cast<const int4*>(sched);   // status, query tiles, key tiles, table entries needed
+  const int total = sched[SCHED_TOTAL], longest = sched[SCHED_MAXLEN], over_64 = sched[SCHED_OVER_64], over_128 = sched[SCHED_OVER_128];
+  const int tid = threadIdx.x;
+  const bool refused = hdr.x != 0 || hdr.w > a.tab_stride || longest > a.max_doc_len;
+  if (a.clear_spare && (refused || total < a.tokens)) {     // every workgroup clears its share
+    const int from = refused ? 0 : total, share = (a.tokens - from + (int)gridDim.x / a.heads - 1) / ((int)gridDim.x / a.heads);
+    const int row0 = min(from + part * share, a.tokens), row1 = min(row0 + share, a.tokens);
+    const unsigned pair = refused ? a.nan_pair : 0u;
+    fill_rows16(a.dq, head, row0, row1, a.head_dim << a.out_f32, pair, tid, W * 64);
+    fill_rows16(a.dk, head, row0, row1, a.head_dim << a.out_f32, pair, tid, W * 64);
+    fill_rows16(a.dv, head, row0, row1, a.head_dim << a.out_f32, pair, tid, W * 64);
+  }
+  if (refused || longest > 32 * NB) return;     // (the second: not reached, a.max_doc_len is no more)
+  // The documents are ranked, longest first: one for a workgroup, then two, then four.
+  const int pairs = (over_64 - over_128 + 1) / 2;
+  const int team_waves = part < over_128 ? W : (part - over_128 < pairs ? W / 2 : W / 4), teams = W / team_waves;
+  const int doc0 = part < over_128 ? part : (part - over_128 < pairs ? over_128 + 2 * (part - over_128) : over_64 + 4 * (part - over_128 - pairs));
+  const int doc_end = min(doc0 + teams, part < over_128 ? over_128 : (part - over_128 < pairs ? over_64 : a.n_docs));
+  if (doc0 >= doc_end) return;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int team = w / team_waves, tw = w - team * team_waves;
+  const int lane = tid & 63, n = lane & 31, h = lane >> 5;
+  const int i16 = lane & 15, blk = (lane >> 4) & 1;
+  unsigned short* const At = smem + 2 * team * team_waves * TILE;
+  unsigned short* const Bt = At + NB * TILE;
+  unsigned short* const own = smem + 2 * NB * TILE + w * 32 * 32;
+  float* const team_sums = sums + team * (NB * (NB + 1) / 2 * 32) / teams;
+  auto sum_at = [&](int b, int q) { return 64 * team_waves * b - 16 * b * (b + 1) + q; };   // (a block's row begins at its own queries)
+  const int rowbase = swz_off<D>(n, h);
+  int xoff[2], ybase[2], tbase[2];
+  auto blk_off = [](int row, int chunk) { return row * 32 + ((chunk ^ ((row >> 2) & 3)) << 3); };   // (see bwd_dkdv_tail_kernel)
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int c = 16 * blk + 4 * (i16 & 3), row = 8 * h + 4 * u + (i16 >> 2);
+    tbase[u] = swz_off<D>(8 * u + 4 * h + (i16 >> 2), c >> 3) + (c & 7);
+    xoff[u] = blk_off(row, c >> 3) + (c & 7);
+    ybase[u] = swz_off<D>(row, c >> 3) + (c & 7);
+  }
+
+  const int doc = min(doc0 + team, doc_end - 1);
+  const int4 about = reinterpret_cast<const int4*>(sched + a.docs_off)[doc];   // first token, length, first table entry
+  const int L = doc0 + team < doc_end ? about.y : 0, n_blocks = (L + 31) / 32, batch = a.clear_spare ? 0 : doc;   // (fixed length: by batch entry)
+  const int64_t tok0 = about.x;
+  auto rows_of = [&](const View& v) {
+    return make_rows(reinterpret_cast<const elem_t*>(v.ptr) + batch * v.sb + head * v.sh + tok0 * v.st, v.st, L, a.head_dim);
+  };
+  const Rows krows = rows_of(a.k), vrows = rows_of(a.v);
+  // a wave's blocks (none: -1)
+  const int block_of[2] = {tw < n_blocks ? tw : -1, n_blocks - 1 - tw >= team_waves ? n_blocks - 1 - tw : -1};
+  {
+    WaveCopy<D, true> kcopy, vcopy;
+    kcopy.init(lane, krows.row_bytes, krows.used_bytes);
+    vcopy.init(lane, vrows.row_bytes, vrows.used_bytes);
+#pragma unroll
+    for (int turn = 0; turn < 2; ++turn) {
+      const int b = block_of[turn];
+      if (b < 0) break;
+      kcopy.issue(krows, 32 * b, At + b * TILE);
+      vcopy.issue(vrows, 32 * b, Bt + b * TILE);
+    }
+  }
+  el8 qf[2][KS], gf[2][KS];
+  {
+    const Rows qrows = rows_of(a.q), grows = rows_of(a.go);
+#pragma unroll
+    for (int turn = 0; turn < 2; ++turn)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int row = block_of[turn] >= 0 ? 32 * block_of[turn] + n : L;   // (outside the document: zeros)
+        qf[turn][ks] = load_frag(qrows, row, 32 * ks + 16 * h);
+        gf[turn][ks] = load_frag(grows, row, 32 * ks + 16 * h);
+      }
+  }
+  float* const stick = a.stick + (int64_t)head * a.tab_stride + about.z;
+  const __amdgpu_buffer_rsrc_t stick_rs = __builtin_amdgcn_make_buffer_rsrc(stick, 0, 4u * (unsigned)tab_doc_entries(L), 0x00020000);
+  // stick left in front of key block b for row `row`
+  auto stick_at = [&](int b, int row, bool ok) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(stick_rs, ok && row < L ? 4 * (tab_seg32(L, b) + row) : OUTSIDE, 0, 0));
+  };
+  wait_loads<0>();
+  lds_barrier();
+
+  // ---- dq ----
+#pragma unroll
+  for (int turn = 0; turn < 2; ++turn) {
+    const int qb = block_of[turn];
+    if (qb >= 0) {
+      const int qrow = 32 * qb + n;
+      const bool qvalid = qrow < L;
+      float e_next = stick_at(0, qrow, true), run;
+      {                                       // D in front of the oldest key (see bwd_dq_small_kernel)
+        float dr = 0.0f;
+        if (a.grem.ptr != nullptr && qvalid)
+          dr = (float)(reinterpret_cast<const elem_t*>(a.grem.ptr) + batch * a.grem.sb + head * a.grem.sh + tok0 * a.grem.st)[(int64_t)qrow * a.grem.st];
+        if (a.fuse) {
+          float dot = 0.0f;
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) {
+            const el8 vown = load_frag(vrows, qrow, 32 * ks + 16 * h);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dot = fmaf((float)gf[turn][ks][e], (float)vown[e], dot);
+          }
+          float lo, hi;
+          both_halves(dot, lo, hi);
+          dr += lo + hi;
+        }
+        run = qvalid ? dr * stick[(unsigned)(tab_rowplane32(L) + qrow)] : 0.0f;
+      }
+      f32x16 dq[DB];
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dq[db][i] = 0.0f;
+#pragma unroll 1
+      for (int b = 0; b <= qb; ++b) {
+        const unsigned short* const Kr = At + b * TILE;
+        const unsigned short* const Vr = Bt + b * TILE;
+        float c = qvalid ? e_next : 1.0f;
+        e_next = stick_at(b + 1, qrow, b < qb);
+        if (h == 0) team_sums[sum_at(b, qrow)] = run;
+        f32x16 x, da;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i] = da[i] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          x = mfma32(lds_row8(Kr + (rowbase ^ (ks << 4))), qf[turn][ks], x);
+          da = mfma32(lds_row8(Vr + (rowbase ^ (ks << 4))), gf[turn][ks], da);
+        }
+        float p[16], m[16], ends[2];
+        grad_weights<AC, true>(x, a.c, 32 * b, 32 * qb, qrow, h, c, p, m, ends);
+        el8 zf[2];
+        grad_dz<true>(p, m, da, ends, h, run, 0.0f, zf);
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+          for (int db = 0; db < DB; ++db)
+            dq[db] = mfma32(lds_tr8(Kr + 16 * tt * D + (tbase[0] ^ (db << 5)), Kr + 16 * tt * D + (tbase[1] ^ (db << 5))), zf[tt], dq[db]);
+      }
+      store_rows(dq, a.inv_temp, rows_of(a.dq), qrow, L, h, a.out_f32);
+    }
+  }
+
+  // ---- dk, dv ----
+  el8 kf[KS], vf[KS];                         // MFMA row n holds key 32 b + kperm(n)
+  {
+    const int at = max(block_of[0], 0) * TILE;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) { kf[ks] = lds_row8(At + at + (rowbase ^ (ks << 4))); vf[ks] = lds_row8(Bt + at + (rowbase ^ (ks << 4))); }
+  }
+  lds_barrier();                              // K and V have been read
+#pragma unroll
+  for (int turn = 0; turn < 2; ++turn)
+    if (block_of[turn] >= 0) {
+      const int at = block_of[turn] * TILE;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        *reinterpret_cast<el8*>(At + at + (rowbase ^ (ks << 4))) = qf[turn][ks];
+        *reinterpret_cast<el8*>(Bt + at + (rowbase ^ (ks << 4))) = gf[turn][ks];
+      }
+    }
+  lds_barrier();
+#pragma unroll 1
+  for (int turn = 0; turn < 2; ++turn) {
+    const int kb = turn == 0 ? block_of[0] : block_of[1];
+    if (kb < 0) break;
+    const int k0 = 32 * kb;
+    float rem_own = 0.0f;                     // fused output: rem_j * do_j reaches dv_j through the diagonal of p (see bwd_dkdv_kernel)
+    if (a.fuse && k0 + n < L) rem_own = stick[(unsigned)(tab_rowplane32(L) + k0 + n)];
+    f32x16 dk[DB], dv[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dk[db][i] = dv[db][i] = 0.0f;
+    float e_next = stick_at(kb, k0 + n, true);
+#pragma unroll 1
+    for (int b = kb; b < n_blocks; ++b) {
+      const int qrow = 32 * b + n;
+      const bool ok = qrow < L;
+      const float c = ok ? e_next : 1.0f;
+      float before = ok ? team_sums[sum_at(kb, qrow)] : 0.0f;
+      e_next = stick_at(kb, qrow + 32, true);
+      const unsigned short* const Qr = At + b * TILE;
+      const unsigned short* const Gr = Bt + b * TILE;
+      f32x16 x, da;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] = da[i] = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        x = mfma32(kf[ks], lds_row8(Qr + (rowbase ^ (ks << 4))), x);
+        da = mfma32(vf[ks], lds_row8(Gr + (rowbase ^ (ks << 4))), da);
+      }
+      float p[16], m[16], ends[2], carry = c;
+      grad_weights<AC, true>(x, a.c, k0, 32 * b, qrow, h, carry, p, m, ends);
+      el8 pz[2], f[2];
+      grad_dz<true>(p, m, da, ends, h, before, 0.0f, pz);
+      // turn the blocks around, dz first: [query][key] rows in, key-major operands out
+      auto turned = [&] {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) *reinterpret_cast<el8*>(own + blk_off(n, 2 * h + k)) = pz[k];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) f[ks] = lds_tr8(own + xoff[0] + 16 * ks * 32, own + xoff[1] + 16 * ks * 32);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      };
+      turned();
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+          dk[db] = mfma32(lds_tr8(Qr + (ybase[0] ^ (db << 5)) + 16 * ks * D, Qr + (ybase[1] ^ (db << 5)) + 16 * ks * D), f[ks], dk[db]);
+      if (a.fuse && b == kb) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) p[j] += 16 * h + j == n ? rem_own : 0.0f;
+      }
+#pragma unroll
+      for (int k = 0; k < 2; ++k) pz[k] = pack8(p + 8 * k);
+      turned();
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+          dv[db] = mfma32(lds_tr8(Gr + (ybase[0] ^ (db << 5)) + 16 * ks * D, Gr + (ybase[1] ^ (db << 5)) + 16 * ks * D), f[ks], dv[db]);
+    }
+    if (turn == 0 && block_of[1] >= 0) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        kf[ks] = load_frag(krows, 32 * block_of[1] + kperm(n), 32 * ks + 16 * h);
+        vf[ks] = load_frag(vrows, 32 * block_of[1] + kperm(n), 32 * ks + 16 * h);
+      }
+    }
+    store_rows(dk, a.inv_temp, rows_of(a.dk), k0 + n, L, h, a.out_f32);
+    store_rows(dv, 1.0f, rows_of(a.dv), k0 + n, L, h, a.out_f32);
+  }
+}
+
 #define SBA_SMALL(D, U)                                                   \
   template __global__ void fwd_small_kernel<D, false, U>(const KArgs);    \
   template __global__ void fwd_small_kernel<D, true, U>(const KArgs);     \
@@ -539,6 +796,10 @@ SBA_SMALL(64, 64)
 SBA_SMALL(128, 96)
 SBA_SMALL(128, 128)
 #undef SBA_SMALL
+template __global__ void bwd_short_kernel<false, 32>(const KArgs);
+template __global__ void bwd_short_kernel<true, 32>(const KArgs);
+template __global__ void bwd_short_kernel<false, 64>(const KArgs);
+template __global__ void bwd_short_kernel<true, 64>(const KArgs);
 
 enum class SmallPass { FWD, DQ, DKDV };
 template <SmallPass PASS, int D, int U>
@@ -560,6 +821,14 @@ static hipError_t launch_small(const KArgs& a, bool ac, int n_q_max, hipStream_t
 hipError_t launch_fwd_small(const KArgs& a, bool ac, int n_q_max, hipStream_t s) { return launch_small<SmallPass::FWD>(a, ac, n_q_max, s); }
 hipError_t launch_bwd_dq_small(const KArgs& a, bool ac, int n_q_max, hipStream_t s) { return launch_small<SmallPass::DQ>(a, ac, n_q_max, s); }
 hipError_t launch_bwd_dkdv_small(const KArgs& a, bool ac, int n_q_max, hipStream_t s) { return launch_small<SmallPass::DKDV>(a, ac, n_q_max, s); }
+
+hipError_t launch_bwd_short(const KArgs& a, bool ac, int parts, hipStream_t s) {
+  const dim3 grid((unsigned)parts * (unsigned)a.heads), block(SMALL_WAVES * 64);
+  auto launch = [&](void (*plain)(KArgs), void (*current)(KArgs)) { hipLaunchKernelGGL(ac ? current : plain, grid, block, 0, s, a); };
+  if (a.head_dim <= 32) launch(bwd_short_kernel<false, 32>, bwd_short_kernel<true, 32>);
+  else launch(bwd_short_kernel<false, 64>, bwd_short_kernel<true, 64>);
+  return hipGetLastError();
+}
 
 }  // inline namespace SBA_ELEM_NS
 }  // namespace sba
