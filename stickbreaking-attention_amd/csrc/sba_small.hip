@@ -528,20 +528,20 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_dkdv_sm
 }
 
 // -------------------------------------------------------------------------------------------
-// Backward of documents of at most 32 x SHORT_BLOCKS tokens, head_dim <= 64, both passes in one: a team of waves takes one (document, head),
+// Backward of documents of at most 32 x SHORT_BLOCKS tokens, both passes in one: a team of waves takes one (document, head),
 // half as many waves as it has blocks of 32 tokens, and a workgroup has one team of four, two of two or four of one.  K and V
 // go to LDS; every wave walks the keys of its own queries, oldest first, for dq, and leaves the running sum D of every block of
 // 32 x 32 in LDS.  Then Q and dO, which the waves hold as their own operands, take the place of K and V, and the waves own keys.
 // Query block i takes i + 1 steps, key block i of n takes n - i: with blocks w and n - 1 - w a wave has n + 1 in either half.
 // What bounds it: the two passes it stands in for ran at the rate of a copy, four operands read by each and the sums D written and read
 // between them; here operands come in once (32 heads x 16 K tokens in documents of 16 .. 256: 228 us for 161, of which 94 are its traffic).  What is
-// left is that a workgroup loads, computes and stores one after the other, two of them (8 waves of 220 registers, 77 KB of LDS) per compute unit.  One document
+// left is that a workgroup loads, computes and stores one after the other, two of them (8 waves of 220 registers, 77 KB of LDS) per compute unit, one above head_dim 64.  One document
 // to a workgroup whatever its length: 204 us, most waves idle; four slots of the tile list to a workgroup, long documents one after the other: 166 us,
 // and 104 for 31 us where there are few of them.
 // -------------------------------------------------------------------------------------------
-template <bool AC, int U>
-__global__ void __launch_bounds__(SMALL_WAVES * 64, 2) bwd_short_kernel(const KArgs a) {
-  constexpr int D = 64, W = SMALL_WAVES, KS = U / 16, DB = U / 32, TILE = 32 * D, NB = SHORT_BLOCKS;
+template <int D, bool AC, int U>
+__global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_kernel(const KArgs a) {
+  constexpr int W = SMALL_WAVES, KS = U / 16, DB = U / 32, TILE = 32 * D, NB = SHORT_BLOCKS;
   static_assert(NB == 2 * W && W == 4, "two blocks for each wave");
   __shared__ __attribute__((aligned(16))) unsigned short smem[2 * NB * TILE + W * 32 * 32];   // K, V blocks, Q, dO blocks in their place; p or dz of a wave
   __shared__ float sums[NB * (NB + 1) / 2 * 32];                  // D in front of key block b, from its own queries on
@@ -790,16 +790,14 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, 2) bwd_short_kernel(const KA
   template __global__ void bwd_dq_small_kernel<D, false, U>(const KArgs);    \
   template __global__ void bwd_dq_small_kernel<D, true, U>(const KArgs);     \
   template __global__ void bwd_dkdv_small_kernel<D, false, U>(const KArgs);  \
-  template __global__ void bwd_dkdv_small_kernel<D, true, U>(const KArgs);
+  template __global__ void bwd_dkdv_small_kernel<D, true, U>(const KArgs);   \
+  template __global__ void bwd_short_kernel<D, false, U>(const KArgs);       \
+  template __global__ void bwd_short_kernel<D, true, U>(const KArgs);
 SBA_SMALL(64, 32)
 SBA_SMALL(64, 64)
 SBA_SMALL(128, 96)
 SBA_SMALL(128, 128)
 #undef SBA_SMALL
-template __global__ void bwd_short_kernel<false, 32>(const KArgs);
-template __global__ void bwd_short_kernel<true, 32>(const KArgs);
-template __global__ void bwd_short_kernel<false, 64>(const KArgs);
-template __global__ void bwd_short_kernel<true, 64>(const KArgs);
 
 enum class SmallPass { FWD, DQ, DKDV };
 template <SmallPass PASS, int D, int U>
@@ -825,8 +823,10 @@ hipError_t launch_bwd_dkdv_small(const KArgs& a, bool ac, int n_q_max, hipStream
 hipError_t launch_bwd_short(const KArgs& a, bool ac, int parts, hipStream_t s) {
   const dim3 grid((unsigned)parts * (unsigned)a.heads), block(SMALL_WAVES * 64);
   auto launch = [&](void (*plain)(KArgs), void (*current)(KArgs)) { hipLaunchKernelGGL(ac ? current : plain, grid, block, 0, s, a); };
-  if (a.head_dim <= 32) launch(bwd_short_kernel<false, 32>, bwd_short_kernel<true, 32>);
-  else launch(bwd_short_kernel<false, 64>, bwd_short_kernel<true, 64>);
+  if (a.head_dim <= 32) launch(bwd_short_kernel<64, false, 32>, bwd_short_kernel<64, true, 32>);
+  else if (a.head_dim <= 64) launch(bwd_short_kernel<64, false, 64>, bwd_short_kernel<64, true, 64>);
+  else if (used_width(a.head_dim) == 96) launch(bwd_short_kernel<128, false, 96>, bwd_short_kernel<128, true, 96>);
+  else launch(bwd_short_kernel<128, false, 128>, bwd_short_kernel<128, true, 128>);
   return hipGetLastError();
 }
 

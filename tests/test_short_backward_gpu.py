@@ -1,4 +1,4 @@
-"""Many short documents take one kernel for the whole backward at head_dim <= 64 (bwd_short_kernel): lengths on either side of its blocks of 32
+"""Many short documents take one kernel for the whole backward (bwd_short_kernel; above head_dim 64 those of up to 64 tokens): lengths on either side of its blocks of 32
 and of its teams (64, 128, 256 tokens), classes that do not fill a workgroup, in every form, against the oracle and the general two passes."""
 import random
 
@@ -17,7 +17,8 @@ EDGES = [256, 1, 255, 225, 64, 129, 128, 0, 127, 97, 96, 65, 63, 224, 33, 32, 31
 _ROUND = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 2.0 ** -7}   # one step of the output (float32 inputs round to bfloat16)
 
 
-@pytest.mark.parametrize("d,lengths", [(64, EDGES), (32, EDGES), (40, [64] * 21), (8, [128, 1] * 11), (64, [128, 65, 64] * 5 + [33]), (64, [17] * 99)])
+@pytest.mark.parametrize("d,lengths", [(64, EDGES), (32, EDGES), (40, [64] * 21), (8, [128, 1] * 11), (64, [128, 65, 64] * 5 + [33]), (64, [17] * 99),
+                                       (128, [64, 1, 63, 33, 32, 31, 0, 2] * 3 + [17]), (72, [64] * 9), (96, [33, 7] * 10)])
 @pytest.mark.parametrize("ac,fused", [(False, False), (True, False), (False, True), (True, True)])
 def test_against_the_oracle(d, lengths, ac, fused):
     T, H = sum(lengths), 40000 // sum(lengths) + 1
@@ -32,7 +33,8 @@ def test_against_the_oracle(d, lengths, ac, fused):
 
 
 @pytest.mark.parametrize("dtype", list(_ROUND))
-@pytest.mark.parametrize("d,shape,layout", [(64, None, "heads"), (48, None, "tokens"), (64, (5, 250), "tokens"), (32, (70, 70), "heads"), (24, (9, 128), "heads")])
+@pytest.mark.parametrize("d,shape,layout", [(64, None, "heads"), (48, None, "tokens"), (64, (5, 250), "tokens"), (32, (70, 70), "heads"), (24, (9, 128), "heads"),
+                                            (128, (33, 50), "heads"), (80, (20, 64), "tokens")])
 @pytest.mark.parametrize("ac,fused,zero_start", [(False, False, False), (True, False, True), (False, True, True)])
 def test_like_the_two_passes(d, shape, layout, dtype, ac, fused, zero_start, form):  # noqa: F811
     """Weights and logit gradients are rounded to 16 bits before the same products, from float32 values that differ in the last bits: now and then a
