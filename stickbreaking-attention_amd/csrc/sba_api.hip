@@ -282,8 +282,10 @@ int forward(const sba_problem* p, bool fixed, const void* schedule, size_t sched
   else { a.v = to_view(v); a.o = to_view_out(o, p); a.rem = to_view_out(rem, p); }
   a.stick = stick;
   a.weights = weights;
-  a.resident = device_cus();
-  a.n_items = (int)std::min<long long>(0x7fffffff, (fixed ? (long long)p->batch * ((p->tokens + BM - 1) / BM) : sz.rows / BM) * p->heads);
+  // (the grid may hold a few slots more than there are items)
+  const long long cus = device_cus(), items = (fixed ? (long long)p->batch * ((p->tokens + BM - 1) / BM) : sz.rows / BM) * p->heads;
+  a.resident = items > cus && items <= fwd_per_cu(p->head_dim) * cus ? (int)cus : NO_DEAL;
+  a.n_items = (int)std::min<long long>(0x7fffffff, (long long)sz.n_q_max * p->heads);
   a.clear_spare = fixed ? 0 : 1;
   a.nan_pair = p->dtype == SBA_F16 && !a.out_f32 ? 0x7e007e00u : 0x7fc07fc0u;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);

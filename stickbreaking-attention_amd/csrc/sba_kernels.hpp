@@ -36,12 +36,15 @@ struct KArgs {
   float inv_temp;
   unsigned* work;              // work counters of the backward's persistent launch (WORK_WORDS words at the end of the
                                // gradient table; the dq pass clears them), or null: one workgroup per work item
-  int n_items;                 // work items of this launch (what the grid would be with one workgroup per item; forward: without spare
-                               // slots and, for packed documents, without their last, partial tiles)
+  int n_items;                 // work items of this launch (what the grid is with one workgroup per item)
   int resident;                // backward, host side: workgroups of a persistent launch (0: never persistent); forward: the
-                               // device's compute units
+                               // device's compute units if it holds the launch at once (see deal_item), or NO_DEAL
   int min_items_each;          // host side: a launch is persistent when it has this many items per workgroup
 };
+
+// Workgroups of the forward that a compute unit holds.
+constexpr int FWD_PER_CU_MAX = 6, NO_DEAL = 0x7fffffff / (FWD_PER_CU_MAX + 1);
+inline int fwd_per_cu(int head_dim) { return head_dim <= 32 ? FWD_PER_CU_MAX : (head_dim <= 64 ? 4 : (head_dim <= 128 ? 3 : 2)); }
 
 // Arguments of the one-pass backward (sba_chain.hip).
 constexpr int CHAIN_QUEUES = 8;            // one per XCD
