@@ -14,16 +14,13 @@ inline namespace SBA_ELEM_NS {
 // The item of this workgroup (items: tiles of every head, most expensive first).  Workgroup b starts on the same CU as
 // b + n_cus, b + 2 n_cus ...; while the chip holds the whole launch at once, whoever comes first gets the most expensive tile of every round
 // (tiles 15, 11, 7 and 3 for one CU against 12, 8, 4 and 0 for another).  Such a launch deals every second round backwards, eight
-// workgroups at a time, which leaves an item's head on its XCD.  A larger launch fills in behind its expensive tiles by itself (n_cus: NO_DEAL).
+// workgroups at a time, which leaves an item's head on its XCD.  A larger launch fills in behind its expensive tiles by itself (lg_cus: NO_DEAL).
 // 4 x 16 x 2048: 58.0 -> 55.7 us at head_dim 64 (with the carry table), 43.9 -> 41.9 at 32.
-// (No branch, no division and the grid's size as an argument: what every workgroup waits for before its first load.  With them 31 heads of
-// 1003 tokens at head_dim 128 took 32.2 us for 31.6.)
-__device__ __forceinline__ int deal_item(int n_cus, int n) {
-  const int b = blockIdx.x;
-  int round = 0;
-#pragma unroll
-  for (int r = 1; r < FWD_PER_CU_MAX; ++r) round += b >= r * n_cus ? 1 : 0;
-  const int first = round * n_cus, eights = min(n_cus, n - first) >> 3, at = (b - first) >> 3;
+// (Shifts, no branch, the grid's size as an argument, and the division by the heads a multiplication: every workgroup waits for this
+// before its first load.  With divisions and a branch 31 heads of 1003 tokens at head_dim 128 took 32.2 us for 31.6, 20 heads x 25 K tokens in 1682
+// documents at head_dim 32 94 for 84.)
+__device__ __forceinline__ unsigned deal_item(int lg_cus, unsigned n) {
+  const unsigned b = blockIdx.x, round = b >> lg_cus, first = round << lg_cus, eights = min(1u << lg_cus, n - first) >> 3, at = (b - first) >> 3;
   return (round & 1) && at < eights ? first + 8 * (eights - 1 - at) + (b & 7) : b;
 }
 
@@ -53,9 +50,8 @@ __global__ void __launch_bounds__(NT, D > 128 ? 2 : 3) fwd_kernel(const KArgs a)
   // Header words and this workgroup's tile are fetched together (the grid never exceeds the
   // allocated list, so the tile read is safe before the count is known): one round trip.
   const int* sched = a.sched;
-  const int item = deal_item(a.resident, a.n_items);
-  const int slot = item / a.heads;
-  const int head = item - slot * a.heads;
+  const unsigned item = deal_item(a.resident, a.n_items), below = __umulhi(item, a.heads_inv);   // (the quotient or one less)
+  const int over = (int)(item - below * a.heads) >= a.heads ? 1 : 0, slot = below + over, head = item - slot * a.heads;
   const int4 hdr = *reinterpret_cast<const int4*>(sched);   // status, query tiles, key tiles, table entries needed
   const Tile t = reinterpret_cast<const Tile*>(sched + SCHED_HDR)[slot];
   asm volatile("" ::"s"(t.tok_start), "s"(t.doc_len), "s"(t.idx), "s"(t.batch));   // keep the tile read above the branch

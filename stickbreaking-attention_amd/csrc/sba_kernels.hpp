@@ -22,6 +22,7 @@ struct KArgs {
   float* weights;              // forward, debug variant only: dense attention weights
                                // [batch][heads][tokens][tokens] (row = query token, column = key token)
   int heads;
+  unsigned heads_inv;          // forward: (2^32 - 1) / heads
   int head_dim;                // a multiple of 8, at most the width D of the kernel (see make_rows)
   int tokens;                  // tokens per batch entry
   int fuse;                    // the output is o + rem * v (and grad_o is the gradient of that)
@@ -38,13 +39,13 @@ struct KArgs {
                                // gradient table; the dq pass clears them), or null: one workgroup per work item
   int n_items;                 // work items of this launch (what the grid is with one workgroup per item)
   int resident;                // backward, host side: workgroups of a persistent launch (0: never persistent); forward: the
-                               // device's compute units if it holds the launch at once (see deal_item), or NO_DEAL
+                               // logarithm of the device's compute units if it holds the launch at once (see deal_item), or NO_DEAL
   int min_items_each;          // host side: a launch is persistent when it has this many items per workgroup
 };
 
 // Workgroups of the forward that a compute unit holds.
-constexpr int FWD_PER_CU_MAX = 6, NO_DEAL = 0x7fffffff / (FWD_PER_CU_MAX + 1);
-inline int fwd_per_cu(int head_dim) { return head_dim <= 32 ? FWD_PER_CU_MAX : (head_dim <= 64 ? 4 : (head_dim <= 128 ? 3 : 2)); }
+constexpr int NO_DEAL = 31;
+inline int fwd_per_cu(int head_dim) { return head_dim <= 32 ? 6 : (head_dim <= 64 ? 4 : (head_dim <= 128 ? 3 : 2)); }
 
 // Arguments of the one-pass backward (sba_chain.hip).
 constexpr int CHAIN_QUEUES = 8;            // one per XCD
