@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 
@@ -210,33 +211,41 @@ int fill_common(const sba_problem* p, bool fixed, const Sizes& sz, const void* s
 }
 
 // Where the kernels for problems that leave most of the chip idle (sba_small.hip) are the faster ones: both times
-// estimated, in us, from what 90 problems of 4 to 32 heads, 128 to 4096 tokens and 1 to 16 documents took at head_dim 32, 64 and 128.
+// estimated, in us, from what 90 problems of 4 to 32 heads, 128 to 4096 tokens and 1 to 16 documents took at head_dim 32, 64, 128 and 256.
 //   The general kernels take at least `base` and `step` for every 32 tokens of the longest document (more, once workgroups share a compute unit);
 //   the small ones their own `small_base` and the longer of what the longest document's rounds of 128 take one after the other (`round` each)
 //   and of what `at_once` workgroups at a time need: `group` each and `per_round` for every round, of which a workgroup has half
-//   its document's and half a one for the remainder.  (By tokens, documents are about halfway between the mean and the longest.)
+//   its document's and half a one for the remainder.  (By tokens, documents are about halfway between the mean and the longest.  A last group
+//   that is not full counts half as if it were: 11 heads of 3 x 686 tokens at head_dim 80, 1.4 groups, took 23.5 us for 21.2.  A group of
+//   workgroups for rows behind their document's end takes 2 us: 3 heads of 2212 tokens in 17 documents at head_dim 256 took 23.6 us for 21.6.)
 // `gain` must be gained, and 2 us, with which four times as many workgroups pay at the dispatcher (the forward of 13 prompts of up to 172 tokens: 9.9 us
 // alone with either, 10.6 for 11.3 in a row).
 struct SmallCost { double base, step, small_base, round, group, per_round; int at_once; };
-bool small_wins(const SmallCost (&costs)[3], double gain, const sba_problem* p, bool fixed, const Sizes& sz) {
-  if (!(p->flags & SBA_PRODUCT_SPACE) || p->head_dim > 128 || sz.n_docs <= 0) return false;
-  const SmallCost& c = costs[p->head_dim <= 32 ? 0 : (p->head_dim <= 64 ? 1 : 2)];
+bool small_wins(const SmallCost* costs, double gain, const sba_problem* p, bool fixed, const Sizes& sz) {
+  if (!(p->flags & SBA_PRODUCT_SPACE) || sz.n_docs <= 0) return false;
+  const SmallCost& c = costs[p->head_dim <= 32 ? 0 : (p->head_dim <= 64 ? 1 : (p->head_dim <= 128 ? 2 : 3))];
   const double longest = declared_max_doc_len(p, fixed), typical = 0.5 * (longest + std::min(longest, (double)sz.rows / sz.n_docs));
-  const double round = 32 * SMALL_WAVES, groups = (double)(sz.rows / 32 + sz.n_docs) * p->heads / c.at_once;
-  const double small = c.small_base + std::max(c.round * longest / round, groups * (c.group + c.per_round * (0.5 * typical / round + 0.5)));
+  const double round = 32 * SMALL_WAVES, blocks = fixed ? (double)p->batch * ((p->tokens + 31) / 32) : sz.rows / 32.0 + 0.5 * sz.n_docs;
+  double groups = blocks * p->heads / c.at_once;
+  if (groups > 1.0) groups = 0.5 * (groups + std::ceil(groups));
+  const double spare = ((double)sz.n_q_max * (BM / 32) - blocks) * p->heads / c.at_once;    // groups of workgroups that find nothing to do
+  const double small = c.small_base + 2.0 * spare + std::max(c.round * longest / round, groups * (c.group + c.per_round * (0.5 * typical / round + 0.5)));
   return std::max(gain * small, small + 2.0) < c.base + c.step * longest / 32;
 }
 // Of the problems taken all gain (head_dim 64: 4 heads x 512 14.4 / 9.7, 16 x 4096 78 / 68, 32 x 1024 24 / 17.5), and of those left to fwd_kernel none
-// would gain more than a tenth (head_dim 64: 16 heads of 4 x 1024 25.6 / 28, 32 x 2048 43 / 40; head_dim 128: 32 x 2048 58 / 74).
+// would gain more than a tenth (head_dim 64: 16 heads of 4 x 1024 25.6 / 28, 32 x 2048 43 / 40; head_dim 128: 32 x 2048 58 / 74; head_dim 256, whose line serves 129 on:
+// taken 4 x 512 28 / 18, 16 x 1024 48 / 35, left out 16 x 2048 89 / 95, 32 x 512 29 / 27.5).
 bool forward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
-  static constexpr SmallCost COSTS[3] = {{5.2, 0.46, 5.5, 0.75, 2.7, 1.33, 1024}, {5.8, 0.55, 6.2, 0.90, 3.4, 1.66, 1024}, {6.5, 0.73, 7.0, 1.19, 4.0, 1.60, 512}};
+  static constexpr SmallCost COSTS[4] = {{5.2, 0.46, 5.5, 0.75, 2.7, 1.33, 1024}, {5.8, 0.55, 6.2, 0.90, 3.4, 1.66, 1024},
+                                         {6.5, 0.73, 7.0, 1.19, 4.0, 1.60, 512}, {8.7, 1.22, 10.0, 1.93, 5.0, 2.0, 256}};
   return small_wins(COSTS, 1.1, p, fixed, sz);
 }
 // The backward, both passes, against the one-pass form (head_dim 64: 4 heads x 512 36.2 / 23.5, 16 x 1024 55 / 38, 16 x 2048 91 / 80, left out
 // 16 x 4096 229 / 219, 32 x 4 x 256 28 / 34; head_dim 128: 4 heads x 512 42 / 32, 16 x 512 43 / 33.5, left out 16 x 1024 66 / 66).  Documents of one or two
-// blocks are with the general two passes (head_dim 64: 64 tokens 16.0 / 16.8).
+// blocks are with the general two passes (head_dim 64: 64 tokens 16.0 / 16.8; 2 heads of 68 documents of 38
+// tokens on average and 95 at most 18.5 / 23.9).
 bool backward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
-  if (backward_form() != 0 || g_dkdv_workgroups.load() != 0 || declared_max_doc_len(p, fixed) <= 64) return false;
+  if (backward_form() != 0 || g_dkdv_workgroups.load() != 0 || p->head_dim > 128 || declared_max_doc_len(p, fixed) <= 64 || sz.rows <= 64ll * sz.n_docs) return false;
   static constexpr SmallCost COSTS[3] = {{16.0, 1.04, 12.5, 1.9, 3.7, 2.35, 512}, {17.0, 1.15, 14.0, 2.34, 6.0, 2.75, 512}, {19.0, 1.42, 18.5, 3.6, 9.5, 3.6, 256}};
   return small_wins(COSTS, 1.05, p, fixed, sz);
 }

@@ -15,7 +15,7 @@ inline namespace SBA_ELEM_NS {
 template <int D, bool KEYS>
 struct WaveCopy {
   static constexpr int C8 = D / 8, RPI = 64 / C8, NCH = 32 / RPI;
-  static constexpr int KINDS = D == 128 ? 4 : 2;      // instructions apart by this many have their rows' swizzle in common
+  static constexpr int KINDS = 16 / RPI;              // instructions apart by this many have their rows' swizzle in common
   int voff[KINDS];
   __device__ __forceinline__ void init(int lane, unsigned row_bytes, int used_bytes) {
 #pragma unroll
@@ -25,7 +25,10 @@ struct WaveCopy {
     }
   }
   // source row of instruction j's first row
-  static constexpr int row_delta(int j) { return !KEYS ? j * RPI : D == 128 ? 16 * (j & 1) + 4 * (j >> 1) : 4 * j; }
+  static constexpr int row_delta(int j) {
+    const int m = j * RPI;
+    return KEYS ? ((m & 4) << 2) | ((m >> 3) << 2) | (m & 3) : m;    // (kperm)
+  }
   __device__ __forceinline__ void issue(const Rows& r, int row0, unsigned short* tile) const {
 #pragma unroll
     for (int j = 0; j < NCH; ++j)
@@ -82,10 +85,11 @@ __device__ __forceinline__ void store_sum(const float* sums, int w, int lane, fl
 // over the waves.  K and V rows come to every wave's own piece of LDS, the next round's as soon as this one's are read.
 // What bounds it: the round's serial chain (products, odds, barrier, weights) while the chip is empty, 0.9 us a round of 128 keys against
 // 0.54 us a step of 32 in fwd_kernel; then the additive time of matrix and vector instructions, with
-// 16 waves per compute unit at head_dim 64 and 8 at 128.  Measured (us, fwd_kernel first): head_dim 64, 4 heads of 512 tokens 14.4 / 9.7,
-// of 2048 40 / 20; 16 heads of 1024 23.7 / 15.2; head_dim 128, 4 heads of 512 18.0 / 11.7, 16 heads of 2048 54 / 43.
+// 16 waves per compute unit at head_dim 64, 8 at 128 and 4 at 256.  Measured (us, fwd_kernel first): head_dim 64, 4 heads of 512 tokens 14.4 / 9.7,
+// of 2048 40 / 20; 16 heads of 1024 23.7 / 15.2; head_dim 128, 4 heads of 512 18.0 / 11.7, 16 heads of 2048 54 / 43;
+// head_dim 256, 4 heads of 512 28 / 18, of 2048 87 / 41.
 template <int D, bool AC, int U>
-__global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 4 : 2) fwd_small_kernel(const KArgs a) {
+__global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 4 : (D <= 128 ? 2 : 1)) fwd_small_kernel(const KArgs a) {
   constexpr int W = SMALL_WAVES, KS = U / 16, DB = U / 32, TILE = 32 * D;
   __shared__ __attribute__((aligned(16))) unsigned short smem[2 * W * TILE];   // per wave: K block, V block; then the waves' outputs
   __shared__ float left[2][W][32];              // by round parity: what a wave's block leaves of a query's stick
@@ -166,7 +170,7 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 4 : 2) fwd_small_k
     {
       el8 kfr[KS];
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) kfr[ks] = lds_row8(Kt + (kbase ^ (ks << 4)));
+      for (int ks = 0; ks < KS; ++ks) kfr[ks] = lds_row8(Kt + (kbase ^ ((ks & 7) << 4)) + 128 * (ks >> 3));   // (the swizzle leaves the upper half of 512-byte rows where it is)
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) x = mfma32(kfr[ks], qf[ks], x);
     }
@@ -204,7 +208,10 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 4 : 2) fwd_small_k
       const el8 pf = pack8(p + 8 * tt);
       const unsigned short* const vrow = Vt + 16 * tt * D;
 #pragma unroll
-      for (int db = 0; db < DB; ++db) o[db] = mfma32(lds_tr8(vrow + (vbase[0] ^ (db << 5)), vrow + (vbase[1] ^ (db << 5))), pf, o[db]);
+      for (int db = 0; db < DB; ++db) {
+        const unsigned short* const vcol = vrow + 128 * (db >> 2);
+        o[db] = mfma32(lds_tr8(vcol + (vbase[0] ^ ((db & 3) << 5)), vcol + (vbase[1] ^ ((db & 3) << 5))), pf, o[db]);
+      }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     vcopy.issue(vrows, r + 1 < n_rounds ? row_of(r + 1) : L, Vt);
@@ -798,6 +805,10 @@ SBA_SMALL(64, 64)
 SBA_SMALL(128, 96)
 SBA_SMALL(128, 128)
 #undef SBA_SMALL
+template __global__ void fwd_small_kernel<256, false, 192>(const KArgs);
+template __global__ void fwd_small_kernel<256, true, 192>(const KArgs);
+template __global__ void fwd_small_kernel<256, false, 256>(const KArgs);
+template __global__ void fwd_small_kernel<256, true, 256>(const KArgs);
 
 enum class SmallPass { FWD, DQ, DKDV };
 template <SmallPass PASS, int D, int U>
@@ -813,7 +824,11 @@ static hipError_t launch_small(const KArgs& a, bool ac, int n_q_max, hipStream_t
   if (a.head_dim <= 32) launch_small_d<PASS, 64, 32>(a, ac, n_q_max, s);
   else if (a.head_dim <= 64) launch_small_d<PASS, 64, 64>(a, ac, n_q_max, s);
   else if (used_width(a.head_dim) == 96) launch_small_d<PASS, 128, 96>(a, ac, n_q_max, s);
-  else launch_small_d<PASS, 128, 128>(a, ac, n_q_max, s);
+  else if (PASS != SmallPass::FWD || a.head_dim <= 128) launch_small_d<PASS, 128, 128>(a, ac, n_q_max, s);
+  else if constexpr (PASS == SmallPass::FWD) {
+    if (used_width(a.head_dim) == 192) launch_small_d<PASS, 256, 192>(a, ac, n_q_max, s);
+    else launch_small_d<PASS, 256, 256>(a, ac, n_q_max, s);
+  }
   return hipGetLastError();
 }
 hipError_t launch_fwd_small(const KArgs& a, bool ac, int n_q_max, hipStream_t s) { return launch_small<SmallPass::FWD>(a, ac, n_q_max, s); }

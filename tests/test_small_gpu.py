@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("d,lengths", [(64, [193, 128, 1]), (64, [129, 31, 32, 33]), (64, [255, 257, 300]), (64, [1, 1025]), (32, [500, 129]),
                                        (8, [385, 384]), (40, [640]), (72, [161, 260]), (96, [513]), (104, [290, 100]), (128, [401, 2]),
-                                       (128, [256, 255, 257])])
+                                       (128, [256, 255, 257]), (136, [300, 31]), (192, [255, 257]), (200, [513]), (256, [129, 385, 33])])
 @pytest.mark.parametrize("ac,fused", [(False, False), (True, False), (False, True), (True, True)])
 def test_packed_edges(d, lengths, ac, fused):
     T = sum(lengths)
@@ -67,7 +67,8 @@ def test_gradients_like_the_general_kernels(d, batch, T, layout, dtype, ac, fuse
 
 
 @pytest.mark.parametrize("dtype", list(_ROUND))
-@pytest.mark.parametrize("d,batch,T,layout", [(64, 1, 600, "heads"), (64, 2, 257, "tokens"), (32, 3, 130, "heads"), (96, 1, 400, "tokens"), (128, 2, 321, "heads")])
+@pytest.mark.parametrize("d,batch,T,layout", [(64, 1, 600, "heads"), (64, 2, 257, "tokens"), (32, 3, 130, "heads"), (96, 1, 400, "tokens"), (128, 2, 321, "heads"),
+                                              (256, 1, 260, "tokens"), (160, 2, 383, "heads")])
 @pytest.mark.parametrize("ac", [False, True])
 def test_the_same_as_the_general_kernels(d, batch, T, layout, dtype, ac):
     """Remainders to the bit (the table goes to the backward of either form), outputs up to the order of a float32 sum."""
