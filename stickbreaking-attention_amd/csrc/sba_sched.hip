@@ -168,15 +168,16 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
   // D. emit tiles: slot -> ranked document by binary search over the prefix
   // The hardware deals workgroups to the CUs round-robin in launch order (workgroups i and
   // i + number of CUs start on the same CU and run side by side), and hands out the rest as
-  // slots free up.  Documents of like length -- a class: more than half as many tiles as its longest -- are therefore
+  // slots free up.  Documents of like length -- a class: more than three quarters of the tiles of its longest -- are therefore
   // listed tile-major, the most expensive tile of every document first: the expensive tiles start together and the cheap
   // ones fill in behind them.  Document-major, the last document's most expensive tile starts when most of the launch is
   // over, and documents of one length put the same tile on the same CU.  Classes follow one another,
-  // so that a workgroup's neighbours still share K/V rows in the caches.  Forward, document-major / one class for all / as
-  // built: 12 heads x 4 x 4096 at head_dim 128 264 / 206 / 206 us, 32 heads x 16 K tokens in 8 documents 422 / 426 / 410, 8 heads
-  // x 32 K tokens in documents of 1024 .. 8192 426 / 384 / 393, 32 heads x 64 K tokens, one document of 32 K among shorter
-  // ones, 10.11 / 10.43 / 10.15 ms.  Documents of less than CLASS_TILES tiles stay document-major: their tiles cost about the
-  // same and share most of their rows (32 heads x 16 K tokens in 207 documents of 16 .. 256: 66.2 / 67.4 us).
+  // so that a workgroup's neighbours still share K/V rows in the caches.  Forward, us, document-major / classes from half the
+  // longest on / as built: 12 heads x 4 x 4096 at head_dim 128 284 / 242 / 241, 9 heads x 28667 tokens in 17 documents of up to
+  // 4148 247 / 217 / 218, 5 heads x 62572 tokens at head_dim 64, one document of 14691 among shorter ones, 395 / 413 / 403.  Documents of less than CLASS_TILES
+  // tiles stay document-major, and so does a class of more documents than its longest has tiles, as a document's K/V rows have left the caches
+  // by its next tile (32 heads x 16 K tokens in 207 documents of 16 .. 256: 66.2 / 67.4 us; 21 heads x 37933 tokens in 61 documents
+  // of about 630 at head_dim 128: 257 / 329 / 259).
   for (int s = tid; s < total_q && ok; s += SCHED_THREADS) {
     int d, idx, rank = 0, slot = s;
     if (fixed) {
@@ -197,11 +198,12 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
       idx = tiles_of(rank) - 1 - (s - q_before[rank]);             // newest (most expensive) query tile first
       if (in_lds && tiles_of(rank) >= CLASS_TILES) {
         int r0 = 0;          // of this document's class: its first rank
-        for (int n = tiles_of(0); 2 * tiles_of(rank) <= n; n = tiles_of(r0)) r0 = first_with_at_most(r0, n / 2);
+        for (int n = tiles_of(0); 4 * tiles_of(rank) <= 3 * n; n = tiles_of(r0)) r0 = first_with_at_most(r0, 3 * n / 4);
+        const int r2 = first_with_at_most(r0, max(3 * tiles_of(r0) / 4, CLASS_TILES - 1));   // its end
         // ahead of tile idx of this document: every tile of the class above idx, then the same tile of longer documents
         const int longer = first_with_at_most(r0, idx + 1) - r0;   // documents of the class that have a tile idx + 1 ...
-        const int r1 = min(r0 + longer, first_with_at_most(r0, max(tiles_of(r0) / 2, CLASS_TILES - 1)));   // ... and are in it
-        slot = q_before[r0] + (q_before[r1] - q_before[r0] - (r1 - r0) * (idx + 1)) + (rank - r0);
+        const int r1 = min(r0 + longer, r2);                       // ... and are in it
+        if (r2 - r0 <= tiles_of(r0)) slot = q_before[r0] + (q_before[r1] - q_before[r0] - (r1 - r0) * (idx + 1)) + (rank - r0);
       }
     }
     Tile t;

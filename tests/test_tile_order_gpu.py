@@ -13,22 +13,25 @@ CLASS_TILES = 4
 
 
 def _listed(lengths):
-    """(length, tile) in the order of the list: classes of documents of more than half as many tiles as their longest, a class tile-major;
-    documents of less than CLASS_TILES tiles one by one."""
+    """(length, tile) in the order of the list: classes of documents of more than three quarters of the tiles of their longest, a class tile-major;
+    documents of less than CLASS_TILES tiles one by one, and those of a class of more documents than its longest has tiles."""
     lengths = sorted(lengths, reverse=True)
     tiles = [-(-n // 128) for n in lengths]
     out, r = [], 0
     while r < len(tiles):
         end = r + 1
-        while tiles[r] >= CLASS_TILES and end < len(tiles) and 2 * tiles[end] > tiles[r] and tiles[end] >= CLASS_TILES:
+        while tiles[r] >= CLASS_TILES and end < len(tiles) and 4 * tiles[end] > 3 * tiles[r] and tiles[end] >= CLASS_TILES:
             end += 1
-        for i in range(tiles[r] - 1, -1, -1):
-            out += [(lengths[x], i) for x in range(r, end) if tiles[x] > i]
+        if end - r > tiles[r]:
+            out += [(lengths[x], i) for x in range(r, end) for i in range(tiles[x] - 1, -1, -1)]
+        else:
+            for i in range(tiles[r] - 1, -1, -1):
+                out += [(lengths[x], i) for x in range(r, end) if tiles[x] > i]
         r = end
     return out
 
 
-@pytest.mark.parametrize("lengths", [[512], [385, 384, 383, 1], [4096] * 4, [100] * 30, [0, 1024, 513, 512, 511, 0, 128, 129],
+@pytest.mark.parametrize("lengths", [[640] * 5 + [500] * 5, [640] * 6 + [512], [1024, 1000, 769, 768, 767, 500], [512], [385, 384, 383, 1], [4096] * 4, [100] * 30, [0, 1024, 513, 512, 511, 0, 128, 129],
                                      [2048, 1025, 1024, 897, 896, 600, 512, 385, 384, 300, 7],
                                      [random.Random(5).randint(1, 3000) for _ in range(40)],
                                      [random.Random(6).choice([200, 400, 500, 900]) for _ in range(600)]])
