@@ -34,22 +34,24 @@ PEAK_HBM_GBS = 8000.0       # MI355X published HBM3E bandwidth
 #     (SQ_VALU_MFMA_COEXEC_CYCLES), over 1024 SIMDs x GRBM_GUI_ACTIVE / 8: profiles/c3_sq_counters_pmc.txt
 #   (c2: profiles/c2_one_pass_backward.txt)
 MEASURED = {"sba_version": 214,
-            "c3": {"fwd_kernel": {"traffic": 1.041e9, "mfma_busy": 0.463, "valu_busy": 0.552, "coexec": 0.191},
-                   "bwd_chain_kernel": {"traffic": 7.872e9, "mfma_busy": 0.344, "valu_busy": 0.376, "coexec": 0.104}},
-            "c2": {"fwd_kernel": {"traffic": 1.135e8, "mfma_busy": 0.245, "valu_busy": 0.541, "coexec": 0.150},
-                   "bwd_chain_kernel": {"traffic": 6.485e8, "mfma_busy": 0.229, "valu_busy": 0.466, "coexec": 0.115}}}
+            "c3": {"fwd_kernel": {"traffic": 9.668e8, "mfma_busy": 0.464, "valu_busy": 0.552, "coexec": 0.192},
+                   "bwd_chain_kernel": {"traffic": 7.886e9, "mfma_busy": 0.344, "valu_busy": 0.377, "coexec": 0.103}},
+            "c2": {"fwd_kernel": {"traffic": 1.129e8, "mfma_busy": 0.254, "valu_busy": 0.561, "coexec": 0.151},
+                   "bwd_chain_kernel": {"traffic": 6.494e8, "mfma_busy": 0.228, "valu_busy": 0.464, "coexec": 0.114}}}
 
 KERNELS = ["fwd_kernel", "bwd_dq_kernel", "bwd_dkdv_kernel"]
-# algorithmic and executed FLOPs per causal pair and head_dim of each, and of the one-pass backward, which takes the
+# algorithmic and executed FLOPs per causal pair and head_dim of each, and of the backward in one kernel, which takes the
 # last one's place (and its event pair) where the library chooses it: no dq pass is recorded then
 ALGORITHMIC, EXECUTED = [4.0, 6.0, 4.0], [4.0, 6.0, 8.0]
-CHAINED = "bwd_chain_kernel"
+CHAINED, SHORT = "bwd_chain_kernel", "bwd_short_kernel"   # (the second: documents of at most 256 tokens at head_dim <= 64; it forms the scores twice)
 
 
 def kernel_figures(m):
     """[(name, ms, algorithmic, executed, tensors moved)] of a measured workload's kernels."""
     if m["backward"] and m["kern_ms"][1] == 0.0:
-        return [(KERNELS[0], m["kern_ms"][0], 4.0, 4.0, 4.0), (CHAINED, m["kern_ms"][2], 10.0, 10.0, 7.0)]
+        short = max(m["lengths"]) <= (256 if m["d"] <= 64 else 64)
+        return [(KERNELS[0], m["kern_ms"][0], 4.0, 4.0, 4.0),
+                (SHORT if short else CHAINED, m["kern_ms"][2], 10.0, 14.0 if short else 10.0, 7.0)]
     return [(n, m["kern_ms"][i], ALGORITHMIC[i], EXECUTED[i], [4.0, 5.0, 6.0][i]) for i, n in enumerate(KERNELS)]
 
 

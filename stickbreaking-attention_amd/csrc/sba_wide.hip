@@ -1,4 +1,5 @@
-// dk / dv pass of head_dim 129 .. 256 (see sba_bwd.hip for the two-pass backward and its other kernels).
+// The two passes of the backward at head_dim 129 .. 256 (see sba_bwd.hip for the two-pass backward and its other kernels): the dk / dv
+// pass, described here, and the dq pass, further down.
 //
 // At twice the width of the eight-wave kernel of sba_bwd.hip a wave's K and V fragments are 128 registers and the accumulators of 64
 // keys of one output 256: neither role fits two waves per SIMD.  So the work is cut smaller.  A workgroup owns 64 keys of
