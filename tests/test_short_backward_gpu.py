@@ -95,3 +95,38 @@ def test_rows_that_are_not_finite_stay_in_their_documents():
         x[which][:, 240 + 20] = float("inf")      # in the third
         for got, want in zip(_run(*x, lengths)[2:], clean):
             assert torch.equal(got[:, :240], want[:, :240]) and torch.equal(got[:, 304:], want[:, 304:]), which
+
+
+def test_replays_from_a_hip_graph():
+    from stickbreaking_attention import _ops
+    lengths, H, d = [256, 40, 128, 90, 64, 33, 200], 64, 64
+    T = sum(lengths) + 7
+    cu = cu_from_lengths(lengths, device=DEV)
+
+    def launch(q, k, v, do):
+        o, rem, state = _ops.run_forward(q, k, v, False, cu, max(lengths), d ** -0.5, False, need_table=True)
+        return (o, rem) + tuple(_ops.run_backward(q, k, v, do, None, False, state, d ** -0.5, False))
+
+    def inputs(seed):
+        return [t.to(DEV) for t in orc.make_inputs((H, T, d), seed)]
+
+    static = inputs(100)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        launch(*static)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = launch(*static)
+    for seed in (101, 102, 103):
+        fresh = inputs(seed)
+        for dst, src in zip(static, fresh):
+            dst.copy_(src)
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = launch(*fresh)
+        torch.cuda.synchronize()
+        for name, a, b in zip(("o", "rem", "dq", "dk", "dv"), captured, eager):
+            assert torch.equal(a, b), (seed, name)
