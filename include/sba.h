@@ -237,7 +237,7 @@ int sba_attn_bwd(const sba_problem* p, const void* schedule, size_t schedule_siz
 /* The backward in one pass: every score is formed once, dq is handed from key tile to key tile through scratch
  * memory (csrc/sba_chain.hip).  For the problems it is the faster form of, sba_chain_scratch_bytes
  * returns the scratch it needs (16-byte aligned, contents irrelevant, one per concurrent call) and 0 for every other;
- * a caller then takes sba_varlen_bwd / sba_attn_bwd.  Same inputs, outputs, table and refusals; it
+ * a caller then takes sba_varlen_bwd / sba_attn_bwd, which choose among their kernels by size.  Same inputs, outputs, table and refusals; it
  * needs no gradient table, and the results differ from the two-pass form's by rounding.  Problems it
  * cannot take (log-space carry, head_dim > 128, a device that is not eight XCDs of 32 compute units)
  * return SBA_E_SHAPE. */
@@ -287,8 +287,8 @@ const char* sba_error_string(int code);
  * compute launch is bracketed by HIP events on the caller's stream (event creation, no waiting:
  * timed kernels follow one another on the device as untimed ones do); sba_last_kernel_ms WAITS
  * for the most recent launch of the kernel asked for and returns its duration in milliseconds
- * (which: 0 = forward, 1 = backward dq pass, 2 = backward dk/dv pass, or the whole of the one-pass
- * backward), 0 if it has not been launched since the switch was turned on.  One process-wide switch
+ * (which: 0 = forward, 1 = backward dq pass, 2 = backward dk/dv pass, or the whole of a
+ * backward in one pass or of short documents in one kernel), 0 if it has not been launched since the switch was turned on.  One process-wide switch
  * and one process-wide set of results (the backward may run on PyTorch's autograd thread): do
  * not use with concurrent callers, under graph capture, or in production.  Off by default;
  * sba_varlen_fwd_static ignores it. */
@@ -301,11 +301,14 @@ float sba_last_kernel_ms(int which);
  * least 8), however few tiles there are per workgroup; n = 0 (default): one per compute unit,
  * and only for problems with at least eight tiles per workgroup; n < 0: always one workgroup per
  * tile.  The results do not depend on it (every tile is computed by the same instructions in the
- * same order whichever workgroup takes it). */
+ * same order whichever workgroup takes it), nor does which kernels a backward runs: problems that
+ * take others than the two passes by themselves never see it. */
 void  sba_set_dkdv_workgroups(int n);
 
-/* Test and tuning switch (process-wide): which form of the backward sba_chain_scratch_bytes asks for.  0: by size,
- * 1: never the one-pass form, 2: wherever it is possible, 3: the same in steps of 64 queries (head_dim <= 64).
+/* Test and tuning switch (process-wide): the form of the backward.  0: by size -- sba_chain_scratch_bytes asks for
+ * the one-pass form where that is the fastest, and sba_*_bwd take the kernels for few tiles or for short documents
+ * where those are (csrc/sba_small.hip).  1: the general two passes, always.  2: the one-pass form wherever it is
+ * possible, 3: the same in steps of 64 queries (head_dim <= 64); sba_*_bwd then run the two passes.  The forms differ by rounding.
  * With SBA_FORM_SHORT_WAITS added, a wait of the one-pass form for the key tile before gives up after its
  * first look, as it otherwise does after about a second: what the missing partial sums belong to is NaN.
  * With SBA_FORM_IDLE_XCDS(mask), the XCDs in `mask` (of bits 0 .. 7, not all) count as without a compute unit for

@@ -245,7 +245,7 @@ bool forward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
 // blocks are with the general two passes (head_dim 64: 64 tokens 16.0 / 16.8; 2 heads of 68 documents of 38
 // tokens on average and 95 at most 18.5 / 23.9).
 bool backward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
-  if (backward_form() != 0 || g_dkdv_workgroups.load() != 0 || p->head_dim > 128 || declared_max_doc_len(p, fixed) <= 64 || sz.rows <= 64ll * sz.n_docs) return false;
+  if (backward_form() != 0 || p->head_dim > 128 || declared_max_doc_len(p, fixed) <= 64 || sz.rows <= 64ll * sz.n_docs) return false;
   static constexpr SmallCost COSTS[3] = {{16.0, 1.04, 12.5, 1.9, 3.7, 2.35, 512}, {17.0, 1.15, 14.0, 2.34, 6.0, 2.75, 512}, {19.0, 1.42, 18.5, 3.6, 9.5, 3.6, 256}};
   return small_wins(COSTS, 1.05, p, fixed, sz);
 }
@@ -256,7 +256,7 @@ bool backward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
 // 32 x 64 16.6 / 19.0).  Above head_dim 64 a compute unit has room for one workgroup, and only what the one-pass form does not take gains (head_dim 128: 16
 // heads of 128 x 64 115 / 74, 32 of 128 x 33 160 / 112; left out: 16 heads of 128 x 128 142 / 166, 32 heads x 16 K tokens in documents of 16 .. 256 417 / 424).
 bool backward_short(const sba_problem* p, bool fixed, const Sizes& sz) {
-  if (backward_form() != 0 || g_dkdv_workgroups.load() != 0) return false;
+  if (backward_form() != 0) return false;
   return (p->flags & SBA_PRODUCT_SPACE) && p->head_dim <= 128 && sz.n_docs > 0 && sz.n_docs <= RANK_LIMIT &&
          declared_max_doc_len(p, fixed) <= (p->head_dim <= 64 ? 32 * SHORT_BLOCKS : 64) && sz.rows * p->heads >= 40000;
 }
@@ -412,7 +412,7 @@ bool chain_wide(const sba_problem* p, bool fixed, const Sizes& sz) {
 // 512 to 16 K tokens in 1 to 128 documents, declared lengths exact).
 bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
   const int form = backward_form();
-  if (form == 1 || g_dkdv_workgroups.load() != 0 || !chain_possible(p, fixed, sz)) return false;
+  if (form == 1 || !chain_possible(p, fixed, sz)) return false;
   if (form == 2 || form == 3) return true;
   if (backward_short(p, fixed, sz) || backward_small(p, fixed, sz)) return false;
   const long long chains = (long long)sz.n_docs * p->heads, items = (long long)sz.n_kv_max * p->heads;

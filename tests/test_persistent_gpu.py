@@ -3,7 +3,8 @@ persistent launch of a fixed number of workgroups that draw their tiles from cou
 the gradient table (own XCD's class first, then the classes of the other XCDs).  Every tile is
 computed by the same instructions in the same order whichever workgroup takes it, so the two forms
 must agree BIT FOR BIT; `sba_set_dkdv_workgroups` forces the persistent form with few workgroups so
-that small problems walk many tiles per workgroup and exhaust and cross the classes."""
+that small problems walk many tiles per workgroup and exhaust and cross the classes.  (Which kernels a backward runs is another
+switch's: the two passes are asked for here, since problems of these sizes take other kernels by themselves.)"""
 import os
 
 import pytest
@@ -22,8 +23,10 @@ def _lib():
     from stickbreaking_attention import _native as nat
     assert os.path.exists(nat.LIB_PATH), "libsba.so must be built before the GPU tests run"
     lib = nat.load()
+    lib.sba_set_backward_form(1)
     yield lib
     lib.sba_set_dkdv_workgroups(0)
+    lib.sba_set_backward_form(0)
 
 
 def _grads_varlen(lib, workgroups, q, k, v, do, cu, max_len, **kw):
@@ -137,3 +140,20 @@ def test_fixed_length_persistent_launch(_lib):
     for other in outs[1:]:
         for a, b in zip(other, outs[0]):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("d,H,lengths", [(64, 3, [600, 130]), (128, 2, [700]), (64, 8, [256, 33] * 20), (128, 16, [64, 17] * 40),
+                                         (64, 40, [1500, 700, 129]), (96, 20, [900, 2000]), (256, 2, [300, 65])])
+def test_the_number_of_workgroups_does_not_choose_the_kernels(_lib, d, H, lengths):
+    """Few tiles, short documents, one pass, wide heads: what a call runs by itself is what it runs with the switch set."""
+    dev = torch.device("cuda:0")
+    q, k, v, do = (t.to(dev) for t in orc.make_inputs((H, sum(lengths), d), 11 + d))
+    cu = hp.cu_from_lengths(lengths, device=dev)
+    _lib.sba_set_backward_form(0)
+    try:
+        base = _grads_varlen(_lib, 0, q, k, v, do, cu, max(lengths))
+        for wg in (-1, 8):
+            for name, a, b in zip(("dq", "dk", "dv"), _grads_varlen(_lib, wg, q, k, v, do, cu, max(lengths)), base):
+                assert torch.equal(a, b), f"{name} differs with {wg}"
+    finally:
+        _lib.sba_set_backward_form(1)
