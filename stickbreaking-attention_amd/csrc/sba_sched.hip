@@ -27,6 +27,7 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
   // workspace are used.
   __shared__ int s_len[RANK_LIMIT], s_ord[RANK_LIMIT], s_qoff[RANK_LIMIT + 1], s_kvoff[RANK_LIMIT + 1];
   __shared__ int s_start[RANK_LIMIT], s_tab[RANK_LIMIT];
+  __shared__ unsigned short s_class[RANK_LIMIT], s_next[RANK_LIMIT];   // by rank: first rank of the document's class; of the class behind one that begins here
   const int tid = threadIdx.x;
   const int nd = a.n_docs;
   int* hdr = a.out;
@@ -89,10 +90,23 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
         const int le = s_len[e];
         r += (le > len) || (le == len && e < d);
       }
+      s_kvoff[r] = len;      // (by rank, until the class is found)
     }
     ranked[r] = d;
   }
   __syncthreads();
+  // The classes of D, found once for a document (us without classes / with every tile searching for its own / as built: 40 documents of up to 3000
+  // tokens 9.1 / 13.2 / 11.4, 600 of 200 .. 900 34.6 / 50.9 / 36.3, 30 of 32768, 24576 ... 11.8 / 22.4 / 14.5, eight of 512 .. 4096 5.7 / 6.8 / 6.8).
+  const bool classes = !fixed && in_lds && s_maxlen > BM * (CLASS_TILES - 1);
+  if (classes) {
+    for (int i = tid; i < nd; i += SCHED_THREADS) {
+      const int limit = BM * max(3 * cdiv(s_kvoff[i], BM) / 4, CLASS_TILES - 1);   // what is longer is in the class that begins with this one
+      int lo = i, hi = nd;
+      while (lo < hi) { const int mid = (lo + hi) >> 1; if (s_kvoff[mid] <= limit) hi = mid; else lo = mid + 1; }
+      s_next[i] = (unsigned short)lo;
+    }
+    __syncthreads();
+  }
 
   // C. exclusive prefix of the tile counts in ranked order.  Key tiles are listed in two groups (see
   // kv_tail_tiles): first, document by document, the tiles that many queries follow; then the rest.
@@ -108,6 +122,11 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
       skv += cdiv(len, BKV) - kv_tail_tiles(len);
       sne += kv_tail_tiles(len);
       stab += tab_doc_entries(len);
+      if (classes && len > BM * (CLASS_TILES - 1)) {
+        int r0 = j > 0 ? s_class[i - 1] : 0;
+        while (s_next[r0] <= i) r0 = s_next[r0];
+        s_class[i] = (unsigned short)r0;
+      }
     }
   }
   s_scan_q[tid] = sq;
@@ -185,25 +204,20 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
       idx = cdiv(len_of[d], BM) - 1 - s / nd;
     } else {
       auto tiles_of = [&](int r) { return q_before[r + 1] - q_before[r]; };
-      // the first rank from r0 on with at most n tiles (ranks are in descending order)
-      auto first_with_at_most = [&](int r0, int n) {
-        int lo = r0, hi = nd;
-        while (lo < hi) { const int mid = (lo + hi) >> 1; if (tiles_of(mid) <= n) hi = mid; else lo = mid + 1; }
-        return lo;
-      };
       int lo = 0, hi = nd;   // largest i with qoff[i] <= s
       while (hi - lo > 1) { const int mid = (lo + hi) >> 1; if (q_before[mid] <= s) lo = mid; else hi = mid; }
       rank = lo;
       d = ranked[lo];
       idx = tiles_of(rank) - 1 - (s - q_before[rank]);             // newest (most expensive) query tile first
-      if (in_lds && tiles_of(rank) >= CLASS_TILES) {
-        int r0 = 0;          // of this document's class: its first rank
-        for (int n = tiles_of(0); 4 * tiles_of(rank) <= 3 * n; n = tiles_of(r0)) r0 = first_with_at_most(r0, 3 * n / 4);
-        const int r2 = first_with_at_most(r0, max(3 * tiles_of(r0) / 4, CLASS_TILES - 1));   // its end
-        // ahead of tile idx of this document: every tile of the class above idx, then the same tile of longer documents
-        const int longer = first_with_at_most(r0, idx + 1) - r0;   // documents of the class that have a tile idx + 1 ...
-        const int r1 = min(r0 + longer, r2);                       // ... and are in it
-        if (r2 - r0 <= tiles_of(r0)) slot = q_before[r0] + (q_before[r1] - q_before[r0] - (r1 - r0) * (idx + 1)) + (rank - r0);
+      if (classes && tiles_of(rank) >= CLASS_TILES) {
+        const int r0 = s_class[rank], r2 = s_next[r0];             // its class
+        if (r2 - r0 > 1 && r2 - r0 <= tiles_of(r0)) {
+          // ahead of tile idx of this document: every tile of the class above idx, then the same tile of longer documents
+          int r1 = r0, end = r2;                                   // (ranks are in descending order: those of the class that have a tile idx + 1)
+          if (tiles_of(r2 - 1) > idx + 1) r1 = r2;
+          else while (r1 < end) { const int mid = (r1 + end) >> 1; if (tiles_of(mid) <= idx + 1) end = mid; else r1 = mid + 1; }
+          slot = q_before[r0] + (q_before[r1] - q_before[r0] - (r1 - r0) * (idx + 1)) + (rank - r0);
+        }
       }
     }
     Tile t;
