@@ -39,7 +39,7 @@
 extern "C" {
 #endif
 
-#define SBA_VERSION 214
+#define SBA_VERSION 215
 
 /* error codes (negative returns) */
 #define SBA_E_NULL      (-1)  /* a required pointer is NULL                         */
@@ -269,7 +269,13 @@ int sba_round_floats(int dtype, int n, const void* const* src, void* const* dst,
  *   dk/dv pass: `dkdv_main_tiles` slots of the key-tile list from its start (room: key_list_tiles),
  *   and `dkdv_tail_tiles` workgroups per head that compare their slot with the list's true length
  *   before they read it.  `long_tiles_bound` / `tail_tiles_bound` are the bounds on the two groups
- *   of the key-tile list the grids are derived from.  Offsets and sizes are in int32 words. */
+ *   of the key-tile list the grids are derived from; `dkdv_main_workgroups` per head, one to a slot, or
+ *   two above head_dim 128;
+ *   problems of few tiles: `fwd_small_workgroups` / `bwd_small_workgroups` per head, four to a slot of the
+ *   query-tile list, 0 where the general kernels run;
+ *   backward of short documents: `bwd_short_workgroups` per head, 0 where others run; it reads the
+ *   ranked documents, four words each from `docs_word` on (up to 4096 documents).
+ * Offsets and sizes are in int32 words. */
 typedef struct sba_geometry {
   int query_list_tiles, key_list_tiles;
   int query_list_word, key_list_word, tile_words;
@@ -277,6 +283,9 @@ typedef struct sba_geometry {
   int fwd_tiles, dq_tiles;
   int long_tiles_bound, tail_tiles_bound;
   int dkdv_main_tiles, dkdv_tail_tiles;
+  int dkdv_main_workgroups;
+  int fwd_small_workgroups, bwd_small_workgroups, bwd_short_workgroups;
+  int docs_word;
 } sba_geometry;
 int sba_launch_geometry(const sba_problem* p, sba_geometry* out);
 

@@ -715,6 +715,12 @@ int sba_launch_geometry(const sba_problem* p, sba_geometry* out) {
   out->tail_tiles_bound = bb.n_tail_max;
   out->dkdv_main_tiles = g.main_tiles;
   out->dkdv_tail_tiles = g.tail_tiles;
+  out->dkdv_main_workgroups = dkdv_main_workgroups(p->head_dim, g.main_tiles);
+  const bool is_short = backward_short(p, fixed, sz);
+  out->fwd_small_workgroups = forward_small(p, fixed, sz) ? small_workgroups(sz.n_q_max) : 0;
+  out->bwd_small_workgroups = !is_short && backward_small(p, fixed, sz) ? small_workgroups(sz.n_q_max) : 0;
+  out->bwd_short_workgroups = is_short ? short_parts(p, fixed, sz) : 0;
+  out->docs_word = SCHED_HDR + TILE_WORDS * (sz.n_q_max + sz.n_kv_max) + chain_docs_offset(sz.n_docs);
   return 0;
 }
 

@@ -164,6 +164,11 @@ inline int used_width(int head_dim) {
   return kernel_width(head_dim);
 }
 inline bool has_dkdv_tail_kernel(int head_dim) { return head_dim <= 64; }
+// Workgroups per head: of the kernels of sba_small.hip that own 32 rows of a query tile, and of the dk/dv main kernel, which
+// above head_dim 128 owns half a key tile.
+inline int small_workgroups(int n_q_max) { return n_q_max * (BM / 32); }
+constexpr int WIDE_KEYS = 64;
+inline int dkdv_main_workgroups(int head_dim, int main_tiles) { return main_tiles * (kernel_width(head_dim) > 128 ? BKV / WIDE_KEYS : 1); }
 
 // One set of compute launchers per element type (sba_fwd.hip and sba_bwd.hip are compiled once
 // for each, see SBA_ELEM_NS).

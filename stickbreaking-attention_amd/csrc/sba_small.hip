@@ -568,7 +568,7 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_k
     fill_rows16(a.dk, head, row0, row1, a.head_dim << a.out_f32, pair, tid, W * 64);
     fill_rows16(a.dv, head, row0, row1, a.head_dim << a.out_f32, pair, tid, W * 64);
   }
-  if (refused || longest > 32 * NB) return;     // (the second: not reached, a.max_doc_len is no more)
+  if (refused) return;                          // (beyond here no document has more than NB blocks: see launch_bwd_short)
   // The documents are ranked, longest first: one for a workgroup, then two, then four.
   const int pairs = (over_64 - over_128 + 1) / 2;
   const int team_waves = part < over_128 ? W : (part - over_128 < pairs ? W / 2 : W / 4), teams = W / team_waves;
@@ -813,7 +813,7 @@ template __global__ void fwd_small_kernel<256, true, 256>(const KArgs);
 enum class SmallPass { FWD, DQ, DKDV };
 template <SmallPass PASS, int D, int U>
 static void launch_small_d(const KArgs& a, bool ac, int n_q_max, hipStream_t s) {
-  const dim3 grid((unsigned)n_q_max * (BM / 32) * (unsigned)a.heads), block(SMALL_WAVES * 64);
+  const dim3 grid((unsigned)small_workgroups(n_q_max) * (unsigned)a.heads), block(SMALL_WAVES * 64);
   auto launch = [&](void (*plain)(KArgs), void (*current)(KArgs)) { hipLaunchKernelGGL(ac ? current : plain, grid, block, 0, s, a); };
   if constexpr (PASS == SmallPass::FWD) launch(fwd_small_kernel<D, false, U>, fwd_small_kernel<D, true, U>);
   else if constexpr (PASS == SmallPass::DQ) launch(bwd_dq_small_kernel<D, false, U>, bwd_dq_small_kernel<D, true, U>);
@@ -824,11 +824,11 @@ static hipError_t launch_small(const KArgs& a, bool ac, int n_q_max, hipStream_t
   if (a.head_dim <= 32) launch_small_d<PASS, 64, 32>(a, ac, n_q_max, s);
   else if (a.head_dim <= 64) launch_small_d<PASS, 64, 64>(a, ac, n_q_max, s);
   else if (used_width(a.head_dim) == 96) launch_small_d<PASS, 128, 96>(a, ac, n_q_max, s);
-  else if (PASS != SmallPass::FWD || a.head_dim <= 128) launch_small_d<PASS, 128, 128>(a, ac, n_q_max, s);
+  else if (a.head_dim <= 128) launch_small_d<PASS, 128, 128>(a, ac, n_q_max, s);
   else if constexpr (PASS == SmallPass::FWD) {
     if (used_width(a.head_dim) == 192) launch_small_d<PASS, 256, 192>(a, ac, n_q_max, s);
     else launch_small_d<PASS, 256, 256>(a, ac, n_q_max, s);
-  }
+  } else return hipErrorInvalidValue;             // (the backward's two have no kernel of that width)
   return hipGetLastError();
 }
 hipError_t launch_fwd_small(const KArgs& a, bool ac, int n_q_max, hipStream_t s) { return launch_small<SmallPass::FWD>(a, ac, n_q_max, s); }
@@ -836,6 +836,7 @@ hipError_t launch_bwd_dq_small(const KArgs& a, bool ac, int n_q_max, hipStream_t
 hipError_t launch_bwd_dkdv_small(const KArgs& a, bool ac, int n_q_max, hipStream_t s) { return launch_small<SmallPass::DKDV>(a, ac, n_q_max, s); }
 
 hipError_t launch_bwd_short(const KArgs& a, bool ac, int parts, hipStream_t s) {
+  if (a.head_dim > 128 || a.max_doc_len > 32 * SHORT_BLOCKS) return hipErrorInvalidValue;   // (longer ones than declared are refused on the device)
   const dim3 grid((unsigned)parts * (unsigned)a.heads), block(SMALL_WAVES * 64);
   auto launch = [&](void (*plain)(KArgs), void (*current)(KArgs)) { hipLaunchKernelGGL(ac ? current : plain, grid, block, 0, s, a); };
   if (a.head_dim <= 32) launch(bwd_short_kernel<64, false, 32>, bwd_short_kernel<64, true, 32>);

@@ -28,7 +28,6 @@
 namespace sba {
 inline namespace SBA_ELEM_NS {
 
-constexpr int WIDE_KEYS = 64;     // keys of a workgroup: half a tile of the key-tile list
 
 template <bool AC, bool PROD, int U>
 __global__ void __launch_bounds__(512, 1) bwd_dkdv_wide_kernel(const KArgs a) {
@@ -691,7 +690,7 @@ hipError_t launch_bwd_dq_wide(const KArgs& a, bool ac, bool prod, int n_q_max, h
 
 // tiles: upper bound on the tiles of the key-tile list, no more than it has room for
 hipError_t launch_bwd_dkdv_wide(const KArgs& a, bool ac, bool prod, int tiles, hipStream_t s) {
-  const dim3 grid((unsigned)tiles * (BKV / WIDE_KEYS) * (unsigned)a.heads), block(512);
+  const dim3 grid((unsigned)dkdv_main_workgroups(a.head_dim, tiles) * (unsigned)a.heads), block(512);
   if (prod && used_width(a.head_dim) == 192) {
     if (ac) hipLaunchKernelGGL((bwd_dkdv_wide_kernel<true, true, 192>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((bwd_dkdv_wide_kernel<false, true, 192>), grid, block, 0, s, a);

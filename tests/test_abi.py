@@ -25,7 +25,7 @@ def test_library_exports_every_declared_symbol():
     for s in syms:
         assert hasattr(lib, s), f"{s} declared in include/sba.h but not exported"
     assert sorted(nat.EXPORTS) == syms
-    assert lib.sba_version() == 214
+    assert lib.sba_version() == 215
 
 
 def problem(**kw):
@@ -279,6 +279,11 @@ def _check_geometry(g, n_docs):
     assert g.key_list_word + g.tile_words * g.dkdv_main_tiles <= g.schedule_words
     # (the tail kernel checks its slot against the true list length before reading: any grid is safe)
     assert g.dkdv_tail_tiles >= 0
+    # the kernels for few tiles: four workgroups to a slot of the query list
+    for n in (g.fwd_small_workgroups, g.bwd_small_workgroups):
+        assert n in (0, 4 * g.query_list_tiles)
+    # the ranked documents, read by the backward of short documents as 16-byte words
+    assert g.docs_word >= lists_end and g.docs_word % 4 == 0 and g.docs_word + 4 * n_docs <= g.schedule_words
 
 
 def _tiles(lengths, rows):
@@ -300,12 +305,18 @@ def test_every_launch_stays_inside_the_schedule_workspace():
         n_docs = rng.choice([0, 1, rng.randint(0, 12), rng.randint(0, 400)])
         mdl = rng.choice([0, 1, rng.randint(0, max(tokens, 1)), tokens, tokens + 7])
         cases.append((tokens, n_docs, mdl))
+    ran = {"small forward": False, "small backward": False}
     for tokens, n_docs, mdl in cases:
         for d in (32, 64, 128, 256):
-            g = _geometry(tokens=tokens, n_docs=n_docs, max_doc_len=mdl, head_dim=d, heads=3)
+            g = _geometry(tokens=tokens, n_docs=n_docs, max_doc_len=mdl, head_dim=d, heads=3, flags=nat.FLAG_PRODUCT_SPACE)
             _check_geometry(g, n_docs)
+            # a workgroup of the dk/dv main kernel at head_dim 256 owns half a tile
+            assert g.dkdv_main_workgroups == (2 if d == 256 else 1) * g.dkdv_main_tiles
+            ran["small forward"] |= g.fwd_small_workgroups > 0
+            ran["small backward"] |= g.bwd_small_workgroups > 0
             # what an earlier version launched at head_dim 128 (both bounds added, no clamp) does NOT stay inside:
             # the test must be able to tell the difference
+    assert all(ran.values())
     g = _geometry(tokens=2112, n_docs=10, max_doc_len=2112, head_dim=128, heads=3)
     assert g.long_tiles_bound + g.tail_tiles_bound > g.key_list_tiles >= g.dkdv_main_tiles
     # fixed length: batch documents of `tokens` tokens each
@@ -342,6 +353,30 @@ def test_launch_bounds_cover_every_split_into_documents():
                 assert n_kv <= g.dkdv_main_tiles           # one kernel takes both groups
             else:
                 assert n_long <= g.dkdv_main_tiles and n_tail <= g.dkdv_tail_tiles
+
+
+def test_the_backward_of_short_documents_covers_every_split():
+    """One workgroup for a document of more than 128 tokens, for two of more than 64, for four shorter ones (the device
+    counts the classes): whatever the split, no more than are launched, or rows of dq, dk and dv stay unwritten."""
+    import random
+    rng = random.Random(11)
+    seen = set()
+    for case in range(4000):
+        n_docs = rng.choice([1, 2, 3, rng.randint(1, 12), rng.randint(1, 300), 4096])
+        longest = rng.choice([1, 33, 64, 65, 128, 129, 200, 256])
+        kind = rng.random()
+        if kind < 0.3: lengths = [rng.randint(0, longest) for _ in range(n_docs)]
+        elif kind < 0.6: lengths = [min(rng.choice([0, 1, 64, 65, 128, 129, 256]), longest) for _ in range(n_docs)]
+        else: lengths = [min(rng.choice([64, 65, 128, 129]), longest)] * n_docs
+        tokens = max(sum(lengths), 1) + rng.choice([0, 0, 5])
+        d = rng.choice([32, 64] if longest > 64 else [32, 64, 128])
+        g = _geometry(tokens=tokens, n_docs=n_docs, max_doc_len=longest, head_dim=d, heads=-(-40000 // tokens), flags=nat.FLAG_PRODUCT_SPACE)
+        assert g.bwd_small_workgroups == 0
+        over_128, over_64 = (sum(n > limit for n in lengths) for limit in (128, 64))
+        needed = over_128 + -(-(over_64 - over_128) // 2) + -(-(n_docs - over_64) // 4)
+        assert needed <= g.bwd_short_workgroups, (lengths, tokens)
+        seen.add(g.bwd_short_workgroups - needed)
+    assert 0 in seen                                           # (the bound is reached)
 
 
 def test_scratch_tables_grow_instead_of_multiplying(monkeypatch):
