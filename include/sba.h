@@ -86,6 +86,15 @@ extern "C" {
                                    results converted, so that a float32 caller needs no pass
                                    of its own for that (grad_o and grad_rem stay 16-bit)   */
 
+/* Which kernel a forward runs in product space, with neither weights nor SBA_TABLE_ONLY.  By itself it goes by the size of the call:
+ * problems of few tiles take one that adds a row of `o` up in another order (csrc/sba_small.hip), so that
+ * the same sequence's `o` may differ in the last bit with the heads and documents beside it, and from
+ * that of the entry points with weights.  `rem` and the stick table are the same bits from either.
+ *   SBA_GENERAL_FORWARD   always the general kernel: `o` of a sequence does not depend on what else the call holds;
+ *   SBA_FEW_TILES_FORWARD the other one wherever there is a document (for tests). */
+#define SBA_GENERAL_FORWARD   128u
+#define SBA_FEW_TILES_FORWARD 256u
+
 /* A strided view over [batch, heads, tokens, head_dim]; the last dimension is contiguous.
  * Strides are in ELEMENTS.  For packed variable-length input batch == 1 and stride_b is
  * ignored.  For per-row tensors (rem, grad_rem) the head_dim axis is absent. */

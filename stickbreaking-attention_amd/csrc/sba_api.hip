@@ -236,6 +236,8 @@ bool small_wins(const SmallCost* costs, double gain, const sba_problem* p, bool 
 // would gain more than a tenth (head_dim 64: 16 heads of 4 x 1024 25.6 / 28, 32 x 2048 43 / 40; head_dim 128: 32 x 2048 58 / 74; head_dim 256, whose line serves 129 on:
 // taken 4 x 512 28 / 18, 16 x 1024 48 / 35, left out 16 x 2048 89 / 95, 32 x 512 29 / 27.5).
 bool forward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
+  if (p->flags & SBA_GENERAL_FORWARD) return false;
+  if (p->flags & SBA_FEW_TILES_FORWARD) return (p->flags & SBA_PRODUCT_SPACE) && sz.n_docs > 0;
   static constexpr SmallCost COSTS[4] = {{5.2, 0.46, 5.5, 0.75, 2.7, 1.33, 1024}, {5.8, 0.55, 6.2, 0.90, 3.4, 1.66, 1024},
                                          {6.5, 0.73, 7.0, 1.19, 4.0, 1.60, 512}, {8.7, 1.22, 10.0, 1.93, 5.0, 2.0, 256}};
   return small_wins(COSTS, 1.1, p, fixed, sz);

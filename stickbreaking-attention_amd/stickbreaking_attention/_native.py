@@ -26,6 +26,8 @@ FLAG_PRODUCT_SPACE = 4
 FLAG_FIXED_LENGTH = 8
 FLAG_FUSE_REMAINDER = 16
 FLAG_TABLE_ONLY = 32
+FLAG_GENERAL_FORWARD = 128
+FLAG_FEW_TILES_FORWARD = 256
 
 STATUS_MESSAGES = {
     1: "cu_seqlens is not a non-decreasing sequence within [0, total_tokens]",

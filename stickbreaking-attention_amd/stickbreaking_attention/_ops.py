@@ -56,6 +56,11 @@ RECOMPUTE_TABLE = os.environ.get("SBA_RECOMPUTE_TABLE", "0") == "1"
 # to a maximum between 4 and 8 by a power of two before it is rounded and the gradients are scaled back (exact).
 F32_AS_F16 = os.environ.get("SBA_F32_AS_F16", "0") == "1"
 
+# By itself a forward of few tiles takes a kernel that adds a row of `o` up in another order, so that a sequence's `o` may
+# differ in the last bit with the heads and documents beside it.  With SBA_GENERAL_FORWARD=1 every forward takes the general
+# kernel: the same bits alone, in any company and with return_attention (small calls take up to twice as long).
+FORWARD_FLAGS = nat.FLAG_GENERAL_FORWARD if os.environ.get("SBA_GENERAL_FORWARD", "0") == "1" else 0
+
 MAX_HEAD_DIM = 256
 
 # Tile sizes the library's workspace formulas are built on (query tile, dk/dv key tile, table block).
@@ -282,7 +287,7 @@ def _launch_fwd(fixed: bool, q, k, v, cu_seqlens, max_doc_len: int, logit_scale:
     if table_only:
         o = rem = None
     prob, _keep = _problem(q, fixed, cu_seqlens, max_doc_len, logit_scale, attend_current, product, fused,
-                           nat.FLAG_TABLE_ONLY if table_only else 0)
+                           FORWARD_FLAGS | (nat.FLAG_TABLE_ONLY if table_only else 0))
     name = ("sba_attn_fwd" if fixed else "sba_varlen_fwd") + ("_weights" if weights is not None else "")
     fn = getattr(lib, name)
     extra = () if weights is None else (weights.data_ptr(), _nbytes(weights))
@@ -523,7 +528,7 @@ def eager(q, k, v, fixed: bool, cu_seqlens, max_seqlens, inv_temp: float, attend
         _warn_reduced_precision(q.dtype)
     sched, build, entry = _cached_schedule(cu, sched_bytes, B, T, q.device)
     flags = ((nat.FLAG_ATTEND_CURRENT if attend_current else 0) | (nat.FLAG_PRODUCT_SPACE if PRODUCT_SPACE else 0) |
-             (nat.FLAG_FUSE_REMAINDER if fused else 0))
+             (nat.FLAG_FUSE_REMAINDER if fused else 0) | FORWARD_FLAGS)
     out = nat.load_ext().attention(q, k, v, cu, sched, build, table_floats, max_len, inv_temp, flags)
     _schedule_built(entry)
     return out

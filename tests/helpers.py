@@ -1,4 +1,5 @@
 """Shared helpers for the parity tests: seeded workloads, error metrics, oracle drivers."""
+import ctypes
 import json
 import math
 import os
@@ -21,6 +22,20 @@ def cu_from_lengths(lengths, leading_zero=False, dtype=torch.int32, device="cpu"
     if leading_zero:
         cu = torch.cat([torch.zeros(1, dtype=torch.int64), cu])
     return cu.to(dtype).to(device)
+
+
+def kernels_of(q, lengths=None, dtype_code=1):
+    """The library's account of the kernels a call on these documents (None: fixed length) runs: sba_launch_geometry."""
+    from stickbreaking_attention import _native as nat, _ops
+    flags = nat.FLAG_PRODUCT_SPACE | _ops.FORWARD_FLAGS
+    H, T, d = q.shape[-3:]
+    if lengths is None:
+        p = nat.SbaProblem(dtype_code, d, H, q.shape[0], T, 0, T, flags | nat.FLAG_FIXED_LENGTH, 1.0, None)
+    else:
+        p = nat.SbaProblem(dtype_code, d, H, 1, T, len(lengths), max(lengths), flags, 1.0, 16)
+    g = nat.SbaGeometry()
+    nat.check(nat.load().sba_launch_geometry(ctypes.byref(p), ctypes.byref(g)), "sba_launch_geometry")
+    return g
 
 
 def err_stats(name, got, ref):

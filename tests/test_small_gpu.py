@@ -1,24 +1,29 @@
 """Problems of few tiles take kernels of their own (sba_small.hip): on either side of their blocks of 32 and rounds of 128, in every form
-that the rule lets in, against the oracle and against the general kernels, which the same heads take when there are enough of them."""
+that the rule lets in, against the oracle and against the general kernels."""
 import pytest
 import torch
 
 from oracle import sb_oracle as orc
 from stickbreaking_attention import sb_attn, sb_attn_fused
-from tests.helpers import assert_close, oracle_varlen
+from stickbreaking_attention import _native as nat
+from stickbreaking_attention import _ops
+from tests.helpers import assert_close, cu_from_lengths, kernels_of, oracle_varlen
 from tests.test_fused_gpu import check, fused_reference
 from tests.test_head_dim_256_gpu import DEV, _need_gpu, _run  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("d,lengths", [(64, [193, 128, 1]), (64, [129, 31, 32, 33]), (64, [255, 257, 300]), (64, [1, 1025]), (32, [500, 129]),
+@pytest.mark.parametrize("d,lengths", [(64, [193, 128, 1]), (64, [129, 31, 32, 33]), (64, [161, 129, 33, 32, 31]), (64, [255, 257, 300]), (64, [1, 1025]), (32, [500, 129]),
                                        (8, [385, 384]), (40, [640]), (72, [161, 260]), (96, [513]), (104, [290, 100]), (128, [401, 2]),
                                        (128, [256, 255, 257]), (136, [300, 31]), (192, [255, 257]), (200, [513]), (256, [129, 385, 33])])
 @pytest.mark.parametrize("ac,fused", [(False, False), (True, False), (False, True), (True, True)])
-def test_packed_edges(d, lengths, ac, fused):
+def test_packed_edges(d, lengths, ac, fused, monkeypatch):
+    monkeypatch.setattr(_ops, "FORWARD_FLAGS", nat.FLAG_FEW_TILES_FORWARD)
     T = sum(lengths)
     q, k, v, do = orc.make_inputs((3, T, d), d + T)
+    ran = kernels_of(q, lengths)
+    assert ran.fwd_small_workgroups > 0 and (ran.bwd_small_workgroups > 0) == (d <= 128 and lengths != [129, 31, 32, 33])
     if fused:
         check(_run(q, k, v, do, lengths, ac, fused=True), fused_reference(q, k, v, do, lengths, ac))
         return
@@ -83,3 +88,44 @@ def test_the_same_as_the_general_kernels(d, batch, T, layout, dtype, ac):
     assert torch.equal(rem, rem_many[:, :2])
     # a float32 sum of T weighted values below 6 in another order, which may round to the neighbour
     torch.testing.assert_close(o, o_many[:, :2], rtol=_ROUND[dtype], atol=T * 6 * 2.0 ** -24)
+
+
+@pytest.mark.parametrize("d,H,lengths", [(64, 2, [700, 40, 129]), (32, 1, [513]), (96, 3, [400, 33]), (128, 2, [321, 1]), (256, 2, [300, 65])])
+def test_a_sequence_in_any_company(d, H, lengths, monkeypatch):
+    """On the general kernels a sequence's outputs and gradients are the same bits alone, beside more heads, beside other documents and
+    where the weights are returned too; by size, its remainders are."""
+    from stickbreaking_attention import sb_attn_varlen
+    from stickbreaking_attention.sb_varlen import varlen_fwd
+    lib = nat.load()
+    gen = torch.Generator(device=DEV).manual_seed(d)
+    T, others = sum(lengths), [900, 31, 128] * 6
+    mine = [torch.randn((H, T, d), generator=gen, device=DEV).to(torch.bfloat16) for _ in range(4)]
+    theirs = [torch.randn((H, sum(others), d), generator=gen, device=DEV).to(torch.bfloat16) for _ in range(4)]
+
+    def run(tensors, lens):
+        q, k, v = (t.requires_grad_() for t in tensors[:3])
+        o, rem = sb_attn_varlen(q, k, v, cu_from_lengths(lens, device=DEV), max(lens), zero_start=False)
+        return [t.detach()[:H, :T] for t in (o, rem) + torch.autograd.grad(o, (q, k, v), tensors[3])]
+
+    def calls():
+        yield run([t.clone() for t in mine], lengths)
+        yield run([t.repeat(200, 1, 1) for t in mine], lengths)
+        yield run([torch.cat([a, b], 1).repeat(12, 1, 1) for a, b in zip(mine, theirs)], lengths + others)
+
+    assert kernels_of(mine[0], lengths).fwd_small_workgroups > 0 and kernels_of(mine[0].repeat(200, 1, 1), lengths).fwd_small_workgroups == 0
+    alone, *company = calls()
+    for other in company:
+        assert torch.equal(alone[1], other[1])
+    monkeypatch.setattr(_ops, "FORWARD_FLAGS", nat.FLAG_GENERAL_FORWARD)
+    lib.sba_set_backward_form(1)
+    try:
+        alone, *company = calls()
+    finally:
+        lib.sba_set_backward_form(0)
+    for other in company:
+        for name, a, b in zip(("o", "rem", "dq", "dk", "dv"), alone, other):
+            assert torch.equal(a, b), name
+    with torch.no_grad():
+        o, rem = varlen_fwd(*(t.detach() for t in mine[:3]), cu_from_lengths(lengths, device=DEV), max(lengths), logit_scale=d ** -0.5,
+                            no_grad=True, return_attention=True)[:2]
+    assert torch.equal(o, alone[0]) and torch.equal(rem, alone[1])
