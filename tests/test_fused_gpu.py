@@ -53,7 +53,7 @@ def run_fused_varlen(q, k, v, dout, lengths, ac=False, prepare=lambda t: t.to(DE
 @pytest.mark.parametrize("lengths", [[1], [3, 1, 1, 2], [63, 64, 65, 127, 128, 129, 1, 31, 33], [257, 640]])
 @pytest.mark.parametrize("ac", [False, True])
 @pytest.mark.parametrize("d", [32, 64, 128, 256])
-def test_fused_varlen_ragged_documents(lengths, ac, d):
+def test_fused_varlen_ragged_documents(lengths, ac, d, kernels):
     T = sum(lengths)
     q, k, v, dout = orc.make_inputs((3, T, d), 11 + T + d, dist="upstream")
     check(run_fused_varlen(q, k, v, dout, lengths, ac), fused_reference(q, k, v, dout, lengths, ac))

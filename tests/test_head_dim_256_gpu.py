@@ -1,6 +1,6 @@
 """head_dim 256 (upstream takes any head_dim through BLOCK_D = next_power_of_2(d), sb_varlen_fwd.py:479).
-The forward and the dq pass are the kernels of the smaller head dims instantiated with two workgroups and one per compute unit; the
-dk/dv pass is a kernel of its own kind (64 keys per workgroup, three kinds of waves).  Everything here goes against the fp32 CPU oracle
+The forward is the kernel of the smaller head dims with two workgroups per compute unit, or that for few tiles; the two passes of the
+backward are kernels of their own kind (a block of queries on two waves; 64 keys per workgroup, three kinds of waves).  Everything here goes against the fp32 CPU oracle
 with the gate of the other head dims: max-abs 2e-2 before the output's own bf16 rounding."""
 import os
 
@@ -41,7 +41,7 @@ def _run(q, k, v, do, lengths, ac=False, drem=None, fused=False):
 
 @pytest.mark.parametrize("product_space", [False, True])
 @pytest.mark.parametrize("ac", [False, True])
-def test_long_documents(ac, product_space, monkeypatch):
+def test_long_documents(ac, product_space, monkeypatch, kernels):
     """Documents of 23 and 5 key tiles and a short one: the queries wrap the ring of the dk/dv kernel many
     times; a gradient for rem as well."""
     from stickbreaking_attention import _ops
@@ -56,7 +56,7 @@ def test_long_documents(ac, product_space, monkeypatch):
 
 
 @pytest.mark.parametrize("seed", range(6))
-def test_random_documents(seed):
+def test_random_documents(seed, kernels):
     import random
     rng = random.Random(2560 + seed)
     H = rng.choice((1, 2, 3))
@@ -68,7 +68,7 @@ def test_random_documents(seed):
         assert_close(f"seed {seed} {name}", g, r)
 
 
-def test_fused_output_on_long_documents():
+def test_fused_output_on_long_documents(kernels):
     lengths = [1100, 437]
     q, k, v, dout = orc.make_inputs((2, sum(lengths), 256), 78)
     qf, kf, vf = (t.float().requires_grad_() for t in (q, k, v))
@@ -80,7 +80,7 @@ def test_fused_output_on_long_documents():
         assert_close(name, g, r)
 
 
-def test_fixed_length_batch():
+def test_fixed_length_batch(kernels):
     from stickbreaking_attention import sb_attn
     q, k, v, do = orc.make_inputs((2, 3, 1024, 256), 31)
     qg, kg, vg = (t.to(DEV).requires_grad_() for t in (q, k, v))

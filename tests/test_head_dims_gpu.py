@@ -13,7 +13,7 @@ DEV = "cuda:0"
 
 @pytest.mark.parametrize("ac", [False, True])
 @pytest.mark.parametrize("d", [8, 24, 40, 72, 80, 96, 104, 136, 160, 192, 200, 248])
-def test_columns_behind_the_head_are_never_read(d, ac):
+def test_columns_behind_the_head_are_never_read(d, ac, kernels):
     from stickbreaking_attention import sb_attn_varlen, sb_attn_varlen_fused
     lengths = [33, 1, 129, 300]
     H, T = 2, sum(lengths) + 7

@@ -93,7 +93,7 @@ def test_log_space_carry_on_long_documents(ac, monkeypatch):
 @pytest.mark.parametrize("lengths", [[1], [2], [3, 1, 1, 2], [63, 64, 65, 127, 128, 129, 1, 31, 33], [257, 640]])
 @pytest.mark.parametrize("ac", [False, True])
 @pytest.mark.parametrize("d", [32, 64, 128, 256])
-def test_ragged_documents(lengths, ac, d):
+def test_ragged_documents(lengths, ac, d, kernels):
     T = sum(lengths)
     q, k, v, do = orc.make_inputs((3, T, d), 7 + T + d, dist="upstream")
     g = torch.Generator().manual_seed(T)
@@ -202,7 +202,7 @@ def test_empty_documents_and_tail_tokens():
 
 @pytest.mark.parametrize("ac", [False, True])
 @pytest.mark.parametrize("d", [32, 64, 128, 256])
-def test_key_tile_group_boundaries(d, ac, monkeypatch):
+def test_key_tile_group_boundaries(d, ac, monkeypatch, kernels):
     """Document lengths on both sides of every boundary of the dk/dv pass's tile grouping (all key
     tiles of a document of up to 256 tokens and the last tile of a longer one go to the four-wave
     kernel at head_dim 64): 1, 32, 33, 128, 129, 255, 256, 257, 384, 385 tokens, with a gradient
@@ -246,7 +246,7 @@ def test_upstream_varlen_grid(H, L, ac):
 @pytest.mark.parametrize("ac", [False, True])
 @pytest.mark.parametrize("B,H,T,d", [(2, 3, 500, 64), (1, 7, 256, 64), (2, 2, 1024, 128), (2, 3, 700, 32), (1, 2, 2048, 32),
                                      (2, 2, 700, 256)])
-def test_fixed_length(B, H, T, d, ac):
+def test_fixed_length(B, H, T, d, ac, kernels):
     from stickbreaking_attention import sb_attn
     q, k, v, do = orc.make_inputs((B, H, T, d), 5 + T, dist="upstream")
     qg, kg, vg = (t.to(DEV).requires_grad_() for t in (q, k, v))

@@ -34,7 +34,7 @@ def _need_gpu():
 
 
 @pytest.mark.parametrize("case", range(60))
-def test_random_case(case):
+def test_random_case(case, kernels):
     from stickbreaking_attention import sb_attn_varlen, sb_attn_varlen_fused
     rng = random.Random(9000 + case)
     lengths = [rng.choice(EDGES) if rng.random() < 0.7 else rng.randint(1, 900) for _ in range(rng.choice([1, 2, 3, 5, 9]))]
