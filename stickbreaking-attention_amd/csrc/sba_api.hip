@@ -295,7 +295,7 @@ int forward(const sba_problem* p, bool fixed, const void* schedule, size_t sched
   a.weights = weights;
   // (the grid may hold a few slots more than there are items)
   const long long cus = device_cus(), items = (fixed ? (long long)p->batch * ((p->tokens + BM - 1) / BM) : sz.rows / BM) * p->heads;
-  a.resident = items > cus && items <= fwd_per_cu(p->head_dim) * cus && (cus & (cus - 1)) == 0 ? __builtin_ctzll(cus) : NO_DEAL;
+  a.lg_deal = items > cus && items <= fwd_per_cu(p->head_dim) * cus && (cus & (cus - 1)) == 0 ? __builtin_ctzll(cus) : NO_DEAL;
   a.heads_inv = 0xffffffffu / (unsigned)p->heads;
   a.n_items = (int)std::min<long long>(0x7fffffff, (long long)sz.n_q_max * p->heads);
   a.clear_spare = fixed ? 0 : 1;

@@ -50,7 +50,7 @@ __global__ void __launch_bounds__(NT, D > 128 ? 2 : 3) fwd_kernel(const KArgs a)
   // Header words and this workgroup's tile are fetched together (the grid never exceeds the
   // allocated list, so the tile read is safe before the count is known): one round trip.
   const int* sched = a.sched;
-  const unsigned item = deal_item(a.resident, a.n_items), below = __umulhi(item, a.heads_inv);   // (the quotient or one less)
+  const unsigned item = deal_item(a.lg_deal, a.n_items), below = __umulhi(item, a.heads_inv);   // (the quotient or one less)
   const int over = (int)(item - below * a.heads) >= a.heads ? 1 : 0, slot = below + over, head = item - slot * a.heads;
   const int4 hdr = *reinterpret_cast<const int4*>(sched);   // status, query tiles, key tiles, table entries needed
   const Tile t = reinterpret_cast<const Tile*>(sched + SCHED_HDR)[slot];

@@ -38,13 +38,13 @@ struct KArgs {
   unsigned* work;              // work counters of the backward's persistent launch (WORK_WORDS words at the end of the
                                // gradient table; the dq pass clears them), or null: one workgroup per work item
   int n_items;                 // work items of this launch (what the grid is with one workgroup per item)
-  int resident;                // backward, host side: workgroups of a persistent launch (0: never persistent); forward: the
-                               // logarithm of the device's compute units if it holds the launch at once (see deal_item), or NO_DEAL
+  int resident;                // backward, host side: workgroups of a persistent launch (0: never persistent)
   int min_items_each;          // host side: a launch is persistent when it has this many items per workgroup
+  int lg_deal;                 // forward: the logarithm of the device's compute units if it holds the launch at once (see deal_item), or NO_DEAL
 };
 
+constexpr int NO_DEAL = 31;    // (no launch has a second round of 2^31 workgroups)
 // Workgroups of the forward that a compute unit holds.
-constexpr int NO_DEAL = 31;
 inline int fwd_per_cu(int head_dim) { return head_dim <= 32 ? 6 : (head_dim <= 64 ? 4 : (head_dim <= 128 ? 3 : 2)); }
 
 // Arguments of the one-pass backward (sba_chain.hip).
