@@ -39,20 +39,31 @@ MEASURED = {"sba_version": 214,
             "c2": {"fwd_kernel": {"traffic": 1.129e8, "mfma_busy": 0.254, "valu_busy": 0.561, "coexec": 0.151},
                    "bwd_chain_kernel": {"traffic": 6.494e8, "mfma_busy": 0.228, "valu_busy": 0.464, "coexec": 0.114}}}
 
-KERNELS = ["fwd_kernel", "bwd_dq_kernel", "bwd_dkdv_kernel"]
-# algorithmic and executed FLOPs per causal pair and head_dim of each, and of the backward in one kernel, which takes the
-# last one's place (and its event pair) where the library chooses it: no dq pass is recorded then
+# algorithmic and executed FLOPs per causal pair and head_dim of a forward and of the backward's two passes
 ALGORITHMIC, EXECUTED = [4.0, 6.0, 4.0], [4.0, 6.0, 8.0]
-CHAINED, SHORT = "bwd_chain_kernel", "bwd_short_kernel"   # (the second: documents of at most 256 tokens at head_dim <= 64; it forms the scores twice)
+
+
+def kernel_names(product, d, heads, lengths, fixed):
+    """What the library launches for a workload's forward, dq pass, dk/dv pass and a backward in one kernel, by its own account."""
+    from stickbreaking_attention import _native as nat, _ops
+    flags = (nat.FLAG_PRODUCT_SPACE if product else 0) | _ops.FORWARD_FLAGS
+    p = (nat.SbaProblem(nat.SBA_BF16, d, heads, len(lengths), lengths[0], 0, lengths[0], flags | nat.FLAG_FIXED_LENGTH, 1.0, None) if fixed else
+         nat.SbaProblem(nat.SBA_BF16, d, heads, 1, sum(lengths), len(lengths), max(lengths), flags, 1.0, 16))
+    g = nat.SbaGeometry()
+    nat.check(nat.load().sba_launch_geometry(ctypes.byref(p), ctypes.byref(g)), "sba_launch_geometry")
+    passes = "_small" if g.bwd_small_workgroups else ("_wide" if d > 128 else "")
+    return ["fwd_small_kernel" if g.fwd_small_workgroups else "fwd_kernel", f"bwd_dq{passes}_kernel", f"bwd_dkdv{passes}_kernel",
+            "bwd_short_kernel" if g.bwd_short_workgroups else "bwd_chain_kernel"]
 
 
 def kernel_figures(m):
-    """[(name, ms, algorithmic, executed, tensors moved)] of a measured workload's kernels."""
+    """[(name, ms, algorithmic, executed, tensors moved)] of a measured workload's kernels.  A backward in one kernel has the event
+    pair of the dk/dv pass, and no dq pass is recorded; that of short documents forms the scores twice."""
+    names = m["kernels"]
     if m["backward"] and m["kern_ms"][1] == 0.0:
-        short = max(m["lengths"]) <= (256 if m["d"] <= 64 else 64)
-        return [(KERNELS[0], m["kern_ms"][0], 4.0, 4.0, 4.0),
-                (SHORT if short else CHAINED, m["kern_ms"][2], 10.0, 14.0 if short else 10.0, 7.0)]
-    return [(n, m["kern_ms"][i], ALGORITHMIC[i], EXECUTED[i], [4.0, 5.0, 6.0][i]) for i, n in enumerate(KERNELS)]
+        return [(names[0], m["kern_ms"][0], 4.0, 4.0, 4.0),
+                (names[3], m["kern_ms"][2], 10.0, 14.0 if names[3] == "bwd_short_kernel" else 10.0, 7.0)]
+    return [(n, m["kern_ms"][i], ALGORITHMIC[i], EXECUTED[i], [4.0, 5.0, 6.0][i]) for i, n in enumerate(names[:3])]
 
 
 def workload(name):
@@ -133,7 +144,7 @@ def cpu_baseline(lengths, d):
 def measure(name, steps, warmup, args, torch, lib, lengths_override=None):
     """Times one workload; returns a dict of raw figures."""
     from oracle import sb_oracle as orc
-    from stickbreaking_attention import sb_attn, sb_attn_fused, sb_attn_varlen, sb_attn_varlen_fused
+    from stickbreaking_attention import _ops, sb_attn, sb_attn_fused, sb_attn_varlen, sb_attn_varlen_fused
     dev = torch.device("cuda:0")
     lengths, cfg = workload(name)
     if lengths_override:
@@ -229,7 +240,8 @@ def measure(name, steps, warmup, args, torch, lib, lengths_override=None):
     del q, k, v, do
     torch.cuda.empty_cache()
     return dict(name=name, lengths=lengths, cfg=cfg, H=H, d=d, T=T, fixed=fixed, backward=backward, pairs=pairs,
-                tensor_bytes=tensor_bytes, ms_step=ms_step, ms_fwd=ms_fwd, kern_ms=kern_ms, ramp_steps=ramp_steps)
+                tensor_bytes=tensor_bytes, ms_step=ms_step, ms_fwd=ms_fwd, kern_ms=kern_ms, ramp_steps=ramp_steps,
+                kernels=kernel_names(_ops.PRODUCT_SPACE, d, H, lengths, fixed))
 
 
 def roofline(m, lib):
