@@ -158,6 +158,8 @@ size_t sba_table_bytes_for_lengths(const sba_problem* p, const int64_t* doc_leng
  * SBA_E_WORKSPACE.  The first int32 of the workspace is a status word (0 = ok, else
  * SBA_STATUS_*) and the fourth the number of table entries per head the documents need, both
  * readable by the caller after the stream has drained (the seventh: the longest document found).
+ * What is listed depends on the documents alone, and a schedule serves every problem on them; the order
+ * of the query tiles, which only decides how fast they are worked off, also goes by `heads` and `head_dim`.
  * Has no upstream counterpart as a
  * separate call: upstream derives the tile of a program from its grid index inside `_forward`
  * (sb_varlen_fwd.py:281-296). */

@@ -270,6 +270,18 @@ int short_parts(const sba_problem* p, bool fixed, const Sizes& sz) {
   return (int)(alone + (sz.n_docs - alone + 1) / 2 + 1);
 }
 
+// Whether the query tiles of documents of like length are listed tile-major (see sched_kernel): in launches of up to four rounds of the
+// chip.  What is gained is the launch's end, where document-major the last document's most expensive tile starts late; what it
+// costs is that the tiles of a (document, head) that are under way at a time share its K/V rows in the caches with the fewer others the more
+// documents and heads there are.  Forward, us, document-major / tile-major, head_dim 128, items (tiles x heads) at 768 a round: 12 heads of 4 x 4096
+// (1536) 249 / 200, 8 of 8 x 4096 (2048) 305 / 256, 12 of 8 x 4096 (3072) 440 / 377, 16 of 8 x 4096 (4096) 545 / 524; but 32 heads of 8 x 2048 (4096)
+// 291 / 341, 12 of 16 x 4096 (6144) 848 / 920, 32 of 8 x 4096 (8192) 1069 / 1410.  head_dim 64 (1024 a round): 8 heads of 16 x 4096 (4096) 352 / 306, 32 of
+// 16 x 2048 (8192) 338 / 365.  head_dim 256 (512 a round): 8 heads of 8 x 4096 (2048) 584 / 533, 32 of 8 x 2048 (4096) 579 / 629.
+bool list_in_classes(const sba_problem* p, const Sizes& sz) {
+  const int cus = device_cus();
+  return sz.rows / BM * p->heads <= 4ll * fwd_per_cu(p->head_dim) * (cus > 0 ? cus : 256);
+}
+
 int forward(const sba_problem* p, bool fixed, const void* schedule, size_t sched_bytes, const sba_view* q,
             const sba_view* k, const sba_view* v, const sba_view* o, const sba_view* rem, float* stick,
             size_t table_bytes, float* weights, size_t weights_bytes, void* stream, bool timed = true) {
@@ -585,6 +597,7 @@ int sba_build_schedule(const sba_problem* p, void* schedule, size_t schedule_siz
   a.tokens = p->tokens;
   a.n_q_max = sz.n_q_max;
   a.n_kv_max = sz.n_kv_max;
+  a.classes = !fixed && list_in_classes(p, sz);
   a.out = reinterpret_cast<int*>(schedule);
   return (int)launch_schedule(a, reinterpret_cast<hipStream_t>(stream));
 }

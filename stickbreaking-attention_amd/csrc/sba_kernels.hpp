@@ -134,6 +134,7 @@ struct SchedArgs {
   int n_docs;       // documents (fixed: batch)
   int tokens;       // T per batch entry
   int n_q_max, n_kv_max;
+  int classes;      // query tiles of documents of like length are listed tile-major
   int* out;
 };
 

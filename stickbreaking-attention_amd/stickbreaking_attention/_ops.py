@@ -390,7 +390,8 @@ def _check_cu(cu_seqlens: torch.Tensor, like: torch.Tensor) -> torch.Tensor:
 # Schedules already built on a device: the tile lists depend only on the documents (cu_seqlens, or
 # batch and length of a fixed-length call) and on the token count, and a model hands the same
 # cu_seqlens tensor to every layer, so the scheduler kernel runs once per tensor instead of once per
-# layer.  Entries: (weak reference to cu_seqlens or None, its version, key, schedule tensor), newest
+# layer.  (The order of the lists, not what is in them, also goes by the heads and head_dim of the call
+# that builds them.)  Entries: (weak reference to cu_seqlens or None, its version, key, schedule tensor), newest
 # last; the key holds the stream, so a schedule is only ever reused behind the launch that wrote it.
 # An entry is made once that launch is on its stream (`_schedule_built`) and not before: a call can
 # fail on its way there (an output that does not fit, a head_dim that is refused), and what it

@@ -19,14 +19,14 @@ DEV = "cuda:0"
 HDR, TILE_WORDS = 16, 8
 
 
-def _schedule(lengths, tokens, fixed_batch=0):
+def _schedule(lengths, tokens, fixed_batch=0, heads=2, head_dim=64):
     lib = nat.load()
     if fixed_batch:
         prob = nat.SbaProblem(nat.SBA_BF16, 64, 2, fixed_batch, tokens, 0, tokens, nat.FLAG_FIXED_LENGTH, 0.125, None)
         n_docs, rows = fixed_batch, fixed_batch * tokens
     else:
         cu = helpers.cu_from_lengths(lengths, device=DEV)
-        prob = nat.SbaProblem(nat.SBA_BF16, 64, 2, 1, tokens, cu.numel(), max(lengths + [1]), 0, 0.125, cu.data_ptr())
+        prob = nat.SbaProblem(nat.SBA_BF16, head_dim, heads, 1, tokens, cu.numel(), max(lengths + [1]), 0, 0.125, cu.data_ptr())
         n_docs, rows = len(lengths), tokens
     nbytes = lib.sba_schedule_bytes(ctypes.byref(prob))
     sched = torch.zeros(nbytes, dtype=torch.uint8, device=DEV)

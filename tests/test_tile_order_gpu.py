@@ -11,6 +11,7 @@ from tests.test_schedule_gpu import DEV, _schedule
 
 pytestmark = pytest.mark.gpu
 CLASS_TILES = 4
+PER_CU = {32: 6, 64: 4, 128: 3, 256: 2}      # workgroups of the general forward that a compute unit holds
 
 
 def _listed(lengths):
@@ -37,11 +38,21 @@ def _listed(lengths):
                                      [random.Random(5).randint(1, 3000) for _ in range(40)],
                                      [random.Random(6).choice([200, 400, 500, 900]) for _ in range(600)]])
 def test_order_of_the_list(lengths):
-    _, q_tiles, _, _ = _schedule(lengths, sum(lengths))
+    _, q_tiles, _, _ = _schedule(lengths, sum(lengths), heads=1)
     assert [(t[1], t[2]) for t in q_tiles] == _listed(lengths)
 
 
-PER_CU = {32: 6, 64: 4, 128: 3, 256: 2}      # workgroups of the general forward that a compute unit holds
+@pytest.mark.parametrize("head_dim", list(PER_CU))
+@pytest.mark.parametrize("lengths", [[4096] * 4, [1024, 1000, 769, 768, 767, 500]])
+def test_long_launches_are_listed_document_by_document(head_dim, lengths):
+    """Beyond four rounds of the chip, where the tiles of a document find its K/V rows in the caches: the longest first."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    most = 4 * PER_CU[head_dim] * cus // (sum(lengths) // 128)          # heads that four rounds hold
+    by_document = [(n, i) for n in sorted(lengths, reverse=True) for i in range(-(-n // 128) - 1, -1, -1)]
+    assert by_document != _listed(lengths)
+    for heads, want in ((most, _listed(lengths)), (most + 1, by_document)):
+        _, q_tiles, _, _ = _schedule(lengths, sum(lengths), heads=heads, head_dim=head_dim)
+        assert [(t[1], t[2]) for t in q_tiles] == want
 
 
 @pytest.mark.parametrize("heads,head_dim,lengths", [(12, 64, [1500, 700, 129, 2100]), (20, 32, [3000, 1, 1111]), (7, 128, [4096, 900]),
