@@ -271,15 +271,16 @@ int short_parts(const sba_problem* p, bool fixed, const Sizes& sz) {
 }
 
 // Whether the query tiles of documents of like length are listed tile-major (see sched_kernel): in launches of up to four rounds of the
-// chip.  What is gained is the launch's end, where document-major the last document's most expensive tile starts late; what it
-// costs is that the tiles of a (document, head) that are under way at a time share its K/V rows in the caches with the fewer others the more
-// documents and heads there are.  Forward, us, document-major / tile-major, head_dim 128, items (tiles x heads) at 768 a round: 12 heads of 4 x 4096
-// (1536) 249 / 200, 8 of 8 x 4096 (2048) 305 / 256, 12 of 8 x 4096 (3072) 440 / 377, 16 of 8 x 4096 (4096) 545 / 524; but 32 heads of 8 x 2048 (4096)
-// 291 / 341, 12 of 16 x 4096 (6144) 848 / 920, 32 of 8 x 4096 (8192) 1069 / 1410.  head_dim 64 (1024 a round): 8 heads of 16 x 4096 (4096) 352 / 306, 32 of
-// 16 x 2048 (8192) 338 / 365.  head_dim 256 (512 a round): 8 heads of 8 x 4096 (2048) 584 / 533, 32 of 8 x 2048 (4096) 579 / 629.
+// chip, and of more the fewer heads there are.  What is gained is the launch's end, where document-major the last document's most expensive tile
+// starts late: the less the more rounds there are.  What it costs is that the tiles of a (document, head) that are under way at a time share its
+// K/V rows in the caches with fewer others, the more heads (and documents) there are.  The line is that of 456 shapes of equal documents (two rounds and more, 1 to 32 heads, 512 to 32768
+// tokens, head_dim 64, 128 and 256, forward and dq pass): 1.067 times as fast as document-major by the geometric mean, tile-major always 1.050.
+// Forward, us, document-major / tile-major, head_dim 128: 12 heads of 4 x 4096 (2 rounds) 249 / 200, 8 of 8 x 4096 (2.7) 305 / 256, 12 of 8 x 4096 (4)
+// 440 / 377, 2 of 16 x 8192 (2.7) 616 / 484; left out 16 heads of 4 x 8192 (5.3) 985 / 1020, 32 of 8 x 2048 (5.3) 291 / 341, 32 of 8 x 4096 (10.7) 1069 / 1410.
 bool list_in_classes(const sba_problem* p, const Sizes& sz) {
   const int cus = device_cus();
-  return sz.rows / BM * p->heads <= 4ll * fwd_per_cu(p->head_dim) * (cus > 0 ? cus : 256);
+  const long long items = sz.rows / BM * p->heads, round = (long long)fwd_per_cu(p->head_dim) * (cus > 0 ? cus : 256);
+  return items <= 4 * round || items * p->heads <= 48 * round;
 }
 
 int forward(const sba_problem* p, bool fixed, const void* schedule, size_t sched_bytes, const sba_view* q,

@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
   // D. emit tiles: slot -> ranked document by binary search over the prefix
   // The hardware deals workgroups to the CUs round-robin in launch order (workgroups i and
   // i + number of CUs start on the same CU and run side by side), and hands out the rest as
-  // slots free up.  Where the launch is short (list_in_classes), documents of like length -- a class: more than three quarters of the tiles of its longest -- are therefore
+  // slots free up.  Where the launch is short or the heads are few (list_in_classes), documents of like length -- a class: more than three quarters of the tiles of its longest -- are therefore
   // listed tile-major, the most expensive tile of every document first: the expensive tiles start together and the cheap
   // ones fill in behind them.  Document-major, the last document's most expensive tile starts when most of the launch is
   // over, and documents of one length put the same tile on the same CU.  Classes follow one another,

@@ -43,11 +43,13 @@ def test_order_of_the_list(lengths):
 
 
 @pytest.mark.parametrize("head_dim", list(PER_CU))
-@pytest.mark.parametrize("lengths", [[4096] * 4, [1024, 1000, 769, 768, 767, 500]])
+@pytest.mark.parametrize("lengths", [[4096] * 4, [1024, 1000, 769, 768, 767, 500], [32768] * 16])
 def test_long_launches_are_listed_document_by_document(head_dim, lengths):
-    """Beyond four rounds of the chip, where the tiles of a document find its K/V rows in the caches: the longest first."""
+    """Beyond four rounds of the chip, or beyond 48 for rounds x heads where that is more, the tiles of a document follow one another."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    most = 4 * PER_CU[head_dim] * cus // (sum(lengths) // 128)          # heads that four rounds hold
+    rounds = lambda heads: sum(lengths) // 128 * heads / (PER_CU[head_dim] * cus)
+    most = max(h for h in range(1, 400) if rounds(h) <= 4 or rounds(h) * h <= 48)
+    assert (rounds(most) > 4) == (len(lengths) == 16)
     by_document = [(n, i) for n in sorted(lengths, reverse=True) for i in range(-(-n // 128) - 1, -1, -1)]
     assert by_document != _listed(lengths)
     for heads, want in ((most, _listed(lengths)), (most + 1, by_document)):
