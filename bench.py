@@ -33,11 +33,11 @@ PEAK_HBM_GBS = 8000.0       # MI355X published HBM3E bandwidth
 #     (SQ_VALU_MFMA_BUSY_CYCLES), a vector instruction is active (4 x SQ_ACTIVE_INST_VALU) and both at once
 #     (SQ_VALU_MFMA_COEXEC_CYCLES), over 1024 SIMDs x GRBM_GUI_ACTIVE / 8: profiles/c3_sq_counters_pmc.txt
 #   (c2: profiles/c2_one_pass_backward.txt)
-MEASURED = {"sba_version": 214,
-            "c3": {"fwd_kernel": {"traffic": 9.668e8, "mfma_busy": 0.464, "valu_busy": 0.552, "coexec": 0.192},
-                   "bwd_chain_kernel": {"traffic": 7.886e9, "mfma_busy": 0.344, "valu_busy": 0.377, "coexec": 0.103}},
-            "c2": {"fwd_kernel": {"traffic": 1.129e8, "mfma_busy": 0.254, "valu_busy": 0.561, "coexec": 0.151},
-                   "bwd_chain_kernel": {"traffic": 6.494e8, "mfma_busy": 0.228, "valu_busy": 0.464, "coexec": 0.114}}}
+MEASURED = {"sba_version": 215,
+            "c3": {"fwd_kernel": {"traffic": 1.065e9, "mfma_busy": 0.457, "valu_busy": 0.544, "coexec": 0.188},
+                   "bwd_chain_kernel": {"traffic": 7.863e9, "mfma_busy": 0.349, "valu_busy": 0.382, "coexec": 0.106}},
+            "c2": {"fwd_kernel": {"traffic": 1.135e8, "mfma_busy": 0.254, "valu_busy": 0.561, "coexec": 0.150},
+                   "bwd_chain_kernel": {"traffic": 6.487e8, "mfma_busy": 0.227, "valu_busy": 0.461, "coexec": 0.114}}}
 
 # algorithmic and executed FLOPs per causal pair and head_dim of a forward and of the backward's two passes
 ALGORITHMIC, EXECUTED = [4.0, 6.0, 4.0], [4.0, 6.0, 8.0]

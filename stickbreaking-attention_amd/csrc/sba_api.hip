@@ -232,9 +232,10 @@ bool small_wins(const SmallCost* costs, double gain, const sba_problem* p, bool 
   const double small = c.small_base + 2.0 * spare + std::max(c.round * longest / round, groups * (c.group + c.per_round * (0.5 * typical / round + 0.5)));
   return std::max(gain * small, small + 2.0) < c.base + c.step * longest / 32;
 }
-// Of the problems taken all gain (head_dim 64: 4 heads x 512 14.4 / 9.7, 16 x 4096 78 / 68, 32 x 1024 24 / 17.5), and of those left to fwd_kernel none
-// would gain more than a tenth (head_dim 64: 16 heads of 4 x 1024 25.6 / 28, 32 x 2048 43 / 40; head_dim 128: 32 x 2048 58 / 74; head_dim 256, whose line serves 129 on:
-// taken 4 x 512 28 / 18, 16 x 1024 48 / 35, left out 16 x 2048 89 / 95, 32 x 512 29 / 27.5).
+// Of 164 problems (general / few tiles, us) none of the 44 taken loses and they gain 1.41 by the geometric mean (head_dim 64: 4 heads x 512 14.4 / 9.7, 16 x 4096 80 / 68,
+// 32 x 1024 23.5 / 17.2; head_dim 256, whose line serves 129 on: 4 x 512 28 / 17, 16 x 1024 48 / 34).  Of the 120 left to fwd_kernel eight would gain more than a tenth, up to
+// 1.24 (12 heads x 3001 tokens in 17 documents 20.8 / 17.7, 13 heads of 2 x 1360 30.2 / 24.5): `base` and `step` are those of a document alone.  Most lose (head_dim 64: 16 heads of
+// 4 x 1024 24.8 / 26.9; head_dim 128: 32 x 2048 57 / 73; head_dim 256: 16 x 2048 88 / 95) or gain less than 4 x the workgroups may cost (32 x 2048 at 64 42 / 39).
 bool forward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
   if (p->flags & SBA_GENERAL_FORWARD) return false;
   if (p->flags & SBA_FEW_TILES_FORWARD) return (p->flags & SBA_PRODUCT_SPACE) && sz.n_docs > 0;
