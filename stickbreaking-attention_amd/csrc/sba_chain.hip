@@ -21,16 +21,25 @@
 //
 // Order and progress.  Queries are walked from the document's end down to the tile's own keys, so that the
 // tiles of a chain start together and end one after the other; the items of a queue are ordered by key tile, so
-// the item an item waits for was drawn before it by a workgroup that is running: waits end.  A tile is
-// published three steps after it was formed (`flags`: steps done per item).
+// the item an item waits for was drawn before it by a workgroup that is running: waits end.  `flags` holds a number per
+// item: at the start of step t a tile publishes t - 2, which stands for the carried sums of its blocks up to t - 2 (formed two
+// steps ago) and the partial dq of those up to t - 3 (formed by the product waves a step after the sums); both have been
+// acknowledged by then.  Step s asks for the carried sum of block s + 1 and the partial dq of block s, so it needs s + 1: a
+// tile runs three steps behind the one before (it was four while a sum was published no earlier than its block's dq).  What the tile
+// before has published is copied to LDS in the background, a step old when it is looked at; only where that is not
+// enough does a score wave -- the one all others wait for -- stop to ask.
 //
-// Measured (kernel time of the backward, two passes -> prep and chain, alternating on one MI355X): 32 heads x 16 K tokens in
-// eight documents, head_dim 128, 1560 -> 1411 us (forward and backward as a program calls them: 1979 -> 1856); 12 x 4 x 4096
-// fused 819 -> 716; 16 x 7001 in six documents, head_dim 96, 187 -> 177; 4 x 16 x 2048, head_dim 64, 213 -> 167; 1 x 4 x 512,
-// head_dim 64, 45 -> 36.  At head_dim 128 it waits: 41 % of the wave cycles on 32 heads x 16 K tokens (22 .. 25 % in the two
-// passes; profiles/c3_sq_counters_pmc.txt), with the matrix pipe busy for 34 %.  Such a launch fetches 4.7 GB from behind
-// the L2s and writes 3.1 GB there, 6.0 TB/s where a plain copy reaches 4.9: of the 2.8 GB of partial dq each way, all
-// that is written leaves L2 (eight chains of 2 MiB share 4 MiB).
+// Measured (kernel time of the backward with its prep kernel, before and after the shorter lag, the poll in the background and leaner
+// product waves, alternating on one MI355X): 32 heads x 16 K tokens in eight documents, head_dim 128, 1311 -> 1292 us; 12 x 4 x 4096
+// 694 -> 683; 16 x 7 K in six documents, head_dim 96, 240 -> 226; 12 heads of 1500, 900 and 601 tokens, head_dim 64, 80.0 -> 69.8
+// and 128, 95.8 -> 88.   At head_dim 128 it waits: 41 % of the wave
+// cycles on 32 heads x 16 K tokens (22 .. 25 % in the two passes; profiles/c3_sq_counters_pmc.txt), with the matrix pipe busy for
+// 34 %.  Such a launch fetches 4.7 GB from behind the L2s and writes 3.1 GB there, 6.0 TB/s where a plain copy reaches 4.9: of the
+// 2.8 GB of partial dq each way, all that is written leaves L2 (eight chains of 2 MiB share 4 MiB).
+//
+// What does not help: waves that are all alike.  Eight of them with 256 registers (steps of 64 queries, two barriers) took 1510 us at
+// head_dim 96 where this takes 1130, four with 512 registers and every matrix instruction placed by hand 1235: a wave alone on its
+// SIMD issues for 56 % of its cycles and has nothing to cover the rest.
 //
 // Carried sum: with C[j] the sum of G over the keys up to j and ex the stick on entering a key, D = C + drem ex
 // obeys D[j] = D[j-1] + p_j (do.v_j) and dz_j = r_j D[j] - D[j-1] (see grad_dz in sba_bwd.hip); the gradient of
@@ -110,6 +119,12 @@ __global__ void __launch_bounds__(NT) chain_prep_kernel(const ChainArgs a) {
 // 128 registers leave room for one score wave per SIMD, whose vector work (180 instructions, 32 of them transcendental,
 // per block) is the step; at 64 and below two fit (168 registers): 16 heads x 4 documents of 2048 at head_dim 64 in steps of 64
 // queries 167 us for 198 in steps of 32, at head_dim 32 139 for 169 (two passes: 213, 174).
+// One dword, the same for every lane, to LDS at dst + 4 * lane.  Counted by vmcnt like async_copy16.
+__device__ __forceinline__ void async_word(const int* from, const int* dst) {
+  const unsigned lds_addr = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2 sc1" ::"s"(lds_addr), "v"(0), "s"(from) : "memory", "m0");
+}
+
 template <int D, int U, bool AC, int NSQ>
 __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const ChainArgs a) {
   constexpr int KS = U / 16, DB = U / 32;
@@ -128,6 +143,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
   __shared__ int prefix[CHAIN_MAX_GROUPS];   // key tiles of the longest chains, up to and including each group's
   __shared__ int place;                      // this XCD's number among those that serve a queue, their count (bits 8 ..)
   __shared__ int mbox[2][8];
+  __shared__ int fbox[64];                   // what the tile before this one had published a step ago
   __shared__ __attribute__((aligned(16))) unsigned short spare[4][512];   // where a product wave's copies of nothing go
   unsigned short* const Ps = PZ;
   unsigned short* const Zs = PZ + PBUF * PTILE;
@@ -252,6 +268,8 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
   Item cur;
   if (!read_box(1, cur)) return;
 
+  using Yes = std::true_type;
+  using No = std::false_type;
   if (scorer) {
     __builtin_amdgcn_s_setprio(3);
     const int kb = w & 3, sq = w >> 2;            // 32-key block and 32-query block of this wave
@@ -330,8 +348,9 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
     };
     // First score wave: the tile before this one has published `steps` steps (all of them: nothing to wait for any more).
     // A wait that runs out -- it cannot while workgroups make progress -- must end in NaN and not in plausible numbers, in
-    // every wave: what it stood for is requested by all of them behind the barrier that follows.  The waves of the oldest
-    // key block add `given_up` to the stick of the block whose weights they form next, the first that is in doubt: its p
+    // every wave: what it stood for is requested by all of them behind the barrier that follows, the partial dq of the block
+    // whose dz is formed there and the carried sum of the next one.  The waves of the oldest key block add `given_up` to that dz,
+    // which makes all of the block's dq NaN, and to the stick of the next block, whose weights they form in the same step: its p
     // and dz are NaN, so is the sum every newer key block takes from `tot` for its D, and with dz of all of the tile's
     // keys dk, dq and what is handed on.
     auto await = [&](int steps) {
@@ -396,8 +415,9 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         if (kb > 2) t2 = tot[par][sq][2][n];
       }
       request_d(w + 1);
-      float e_in = se;
-      if (kb == 0) e_in += given_up;
+      float e_in = se, doubt = 0.0f;
+      if (kb == 0) doubt = given_up;
+      e_in += doubt;
       request_e(w + 4, se);
       const unsigned short* Qt = Qs + slot * QTILE;
       const unsigned short* Gt = Gs + slot * QTILE;
@@ -442,7 +462,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       pre(2);
       const int row = n;
       if constexpr (!FIRST) {
-        const float before = d_in + ((t0 + t1) + t2);
+        const float before = (d_in + doubt) + ((t0 + t1) + t2);
         float dprev = h == 1 ? before + wc.lo : before;
         float dz[16];
 #pragma unroll
@@ -514,8 +534,9 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         if (kb > 2) t2 = tot[par][sq][2][n];
       }
       request_d(w + 1);
-      float e_in = se;
-      if (kb == 0) e_in += given_up;
+      float e_in = se, doubt = 0.0f;
+      if (kb == 0) doubt = given_up;
+      e_in += doubt;
       request_e(w + 3, se);
       const unsigned short* Qt = Qs + slot * QTILE;
       const unsigned short* Gt = Gs + slot * QTILE;
@@ -540,7 +561,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       pre(1);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (!FIRST) {
-        const float before = d_in + ((t0 + t1) + t2);
+        const float before = (d_in + doubt) + ((t0 + t1) + t2);
         float dprev = h == 1 ? before + wc.lo : before;
         float dz[16];
 #pragma unroll
@@ -588,12 +609,18 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       if constexpr (BAND && !FIRST) hide(qw0, par);
     };
     // ends a step: the first score wave makes sure that what the others request behind the barrier is there, the second
-    // publishes what this tile has finished (formed two steps ago and acknowledged since)
+    // publishes what this tile has finished and, before a step, asks in the background how far the tile before is
     auto finish = [&](int w) {
-      if (sq == 0 && kb == 0 && n_wait > 0) await(w + 3);
+      // (what a step issues: two requests and this store)
+      if (kb == 3) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");     // the carried sum stored a step ago is acknowledged
+      if (sq == 0 && kb == 0 && n_wait > 0) {
+        if (seen < min(w + 2, n_wait)) seen = max(seen, __builtin_amdgcn_readfirstlane(fbox[0]));
+        await(w + 2);
+      }
       lds_barrier();
     };
     auto publish = [&](int w) {
+      if (sq == 0 && kb == 0 && seen < min(w + 2, n_wait)) async_word(pred, fbox);
       if (sq == 0 && kb == 1 && w >= 3 && lane == 0) __hip_atomic_store(mine, w - 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
     const bool keeper = w == 0;
@@ -607,8 +634,6 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
     };
 
     using std::integral_constant;
-    using Yes = std::true_type;
-    using No = std::false_type;
     using RT = integral_constant<int, -1>;
     open_item(a, cur);
     open_tiles(a, cur);
@@ -618,6 +643,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       wait_loads<0>();
       lds_barrier();                 // tiles 0 .. AHEAD-1 and the K and V tiles have landed
       take_fragments();
+      if (keeper) fbox[lane] = 0;
       lds_barrier();                 // every wave has its share of K and V in registers: their places are free
       if constexpr (DEEP) {
         f32x16 x0, x1, da0, da1, da2;
@@ -625,7 +651,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         chains(0, x0, da0);
         // weights of block 0 (as step -1), chains of block 1
         step(Yes{}, Yes{}, RT{}, -1, wb, da2, x0, da0, wa, x1, da1, se0);
-        if (keeper) await(2);
+        if (keeper) await(1);
         lds_barrier();
         int i = 0;
         // Everything repeats with period six (ring slots, staging buffers, weights, scores, do.v sums, carries): step i = 6 m has
@@ -658,7 +684,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         f32x16 da0, da1;
         Weights wa;
         shallow(Yes{}, Yes{}, -1, 0, wa, da1, da0, se0);
-        if (keeper) await(2);
+        if (keeper) await(1);
         lds_barrier();
         int i = 0, slot = 1;
         auto advance = [&]() { slot = slot + 1 == RING ? 0 : slot + 1; };
@@ -696,17 +722,20 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       for (int j = 0; j < DB; ++j)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[kb2][j][i] = 0.0f;
-    // Offsets (elements) of this lane's reads.  The swizzle is an XOR of the chunk number, so the offset of a further chunk
+    // Offsets (bytes) of this lane's reads.  The swizzle is an XOR of the chunk number, so the offset of a further chunk
     // is the first one's with a constant XORed in: one register per row instead of one per read -- there is none to
-    // spare, and a spilled one would be reloaded through the counter that the waits below count on.
+    // spare, and a spilled one would be reloaded through the counter that the waits below count on.  In bytes, and added to the
+    // tile's place as an integer: XOR and addition are then one instruction.
     int xb[2], yb[2];      // transpose reads of rows 8 h + 4 u + i16 / 4: staged block (chunk of key 64 half), tile (chunk of column 0)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int r = 8 * h + 4 * u + (i16 >> 2), c = 16 * blk + 4 * (i16 & 3);
-      xb[u] = swz_off<BKV>(r, (64 * half + c) >> 3) + (c & 7);
-      yb[u] = swz_off<D>(r, c >> 3) + (c & 7);
+      xb[u] = 2 * (swz_off<BKV>(r, (64 * half + c) >> 3) + (c & 7));
+      yb[u] = 2 * (swz_off<D>(r, c >> 3) + (c & 7));
     }
-    int zb = swz_off<BKV>(32 * dsq + n, h);      // row reads of staged dz: chunk 2 ks + h of row n
+    int zb = 2 * swz_off<BKV>(32 * dsq + n, h);      // row reads of staged dz: chunk 2 ks + h of row n
+    auto place_of = [](const unsigned short* p) { return (int)(unsigned)(size_t)p; };     // LDS address
+    auto tr8 = [](int at0, int at1) { return lds_tr8_at(at0, at1); };
     Copy qcopy, gcopy;
     qcopy.init(ptid, (unsigned)a.q.st * 2u, 2 * a.head_dim);
     gcopy.init(ptid, (unsigned)a.go.st * 2u, 2 * a.head_dim);
@@ -750,7 +779,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       if (has_dq) {
 #pragma unroll
         for (int ks = 0; ks < BKV / 16; ++ks)
-          kt_f[ks] = lds_tr8(PZ + (yb[0] ^ (dcol << 5)) + 16 * ks * D, PZ + (yb[1] ^ (dcol << 5)) + 16 * ks * D);
+          kt_f[ks] = tr8((yb[0] ^ (dcol << 6)) + place_of(PZ) + 32 * ks * D, (yb[1] ^ (dcol << 6)) + place_of(PZ) + 32 * ks * D);
       } else {
 #pragma unroll
         for (int ks = 0; ks < BKV / 16; ++ks) kt_f[ks] = zero8();
@@ -776,61 +805,80 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       // same order, with an offset outside the resource where there is nothing to store, request or copy, so that
       // the waits count constants and no value on its way has to be moved where two paths join.
       f32x4 l0, l1, l2, l3;           // partial dq on its way in
-      const unsigned short* const Ys = mat ? Qs : Gs;
       constexpr int KQ = TQ / 16, KZ = BKV / 16, ZH = DEEP ? KZ / 2 : 2;
-      auto store_part = [&](const int w, const int i, const f32x16& dq, const bool store) __attribute__((always_inline)) {
-        const f32x4 part = {dq[4 * i], dq[4 * i + 1], dq[4 * i + 2], dq[4 * i + 3]};
-        const int soff = ((t_last - w + 1) * NSQ + dsq) * (D * 128);    // bytes of partial dq ahead of this query tile's 32 rows
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, part), part_rs, (store ? lane16 : OUTSIDE) + 1024 * i, soff, 0);
-      };
+      constexpr int QB = 2 * QTILE, PB = 2 * PTILE;      // bytes of a tile, of a staged block
+      constexpr bool ALL_DQ = NSQ * DB >= 4;             // every product wave has a block of dq
       constexpr int FETCH_OPS = 4 + 2 * Copy::NCH;
-      auto fetch = [&](const int w, const int i) __attribute__((always_inline)) {
-        const int soff = (max(t_last - w, 0) * NSQ + dsq) * (D * 128);
-        const int l_off = has_dq && kt > 0 && w < nsteps ? lane16 : OUTSIDE;
-        if (i == 0) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen sc1" : "=&v"(l0) : "v"(l_off), "s"(part_rs), "s"(soff) : "memory");
-        if (i == 1) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:1024 sc1" : "=&v"(l1) : "v"(l_off), "s"(part_rs), "s"(soff) : "memory");
-        if (i == 2) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:2048 sc1" : "=&v"(l2) : "v"(l_off), "s"(part_rs), "s"(soff) : "memory");
-        if (i == 3) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:3072 sc1" : "=&v"(l3) : "v"(l_off), "s"(part_rs), "s"(soff) : "memory");
-        const bool fetched = w + AHEAD < nsteps;
-        const int row0 = (t_last - (w + AHEAD)) * TQ, slot = (w + AHEAD) % RING;
-        if (i >= 4 && i < 4 + Copy::NCH) qcopy.issue_one(qrows, row0, Qs + slot * QTILE, i - 4, fetched, spare[pw]);
-        if (i >= 4 + Copy::NCH && i < FETCH_OPS) gcopy.issue_one(grows, row0, Gs + slot * QTILE, i - 4 - Copy::NCH, fetched, spare[pw]);
+      constexpr int N_PRODUCTS = KQ * 2 * DB, REST = N_PRODUCTS - KZ / 2, OPS = 4 + FETCH_OPS;
+      // What a block needs besides its products: 45 vector and 41 scalar instructions an iteration (108 and about 100 with the places
+      // computed from the block's number and selects for what only an item's last iterations need).
+      // Places that move on with the blocks: staged blocks, tile read by dk / dv, ring slot that is copied to, and in memory the
+      // partial dq of the block that is stored and the rows that are copied.
+      const int y0 = place_of(mat ? Qs : Gs), x0 = place_of(mat ? Zs : Ps), x_end = x0 + (mat ? 2 : PBUF) * PB;
+      int y_at = y0, x_at = x0, z_at = place_of(Zs), c_at = AHEAD * QB;
+      int part_at = (t_last * NSQ + dsq) * (D * 128);                  // bytes of partial dq ahead of the next request's 32 rows
+      int q_row = (t_last - AHEAD) * TQ * (int)qrows.row_bytes, g_row = (t_last - AHEAD) * TQ * (int)grows.row_bytes;
+      const bool takes = has_dq && kt > 0;
+      auto store_part = [&](const int i, const f32x16& dq, const bool store) __attribute__((always_inline)) {
+        const f32x4 part = {dq[4 * i], dq[4 * i + 1], dq[4 * i + 2], dq[4 * i + 3]};
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, part), part_rs, (store ? lane16 : OUTSIDE) + 1024 * i, part_at + NSQ * D * 128, 0);
+        // The registers must not be written right behind the store.  The compiler leaves the wait state for that out where the
+        // store's offset is in a scalar register; an address computed into one by the next instruction was stored in its place
+        // in lanes 12 .. 15, now and then.  (The registers are an operand so that nothing else is put in between.)
+        asm volatile("s_nop 0" ::"v"(part) : "memory");
       };
-      auto read_y = [&](const unsigned short* Yt, const int j) { return lds_tr8(Yt + (yb[0] ^ (j << 5)), Yt + (yb[1] ^ (j << 5))); };
+      // operation i of those that request: partial dq of the block whose rows part_at names, then the tile AHEAD of it
+      auto fetch = [&](const int i, const bool more, const bool fetched) __attribute__((always_inline)) {
+        const int l_off = takes && more ? lane16 : OUTSIDE;
+        if (i == 0) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen sc1" : "=&v"(l0) : "v"(l_off), "s"(part_rs), "s"(part_at) : "memory");
+        if (i == 1) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:1024 sc1" : "=&v"(l1) : "v"(l_off), "s"(part_rs), "s"(part_at) : "memory");
+        if (i == 2) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:2048 sc1" : "=&v"(l2) : "v"(l_off), "s"(part_rs), "s"(part_at) : "memory");
+        if (i == 3) asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:3072 sc1" : "=&v"(l3) : "v"(l_off), "s"(part_rs), "s"(part_at) : "memory");
+        if (i >= 4 && i < 4 + Copy::NCH) qcopy.issue_at(qrows, q_row, Qs, c_at, i - 4, fetched, spare[pw]);
+        if (i >= 4 + Copy::NCH && i < FETCH_OPS) gcopy.issue_at(grows, g_row, Gs, c_at, i - 4 - Copy::NCH, fetched, spare[pw]);
+      };
+      // (the partial dq of queries older than the tile's own keys is never asked for: the row may not exist)
+      auto advance = [&]() {
+        part_at = max(part_at - NSQ * D * 128, 0);
+        c_at = c_at == (RING - 1) * QB ? 0 : c_at + QB;
+        q_row -= TQ * (int)qrows.row_bytes;
+        g_row -= TQ * (int)grows.row_bytes;
+      };
+      auto read_y = [&](const int at, const int j) { return tr8((yb[0] ^ (j << 6)) + at, (yb[1] ^ (j << 6)) + at); };
+      el8 bf[DB];       // columns of the tile for the next contraction step, the next block's first one included
       // iteration 0 has no block yet
 #pragma unroll
-      for (int i = 0; i < FETCH_OPS; ++i) fetch(0, i);
+      for (int i = 0; i < FETCH_OPS; ++i) fetch(i, true, AHEAD < nsteps);
+      advance();
+#pragma unroll
+      for (int j = 0; j < DB; ++j) bf[j] = read_y(y_at, j);
       lds_barrier();
-      constexpr int N_PRODUCTS = KQ * 2 * DB, REST = N_PRODUCTS - KZ / 2, OPS = 4 + FETCH_OPS;
-#pragma unroll 1
-      for (int w = 1; w <= nsteps; ++w) {
+      // TAIL: the item's last iterations, which have nothing left to copy, dq to finish, nothing to request in the end.
+      auto iteration = [&](auto tail_tag, const int w) __attribute__((always_inline)) {
+        constexpr bool TAIL = decltype(tail_tag)::value;
         asm volatile("" : "+v"(xb[0]), "+v"(xb[1]), "+v"(yb[0]), "+v"(yb[1]), "+v"(zb));   // (the XORs stay in the loop)
         const int b = w - 1;
-        const unsigned short* Zt = Zs + (b & 1) * PTILE;
-        const unsigned short* Xt = mat ? Zt : Ps + (b % PBUF) * PTILE;
-        const unsigned short* Yt = Ys + (b % RING) * QTILE;
-        const bool finished = b >= nsteps - DIAG;               // the queries of this tile's own keys: nothing is missing any more
+        const bool finished = TAIL && b >= nsteps - DIAG;       // the queries of this tile's own keys: nothing is missing any more
         if (finished) {    // key blocks behind these queries stay out of their dq, finite or not (later steps have older queries)
           const int newest = (t_last - b) * NSQ + dsq - (BKV / 32) * kt;
 #pragma unroll
           for (int kb = 1; kb < BKV / 32; ++kb)
             if (kb > newest) kt_f[2 * kb] = kt_f[2 * kb + 1] = zero8();
         }
-        el8 zf[ZH], af[2], bf[DB];
-        auto read_x = [&](int ks, int kb2) { return lds_tr8(Xt + (xb[0] ^ (kb2 << 5)) + 16 * ks * BKV, Xt + (xb[1] ^ (kb2 << 5)) + 16 * ks * BKV); };
-#pragma unroll
-        for (int ks = 0; ks < ZH; ++ks) zf[ks] = lds_row8(Zt + (zb ^ (ks << 4)));
+        const int y_next = y_at == y0 + (RING - 1) * QB ? y0 : y_at + QB;
+        el8 zf[ZH], af[2];
+        auto read_x = [&](int ks, int kb2) { return tr8((xb[0] ^ (kb2 << 6)) + x_at + 32 * ks * BKV, (xb[1] ^ (kb2 << 6)) + x_at + 32 * ks * BKV); };
+        auto read_z = [&](int ks) { return lds_row8_at((zb ^ (ks << 5)) + z_at); };
         af[0] = read_x(0, 0);
-        bf[0] = read_y(Yt, 0);
         af[1] = read_x(0, 1);
 #pragma unroll
-        for (int j = 1; j < DB; ++j) bf[j] = read_y(Yt, j);
+        for (int ks = 0; ks < ZH; ++ks) zf[ks] = read_z(ks);
         // product number i of dk / dv: contraction step i / (2 DB), column block, 32-key block; the fragment a column block
-        // is done with gives way to the next step's
+        // is done with gives way to the next step's (the columns of the next block's tile have landed long ago)
         auto product = [&](const int i) __attribute__((always_inline)) {
           const int ks = i / (2 * DB), j = (i / 2) % DB, kb2 = i & 1;
           acc[kb2][j] = mfma32(bf[j], af[kb2], acc[kb2][j]);
-          if (kb2 == 1 && ks + 1 < KQ) bf[j] = read_y(Yt + 16 * (ks + 1) * D, j);
+          if (kb2 == 1) bf[j] = ks + 1 < KQ ? read_y(y_at + 32 * (ks + 1) * D, j) : read_y(y_next, j);
           if (j == DB - 1 && ks + 1 < KQ) af[kb2] = read_x(ks + 1, kb2);
           __builtin_amdgcn_sched_barrier(0);
         };
@@ -840,7 +888,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
 #pragma unroll
         for (int ks = 0; ks < KZ; ++ks) {
           dq = mfma32(kt_f[ks], zf[ks % ZH], dq);
-          if (ks + ZH < KZ) zf[ks % ZH] = lds_row8(Zt + (zb ^ ((ks + ZH) << 4)));
+          if (ks + ZH < KZ) zf[ks % ZH] = read_z(ks + ZH);
           if (ks & 1) product(ks >> 1);
         }
         if (finished) {
@@ -855,16 +903,27 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         }
 #pragma unroll
         for (int i = 0; i < (REST > OPS ? REST : OPS); ++i) {
-          if (i < 4) store_part(w, i, dq, has_dq && !finished);
-          else if (i < OPS) fetch(w, i - 4);
+          if (i < 4) store_part(i, dq, (ALL_DQ || has_dq) && !finished);
+          else if (i < OPS) fetch(i - 4, !TAIL || w < nsteps, !TAIL || w + AHEAD < nsteps);
           if (i < REST) product(KZ / 2 + i);
         }
+        advance();
+        y_at = y_next;
+        x_at = x_at + PB == x_end ? x0 : x_at + PB;
+        z_at = 2 * place_of(Zs) + PB - z_at;
         // The tile copied an iteration ago (read behind this barrier) has landed, what came after it may be in flight.  An item's
         // last request, of nothing, has to come back all the same before its registers are used for something else.
-        if (w < nsteps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + LOADS_PER_TILE) : "memory");
+        if (!TAIL || w < nsteps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + LOADS_PER_TILE) : "memory");
         else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS_PER_TILE) : "memory");
-        lds_barrier();
-      }
+        // (no wait for LDS: what was read of the staged blocks has been multiplied, the columns on their way stay where they are)
+        asm volatile("s_barrier" ::: "memory");
+      };
+      int w = 1;
+      const int plain = nsteps - (AHEAD > DIAG ? AHEAD : DIAG);
+#pragma unroll 1
+      for (; w < plain; ++w) iteration(No{}, w);
+#pragma unroll 1
+      for (; w <= nsteps; ++w) iteration(Yes{}, w);
       // (behind the barrier of the last iteration every product wave is done with the staged blocks and the last tiles)
       const bool more = read_box(m & 1, nxt);
       const Item done = cur;

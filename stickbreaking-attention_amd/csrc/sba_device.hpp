@@ -254,6 +254,15 @@ __device__ __forceinline__ el8 lds_row8(const unsigned short* p) {
   return *reinterpret_cast<const el8*>(p);
 }
 
+// The same by LDS address (a byte count): an address that is an XOR and a sum is one instruction.
+__device__ __forceinline__ el8 lds_tr8_at(int at0, int at1) {
+  s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(unsigned)at0);
+  s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(unsigned)at1);
+  s16x8 r = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  return __builtin_bit_cast(el8, r);
+}
+__device__ __forceinline__ el8 lds_row8_at(int at) { return *(const __attribute__((address_space(3))) el8*)(unsigned)at; }
+
 // ---------------------------------------------------------------------------------------------
 // Key ownership.  Row m of the S^T MFMA is fed with key  kperm(m) = 16*((m>>2)&1) + 4*(m>>3) + (m&3)
 // of the sub-block (the lane that supplies A-operand row m simply loads that key), so that in
@@ -718,6 +727,14 @@ struct TileCopy {
     static_assert(!TWO_PHASE, "one offset per lane");
     const int soff = wanted ? (row0 + row_delta(j)) * (int)r.row_bytes : 0;
     async_copy16<STREAM>(r.rsrc, wanted ? lds_tile + (j * STEP + wave * RPI) * D : spare, wanted ? voff : OUTSIDE, __builtin_amdgcn_readfirstlane(soff));
+  }
+
+  // The same with the first row's byte offset in the resource and the tile's place in bytes behind `ring`.
+  __device__ __forceinline__ void issue_at(const Rows& r, int row_offset, const unsigned short* ring, int at, int j, bool wanted, unsigned short* spare) const {
+    static_assert(!TWO_PHASE, "one offset per lane");
+    const int soff = wanted ? row_offset + row_delta(j) * (int)r.row_bytes : 0;
+    const unsigned short* dst = ring + at / 2 + (j * STEP + wave * RPI) * D;
+    async_copy16<STREAM>(r.rsrc, wanted ? dst : spare, wanted ? voff : OUTSIDE, __builtin_amdgcn_readfirstlane(soff));
   }
 
   // `rows_needed` (uniform): instructions whose rows all lie at or beyond it are skipped; the tile

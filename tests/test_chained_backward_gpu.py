@@ -70,6 +70,24 @@ def test_queues(form, steps, H, lengths):
         assert torch.equal(b, c)
 
 
+@pytest.mark.parametrize("steps,d", [(2, 128), (2, 96), (2, 64), (3, 64), (2, 32), (3, 32)])
+def test_the_same_bits_from_run_to_run(form, steps, d):
+    """Items of one step up to one more than the steps in flight, with product waves that have a block of dq and without."""
+    from stickbreaking_attention import sb_attn_varlen
+    lengths = [300, 131, 32, 161, 193, 288, 609]
+    H, T = 6, sum(lengths)
+    tensors = orc.make_inputs((H, T, d), 60 + d)
+    drem = torch.randn((H, T), generator=torch.Generator().manual_seed(d)).to(torch.bfloat16)
+    cu = cu_from_lengths(lengths, device=DEV)
+    form(1)
+    two = gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem))
+    form(steps)
+    runs = [gradients(sb_attn_varlen, tensors[:3], cu, max(lengths), False, (tensors[3], drem)) for _ in range(8)]
+    for i, name in enumerate(("dq", "dk", "dv")):
+        assert_close(name, runs[0][i], two[i].float())
+        assert all(torch.equal(runs[0][i], r[i]) for r in runs[1:]), name
+
+
 @pytest.mark.parametrize("steps,d", [(2, 128), (2, 64), (3, 64), (2, 32), (3, 32)])
 def test_a_wait_that_runs_out_gives_nan_and_nothing_else(form, steps, d):
     """Every wait for the key tile before ends after one look, so that tiles go on without the partial sums they
