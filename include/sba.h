@@ -245,13 +245,15 @@ int sba_attn_bwd(const sba_problem* p, const void* schedule, size_t schedule_siz
                  const sba_view* dq, const sba_view* dk, const sba_view* dv,
                  void* stream);
 
-/* The backward in one pass: every score is formed once, dq is handed from key tile to key tile through scratch
- * memory (csrc/sba_chain.hip).  For the problems it is the faster form of, sba_chain_scratch_bytes
- * returns the scratch it needs (16-byte aligned, contents irrelevant, one per concurrent call) and 0 for every other;
- * a caller then takes sba_varlen_bwd / sba_attn_bwd, which choose among their kernels by size.  Same inputs, outputs, table and refusals; it
+/* The backward with every score formed once.  Up to head_dim 128 it is one pass, dq is handed from key tile to key tile
+ * through scratch memory (csrc/sba_chain.hip); above, the dq pass hands the weights and the gradients of the logits
+ * to the dk/dv pass through scratch memory, 4 bytes per causal pair (csrc/sba_wide.hip).  For the problems it is the
+ * faster form of, sba_chain_scratch_bytes returns the scratch it needs (16-byte aligned, contents irrelevant, one per
+ * concurrent call; never more than 3.75 GiB above head_dim 128) and 0 for every other; a caller then takes
+ * sba_varlen_bwd / sba_attn_bwd, which choose among their kernels by size.  Same inputs, outputs, table and refusals; it
  * needs no gradient table, and the results differ from the two-pass form's by rounding.  Problems it
- * cannot take (log-space carry, head_dim > 128, a device that is not eight XCDs of 32 compute units)
- * return SBA_E_SHAPE. */
+ * cannot take (log-space carry; up to head_dim 128 a device that is not eight XCDs of 32 compute units; above, more
+ * scratch than that) return SBA_E_SHAPE. */
 size_t sba_chain_scratch_bytes(const sba_problem* p);
 int sba_varlen_bwd_chained(const sba_problem* p, const void* schedule, size_t schedule_size,
                            const sba_view* q, const sba_view* k, const sba_view* v,
@@ -328,7 +330,7 @@ void  sba_set_dkdv_workgroups(int n);
 /* Test and tuning switch (process-wide): the form of the backward.  0: by size -- sba_chain_scratch_bytes asks for
  * the one-pass form where that is the fastest, and sba_*_bwd take the kernels for few tiles or for short documents
  * where those are (csrc/sba_small.hip).  1: the general two passes, always.  2: the one-pass form wherever it is
- * possible, 3: the same in steps of 64 queries (head_dim <= 64); sba_*_bwd then run the two passes.  The forms differ by rounding.
+ * possible (head_dim <= 128), 3: the same in steps of 64 queries (head_dim <= 64); sba_*_bwd then run the two passes.  The forms differ by rounding.
  * With SBA_FORM_SHORT_WAITS added, a wait of the one-pass form for the key tile before gives up after its
  * first look, as it otherwise does after about a second: what the missing partial sums belong to is NaN.
  * With SBA_FORM_IDLE_XCDS(mask), the XCDs in `mask` (of bits 0 .. 7, not all) count as without a compute unit for

@@ -405,6 +405,35 @@ ChainScratch chain_scratch(const sba_problem* p, const Sizes& sz) {
   return c;
 }
 
+// ---- the two passes of head_dim 129 .. 256 with p and dz handed on (sba_wide.hip) -----------------------
+// The dq pass stores p and dz, 4 bytes per causal pair, and the dk/dv pass multiplies them instead of forming both again.  It is the faster
+// form of 99 problems of 2 to 16 heads and 256 to 8192 tokens in 1 to 60 documents at head_dim 136, 160 and 256 (1.12 by the geometric mean, 0.98 ..
+// 1.39) and of the larger ones (16 heads x 16 K tokens in eight documents at 256: 1515 -> 1180 us, 12 x 4 x 4096 1520 -> 1203).  The line is the room: 32 times
+// a carry table, 32 bytes more for every query and 32 keys than GIVEN_SCRATCH_MAX has are with the passes that form the scores twice.
+size_t given_scratch(const sba_problem* p, bool fixed) { return (size_t)p->heads * (size_t)table_entries_bound(p, fixed) * (2 * PZ_WORDS); }
+bool given_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
+  return (p->flags & SBA_PRODUCT_SPACE) && p->head_dim > 128 && sz.n_docs > 0 && given_scratch(p, fixed) <= GIVEN_SCRATCH_MAX;
+}
+bool given_wanted(const sba_problem* p, bool fixed, const Sizes& sz) { return backward_form() != 1 && given_possible(p, fixed, sz); }
+
+int backward_given(const sba_problem* p, bool fixed, const Sizes& sz, KArgs& a, void* scratch, size_t scratch_bytes, hipStream_t s) {
+  a.pz = static_cast<unsigned short*>(scratch);
+  a.pz_entries = (int64_t)(scratch_bytes / (2 * PZ_WORDS) / (size_t)p->heads) & ~(int64_t)31;
+  const BwdBounds bb = backward_bounds(p, fixed, sz);
+  const DkdvGrid g = dkdv_grid(false, bb.n_long_max, bb.n_tail_max, sz.n_kv_max);
+  const bool ac = (p->flags & SBA_ATTEND_CURRENT) != 0, f16 = p->dtype == SBA_F16;
+  hipError_t he;
+  {
+    Timer tm(1, s);
+    he = (f16 ? f16::launch_bwd_dq_wide : bf16::launch_bwd_dq_wide)(a, ac, true, sz.n_q_max, s);
+  }
+  if (he == hipSuccess) {
+    Timer tm(2, s);
+    he = (f16 ? f16::launch_bwd_dkdv_given : bf16::launch_bwd_dkdv_given)(a, g.main_tiles, s);
+  }
+  return (int)he;
+}
+
 // Whether the kernels can take the problem at all: a device of eight XCDs with 32 compute units each, ranked documents, room for the queue's groups in LDS and 32-bit
 // offsets into a document's partial dq.
 bool chain_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
@@ -468,6 +497,19 @@ int backward_chained(const sba_problem* p, bool fixed, const void* schedule, siz
   KArgs c;
   std::memset(&c, 0, sizeof(c));
   if ((e = fill_common(p, fixed, sz, schedule, sched_bytes, true, table_bytes, &c))) return e;
+  if (p->head_dim > 128) {
+    if (sz.rows > 0 && !given_possible(p, fixed, sz)) return SBA_E_SHAPE;
+    if (scratch_bytes < given_scratch(p, fixed) || (reinterpret_cast<uintptr_t>(scratch) & 15)) return SBA_E_WORKSPACE;
+    if ((e = check_arch())) return e;
+    if (sz.rows == 0) return 0;
+    c.q = to_view(q); c.k = to_view(k); c.v = to_view(v); c.go = to_view(go); c.grem = to_view(grem);
+    c.dq = to_view_out(dq, p); c.dk = to_view_out(dk, p); c.dv = to_view_out(dv, p);
+    c.stick = const_cast<float*>(stick);
+    c.max_doc_len = declared_max_doc_len(p, fixed);
+    c.clear_spare = fixed ? 0 : 1;
+    c.nan_pair = p->dtype == SBA_F16 && !c.out_f32 ? 0x7e007e00u : 0x7fc07fc0u;
+    return backward_given(p, fixed, sz, c, scratch, scratch_bytes, reinterpret_cast<hipStream_t>(stream));
+  }
   const ChainScratch at = chain_scratch(p, sz);
   if (scratch_bytes < at.total || (reinterpret_cast<uintptr_t>(scratch) & 15)) return SBA_E_WORKSPACE;
   if ((e = check_arch())) return e;
@@ -653,8 +695,9 @@ int sba_attn_bwd(const sba_problem* p, const void* schedule, size_t schedule_siz
 size_t sba_chain_scratch_bytes(const sba_problem* p) {
   Sizes sz;
   const bool fixed = p != nullptr && (p->flags & SBA_FIXED_LENGTH) != 0;
-  if (check_problem(p, fixed, &sz) || !chain_wanted(p, fixed, sz)) return 0;
-  return chain_scratch(p, sz).total;
+  if (check_problem(p, fixed, &sz)) return 0;
+  if (given_wanted(p, fixed, sz)) return given_scratch(p, fixed);
+  return chain_wanted(p, fixed, sz) ? chain_scratch(p, sz).total : 0;
 }
 
 int sba_varlen_bwd_chained(const sba_problem* p, const void* schedule, size_t schedule_size, const sba_view* q,

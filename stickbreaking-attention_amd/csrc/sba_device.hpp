@@ -63,6 +63,10 @@ constexpr int RANK_LIMIT = 4096; // beyond this many documents the input order i
 // 4 n_docs once it is done (16-byte aligned: the lists are whole 32-byte tiles).
 __host__ __device__ inline int chain_docs_offset(int n_docs) { return (2 * n_docs + 3) & ~3; }
 
+// 16-bit words that p and dz of a 32 x 32 block take per carry-table entry of the block (32 of them), where the wide backward
+// keeps them: see bwd_dq_wide_kernel.
+constexpr int PZ_WORDS = 64;
+
 struct Tile {
   int tok_start;  // first token of the document inside the packed token axis (0 for fixed-length)
   int doc_len;

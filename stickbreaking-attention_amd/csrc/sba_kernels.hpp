@@ -40,8 +40,12 @@ struct KArgs {
   int n_items;                 // work items of this launch (what the grid is with one workgroup per item)
   int resident;                // backward, host side: workgroups of a persistent launch (0: never persistent)
   int min_items_each;          // host side: a launch is persistent when it has this many items per workgroup
+  unsigned short* pz;          // backward at head_dim 129 .. 256: p and dz of every 32 x 32 block, left by the dq pass for the dk/dv pass
+  int64_t pz_entries;          // carry-table entries per head it has room for: 128 bytes each
   int lg_deal;                 // forward: the logarithm of the device's compute units if it holds the launch at once (see deal_item), or NO_DEAL
 };
+
+constexpr size_t GIVEN_SCRATCH_MAX = 0xf0000000u;   // bytes of p and dz that are handed on: 32-bit offsets reach them
 
 constexpr int NO_DEAL = 31;    // (no launch has a second round of 2^31 workgroups)
 // Workgroups of the forward that a compute unit holds.
@@ -86,7 +90,7 @@ __device__ __forceinline__ void as_global(T*& p) {
 __device__ __forceinline__ void globals_of(KArgs& a) {
   as_global(a.q.ptr); as_global(a.k.ptr); as_global(a.v.ptr); as_global(a.o.ptr); as_global(a.rem.ptr);
   as_global(a.go.ptr); as_global(a.grem.ptr); as_global(a.dq.ptr); as_global(a.dk.ptr); as_global(a.dv.ptr);
-  as_global(a.sched); as_global(a.stick); as_global(a.gtab); as_global(a.weights); as_global(a.work);
+  as_global(a.sched); as_global(a.stick); as_global(a.gtab); as_global(a.weights); as_global(a.work); as_global(a.pz);
 }
 __device__ __forceinline__ void globals_of(ChainArgs& a) {
   as_global(a.q.ptr); as_global(a.k.ptr); as_global(a.v.ptr); as_global(a.go.ptr); as_global(a.grem.ptr);
@@ -189,6 +193,7 @@ inline int dkdv_main_workgroups(int head_dim, int main_tiles) { return main_tile
   hipError_t launch_bwd_dkdv(const KArgs& a, int head_dim, bool attend_current, bool product, int n_long_max,    \
                              int n_last_max, hipStream_t s);                                                     \
   hipError_t launch_bwd_dq_wide(const KArgs& a, bool attend_current, bool product, int n_q_max, hipStream_t s);   \
+  hipError_t launch_bwd_dkdv_given(const KArgs& a, int tiles, hipStream_t s);                                    \
   hipError_t launch_bwd_dkdv_wide(const KArgs& a, bool attend_current, bool product, int tiles, hipStream_t s);   \
   hipError_t launch_fwd_small(const KArgs& a, bool attend_current, int n_q_max, hipStream_t s);                  \
   hipError_t launch_bwd_short(const KArgs& a, bool attend_current, int parts, hipStream_t s);                  \

@@ -28,7 +28,6 @@
 namespace sba {
 inline namespace SBA_ELEM_NS {
 
-
 template <bool AC, bool PROD, int U>
 __global__ void __launch_bounds__(512, 1) bwd_dkdv_wide_kernel(const KArgs a) {
   constexpr int D = 256, KS = U / 16, DBH = U / 64;     // U: columns multiplied; DBH: 32-wide column blocks of a product wave
@@ -370,7 +369,7 @@ __global__ void __launch_bounds__(512, 1) bwd_dkdv_wide_kernel(const KArgs a) {
 // eight documents, head_dim 256: 795 -> 620 us against one wave per SIMD with 512 registers for everything.  Reading
 // operands six or eight instead of four products ahead changes nothing.
 // -------------------------------------------------------------------------------------------
-template <bool AC, bool PROD, int U>
+template <bool AC, bool PROD, int U, bool GIVE>
 __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
   constexpr int D = 256, KS = U / 16, DB = U / 32;
   constexpr int BF = 32, SLOTS = 4, TILE = BF * D;
@@ -390,7 +389,7 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
   const Tile t = reinterpret_cast<const Tile*>(sched + SCHED_HDR)[slot];
   asm volatile("" ::"s"(t.tok_start), "s"(t.doc_len), "s"(t.idx), "s"(t.batch), "s"(t.tab_base));   // keep the tile read above the branch
   const int tid = threadIdx.x;
-  const bool refused = hdr.x != 0 || hdr.w > a.tab_stride || longest > a.max_doc_len;
+  const bool refused = hdr.x != 0 || hdr.w > a.tab_stride || longest > a.max_doc_len || (GIVE && hdr.w > a.pz_entries);
   if (refused || slot >= hdr.y) {
     if (a.clear_spare) {     // for the dk/dv pass as well, which has no slots to spare
       int row0, row1;
@@ -447,6 +446,20 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   lds_barrier();                              // the places are free
   float* const mine = hand + HAND * rb + 4 * lane;
+  // GIVE: p and dz of a block as the lanes hold them, eight keys of a query in 16 bytes: lane's first eight keys, then the lanes'
+  // other eight.  A block's place goes by the carry table's.
+  const bool gives = GIVE && qw0 < L;         // (a block of queries behind the document's end has no place)
+  __amdgpu_buffer_rsrc_t give_rs;
+  if constexpr (GIVE)
+    give_rs = __builtin_amdgcn_make_buffer_rsrc(a.pz + ((int64_t)head * a.pz_entries + t.tab_base) * PZ_WORDS, 0, (unsigned)tab_doc_entries(L) * (2u * PZ_WORDS), 0x00020000);
+  auto give = [&](const el8 (&v)[2], int block, int part) __attribute__((always_inline)) {
+    const unsigned at = (unsigned)(tab_seg32(L, block) + qw0) * (2u * PZ_WORDS) + 2048u * part;
+    int give_at = 16 * lane;
+    asm volatile("" : "+v"(give_at));         // (no register for it through the steps)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[c]), give_rs, give_at + 1024 * c, (int)at, 2 /* nt */);
+    asm volatile("s_nop 0" ::"v"(v[0]), "v"(v[1]) : "memory");      // (the registers stay as they are behind the stores: see bwd_chain_kernel)
+  };
 
   using std::integral_constant;
   if (w < 4) {
@@ -469,7 +482,7 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
     float carry_c = 0.0f;
     lds_barrier();                            // tile 0 has landed, do . v_row is there
     if (a.fuse) dr += drs[rb][n];
-    if (qvalid && h == 0) gtab[(unsigned)(tab_rowplane32(L) + qrow)] = dr;
+    if (!GIVE && qvalid && h == 0) gtab[(unsigned)(tab_rowplane32(L) + qrow)] = dr;
     f32x16 x;
     clear(x);
     chain_begin(Ks);
@@ -482,10 +495,23 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
       const bool visible = i <= own;
       float p[16], r[16], ends[2] = {0.0f, 0.0f};
       if (visible) {
-        if (qvalid && h == 0) gtab[(unsigned)(tab_seg32(L, i) + qrow)] = carry_c;
+        if (!GIVE && qvalid && h == 0) gtab[(unsigned)(tab_seg32(L, i) + qrow)] = carry_c;
         float c = e;
         if (i < own) stick_weights<AC, PROD, false, true>(x, a.c, i * BF, qrow, h, c, p, r, ends);
         else stick_weights<AC, PROD, true, true>(x, a.c, i * BF, qrow, h, c, p, r, ends);
+        if (gives) {
+          el8 pf[2] = {pack8(p), pack8(p + 8)};
+          if (i == own && a.fuse) {           // fused output: rem_j * do_j reaches dv_j through the diagonal of p (see bwd_dkdv_kernel)
+            float pd[16], rem_own = 0.0f;
+            if (qvalid) rem_own = stick[(unsigned)(tab_rowplane32(L) + qrow)];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) pd[j] = p[j] + (16 * h + j == n ? rem_own : 0.0f);
+            pf[0] = pack8(pd);
+            pf[1] = pack8(pd + 8);
+          }
+          if (qw0 + 32 > L && !qvalid) pf[0] = pf[1] = zero8();     // (rows behind the document's end leave nothing to be multiplied, finite or not)
+          give(pf, i, 0);
+        }
       }
       lds_barrier();
       if (visible) {
@@ -531,6 +557,7 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
           for (int k = 0; k < KS; ++k) chain_step(Tn, x, k);
           grad_dz<PROD>(p, r, da, ends, h, carry_c, dr, zf);
         }
+        if (GIVE && qw0 + 32 > L && !qvalid) zf[0] = zf[1] = zero8();
         *reinterpret_cast<el8*>(mine + HAND_Z) = zf[0];
         *reinterpret_cast<el8*>(mine + HAND_Z + 256) = zf[1];
       }
@@ -597,8 +624,9 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
 #pragma unroll
     for (int k = 0; k < KS; ++k) chain_step(Vs, da, k);
     // dq += dz K of a block, whose tile is at Kt
-    auto product = [&](const unsigned short* Kt) __attribute__((always_inline)) {
+    auto product = [&](const unsigned short* Kt, int block) __attribute__((always_inline)) {
       const el8 zf[2] = {*reinterpret_cast<const el8*>(mine + HAND_Z), *reinterpret_cast<const el8*>(mine + HAND_Z + 256)};
+      if (gives) give(zf, block, 1);
       constexpr int N = 2 * DB, AHEAD = 4;    // operand reads run AHEAD products ahead
       el8 kt[AHEAD];
       auto read_k = [&](int m) {
@@ -626,9 +654,11 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
           *reinterpret_cast<f32x4*>(mine + 256 * g) = q4;
         }
       }
-      if (i > 0 && i - 1 <= own) product(Ks + ((SLOT + SLOTS - 1) % SLOTS) * TILE);
-      // tile i + 1, which everyone reads behind this barrier, has landed
-      if (i + 2 < nblk) wait_loads<LOADS_PER_TILE>();
+      const bool multiplied = i > 0 && i - 1 <= own;
+      if (multiplied) product(Ks + ((SLOT + SLOTS - 1) % SLOTS) * TILE, i - 1);
+      // tile i + 1, which everyone reads behind this barrier, has landed (what the products stored came after tile i + 2)
+      if (gives && multiplied && i + 2 < nblk) wait_loads<LOADS_PER_TILE + 2>();
+      else if (i + 2 < nblk) wait_loads<LOADS_PER_TILE>();
       else wait_loads<0>();
       lds_barrier();
       if (i + 3 < nblk) fetch(i + 3);
@@ -654,8 +684,150 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
       step(integral_constant<int, 3>{}, i + 3);
       if (i + 4 >= nblk) break;
     }
-    if (nblk - 1 <= own) product(Ks + ((nblk - 1) % SLOTS) * TILE);
+    if (nblk - 1 <= own) product(Ks + ((nblk - 1) % SLOTS) * TILE, nblk - 1);
     store_rows(dq, a.inv_temp, rows_of(a.dq), qrow, L, h, a.out_f32);
+  }
+}
+
+// -------------------------------------------------------------------------------------------
+// dk / dv pass of the same head dims where the dq pass has left p and dz of every block in memory (GIVE, above): 128 keys of one
+// (document, head) per workgroup, dv = p^T dO and dk = dz^T Q over the queries that can see them, 32 per step.  All eight waves are alike: 64
+// keys x half of the columns of one output each (128 registers), and a share of the copies.  A tile is 48 KiB (Q, dO, p, dz), three of
+// them in a ring; one barrier per step, operands read a step ahead.
+//
+// Bound by what it reads: 16 heads x 16 K tokens in eight documents at head_dim 256, 456 us for 1.45 GB of p and dz, which are read once, and
+// Q and dO, of which every key tile takes its own (398 without the former, 367 without the latter, both timing only); the matrix pipes are busy
+// for 40 %.  So the queries are walked from the document's end: the key tiles of a (document, head) that start together then read
+// the same rows at the same time (from the tile's own keys on 816 us for 678, 12 heads of 4 x 4096), and p and dz stream past the L2s that Q and dO
+// are kept in (as do the dq pass's stores of them: 568 -> 456).  The pass that forms p and dz itself: 890.  Handing them on costs the dq
+// pass 100 of 724 us, a third of it the packing.
+// -------------------------------------------------------------------------------------------
+template <int U>
+__global__ void __launch_bounds__(512, 1) bwd_dkdv_given_kernel(const KArgs a) {
+  constexpr int D = 256, DBH = U / 64;       // DBH: 32-wide column blocks of a wave
+  constexpr int TQ = 32, SLOTS = 3, QTILE = TQ * D, PTILE = TQ * BKV, SLOT = 2 * QTILE + 2 * PTILE;
+  __shared__ __attribute__((aligned(1024))) unsigned short tiles[SLOTS * SLOT];     // Q, dO, p, dz
+
+  // (the grid never exceeds the room of the list: its tile is read along with the header)
+  const int* sched = a.sched;
+  const int which = blockIdx.x / a.heads;
+  const int head = blockIdx.x - which * a.heads;
+  const int4 hdr = *reinterpret_cast<const int4*>(sched);   // status, query tiles, key tiles, table entries needed
+  const int longest = sched[SCHED_MAXLEN];
+  const Tile t = reinterpret_cast<const Tile*>(sched + a.kv_list_off)[which];
+  asm volatile("" ::"s"(t.tok_start), "s"(t.doc_len), "s"(t.idx), "s"(t.batch), "s"(t.tab_base));   // keep the tile read above the branch
+  if (hdr.x != 0 || hdr.w > a.tab_stride || hdr.w > a.pz_entries || longest > a.max_doc_len || which >= hdr.z) return;
+  const int L = t.doc_len, q_first = t.idx * BKV;
+  const int nsteps = (L - q_first + TQ - 1) / TQ;
+
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, n = lane & 31, h = lane >> 5;
+  const int i16 = lane & 15, blk = (lane >> 4) & 1;
+  const int mat = w >> 2, khalf = (w >> 1) & 1, chalf = w & 1;       // (dv | dk), 64 keys, half of the columns
+  const int64_t tok0 = t.tok_start;
+  auto rows_of = [&](const View& v) {
+    return make_rows(reinterpret_cast<const elem_t*>(v.ptr) + t.batch * v.sb + head * v.sh + tok0 * v.st, v.st, L, a.head_dim);
+  };
+  const Rows qrows = rows_of(a.q), grows = rows_of(a.go);
+  using Copy = TileCopy<D, TQ, 512, false>;
+  Copy qcopy, gcopy;
+  qcopy.init(tid, qrows.row_bytes, qrows.used_bytes);
+  gcopy.init(tid, grows.row_bytes, grows.used_bytes);
+  // Staged p or dz: four blocks one behind the other, each as it lies in memory: eight keys of a query in 16 bytes, the first eight keys of a
+  // half-wave's sixteen, then the other eight.  A wave copies one of those halves of a block.  The queries are XORed with four times the
+  // number of the eight keys, so that the transpose reads of all of them take different banks.  (Of the first three blocks of queries
+  // the newer key blocks do not exist: what is copied in their place is not multiplied.)
+  const int from = 1024 * (w & 1) + 16 * (lane ^ (4 * ((lane >> 5) + 2 * (w & 1))));
+  const int place = tab_seg32(L, min((BKV / 32) * t.idx + (w >> 1), (L - 1) / 32)) + q_first;
+  const __amdgpu_buffer_rsrc_t pz_rs = __builtin_amdgcn_make_buffer_rsrc(a.pz + ((int64_t)head * a.pz_entries + t.tab_base) * PZ_WORDS, 0,
+                                                                       (unsigned)tab_doc_entries(L) * (2u * PZ_WORDS), 0x00020000);
+  constexpr int LOADS_PER_TILE = 2 * Copy::NCH + 2;
+  auto fetch = [&](int turn, int slot) {
+    const int step = nsteps - 1 - turn;
+    unsigned short* const T = tiles + slot * SLOT;
+    qcopy.issue(qrows, q_first + step * TQ, T);
+    gcopy.issue(grows, q_first + step * TQ, T + QTILE);
+    const int soff = __builtin_amdgcn_readfirstlane((place + step * TQ) * (2 * PZ_WORDS));
+    async_copy16<true>(pz_rs, T + 2 * QTILE + 512 * w, from, soff);
+    async_copy16<true>(pz_rs, T + 2 * QTILE + PTILE + 512 * w, from, soff + 2048);
+  };
+  fetch(0, 0);
+  if (nsteps > 1) fetch(1, 1);
+  if (nsteps > 2) fetch(2, 2);
+  f32x16 acc[2][DBH];
+#pragma unroll
+  for (int kb2 = 0; kb2 < 2; ++kb2)
+#pragma unroll
+    for (int j = 0; j < DBH; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[kb2][j][e] = 0.0f;
+  // transpose reads of rows 8 h + 4 u + i16 / 4 (+ 16 ks): staged block, tile (bytes)
+  const int base = (int)(unsigned)(size_t)tiles;
+  int xoff[2][2], yoff[2][DBH];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int r = 8 * h + 4 * u + (i16 >> 2), c = 16 * blk + 4 * (i16 & 3);
+#pragma unroll
+    for (int kb2 = 0; kb2 < 2; ++kb2)
+      xoff[u][kb2] = base + 2 * (2 * QTILE + mat * PTILE) + 2048 * (2 * khalf + kb2) + 1024 * ((c >> 3) & 1) +
+                     16 * (32 * blk + (r ^ (4 * (blk + 2 * ((c >> 3) & 1))))) + 2 * (c & 7);
+#pragma unroll
+    for (int j = 0; j < DBH; ++j)
+      yoff[u][j] = base + 2 * ((mat ? 0 : QTILE) + swz_off<D>(r, (32 * (chalf * DBH + j) + c) >> 3) + (c & 7));
+  }
+  // Turn i multiplies what was read of tile i during turn i - 1, and a fragment that is done with gives way to tile i + 1's.
+  el8 af[2][2], bf[2][DBH];
+  auto read_x = [&](int at, int kb2, int ks) { af[kb2][ks] = lds_tr8_at(xoff[0][kb2] + at + 256 * ks, xoff[1][kb2] + at + 256 * ks); };
+  auto read_y = [&](int at, int j, int ks) { bf[ks][j] = lds_tr8_at(yoff[0][j] + at + 32 * ks * D, yoff[1][j] + at + 32 * ks * D); };
+  int slot = 0;                               // of tile i
+  // LAST: the last three, whose queries may not see all key blocks: those stay out, finite or not.
+  auto turn = [&](auto last_tag, const int i) __attribute__((always_inline)) {
+    constexpr bool LAST = decltype(last_tag)::value;
+    if (i + 2 < nsteps) wait_loads<LOADS_PER_TILE>();
+    else wait_loads<0>();
+    lds_barrier();                            // tile i + 1 has landed, everyone has read tile i
+    if (i + 3 < nsteps) fetch(i + 3, slot);
+    slot = slot == SLOTS - 1 ? 0 : slot + 1;
+    const int at = slot * (2 * SLOT);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int j = 0; j < DBH; ++j) {
+#pragma unroll
+        for (int kb2 = 0; kb2 < 2; ++kb2)
+          if (!LAST || 2 * khalf + kb2 <= nsteps - 1 - i) acc[kb2][j] = mfma32(bf[ks][j], af[kb2][ks], acc[kb2][j]);
+        read_y(at, j, ks);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      read_x(at, 0, ks);
+      read_x(at, 1, ks);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (nsteps > 2) wait_loads<2 * LOADS_PER_TILE>();
+  else if (nsteps > 1) wait_loads<LOADS_PER_TILE>();
+  else wait_loads<0>();
+  lds_barrier();
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+    for (int j = 0; j < DBH; ++j) read_y(0, j, ks);
+    read_x(0, 0, ks);
+    read_x(0, 1, ks);
+  }
+  int i = 0;
+#pragma unroll 1
+  for (; i + 3 < nsteps; ++i) turn(std::false_type{}, i);
+#pragma unroll 1
+  for (; i < nsteps; ++i) turn(std::true_type{}, i);
+  const Rows out = rows_of(mat ? a.dk : a.dv);
+#pragma unroll
+  for (int kb2 = 0; kb2 < 2; ++kb2) {
+    const int row = q_first + 64 * khalf + 32 * kb2 + n;
+#pragma unroll
+    for (int j = 0; j < DBH; ++j)
+      store_block32_rows(acc[kb2][j], mat ? a.inv_temp : 1.0f, out, row * (int)out.row_bytes, row < L, 32 * (chalf * DBH + j), h, a.out_f32);
   }
 }
 
@@ -666,25 +838,41 @@ template __global__ void bwd_dkdv_wide_kernel<true, true, 256>(const KArgs);
 template __global__ void bwd_dkdv_wide_kernel<false, true, 192>(const KArgs);
 template __global__ void bwd_dkdv_wide_kernel<true, true, 192>(const KArgs);
 
-template __global__ void bwd_dq_wide_kernel<false, false, 256>(const KArgs);
-template __global__ void bwd_dq_wide_kernel<true, false, 256>(const KArgs);
-template __global__ void bwd_dq_wide_kernel<false, true, 256>(const KArgs);
-template __global__ void bwd_dq_wide_kernel<true, true, 256>(const KArgs);
-template __global__ void bwd_dq_wide_kernel<false, true, 192>(const KArgs);
-template __global__ void bwd_dq_wide_kernel<true, true, 192>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<false, false, 256, false>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<true, false, 256, false>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<false, true, 256, false>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<true, true, 256, false>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<false, true, 192, false>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<true, true, 192, false>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<false, true, 256, true>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<true, true, 256, true>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<false, true, 192, true>(const KArgs);
+template __global__ void bwd_dq_wide_kernel<true, true, 192, true>(const KArgs);
 
+template __global__ void bwd_dkdv_given_kernel<256>(const KArgs);
+template __global__ void bwd_dkdv_given_kernel<192>(const KArgs);
+
+template <int U, bool GIVE>
+static void launch_dq_product(const KArgs& a, bool ac, int n_q_max, hipStream_t s) {
+  const dim3 grid((unsigned)n_q_max * (unsigned)a.heads), block(512);
+  if (ac) hipLaunchKernelGGL((bwd_dq_wide_kernel<true, true, U, GIVE>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((bwd_dq_wide_kernel<false, true, U, GIVE>), grid, block, 0, s, a);
+}
 hipError_t launch_bwd_dq_wide(const KArgs& a, bool ac, bool prod, int n_q_max, hipStream_t s) {
   const dim3 grid((unsigned)n_q_max * (unsigned)a.heads), block(512);
-  if (prod && used_width(a.head_dim) == 192) {
-    if (ac) hipLaunchKernelGGL((bwd_dq_wide_kernel<true, true, 192>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((bwd_dq_wide_kernel<false, true, 192>), grid, block, 0, s, a);
-  } else if (ac) {
-    if (prod) hipLaunchKernelGGL((bwd_dq_wide_kernel<true, true, 256>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((bwd_dq_wide_kernel<true, false, 256>), grid, block, 0, s, a);
-  } else {
-    if (prod) hipLaunchKernelGGL((bwd_dq_wide_kernel<false, true, 256>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((bwd_dq_wide_kernel<false, false, 256>), grid, block, 0, s, a);
-  }
+  const bool narrow = used_width(a.head_dim) == 192;
+  if (prod && a.pz != nullptr) narrow ? launch_dq_product<192, true>(a, ac, n_q_max, s) : launch_dq_product<256, true>(a, ac, n_q_max, s);
+  else if (prod) narrow ? launch_dq_product<192, false>(a, ac, n_q_max, s) : launch_dq_product<256, false>(a, ac, n_q_max, s);
+  else if (ac) hipLaunchKernelGGL((bwd_dq_wide_kernel<true, false, 256, false>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((bwd_dq_wide_kernel<false, false, 256, false>), grid, block, 0, s, a);
+  return hipGetLastError();
+}
+
+// tiles: see launch_bwd_dkdv_wide
+hipError_t launch_bwd_dkdv_given(const KArgs& a, int tiles, hipStream_t s) {
+  const dim3 grid((unsigned)tiles * (unsigned)a.heads), block(512);
+  if (used_width(a.head_dim) == 192) hipLaunchKernelGGL((bwd_dkdv_given_kernel<192>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((bwd_dkdv_given_kernel<256>), grid, block, 0, s, a);
   return hipGetLastError();
 }
 

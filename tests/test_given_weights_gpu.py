@@ -1,0 +1,102 @@
+"""The backward at head_dim 129 .. 256 whose dq pass leaves p and dz in memory for the dk/dv pass (csrc/sba_wide.hip), where its steps, its
+ring of three tiles and the places of its blocks can go wrong, against the passes that form the scores twice; and its scratch."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import sb_oracle as orc
+from tests.helpers import assert_close, cu_from_lengths, oracle_varlen
+from tests.test_abi import problem
+
+DEV = "cuda:0"
+EDGES = [1, 31, 32, 33, 96, 97, 127, 128, 129, 160, 161, 256, 257, 385]
+
+
+@pytest.fixture
+def form():
+    from stickbreaking_attention import _native
+    lib = _native.load()
+    yield lib.sba_set_backward_form
+    lib.sba_set_backward_form(0)
+
+
+def gradients(op, tensors, cu, longest, ac, grads):
+    x = [t.to(DEV).requires_grad_() for t in tensors]
+    out = op(*x, cu, longest, zero_start=False, attend_current=ac)
+    out = out if isinstance(out, tuple) else (out,)
+    return torch.autograd.grad(out, x, [g.to(DEV) for g in grads[:len(out)]])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ac", [False, True])
+@pytest.mark.parametrize("d,dtype", [(256, torch.bfloat16), (200, torch.float16), (192, torch.bfloat16), (136, torch.bfloat16), (256, torch.float32)])
+def test_edges(form, d, dtype, ac):
+    from stickbreaking_attention import sb_attn_varlen, sb_attn_varlen_fused
+    H, used = 2, sum(EDGES)
+    T = used + 7
+    q, k, v, do = (t.to(dtype) for t in orc.make_inputs((H, T, d), 20 + d))
+    drem = torch.randn((H, T), generator=torch.Generator().manual_seed(d)).to(torch.bfloat16).to(dtype)
+    cu = cu_from_lengths(EDGES, device=DEV)
+    got = gradients(sb_attn_varlen, (q, k, v), cu, max(EDGES), ac, (do, drem))
+    again = gradients(sb_attn_varlen, (q, k, v), cu, max(EDGES), ac, (do, drem))
+    fused = gradients(sb_attn_varlen_fused, (q, k, v), cu, max(EDGES), ac, (do,))
+    form(1)
+    twice = gradients(sb_attn_varlen, (q, k, v), cu, max(EDGES), ac, (do, drem))
+    fused_twice = gradients(sb_attn_varlen_fused, (q, k, v), cu, max(EDGES), ac, (do,))
+    ref = oracle_varlen(q[:, :used], k[:, :used], v[:, :used], do[:, :used], EDGES, ac, drem=drem[:, :used])[2:]
+    for name, g, a, r, t, f, ft in zip(("dq", "dk", "dv"), got, again, ref, twice, fused, fused_twice):
+        assert torch.equal(g, a)
+        assert not g[:, used:].any() and not f[:, used:].any()
+        assert_close(name, g[:, :used], r)
+        # the passes that form the scores twice stay as they were
+        assert_close(name + ", scores formed twice", t[:, :used], r)
+        assert_close(name + " of o + rem v", f[:, :used], ft[:, :used].float())
+
+
+@pytest.mark.gpu
+def test_fixed_length_and_token_major(form):
+    from stickbreaking_attention import sb_attn
+    B, H, T, d = 2, 3, 290, 160
+    gen = torch.Generator().manual_seed(3)
+    x = [torch.randn((B, T, H, d), generator=gen).to(torch.bfloat16).to(DEV).transpose(1, 2).requires_grad_() for _ in range(3)]
+    do = torch.randn((B, T, H, d), generator=gen).to(torch.bfloat16).to(DEV).transpose(1, 2)
+    run = lambda: torch.autograd.grad(sb_attn(*x)[0], x, do)
+    got = run()
+    form(1)
+    for name, g, t in zip(("dq", "dk", "dv"), got, run()):
+        assert_close(name, g, t.float())
+
+
+@pytest.mark.gpu
+def test_a_document_longer_than_declared_gives_nan(monkeypatch):
+    """Room for p and dz goes by the declared length: what does not fit is refused by the kernels, and every gradient is NaN."""
+    from stickbreaking_attention import _ops, sb_attn_varlen
+    monkeypatch.setattr(_ops, "SYNC_FREE", True)
+    tensors = orc.make_inputs((2, 700, 256), 4)
+    cu = cu_from_lengths([600, 100], device=DEV)
+    for g in gradients(sb_attn_varlen, tensors[:3], cu, 128, False, (tensors[3], torch.zeros((2, 700), dtype=torch.bfloat16))):
+        assert torch.isnan(g).all()
+
+
+def test_scratch(form):
+    from stickbreaking_attention import _native as nat
+    lib = nat.load()
+    p = problem(head_dim=256, heads=16, flags=nat.FLAG_PRODUCT_SPACE)
+    need = lib.sba_chain_scratch_bytes(ctypes.byref(p))
+    assert need == (lib.sba_table_bytes(ctypes.byref(p)) - 256) * 32      # 128 bytes for every entry of a carry table
+    view = ctypes.byref(nat.SbaView(0x1000, 0, 256 * 16384, 256))
+    row = ctypes.byref(nat.SbaView(0x1000, 0, 16384, 1))
+    at = ctypes.c_void_p(0x1000)
+    def call(problem, scratch, size):
+        return lib.sba_varlen_bwd_chained(ctypes.byref(problem), at, lib.sba_schedule_bytes(ctypes.byref(problem)), view, view, view, view, row,
+                                          at, 1 << 31, ctypes.c_void_p(scratch), size, view, view, view, None)
+    assert call(p, 0x1000, need - 1) == -6 and call(p, 0x1004, need) == -6
+    # more than 32-bit offsets reach, and the log-space carry: the other passes
+    large = problem(head_dim=256, heads=32, flags=nat.FLAG_PRODUCT_SPACE)
+    log = problem(head_dim=256, heads=16)
+    for other in (large, log):
+        assert lib.sba_chain_scratch_bytes(ctypes.byref(other)) == 0
+        assert call(other, 0x1000, 1 << 40) == -4
+    form(1)
+    assert lib.sba_chain_scratch_bytes(ctypes.byref(p)) == 0
