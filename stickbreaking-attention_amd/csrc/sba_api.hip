@@ -453,6 +453,16 @@ bool chain_wide(const sba_problem* p, bool fixed, const Sizes& sz) {
   const long long mean = sz.rows / sz.n_docs, longest = declared_max_doc_len(p, fixed);
   return 2 * (long long)sz.n_docs * p->heads * mean * mean >= longest * (longest > 2048 ? 3 : 2) * 65536;
 }
+// Whether Q and dO rows stream past an XCD's L2 (4 MiB) instead of staying in it, where they compete with the partial dq on its way from key tile to
+// key tile.  They are better kept (backward, us, streamed / kept: 16 heads of 7 K tokens in six documents of up to 3000 at head_dim 128 239 / 228,
+// 4 x 16 x 2048 270 / 265, 12 heads of 3 K tokens 89 / 87; 32 heads x 16 K tokens in eight documents at 96 1122 / 1095, at 64 935 / 890, at 32 746 / 731)
+// but where the chains an XCD interleaves have two to three times as much of it as the L2 holds (head_dim 128, 512 bytes a
+// token: 32 heads x 16 K tokens 1320 / 1352, 12 x 4 x 4096 696 / 710, 16 heads of 2 x 8192 1715 / 1790; one chain of 16 K tokens per XCD 1744 / 1753).
+bool chain_streams(const sba_problem* p, bool fixed, const Sizes& sz) {
+  const long long chains = (long long)sz.n_docs * p->heads, at_once = std::min<long long>((chains + CHAIN_QUEUES - 1) / CHAIN_QUEUES, CHAIN_GROUP);
+  const long long typical = (declared_max_doc_len(p, fixed) + sz.rows / sz.n_docs) / 2;
+  return used_width(p->head_dim) == 128 && at_once * typical * 128 * 4 > (10ll << 20);
+}
 // Where the one-pass form is the faster one (gain over the two passes, measured on 270 problems of 1 to 32 heads and
 // 512 to 16 K tokens in 1 to 128 documents, declared lengths exact).
 bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
@@ -548,8 +558,8 @@ int backward_chained(const sba_problem* p, bool fixed, const void* schedule, siz
   a.inv_temp = c.inv_temp;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   Timer tm(2, s);
-  return (int)(p->dtype == SBA_F16 ? f16::launch_bwd_chain : bf16::launch_bwd_chain)(a, (p->flags & SBA_ATTEND_CURRENT) != 0, chain_wide(p, fixed, sz), sz.n_q_max,
-                                                                                    device_cus(), s);
+  return (int)(p->dtype == SBA_F16 ? f16::launch_bwd_chain : bf16::launch_bwd_chain)(a, (p->flags & SBA_ATTEND_CURRENT) != 0, chain_wide(p, fixed, sz),
+                                                                                    chain_streams(p, fixed, sz), sz.n_q_max, device_cus(), s);
 }
 
 // Schedule workspace of sba_varlen_fwd_static: one array per GPU, inside the code object, so the

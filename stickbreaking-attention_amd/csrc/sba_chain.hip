@@ -125,7 +125,8 @@ __device__ __forceinline__ void async_word(const int* from, const int* dst) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2 sc1" ::"s"(lds_addr), "v"(0), "s"(from) : "memory", "m0");
 }
 
-template <int D, int U, bool AC, int NSQ>
+// STREAM: Q and dO rows, which every key tile of the chain reads again, stream past the L2 (see chain_streams).
+template <int D, int U, bool AC, int NSQ, bool STREAM>
 __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const ChainArgs a) {
   constexpr int KS = U / 16, DB = U / 32;
   constexpr int TQ = 32 * NSQ;      // queries per step
@@ -177,9 +178,7 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
     it.batch = __builtin_amdgcn_readfirstlane(mbox[parity][6]);
     return it.kt >= 0;
   };
-  // Q and dO rows, which every key tile of the chain reads again, stream past L2's partial sums of dq: those are written
-  // back and fetched again where they do not stay (1.50 -> 1.41 ms on 32 heads x 16 K tokens in 8 documents)
-  using Copy = TileCopy<D, TQ, 256, false, true>;
+  using Copy = TileCopy<D, TQ, 256, false, STREAM>;
   constexpr int LOADS_PER_TILE = 2 * Copy::NCH;
 
   // ---- the queue of this XCD ---------------------------------------------------------------------
@@ -951,34 +950,36 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
   }
 }
 
-template __global__ void bwd_chain_kernel<128, 128, false, 1>(const ChainArgs);
-template __global__ void bwd_chain_kernel<128, 128, true, 1>(const ChainArgs);
-template __global__ void bwd_chain_kernel<128, 96, false, 1>(const ChainArgs);
-template __global__ void bwd_chain_kernel<128, 96, true, 1>(const ChainArgs);
+template __global__ void bwd_chain_kernel<128, 128, false, 1, false>(const ChainArgs);
+template __global__ void bwd_chain_kernel<128, 128, true, 1, false>(const ChainArgs);
+template __global__ void bwd_chain_kernel<128, 128, false, 1, true>(const ChainArgs);
+template __global__ void bwd_chain_kernel<128, 128, true, 1, true>(const ChainArgs);
+template __global__ void bwd_chain_kernel<128, 96, false, 1, false>(const ChainArgs);
+template __global__ void bwd_chain_kernel<128, 96, true, 1, false>(const ChainArgs);
 
-template __global__ void bwd_chain_kernel<64, 64, false, 1>(const ChainArgs);
-template __global__ void bwd_chain_kernel<64, 64, true, 1>(const ChainArgs);
-template __global__ void bwd_chain_kernel<64, 64, false, 2>(const ChainArgs);
-template __global__ void bwd_chain_kernel<64, 64, true, 2>(const ChainArgs);
-template __global__ void bwd_chain_kernel<64, 32, false, 1>(const ChainArgs);
-template __global__ void bwd_chain_kernel<64, 32, true, 1>(const ChainArgs);
-template __global__ void bwd_chain_kernel<64, 32, false, 2>(const ChainArgs);
-template __global__ void bwd_chain_kernel<64, 32, true, 2>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 64, false, 1, false>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 64, true, 1, false>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 64, false, 2, false>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 64, true, 2, false>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 32, false, 1, false>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 32, true, 1, false>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 32, false, 2, false>(const ChainArgs);
+template __global__ void bwd_chain_kernel<64, 32, true, 2, false>(const ChainArgs);
 
-template <int D, int U, int NSQ>
+template <int D, int U, int NSQ, bool STREAM = false>
 static hipError_t launch_chain_d(const ChainArgs& a, bool ac, int n_q_max, int workgroups, hipStream_t s) {
   hipLaunchKernelGGL((chain_prep_kernel<D>), dim3((unsigned)n_q_max * (unsigned)a.heads), dim3(NT), 0, s, a);
   const dim3 grid(workgroups), block((4 * NSQ + 4) * 64);
-  if (ac) hipLaunchKernelGGL((bwd_chain_kernel<D, U, true, NSQ>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((bwd_chain_kernel<D, U, false, NSQ>), grid, block, 0, s, a);
+  if (ac) hipLaunchKernelGGL((bwd_chain_kernel<D, U, true, NSQ, STREAM>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((bwd_chain_kernel<D, U, false, NSQ, STREAM>), grid, block, 0, s, a);
   return hipGetLastError();
 }
 
-hipError_t launch_bwd_chain(const ChainArgs& a, bool ac, bool wide, int n_q_max, int workgroups, hipStream_t s) {
+hipError_t launch_bwd_chain(const ChainArgs& a, bool ac, bool wide, bool stream, int n_q_max, int workgroups, hipStream_t s) {
   if (a.head_dim <= 32) return wide ? launch_chain_d<64, 32, 2>(a, ac, n_q_max, workgroups, s) : launch_chain_d<64, 32, 1>(a, ac, n_q_max, workgroups, s);
   if (a.head_dim <= 64) return wide ? launch_chain_d<64, 64, 2>(a, ac, n_q_max, workgroups, s) : launch_chain_d<64, 64, 1>(a, ac, n_q_max, workgroups, s);
   if (used_width(a.head_dim) == 96) return launch_chain_d<128, 96, 1>(a, ac, n_q_max, workgroups, s);
-  return launch_chain_d<128, 128, 1>(a, ac, n_q_max, workgroups, s);
+  return stream ? launch_chain_d<128, 128, 1, true>(a, ac, n_q_max, workgroups, s) : launch_chain_d<128, 128, 1>(a, ac, n_q_max, workgroups, s);
 }
 
 }  // inline namespace SBA_ELEM_NS

@@ -199,8 +199,8 @@ inline int dkdv_main_workgroups(int head_dim, int main_tiles) { return main_tile
   hipError_t launch_bwd_short(const KArgs& a, bool attend_current, int parts, hipStream_t s);                  \
   hipError_t launch_bwd_dq_small(const KArgs& a, bool attend_current, int n_q_max, hipStream_t s);                  \
   hipError_t launch_bwd_dkdv_small(const KArgs& a, bool attend_current, int n_q_max, hipStream_t s);                  \
-  hipError_t launch_bwd_chain(const ChainArgs& a, bool attend_current, bool wide, int n_q_max, int workgroups,              \
-                              hipStream_t s);                                                                    \
+  hipError_t launch_bwd_chain(const ChainArgs& a, bool attend_current, bool wide, bool stream, int n_q_max,      \
+                              int workgroups, hipStream_t s);                                                                    \
   }
 SBA_DECLARE_LAUNCHERS(bf16)
 SBA_DECLARE_LAUNCHERS(f16)

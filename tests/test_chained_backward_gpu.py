@@ -88,6 +88,21 @@ def test_the_same_bits_from_run_to_run(form, steps, d):
         assert all(torch.equal(runs[0][i], r[i]) for r in runs[1:]), name
 
 
+@pytest.mark.parametrize("attend_current", [False, True])
+def test_rows_streamed_past_the_l2_give_the_same_bits(form, attend_current):
+    """At head_dim 128 the rows are streamed where the declared lengths say that the chains under way overfill the L2."""
+    from stickbreaking_attention import sb_attn_varlen
+    lengths = [300, 131, 32, 161, 193, 288, 609]
+    H, T = 6, sum(lengths)
+    tensors = orc.make_inputs((H, T, 128), 5)
+    drem = torch.randn((H, T), generator=torch.Generator().manual_seed(5)).to(torch.bfloat16)
+    cu = cu_from_lengths(lengths, device=DEV)
+    form(2)
+    kept, streamed = (gradients(sb_attn_varlen, tensors[:3], cu, m, attend_current, (tensors[3], drem)) for m in (max(lengths), 16384))
+    for name, a, b in zip(("dq", "dk", "dv"), kept, streamed):
+        assert torch.equal(a, b), name
+
+
 @pytest.mark.parametrize("steps,d", [(2, 128), (2, 64), (3, 64), (2, 32), (3, 32)])
 def test_a_wait_that_runs_out_gives_nan_and_nothing_else(form, steps, d):
     """Every wait for the key tile before ends after one look, so that tiles go on without the partial sums they
