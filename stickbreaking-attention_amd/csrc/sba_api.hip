@@ -255,9 +255,10 @@ bool backward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
 
 // Where bwd_short_kernel (sba_small.hip) is the faster one: short documents, and enough of them for a wave on two of three SIMDs (a wave has 64
 // tokens; dq and dk/dv passes / one-pass form before, us, at head_dim 64: 32 heads of 8 x 256 tokens 44.5 / 31.6, of 32 x 128 49.6 / 35.3, of
-// 128 x 33 75 / 45.5, of 128 x 256 390 / 322, 8 heads of 5000 tokens in documents of 1 .. 256 33.6 / 30.3; left out: 4 heads of 128 x 64 20.1 / 19.9, of
+// 128 x 33 75 / 44.3, of 128 x 256 390 / 320, 8 heads of 5000 tokens in documents of 1 .. 256 33.6 / 30.3; left out: 4 heads of 128 x 64 20.1 / 19.9, of
 // 32 x 64 16.6 / 19.0).  Above head_dim 64 a compute unit has room for one workgroup, and only what the one-pass form does not take gains (head_dim 128: 16
-// heads of 128 x 64 115 / 74, 32 of 128 x 33 160 / 112; left out: 16 heads of 128 x 128 142 / 166, 32 heads x 16 K tokens in documents of 16 .. 256 417 / 424).
+// heads of 128 x 64 115 / 68, 32 of 128 x 33 160 / 106; left out: 16 heads of 128 x 128 153 / 164, of 100 x 96 106 / 115, of 64 x 256 191 / 204, though 32 heads x
+// 16 K tokens in documents of 16 .. 256, most of them far shorter than the longest, would gain, 438 / 406).
 bool backward_short(const sba_problem* p, bool fixed, const Sizes& sz) {
   if (backward_form() != 0) return false;
   return (p->flags & SBA_PRODUCT_SPACE) && p->head_dim <= 128 && sz.n_docs > 0 && sz.n_docs <= RANK_LIMIT &&

@@ -36,6 +36,12 @@ struct WaveCopy {
   }
 };
 
+// One word for each lane, from byte offset voff of the buffer to LDS at dst + 4 * lane (see async_copy16).
+__device__ __forceinline__ void async_words(__amdgpu_buffer_rsrc_t rsrc, const float* dst, int voff) {
+  const unsigned lds_addr = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds_addr), "v"(voff), "s"(rsrc) : "memory", "m0");
+}
+
 // Four consecutive columns of a lane's output row, from `col` on (see store_rows_axpy for the sum).
 __device__ __forceinline__ void store_quad(f32x4 v, const Rows& out, const Rows& addend, int row, bool ok, int col, bool fuse, float factor, bool f32) {
   typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
@@ -542,16 +548,23 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_dkdv_sm
 // Query block i takes i + 1 steps, key block i of n takes n - i: with blocks w and n - 1 - w a wave has n + 1 in either half.
 // What bounds it: the two passes it stands in for ran at the rate of a copy, four operands read by each and the sums D written and read
 // between them; here operands come in once (32 heads x 16 K tokens in documents of 16 .. 256: 228 us for 161, of which 94 are its traffic).  What is
-// left is that a workgroup loads, computes and stores one after the other, two of them (8 waves of 220 registers, 77 KB of LDS) per compute unit, one above head_dim 64.  One document
-// to a workgroup whatever its length: 204 us, most waves idle; four slots of the tile list to a workgroup, long documents one after the other: 166 us,
+// left is that a workgroup loads, computes and stores one after the other, two of them (8 waves of 239 registers, 80 KB of LDS) per compute unit, one above head_dim 64:
+// loads and stores alone take 115 us, and neither workgroups that start late nor an order that mixes long and short documents overlaps them better.
+// So nothing is read from memory behind the first barrier: a load there is waited for behind the stores of dq, in order, and the sticks one step ahead were
+// later than a step.  Sticks come to LDS with K and V, K and V rows of both key blocks are kept from there; the document's
+// place is made scalar, which takes a loop over lanes away from every access, and operands are read four steps ahead of their multiplication.
+// On one GPU, us: these documents at head_dim 64 175 -> 164, at 32 104 -> 95; 32 heads of 128 x 256 tokens 342 -> 320, of 128 x 33 46.3 -> 44.3; at
+// head_dim 128 16 heads of 128 x 64 76 -> 68.  Streaming stores (nt) cost a third: they leave in quarters of a line.
+// One document to a workgroup whatever its length: 204 us, most waves idle; four slots of the tile list to a workgroup, long documents one after the other: 166 us,
 // and 104 for 31 us where there are few of them.
 // -------------------------------------------------------------------------------------------
 template <int D, bool AC, int U>
 __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_kernel(const KArgs a) {
-  constexpr int W = SMALL_WAVES, KS = U / 16, DB = U / 32, TILE = 32 * D, NB = SHORT_BLOCKS;
+  constexpr int W = SMALL_WAVES, KS = U / 16, DB = U / 32, TILE = 32 * D, NB = SHORT_BLOCKS, AHEAD = KS < 4 ? KS : 4;
   static_assert(NB == 2 * W && W == 4, "two blocks for each wave");
   __shared__ __attribute__((aligned(16))) unsigned short smem[2 * NB * TILE + W * 32 * 32];   // K, V blocks, Q, dO blocks in their place; p or dz of a wave
   __shared__ float sums[NB * (NB + 1) / 2 * 32];                  // D in front of key block b, from its own queries on
+  __shared__ float newer[W * (NB - 1) * 32];                      // per wave: stick left in front of its key blocks, for the queries of later blocks
 
   const int* sched = a.sched;
   const int part = blockIdx.x / a.heads;
@@ -582,6 +595,8 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_k
   unsigned short* const At = smem + 2 * team * team_waves * TILE;
   unsigned short* const Bt = At + NB * TILE;
   unsigned short* const own = smem + 2 * NB * TILE + w * 32 * 32;
+  float* const own_left = reinterpret_cast<float*>(own);          // during dq: stick left in front of the key blocks, for the wave's queries (turn 1 from 4 * 32 on)
+  float* const newer_left = newer + w * (NB - 1) * 32;
   float* const team_sums = sums + team * (NB * (NB + 1) / 2 * 32) / teams;
   auto sum_at = [&](int b, int q) { return 64 * team_waves * b - 16 * b * (b + 1) + q; };   // (a block's row begins at its own queries)
   const int rowbase = swz_off<D>(n, h);
@@ -596,7 +611,10 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_k
   }
 
   const int doc = min(doc0 + team, doc_end - 1);
-  const int4 about = reinterpret_cast<const int4*>(sched + a.docs_off)[doc];   // first token, length, first table entry
+  int4 about = reinterpret_cast<const int4*>(sched + a.docs_off)[doc];   // first token, length, first table entry
+  about.x = __builtin_amdgcn_readfirstlane(about.x);
+  about.y = __builtin_amdgcn_readfirstlane(about.y);
+  about.z = __builtin_amdgcn_readfirstlane(about.z);
   const int L = doc0 + team < doc_end ? about.y : 0, n_blocks = (L + 31) / 32, batch = a.clear_spare ? 0 : doc;   // (fixed length: by batch entry)
   const int64_t tok0 = about.x;
   auto rows_of = [&](const View& v) {
@@ -629,12 +647,52 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_k
         gf[turn][ks] = load_frag(grows, row, 32 * ks + 16 * h);
       }
   }
-  float* const stick = a.stick + (int64_t)head * a.tab_stride + about.z;
-  const __amdgpu_buffer_rsrc_t stick_rs = __builtin_amdgcn_make_buffer_rsrc(stick, 0, 4u * (unsigned)tab_doc_entries(L), 0x00020000);
-  // stick left in front of key block b for row `row`
-  auto stick_at = [&](int b, int row, bool ok) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(stick_rs, ok && row < L ? 4 * (tab_seg32(L, b) + row) : OUTSIDE, 0, 0));
-  };
+  // Everything else that is read from memory is asked for here as well: a load further down would be waited for behind the stores of dq.
+  const float* const stick = a.stick + (int64_t)head * a.tab_stride + about.z;
+  const __amdgpu_buffer_rsrc_t stick_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(stick), 0, 4u * (unsigned)tab_doc_entries(L), 0x00020000);
+  // byte offset of the stick left in front of key block b for row `row`
+  auto stick_off = [&](int b, int row, bool ok) { return ok && row < L ? 4 * (tab_seg32(L, b) + row) : OUTSIDE; };
+#pragma unroll
+  for (int turn = 0; turn < 2; ++turn)
+#pragma unroll
+    for (int i = 0; i < W * (turn + 1); i += 2)         // two key blocks an instruction
+      if (i <= block_of[turn]) async_words(stick_rs, own_left + 32 * (W * turn + i), stick_off(i + h, 32 * block_of[turn] + n, i + h <= block_of[turn]));
+  const int later[2] = {block_of[0] >= 0 ? n_blocks - 1 - block_of[0] : 0, block_of[1] >= 0 ? n_blocks - 1 - block_of[1] : 0};   // (at most NB - 1 together)
+#pragma unroll
+  for (int i = 0; i < NB - 1; i += 2)
+    if (i < later[0] + later[1] && (i < NB - 2 || h == 0)) {
+      const int at = i + h, turn = at < later[0] ? 0 : 1;
+      const int kb = turn == 0 ? block_of[0] : block_of[1], b = kb + 1 + (turn == 0 ? at : at - later[0]);
+      async_words(stick_rs, newer_left + 32 * i, stick_off(kb, 32 * b + n, at < later[0] + later[1]));
+    }
+  float newest_left[2], rem[2], run0[2];      // stick left in front of the wave's own blocks on the diagonal; of its rows, at last; D in front of the oldest key (see bwd_dq_small_kernel)
+#pragma unroll
+  for (int turn = 0; turn < 2; ++turn) {
+    const int qrow = block_of[turn] >= 0 ? 32 * block_of[turn] + n : L;
+    const auto word = [&](int off) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(stick_rs, off, 0, 0)); };
+    newest_left[turn] = word(stick_off(block_of[turn], qrow, true));
+    rem[turn] = word(qrow < L ? 4 * (tab_rowplane32(L) + qrow) : OUTSIDE);
+    run0[turn] = 0.0f;
+    if (a.grem.ptr != nullptr && qrow < L)
+      run0[turn] = (float)(reinterpret_cast<const elem_t*>(a.grem.ptr) + batch * a.grem.sb + head * a.grem.sh + tok0 * a.grem.st)[(int64_t)qrow * a.grem.st];
+  }
+  if (a.fuse) {
+#pragma unroll
+    for (int turn = 0; turn < 2; ++turn) {
+      float dot = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const el8 vown = load_frag(vrows, block_of[turn] >= 0 ? 32 * block_of[turn] + n : L, 32 * ks + 16 * h);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dot = fmaf((float)gf[turn][ks][e], (float)vown[e], dot);
+      }
+      float lo, hi;
+      both_halves(dot, lo, hi);
+      run0[turn] += lo + hi;
+    }
+  }
+#pragma unroll
+  for (int turn = 0; turn < 2; ++turn) run0[turn] *= rem[turn];
   wait_loads<0>();
   lds_barrier();
 
@@ -645,25 +703,7 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_k
     if (qb >= 0) {
       const int qrow = 32 * qb + n;
       const bool qvalid = qrow < L;
-      float e_next = stick_at(0, qrow, true), run;
-      {                                       // D in front of the oldest key (see bwd_dq_small_kernel)
-        float dr = 0.0f;
-        if (a.grem.ptr != nullptr && qvalid)
-          dr = (float)(reinterpret_cast<const elem_t*>(a.grem.ptr) + batch * a.grem.sb + head * a.grem.sh + tok0 * a.grem.st)[(int64_t)qrow * a.grem.st];
-        if (a.fuse) {
-          float dot = 0.0f;
-#pragma unroll
-          for (int ks = 0; ks < KS; ++ks) {
-            const el8 vown = load_frag(vrows, qrow, 32 * ks + 16 * h);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) dot = fmaf((float)gf[turn][ks][e], (float)vown[e], dot);
-          }
-          float lo, hi;
-          both_halves(dot, lo, hi);
-          dr += lo + hi;
-        }
-        run = qvalid ? dr * stick[(unsigned)(tab_rowplane32(L) + qrow)] : 0.0f;
-      }
+      float run = run0[turn];
       f32x16 dq[DB];
 #pragma unroll
       for (int db = 0; db < DB; ++db)
@@ -673,16 +713,22 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_k
       for (int b = 0; b <= qb; ++b) {
         const unsigned short* const Kr = At + b * TILE;
         const unsigned short* const Vr = Bt + b * TILE;
-        float c = qvalid ? e_next : 1.0f;
-        e_next = stick_at(b + 1, qrow, b < qb);
+        float c = own_left[32 * (W * turn + b) + n];
+        if (!qvalid) c = 1.0f;
         if (h == 0) team_sums[sum_at(b, qrow)] = run;
         f32x16 x, da;
 #pragma unroll
         for (int i = 0; i < 16; ++i) x[i] = da[i] = 0.0f;
+        el8 kr[AHEAD], vr[AHEAD];
+#pragma unroll
+        for (int ks = 0; ks < AHEAD; ++ks) { kr[ks] = lds_row8(Kr + (rowbase ^ (ks << 4))); vr[ks] = lds_row8(Vr + (rowbase ^ (ks << 4))); }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-          x = mfma32(lds_row8(Kr + (rowbase ^ (ks << 4))), qf[turn][ks], x);
-          da = mfma32(lds_row8(Vr + (rowbase ^ (ks << 4))), gf[turn][ks], da);
+          x = mfma32(kr[ks % AHEAD], qf[turn][ks], x);
+          da = mfma32(vr[ks % AHEAD], gf[turn][ks], da);
+          if (ks + AHEAD < KS) { kr[ks % AHEAD] = lds_row8(Kr + (rowbase ^ ((ks + AHEAD) << 4))); vr[ks % AHEAD] = lds_row8(Vr + (rowbase ^ ((ks + AHEAD) << 4))); }
+          __builtin_amdgcn_sched_barrier(0);
         }
         float p[16], m[16], ends[2];
         grad_weights<AC, true>(x, a.c, 32 * b, 32 * qb, qrow, h, c, p, m, ends);
@@ -699,11 +745,16 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_k
   }
 
   // ---- dk, dv ----
-  el8 kf[KS], vf[KS];                         // MFMA row n holds key 32 b + kperm(n)
+  el8 kf[KS], vf[KS], kf1[KS], vf1[KS];       // MFMA row n holds key 32 b + kperm(n)
   {
-    const int at = max(block_of[0], 0) * TILE;
+    const int at = max(block_of[0], 0) * TILE, at1 = max(block_of[1], 0) * TILE;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) { kf[ks] = lds_row8(At + at + (rowbase ^ (ks << 4))); vf[ks] = lds_row8(Bt + at + (rowbase ^ (ks << 4))); }
+    for (int ks = 0; ks < KS; ++ks) {
+      kf[ks] = lds_row8(At + at + (rowbase ^ (ks << 4)));
+      vf[ks] = lds_row8(Bt + at + (rowbase ^ (ks << 4)));
+      kf1[ks] = lds_row8(At + at1 + (rowbase ^ (ks << 4)));
+      vf1[ks] = lds_row8(Bt + at1 + (rowbase ^ (ks << 4)));
+    }
   }
   lds_barrier();                              // K and V have been read
 #pragma unroll
@@ -722,30 +773,35 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_k
     const int kb = turn == 0 ? block_of[0] : block_of[1];
     if (kb < 0) break;
     const int k0 = 32 * kb;
-    float rem_own = 0.0f;                     // fused output: rem_j * do_j reaches dv_j through the diagonal of p (see bwd_dkdv_kernel)
-    if (a.fuse && k0 + n < L) rem_own = stick[(unsigned)(tab_rowplane32(L) + k0 + n)];
+    const float rem_own = turn == 0 ? rem[0] : rem[1];   // fused output: rem_j * do_j reaches dv_j through the diagonal of p (see bwd_dkdv_kernel)
+    const float newest = turn == 0 ? newest_left[0] : newest_left[1];
+    const float* const left = newer_left + (turn == 0 ? 0 : 32 * later[0]) + n;
     f32x16 dk[DB], dv[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int i = 0; i < 16; ++i) dk[db][i] = dv[db][i] = 0.0f;
-    float e_next = stick_at(kb, k0 + n, true);
 #pragma unroll 1
     for (int b = kb; b < n_blocks; ++b) {
       const int qrow = 32 * b + n;
       const bool ok = qrow < L;
-      const float c = ok ? e_next : 1.0f;
+      const float c = !ok ? 1.0f : b == kb ? newest : left[32 * max(b - kb - 1, 0)];
       float before = ok ? team_sums[sum_at(kb, qrow)] : 0.0f;
-      e_next = stick_at(kb, qrow + 32, true);
       const unsigned short* const Qr = At + b * TILE;
       const unsigned short* const Gr = Bt + b * TILE;
       f32x16 x, da;
 #pragma unroll
       for (int i = 0; i < 16; ++i) x[i] = da[i] = 0.0f;
+      el8 qr[AHEAD], gr[AHEAD];
+#pragma unroll
+      for (int ks = 0; ks < AHEAD; ++ks) { qr[ks] = lds_row8(Qr + (rowbase ^ (ks << 4))); gr[ks] = lds_row8(Gr + (rowbase ^ (ks << 4))); }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        x = mfma32(kf[ks], lds_row8(Qr + (rowbase ^ (ks << 4))), x);
-        da = mfma32(vf[ks], lds_row8(Gr + (rowbase ^ (ks << 4))), da);
+        x = mfma32(kf[ks], qr[ks % AHEAD], x);
+        da = mfma32(vf[ks], gr[ks % AHEAD], da);
+        if (ks + AHEAD < KS) { qr[ks % AHEAD] = lds_row8(Qr + (rowbase ^ ((ks + AHEAD) << 4))); gr[ks % AHEAD] = lds_row8(Gr + (rowbase ^ ((ks + AHEAD) << 4))); }
+        __builtin_amdgcn_sched_barrier(0);
       }
       float p[16], m[16], ends[2], carry = c;
       grad_weights<AC, true>(x, a.c, k0, 32 * b, qrow, h, carry, p, m, ends);
@@ -781,10 +837,7 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_k
     }
     if (turn == 0 && block_of[1] >= 0) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        kf[ks] = load_frag(krows, 32 * block_of[1] + kperm(n), 32 * ks + 16 * h);
-        vf[ks] = load_frag(vrows, 32 * block_of[1] + kperm(n), 32 * ks + 16 * h);
-      }
+      for (int ks = 0; ks < KS; ++ks) { kf[ks] = kf1[ks]; vf[ks] = vf1[ks]; }
     }
     store_rows(dk, a.inv_temp, rows_of(a.dk), k0 + n, L, h, a.out_f32);
     store_rows(dv, 1.0f, rows_of(a.dv), k0 + n, L, h, a.out_f32);
