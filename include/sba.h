@@ -247,13 +247,13 @@ int sba_attn_bwd(const sba_problem* p, const void* schedule, size_t schedule_siz
 
 /* The backward with every score formed once.  Up to head_dim 128 it is one pass, dq is handed from key tile to key tile
  * through scratch memory (csrc/sba_chain.hip); above, the dq pass hands the weights and the gradients of the logits
- * to the dk/dv pass through scratch memory, 4 bytes per causal pair (csrc/sba_wide.hip).  For the problems it is the
- * faster form of, sba_chain_scratch_bytes returns the scratch it needs (16-byte aligned, contents irrelevant, one per
+ * to the dk/dv pass through scratch memory, 4 bytes per causal pair (csrc/sba_wide.hip), for as many heads at a time as
+ * 3.75 GiB hold.  For the problems it is the faster form of, sba_chain_scratch_bytes returns the scratch it needs (16-byte aligned, contents irrelevant, one per
  * concurrent call; never more than 3.75 GiB above head_dim 128) and 0 for every other; a caller then takes
  * sba_varlen_bwd / sba_attn_bwd, which choose among their kernels by size.  Same inputs, outputs, table and refusals; it
  * needs no gradient table, and the results differ from the two-pass form's by rounding.  Problems it
- * cannot take (log-space carry; up to head_dim 128 a device that is not eight XCDs of 32 compute units; above, more
- * scratch than that) return SBA_E_SHAPE. */
+ * cannot take (log-space carry; up to head_dim 128 a device that is not eight XCDs of 32 compute units; above, heads of
+ * which too few fit at a time to fill the device) return SBA_E_SHAPE. */
 size_t sba_chain_scratch_bytes(const sba_problem* p);
 int sba_varlen_bwd_chained(const sba_problem* p, const void* schedule, size_t schedule_size,
                            const sba_view* q, const sba_view* k, const sba_view* v,

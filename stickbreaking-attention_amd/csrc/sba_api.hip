@@ -409,28 +409,49 @@ ChainScratch chain_scratch(const sba_problem* p, const Sizes& sz) {
 // ---- the two passes of head_dim 129 .. 256 with p and dz handed on (sba_wide.hip) -----------------------
 // The dq pass stores p and dz, 4 bytes per causal pair, and the dk/dv pass multiplies them instead of forming both again.  It is the faster
 // form of 99 problems of 2 to 16 heads and 256 to 8192 tokens in 1 to 60 documents at head_dim 136, 160 and 256 (1.12 by the geometric mean, 0.98 ..
-// 1.39) and of the larger ones (16 heads x 16 K tokens in eight documents at 256: 1515 -> 1180 us, 12 x 4 x 4096 1520 -> 1203).  The line is the room: 32 times
-// a carry table, 32 bytes more for every query and 32 keys than GIVEN_SCRATCH_MAX has are with the passes that form the scores twice.
-size_t given_scratch(const sba_problem* p, bool fixed) { return (size_t)p->heads * (size_t)table_entries_bound(p, fixed) * (2 * PZ_WORDS); }
+// 1.39) and of the larger ones (16 heads x 16 K tokens in eight documents at 256: 1515 -> 1180 us, 12 x 4 x 4096 1520 -> 1203).
+// Heads are independent: where the room (32 times a carry table, 32 bytes more for every query and 32 keys) does not hold them all, equal groups
+// of them are taken one after the other in the same place (head_dim 256, us, scores formed twice / in groups: 16 heads of 2 x 8192 3826 / 2960, 32 of 16 x 2048
+// 4527 / 3690, 16 of 8 x 4096 3948 / 3342, 5 of 2 x 16384 4823 / 3741).  A group has to fill the chip by itself, its launches ending with
+// the most expensive of its tiles: the line is at three quarters as many of its blocks per compute unit as that tile has (3 heads of 20000, 0.92 of them, 4241 / 3236;
+// 2 of 24576, 0.75, 4035 / 3604; 1 of 32768, 0.5, 7045 / 8998).
+size_t given_head(const sba_problem* p, bool fixed) { return (size_t)table_entries_bound(p, fixed) * (2 * PZ_WORDS); }
+int given_group(const sba_problem* p, bool fixed) {
+  const long long room = (long long)(GIVEN_SCRATCH_MAX / std::max<size_t>(given_head(p, fixed), 1));
+  if (room >= p->heads) return p->heads;
+  if (room == 0) return 0;
+  const int groups = (int)((p->heads + room - 1) / room), each = (p->heads + groups - 1) / groups;
+  const long long cus = device_cus() > 0 ? device_cus() : 256;
+  return each * table_entries_bound(p, fixed) >= 3 * cus * declared_max_doc_len(p, fixed) ? each : 0;
+}
+size_t given_scratch(const sba_problem* p, bool fixed) { return (size_t)given_group(p, fixed) * given_head(p, fixed); }
 bool given_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
-  return (p->flags & SBA_PRODUCT_SPACE) && p->head_dim > 128 && sz.n_docs > 0 && given_scratch(p, fixed) <= GIVEN_SCRATCH_MAX;
+  return (p->flags & SBA_PRODUCT_SPACE) && p->head_dim > 128 && sz.n_docs > 0 && given_group(p, fixed) > 0;
 }
 bool given_wanted(const sba_problem* p, bool fixed, const Sizes& sz) { return backward_form() != 1 && given_possible(p, fixed, sz); }
 
 int backward_given(const sba_problem* p, bool fixed, const Sizes& sz, KArgs& a, void* scratch, size_t scratch_bytes, hipStream_t s) {
+  const int group = given_group(p, fixed);
   a.pz = static_cast<unsigned short*>(scratch);
-  a.pz_entries = (int64_t)(scratch_bytes / (2 * PZ_WORDS) / (size_t)p->heads) & ~(int64_t)31;
+  a.pz_entries = (int64_t)(scratch_bytes / (2 * PZ_WORDS) / (size_t)group) & ~(int64_t)31;
   const BwdBounds bb = backward_bounds(p, fixed, sz);
   const DkdvGrid g = dkdv_grid(false, bb.n_long_max, bb.n_tail_max, sz.n_kv_max);
-  const bool ac = (p->flags & SBA_ATTEND_CURRENT) != 0, f16 = p->dtype == SBA_F16;
-  hipError_t he;
-  {
-    Timer tm(1, s);
-    he = (f16 ? f16::launch_bwd_dq_wide : bf16::launch_bwd_dq_wide)(a, ac, true, sz.n_q_max, s);
-  }
-  if (he == hipSuccess) {
-    Timer tm(2, s);
-    he = (f16 ? f16::launch_bwd_dkdv_given : bf16::launch_bwd_dkdv_given)(a, g.main_tiles, s);
+  const bool ac = (p->flags & SBA_ATTEND_CURRENT) != 0, f16 = p->dtype == SBA_F16, whole = group == p->heads;
+  hipError_t he = hipSuccess;
+  Timer all(2, s, !whole);                    // (several groups: one figure for everything, like the one-pass form)
+  for (int head = 0; head < p->heads && he == hipSuccess; head += group) {
+    a.heads = std::min(group, p->heads - head);
+    {
+      Timer tm(1, s, whole);
+      he = (f16 ? f16::launch_bwd_dq_wide : bf16::launch_bwd_dq_wide)(a, ac, true, sz.n_q_max, s);
+    }
+    if (he == hipSuccess) {
+      Timer tm(2, s, whole);
+      he = (f16 ? f16::launch_bwd_dkdv_given : bf16::launch_bwd_dkdv_given)(a, g.main_tiles, s);
+    }
+    for (View* v : {&a.q, &a.k, &a.v, &a.go, &a.grem, &a.dq, &a.dk, &a.dv})
+      if (v->ptr != nullptr) v->ptr += 2 * (int64_t)group * v->sh;   // (strides count 16-bit words)
+    a.stick += (int64_t)group * a.tab_stride;
   }
   return (int)he;
 }

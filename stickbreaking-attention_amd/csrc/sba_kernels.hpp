@@ -45,7 +45,7 @@ struct KArgs {
   int lg_deal;                 // forward: the logarithm of the device's compute units if it holds the launch at once (see deal_item), or NO_DEAL
 };
 
-constexpr size_t GIVEN_SCRATCH_MAX = 0xf0000000u;   // bytes of p and dz that are handed on: 32-bit offsets reach them
+constexpr size_t GIVEN_SCRATCH_MAX = 0xf0000000u;   // bytes of p and dz that are handed on at a time: 32-bit offsets reach them
 
 constexpr int NO_DEAL = 31;    // (no launch has a second round of 2^31 workgroups)
 // Workgroups of the forward that a compute unit holds.

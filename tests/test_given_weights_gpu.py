@@ -69,6 +69,25 @@ def test_fixed_length_and_token_major(form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("fixed", [False, True])
+def test_heads_in_groups(form, fixed):
+    """33 heads, of which 3.75 GiB hold 29: groups of 17 and 16."""
+    from stickbreaking_attention import sb_attn, sb_attn_varlen
+    H, B, T, d = 33, 16, 2048, 136
+    gen = torch.Generator(device=DEV).manual_seed(8)
+    draw = lambda *shape: torch.randn(shape, generator=gen, device=DEV).to(torch.bfloat16)
+    shape = (B, H, T, d) if fixed else (H, B * T, d)
+    x, do, drem = [draw(*shape).requires_grad_() for _ in range(3)], draw(*shape), draw(*shape[:-1])
+    cu = cu_from_lengths([T] * B, device=DEV)
+    run = lambda: torch.autograd.grad(sb_attn(*x) if fixed else sb_attn_varlen(*x, cu, T, zero_start=False), x, (do, drem))
+    got = run()
+    form(1)
+    for name, g, t in zip(("dq", "dk", "dv"), got, run()):
+        for head in (0, 16, 17, 32):
+            assert_close(name, *((t.movedim(-3, 0) if fixed else t)[head].float() for t in (g, t)))
+
+
+@pytest.mark.gpu
 def test_a_document_longer_than_declared_gives_nan(monkeypatch):
     """Room for p and dz goes by the declared length: what does not fit is refused by the kernels, and every gradient is NaN."""
     from stickbreaking_attention import _ops, sb_attn_varlen
@@ -92,10 +111,14 @@ def test_scratch(form):
         return lib.sba_varlen_bwd_chained(ctypes.byref(problem), at, lib.sba_schedule_bytes(ctypes.byref(problem)), view, view, view, view, row,
                                           at, 1 << 31, ctypes.c_void_p(scratch), size, view, view, view, None)
     assert call(p, 0x1000, need - 1) == -6 and call(p, 0x1004, need) == -6
-    # more than 32-bit offsets reach, and the log-space carry: the other passes
-    large = problem(head_dim=256, heads=32, flags=nat.FLAG_PRODUCT_SPACE)
+    # heads that do not fit together share the room in equal groups
+    shared = problem(head_dim=256, heads=33, flags=nat.FLAG_PRODUCT_SPACE)
+    assert lib.sba_chain_scratch_bytes(ctypes.byref(shared)) == need // 16 * 17
+    # a group too small to fill the device, a head beyond the room, and the log-space carry: the other passes
+    large = problem(head_dim=256, heads=8, tokens=32768, n_docs=1, max_doc_len=32768, flags=nat.FLAG_PRODUCT_SPACE)
+    longer = problem(head_dim=256, heads=8, tokens=65536, n_docs=1, max_doc_len=65536, flags=nat.FLAG_PRODUCT_SPACE)
     log = problem(head_dim=256, heads=16)
-    for other in (large, log):
+    for other in (large, longer, log):
         assert lib.sba_chain_scratch_bytes(ctypes.byref(other)) == 0
         assert call(other, 0x1000, 1 << 40) == -4
     form(1)
