@@ -161,20 +161,22 @@ __global__ void __launch_bounds__(NT, D > 128 ? 2 : 3) fwd_kernel(const KArgs a)
 #pragma unroll
     for (int i = 0; i < 16; ++i) x[i] = 0.0f;
     {
-      // K fragments are read four ahead of their multiplication, in an order that is pinned: left to itself the compiler reads one or two ahead
+      // Beyond head_dim 64 K fragments are read four ahead of their multiplication, in an order that is pinned: left to itself the compiler reads one or two ahead
       // and waits for each.  32 heads of 64 K tokens, longest document 32 K, at head_dim 128 10.98 -> 10.81 ms (sustained, at a lower clock than
       // the 9.47 -> 9.41 of a few launches), 12 heads of 4 x 4096 218 -> 211 us, 16 heads x 16 K in eight documents at 256 430 -> 415, at
-      // 192 322 -> 315, at 64 and 32 within 1 %.  (Half of V's fragments read before the weights are formed: nothing at 64 and 96, spills from 128 on.)
+      // 192 322 -> 315.  (Four or two fragments pinned at 64 and 32: 0.8 % slower to 0.  Half of V's fragments read before the weights are formed: nothing at
+      // 64 and 96, spills from 128 on.)
+      constexpr bool PIN = KS > 4;
       constexpr int AHEAD = KS < 4 ? KS : 4;
       el8 kfr[AHEAD];
 #pragma unroll
       for (int ks = 0; ks < AHEAD; ++ks) kfr[ks] = lds_row8(Kt + koff[ks % KO] + 128 * (ks / KO));
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         x = mfma32(kfr[ks % AHEAD], qf[ks], x);
         if (ks + AHEAD < KS) kfr[ks % AHEAD] = lds_row8(Kt + koff[(ks + AHEAD) % KO] + 128 * ((ks + AHEAD) / KO));
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
       }
     }
     float p[16];
