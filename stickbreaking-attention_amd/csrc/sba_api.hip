@@ -464,16 +464,28 @@ bool chain_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
          chains <= (long long)CHAIN_QUEUES * CHAIN_GROUP * CHAIN_MAX_GROUPS &&
          ((long long)declared_max_doc_len(p, fixed) + BM) * chain_width(p->head_dim) * 4 < (1ll << 31) && device_cus() == 256;
 }
-// Steps of 64 queries instead of 32 (head_dim <= 64).  They do more per step and CU (4 x 16 x 2048 at head_dim 64: 167 us
-// for 198) but a key tile lags its predecessor by four steps of either size, so as long as that lag is what a problem takes
-// (one head of 1024 keys: 58 us for 49) the small ones are the better ones.  The line: the work of a CU in steps, chains mean^2
-// / (2 x 64 x 128 x 256 CUs), against the steps of the longest document, where beyond 2048 keys more of a chain's tiles
-// start behind one another than side by side (16 x 4096: 250 us for 224, 16 x 8192: 589 for 653).
+// What a problem's chains look like from the host: one document of the longest declared length, the others alike.
+struct Chains { long long number, longest, other, squares, per_xcd, long_per_xcd; };   // squares: of a chain's length, over all of them
+Chains chains_of(const sba_problem* p, bool fixed, const Sizes& sz) {
+  Chains c;
+  c.number = (long long)sz.n_docs * p->heads;
+  c.longest = std::min<long long>(declared_max_doc_len(p, fixed), sz.rows);
+  c.other = sz.n_docs > 1 ? (sz.rows - c.longest) / (sz.n_docs - 1) : 0;
+  c.squares = p->heads * (c.longest * c.longest + (sz.n_docs - 1) * c.other * c.other);
+  c.per_xcd = (c.number + CHAIN_QUEUES - 1) / CHAIN_QUEUES;          // (dealt out longest first)
+  c.long_per_xcd = (p->heads + CHAIN_QUEUES - 1) / CHAIN_QUEUES;
+  return c;
+}
+// Steps of 64 queries instead of 32 (head_dim <= 64).  They do more per step and CU (4 x 16 x 2048 at head_dim 64: 153 us
+// for 179) but a key tile lags its predecessor by three steps of either size, so as long as that lag is what a problem takes
+// (8 heads of 8192 keys: 430 us for 372) the small ones are the better ones.  The line: the work of a CU in steps, squares
+// / (2 x 64 x 128 x 256 CUs), against the steps of the longest document and a twentieth more (32 heads of 7 K tokens in six documents of up to
+// 3000 264 us for 298, 12 x 3 x 2500 161 for 175, 4 x 2 x 8192 428 for 371).
 bool chain_wide(const sba_problem* p, bool fixed, const Sizes& sz) {
   const int form = backward_form();
   if (form == 2 || form == 3) return form == 3;
-  const long long mean = sz.rows / sz.n_docs, longest = declared_max_doc_len(p, fixed);
-  return 2 * (long long)sz.n_docs * p->heads * mean * mean >= longest * (longest > 2048 ? 3 : 2) * 65536;
+  const Chains c = chains_of(p, fixed, sz);
+  return 20 * c.squares >= 21 * c.longest * 65536;
 }
 // Whether Q and dO rows stream past an XCD's L2 (4 MiB) instead of staying in it, where they compete with the partial dq on its way from key tile to
 // key tile.  They are better kept (backward, us, streamed / kept: 16 heads of 7 K tokens in six documents of up to 3000 at head_dim 128 239 / 228,
@@ -485,25 +497,25 @@ bool chain_streams(const sba_problem* p, bool fixed, const Sizes& sz) {
   const long long typical = (declared_max_doc_len(p, fixed) + sz.rows / sz.n_docs) / 2;
   return used_width(p->head_dim) == 128 && at_once * typical * 128 * 4 > (10ll << 20);
 }
-// Where the one-pass form is the faster one (gain over the two passes, measured on 270 problems of 1 to 32 heads and
-// 512 to 16 K tokens in 1 to 128 documents, declared lengths exact).
+// Where the one-pass form is the faster one (gain over the two passes; measured on 1220 problems of 1 to 32 heads and 512 to 200 K tokens in
+// 1 to 128 documents, declared lengths exact: 1.003 of the faster form's time at head_dim 96 and 128, 1.01 at 64, 1.015 at 32, by the geometric mean).
 bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
   const int form = backward_form();
   if (form == 1 || !chain_possible(p, fixed, sz)) return false;
   if (form == 2 || form == 3) return true;
   if (backward_short(p, fixed, sz) || backward_small(p, fixed, sz)) return false;
-  const long long chains = (long long)sz.n_docs * p->heads, items = (long long)sz.n_kv_max * p->heads;
-  const long long mean = sz.rows / sz.n_docs, longest = declared_max_doc_len(p, fixed);
+  const Chains c = chains_of(p, fixed, sz);
+  const long long items = (long long)sz.n_kv_max * p->heads, mean = sz.rows / sz.n_docs, longest = declared_max_doc_len(p, fixed);
   // a document of one or two steps: nothing to hand on, and one launch more (0.85 .. 1.01)
   if (longest <= 64) return false;
-  // Every chain stays on one XCD.  While an XCD holds all its tiles at once (32 CUs, 4096 keys) how the chains fall on the
-  // XCDs does not matter (1.1 .. 1.4, one chain alone included); beyond, the XCDs have to come out even: no more than a tenth idle
-  // in the last round (12 chains of 4096 and more: 0.87 .. 0.95), and no chain longer than its share of the whole (one
-  // of 8192 next to seven short ones: 0.89).
-  const long long per_xcd = (chains + CHAIN_QUEUES - 1) / CHAIN_QUEUES;
-  if (per_xcd * longest > 32 * BKV) {
-    if (10 * chains < 9 * CHAIN_QUEUES * per_xcd) return false;
-    if (longest > 32 * BKV && chains * mean * mean < (CHAIN_QUEUES + 4) * longest * longest) return false;
+  // Every chain stays on one XCD.  While an XCD holds nearly all its tiles at once (32 CUs, 4096 keys; twice that for its few last chains) how
+  // the chains fall on the XCDs does not matter (1.1 .. 1.4, one chain alone included; 3 heads of 2 documents of 2500 at head_dim 128 1.21).  Beyond, the XCDs
+  // have to come out even, the more the longer the chains are: one that has half as much again to do as their mean is made up for by chains of up to
+  // 4096 keys (12 heads of 4096 1.05), a third more is too much for longer ones (12 heads of 16384 0.91; two heads of 20000 next to short documents
+  // 0.55).  Even ones gain at any length (8 heads of 8192 1.12, of 16384 and 8192 1.3, of 8192, 4096 and 2048 1.23 .. 1.38).
+  if (std::max(c.long_per_xcd * c.longest, c.per_xcd * mean) > 64 * BKV) {
+    const long long most = c.long_per_xcd * c.longest * c.longest + (c.per_xcd - c.long_per_xcd) * c.other * c.other;
+    if (10 * CHAIN_QUEUES * most > (longest <= 32 * BKV ? 15 : 13) * c.squares) return false;
   }
   // Wide heads gain from there on (1.03 .. 1.38; 0.96 where every document ends in a nearly empty tile).  For narrow ones what
   // an item costs before its first step weighs more: with several items per CU only documents of some length gain

@@ -1,6 +1,8 @@
 """The one-pass backward (csrc/sba_chain.hip), forced wherever it is possible: documents at the edges of its steps of 32 and
 64 queries and 128-key tiles and of the three steps a tile lags behind its predecessor, both kernel widths and heads
 narrower than them, against the oracle; and queues of many items per workgroup and many groups, against the two-pass form."""
+import ctypes
+
 import pytest
 import torch
 
@@ -86,6 +88,30 @@ def test_the_same_bits_from_run_to_run(form, steps, d):
     for i, name in enumerate(("dq", "dk", "dv")):
         assert_close(name, runs[0][i], two[i].float())
         assert all(torch.equal(runs[0][i], r[i]) for r in runs[1:]), name
+
+
+@pytest.mark.parametrize("H,d,lengths,declared,chained", [
+    (4, 96, [2500] * 3, 2500, True),                    # 12 chains on 8 XCDs, few enough tiles to be held at once
+    (12, 64, [4096], 4096, True),
+    (18, 64, [3000], 3000, True), (12, 64, [4500], 4500, False),      # a third more than the mean on the worst XCD, which does not hold them: up to 4096 keys
+    (16, 64, [6000, 500, 500, 500], 6000, True),        # even chains of any length
+    (2, 128, [9000, 300, 200], 9000, False),            # two long ones, each on an XCD of its own
+    (16, 32, [5000, 4000], 16384, True),                # declared longer than there are rows
+])
+def test_the_choice_between_one_pass_and_two(form, H, d, lengths, declared, chained):
+    from stickbreaking_attention import _native as nat, sb_attn_varlen
+    T = sum(lengths)
+    p = nat.SbaProblem(1, d, H, 1, T, len(lengths), declared, nat.FLAG_PRODUCT_SPACE, d ** -0.5, 0x1000)
+    assert (nat.load().sba_chain_scratch_bytes(ctypes.byref(p)) > 0) == chained
+    gen = torch.Generator(device=DEV).manual_seed(T)
+    x = [torch.randn((H, T, d), generator=gen, device=DEV).to(torch.bfloat16).requires_grad_() for _ in range(3)]
+    do = torch.randn((H, T, d), generator=gen, device=DEV).to(torch.bfloat16)
+    cu = cu_from_lengths(lengths, device=DEV)
+    run = lambda: torch.autograd.grad(sb_attn_varlen(*x, cu, declared, zero_start=False)[0], x, do)
+    got = run()
+    form(1)
+    for name, g, t in zip(("dq", "dk", "dv"), got, run()):
+        assert_close(name, g, t.float())
 
 
 @pytest.mark.parametrize("attend_current", [False, True])
