@@ -24,7 +24,7 @@ for p in (ROOT, os.path.join(ROOT, "stickbreaking-attention_amd")):
 PEAK_BF16_TFLOPS = 2500.0   # MI355X published dense bf16 MFMA peak
 PEAK_HBM_GBS = 8000.0       # MI355X published HBM3E bandwidth
 
-# Figures that only rocprofv3 can see, on workloads c3 and c2, recorded from the runs whose summaries are under profiles/
+# Figures that only rocprofv3 can see, on workloads c3, c2 and d256, recorded from the runs whose summaries are under profiles/
 # and valid for the library version they were measured with (any other version of libsba.so reports null).
 #   traffic: bytes per launch between the L2s and the fabric from two `--pmc` runs of this script (FETCH_SIZE, then
 #     WRITE_SIZE, KiB per dispatch, summed over XCDs), each scaled by what the same counter reads for the 256 MiB device
@@ -32,12 +32,15 @@ PEAK_HBM_GBS = 8000.0       # MI355X published HBM3E bandwidth
 #   mfma_busy, valu_busy, coexec: fractions of the launch's SIMD-cycles in which the matrix pipe is busy
 #     (SQ_VALU_MFMA_BUSY_CYCLES), a vector instruction is active (4 x SQ_ACTIVE_INST_VALU) and both at once
 #     (SQ_VALU_MFMA_COEXEC_CYCLES), over 1024 SIMDs x GRBM_GUI_ACTIVE / 8: profiles/c3_sq_counters_pmc.txt
-#   (c2: profiles/c2_one_pass_backward.txt)
+#   (c2: profiles/c2_one_pass_backward.txt, d256: profiles/d256_fwd_bwd_kernel_trace.txt)
 MEASURED = {"sba_version": 215,
-            "c3": {"fwd_kernel": {"traffic": 1.065e9, "mfma_busy": 0.457, "valu_busy": 0.544, "coexec": 0.188},
-                   "bwd_chain_kernel": {"traffic": 7.863e9, "mfma_busy": 0.349, "valu_busy": 0.382, "coexec": 0.106}},
-            "c2": {"fwd_kernel": {"traffic": 1.135e8, "mfma_busy": 0.254, "valu_busy": 0.561, "coexec": 0.150},
-                   "bwd_chain_kernel": {"traffic": 6.487e8, "mfma_busy": 0.227, "valu_busy": 0.461, "coexec": 0.114}}}
+            "c3": {"fwd_kernel": {"traffic": 1.070e9, "mfma_busy": 0.464, "valu_busy": 0.552, "coexec": 0.196},
+                   "bwd_chain_kernel": {"traffic": 7.599e9, "mfma_busy": 0.358, "valu_busy": 0.397, "coexec": 0.131}},
+            "c2": {"fwd_kernel": {"traffic": 1.134e8, "mfma_busy": 0.257, "valu_busy": 0.567, "coexec": 0.152},
+                   "bwd_chain_kernel": {"traffic": 6.510e8, "mfma_busy": 0.237, "valu_busy": 0.496, "coexec": 0.120}},
+            "d256": {"fwd_kernel": {"traffic": 1.598e9, "mfma_busy": 0.465, "valu_busy": 0.319, "coexec": 0.092},
+                     "bwd_dq_wide_kernel": {"traffic": 2.719e9, "mfma_busy": 0.372, "valu_busy": 0.385, "coexec": 0.121},
+                     "bwd_dkdv_given_kernel": {"traffic": 2.203e9, "mfma_busy": 0.345, "valu_busy": 0.134, "coexec": 0.047}}}
 
 # algorithmic and executed FLOPs per causal pair and head_dim of a forward and of the backward's two passes
 ALGORITHMIC, EXECUTED = [4.0, 6.0, 4.0], [4.0, 6.0, 8.0]
@@ -52,18 +55,21 @@ def kernel_names(product, d, heads, lengths, fixed):
     g = nat.SbaGeometry()
     nat.check(nat.load().sba_launch_geometry(ctypes.byref(p), ctypes.byref(g)), "sba_launch_geometry")
     passes = "_small" if g.bwd_small_workgroups else ("_wide" if d > 128 else "")
-    return ["fwd_small_kernel" if g.fwd_small_workgroups else "fwd_kernel", f"bwd_dq{passes}_kernel", f"bwd_dkdv{passes}_kernel",
+    given = d > 128 and nat.load().sba_chain_scratch_bytes(ctypes.byref(p)) > 0     # p and dz handed on by the dq pass
+    return ["fwd_small_kernel" if g.fwd_small_workgroups else "fwd_kernel", f"bwd_dq{passes}_kernel", f"bwd_dkdv{'_given' if given else passes}_kernel",
             "bwd_short_kernel" if g.bwd_short_workgroups else "bwd_chain_kernel"]
 
 
 def kernel_figures(m):
     """[(name, ms, algorithmic, executed, tensors moved)] of a measured workload's kernels.  A backward in one kernel has the event
-    pair of the dk/dv pass, and no dq pass is recorded; that of short documents forms the scores twice."""
+    pair of the dk/dv pass, and no dq pass is recorded; that of short documents forms the scores twice.  So do two passes, but where the first hands
+    p and dz on."""
     names = m["kernels"]
     if m["backward"] and m["kern_ms"][1] == 0.0:
         return [(names[0], m["kern_ms"][0], 4.0, 4.0, 4.0),
                 (names[3], m["kern_ms"][2], 10.0, 14.0 if names[3] == "bwd_short_kernel" else 10.0, 7.0)]
-    return [(n, m["kern_ms"][i], ALGORITHMIC[i], EXECUTED[i], [4.0, 5.0, 6.0][i]) for i, n in enumerate(names[:3])]
+    return [(n, m["kern_ms"][i], ALGORITHMIC[i], ALGORITHMIC[i] if "given" in n else EXECUTED[i], [4.0, 5.0, 6.0][i])
+            for i, n in enumerate(names[:3])]
 
 
 def workload(name):
