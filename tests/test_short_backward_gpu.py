@@ -1,5 +1,6 @@
 """Many short documents take one kernel for the whole backward (bwd_short_kernel; above head_dim 64 those of up to 64 tokens): lengths on either side of its blocks of 32
 and of its teams (64, 128, 256 tokens), classes that do not fill a workgroup, in every form, against the oracle and the general two passes."""
+import ctypes
 import random
 
 import pytest
@@ -30,6 +31,19 @@ def test_against_the_oracle(d, lengths, ac, fused):
     ref = oracle_varlen(q, k, v, do, lengths, ac, drem=drem)
     for name, g, r in zip(("o", "rem", "dq", "dk", "dv"), _run(q, k, v, do, lengths, ac, drem=drem), ref):
         assert_close(name, g, r)
+
+
+@pytest.mark.parametrize("d,lengths,taken", [(128, EDGES, True), (96, EDGES, True), (72, [128, 1, 31, 97] * 7, True), (128, [200] * 3 + [17] * 40, True),
+                                             (128, [128, 60, 33] * 5, False), (96, [200, 100] * 5, False)])
+@pytest.mark.parametrize("ac,fused", [(False, False), (True, False), (False, True)])
+def test_long_documents_among_short_ones_above_head_dim_64(d, lengths, taken, ac, fused):
+    from stickbreaking_attention import _native as nat
+    T, H = sum(lengths), 40000 // sum(lengths) + 1
+    p = nat.SbaProblem(nat.SBA_BF16, d, H, 1, T, len(lengths), max(lengths), nat.FLAG_PRODUCT_SPACE, 1.0, 16)
+    g = nat.SbaGeometry()
+    nat.check(nat.load().sba_launch_geometry(ctypes.byref(p), ctypes.byref(g)), "sba_launch_geometry")
+    assert (g.bwd_short_workgroups > 0) == taken
+    test_against_the_oracle(d, lengths, ac, fused)
 
 
 @pytest.mark.parametrize("dtype", list(_ROUND))
