@@ -492,14 +492,15 @@ bool chain_wide(const sba_problem* p, bool fixed, const Sizes& sz) {
   return 20 * c.squares >= 21 * c.longest * 65536;
 }
 // Whether Q and dO rows stream past an XCD's L2 (4 MiB) instead of staying in it, where they compete with the partial dq on its way from key tile to
-// key tile.  They are better kept (backward, us, streamed / kept: 16 heads of 7 K tokens in six documents of up to 3000 at head_dim 128 239 / 228,
-// 4 x 16 x 2048 270 / 265, 12 heads of 3 K tokens 89 / 87; 32 heads x 16 K tokens in eight documents at 96 1122 / 1095, at 64 935 / 890, at 32 746 / 731)
-// but where the chains an XCD interleaves have two to three times as much of it as the L2 holds (head_dim 128, 512 bytes a
-// token: 32 heads x 16 K tokens 1320 / 1352, 12 x 4 x 4096 696 / 710, 16 heads of 2 x 8192 1715 / 1790; one chain of 16 K tokens per XCD 1744 / 1753).
+// key tile.  They are better kept until the rows an XCD has to do, whatever their documents, are several times what it holds: time streamed over kept, on 420 problems of
+// 8 to 32 heads in documents of 128 to 8192 tokens, at head_dim 128 (512 bytes a row) 1.03 .. 1.08 up to 16 K rows and 0.96 .. 1.0 from 24 K on, at 96 1.03 .. 1.08
+// up to 16 K rows, and of documents of up to 1024 1.0 at 24 K and 0.97 .. 1.0 at 32 K, of longer ones 1.0 .. 1.08 everywhere, at 64 1.0 .. 1.08 up to 32 K.  A document of one tile
+// hands nothing on (0.93 .. 1.0).
 bool chain_streams(const sba_problem* p, bool fixed, const Sizes& sz) {
-  const long long chains = (long long)sz.n_docs * p->heads, at_once = std::min<long long>((chains + CHAIN_QUEUES - 1) / CHAIN_QUEUES, CHAIN_GROUP);
-  const long long typical = (declared_max_doc_len(p, fixed) + sz.rows / sz.n_docs) / 2;
-  return used_width(p->head_dim) == 128 && at_once * typical * 128 * 4 > (10ll << 20);
+  const int width = used_width(p->head_dim);
+  const long long longest = declared_max_doc_len(p, fixed), rows = sz.rows * p->heads / CHAIN_QUEUES;
+  if (width < 96) return false;
+  return longest <= BKV || (width == 128 ? rows > 20 * 1024 : rows > 28 * 1024 && longest + sz.rows / sz.n_docs <= 2048);
 }
 // Where the one-pass form is the faster one (gain over the two passes; measured on 1220 problems of 1 to 32 heads and 512 to 200 K tokens in
 // 1 to 128 documents, declared lengths exact: 1.003 of the faster form's time at head_dim 96 and 128, 1.01 at 64, 1.015 at 32, by the geometric mean).

@@ -956,6 +956,8 @@ template __global__ void bwd_chain_kernel<128, 128, false, 1, true>(const ChainA
 template __global__ void bwd_chain_kernel<128, 128, true, 1, true>(const ChainArgs);
 template __global__ void bwd_chain_kernel<128, 96, false, 1, false>(const ChainArgs);
 template __global__ void bwd_chain_kernel<128, 96, true, 1, false>(const ChainArgs);
+template __global__ void bwd_chain_kernel<128, 96, false, 1, true>(const ChainArgs);
+template __global__ void bwd_chain_kernel<128, 96, true, 1, true>(const ChainArgs);
 
 template __global__ void bwd_chain_kernel<64, 64, false, 1, false>(const ChainArgs);
 template __global__ void bwd_chain_kernel<64, 64, true, 1, false>(const ChainArgs);
@@ -978,7 +980,7 @@ static hipError_t launch_chain_d(const ChainArgs& a, bool ac, int n_q_max, int w
 hipError_t launch_bwd_chain(const ChainArgs& a, bool ac, bool wide, bool stream, int n_q_max, int workgroups, hipStream_t s) {
   if (a.head_dim <= 32) return wide ? launch_chain_d<64, 32, 2>(a, ac, n_q_max, workgroups, s) : launch_chain_d<64, 32, 1>(a, ac, n_q_max, workgroups, s);
   if (a.head_dim <= 64) return wide ? launch_chain_d<64, 64, 2>(a, ac, n_q_max, workgroups, s) : launch_chain_d<64, 64, 1>(a, ac, n_q_max, workgroups, s);
-  if (used_width(a.head_dim) == 96) return launch_chain_d<128, 96, 1>(a, ac, n_q_max, workgroups, s);
+  if (used_width(a.head_dim) == 96) return stream ? launch_chain_d<128, 96, 1, true>(a, ac, n_q_max, workgroups, s) : launch_chain_d<128, 96, 1>(a, ac, n_q_max, workgroups, s);
   return stream ? launch_chain_d<128, 128, 1, true>(a, ac, n_q_max, workgroups, s) : launch_chain_d<128, 128, 1>(a, ac, n_q_max, workgroups, s);
 }
 
