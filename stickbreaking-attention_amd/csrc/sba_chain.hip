@@ -32,9 +32,10 @@
 // Measured (kernel time of the backward with its prep kernel, before and after the shorter lag, the poll in the background and leaner
 // product waves, alternating on one MI355X): 32 heads x 16 K tokens in eight documents, head_dim 128, 1311 -> 1292 us; 12 x 4 x 4096
 // 694 -> 683; 16 x 7 K in six documents, head_dim 96, 240 -> 226; 12 heads of 1500, 900 and 601 tokens, head_dim 64, 80.0 -> 69.8
-// and 128, 95.8 -> 88.   At head_dim 128 it waits: 41 % of the wave
+// and 128, 95.8 -> 88.  (Documents of one or two tiles, where what an item costs before its first step is the time, are 1 to 2 % slower: 32 heads of 64 x 256 at
+// 128 349 -> 354.)  At head_dim 128 it waits: 44 % of the wave
 // cycles on 32 heads x 16 K tokens (22 .. 25 % in the two passes; profiles/c3_sq_counters_pmc.txt), with the matrix pipe busy for
-// 34 %.  Such a launch fetches 4.7 GB from behind the L2s and writes 3.1 GB there, 6.0 TB/s where a plain copy reaches 4.9: of the
+// 36 %.  Such a launch fetches 4.5 GB from behind the L2s and writes 3.1 GB there, 5.8 TB/s where a plain copy reaches 4.9: of the
 // 2.8 GB of partial dq each way, all that is written leaves L2 (eight chains of 2 MiB share 4 MiB).
 //
 // What does not help: waves that are all alike.  Eight of them with 256 registers (steps of 64 queries, two barriers) took 1510 us at

@@ -1,4 +1,4 @@
-"""Many short documents take one kernel for the whole backward (bwd_short_kernel; above head_dim 64 those of up to 64 tokens): lengths on either side of its blocks of 32
+"""Many short documents take one kernel for the whole backward (bwd_short_kernel; above head_dim 64 those of up to 64 tokens, and long ones among many short): lengths on either side of its blocks of 32
 and of its teams (64, 128, 256 tokens), classes that do not fill a workgroup, in every form, against the oracle and the general two passes."""
 import ctypes
 import random
