@@ -253,27 +253,30 @@ bool backward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
   return small_wins(COSTS, 1.05, p, fixed, sz);
 }
 
-// Where bwd_short_kernel (sba_small.hip) is the faster one: short documents, and enough of them for a wave on two of three SIMDs (a wave has 64
-// tokens; dq and dk/dv passes / one-pass form before, us, at head_dim 64: 32 heads of 8 x 256 tokens 44.5 / 31.6, of 32 x 128 49.6 / 35.3, of
-// 128 x 33 75 / 44.3, of 128 x 256 390 / 320, 8 heads of 5000 tokens in documents of 1 .. 256 33.6 / 30.3; left out: 4 heads of 128 x 64 20.1 / 19.9, of
-// 32 x 64 16.6 / 19.0).  Above head_dim 64 a compute unit has room for one workgroup, and only what the one-pass form does not take gains (head_dim 128: 16
-// heads of 128 x 64 115 / 68, 32 of 128 x 33 160 / 106), or what has most documents far shorter than the longest, each of which is a key tile, nearly empty, to the
-// one-pass form: 172 problems of 4 to 32 heads and 2 K to 32 K tokens at head_dim 96 and 128 whose mean is up to 0.45 of the longest 1.40 times as fast by the geometric mean (0.98 .. 2.04; 32 heads
-// x 16 K tokens in documents of 16 .. 256 438 / 406), with the longest up to 128 also up to 0.55 (1.08 .. 1.31).  Beyond it loses where there are many
-// (16 heads of 128 x 128 153 / 164, of 100 x 96 106 / 115, of 64 x 256 191 / 204).
-bool backward_short(const sba_problem* p, bool fixed, const Sizes& sz) {
-  if (backward_form() != 0) return false;
-  if (!(p->flags & SBA_PRODUCT_SPACE) || p->head_dim > 128 || sz.n_docs <= 0 || sz.n_docs > RANK_LIMIT || sz.rows * p->heads < 40000) return false;
-  const long long longest = declared_max_doc_len(p, fixed);
-  if (longest > 32 * SHORT_BLOCKS) return false;
-  return p->head_dim <= 64 || longest <= 64 || 20ll * sz.rows <= (longest <= 128 ? 11 : 9) * longest * sz.n_docs;
-}
 // Workgroups per head: documents of more than 128 tokens one each, the others two or four (each class rounded up).
 int short_parts(const sba_problem* p, bool fixed, const Sizes& sz) {
   const int longest = declared_max_doc_len(p, fixed);
   if (longest <= 64) return (sz.n_docs + 3) / 4;
   const long long alone = longest <= 128 ? 0 : std::min<long long>(sz.n_docs, sz.rows / 129);
   return (int)(alone + (sz.n_docs - alone + 1) / 2 + 1);
+}
+// Where bwd_short_kernel (sba_small.hip) is the faster one: short documents, and enough of them for a wave on two of five SIMDs (a wave has 64
+// tokens; dq and dk/dv passes / one-pass form before, us, at head_dim 64: 32 heads of 8 x 256 tokens 44.5 / 31.6, of 32 x 128 49.6 / 35.3, of
+// 128 x 33 75 / 44.3, of 128 x 256 390 / 320, 8 heads of 5000 tokens in documents of 1 .. 256 33.6 / 30.3).  With 24 K to 40 K rows (tokens x heads), gain over the
+// kernels for few tiles and the one-pass form by kinds of lengths: head_dim 32 1.07 .. 1.66, 64 0.98 .. 1.60, documents of up to 64 tokens at 96 and 128 1.05 .. 1.99; with 16 K 0.87 .. 1.23.
+// Above head_dim 64 a compute unit has room for one workgroup, and of longer documents only what the one-pass form does not take well gains:
+// - most documents far shorter than the longest, each of which is a key tile, nearly empty, to the one-pass form: 172 problems of 4 to 32 heads and 2 K to 32 K tokens at
+//   head_dim 96 and 128 whose mean is up to 0.45 of the longest 1.40 times as fast by the geometric mean (0.98 .. 2.04; 32 heads x 16 K tokens in documents of
+//   16 .. 256 438 / 406), with the longest up to 128 also up to 0.55 (1.08 .. 1.31);
+// - what one round of workgroups does, and 256 key tiles would not: 201 problems of 40 K to 64 K rows at head_dim 72, 96 and 128 1.21 (0.99 .. 1.36).
+// Beyond it loses (head_dim 128: 16 heads of 128 x 128 153 / 164, of 100 x 96 106 / 115, of 64 x 256 191 / 204; 16 heads of 16 x 128 20 % slower).
+bool backward_short(const sba_problem* p, bool fixed, const Sizes& sz) {
+  if (backward_form() != 0) return false;
+  const long long longest = declared_max_doc_len(p, fixed);
+  if (!(p->flags & SBA_PRODUCT_SPACE) || p->head_dim > 128 || sz.n_docs <= 0 || sz.n_docs > RANK_LIMIT || longest > 32 * SHORT_BLOCKS) return false;
+  if (p->head_dim <= 64 || longest <= 64) return sz.rows * p->heads >= 24000;
+  return sz.rows * p->heads >= 40000 &&
+         (20ll * sz.rows <= (longest <= 128 ? 11 : 9) * longest * sz.n_docs || (short_parts(p, fixed, sz) - 1) * (long long)p->heads <= device_cus());
 }
 
 // Whether the query tiles of documents of like length are listed tile-major (see sched_kernel): in launches of up to four rounds of the
