@@ -66,6 +66,8 @@ __host__ __device__ inline int chain_docs_offset(int n_docs) { return (2 * n_doc
 // 16-bit words that p and dz of a 32 x 32 block take per carry-table entry of the block (32 of them), where the wide backward
 // keeps them: see bwd_dq_wide_kernel.
 constexpr int PZ_WORDS = 64;
+// Byte offset of what stands for `entry` of the carry table.  Unsigned: beyond 32 K tokens a document's offsets pass 2 GiB.
+__host__ __device__ constexpr unsigned pz_offset(int entry) { return (unsigned)entry * (2u * PZ_WORDS); }
 
 struct Tile {
   int tok_start;  // first token of the document inside the packed token axis (0 for fixed-length)

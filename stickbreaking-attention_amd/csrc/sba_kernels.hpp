@@ -46,6 +46,7 @@ struct KArgs {
 };
 
 constexpr size_t GIVEN_SCRATCH_MAX = 0xf0000000u;   // bytes of p and dz that are handed on at a time: 32-bit offsets reach them
+static_assert(pz_offset((int)(GIVEN_SCRATCH_MAX / (2 * PZ_WORDS)) - 32) == GIVEN_SCRATCH_MAX - 32 * 2 * PZ_WORDS, "the last block's place");
 
 constexpr int NO_DEAL = 31;    // (no launch has a second round of 2^31 workgroups)
 // Workgroups of the forward that a compute unit holds.

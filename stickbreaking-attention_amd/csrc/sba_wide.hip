@@ -451,9 +451,9 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
   const bool gives = GIVE && qw0 < L;         // (a block of queries behind the document's end has no place)
   __amdgpu_buffer_rsrc_t give_rs;
   if constexpr (GIVE)
-    give_rs = __builtin_amdgcn_make_buffer_rsrc(a.pz + ((int64_t)head * a.pz_entries + t.tab_base) * PZ_WORDS, 0, (unsigned)tab_doc_entries(L) * (2u * PZ_WORDS), 0x00020000);
+    give_rs = __builtin_amdgcn_make_buffer_rsrc(a.pz + ((int64_t)head * a.pz_entries + t.tab_base) * PZ_WORDS, 0, pz_offset(tab_doc_entries(L)), 0x00020000);
   auto give = [&](const el8 (&v)[2], int block, int part) __attribute__((always_inline)) {
-    const unsigned at = (unsigned)(tab_seg32(L, block) + qw0) * (2u * PZ_WORDS) + 2048u * part;
+    const unsigned at = pz_offset(tab_seg32(L, block) + qw0) + 2048u * part;
     int give_at = 16 * lane;
     asm volatile("" : "+v"(give_at));         // (no register for it through the steps)
 #pragma unroll
@@ -741,16 +741,16 @@ __global__ void __launch_bounds__(512, 1) bwd_dkdv_given_kernel(const KArgs a) {
   const int from = 1024 * (w & 1) + 16 * (lane ^ (4 * ((lane >> 5) + 2 * (w & 1))));
   const int place = tab_seg32(L, min((BKV / 32) * t.idx + (w >> 1), (L - 1) / 32)) + q_first;
   const __amdgpu_buffer_rsrc_t pz_rs = __builtin_amdgcn_make_buffer_rsrc(a.pz + ((int64_t)head * a.pz_entries + t.tab_base) * PZ_WORDS, 0,
-                                                                       (unsigned)tab_doc_entries(L) * (2u * PZ_WORDS), 0x00020000);
+                                                                       pz_offset(tab_doc_entries(L)), 0x00020000);
   constexpr int LOADS_PER_TILE = 2 * Copy::NCH + 2;
   auto fetch = [&](int turn, int slot) {
     const int step = nsteps - 1 - turn;
     unsigned short* const T = tiles + slot * SLOT;
     qcopy.issue(qrows, q_first + step * TQ, T);
     gcopy.issue(grows, q_first + step * TQ, T + QTILE);
-    const int soff = __builtin_amdgcn_readfirstlane((place + step * TQ) * (2 * PZ_WORDS));
-    async_copy16<true>(pz_rs, T + 2 * QTILE + 512 * w, from, soff);
-    async_copy16<true>(pz_rs, T + 2 * QTILE + PTILE + 512 * w, from, soff + 2048);
+    const unsigned soff = __builtin_amdgcn_readfirstlane(pz_offset(place + step * TQ));
+    async_copy16<true>(pz_rs, T + 2 * QTILE + 512 * w, from, (int)soff);
+    async_copy16<true>(pz_rs, T + 2 * QTILE + PTILE + 512 * w, from, (int)(soff + 2048));
   };
   fetch(0, 0);
   if (nsteps > 1) fetch(1, 1);

@@ -88,6 +88,25 @@ def test_heads_in_groups(form, fixed):
 
 
 @pytest.mark.gpu
+def test_a_document_whose_places_pass_2_gib(form):
+    """32-bit offsets from a document's first block, beyond what a signed one holds: the newest keys' blocks are the last."""
+    from stickbreaking_attention import _native as nat, sb_attn_varlen
+    T, d = 38000, 136
+    p = problem(head_dim=d, heads=1, tokens=T, n_docs=1, max_doc_len=T, flags=nat.FLAG_PRODUCT_SPACE)
+    assert nat.load().sba_chain_scratch_bytes(ctypes.byref(p)) > 1 << 31
+    gen = torch.Generator(device=DEV).manual_seed(9)
+    x = [torch.randn((1, T, d), generator=gen, device=DEV).to(torch.bfloat16).requires_grad_() for _ in range(3)]
+    do = torch.randn((1, T, d), generator=gen, device=DEV).to(torch.bfloat16)
+    cu = cu_from_lengths([T], device=DEV)
+    run = lambda: torch.autograd.grad(sb_attn_varlen(*x, cu, T, zero_start=False)[0], x, do)
+    got = run()
+    form(1)
+    for name, g, t in zip(("dq", "dk", "dv"), got, run()):
+        for rows in (slice(0, 20000), slice(20000, 34000), slice(34000, T)):
+            assert_close(name, g[:, rows], t[:, rows].float())
+
+
+@pytest.mark.gpu
 def test_a_document_longer_than_declared_gives_nan(monkeypatch):
     """Room for p and dz goes by the declared length: what does not fit is refused by the kernels, and every gradient is NaN."""
     from stickbreaking_attention import _ops, sb_attn_varlen
