@@ -287,7 +287,8 @@ int sba_round_floats(int dtype, int n, const void* const* src, void* const* dst,
  *   problems of few tiles: `fwd_small_workgroups` / `bwd_small_workgroups` per head, four to a slot of the
  *   query-tile list, 0 where the general kernels run;
  *   backward of short documents: `bwd_short_workgroups` per head, 0 where others run; it reads the
- *   ranked documents, four words each from `docs_word` on (up to 4096 documents).
+ *   ranked documents, four words each from `docs_word` on (up to 4096 documents);
+ *   one-pass backward: `bwd_rows_streamed` is 1 where Q and dO rows stream past the L2s instead of staying in them.
  * Offsets and sizes are in int32 words. */
 typedef struct sba_geometry {
   int query_list_tiles, key_list_tiles;
@@ -299,6 +300,7 @@ typedef struct sba_geometry {
   int dkdv_main_workgroups;
   int fwd_small_workgroups, bwd_small_workgroups, bwd_short_workgroups;
   int docs_word;
+  int bwd_rows_streamed;
 } sba_geometry;
 int sba_launch_geometry(const sba_problem* p, sba_geometry* out);
 

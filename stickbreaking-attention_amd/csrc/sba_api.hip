@@ -833,6 +833,7 @@ int sba_launch_geometry(const sba_problem* p, sba_geometry* out) {
   out->bwd_small_workgroups = !is_short && backward_small(p, fixed, sz) ? small_workgroups(sz.n_q_max) : 0;
   out->bwd_short_workgroups = is_short ? short_parts(p, fixed, sz) : 0;
   out->docs_word = SCHED_HDR + TILE_WORDS * (sz.n_q_max + sz.n_kv_max) + chain_docs_offset(sz.n_docs);
+  out->bwd_rows_streamed = sz.n_docs > 0 && p->head_dim <= 128 && chain_streams(p, fixed, sz) ? 1 : 0;
   return 0;
 }
 

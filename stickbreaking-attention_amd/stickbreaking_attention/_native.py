@@ -56,7 +56,8 @@ class SbaGeometry(ctypes.Structure):
                 ("long_tiles_bound", ctypes.c_int), ("tail_tiles_bound", ctypes.c_int),
                 ("dkdv_main_tiles", ctypes.c_int), ("dkdv_tail_tiles", ctypes.c_int),
                 ("dkdv_main_workgroups", ctypes.c_int), ("fwd_small_workgroups", ctypes.c_int),
-                ("bwd_small_workgroups", ctypes.c_int), ("bwd_short_workgroups", ctypes.c_int), ("docs_word", ctypes.c_int)]
+                ("bwd_small_workgroups", ctypes.c_int), ("bwd_short_workgroups", ctypes.c_int), ("docs_word", ctypes.c_int),
+                ("bwd_rows_streamed", ctypes.c_int)]
 
 
 EXPORTS = (

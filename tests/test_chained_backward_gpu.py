@@ -119,56 +119,20 @@ def test_the_choice_between_one_pass_and_two(form, H, d, lengths, declared, chai
 def test_rows_streamed_past_the_l2_give_the_same_bits(form, d, attend_current):
     """The rows are streamed where an XCD has several times the L2 of them to do: 144 heads at once and a few of them alone."""
     from stickbreaking_attention import sb_attn_varlen
+    from tests.helpers import kernels_of
     lengths = [300, 131, 32, 161, 193, 288, 609]
     H, T = 144, sum(lengths)
     q, k, v, do = orc.make_inputs((H, T, d), 5)
     drem = torch.randn((H, T), generator=torch.Generator().manual_seed(5)).to(torch.bfloat16)
     cu = cu_from_lengths(lengths, device=DEV)
     form(2)
+    assert kernels_of(q, lengths).bwd_rows_streamed
     streamed = gradients(sb_attn_varlen, (q, k, v), cu, max(lengths), attend_current, (do, drem))
     for heads in (slice(0, 6), slice(140, 144)):
+        assert not kernels_of(q[heads], lengths).bwd_rows_streamed
         kept = gradients(sb_attn_varlen, (q[heads], k[heads], v[heads]), cu, max(lengths), attend_current, (do[heads], drem[heads]))
         for name, a, b in zip(("dq", "dk", "dv"), kept, streamed):
             assert torch.equal(a, b[heads]), name
-
-
-@pytest.mark.parametrize("H,d,lengths,declared,chained", [
-    (4, 96, [2500] * 3, 2500, True),                    # 12 chains on 8 XCDs, few enough tiles to be held at once
-    (12, 64, [4096], 4096, True),
-    (18, 64, [3000], 3000, True), (12, 64, [4500], 4500, False),      # a third more than the mean on the worst XCD, which does not hold them: up to 4096 keys
-    (16, 64, [6000, 500, 500, 500], 6000, True),        # even chains of any length
-    (2, 128, [9000, 300, 200], 9000, False),            # two long ones, each on an XCD of its own
-    (16, 32, [5000, 4000], 16384, True),                # declared longer than there are rows
-])
-def test_the_choice_between_one_pass_and_two(form, H, d, lengths, declared, chained):
-    from stickbreaking_attention import _native as nat, sb_attn_varlen
-    T = sum(lengths)
-    p = nat.SbaProblem(1, d, H, 1, T, len(lengths), declared, nat.FLAG_PRODUCT_SPACE, d ** -0.5, 0x1000)
-    assert (nat.load().sba_chain_scratch_bytes(ctypes.byref(p)) > 0) == chained
-    gen = torch.Generator(device=DEV).manual_seed(T)
-    x = [torch.randn((H, T, d), generator=gen, device=DEV).to(torch.bfloat16).requires_grad_() for _ in range(3)]
-    do = torch.randn((H, T, d), generator=gen, device=DEV).to(torch.bfloat16)
-    cu = cu_from_lengths(lengths, device=DEV)
-    run = lambda: torch.autograd.grad(sb_attn_varlen(*x, cu, declared, zero_start=False)[0], x, do)
-    got = run()
-    form(1)
-    for name, g, t in zip(("dq", "dk", "dv"), got, run()):
-        assert_close(name, g, t.float())
-
-
-@pytest.mark.parametrize("attend_current", [False, True])
-def test_rows_streamed_past_the_l2_give_the_same_bits(form, attend_current):
-    """At head_dim 128 the rows are streamed where the declared lengths say that the chains under way overfill the L2."""
-    from stickbreaking_attention import sb_attn_varlen
-    lengths = [300, 131, 32, 161, 193, 288, 609]
-    H, T = 6, sum(lengths)
-    tensors = orc.make_inputs((H, T, 128), 5)
-    drem = torch.randn((H, T), generator=torch.Generator().manual_seed(5)).to(torch.bfloat16)
-    cu = cu_from_lengths(lengths, device=DEV)
-    form(2)
-    kept, streamed = (gradients(sb_attn_varlen, tensors[:3], cu, m, attend_current, (tensors[3], drem)) for m in (max(lengths), 16384))
-    for name, a, b in zip(("dq", "dk", "dv"), kept, streamed):
-        assert torch.equal(a, b), name
 
 
 @pytest.mark.parametrize("steps,d", [(2, 128), (2, 64), (3, 64), (2, 32), (3, 32)])
