@@ -55,7 +55,8 @@ def kernel_names(product, d, heads, lengths, fixed):
     g = nat.SbaGeometry()
     nat.check(nat.load().sba_launch_geometry(ctypes.byref(p), ctypes.byref(g)), "sba_launch_geometry")
     passes = "_small" if g.bwd_small_workgroups else ("_wide" if d > 128 else "")
-    given = d > 128 and nat.load().sba_chain_scratch_bytes(ctypes.byref(p)) > 0     # p and dz handed on by the dq pass
+    table = 4 * _ops.workspace_sizes(fixed, len(lengths) if fixed else 1, heads, lengths[0] if fixed else sum(lengths), len(lengths), max(lengths), lengths)[1]
+    given = d > 128 and nat.load().sba_bwd_scratch_bytes(ctypes.byref(p), table) > 0     # p and dz handed on by the dq pass
     return ["fwd_small_kernel" if g.fwd_small_workgroups else "fwd_kernel", f"bwd_dq{passes}_kernel", f"bwd_dkdv{'_given' if given else passes}_kernel",
             "bwd_short_kernel" if g.bwd_short_workgroups else "bwd_chain_kernel"]
 

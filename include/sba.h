@@ -248,12 +248,17 @@ int sba_attn_bwd(const sba_problem* p, const void* schedule, size_t schedule_siz
 /* The backward with every score formed once.  Up to head_dim 128 it is one pass, dq is handed from key tile to key tile
  * through scratch memory (csrc/sba_chain.hip); above, the dq pass hands the weights and the gradients of the logits
  * to the dk/dv pass through scratch memory, 4 bytes per causal pair (csrc/sba_wide.hip), for as many heads at a time as
- * 3.75 GiB hold.  For the problems it is the faster form of, sba_chain_scratch_bytes returns the scratch it needs (16-byte aligned, contents irrelevant, one per
- * concurrent call; never more than 3.75 GiB above head_dim 128) and 0 for every other; a caller then takes
- * sba_varlen_bwd / sba_attn_bwd, which choose among their kernels by size.  Same inputs, outputs, table and refusals; it
- * needs no gradient table, and the results differ from the two-pass form's by rounding.  Problems it
- * cannot take (log-space carry; up to head_dim 128 a device that is not eight XCDs of 32 compute units; above, heads of
- * which too few fit at a time to fill the device) return SBA_E_SHAPE. */
+ * 3.75 GiB hold.  For the problems it is the faster form of, sba_bwd_scratch_bytes returns the scratch it needs (16-byte
+ * aligned, contents irrelevant, one per concurrent call; never more than 3.75 GiB above head_dim 128) and 0 for every other;
+ * a caller then takes sba_varlen_bwd / sba_attn_bwd, which choose among their kernels by size, and may do so at any
+ * time, for instance when that much memory is not to be had.  `table_bytes` is the size of the carry table the
+ * backward will be given: one sized by the documents' lengths (sba_table_bytes_for_lengths) says how many
+ * causal pairs there are.  sba_chain_scratch_bytes(p) is the same for a table of sba_table_bytes(p), the most that the declared
+ * sizes allow.  Same inputs, outputs, table and refusals; the chained entry points need no gradient table, and the results
+ * differ from the two-pass form's by rounding.  Problems they cannot take (log-space carry; up to head_dim 128 a device
+ * that is not eight XCDs of 32 compute units; above, heads of which too few fit at a time to fill the device) return
+ * SBA_E_SHAPE. */
+size_t sba_bwd_scratch_bytes(const sba_problem* p, size_t table_bytes);
 size_t sba_chain_scratch_bytes(const sba_problem* p);
 int sba_varlen_bwd_chained(const sba_problem* p, const void* schedule, size_t schedule_size,
                            const sba_view* q, const sba_view* k, const sba_view* v,
@@ -329,7 +334,7 @@ float sba_last_kernel_ms(int which);
  * take others than the two passes by themselves never see it. */
 void  sba_set_dkdv_workgroups(int n);
 
-/* Test and tuning switch (process-wide): the form of the backward.  0: by size -- sba_chain_scratch_bytes asks for
+/* Test and tuning switch (process-wide): the form of the backward.  0: by size -- sba_bwd_scratch_bytes asks for
  * the one-pass form where that is the fastest, and sba_*_bwd take the kernels for few tiles or for short documents
  * where those are (csrc/sba_small.hip).  1: the general two passes, always.  2: the one-pass form wherever it is
  * possible (head_dim <= 128), 3: the same in steps of 64 queries (head_dim <= 64); sba_*_bwd then run the two passes.  The forms differ by rounding.

@@ -178,6 +178,12 @@ struct Timer {
   }
 };
 
+// Entries per head that a table workspace holds: its last WORK_WORDS words are the work counters of the call's persistent launches.
+int64_t table_stride(const sba_problem* p, size_t table_bytes) {
+  if (table_bytes < WORK_WORDS * sizeof(unsigned)) return 0;
+  return (int64_t)((table_bytes - WORK_WORDS * sizeof(unsigned)) / sizeof(float) / (size_t)p->heads) & ~(int64_t)31;   // heads start on 128-byte lines
+}
+
 // `table_bytes`: size of EACH carry table handed in (ignored when none is).
 int fill_common(const sba_problem* p, bool fixed, const Sizes& sz, const void* schedule, size_t sched_bytes,
                 bool with_table, size_t table_bytes, KArgs* a) {
@@ -186,10 +192,8 @@ int fill_common(const sba_problem* p, bool fixed, const Sizes& sz, const void* s
   if (sched_bytes < schedule_bytes(sz)) return SBA_E_WORKSPACE;
   a->tab_stride = -1;
   if (with_table) {
-    // (the last WORK_WORDS words of a table workspace are the work counters of the call's persistent launches)
     if (table_bytes < WORK_WORDS * sizeof(unsigned)) return SBA_E_WORKSPACE;
-    table_bytes -= WORK_WORDS * sizeof(unsigned);
-    a->tab_stride = (int64_t)(table_bytes / sizeof(float) / (size_t)p->heads) & ~(int64_t)31;   // heads start on 128-byte lines
+    a->tab_stride = table_stride(p, table_bytes);
     // fixed-length needs are known here; packed documents are checked on the device against
     // what the scheduler found (kernels refuse to run, outputs are filled with NaN)
     if (fixed && a->tab_stride < table_entries_bound(p, true)) return SBA_E_WORKSPACE;
@@ -413,36 +417,56 @@ ChainScratch chain_scratch(const sba_problem* p, const Sizes& sz) {
   return c;
 }
 
+// What a problem's chains look like from the host: one document of the longest declared length, the others alike.
+struct Chains { long long number, longest, other, squares, per_xcd, long_per_xcd; };   // squares: of a chain's length, over all of them
+Chains chains_of(const sba_problem* p, bool fixed, const Sizes& sz) {
+  Chains c;
+  c.number = (long long)sz.n_docs * p->heads;
+  c.longest = std::min<long long>(declared_max_doc_len(p, fixed), sz.rows);
+  c.other = sz.n_docs > 1 ? (sz.rows - c.longest) / (sz.n_docs - 1) : 0;
+  c.squares = p->heads * (c.longest * c.longest + (sz.n_docs - 1) * c.other * c.other);
+  c.per_xcd = (c.number + CHAIN_QUEUES - 1) / CHAIN_QUEUES;          // (dealt out longest first)
+  c.long_per_xcd = (p->heads + CHAIN_QUEUES - 1) / CHAIN_QUEUES;
+  return c;
+}
+
 // ---- the two passes of head_dim 129 .. 256 with p and dz handed on (sba_wide.hip) -----------------------
 // The dq pass stores p and dz, 4 bytes per causal pair, and the dk/dv pass multiplies them instead of forming both again.  It is the faster
 // form of 99 problems of 2 to 16 heads and 256 to 8192 tokens in 1 to 60 documents at head_dim 136, 160 and 256 (1.12 by the geometric mean, 0.98 ..
 // 1.39) and of the larger ones (16 heads x 16 K tokens in eight documents at 256: 1515 -> 1180 us, 12 x 4 x 4096 1520 -> 1203).
 // Heads are independent: where the room (32 times a carry table, 32 bytes more for every query and 32 keys) does not hold them all, equal groups
-// of them are taken one after the other in the same place (head_dim 256, us, scores formed twice / in groups: 16 heads of 2 x 8192 3826 / 2960, 32 of 16 x 2048
-// 4527 / 3690, 16 of 8 x 4096 3948 / 3342, 5 of 2 x 16384 4823 / 3741).  A group has to fill the chip by itself, its launches ending with
-// the most expensive of its tiles: the line is at three quarters as many of its blocks per compute unit as that tile has (3 heads of 20000, 0.92 of them, 4241 / 3236;
-// 2 of 24576, 0.75, 4035 / 3604; 1 of 32768, 0.5, 7045 / 8998).
-size_t given_head(const sba_problem* p, bool fixed) { return (size_t)table_entries_bound(p, fixed) * (2 * PZ_WORDS); }
-int given_group(const sba_problem* p, bool fixed) {
-  const long long room = (long long)(GIVEN_SCRATCH_MAX / std::max<size_t>(given_head(p, fixed), 1));
-  if (room >= p->heads) return p->heads;
-  if (room == 0) return 0;
-  const int groups = (int)((p->heads + room - 1) / room), each = (p->heads + groups - 1) / groups;
-  const long long cus = device_cus() > 0 ? device_cus() : 256;
-  return each * table_entries_bound(p, fixed) >= 3 * cus * declared_max_doc_len(p, fixed) ? each : 0;
+// of them are taken one after the other in the same place (head_dim 256, us, scores formed twice / in groups: 16 heads of 2 x 8192
+// 3826 / 2960, 32 of 16 x 2048 4527 / 3690, 16 of 8 x 4096 3948 / 3342, 5 of 2 x 16384 4823 / 3741).  A group has to fill the chip by
+// itself, its launches ending with the most expensive of its tiles: the line is at three quarters as many of its blocks per compute
+// unit as that tile has (3 heads of 20000, 0.92 of them, 4241 / 3236; 2 of 24576, 0.75, 4035 / 3604; 1 of 32768, 0.5, 7045 / 8998).
+// How many blocks there are is what the carry table holds, if it was sized by the documents' lengths.  A table of the most that the
+// declared sizes allow says nothing about them: the room goes by that, the line by the least they allow (16 heads of one document of 16384
+// and 96 of 512 9280 us with scores formed twice, 7276 in groups of six by the lengths; the most leaves room for one head at a time, 17740).
+struct Given { int group; long long entries; size_t bytes; };   // heads at a time (0: not in this form), table entries of each, room for all
+Given given(const sba_problem* p, bool fixed, const Sizes& sz, size_t table_bytes) {
+  const long long most = table_entries_bound(p, fixed), held = table_bytes ? (long long)table_stride(p, table_bytes) : most;
+  Given g = {0, std::min(most, held), 0};
+  if (!(p->flags & SBA_PRODUCT_SPACE) || p->head_dim <= 128 || sz.n_docs <= 0) return g;
+  const size_t each = (size_t)g.entries * (2 * PZ_WORDS);
+  const long long room = (long long)(GIVEN_SCRATCH_MAX / std::max<size_t>(each, 1));
+  if (room >= p->heads) {
+    g.group = p->heads;
+  } else if (room > 0) {
+    const int groups = (int)((p->heads + room - 1) / room), heads = (p->heads + groups - 1) / groups;
+    const long long cus = device_cus() > 0 ? device_cus() : 256;
+    const long long blocks = held < most ? g.entries : std::min(g.entries, chains_of(p, fixed, sz).squares / p->heads / 64);
+    if (heads * blocks >= 3 * cus * declared_max_doc_len(p, fixed)) g.group = heads;
+  }
+  g.bytes = (size_t)g.group * each;
+  return g;
 }
-size_t given_scratch(const sba_problem* p, bool fixed) { return (size_t)given_group(p, fixed) * given_head(p, fixed); }
-bool given_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
-  return (p->flags & SBA_PRODUCT_SPACE) && p->head_dim > 128 && sz.n_docs > 0 && given_group(p, fixed) > 0;
-}
-bool given_wanted(const sba_problem* p, bool fixed, const Sizes& sz) { return backward_form() != 1 && given_possible(p, fixed, sz); }
 
-int backward_given(const sba_problem* p, bool fixed, const Sizes& sz, KArgs& a, void* scratch, size_t scratch_bytes, hipStream_t s) {
-  const int group = given_group(p, fixed);
+int backward_given(const sba_problem* p, bool fixed, const Sizes& sz, KArgs& a, void* scratch, const Given& g, hipStream_t s) {
+  const int group = g.group;
   a.pz = static_cast<unsigned short*>(scratch);
-  a.pz_entries = (int64_t)(scratch_bytes / (2 * PZ_WORDS) / (size_t)group) & ~(int64_t)31;
+  a.pz_entries = g.entries;
   const BwdBounds bb = backward_bounds(p, fixed, sz);
-  const DkdvGrid g = dkdv_grid(false, bb.n_long_max, bb.n_tail_max, sz.n_kv_max);
+  const DkdvGrid grid = dkdv_grid(false, bb.n_long_max, bb.n_tail_max, sz.n_kv_max);
   const bool ac = (p->flags & SBA_ATTEND_CURRENT) != 0, f16 = p->dtype == SBA_F16, whole = group == p->heads;
   hipError_t he = hipSuccess;
   Timer all(2, s, !whole);                    // (several groups: one figure for everything, like the one-pass form)
@@ -454,7 +478,7 @@ int backward_given(const sba_problem* p, bool fixed, const Sizes& sz, KArgs& a, 
     }
     if (he == hipSuccess) {
       Timer tm(2, s, whole);
-      he = (f16 ? f16::launch_bwd_dkdv_given : bf16::launch_bwd_dkdv_given)(a, g.main_tiles, s);
+      he = (f16 ? f16::launch_bwd_dkdv_given : bf16::launch_bwd_dkdv_given)(a, grid.main_tiles, s);
     }
     for (View* v : {&a.q, &a.k, &a.v, &a.go, &a.grem, &a.dq, &a.dk, &a.dv})
       if (v->ptr != nullptr) v->ptr += 2 * (int64_t)group * v->sh;   // (strides count 16-bit words)
@@ -470,18 +494,6 @@ bool chain_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
   return (p->flags & SBA_PRODUCT_SPACE) && p->head_dim <= 128 && sz.n_docs > 0 && sz.n_docs <= RANK_LIMIT &&
          chains <= (long long)CHAIN_QUEUES * CHAIN_GROUP * CHAIN_MAX_GROUPS &&
          ((long long)declared_max_doc_len(p, fixed) + BM) * chain_width(p->head_dim) * 4 < (1ll << 31) && device_cus() == 256;
-}
-// What a problem's chains look like from the host: one document of the longest declared length, the others alike.
-struct Chains { long long number, longest, other, squares, per_xcd, long_per_xcd; };   // squares: of a chain's length, over all of them
-Chains chains_of(const sba_problem* p, bool fixed, const Sizes& sz) {
-  Chains c;
-  c.number = (long long)sz.n_docs * p->heads;
-  c.longest = std::min<long long>(declared_max_doc_len(p, fixed), sz.rows);
-  c.other = sz.n_docs > 1 ? (sz.rows - c.longest) / (sz.n_docs - 1) : 0;
-  c.squares = p->heads * (c.longest * c.longest + (sz.n_docs - 1) * c.other * c.other);
-  c.per_xcd = (c.number + CHAIN_QUEUES - 1) / CHAIN_QUEUES;          // (dealt out longest first)
-  c.long_per_xcd = (p->heads + CHAIN_QUEUES - 1) / CHAIN_QUEUES;
-  return c;
 }
 // Steps of 64 queries instead of 32 (head_dim <= 64).  They do more per step and CU (4 x 16 x 2048 at head_dim 64: 153 us
 // for 179) but a key tile lags its predecessor by three steps of either size, so as long as that lag is what a problem takes
@@ -550,8 +562,11 @@ int backward_chained(const sba_problem* p, bool fixed, const void* schedule, siz
   std::memset(&c, 0, sizeof(c));
   if ((e = fill_common(p, fixed, sz, schedule, sched_bytes, true, table_bytes, &c))) return e;
   if (p->head_dim > 128) {
-    if (sz.rows > 0 && !given_possible(p, fixed, sz)) return SBA_E_SHAPE;
-    if (scratch_bytes < given_scratch(p, fixed) || (reinterpret_cast<uintptr_t>(scratch) & 15)) return SBA_E_WORKSPACE;
+    Given g = given(p, fixed, sz, table_bytes);
+    const Given most = given(p, fixed, sz, 0);                 // (what sba_chain_scratch_bytes goes by)
+    if (sz.rows > 0 && g.group == 0 && most.group == 0) return SBA_E_SHAPE;
+    if (g.group == 0 || (scratch_bytes < g.bytes && most.group > 0)) g = most;
+    if (scratch_bytes < g.bytes || (reinterpret_cast<uintptr_t>(scratch) & 15)) return SBA_E_WORKSPACE;
     if ((e = check_arch())) return e;
     if (sz.rows == 0) return 0;
     c.q = to_view(q); c.k = to_view(k); c.v = to_view(v); c.go = to_view(go); c.grem = to_view(grem);
@@ -560,7 +575,7 @@ int backward_chained(const sba_problem* p, bool fixed, const void* schedule, siz
     c.max_doc_len = declared_max_doc_len(p, fixed);
     c.clear_spare = fixed ? 0 : 1;
     c.nan_pair = p->dtype == SBA_F16 && !c.out_f32 ? 0x7e007e00u : 0x7fc07fc0u;
-    return backward_given(p, fixed, sz, c, scratch, scratch_bytes, reinterpret_cast<hipStream_t>(stream));
+    return backward_given(p, fixed, sz, c, scratch, g, reinterpret_cast<hipStream_t>(stream));
   }
   const ChainScratch at = chain_scratch(p, sz);
   if (scratch_bytes < at.total || (reinterpret_cast<uintptr_t>(scratch) & 15)) return SBA_E_WORKSPACE;
@@ -744,13 +759,14 @@ int sba_attn_bwd(const sba_problem* p, const void* schedule, size_t schedule_siz
                   dq, dk, dv, stream);
 }
 
-size_t sba_chain_scratch_bytes(const sba_problem* p) {
+size_t sba_bwd_scratch_bytes(const sba_problem* p, size_t table_bytes) {
   Sizes sz;
   const bool fixed = p != nullptr && (p->flags & SBA_FIXED_LENGTH) != 0;
   if (check_problem(p, fixed, &sz)) return 0;
-  if (given_wanted(p, fixed, sz)) return given_scratch(p, fixed);
+  if (p->head_dim > 128) return backward_form() == 1 ? 0 : given(p, fixed, sz, table_bytes).bytes;
   return chain_wanted(p, fixed, sz) ? chain_scratch(p, sz).total : 0;
 }
+size_t sba_chain_scratch_bytes(const sba_problem* p) { return sba_bwd_scratch_bytes(p, 0); }
 
 int sba_varlen_bwd_chained(const sba_problem* p, const void* schedule, size_t schedule_size, const sba_view* q,
                            const sba_view* k, const sba_view* v, const sba_view* grad_o, const sba_view* grad_rem,

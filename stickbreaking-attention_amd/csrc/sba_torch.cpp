@@ -240,7 +240,7 @@ struct Attention : public torch::autograd::Function<Attention> {
     if (f32) p.flags |= SBA_F32_OUT;
     const sba_view vq = view(qp, c.fixed), vk = view(kp, c.fixed), vv = view(vp, c.fixed), vg = view(go, c.fixed), vr = view(gr, c.fixed);
     const sba_view wq = view(dq, c.fixed), wk = view(dk, c.fixed), wv = view(dv, c.fixed);
-    const size_t chain_bytes = sba_chain_scratch_bytes(&p);   // 0: the two-pass form
+    const size_t chain_bytes = sba_bwd_scratch_bytes(&p, (size_t)table.numel() * 4);   // 0: the two-pass form
     const int64_t scratch_floats = chain_bytes ? (int64_t)(chain_bytes / 4) : table.numel();
     auto launch = [&](const Tensor& scratch) {
       if (chain_bytes) {

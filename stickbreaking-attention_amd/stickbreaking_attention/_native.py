@@ -65,7 +65,7 @@ EXPORTS = (
     "sba_build_schedule",
     "sba_varlen_fwd", "sba_varlen_bwd", "sba_attn_fwd", "sba_attn_bwd", "sba_set_timing", "sba_set_dkdv_workgroups",
     "sba_last_kernel_ms", "sba_varlen_fwd_weights", "sba_attn_fwd_weights", "sba_varlen_fwd_static",
-    "sba_launch_geometry", "sba_chain_scratch_bytes", "sba_varlen_bwd_chained", "sba_attn_bwd_chained", "sba_set_backward_form",
+    "sba_launch_geometry", "sba_bwd_scratch_bytes", "sba_chain_scratch_bytes", "sba_varlen_bwd_chained", "sba_attn_bwd_chained", "sba_set_backward_form",
     "sba_round_floats",
 )
 
@@ -119,6 +119,8 @@ def load():
             f.argtypes = [P, vp, sz, V, V, V, V, V, vp, sz, vp, sz, V, V, V, vp]
         lib.sba_round_floats.restype = ctypes.c_int
         lib.sba_round_floats.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.POINTER(vp), ctypes.POINTER(vp), ctypes.POINTER(ctypes.c_int64), vp]
+        lib.sba_bwd_scratch_bytes.restype = sz
+        lib.sba_bwd_scratch_bytes.argtypes = [P, sz]
         lib.sba_chain_scratch_bytes.restype = sz
         lib.sba_chain_scratch_bytes.argtypes = [P]
         lib.sba_set_backward_form.restype = None

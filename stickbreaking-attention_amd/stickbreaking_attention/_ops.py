@@ -314,7 +314,7 @@ def _launch_bwd(fixed: bool, do, dr, q, k, v, cu_seqlens, max_doc_len: int, logi
         raise ValueError("the backward needs the carry table of a forward that ran with gradients enabled")
     name = "sba_attn_bwd" if fixed else "sba_varlen_bwd"
     with torch.cuda.device(q.device):
-        chain = lib.sba_chain_scratch_bytes(ctypes.byref(prob))   # 0: the two-pass form
+        chain = lib.sba_bwd_scratch_bytes(ctypes.byref(prob), _nbytes(table))   # 0: the two-pass form
         if chain:
             name += "_chained"
             if _nbytes(gtab) < chain:
@@ -331,10 +331,10 @@ def _launch_bwd(fixed: bool, do, dr, q, k, v, cu_seqlens, max_doc_len: int, logi
     nat.check(code, name)
 
 
-def _runs_chained(q: torch.Tensor, fixed: bool, cu_seqlens, max_doc_len: int, product: bool) -> bool:
+def _runs_chained(q: torch.Tensor, fixed: bool, cu_seqlens, max_doc_len: int, product: bool, table: torch.Tensor) -> bool:
     prob, _keep = _problem(q, fixed, cu_seqlens, max_doc_len, 1.0, False, product, False)
     with torch.cuda.device(q.device):
-        return nat.load().sba_chain_scratch_bytes(ctypes.byref(prob)) > 0
+        return nat.load().sba_bwd_scratch_bytes(ctypes.byref(prob), _nbytes(table)) > 0
 
 
 # The four operators under upstream's names.  Outputs and workspaces are arguments that are
@@ -655,7 +655,7 @@ def run_backward(q, k, v, do, drem, fixed: bool, state, inv_temp: float, attend_
         table = _rebuild_table(qp, kp, vp, fixed, sched, cu, max_len, float(inv_temp), bool(attend_current), product,
                                bool(fused))
     # (the one-pass form needs no gradient table and finds its own scratch memory; a compiled graph cannot know yet)
-    chained = not torch.compiler.is_compiling() and _runs_chained(qp, fixed, cu, max_len, product)
+    chained = not torch.compiler.is_compiling() and _runs_chained(qp, fixed, cu, max_len, product, table)
     gtab = torch.empty(0, dtype=torch.float32, device=q.device) if chained else _grad_table(table)
     if fixed:
         _compileable_bwd(dop, dremp, qp, kp, vp, float(inv_temp), bool(attend_current), product, bool(fused),

@@ -87,6 +87,43 @@ def test_heads_in_groups(form, fixed):
             assert_close(name, *((t.movedim(-3, 0) if fixed else t)[head].float() for t in (g, t)))
 
 
+SKEWED = [16384] + [512] * 60      # as many longest documents as fit are three times what there is
+
+
+def test_the_room_goes_by_what_the_table_holds():
+    """A carry table sized by the documents' lengths says how many blocks there are; the most that the declared sizes allow would be one
+    head at a time, a quarter of the chip, and that is not taken."""
+    from stickbreaking_attention import _native as nat, _ops
+    lib = nat.load()
+    def ask(heads, lengths, known):
+        p = problem(head_dim=136, heads=heads, tokens=sum(lengths), n_docs=len(lengths), max_doc_len=max(lengths), flags=nat.FLAG_PRODUCT_SPACE)
+        table = 4 * _ops.workspace_sizes(False, 1, heads, sum(lengths), len(lengths), max(lengths), lengths if known else None)[1]
+        return lib.sba_bwd_scratch_bytes(ctypes.byref(p), table), lib.sba_chain_scratch_bytes(ctypes.byref(p))
+    entries = sum(_ops.table_entries(n) for n in SKEWED)
+    assert ask(8, SKEWED, True) == (4 * 128 * entries, 0)       # two groups of four
+    assert ask(8, SKEWED, False) == (0, 0)
+    assert ask(4, SKEWED, True)[0] == 4 * 128 * entries
+    for lengths in ([2048] * 16, [4096]):                       # all alike: the table is all but the most there can be
+        exact, most = ask(33, lengths, True)
+        assert ask(33, lengths, False) == (most, most) and exact <= most < 1.03 * exact
+
+
+@pytest.mark.gpu
+def test_heads_in_groups_by_what_the_table_holds(form):
+    from stickbreaking_attention import sb_attn_varlen
+    H, T, d = 8, sum(SKEWED), 136
+    gen = torch.Generator(device=DEV).manual_seed(10)
+    draw = lambda *shape: torch.randn(shape, generator=gen, device=DEV).to(torch.bfloat16)
+    x, do = [draw(H, T, d).requires_grad_() for _ in range(3)], draw(H, T, d)
+    cu = cu_from_lengths(SKEWED, device=DEV)
+    run = lambda: torch.autograd.grad(sb_attn_varlen(*x, cu, max(SKEWED), zero_start=False)[0], x, do)
+    got = run()
+    form(1)
+    for name, g, t in zip(("dq", "dk", "dv"), got, run()):
+        for head in (0, 3, 4, 7):
+            assert_close(name, g[head].float(), t[head].float())
+
+
 @pytest.mark.gpu
 def test_a_document_whose_places_pass_2_gib(form):
     """32-bit offsets from a document's first block, beyond what a signed one holds: the newest keys' blocks are the last."""
