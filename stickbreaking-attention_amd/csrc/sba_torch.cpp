@@ -143,7 +143,7 @@ bool writes_f32(const Tensor& like, int64_t d, bool fixed) {
   return like.size(-1) == d && (like.size(fixed ? 2 : 1) + 1024) * like.stride(fixed ? 2 : 1) * 4 < (int64_t(1) << 31);
 }
 
-// The scratch of a backward (gradient table, or the one-pass form's): one grow-only buffer per (device, stream), shared by every layer (the dk/dv pass
+// The scratch of a backward (gradient table, or the one-pass form's; not p and dz of head_dim 129 .. 256): one grow-only buffer per (device, stream), shared by every layer (the dk/dv pass
 // of one backward has read it before the next backward on that stream writes it).  Packed documents change
 // the size with every batch; growth goes to the next eighth of a power of two, and by at least a quarter.
 // The lock is held while a backward's kernels are enqueued: two threads on one stream must not interleave theirs.
@@ -240,7 +240,17 @@ struct Attention : public torch::autograd::Function<Attention> {
     if (f32) p.flags |= SBA_F32_OUT;
     const sba_view vq = view(qp, c.fixed), vk = view(kp, c.fixed), vv = view(vp, c.fixed), vg = view(go, c.fixed), vr = view(gr, c.fixed);
     const sba_view wq = view(dq, c.fixed), wk = view(dk, c.fixed), wv = view(dv, c.fixed);
-    const size_t chain_bytes = sba_bwd_scratch_bytes(&p, (size_t)table.numel() * 4);   // 0: the two-pass form
+    size_t chain_bytes = sba_bwd_scratch_bytes(&p, (size_t)table.numel() * 4);   // 0: the two-pass form
+    // p and dz of head_dim 129 .. 256 are 32 times a gradient table, up to 3.75 GiB: they are asked for and given back by every call, so that
+    // between two of them the memory is the allocator's for anything else, and where it is not to be had the scores are formed twice.
+    Tensor handed_on;
+    if (chain_bytes && p.head_dim > 128) {
+      try {
+        handed_on = at::empty({(int64_t)(chain_bytes / 4)}, table.options());
+      } catch (const c10::OutOfMemoryError&) {
+        chain_bytes = 0;
+      }
+    }
     const int64_t scratch_floats = chain_bytes ? (int64_t)(chain_bytes / 4) : table.numel();
     auto launch = [&](const Tensor& scratch) {
       if (chain_bytes) {
@@ -255,7 +265,9 @@ struct Attention : public torch::autograd::Function<Attention> {
                                                       &wq, &wk, &wv, stream),
             c.fixed ? "sba_attn_bwd" : "sba_varlen_bwd");
     };
-    if (capturing(stream)) {   // a graph's replays must not depend on a buffer that may be replaced
+    if (handed_on.defined()) {
+      launch(handed_on);
+    } else if (capturing(stream)) {   // a graph's replays must not depend on a buffer that may be replaced
       launch(at::empty({scratch_floats}, table.options()));
     } else {
       GradTables& g = grad_tables();

@@ -315,12 +315,20 @@ def _launch_bwd(fixed: bool, do, dr, q, k, v, cu_seqlens, max_doc_len: int, logi
     name = "sba_attn_bwd" if fixed else "sba_varlen_bwd"
     with torch.cuda.device(q.device):
         chain = lib.sba_bwd_scratch_bytes(ctypes.byref(prob), _nbytes(table))   # 0: the two-pass form
+        if chain and q.shape[-1] > 128:
+            # up to 3.75 GiB: asked for and given back by every call; where they are not to be had, the other form
+            try:
+                gtab = torch.empty((chain + 3) // 4, dtype=torch.float32, device=q.device)
+            except torch.OutOfMemoryError:
+                chain = 0
         if chain:
             name += "_chained"
             if _nbytes(gtab) < chain:
                 gtab = _scratch_table((chain + 3) // 4, q.device, "grad")
             work = (_nbytes(table), gtab.data_ptr(), _nbytes(gtab))
         else:
+            if gtab.numel() == 0:       # (the caller expected the form that needs none)
+                gtab = _grad_table(table)
             work = (gtab.data_ptr(), min(_nbytes(table), _nbytes(gtab)))
         code = getattr(lib, name)(ctypes.byref(prob), sched.data_ptr(), _nbytes(sched),
                                   ctypes.byref(nat.view4(q, fixed)), ctypes.byref(nat.view4(k, fixed)),

@@ -125,6 +125,43 @@ def test_heads_in_groups_by_what_the_table_holds(form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+def test_the_room_is_given_back_and_done_without(form, monkeypatch, native):
+    """p and dz take 1.1 GiB here.  The memory is the allocator's again after the call, and where it is not to be had the
+    gradients are those of the passes that form the scores twice, bit for bit."""
+    from stickbreaking_attention import _ops, sb_attn_varlen
+    if not native:
+        monkeypatch.setattr(_ops, "VALIDATE", True)      # (takes the launchers in Python)
+    _ops.release_workspaces()
+    torch.cuda.empty_cache()        # (nothing of what follows lies in a large block that an earlier test left)
+    H, T, d = 16, 8192, 136
+    gen = torch.Generator(device=DEV).manual_seed(11)
+    draw = lambda *shape: torch.randn(shape, generator=gen, device=DEV).to(torch.bfloat16)
+    x, do = [draw(H, T, d).requires_grad_() for _ in range(3)], draw(H, T, d)
+    cu = cu_from_lengths([4096, 4096], device=DEV)
+    run = lambda: torch.autograd.grad(sb_attn_varlen(*x, cu, 4096, zero_start=False)[0], x, do)
+    form(1)
+    twice = run()
+    form(0)
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    once = run()
+    assert torch.cuda.max_memory_allocated() - before > 1 << 30
+    assert torch.cuda.memory_allocated() - before < 1 << 28         # the gradients themselves
+    assert not all(torch.equal(a, b) for a, b in zip(once, twice))
+    del once
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    device = torch.cuda.get_device_properties(DEV)
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 29)) / device.total_memory)
+        for a, b in zip(run(), twice):
+            assert torch.equal(a, b)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+@pytest.mark.gpu
 def test_a_document_whose_places_pass_2_gib(form):
     """32-bit offsets from a document's first block, beyond what a signed one holds: the newest keys' blocks are the last."""
     from stickbreaking_attention import _native as nat, sb_attn_varlen
