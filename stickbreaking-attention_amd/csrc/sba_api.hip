@@ -533,9 +533,13 @@ bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
   // have to come out even, the more the longer the chains are: one that has half as much again to do as their mean is made up for by chains of up to
   // 4096 keys (12 heads of 4096 1.05), a third more is too much for longer ones (12 heads of 16384 0.91; two heads of 20000 next to short documents
   // 0.55).  Even ones gain at any length (8 heads of 8192 1.12, of 16384 and 8192 1.3, of 8192, 4096 and 2048 1.23 .. 1.38).
+  // Of many chains the estimate takes all but the longest for alike, and puts the longest with as many others as any: they do come out even by their number,
+  // with a tenth of the last round idle at most and, beyond 4096 keys, none longer than its share of the whole (2 heads of 2796 and 118 x 322 at
+  // head_dim 96 1.28; 9 of 4881 and twelve shorter ones 1.23; seven such problems of 1600 drawn ones 1.10 .. 1.28).
   if (std::max(c.long_per_xcd * c.longest, c.per_xcd * mean) > 64 * BKV) {
     const long long most = c.long_per_xcd * c.longest * c.longest + (c.per_xcd - c.long_per_xcd) * c.other * c.other;
-    if (10 * CHAIN_QUEUES * most > (longest <= 32 * BKV ? 15 : 13) * c.squares) return false;
+    const bool even = 10 * c.number >= 9 * CHAIN_QUEUES * c.per_xcd && (longest <= 32 * BKV || c.number * mean * mean >= (CHAIN_QUEUES + 4) * longest * longest);
+    if (!even && 10 * CHAIN_QUEUES * most > (longest <= 32 * BKV ? 15 : 13) * c.squares) return false;
   }
   // Wide heads gain from there on (1.03 .. 1.38; 0.96 where every document ends in a nearly empty tile).  For narrow ones what
   // an item costs before its first step weighs more: with several items per CU only documents of some length gain
