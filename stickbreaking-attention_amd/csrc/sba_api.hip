@@ -418,7 +418,7 @@ ChainScratch chain_scratch(const sba_problem* p, const Sizes& sz) {
 }
 
 // What a problem's chains look like from the host: one document of the longest declared length, the others alike.
-struct Chains { long long number, longest, other, squares, per_xcd, long_per_xcd; };   // squares: of a chain's length, over all of them
+struct Chains { long long number, longest, other, squares, per_xcd, long_per_xcd, most; };   // squares: of a chain's length, over all of them; most: over those of one XCD
 Chains chains_of(const sba_problem* p, bool fixed, const Sizes& sz) {
   Chains c;
   c.number = (long long)sz.n_docs * p->heads;
@@ -427,6 +427,7 @@ Chains chains_of(const sba_problem* p, bool fixed, const Sizes& sz) {
   c.squares = p->heads * (c.longest * c.longest + (sz.n_docs - 1) * c.other * c.other);
   c.per_xcd = (c.number + CHAIN_QUEUES - 1) / CHAIN_QUEUES;          // (dealt out longest first)
   c.long_per_xcd = (p->heads + CHAIN_QUEUES - 1) / CHAIN_QUEUES;
+  c.most = c.long_per_xcd * c.longest * c.longest + (c.per_xcd - c.long_per_xcd) * c.other * c.other;
   return c;
 }
 
@@ -499,12 +500,13 @@ bool chain_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
 // for 179) but a key tile lags its predecessor by three steps of either size, so as long as that lag is what a problem takes
 // (8 heads of 8192 keys: 430 us for 372) the small ones are the better ones.  The line: the work of a CU in steps, squares
 // / (2 x 64 x 128 x 256 CUs), against the steps of the longest document and a twentieth more (32 heads of 7 K tokens in six documents of up to
-// 3000 264 us for 298, 12 x 3 x 2500 161 for 175, 4 x 2 x 8192 428 for 371).
+// 3000 264 us for 298, 12 x 3 x 2500 161 for 175, 4 x 2 x 8192 428 for 371).  Up to 4096 keys, where the XCDs need not come out even (see
+// chain_wanted), it is the work of a CU of the busiest one (20 heads of 3000 at head_dim 32 142 us for 152, 26 of 2200 114 for 120).
 bool chain_wide(const sba_problem* p, bool fixed, const Sizes& sz) {
   const int form = backward_form();
   if (form == 2 || form == 3) return form == 3;
   const Chains c = chains_of(p, fixed, sz);
-  return 20 * c.squares >= 21 * c.longest * 65536;
+  return 20 * (c.longest <= 32 * BKV ? CHAIN_QUEUES * c.most : c.squares) >= 21 * c.longest * 65536;
 }
 // Whether Q and dO rows stream past an XCD's L2 (4 MiB) instead of staying in it, where they compete with the partial dq on its way from key tile to
 // key tile.  They are better kept until the rows an XCD has to do, whatever their documents, are several times what it holds: time streamed over kept, on 420 problems of
@@ -532,14 +534,13 @@ bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
   // the chains fall on the XCDs does not matter (1.1 .. 1.4, one chain alone included; 3 heads of 2 documents of 2500 at head_dim 128 1.21).  Beyond, the XCDs
   // have to come out even, the more the longer the chains are: one that has half as much again to do as their mean is made up for by chains of up to
   // 4096 keys (12 heads of 4096 1.05), a third more is too much for longer ones (12 heads of 16384 0.91; two heads of 20000 next to short documents
-  // 0.55).  Even ones gain at any length (8 heads of 8192 1.12, of 16384 and 8192 1.3, of 8192, 4096 and 2048 1.23 .. 1.38).
+  // 0.55) and at head_dim 32 (18 heads of 3000 0.95, of 4096 1.01).  Even ones gain at any length (8 heads of 8192 1.12, of 16384 and 8192 1.3, of 8192, 4096 and 2048 1.23 .. 1.38).
   // Of many chains the estimate takes all but the longest for alike, and puts the longest with as many others as any: they do come out even by their number,
   // with a tenth of the last round idle at most and, beyond 4096 keys, none longer than its share of the whole (2 heads of 2796 and 118 x 322 at
   // head_dim 96 1.28; 9 of 4881 and twelve shorter ones 1.23; seven such problems of 1600 drawn ones 1.10 .. 1.28).
   if (std::max(c.long_per_xcd * c.longest, c.per_xcd * mean) > 64 * BKV) {
-    const long long most = c.long_per_xcd * c.longest * c.longest + (c.per_xcd - c.long_per_xcd) * c.other * c.other;
     const bool even = 10 * c.number >= 9 * CHAIN_QUEUES * c.per_xcd && (longest <= 32 * BKV || c.number * mean * mean >= (CHAIN_QUEUES + 4) * longest * longest);
-    if (!even && 10 * CHAIN_QUEUES * most > (longest <= 32 * BKV ? 15 : 13) * c.squares) return false;
+    if (!even && 10 * CHAIN_QUEUES * c.most > (longest <= 32 * BKV && p->head_dim > 32 ? 15 : 13) * c.squares) return false;
   }
   // Wide heads gain from there on (1.03 .. 1.38; 0.96 where every document ends in a nearly empty tile).  For narrow ones what
   // an item costs before its first step weighs more: with several items per CU only documents of some length gain

@@ -97,6 +97,7 @@ def test_the_same_bits_from_run_to_run(form, steps, d):
     (16, 64, [6000, 500, 500, 500], 6000, True),        # even chains of any length
     (2, 128, [9000, 300, 200], 9000, False),            # two long ones, each on an XCD of its own
     (16, 32, [5000, 4000], 16384, True),                # declared longer than there are rows
+    (18, 32, [3000], 3000, False), (20, 32, [3000], 3000, True),      # at head_dim 32 that is too much
     (2, 96, [2796] + [322] * 118, 2796, True),          # many chains come out even by their number
     (9, 96, [4881, 4881, 3341, 3186, 2728, 2219, 187, 100, 100, 100, 100, 60, 40], 4881, True),
     (2, 64, [20000] + [200] * 30, 20000, False),        # but not next to one longer than its share
