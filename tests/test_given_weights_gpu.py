@@ -216,3 +216,62 @@ def test_scratch(form):
         assert call(other, 0x1000, 1 << 40) == -4
     form(1)
     assert lib.sba_chain_scratch_bytes(ctypes.byref(p)) == 0
+
+
+@pytest.mark.gpu
+def test_replays_from_a_hip_graph():
+    """The room is the graph's own; replays with the program's own work on the same memory sizes in between."""
+    from stickbreaking_attention import _ops
+    H, T, d = 3, sum(EDGES), 160
+    cu = cu_from_lengths(EDGES, device=DEV)
+
+    def launch(q, k, v, do):
+        o, rem, state = _ops.run_forward(q, k, v, False, cu, max(EDGES), d ** -0.5, False, need_table=True)
+        return (o, rem) + _ops.run_backward(q, k, v, do, None, False, state, d ** -0.5, False)
+
+    inputs = lambda seed: [t.to(DEV) for t in orc.make_inputs((H, T, d), seed)]
+    static = inputs(300)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        launch(*static)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = launch(*static)
+    for seed in (301, 302, 303):
+        fresh = inputs(seed)
+        for dst, src in zip(static, fresh):
+            dst.copy_(src)
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = launch(*fresh)
+        torch.cuda.synchronize()
+        for name, a, b in zip(("o", "rem", "dq", "dk", "dv"), captured, eager):
+            assert torch.equal(a, b), f"replay with seed {seed}: {name}"
+
+
+@pytest.mark.gpu
+def test_rows_that_are_not_finite_stay_where_they_are_seen():
+    """What is not finite in a row reaches the keys before it or the queries behind it, up to the end of a block of 32: the rest of its document
+    and the others keep the bits that they have without it, though a step's copies bring blocks that its queries cannot see."""
+    from stickbreaking_attention import sb_attn_varlen
+    lengths = [70, 300, 33]
+    row, block, behind, end = 70 + 150, 70 + 128, 70 + 160, 70 + 300
+    tensors = orc.make_inputs((2, sum(lengths), 136), 12)
+    cu = cu_from_lengths(lengths, device=DEV)
+    drem = torch.zeros(tensors[0].shape[:-1], dtype=torch.bfloat16)
+    grads = lambda x: gradients(sb_attn_varlen, x[:3], cu, max(lengths), False, (x[3], drem))
+    clean = grads(tensors)
+    for which in range(4):
+        x = [t.clone() for t in tensors]
+        x[which][:, row] = float("inf")
+        for name, got, want in zip(("dq", "dk", "dv"), grads(x), clean):
+            same = lambda a, b: torch.equal(got[:, a:b], want[:, a:b])
+            assert same(0, 70) and same(end, None), (which, name)
+            if which in (0, 3):             # q or do: the keys behind it, and every other query
+                assert same(behind, end), (which, name)
+                assert name != "dq" or same(70, row) and same(row + 1, end), which
+            elif name == "dq":              # k or v: the queries before it
+                assert same(70, block), which
