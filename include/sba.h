@@ -39,7 +39,7 @@
 extern "C" {
 #endif
 
-#define SBA_VERSION 215
+#define SBA_VERSION 216
 
 /* error codes (negative returns) */
 #define SBA_E_NULL      (-1)  /* a required pointer is NULL                         */
@@ -337,9 +337,10 @@ void  sba_set_dkdv_workgroups(int n);
 /* Test and tuning switch (process-wide): the form of the backward.  0: by size -- sba_bwd_scratch_bytes asks for
  * the one-pass form where that is the fastest, and sba_*_bwd take the kernels for few tiles or for short documents
  * where those are (csrc/sba_small.hip).  1: the general two passes, always.  2: the one-pass form wherever it is
- * possible (head_dim <= 128), 3: the same in steps of 64 queries (head_dim <= 64); sba_*_bwd then run the two passes.  The forms differ by rounding.
- * With SBA_FORM_SHORT_WAITS added, a wait of the one-pass form for the key tile before gives up after its
- * first look, as it otherwise does after about a second: what the missing partial sums belong to is NaN.
+ * possible (head_dim <= 128), 3: the same in steps of 64 queries (head_dim <= 64); sba_*_bwd then run the two passes.
+ * The forms differ by rounding.  With SBA_FORM_SHORT_WAITS added, a wait of the one-pass form for the key tile before
+ * gives up after its first look, as it otherwise does after about a second: what the missing partial sums belong to is
+ * NaN.
  * With SBA_FORM_IDLE_XCDS(mask), the XCDs in `mask` (of bits 0 .. 7, not all) count as without a compute unit for
  * the one-pass form, as a CU mask may leave them. */
 #define SBA_FORM_SHORT_WAITS 0x100

@@ -178,7 +178,8 @@ struct Timer {
   }
 };
 
-// Entries per head that a table workspace holds: its last WORK_WORDS words are the work counters of the call's persistent launches.
+// Entries per head that a table workspace holds: its last WORK_WORDS words are the work counters of the call's
+// persistent launches.
 int64_t table_stride(const sba_problem* p, size_t table_bytes) {
   if (table_bytes < WORK_WORDS * sizeof(unsigned)) return 0;
   return (int64_t)((table_bytes - WORK_WORDS * sizeof(unsigned)) / sizeof(float) / (size_t)p->heads) & ~(int64_t)31;   // heads start on 128-byte lines
@@ -215,15 +216,18 @@ int fill_common(const sba_problem* p, bool fixed, const Sizes& sz, const void* s
 }
 
 // Where the kernels for problems that leave most of the chip idle (sba_small.hip) are the faster ones: both times
-// estimated, in us, from what 90 problems of 4 to 32 heads, 128 to 4096 tokens and 1 to 16 documents took at head_dim 32, 64, 128 and 256.
-//   The general kernels take at least `base` and `step` for every 32 tokens of the longest document (more, once workgroups share a compute unit);
-//   the small ones their own `small_base` and the longer of what the longest document's rounds of 128 take one after the other (`round` each)
-//   and of what `at_once` workgroups at a time need: `group` each and `per_round` for every round, of which a workgroup has half
-//   its document's and half a one for the remainder.  (By tokens, documents are about halfway between the mean and the longest.  A last group
-//   that is not full counts half as if it were: 11 heads of 3 x 686 tokens at head_dim 80, 1.4 groups, took 23.5 us for 21.2.  A group of
-//   workgroups for rows behind their document's end takes 2 us: 3 heads of 2212 tokens in 17 documents at head_dim 256 took 23.6 us for 21.6.)
-// `gain` must be gained, and 2 us, with which four times as many workgroups pay at the dispatcher (the forward of 13 prompts of up to 172 tokens: 9.9 us
-// alone with either, 10.6 for 11.3 in a row).
+// estimated, in us, from what 90 problems of 4 to 32 heads, 128 to 4096 tokens and 1 to 16 documents took at head_dim
+// 32, 64, 128 and 256.
+//   The general kernels take at least `base` and `step` for every 32 tokens of the longest document (more, once
+//   workgroups share a compute unit); the small ones their own `small_base` and the longer of what the longest
+//   document's rounds of 128 take one after the other (`round` each) and of what `at_once` workgroups at a time need:
+//   `group` each and `per_round` for every round, of which a workgroup has half its document's and half a one for the
+//   remainder.  (By tokens, documents are about halfway between the mean and the longest.  A last group that is not
+//   full counts half as if it were: 11 heads of 3 x 686 tokens at head_dim 80, 1.4 groups, took 23.5 us for 21.2.  A
+//   group of workgroups for rows behind their document's end takes 2 us: 3 heads of 2212 tokens in 17 documents at
+//   head_dim 256 took 23.6 us for 21.6.)
+// `gain` must be gained, and 2 us, with which four times as many workgroups pay at the dispatcher (the forward of 13
+// prompts of up to 172 tokens: 9.9 us alone with either, 10.6 for 11.3 in a row).
 struct SmallCost { double base, step, small_base, round, group, per_round; int at_once; };
 bool small_wins(const SmallCost* costs, double gain, const sba_problem* p, bool fixed, const Sizes& sz) {
   if (!(p->flags & SBA_PRODUCT_SPACE) || sz.n_docs <= 0) return false;
@@ -236,10 +240,12 @@ bool small_wins(const SmallCost* costs, double gain, const sba_problem* p, bool 
   const double small = c.small_base + 2.0 * spare + std::max(c.round * longest / round, groups * (c.group + c.per_round * (0.5 * typical / round + 0.5)));
   return std::max(gain * small, small + 2.0) < c.base + c.step * longest / 32;
 }
-// Of 164 problems (general / few tiles, us) none of the 44 taken loses and they gain 1.41 by the geometric mean (head_dim 64: 4 heads x 512 14.4 / 9.7, 16 x 4096 80 / 68,
-// 32 x 1024 23.5 / 17.2; head_dim 256, whose line serves 129 on: 4 x 512 28 / 17, 16 x 1024 48 / 34).  Of the 120 left to fwd_kernel eight would gain more than a tenth, up to
-// 1.24 (12 heads x 3001 tokens in 17 documents 20.8 / 17.7, 13 heads of 2 x 1360 30.2 / 24.5): `base` and `step` are those of a document alone.  Most lose (head_dim 64: 16 heads of
-// 4 x 1024 24.8 / 26.9; head_dim 128: 32 x 2048 57 / 73; head_dim 256: 16 x 2048 88 / 95) or gain less than 4 x the workgroups may cost (32 x 2048 at 64 42 / 39).
+// Of 164 problems (general / few tiles, us) none of the 44 taken loses and they gain 1.41 by the geometric mean
+// (head_dim 64: 4 heads x 512 14.4 / 9.7, 16 x 4096 80 / 68, 32 x 1024 23.5 / 17.2; head_dim 256, whose line serves 129
+// on: 4 x 512 28 / 17, 16 x 1024 48 / 34).  Of the 120 left to fwd_kernel eight would gain more than a tenth, up to
+// 1.24 (12 heads x 3001 tokens in 17 documents 20.8 / 17.7, 13 heads of 2 x 1360 30.2 / 24.5): `base` and `step` are
+// those of a document alone.  Most lose (head_dim 64: 16 heads of 4 x 1024 24.8 / 26.9; head_dim 128: 32 x 2048 57 /
+// 73; head_dim 256: 16 x 2048 88 / 95) or gain less than 4 x the workgroups may cost (32 x 2048 at 64 42 / 39).
 bool forward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
   if (p->flags & SBA_GENERAL_FORWARD) return false;
   if (p->flags & SBA_FEW_TILES_FORWARD) return (p->flags & SBA_PRODUCT_SPACE) && sz.n_docs > 0;
@@ -247,10 +253,10 @@ bool forward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
                                          {6.5, 0.73, 7.0, 1.19, 4.0, 1.60, 512}, {8.7, 1.22, 10.0, 1.93, 5.0, 2.0, 256}};
   return small_wins(COSTS, 1.1, p, fixed, sz);
 }
-// The backward, both passes, against the one-pass form (head_dim 64: 4 heads x 512 36.2 / 23.5, 16 x 1024 55 / 38, 16 x 2048 91 / 80, left out
-// 16 x 4096 229 / 219, 32 x 4 x 256 28 / 34; head_dim 128: 4 heads x 512 42 / 32, 16 x 512 43 / 33.5, left out 16 x 1024 66 / 66).  Documents of one or two
-// blocks are with the general two passes (head_dim 64: 64 tokens 16.0 / 16.8; 2 heads of 68 documents of 38
-// tokens on average and 95 at most 18.5 / 23.9).
+// The backward, both passes, against the one-pass form (head_dim 64: 4 heads x 512 36.2 / 23.5, 16 x 1024 55 / 38, 16 x
+// 2048 91 / 80, left out 16 x 4096 229 / 219, 32 x 4 x 256 28 / 34; head_dim 128: 4 heads x 512 42 / 32, 16 x 512 43 /
+// 33.5, left out 16 x 1024 66 / 66).  Documents of one or two blocks are with the general two passes (head_dim 64: 64
+// tokens 16.0 / 16.8; 2 heads of 68 documents of 38 tokens on average and 95 at most 18.5 / 23.9).
 bool backward_small(const sba_problem* p, bool fixed, const Sizes& sz) {
   if (backward_form() != 0 || p->head_dim > 128 || declared_max_doc_len(p, fixed) <= 64 || sz.rows <= 64ll * sz.n_docs) return false;
   static constexpr SmallCost COSTS[3] = {{16.0, 1.04, 12.5, 1.9, 3.7, 2.35, 512}, {17.0, 1.15, 14.0, 2.34, 6.0, 2.75, 512}, {19.0, 1.42, 18.5, 3.6, 9.5, 3.6, 256}};
@@ -264,16 +270,21 @@ int short_parts(const sba_problem* p, bool fixed, const Sizes& sz) {
   const long long alone = longest <= 128 ? 0 : std::min<long long>(sz.n_docs, sz.rows / 129);
   return (int)(alone + (sz.n_docs - alone + 1) / 2 + 1);
 }
-// Where bwd_short_kernel (sba_small.hip) is the faster one: short documents, and enough of them for a wave on two of five SIMDs (a wave has 64
-// tokens; dq and dk/dv passes / one-pass form before, us, at head_dim 64: 32 heads of 8 x 256 tokens 44.5 / 31.6, of 32 x 128 49.6 / 35.3, of
-// 128 x 33 75 / 44.3, of 128 x 256 390 / 320, 8 heads of 5000 tokens in documents of 1 .. 256 33.6 / 30.3).  With 24 K to 40 K rows (tokens x heads), gain over the
-// kernels for few tiles and the one-pass form by kinds of lengths: head_dim 32 1.07 .. 1.66, 64 0.98 .. 1.60, documents of up to 64 tokens at 96 and 128 1.05 .. 1.99; with 16 K 0.87 .. 1.23.
-// Above head_dim 64 a compute unit has room for one workgroup, and of longer documents only what the one-pass form does not take well gains:
-// - most documents far shorter than the longest, each of which is a key tile, nearly empty, to the one-pass form: 172 problems of 4 to 32 heads and 2 K to 32 K tokens at
-//   head_dim 96 and 128 whose mean is up to 0.45 of the longest 1.40 times as fast by the geometric mean (0.98 .. 2.04; 32 heads x 16 K tokens in documents of
-//   16 .. 256 438 / 406), with the longest up to 128 also up to 0.55 (1.08 .. 1.31);
-// - what one round of workgroups does, and 256 key tiles would not: 201 problems of 40 K to 64 K rows at head_dim 72, 96 and 128 1.21 (0.99 .. 1.36).
-// Beyond it loses (head_dim 128: 16 heads of 128 x 128 153 / 164, of 100 x 96 106 / 115, of 64 x 256 191 / 204; 16 heads of 16 x 128 20 % slower).
+// Where bwd_short_kernel (sba_small.hip) is the faster one: short documents, and enough of them for a wave on two of
+// five SIMDs (a wave has 64 tokens; dq and dk/dv passes / one-pass form before, us, at head_dim 64: 32 heads of 8 x 256
+// tokens 44.5 / 31.6, of 32 x 128 49.6 / 35.3, of 128 x 33 75 / 44.3, of 128 x 256 390 / 320, 8 heads of 5000 tokens in
+// documents of 1 .. 256 33.6 / 30.3).  With 24 K to 40 K rows (tokens x heads), gain over the kernels for few tiles and
+// the one-pass form by kinds of lengths: head_dim 32 1.07 .. 1.66, 64 0.98 .. 1.60, documents of up to 64 tokens at 96
+// and 128 1.05 .. 1.99; with 16 K 0.87 .. 1.23.  Above head_dim 64 a compute unit has room for one workgroup, and of
+// longer documents only what the one-pass form does not take well gains:
+// - most documents far shorter than the longest, each of which is a key tile, nearly empty, to the one-pass form: 172
+//   problems of 4 to 32 heads and 2 K to 32 K tokens at head_dim 96 and 128 whose mean is up to 0.45 of the longest
+//   1.40 times as fast by the geometric mean (0.98 .. 2.04; 32 heads x 16 K tokens in documents of 16 .. 256 438 /
+//   406), with the longest up to 128 also up to 0.55 (1.08 .. 1.31);
+// - what one round of workgroups does, and 256 key tiles would not: 201 problems of 40 K to 64 K rows at head_dim 72,
+//   96 and 128 1.21 (0.99 .. 1.36).
+// Beyond it loses (head_dim 128: 16 heads of 128 x 128 153 / 164, of 100 x 96 106 / 115, of 64 x 256 191 / 204; 16
+// heads of 16 x 128 20 % slower).
 bool backward_short(const sba_problem* p, bool fixed, const Sizes& sz) {
   if (backward_form() != 0) return false;
   const long long longest = declared_max_doc_len(p, fixed);
@@ -283,13 +294,16 @@ bool backward_short(const sba_problem* p, bool fixed, const Sizes& sz) {
          (20ll * sz.rows <= (longest <= 128 ? 11 : 9) * longest * sz.n_docs || (short_parts(p, fixed, sz) - 1) * (long long)p->heads <= device_cus());
 }
 
-// Whether the query tiles of documents of like length are listed tile-major (see sched_kernel): in launches of up to four rounds of the
-// chip, and of more the fewer heads there are.  What is gained is the launch's end, where document-major the last document's most expensive tile
-// starts late: the less the more rounds there are.  What it costs is that the tiles of a (document, head) that are under way at a time share its
-// K/V rows in the caches with fewer others, the more heads (and documents) there are.  The line is that of 456 shapes of equal documents (two rounds and more, 1 to 32 heads, 512 to 32768
-// tokens, head_dim 64, 128 and 256, forward and dq pass): 1.067 times as fast as document-major by the geometric mean, tile-major always 1.050.
-// Forward, us, document-major / tile-major, head_dim 128: 12 heads of 4 x 4096 (2 rounds) 249 / 200, 8 of 8 x 4096 (2.7) 305 / 256, 12 of 8 x 4096 (4)
-// 440 / 377, 2 of 16 x 8192 (2.7) 616 / 484; left out 16 heads of 4 x 8192 (5.3) 985 / 1020, 32 of 8 x 2048 (5.3) 291 / 341, 32 of 8 x 4096 (10.7) 1069 / 1410.
+// Whether the query tiles of documents of like length are listed tile-major (see sched_kernel): in launches of up to
+// four rounds of the chip, and of more the fewer heads there are.  What is gained is the launch's end, where
+// document-major the last document's most expensive tile starts late: the less the more rounds there are.  What it
+// costs is that the tiles of a (document, head) that are under way at a time share its K/V rows in the caches with
+// fewer others, the more heads (and documents) there are.  The line is that of 456 shapes of equal documents (two
+// rounds and more, 1 to 32 heads, 512 to 32768 tokens, head_dim 64, 128 and 256, forward and dq pass): 1.067 times as
+// fast as document-major by the geometric mean, tile-major always 1.050.  Forward, us, document-major / tile-major,
+// head_dim 128: 12 heads of 4 x 4096 (2 rounds) 249 / 200, 8 of 8 x 4096 (2.7) 305 / 256, 12 of 8 x 4096 (4) 440 / 377,
+// 2 of 16 x 8192 (2.7) 616 / 484; left out 16 heads of 4 x 8192 (5.3) 985 / 1020, 32 of 8 x 2048 (5.3) 291 / 341, 32 of
+// 8 x 4096 (10.7) 1069 / 1410.
 bool list_in_classes(const sba_problem* p, const Sizes& sz) {
   const int cus = device_cus();
   const long long items = sz.rows / BM * p->heads, round = (long long)fwd_per_cu(p->head_dim) * (cus > 0 ? cus : 256);
@@ -432,17 +446,19 @@ Chains chains_of(const sba_problem* p, bool fixed, const Sizes& sz) {
 }
 
 // ---- the two passes of head_dim 129 .. 256 with p and dz handed on (sba_wide.hip) -----------------------
-// The dq pass stores p and dz, 4 bytes per causal pair, and the dk/dv pass multiplies them instead of forming both again.  It is the faster
-// form of 99 problems of 2 to 16 heads and 256 to 8192 tokens in 1 to 60 documents at head_dim 136, 160 and 256 (1.12 by the geometric mean, 0.98 ..
-// 1.39) and of the larger ones (16 heads x 16 K tokens in eight documents at 256: 1515 -> 1180 us, 12 x 4 x 4096 1520 -> 1203).
-// Heads are independent: where the room (32 times a carry table, 32 bytes more for every query and 32 keys) does not hold them all, equal groups
-// of them are taken one after the other in the same place (head_dim 256, us, scores formed twice / in groups: 16 heads of 2 x 8192
-// 3826 / 2960, 32 of 16 x 2048 4527 / 3690, 16 of 8 x 4096 3948 / 3342, 5 of 2 x 16384 4823 / 3741).  A group has to fill the chip by
-// itself, its launches ending with the most expensive of its tiles: the line is at three quarters as many of its blocks per compute
-// unit as that tile has (3 heads of 20000, 0.92 of them, 4241 / 3236; 2 of 24576, 0.75, 4035 / 3604; 1 of 32768, 0.5, 7045 / 8998).
-// How many blocks there are is what the carry table holds, if it was sized by the documents' lengths.  A table of the most that the
-// declared sizes allow says nothing about them: the room goes by that, the line by the least they allow (16 heads of one document of 16384
-// and 96 of 512 9280 us with scores formed twice, 7276 in groups of six by the lengths; the most leaves room for one head at a time, 17740).
+// The dq pass stores p and dz, 4 bytes per causal pair, and the dk/dv pass multiplies them instead of forming both
+// again.  It is the faster form of 99 problems of 2 to 16 heads and 256 to 8192 tokens in 1 to 60 documents at head_dim
+// 136, 160 and 256 (1.12 by the geometric mean, 0.98 ..  1.39) and of the larger ones (16 heads x 16 K tokens in eight
+// documents at 256: 1515 -> 1180 us, 12 x 4 x 4096 1520 -> 1203).  Heads are independent: where the room (32 times a
+// carry table, 32 bytes more for every query and 32 keys) does not hold them all, equal groups of them are taken one
+// after the other in the same place (head_dim 256, us, scores formed twice / in groups: 16 heads of 2 x 8192 3826 /
+// 2960, 32 of 16 x 2048 4527 / 3690, 16 of 8 x 4096 3948 / 3342, 5 of 2 x 16384 4823 / 3741).  A group has to fill the
+// chip by itself, its launches ending with the most expensive of its tiles: the line is at three quarters as many of
+// its blocks per compute unit as that tile has (3 heads of 20000, 0.92 of them, 4241 / 3236; 2 of 24576, 0.75, 4035 /
+// 3604; 1 of 32768, 0.5, 7045 / 8998).  How many blocks there are is what the carry table holds, if it was sized by the
+// documents' lengths.  A table of the most that the declared sizes allow says nothing about them: the room goes by
+// that, the line by the least they allow (16 heads of one document of 16384 and 96 of 512 9280 us with scores formed
+// twice, 7276 in groups of six by the lengths; the most leaves room for one head at a time, 17740).
 struct Given { int group; long long entries; size_t bytes; };   // heads at a time (0: not in this form), table entries of each, room for all
 Given given(const sba_problem* p, bool fixed, const Sizes& sz, size_t table_bytes) {
   const long long most = table_entries_bound(p, fixed), held = table_bytes ? (long long)table_stride(p, table_bytes) : most;
@@ -488,39 +504,42 @@ int backward_given(const sba_problem* p, bool fixed, const Sizes& sz, KArgs& a, 
   return (int)he;
 }
 
-// Whether the kernels can take the problem at all: a device of eight XCDs with 32 compute units each, ranked documents, room for the queue's groups in LDS and 32-bit
-// offsets into a document's partial dq.
+// Whether the kernels can take the problem at all: a device of eight XCDs with 32 compute units each, ranked documents,
+// room for the queue's groups in LDS and 32-bit offsets into a document's partial dq.
 bool chain_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
   const long long chains = (long long)sz.n_docs * p->heads;
   return (p->flags & SBA_PRODUCT_SPACE) && p->head_dim <= 128 && sz.n_docs > 0 && sz.n_docs <= RANK_LIMIT &&
          chains <= (long long)CHAIN_QUEUES * CHAIN_GROUP * CHAIN_MAX_GROUPS &&
          ((long long)declared_max_doc_len(p, fixed) + BM) * chain_width(p->head_dim) * 4 < (1ll << 31) && device_cus() == 256;
 }
-// Steps of 64 queries instead of 32 (head_dim <= 64).  They do more per step and CU (4 x 16 x 2048 at head_dim 64: 153 us
-// for 179) but a key tile lags its predecessor by three steps of either size, so as long as that lag is what a problem takes
-// (8 heads of 8192 keys: 430 us for 372) the small ones are the better ones.  The line: the work of a CU in steps, squares
-// / (2 x 64 x 128 x 256 CUs), against the steps of the longest document and a twentieth more (32 heads of 7 K tokens in six documents of up to
-// 3000 264 us for 298, 12 x 3 x 2500 161 for 175, 4 x 2 x 8192 428 for 371).  Up to 4096 keys, where the XCDs need not come out even (see
-// chain_wanted), it is the work of a CU of the busiest one (20 heads of 3000 at head_dim 32 142 us for 152, 26 of 2200 114 for 120).
+// Steps of 64 queries instead of 32 (head_dim <= 64).  They do more per step and CU (4 x 16 x 2048 at head_dim 64: 153
+// us for 179) but a key tile lags its predecessor by three steps of either size, so as long as that lag is what a
+// problem takes (8 heads of 8192 keys: 430 us for 372) the small ones are the better ones.  The line: the work of a CU
+// in steps, squares / (2 x 64 x 128 x 256 CUs), against the steps of the longest document and a twentieth more (32
+// heads of 7 K tokens in six documents of up to 3000 264 us for 298, 12 x 3 x 2500 161 for 175, 4 x 2 x 8192 428 for
+// 371).  Up to 4096 keys, where the XCDs need not come out even (see chain_wanted), it is the work of a CU of the
+// busiest one (20 heads of 3000 at head_dim 32 142 us for 152, 26 of 2200 114 for 120).
 bool chain_wide(const sba_problem* p, bool fixed, const Sizes& sz) {
   const int form = backward_form();
   if (form == 2 || form == 3) return form == 3;
   const Chains c = chains_of(p, fixed, sz);
   return 20 * (c.longest <= 32 * BKV ? CHAIN_QUEUES * c.most : c.squares) >= 21 * c.longest * 65536;
 }
-// Whether Q and dO rows stream past an XCD's L2 (4 MiB) instead of staying in it, where they compete with the partial dq on its way from key tile to
-// key tile.  They are better kept until the rows an XCD has to do, whatever their documents, are several times what it holds: time streamed over kept, on 420 problems of
-// 8 to 32 heads in documents of 128 to 8192 tokens, at head_dim 128 (512 bytes a row) 1.03 .. 1.08 up to 16 K rows and 0.96 .. 1.0 from 24 K on, at 96 1.03 .. 1.08
-// up to 16 K rows, and of documents of up to 1024 1.0 at 24 K and 0.97 .. 1.0 at 32 K, of longer ones 1.0 .. 1.08 everywhere, at 64 1.0 .. 1.08 up to 32 K.  A document of one tile
-// hands nothing on (0.93 .. 1.0).
+// Whether Q and dO rows stream past an XCD's L2 (4 MiB) instead of staying in it, where they compete with the partial
+// dq on its way from key tile to key tile.  They are better kept until the rows an XCD has to do, whatever their
+// documents, are several times what it holds: time streamed over kept, on 420 problems of 8 to 32 heads in documents of
+// 128 to 8192 tokens, at head_dim 128 (512 bytes a row) 1.03 .. 1.08 up to 16 K rows and 0.96 .. 1.0 from 24 K on, at
+// 96 1.03 .. 1.08 up to 16 K rows, and of documents of up to 1024 1.0 at 24 K and 0.97 .. 1.0 at 32 K, of longer ones
+// 1.0 .. 1.08 everywhere, at 64 1.0 .. 1.08 up to 32 K.  A document of one tile hands nothing on (0.93 .. 1.0).
 bool chain_streams(const sba_problem* p, bool fixed, const Sizes& sz) {
   const int width = used_width(p->head_dim);
   const long long longest = declared_max_doc_len(p, fixed), rows = sz.rows * p->heads / CHAIN_QUEUES;
   if (width < 96) return false;
   return longest <= BKV || (width == 128 ? rows > 20 * 1024 : rows > 28 * 1024 && longest + sz.rows / sz.n_docs <= 2048);
 }
-// Where the one-pass form is the faster one (gain over the two passes; measured on 1220 problems of 1 to 32 heads and 512 to 200 K tokens in
-// 1 to 128 documents, declared lengths exact: 1.003 of the faster form's time at head_dim 96 and 128, 1.01 at 64, 1.015 at 32, by the geometric mean).
+// Where the one-pass form is the faster one (gain over the two passes; measured on 1220 problems of 1 to 32 heads and
+// 512 to 200 K tokens in 1 to 128 documents, declared lengths exact: 1.003 of the faster form's time at head_dim 96 and
+// 128, 1.01 at 64, 1.015 at 32, by the geometric mean).
 bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
   const int form = backward_form();
   if (form == 1 || !chain_possible(p, fixed, sz)) return false;
@@ -530,22 +549,26 @@ bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
   const long long items = (long long)sz.n_kv_max * p->heads, mean = sz.rows / sz.n_docs, longest = declared_max_doc_len(p, fixed);
   // a document of one or two steps: nothing to hand on, and one launch more (0.85 .. 1.01)
   if (longest <= 64) return false;
-  // Every chain stays on one XCD.  While an XCD holds nearly all its tiles at once (32 CUs, 4096 keys; twice that for its few last chains) how
-  // the chains fall on the XCDs does not matter (1.1 .. 1.4, one chain alone included; 3 heads of 2 documents of 2500 at head_dim 128 1.21).  Beyond, the XCDs
-  // have to come out even, the more the longer the chains are: one that has half as much again to do as their mean is made up for by chains of up to
-  // 4096 keys (12 heads of 4096 1.05), a third more is too much for longer ones (12 heads of 16384 0.91; two heads of 20000 next to short documents
-  // 0.55) and at head_dim 32 (18 heads of 3000 0.95, of 4096 1.01).  Even ones gain at any length (8 heads of 8192 1.12, of 16384 and 8192 1.3, of 8192, 4096 and 2048 1.23 .. 1.38).
-  // Of many chains the estimate takes all but the longest for alike, and puts the longest with as many others as any: they do come out even by their number,
-  // with a tenth of the last round idle at most and, beyond 4096 keys, none longer than its share of the whole (2 heads of 2796 and 118 x 322 at
-  // head_dim 96 1.28; 9 of 4881 and twelve shorter ones 1.23; seven such problems of 1600 drawn ones 1.10 .. 1.28).
+  // Every chain stays on one XCD.  While an XCD holds nearly all its tiles at once (32 CUs, 4096 keys; twice that for
+  // its few last chains) how the chains fall on the XCDs does not matter (1.1 .. 1.4, one chain alone included; 3 heads
+  // of 2 documents of 2500 at head_dim 128 1.21).  Beyond, the XCDs have to come out even, the more the longer the
+  // chains are: one that has half as much again to do as their mean is made up for by chains of up to 4096 keys (12
+  // heads of 4096 1.05), a third more is too much for longer ones (12 heads of 16384 0.91; two heads of 20000 next to
+  // short documents 0.55) and at head_dim 32 (18 heads of 3000 0.95, of 4096 1.01).  Even ones gain at any length (8
+  // heads of 8192 1.12, of 16384 and 8192 1.3, of 8192, 4096 and 2048 1.23 .. 1.38).  Of many chains the estimate takes
+  // all but the longest for alike, and puts the longest with as many others as any: they do come out even by their
+  // number, with a tenth of the last round idle at most and, beyond 4096 keys, none longer than its share of the whole
+  // (2 heads of 2796 and 118 x 322 at head_dim 96 1.28; 9 of 4881 and twelve shorter ones 1.23; seven such problems of
+  // 1600 drawn ones 1.10 .. 1.28).
   if (std::max(c.long_per_xcd * c.longest, c.per_xcd * mean) > 64 * BKV) {
     const bool even = 10 * c.number >= 9 * CHAIN_QUEUES * c.per_xcd && (longest <= 32 * BKV || c.number * mean * mean >= (CHAIN_QUEUES + 4) * longest * longest);
     if (!even && 10 * CHAIN_QUEUES * c.most > (longest <= 32 * BKV && p->head_dim > 32 ? 15 : 13) * c.squares) return false;
   }
-  // Wide heads gain from there on (1.03 .. 1.38; 0.96 where every document ends in a nearly empty tile).  For narrow ones what
-  // an item costs before its first step weighs more: with several items per CU only documents of some length gain
-  // (head_dim 64: 320 long 0.94 .. 1.02, 512 1.04 .. 1.25, 2048 1.3; head_dim 32: 512 long 0.92 .. 1.06, 768 1.01 .. 1.07,
-  // 2048 1.3 .. 1.5), with about one per CU also shorter ones (head_dim 64: 1.03 .. 1.5; head_dim 32: 200 long 1.0, 384 1.2).
+  // Wide heads gain from there on (1.03 .. 1.38; 0.96 where every document ends in a nearly empty tile).  For narrow
+  // ones what an item costs before its first step weighs more: with several items per CU only documents of some length
+  // gain (head_dim 64: 320 long 0.94 .. 1.02, 512 1.04 .. 1.25, 2048 1.3; head_dim 32: 512 long 0.92 .. 1.06, 768 1.01
+  // .. 1.07, 2048 1.3 .. 1.5), with about one per CU also shorter ones (head_dim 64: 1.03 .. 1.5; head_dim 32: 200 long
+  // 1.0, 384 1.2).
   if (chain_width(p->head_dim) == 128) return true;
   const bool narrow = p->head_dim <= 32;
   return mean >= (narrow ? 5 * BKV : 7 * BKV / 2) || (items <= 512 && longest >= (narrow ? 3 * BKV : BKV)) ||

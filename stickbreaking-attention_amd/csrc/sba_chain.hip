@@ -19,28 +19,31 @@
 // store is visible to the XCD's other CUs when vmcnt says it has been acknowledged; consumers read with sc1,
 // which L1 does not answer.
 //
-// Order and progress.  Queries are walked from the document's end down to the tile's own keys, so that the
-// tiles of a chain start together and end one after the other; the items of a queue are ordered by key tile, so
-// the item an item waits for was drawn before it by a workgroup that is running: waits end.  `flags` holds a number per
-// item: at the start of step t a tile publishes t - 2, which stands for the carried sums of its blocks up to t - 2 (formed two
-// steps ago) and the partial dq of those up to t - 3 (formed by the product waves a step after the sums); both have been
-// acknowledged by then.  Step s asks for the carried sum of block s + 1 and the partial dq of block s, so it needs s + 1: a
-// tile runs three steps behind the one before (it was four while a sum was published no earlier than its block's dq).  What the tile
-// before has published is copied to LDS in the background, a step old when it is looked at; only where that is not
-// enough does a score wave -- the one all others wait for -- stop to ask.
+// Order and progress.  Queries are walked from the document's end down to the tile's own keys, so that the tiles of a
+// chain start together and end one after the other; the items of a queue are ordered by key tile, so the item an item
+// waits for was drawn before it by a workgroup that is running: waits end.  `flags` holds a number per item: at the
+// start of step t a tile publishes t - 2, which stands for the carried sums of its blocks up to t - 2 (formed two steps
+// ago) and the partial dq of those up to t - 3 (formed by the product waves a step after the sums); both have been
+// acknowledged by then.  Step s asks for the carried sum of block s + 1 and the partial dq of block s, so it needs s +
+// 1: a tile runs three steps behind the one before (it was four while a sum was published no earlier than its block's
+// dq).  What the tile before has published is copied to LDS in the background, a step old when it is looked at; only
+// where that is not enough does a score wave -- the one all others wait for -- stop to ask.
 //
-// Measured (kernel time of the backward with its prep kernel, before and after the shorter lag, the poll in the background and leaner
-// product waves, alternating on one MI355X): 32 heads x 16 K tokens in eight documents, head_dim 128, 1311 -> 1292 us; 12 x 4 x 4096
-// 694 -> 683; 16 x 7 K in six documents, head_dim 96, 240 -> 226; 12 heads of 1500, 900 and 601 tokens, head_dim 64, 80.0 -> 69.8
-// and 128, 95.8 -> 88.  (Documents of one or two tiles, where what an item costs before its first step is the time, are 1 to 2 % slower: 32 heads of 64 x 256 at
-// 128 349 -> 354.)  At head_dim 128 it waits: 44 % of the wave
-// cycles on 32 heads x 16 K tokens (22 .. 25 % in the two passes; profiles/c3_sq_counters_pmc.txt), with the matrix pipe busy for
-// 36 %.  Such a launch fetches 4.5 GB from behind the L2s and writes 3.1 GB there, 5.8 TB/s where a plain copy reaches 4.9: of the
-// 2.8 GB of partial dq each way, all that is written leaves L2 (eight chains of 2 MiB share 4 MiB).
+// Measured (kernel time of the backward with its prep kernel, before and after the shorter lag, the poll in the
+// background and leaner product waves, alternating on one MI355X): 32 heads x 16 K tokens in eight documents, head_dim
+// 128, 1311 -> 1292 us; 12 x 4 x 4096 694 -> 683; 16 x 7 K in six documents, head_dim 96, 240 -> 226; 12 heads of 1500,
+// 900 and 601 tokens, head_dim 64, 80.0 -> 69.8 and 128, 95.8 -> 88.  (Documents of one or two
+// tiles above head_dim 64, where an item's beginning and end are the time, are up to 3 % slower: 32 heads of 64 x 256 at
+// 128 346 -> 354, 19 of 235 x 118 309 -> 316.  None of the changes gives that back alone: no poll, no wait for the
+// carried sum, columns read behind the barrier and one kind of iteration are all within 1 % of it or slower.)
+// At head_dim 128 it waits: 44 % of the wave cycles on 32 heads x 16 K tokens (22 .. 25 % in the two passes;
+// profiles/c3_sq_counters_pmc.txt), with the matrix pipe busy for 36 %.  Such a launch fetches 4.5 GB from behind the
+// L2s and writes 3.1 GB there, 5.8 TB/s where a plain copy reaches 4.9: of the 2.8 GB of partial dq each way, all that
+// is written leaves L2 (eight chains of 2 MiB share 4 MiB).
 //
-// What does not help: waves that are all alike.  Eight of them with 256 registers (steps of 64 queries, two barriers) took 1510 us at
-// head_dim 96 where this takes 1130, four with 512 registers and every matrix instruction placed by hand 1235: a wave alone on its
-// SIMD issues for 56 % of its cycles and has nothing to cover the rest.
+// What does not help: waves that are all alike.  Eight of them with 256 registers (steps of 64 queries, two barriers)
+// took 1510 us at head_dim 96 where this takes 1130, four with 512 registers and every matrix instruction placed by
+// hand 1235: a wave alone on its SIMD issues for 56 % of its cycles and has nothing to cover the rest.
 //
 // Carried sum: with C[j] the sum of G over the keys up to j and ex the stick on entering a key, D = C + drem ex
 // obeys D[j] = D[j-1] + p_j (do.v_j) and dz_j = r_j D[j] - D[j-1] (see grad_dz in sba_bwd.hip); the gradient of
@@ -116,16 +119,16 @@ __global__ void __launch_bounds__(NT) chain_prep_kernel(const ChainArgs a) {
   }
 }
 
-// NSQ: 32-query blocks per step.  4 * NSQ score waves (one per 32-key block and query block) and 4 product waves.  At head_dim
-// 128 registers leave room for one score wave per SIMD, whose vector work (180 instructions, 32 of them transcendental,
-// per block) is the step; at 64 and below two fit (168 registers): 16 heads x 4 documents of 2048 at head_dim 64 in steps of 64
-// queries 167 us for 198 in steps of 32, at head_dim 32 139 for 169 (two passes: 213, 174).
 // One dword, the same for every lane, to LDS at dst + 4 * lane.  Counted by vmcnt like async_copy16.
 __device__ __forceinline__ void async_word(const int* from, const int* dst) {
   const unsigned lds_addr = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2 sc1" ::"s"(lds_addr), "v"(0), "s"(from) : "memory", "m0");
 }
 
+// NSQ: 32-query blocks per step.  4 * NSQ score waves (one per 32-key block and query block) and 4 product waves.  At
+// head_dim 128 registers leave room for one score wave per SIMD, whose vector work (180 instructions, 32 of them
+// transcendental, per block) is the step; at 64 and below two fit (168 registers): 16 heads x 4 documents of 2048 at
+// head_dim 64 in steps of 64 queries 159 us for 187 in steps of 32, at head_dim 32 135 for 164 (two passes: 225, 173).
 // STREAM: Q and dO rows, which every key tile of the chain reads again, stream past the L2 (see chain_streams).
 template <int D, int U, bool AC, int NSQ, bool STREAM>
 __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const ChainArgs a) {
@@ -346,13 +349,13 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
-    // First score wave: the tile before this one has published `steps` steps (all of them: nothing to wait for any more).
-    // A wait that runs out -- it cannot while workgroups make progress -- must end in NaN and not in plausible numbers, in
-    // every wave: what it stood for is requested by all of them behind the barrier that follows, the partial dq of the block
-    // whose dz is formed there and the carried sum of the next one.  The waves of the oldest key block add `given_up` to that dz,
-    // which makes all of the block's dq NaN, and to the stick of the next block, whose weights they form in the same step: its p
-    // and dz are NaN, so is the sum every newer key block takes from `tot` for its D, and with dz of all of the tile's
-    // keys dk, dq and what is handed on.
+    // First score wave: the tile before this one has published `steps` steps (all of them: nothing to wait for any
+    // more).  A wait that runs out -- it cannot while workgroups make progress -- must end in NaN and not in plausible
+    // numbers, in every wave: what it stood for is requested by all of them behind the barrier that follows, the
+    // partial dq of the block whose dz is formed there and the carried sum of the next one.  The waves of the oldest
+    // key block add `given_up` to that dz, which makes all of the block's dq NaN, and to the stick of the next block,
+    // whose weights they form in the same step: its p and dz are NaN, so is the sum every newer key block takes from
+    // `tot` for its D, and with dz of all of the tile's keys dk, dq and what is handed on.
     auto await = [&](int steps) {
       const int need = min(steps, n_wait);
       auto published = [&]() {
@@ -383,9 +386,9 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       }
     };
 
-    // A block none of whose keys the queries from qw0 on may see: zeros in the place of its dz, staged before.  (By a second
-    // store: with a choice between the two values in the step itself the values alive across it do not fit the registers, and a
-    // mask costs every step.)
+    // A block none of whose keys the queries from qw0 on may see: zeros in the place of its dz, staged before.  (By a
+    // second store: with a choice between the two values in the step itself the values alive across it do not fit the
+    // registers, and a mask costs every step.)
     auto hide = [&](int qw0, int par) {
       if (!sub_skip<AC>(k0, qw0)) return;
 #pragma unroll
@@ -395,10 +398,11 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
     struct Weights { float p[16], r[16], lo; };
     // Step w: dz of block w (weights and do.v in `wc`, `dc`, formed a step ago), weights of block w + 1 (scores `xn`,
     // do.v `dn`) into `wn`, and the two MFMA chains of block w + 2 into `xf`, `df`, interleaved with the vector work in
-    // eight chunks (see bulk in sba_bwd.hip).  The sum over the key blocks before this wave's goes through `tot`: written
-    // with the weights, read a step later.  FIRST: there is no block w yet.  BAND: block w or w + 1 may hold keys its
-    // queries must not see.  A block that hides all of them stages zeros and nothing computed: where a key has a value that is
-    // not finite, or a query a running sum that is not, 0 times it is not zero.  SLOT >= 0: ring slot of tile w + 2, else taken from w.
+    // eight chunks (see bulk in sba_bwd.hip).  The sum over the key blocks before this wave's goes through `tot`:
+    // written with the weights, read a step later.  FIRST: there is no block w yet.  BAND: block w or w + 1 may hold
+    // keys its queries must not see.  A block that hides all of them stages zeros and nothing computed: where a key has
+    // a value that is not finite, or a query a running sum that is not, 0 times it is not zero.  SLOT >= 0: ring slot
+    // of tile w + 2, else taken from w.
     auto step = [&](auto first_tag, auto band_tag, auto slot_tag, const int w, Weights& wc, f32x16& dc, f32x16& xn, f32x16& dn,
                     Weights& wn, f32x16& xf, f32x16& df, float& se) __attribute__((always_inline)) {
       constexpr bool FIRST = decltype(first_tag)::value, BAND = decltype(band_tag)::value;
@@ -654,8 +658,8 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         if (keeper) await(1);
         lds_barrier();
         int i = 0;
-        // Everything repeats with period six (ring slots, staging buffers, weights, scores, do.v sums, carries): step i = 6 m has
-        // block i's weights in wa, its do.v in da0, block i+1's scores in x1 and do.v in da1.
+        // Everything repeats with period six (ring slots, staging buffers, weights, scores, do.v sums, carries): step i
+        // = 6 m has block i's weights in wa, its do.v in da0, block i+1's scores in x1 and do.v in da1.
 #pragma unroll 1
         for (; i + 6 < nsteps - DIAG - 2; i += 6) {
           publish(i);     step(No{}, No{}, integral_constant<int, 2>{}, i, wa, da0, x1, da1, wb, x0, da2, se1);     finish(i);
@@ -722,10 +726,10 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       for (int j = 0; j < DB; ++j)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[kb2][j][i] = 0.0f;
-    // Offsets (bytes) of this lane's reads.  The swizzle is an XOR of the chunk number, so the offset of a further chunk
-    // is the first one's with a constant XORed in: one register per row instead of one per read -- there is none to
-    // spare, and a spilled one would be reloaded through the counter that the waits below count on.  In bytes, and added to the
-    // tile's place as an integer: XOR and addition are then one instruction.
+    // Offsets (bytes) of this lane's reads.  The swizzle is an XOR of the chunk number, so the offset of a further
+    // chunk is the first one's with a constant XORed in: one register per row instead of one per read -- there is none
+    // to spare, and a spilled one would be reloaded through the counter that the waits below count on.  In bytes, and
+    // added to the tile's place as an integer: XOR and addition are then one instruction.
     int xb[2], yb[2];      // transpose reads of rows 8 h + 4 u + i16 / 4: staged block (chunk of key 64 half), tile (chunk of column 0)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -810,10 +814,10 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       constexpr bool ALL_DQ = NSQ * DB >= 4;             // every product wave has a block of dq
       constexpr int FETCH_OPS = 4 + 2 * Copy::NCH;
       constexpr int N_PRODUCTS = KQ * 2 * DB, REST = N_PRODUCTS - KZ / 2, OPS = 4 + FETCH_OPS;
-      // What a block needs besides its products: 45 vector and 41 scalar instructions an iteration (108 and about 100 with the places
-      // computed from the block's number and selects for what only an item's last iterations need).
-      // Places that move on with the blocks: staged blocks, tile read by dk / dv, ring slot that is copied to, and in memory the
-      // partial dq of the block that is stored and the rows that are copied.
+      // What a block needs besides its products: 45 vector and 41 scalar instructions an iteration (108 and about 100
+      // with the places computed from the block's number and selects for what only an item's last iterations need).
+      // Places that move on with the blocks: staged blocks, tile read by dk / dv, ring slot that is copied to, and in
+      // memory the partial dq of the block that is stored and the rows that are copied.
       const int y0 = place_of(mat ? Qs : Gs), x0 = place_of(mat ? Zs : Ps), x_end = x0 + (mat ? 2 : PBUF) * PB;
       int y_at = y0, x_at = x0, z_at = place_of(Zs), c_at = AHEAD * QB;
       int part_at = (t_last * NSQ + dsq) * (D * 128);                  // bytes of partial dq ahead of the next request's 32 rows
@@ -822,9 +826,10 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
       auto store_part = [&](const int i, const f32x16& dq, const bool store) __attribute__((always_inline)) {
         const f32x4 part = {dq[4 * i], dq[4 * i + 1], dq[4 * i + 2], dq[4 * i + 3]};
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, part), part_rs, (store ? lane16 : OUTSIDE) + 1024 * i, part_at + NSQ * D * 128, 0);
-        // The registers must not be written right behind the store.  The compiler leaves the wait state for that out where the
-        // store's offset is in a scalar register; an address computed into one by the next instruction was stored in its place
-        // in lanes 12 .. 15, now and then.  (The registers are an operand so that nothing else is put in between.)
+        // The registers must not be written right behind the store.  The compiler leaves the wait state for that out
+        // where the store's offset is in a scalar register; an address computed into one by the next instruction was
+        // stored in its place in lanes 12 .. 15, now and then.  (The registers are an operand so that nothing else is
+        // put in between.)
         asm volatile("s_nop 0" ::"v"(part) : "memory");
       };
       // operation i of those that request: partial dq of the block whose rows part_at names, then the tile AHEAD of it
@@ -911,11 +916,13 @@ __global__ void __launch_bounds__((4 * NSQ + 4) * 64, 1) bwd_chain_kernel(const 
         y_at = y_next;
         x_at = x_at + PB == x_end ? x0 : x_at + PB;
         z_at = 2 * place_of(Zs) + PB - z_at;
-        // The tile copied an iteration ago (read behind this barrier) has landed, what came after it may be in flight.  An item's
-        // last request, of nothing, has to come back all the same before its registers are used for something else.
+        // The tile copied an iteration ago (read behind this barrier) has landed, what came after it may be in flight.
+        // An item's last request, of nothing, has to come back all the same before its registers are used for something
+        // else.
         if (!TAIL || w < nsteps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + LOADS_PER_TILE) : "memory");
         else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS_PER_TILE) : "memory");
-        // (no wait for LDS: what was read of the staged blocks has been multiplied, the columns on their way stay where they are)
+        // (no wait for LDS: what was read of the staged blocks has been multiplied, the columns on their way stay where
+        // they are)
         asm volatile("s_barrier" ::: "memory");
       };
       int w = 1;

@@ -1,12 +1,11 @@
 // Device-side building blocks shared by the forward and backward kernels (gfx950 only).
 //
-// Orientation used everywhere: the score tile is computed TRANSPOSED, S^T = K . Q^T, with the
-// 32x32x16 bf16 MFMA.  In the accumulator layout of that instruction a lane owns ONE query
-// (column n = lane % 32) and 16 of the 32 rows of the sub-block (rows 8*(i/4) + 4*h + i%4 for
-// register i, h = lane / 32); the lane with the other h owns the other 16 rows of the same
-// query.  Which key sits in which row is ours to choose (see kperm).  The running sums / products of stick-breaking attention run along the key axis, so
-// they become in-register chains plus one exchange between the two half-waves
-// (v_permlane32_swap) -- no LDS, no DPP row scans.
+// Orientation used everywhere: the score tile is computed TRANSPOSED, S^T = K . Q^T, with the 32x32x16 bf16 MFMA.  In
+// the accumulator layout of that instruction a lane owns ONE query (column n = lane % 32) and 16 of the 32 rows of the
+// sub-block (rows 8*(i/4) + 4*h + i%4 for register i, h = lane / 32); the lane with the other h owns the other 16 rows
+// of the same query.  Which key sits in which row is ours to choose (see kperm).  The running sums / products of
+// stick-breaking attention run along the key axis, so they become in-register chains plus one exchange between the two
+// half-waves (v_permlane32_swap) -- no LDS, no DPP row scans.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -12,26 +12,26 @@ namespace sba {
 inline namespace SBA_ELEM_NS {
 
 // The item of this workgroup (items: tiles of every head, most expensive first).  Workgroup b starts on the same CU as
-// b + n_cus, b + 2 n_cus ...; while the chip holds the whole launch at once, whoever comes first gets the most expensive tile of every round
-// (tiles 15, 11, 7 and 3 for one CU against 12, 8, 4 and 0 for another).  Such a launch deals every second round backwards, eight
-// workgroups at a time, which leaves an item's head on its XCD.  A larger launch fills in behind its expensive tiles by itself (lg_cus: NO_DEAL).
-// 4 x 16 x 2048: 58.0 -> 55.7 us at head_dim 64 (with the carry table), 43.9 -> 41.9 at 32.
-// (Shifts, no branch, the grid's size as an argument, and the division by the heads a multiplication: every workgroup waits for this
-// before its first load.  With divisions and a branch 31 heads of 1003 tokens at head_dim 128 took 32.2 us for 31.6, 20 heads x 25 K tokens in 1682
-// documents at head_dim 32 94 for 84.)
+// b + n_cus, b + 2 n_cus ...; while the chip holds the whole launch at once, whoever comes first gets the most
+// expensive tile of every round (tiles 15, 11, 7 and 3 for one CU against 12, 8, 4 and 0 for another).  Such a launch
+// deals every second round backwards, eight workgroups at a time, which leaves an item's head on its XCD.  A larger
+// launch fills in behind its expensive tiles by itself (lg_cus: NO_DEAL).  4 x 16 x 2048: 58.0 -> 55.7 us at head_dim
+// 64 (with the carry table), 43.9 -> 41.9 at 32.  (Shifts, no branch, the grid's size as an argument, and the division
+// by the heads a multiplication: every workgroup waits for this before its first load.  With divisions and a branch 31
+// heads of 1003 tokens at head_dim 128 took 32.2 us for 31.6, 20 heads x 25 K tokens in 1682 documents at head_dim 32
+// 94 for 84.)
 __device__ __forceinline__ unsigned deal_item(int lg_cus, unsigned n) {
   const unsigned b = blockIdx.x, round = b >> lg_cus, first = round << lg_cus, eights = min(1u << lg_cus, n - first) >> 3, at = (b - first) >> 3;
   return (round & 1) && at < eights ? first + 8 * (eights - 1 - at) + (b & 7) : b;
 }
 
-// MODE 1 (WOUT): also write the attention weights (fp32, before their bf16 rounding) into a dense
-// [tokens x tokens] matrix per (batch, head) -- upstream's `return_attention` debug output
-// (sb_varlen_fwd.py:195-202).  MODE 2 (TAB): write the carry table and nothing else -- no V tiles,
-// no P.V products, no o, no rem -- for a backward whose forward kept no table.  Separate
-// instantiations, so the production kernel (MODE 0) carries none of it.
-// head_dim 256: two workgroups per CU, so that a wave's waits are another's time: a ring of two slots (64 KiB) and 256 registers, 64 of them
-// Q fragments and 128 accumulators, the tile offsets of columns 128 .. 255 as immediates.  (One workgroup per CU, one wave per SIMD with
-// 512 registers and three slots: 554 us on 16 heads x 16 K tokens in eight documents, this 415.)
+// MODE 1 (WOUT): also write the attention weights (fp32, before their bf16 rounding) into a dense [tokens x tokens]
+// matrix per (batch, head) -- upstream's `return_attention` debug output (sb_varlen_fwd.py:195-202).  MODE 2 (TAB):
+// write the carry table and nothing else -- no V tiles, no P.V products, no o, no rem -- for a backward whose forward
+// kept no table.  Separate instantiations, so the production kernel (MODE 0) carries none of it.  head_dim 256: two
+// workgroups per CU, so that a wave's waits are another's time: a ring of two slots (64 KiB) and 256 registers, 64 of
+// them Q fragments and 128 accumulators, the tile offsets of columns 128 .. 255 as immediates.  (One workgroup per CU,
+// one wave per SIMD with 512 registers and three slots: 554 us on 16 heads x 16 K tokens in eight documents, this 415.)
 // U: columns that are multiplied (see used_width); tile rows in LDS keep the width D.
 template <int D, bool AC, bool PROD, int MODE, int U = D>
 __global__ void __launch_bounds__(NT, D > 128 ? 2 : 3) fwd_kernel(const KArgs a) {
@@ -161,11 +161,12 @@ __global__ void __launch_bounds__(NT, D > 128 ? 2 : 3) fwd_kernel(const KArgs a)
 #pragma unroll
     for (int i = 0; i < 16; ++i) x[i] = 0.0f;
     {
-      // Beyond head_dim 64 K fragments are read four ahead of their multiplication, in an order that is pinned: left to itself the compiler reads one or two ahead
-      // and waits for each.  32 heads of 64 K tokens, longest document 32 K, at head_dim 128 10.98 -> 10.81 ms (sustained, at a lower clock than
-      // the 9.47 -> 9.41 of a few launches), 12 heads of 4 x 4096 218 -> 211 us, 16 heads x 16 K in eight documents at 256 430 -> 415, at
-      // 192 322 -> 315.  (Four or two fragments pinned at 64 and 32: 0.8 % slower to 0.  Half of V's fragments read before the weights are formed: nothing at
-      // 64 and 96, spills from 128 on.)
+      // Beyond head_dim 64 K fragments are read four ahead of their multiplication, in an order that is pinned: left to
+      // itself the compiler reads one or two ahead and waits for each.  32 heads of 64 K tokens, longest document 32 K,
+      // at head_dim 128 10.98 -> 10.81 ms (sustained, at a lower clock than the 9.47 -> 9.41 of a few launches), 12
+      // heads of 4 x 4096 218 -> 211 us, 16 heads x 16 K in eight documents at 256 430 -> 415, at 192 322 -> 315.
+      // (Four or two fragments pinned at 64 and 32: 0.8 % slower to 0.  Half of V's fragments read before the weights
+      // are formed: nothing at 64 and 96, spills from 128 on.)
       constexpr bool PIN = KS > 4;
       constexpr int AHEAD = KS < 4 ? KS : 4;
       el8 kfr[AHEAD];

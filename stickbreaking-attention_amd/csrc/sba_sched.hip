@@ -95,8 +95,9 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
     ranked[r] = d;
   }
   __syncthreads();
-  // The classes of D, found once for a document (us without classes / with every tile searching for its own / as built: 40 documents of up to 3000
-  // tokens 9.1 / 13.2 / 11.4, 600 of 200 .. 900 34.6 / 50.9 / 36.3, 30 of 32768, 24576 ... 11.8 / 22.4 / 14.5, eight of 512 .. 4096 5.7 / 6.8 / 6.8).
+  // The classes of D, found once for a document (us without classes / with every tile searching for its own / as built:
+  // 40 documents of up to 3000 tokens 9.1 / 13.2 / 11.4, 600 of 200 .. 900 34.6 / 50.9 / 36.3, 30 of 32768, 24576 ...
+  // 11.8 / 22.4 / 14.5, eight of 512 .. 4096 5.7 / 6.8 / 6.8).
   const bool classes = a.classes && in_lds && s_maxlen > BM * (CLASS_TILES - 1);
   if (classes) {
     for (int i = tid; i < nd; i += SCHED_THREADS) {
@@ -184,19 +185,20 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
   if (tid == 0) { q_before[nd] = total_q; kv_before[nd] = total_long; }
   __syncthreads();
 
-  // D. emit tiles: slot -> ranked document by binary search over the prefix
-  // The hardware deals workgroups to the CUs round-robin in launch order (workgroups i and
-  // i + number of CUs start on the same CU and run side by side), and hands out the rest as
-  // slots free up.  Where the launch is short or the heads are few (list_in_classes), documents of like length -- a class: more than three quarters of the tiles of its longest -- are therefore
-  // listed tile-major, the most expensive tile of every document first: the expensive tiles start together and the cheap
-  // ones fill in behind them.  Document-major, the last document's most expensive tile starts when most of the launch is
-  // over, and documents of one length put the same tile on the same CU.  Classes follow one another,
-  // so that a workgroup's neighbours still share K/V rows in the caches.  Forward, us, document-major / classes from half the
-  // longest on / classes from three quarters on: 12 heads x 4 x 4096 at head_dim 128 284 / 242 / 241, 9 heads x 28667 tokens in 17 documents of up to
-  // 4148 247 / 217 / 218, 5 heads x 62572 tokens at head_dim 64, one document of 14691 among shorter ones, 395 / 413 / 403.  Documents of less than CLASS_TILES
-  // tiles stay document-major, and so does a class of more documents than its longest has tiles, as a document's K/V rows have left the caches
-  // by its next tile (32 heads x 16 K tokens in 207 documents of 16 .. 256: 66.2 / 67.4 us; 21 heads x 37933 tokens in 61 documents
-  // of about 630 at head_dim 128: 257 / 329 / 259).
+  // D. emit tiles: slot -> ranked document by binary search over the prefix The hardware deals workgroups to the CUs
+  // round-robin in launch order (workgroups i and i + number of CUs start on the same CU and run side by side), and
+  // hands out the rest as slots free up.  Where the launch is short or the heads are few (list_in_classes), documents
+  // of like length -- a class: more than three quarters of the tiles of its longest -- are therefore listed tile-major,
+  // the most expensive tile of every document first: the expensive tiles start together and the cheap ones fill in
+  // behind them.  Document-major, the last document's most expensive tile starts when most of the launch is over, and
+  // documents of one length put the same tile on the same CU.  Classes follow one another, so that a workgroup's
+  // neighbours still share K/V rows in the caches.  Forward, us, document-major / classes from half the longest on /
+  // classes from three quarters on: 12 heads x 4 x 4096 at head_dim 128 284 / 242 / 241, 9 heads x 28667 tokens in 17
+  // documents of up to 4148 247 / 217 / 218, 5 heads x 62572 tokens at head_dim 64, one document of 14691 among shorter
+  // ones, 395 / 413 / 403.  Documents of less than CLASS_TILES tiles stay document-major, and so does a class of more
+  // documents than its longest has tiles, as a document's K/V rows have left the caches by its next tile (32 heads x 16
+  // K tokens in 207 documents of 16 .. 256: 66.2 / 67.4 us; 21 heads x 37933 tokens in 61 documents of about 630 at
+  // head_dim 128: 257 / 329 / 259).
   for (int s = tid; s < total_q && ok; s += SCHED_THREADS) {
     int d, idx, rank = 0, slot = s;
     if (fixed) {
@@ -248,7 +250,8 @@ __global__ void __launch_bounds__(SCHED_THREADS) sched_kernel(const SchedArgs a)
     kvtiles[s] = t;
   }
   // E. the documents in ranked order, {first token, length, first table entry, 128-row tiles before}: what the one-pass
-  // backward names its chains by and bwd_short_kernel goes by.  With the working arrays in LDS their places in the workspace are free.
+  // backward names its chains by and bwd_short_kernel goes by.  With the working arrays in LDS their places in the
+  // workspace are free.
   if (in_lds && ok) {
     int2* const docs = reinterpret_cast<int2*>(dstart + chain_docs_offset(nd));
     for (int i = tid; i < nd; i += SCHED_THREADS) {

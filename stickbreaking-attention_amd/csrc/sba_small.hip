@@ -1,9 +1,10 @@
 // Kernels for problems that leave most of the chip idle.
 //
-// With few tiles a launch takes as long as one workgroup's walk along the other axis, a block of 32 at a time: 47 steps of 0.65 us
-// for the forward of 1500 tokens, whatever the chip could do beside them.  Here a workgroup owns 32 rows instead of 128, and
-// its four waves take four consecutive blocks of the other axis at a time.  (Eight waves: a single head of 4096 keys 30 us for 35, but
-// a full chip is served worse, since the last round of every walk is the emptier: 16 x 2048 29 us for 26, 16 x 4 x 1024 38 for 28.)
+// With few tiles a launch takes as long as one workgroup's walk along the other axis, a block of 32 at a time: 47 steps
+// of 0.65 us for the forward of 1500 tokens, whatever the chip could do beside them.  Here a workgroup owns 32 rows
+// instead of 128, and its four waves take four consecutive blocks of the other axis at a time.  (Eight waves: a single
+// head of 4096 keys 30 us for 35, but a full chip is served worse, since the last round of every walk is the emptier:
+// 16 x 2048 29 us for 26, 16 x 4 x 1024 38 for 28.)
 #include <type_traits>
 
 #include "sba_kernels.hpp"
@@ -11,7 +12,8 @@
 namespace sba {
 inline namespace SBA_ELEM_NS {
 
-// One wave's copy of a 32 x D block into its own unpadded, swizzled tile; KEYS: rows permuted as by TileCopy<.., KEYS = true>.
+// One wave's copy of a 32 x D block into its own unpadded, swizzled tile; KEYS: rows permuted as by TileCopy<.., KEYS =
+// true>.
 template <int D, bool KEYS>
 struct WaveCopy {
   static constexpr int C8 = D / 8, RPI = 64 / C8, NCH = 32 / RPI;
@@ -63,7 +65,8 @@ __device__ __forceinline__ void store_quad(f32x4 v, const Rows& out, const Rows&
   }
 }
 
-// The waves' accumulators of one output, a quad of every lane at a time, into LDS; behind a barrier wave w adds up and stores quads w, w + W ..
+// The waves' accumulators of one output, a quad of every lane at a time, into LDS; behind a barrier wave w adds up and
+// stores quads w, w + W ..
 template <int DB, int W>
 __device__ __forceinline__ void add_waves(float* sums, const f32x16 (&acc)[DB], int w, int lane) {
 #pragma unroll
@@ -85,15 +88,16 @@ __device__ __forceinline__ void store_sum(const float* sums, int w, int lane, fl
   for (int q = w; q < 4 * DB; q += W) store_quad(sum_quad<W>(sums, q, lane) * scale, out, out, row, ok, 32 * (q >> 2) + 8 * (q & 3) + 4 * h, false, 0.0f, f32);
 }
 
-// Forward.  32 query rows of one (document, head); in a round wave w has the w-th newest key block that is left.  What a block leaves of
-// the stick (its product of 1 - beta) is known before its weights are, so the waves form odds and products side by side,
-// exchange the products through LDS (one barrier a round) and go on to weights and p V each on its own.  The output is the sum
-// over the waves.  K and V rows come to every wave's own piece of LDS, the next round's as soon as this one's are read.
-// What bounds it: the round's serial chain (products, odds, barrier, weights) while the chip is empty, 0.9 us a round of 128 keys against
-// 0.54 us a step of 32 in fwd_kernel; then the additive time of matrix and vector instructions, with
-// 16 waves per compute unit at head_dim 64, 8 at 128 and 4 at 256.  Measured (us, fwd_kernel first): head_dim 64, 4 heads of 512 tokens 14.4 / 9.7,
-// of 2048 40 / 20; 16 heads of 1024 23.7 / 15.2; head_dim 128, 4 heads of 512 18.0 / 11.7, 16 heads of 2048 54 / 43;
-// head_dim 256, 4 heads of 512 28 / 18, of 2048 87 / 41.
+// Forward.  32 query rows of one (document, head); in a round wave w has the w-th newest key block that is left.  What
+// a block leaves of the stick (its product of 1 - beta) is known before its weights are, so the waves form odds and
+// products side by side, exchange the products through LDS (one barrier a round) and go on to weights and p V each on
+// its own.  The output is the sum over the waves.  K and V rows come to every wave's own piece of LDS, the next round's
+// as soon as this one's are read.  What bounds it: the round's serial chain (products, odds, barrier, weights) while
+// the chip is empty, 0.9 us a round of 128 keys against 0.54 us a step of 32 in fwd_kernel; then the additive time of
+// matrix and vector instructions, with 16 waves per compute unit at head_dim 64, 8 at 128 and 4 at 256.  Measured (us,
+// fwd_kernel first): head_dim 64, 4 heads of 512 tokens 14.4 / 9.7, of 2048 40 / 20; 16 heads of 1024 23.7 / 15.2;
+// head_dim 128, 4 heads of 512 18.0 / 11.7, 16 heads of 2048 54 / 43; head_dim 256, 4 heads of 512 28 / 18, of 2048 87
+// / 41.
 template <int D, bool AC, int U>
 __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 4 : (D <= 128 ? 2 : 1)) fwd_small_kernel(const KArgs a) {
   constexpr int W = SMALL_WAVES, KS = U / 16, DB = U / 32, TILE = 32 * D;
@@ -239,16 +243,17 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 4 : (D <= 128 ? 2 
 }
 
 // -------------------------------------------------------------------------------------------
-// Backward, in two passes of the same kind.  The first owns 32 queries, four waves walk the keys from the oldest
-// on, a block each at a time; they exchange every block's sum of p (do.v) and with it each knows the running sum D in front of its block (see
-// sba_chain.hip), which goes into the gradient table.  With the table the second, which owns 32 keys, needs no order at all: its
-// waves take the query blocks that can see them in turn.  Sums over the waves at the end.
-// What bounds them: up to 8 waves per compute unit (head_dim 64; 4 at 128) each a round's chain of its own: two products, odds and weights, the
-// barrier, the gradient of the logits, one or two products more: 1.1 us a round.  That is no shorter than a step of bwd_chain_kernel, but
-// a round is 128 keys, and nothing is handed from one workgroup to the next.  Measured (us, one-pass form first): head_dim 64, 4 heads of 512 tokens
-// 36.2 / 11.3 + 12.2, of 2048 89 / 25 + 26; 16 heads of 1024 55 / 17 + 21; 2 x 8 of 1500 78 / 23 + 33; head_dim 128, 4 heads of 512 42 / 15 + 16.
-// Eight waves a workgroup gain where 4 heads are all there is (2048 tokens: 51 to 43) and lose from 16 heads on (1024 tokens: 37 to 45); two lose everywhere
-// else (2 x 8 of 1500: 57 to 75).
+// Backward, in two passes of the same kind.  The first owns 32 queries, four waves walk the keys from the oldest on, a
+// block each at a time; they exchange every block's sum of p (do.v) and with it each knows the running sum D in front
+// of its block (see sba_chain.hip), which goes into the gradient table.  With the table the second, which owns 32 keys,
+// needs no order at all: its waves take the query blocks that can see them in turn.  Sums over the waves at the end.
+// What bounds them: up to 8 waves per compute unit (head_dim 64; 4 at 128) each a round's chain of its own: two
+// products, odds and weights, the barrier, the gradient of the logits, one or two products more: 1.1 us a round.  That
+// is no shorter than a step of bwd_chain_kernel, but a round is 128 keys, and nothing is handed from one workgroup to
+// the next.  Measured (us, one-pass form first): head_dim 64, 4 heads of 512 tokens 36.2 / 11.3 + 12.2, of 2048 89 / 25
+// + 26; 16 heads of 1024 55 / 17 + 21; 2 x 8 of 1500 78 / 23 + 33; head_dim 128, 4 heads of 512 42 / 15 + 16.  Eight
+// waves a workgroup gain where 4 heads are all there is (2048 tokens: 51 to 43) and lose from 16 heads on (1024 tokens:
+// 37 to 45); two lose everywhere else (2 x 8 of 1500: 57 to 75).
 // -------------------------------------------------------------------------------------------
 template <int D, bool AC, int U>
 __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_dq_small_kernel(const KArgs a) {
@@ -541,22 +546,25 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_dkdv_sm
 }
 
 // -------------------------------------------------------------------------------------------
-// Backward of documents of at most 32 x SHORT_BLOCKS tokens, both passes in one: a team of waves takes one (document, head),
-// half as many waves as it has blocks of 32 tokens, and a workgroup has one team of four, two of two or four of one.  K and V
-// go to LDS; every wave walks the keys of its own queries, oldest first, for dq, and leaves the running sum D of every block of
-// 32 x 32 in LDS.  Then Q and dO, which the waves hold as their own operands, take the place of K and V, and the waves own keys.
-// Query block i takes i + 1 steps, key block i of n takes n - i: with blocks w and n - 1 - w a wave has n + 1 in either half.
-// What bounds it: the two passes it stands in for ran at the rate of a copy, four operands read by each and the sums D written and read
-// between them; here operands come in once (32 heads x 16 K tokens in documents of 16 .. 256: 228 us for 161, of which 94 are its traffic).  What is
-// left is that a workgroup loads, computes and stores one after the other, two of them (8 waves of 239 registers, 80 KB of LDS) per compute unit, one above head_dim 64:
-// loads and stores alone take 115 us, and neither workgroups that start late nor an order that mixes long and short documents overlaps them better.
-// So nothing is read from memory behind the first barrier: a load there is waited for behind the stores of dq, in order, and the sticks one step ahead were
-// later than a step.  Sticks come to LDS with K and V, K and V rows of both key blocks are kept from there; the document's
-// place is made scalar, which takes a loop over lanes away from every access, and operands are read four steps ahead of their multiplication.
-// On one GPU, us: these documents at head_dim 64 175 -> 164, at 32 104 -> 95; 32 heads of 128 x 256 tokens 342 -> 320, of 128 x 33 46.3 -> 44.3; at
-// head_dim 128 16 heads of 128 x 64 76 -> 68.  Streaming stores (nt) cost a third: they leave in quarters of a line.
-// One document to a workgroup whatever its length: 204 us, most waves idle; four slots of the tile list to a workgroup, long documents one after the other: 166 us,
-// and 104 for 31 us where there are few of them.
+// Backward of documents of at most 32 x SHORT_BLOCKS tokens, both passes in one: a team of waves takes one (document,
+// head), half as many waves as it has blocks of 32 tokens, and a workgroup has one team of four, two of two or four of
+// one.  K and V go to LDS; every wave walks the keys of its own queries, oldest first, for dq, and leaves the running
+// sum D of every block of 32 x 32 in LDS.  Then Q and dO, which the waves hold as their own operands, take the place of
+// K and V, and the waves own keys.  Query block i takes i + 1 steps, key block i of n takes n - i: with blocks w and n
+// - 1 - w a wave has n + 1 in either half.  What bounds it: the two passes it stands in for ran at the rate of a copy,
+// four operands read by each and the sums D written and read between them; here operands come in once (32 heads x 16 K
+// tokens in documents of 16 .. 256: 228 us for 161, of which 94 are its traffic).  What is left is that a workgroup
+// loads, computes and stores one after the other, two of them (8 waves of 239 registers, 80 KB of LDS) per compute
+// unit, one above head_dim 64: loads and stores alone take 115 us, and neither workgroups that start late nor an order
+// that mixes long and short documents overlaps them better.  So nothing is read from memory behind the first barrier: a
+// load there is waited for behind the stores of dq, in order, and the sticks one step ahead were later than a step.
+// Sticks come to LDS with K and V, K and V rows of both key blocks are kept from there; the document's place is made
+// scalar, which takes a loop over lanes away from every access, and operands are read four steps ahead of their
+// multiplication.  On one GPU, us: these documents at head_dim 64 175 -> 164, at 32 104 -> 95; 32 heads of 128 x 256
+// tokens 342 -> 320, of 128 x 33 46.3 -> 44.3; at head_dim 128 16 heads of 128 x 64 76 -> 68.  Streaming stores (nt)
+// cost a third: they leave in quarters of a line.  One document to a workgroup whatever its length: 204 us, most waves
+// idle; four slots of the tile list to a workgroup, long documents one after the other: 166 us, and 104 for 31 us where
+// there are few of them.
 // -------------------------------------------------------------------------------------------
 template <int D, bool AC, int U>
 __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_kernel(const KArgs a) {
@@ -647,7 +655,8 @@ __global__ void __launch_bounds__(SMALL_WAVES * 64, D <= 64 ? 2 : 1) bwd_short_k
         gf[turn][ks] = load_frag(grows, row, 32 * ks + 16 * h);
       }
   }
-  // Everything else that is read from memory is asked for here as well: a load further down would be waited for behind the stores of dq.
+  // Everything else that is read from memory is asked for here as well: a load further down would be waited for behind
+  // the stores of dq.
   const float* const stick = a.stick + (int64_t)head * a.tab_stride + about.z;
   const __amdgpu_buffer_rsrc_t stick_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(stick), 0, 4u * (unsigned)tab_doc_entries(L), 0x00020000);
   // byte offset of the stick left in front of key block b for row `row`

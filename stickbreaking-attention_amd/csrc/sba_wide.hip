@@ -1,9 +1,9 @@
-// The two passes of the backward at head_dim 129 .. 256 (see sba_bwd.hip for the two-pass backward and its other kernels): the dk / dv
-// pass, described here, and the dq pass, further down.
+// The two passes of the backward at head_dim 129 .. 256 (see sba_bwd.hip for the two-pass backward and its other
+// kernels): the dk / dv pass, described here, and the dq pass, further down.
 //
-// At twice the width of the eight-wave kernel of sba_bwd.hip a wave's K and V fragments are 128 registers and the accumulators of 64
-// keys of one output 256: neither role fits two waves per SIMD.  So the work is cut smaller.  A workgroup owns 64 keys of
-// one (document, head) and walks the queries that can see them, 32 per step:
+// At twice the width of the eight-wave kernel of sba_bwd.hip a wave's K and V fragments are 128 registers and the
+// accumulators of 64 keys of one output 256: neither role fits two waves per SIMD.  So the work is cut smaller.  A
+// workgroup owns 64 keys of one (document, head) and walks the queries that can see them, 32 per step:
 //
 //   waves 0, 1   "weights", one 32-key block each, K fragments in registers: scores, p, dz
 //   waves 2, 3   "do.v" of the same blocks, V fragments in registers; handed to the weights wave through LDS in fp32
@@ -15,12 +15,13 @@
 // scores of block i + 1 between the vector instructions of dz, the do.v waves theirs, and the product waves read the Q / dO
 // fragments of block i.  A tile is requested two steps before it is read (four slots of 32 KiB).
 //
-// Bound by the vector work of the two weights waves, alone with it on their SIMDs (of 2400 cycles of a step, stamped, they wait 350,
-// the product waves 650, the do.v waves 1300), and by what a work item costs beside its steps (8000 cycles, 45 steps on average);
-// the matrix pipes are busy for a third of the time.  16 heads x 16 K tokens in eight documents, head_dim 256: 1525 -> 890 us against
-// four independent waves of 32 keys each, which formed the scores twice, once for dv and once for dk, because both outputs'
-// accumulators (256 registers) left the chains nowhere to go.  Tried: a quarter or half of a block's products in the second phase (942,
-// 970 for 922), the next tile requested ahead of the products (950).
+// Bound by the vector work of the two weights waves, alone with it on their SIMDs (of 2400 cycles of a step, stamped,
+// they wait 350, the product waves 650, the do.v waves 1300), and by what a work item costs beside its steps (8000
+// cycles, 45 steps on average); the matrix pipes are busy for a third of the time.  16 heads x 16 K tokens in eight
+// documents, head_dim 256: 1525 -> 890 us against four independent waves of 32 keys each, which formed the scores
+// twice, once for dv and once for dk, because both outputs' accumulators (256 registers) left the chains nowhere to go.
+// Tried: a quarter or half of a block's products in the second phase (942, 970 for 922), the next tile requested ahead
+// of the products (950).
 #include <type_traits>
 
 #include "sba_kernels.hpp"
@@ -104,7 +105,8 @@ __global__ void __launch_bounds__(512, 1) bwd_dkdv_wide_kernel(const KArgs a) {
       // fused output: rem_j * do_j reaches dv_j through the diagonal of p (see bwd_dkdv_kernel)
       float rem_own = 0.0f;
       if (a.fuse && k0 + n < L) rem_own = a.stick[tab_rowval + k0 + n];
-      // carries of a step, requested three steps ahead; rows past the document's end take its last row's (see bwd_dkdv_kernel)
+      // carries of a step, requested three steps ahead; rows past the document's end take its last row's (see
+      // bwd_dkdv_kernel)
       const unsigned run_bytes = (unsigned)L * 4u;
       const __amdgpu_buffer_rsrc_t stick_rs = __builtin_amdgcn_make_buffer_rsrc(a.stick + tab, 0, run_bytes, 0x00020000);
       const __amdgpu_buffer_rsrc_t gtab_rs = __builtin_amdgcn_make_buffer_rsrc(a.gtab + tab, 0, run_bytes, 0x00020000);
@@ -323,8 +325,9 @@ __global__ void __launch_bounds__(512, 1) bwd_dkdv_wide_kernel(const KArgs a) {
       half_of(0);
       if (b > 0) half_of(1);
     };
-    // Behind the products of step i - 1: tile i + 1, which the others read behind the barrier, has landed; the fragments of
-    // tile i; tile i + 3 is requested (into the slot of tile i - 1; here and not ahead of the products, which the weights waves wait for).
+    // Behind the products of step i - 1: tile i + 1, which the others read behind the barrier, has landed; the
+    // fragments of tile i; tile i + 3 is requested (into the slot of tile i - 1; here and not ahead of the products,
+    // which the weights waves wait for).
     auto turn = [&](int i) __attribute__((always_inline)) {
       if (i + 2 < nsteps) wait_loads<LOADS_PER_TILE>();
       else wait_loads<0>();
@@ -356,18 +359,20 @@ __global__ void __launch_bounds__(512, 1) bwd_dkdv_wide_kernel(const KArgs a) {
 }
 
 // -------------------------------------------------------------------------------------------
-// dq pass of the same head dims: 128 queries of one (document, head) per workgroup, the keys walked from the oldest to the diagonal, 32
-// per step.  Q and dO fragments of 32 queries and their dq are 256 registers, so two waves of a SIMD share a block of 32 queries:
+// dq pass of the same head dims: 128 queries of one (document, head) per workgroup, the keys walked from the oldest to
+// the diagonal, 32 per step.  Q and dO fragments of 32 queries and their dq are 256 registers, so two waves of a SIMD
+// share a block of 32 queries:
 //
-//   waves 0 .. 3  "scores": Q fragments; p, dz, the running sum and the gradient table
-//   waves 4 .. 7  "sums": dO fragments and dq; do.v of a block, handed to the scores wave through LDS in fp32, and dq += dz K of the
+//   waves 0 .. 3  "scores": Q fragments; p, dz, the running sum and the gradient table waves 4 .. 7  "sums": dO
+//   fragments and dq; do.v of a block, handed to the scores wave through LDS in fp32, and dq += dz K of the
 //                 block before, whose dz comes back the same way; they also copy the K / V tiles
 //
-// A step has two phases with a barrier behind each: weights of block i next to the products of block i - 1, then dz of block i
-// between the scores of block i + 1 next to its do.v.  A tile is requested two steps before it is read (four slots of 32 KiB).
-// Bound by the two phases, 3300 cycles of a step: vector work of one wave, then 32 matrix instructions of two.  16 heads x 16 K tokens in
-// eight documents, head_dim 256: 795 -> 620 us against one wave per SIMD with 512 registers for everything.  Reading
-// operands six or eight instead of four products ahead changes nothing.
+// A step has two phases with a barrier behind each: weights of block i next to the products of block i - 1, then dz of
+// block i between the scores of block i + 1 next to its do.v.  A tile is requested two steps before it is read (four
+// slots of 32 KiB).  Bound by the two phases, 3300 cycles of a step: vector work of one wave, then 32 matrix
+// instructions of two.  16 heads x 16 K tokens in eight documents, head_dim 256: 795 -> 620 us against one wave per
+// SIMD with 512 registers for everything.  Reading operands six or eight instead of four products ahead changes
+// nothing.
 // -------------------------------------------------------------------------------------------
 template <bool AC, bool PROD, int U, bool GIVE>
 __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
@@ -376,7 +381,8 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
   static_assert(SLOTS * BF == BM, "the query rows wait in the ring first");
   __shared__ __attribute__((aligned(16))) unsigned short Ks[SLOTS * TILE];
   __shared__ __attribute__((aligned(16))) unsigned short Vs[SLOTS * TILE];
-  // per block of queries: do.v of a key block as the accumulators lie, a quad of every lane at a time, and dz as operand fragments
+  // per block of queries: do.v of a key block as the accumulators lie, a quad of every lane at a time, and dz as
+  // operand fragments
   constexpr int HAND_Z = 16 * 64, HAND = HAND_Z + 2 * 64 * 4;
   __shared__ __attribute__((aligned(16))) float hand[4 * HAND];
   __shared__ float drs[4][32];                                               // do . v_row of the fused output
@@ -413,8 +419,9 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
   auto rows_of = [&](const View& v) {
     return make_rows(reinterpret_cast<const elem_t*>(v.ptr) + t.batch * v.sb + head * v.sh + tok0 * v.st, v.st, L, a.head_dim);
   };
-  // Row reads of chunk 2 ks + h: the swizzle is an XOR of the chunk number's low four bits, so the offset of a further chunk is
-  // the first one's with a constant XORed in, and of the upper half's 256 bytes on: one register instead of sixteen.
+  // Row reads of chunk 2 ks + h: the swizzle is an XOR of the chunk number's low four bits, so the offset of a further
+  // chunk is the first one's with a constant XORed in, and of the upper half's 256 bytes on: one register instead of
+  // sixteen.
   int rbase = swz_off<D>(n, h);
   el8 fr[KS];                                            // Q or dO: operand column n is query qw0 + n
   constexpr int LEAD = 4;
@@ -446,8 +453,8 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   lds_barrier();                              // the places are free
   float* const mine = hand + HAND * rb + 4 * lane;
-  // GIVE: p and dz of a block as the lanes hold them, eight keys of a query in 16 bytes: lane's first eight keys, then the lanes'
-  // other eight.  A block's place goes by the carry table's.
+  // GIVE: p and dz of a block as the lanes hold them, eight keys of a query in 16 bytes: lane's first eight keys, then
+  // the lanes' other eight.  A block's place goes by the carry table's.
   const bool gives = GIVE && qw0 < L;         // (a block of queries behind the document's end has no place)
   __amdgpu_buffer_rsrc_t give_rs;
   if constexpr (GIVE)
@@ -690,17 +697,19 @@ __global__ void __launch_bounds__(512, 1) bwd_dq_wide_kernel(const KArgs a) {
 }
 
 // -------------------------------------------------------------------------------------------
-// dk / dv pass of the same head dims where the dq pass has left p and dz of every block in memory (GIVE, above): 128 keys of one
-// (document, head) per workgroup, dv = p^T dO and dk = dz^T Q over the queries that can see them, 32 per step.  All eight waves are alike: 64
-// keys x half of the columns of one output each (128 registers), and a share of the copies.  A tile is 48 KiB (Q, dO, p, dz), three of
-// them in a ring; one barrier per step, operands read a step ahead.
+// dk / dv pass of the same head dims where the dq pass has left p and dz of every block in memory (GIVE, above): 128
+// keys of one (document, head) per workgroup, dv = p^T dO and dk = dz^T Q over the queries that can see them, 32 per
+// step.  All eight waves are alike: 64 keys x half of the columns of one output each (128 registers), and a share of
+// the copies.  A tile is 48 KiB (Q, dO, p, dz), three of them in a ring; one barrier per step, operands read a step
+// ahead.
 //
-// Bound by what it reads: 16 heads x 16 K tokens in eight documents at head_dim 256, 456 us for 1.45 GB of p and dz, which are read once, and
-// Q and dO, of which every key tile takes its own (398 without the former, 367 without the latter, both timing only); the matrix pipes are busy
-// for 40 %.  So the queries are walked from the document's end: the key tiles of a (document, head) that start together then read
-// the same rows at the same time (from the tile's own keys on 816 us for 678, 12 heads of 4 x 4096), and p and dz stream past the L2s that Q and dO
-// are kept in (as do the dq pass's stores of them: 568 -> 456).  The pass that forms p and dz itself: 890.  Handing them on costs the dq
-// pass 100 of 724 us, a third of it the packing.
+// Bound by what it reads: 16 heads x 16 K tokens in eight documents at head_dim 256, 456 us for 1.45 GB of p and dz,
+// which are read once, and Q and dO, of which every key tile takes its own (398 without the former, 367 without the
+// latter, both timing only); the matrix pipes are busy for 40 %.  So the queries are walked from the document's end:
+// the key tiles of a (document, head) that start together then read the same rows at the same time (from the tile's own
+// keys on 816 us for 678, 12 heads of 4 x 4096), and p and dz stream past the L2s that Q and dO are kept in (as do the
+// dq pass's stores of them: 568 -> 456).  The pass that forms p and dz itself: 890.  Handing them on costs the dq pass
+// 100 of 724 us, a third of it the packing.
 // -------------------------------------------------------------------------------------------
 template <int U>
 __global__ void __launch_bounds__(512, 1) bwd_dkdv_given_kernel(const KArgs a) {
@@ -734,10 +743,11 @@ __global__ void __launch_bounds__(512, 1) bwd_dkdv_given_kernel(const KArgs a) {
   Copy qcopy, gcopy;
   qcopy.init(tid, qrows.row_bytes, qrows.used_bytes);
   gcopy.init(tid, grows.row_bytes, grows.used_bytes);
-  // Staged p or dz: four blocks one behind the other, each as it lies in memory: eight keys of a query in 16 bytes, the first eight keys of a
-  // half-wave's sixteen, then the other eight.  A wave copies one of those halves of a block.  The queries are XORed with four times the
-  // number of the eight keys, so that the transpose reads of all of them take different banks.  (Of the first three blocks of queries
-  // the newer key blocks do not exist: what is copied in their place is not multiplied.)
+  // Staged p or dz: four blocks one behind the other, each as it lies in memory: eight keys of a query in 16 bytes, the
+  // first eight keys of a half-wave's sixteen, then the other eight.  A wave copies one of those halves of a block.
+  // The queries are XORed with four times the number of the eight keys, so that the transpose reads of all of them take
+  // different banks.  (Of the first three blocks of queries the newer key blocks do not exist: what is copied in their
+  // place is not multiplied.)
   const int from = 1024 * (w & 1) + 16 * (lane ^ (4 * ((lane >> 5) + 2 * (w & 1))));
   const int place = tab_seg32(L, min((BKV / 32) * t.idx + (w >> 1), (L - 1) / 32)) + q_first;
   const __amdgpu_buffer_rsrc_t pz_rs = __builtin_amdgcn_make_buffer_rsrc(a.pz + ((int64_t)head * a.pz_entries + t.tab_base) * PZ_WORDS, 0,
