@@ -24,23 +24,27 @@ for p in (ROOT, os.path.join(ROOT, "stickbreaking-attention_amd")):
 PEAK_BF16_TFLOPS = 2500.0   # MI355X published dense bf16 MFMA peak
 PEAK_HBM_GBS = 8000.0       # MI355X published HBM3E bandwidth
 
-# Figures that only rocprofv3 can see, on workloads c3, c2 and d256, recorded from the runs whose summaries are under profiles/
-# and valid for the library version they were measured with (any other version of libsba.so reports null).
+# Figures that only rocprofv3 can see, recorded from the runs whose summaries are under profiles/ and valid for the
+# library version they were measured with (any other version of libsba.so reports null).
 #   traffic: bytes per launch between the L2s and the fabric from two `--pmc` runs of this script (FETCH_SIZE, then
 #     WRITE_SIZE, KiB per dispatch, summed over XCDs), each scaled by what the same counter reads for the 256 MiB device
 #     copy of --calibrate-copy (FETCH_SIZE x2.0, WRITE_SIZE x1.0): profiles/c3_hbm_traffic_pmc.txt
 #   mfma_busy, valu_busy, coexec: fractions of the launch's SIMD-cycles in which the matrix pipe is busy
 #     (SQ_VALU_MFMA_BUSY_CYCLES), a vector instruction is active (4 x SQ_ACTIVE_INST_VALU) and both at once
 #     (SQ_VALU_MFMA_COEXEC_CYCLES), over 1024 SIMDs x GRBM_GUI_ACTIVE / 8: profiles/c3_sq_counters_pmc.txt
-#   (c2: profiles/c2_one_pass_backward.txt, d256: profiles/d256_fwd_bwd_kernel_trace.txt)
-MEASURED = {"sba_version": 215,
-            "c3": {"fwd_kernel": {"traffic": 1.070e9, "mfma_busy": 0.464, "valu_busy": 0.552, "coexec": 0.196},
-                   "bwd_chain_kernel": {"traffic": 7.599e9, "mfma_busy": 0.358, "valu_busy": 0.397, "coexec": 0.131}},
-            "c2": {"fwd_kernel": {"traffic": 1.134e8, "mfma_busy": 0.257, "valu_busy": 0.567, "coexec": 0.152},
-                   "bwd_chain_kernel": {"traffic": 6.510e8, "mfma_busy": 0.237, "valu_busy": 0.496, "coexec": 0.120}},
-            "d256": {"fwd_kernel": {"traffic": 1.598e9, "mfma_busy": 0.465, "valu_busy": 0.319, "coexec": 0.092},
-                     "bwd_dq_wide_kernel": {"traffic": 2.719e9, "mfma_busy": 0.372, "valu_busy": 0.385, "coexec": 0.121},
-                     "bwd_dkdv_given_kernel": {"traffic": 2.203e9, "mfma_busy": 0.345, "valu_busy": 0.134, "coexec": 0.047}}}
+#   (c2: profiles/c2_one_pass_backward.txt, c4: profiles/c4_fwd_bwd_kernel_trace.txt, c5: profiles/c5_fwd_kernel_trace.txt,
+#   d256: profiles/d256_fwd_bwd_kernel_trace.txt)
+MEASURED = {"sba_version": 216,
+            "c3": {"fwd_kernel": {"traffic": 1.073e9, "mfma_busy": 0.465, "valu_busy": 0.553, "coexec": 0.196},
+                   "bwd_chain_kernel": {"traffic": 7.587e9, "mfma_busy": 0.360, "valu_busy": 0.400, "coexec": 0.133}},
+            "c2": {"fwd_kernel": {"traffic": 1.134e8, "mfma_busy": 0.256, "valu_busy": 0.565, "coexec": 0.151},
+                   "bwd_chain_kernel": {"traffic": 6.514e8, "mfma_busy": 0.237, "valu_busy": 0.498, "coexec": 0.120}},
+            "c4": {"fwd_kernel": {"traffic": 2.783e8, "mfma_busy": 0.111, "valu_busy": 0.385, "coexec": 0.049},
+                   "bwd_short_kernel": {"traffic": 4.790e8, "mfma_busy": 0.124, "valu_busy": 0.430, "coexec": 0.041}},
+            "c5": {"fwd_kernel": {"traffic": 3.503e10, "mfma_busy": 0.611, "valu_busy": 0.684, "coexec": 0.275}},
+            "d256": {"fwd_kernel": {"traffic": 1.600e9, "mfma_busy": 0.467, "valu_busy": 0.320, "coexec": 0.093},
+                     "bwd_dq_wide_kernel": {"traffic": 2.715e9, "mfma_busy": 0.373, "valu_busy": 0.388, "coexec": 0.123},
+                     "bwd_dkdv_given_kernel": {"traffic": 2.201e9, "mfma_busy": 0.352, "valu_busy": 0.137, "coexec": 0.048}}}
 
 # algorithmic and executed FLOPs per causal pair and head_dim of a forward and of the backward's two passes
 ALGORITHMIC, EXECUTED = [4.0, 6.0, 4.0], [4.0, 6.0, 8.0]

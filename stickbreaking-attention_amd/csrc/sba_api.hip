@@ -512,8 +512,8 @@ bool chain_possible(const sba_problem* p, bool fixed, const Sizes& sz) {
          chains <= (long long)CHAIN_QUEUES * CHAIN_GROUP * CHAIN_MAX_GROUPS &&
          ((long long)declared_max_doc_len(p, fixed) + BM) * chain_width(p->head_dim) * 4 < (1ll << 31) && device_cus() == 256;
 }
-// Steps of 64 queries instead of 32 (head_dim <= 64).  They do more per step and CU (4 x 16 x 2048 at head_dim 64: 153
-// us for 179) but a key tile lags its predecessor by three steps of either size, so as long as that lag is what a
+// Steps of 64 queries instead of 32 (head_dim <= 64).  They do more per step and CU (4 x 16 x 2048 at head_dim 64: 159
+// us for 187) but a key tile lags its predecessor by three steps of either size, so as long as that lag is what a
 // problem takes (8 heads of 8192 keys: 430 us for 372) the small ones are the better ones.  The line: the work of a CU
 // in steps, squares / (2 x 64 x 128 x 256 CUs), against the steps of the longest document and a twentieth more (32
 // heads of 7 K tokens in six documents of up to 3000 264 us for 298, 12 x 3 x 2500 161 for 175, 4 x 2 x 8192 428 for
@@ -538,8 +538,9 @@ bool chain_streams(const sba_problem* p, bool fixed, const Sizes& sz) {
   return longest <= BKV || (width == 128 ? rows > 20 * 1024 : rows > 28 * 1024 && longest + sz.rows / sz.n_docs <= 2048);
 }
 // Where the one-pass form is the faster one (gain over the two passes; measured on 1220 problems of 1 to 32 heads and
-// 512 to 200 K tokens in 1 to 128 documents, declared lengths exact: 1.003 of the faster form's time at head_dim 96 and
-// 128, 1.01 at 64, 1.015 at 32, by the geometric mean).
+// 512 to 200 K tokens in 1 to 128 documents, declared lengths exact).  On 1600 others, drawn with more spread among a
+// problem's lengths, the choice of form and step costs 0.6 % against the best at head_dim 80 to 128, 3.1 % at 64 and
+// 4.0 % at 32 by the geometric mean, 1.4 to 1.5 times at the worst.
 bool chain_wanted(const sba_problem* p, bool fixed, const Sizes& sz) {
   const int form = backward_form();
   if (form == 1 || !chain_possible(p, fixed, sz)) return false;

@@ -34,8 +34,8 @@
 // 128, 1311 -> 1292 us; 12 x 4 x 4096 694 -> 683; 16 x 7 K in six documents, head_dim 96, 240 -> 226; 12 heads of 1500,
 // 900 and 601 tokens, head_dim 64, 80.0 -> 69.8 and 128, 95.8 -> 88.  (Documents of one or two
 // tiles above head_dim 64, where an item's beginning and end are the time, are up to 3 % slower: 32 heads of 64 x 256 at
-// 128 346 -> 354, 19 of 235 x 118 309 -> 316.  None of the changes gives that back alone: no poll, no wait for the
-// carried sum, columns read behind the barrier and one kind of iteration are all within 1 % of it or slower.)
+// 128 346 -> 354, 19 of 235 x 118 310 -> 317.  Each role's change costs half of it, and each makes long documents 1 to
+// 2 % faster; of the changes one by one only the poll's absence gives back 1 %, and takes 1 % from long documents.)
 // At head_dim 128 it waits: 44 % of the wave cycles on 32 heads x 16 K tokens (22 .. 25 % in the two passes;
 // profiles/c3_sq_counters_pmc.txt), with the matrix pipe busy for 36 %.  Such a launch fetches 4.5 GB from behind the
 // L2s and writes 3.1 GB there, 5.8 TB/s where a plain copy reaches 4.9: of the 2.8 GB of partial dq each way, all that
